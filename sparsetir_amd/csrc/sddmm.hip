@@ -32,9 +32,17 @@ __device__ __forceinline__ float group_allreduce(float p) {
   return p;
 }
 
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+// a row whose width is no multiple of four starts at any float: 16-byte loads need 4-byte alignment only
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld4(const float* p) {
+  const f32x4u v = *reinterpret_cast<const f32x4u*>(p);
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
 
-template <int G, int REP>
+// TAIL: feat is no multiple of 4.  The row's last chunk of four features is then loaded from feat - 4
+// on (it must not reach past the end of the array), and the features it shares with the chunk before
+// it are left out of the product.
+template <int G, int REP, bool TAIL>
 __global__ __launch_bounds__(256) void sddmm_kernel(int64_t nnz, int feat, const float* __restrict__ A,
                                                     const float* __restrict__ B, float* __restrict__ C,
                                                     const int32_t* __restrict__ indices,
@@ -59,14 +67,20 @@ __global__ __launch_bounds__(256) void sddmm_kernel(int64_t nnz, int feat, const
       const int sl = g * G + c + u;
       const int r = __shfl(my_row, sl, kWave);
       const int col = __shfl(my_col, sl, kWave);
-      const float* ap = A + (int64_t)r * feat + gl * 4;
-      const float* bp = B + (int64_t)col * feat + gl * 4;
+      const float* ap = A + (int64_t)r * feat;
+      const float* bp = B + (int64_t)col * feat;
 #pragma unroll
       for (int q = 0; q < REP; ++q) {
         // feat below 4*G*REP: the lanes beyond feat / 4 hold padding
-        const bool live = gl * 4 + q * G * 4 < feat;
-        a[u][q] = live ? ld4(ap + q * G * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
-        b[u][q] = live ? ld4(bp + q * G * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const int c0 = gl * 4 + q * G * 4, at = TAIL ? min(c0, feat - 4) : c0;
+        a[u][q] = c0 < feat ? ld4(ap + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+        b[u][q] = c0 < feat ? ld4(bp + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+        if constexpr (TAIL) {
+          const int over = c0 - at;  // features of the chunk that belong to the one before
+          a[u][q].x = over > 0 ? 0.f : a[u][q].x, b[u][q].x = over > 0 ? 0.f : b[u][q].x;
+          a[u][q].y = over > 1 ? 0.f : a[u][q].y, b[u][q].y = over > 1 ? 0.f : b[u][q].y;
+          a[u][q].z = over > 2 ? 0.f : a[u][q].z, b[u][q].z = over > 2 ? 0.f : b[u][q].z;
+        }
       }
     }
 #pragma unroll
@@ -86,7 +100,8 @@ __global__ __launch_bounds__(256) void sddmm_kernel(int64_t nnz, int feat, const
   if (e < nnz) __builtin_nontemporal_store(scale ? out * __builtin_nontemporal_load(scale + e) : out, C + e);
 }
 
-// Any feature width: one wavefront per 64 nonzeros, lanes stride over the features.
+// Rows narrower than one float4 or wider than two per lane: one wavefront per 64 nonzeros, lanes
+// stride over the features.
 __global__ __launch_bounds__(256) void sddmm_generic_kernel(int64_t nnz, int feat, const float* __restrict__ A,
                                                             const float* __restrict__ B, float* __restrict__ C,
                                                             const int32_t* __restrict__ indices,
@@ -154,12 +169,15 @@ static int sddmm_launch(int32_t m, int32_t n, int32_t feat, int64_t nnz, const f
   hipStream_t st = static_cast<hipStream_t>(stream);
   dim3 grid((unsigned)blocks), block(256);
 #define STIR_SDDMM(G, REP)                                                                             \
-  hipLaunchKernelGGL((sddmm_kernel<G, REP>), grid, block, 0, st, nnz, feat, d_A, d_B, d_C, d_indices, d_mid, \
-                     d_scale)
-  // feature widths that are a multiple of 4 take the vectorised kernel with the smallest lane
-  // group that covers them; anything else the generic one
+  if (feat % 4 == 0)                                                                                   \
+    hipLaunchKernelGGL((sddmm_kernel<G, REP, false>), grid, block, 0, st, nnz, feat, d_A, d_B, d_C, d_indices, d_mid, \
+                       d_scale);                                                                       \
+  else                                                                                                 \
+    hipLaunchKernelGGL((sddmm_kernel<G, REP, true>), grid, block, 0, st, nnz, feat, d_A, d_B, d_C, d_indices, d_mid, \
+                       d_scale)
+  // the smallest lane group that covers the feature width
   int cls = -1;
-  if (feat % 4 == 0 && feat <= 512)
+  if (feat >= 4 && feat <= 512)
     for (cls = 0; (16 << cls) < feat; ++cls) {
     }
   switch (cls) {

@@ -43,7 +43,26 @@ struct alignas(16) HybBucket {
 // wavefront each, so that a hub row does not serialise on a single wavefront.
 constexpr int kRowChunk = 256;
 
-__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+// four consecutive floats; a row of B whose width is no multiple of four starts at any float, and a
+// 16-byte load only needs its address to be a multiple of four bytes
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld4(const float* p) {
+  const f32x4u v = *reinterpret_cast<const f32x4u*>(p);
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// Feature widths: a lane's chunk number r is the four features from c0 = 4 * (lane in group + r * G)
+// on.  In a row whose width is no multiple of four the last chunk would reach into the next row (or
+// past the end of B): it is loaded from feat - 4 instead, four features of this row again; a store
+// writes the shared ones twice with the same value, an addition moves the ones that are not shared to
+// the front first (tail_chunk).
+__device__ __forceinline__ int chunk_offset(int c0, int feat) { return min(c0, feat - 4); }
+
+__device__ __forceinline__ float4 tail_chunk(float4 a, int over) {  // over: features of `a` before c0
+  if (over & 1) a = make_float4(a.y, a.z, a.w, 0.f);
+  if (over & 2) a = make_float4(a.z, a.w, 0.f, 0.f);
+  return a;
+}
 
 __device__ __forceinline__ void fma4(float4& acc, float a, const float4& x) {
   acc.x = fmaf(a, x.x, acc.x);
@@ -81,23 +100,32 @@ __device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int l
                                           const float4 (&acc)[REP], int atomic, float* stage) {
   const int g = lane / G, gl = lane % G;
   if (atomic == 2) {
-    // the only writer of this row in this launch: no atomics needed to add
-    float* base = C + row * feat + gl * 4;
+    // the only writer of this row in this launch: no atomics needed to add.  All of the row is read
+    // before any of it is written: of a width that is no multiple of four, two chunks share features.
+    float* base = C + row * feat;
+    float4 old[REP];
 #pragma unroll
     for (int r = 0; r < REP; ++r) {
-      if (gl * 4 + r * G * 4 >= feat) continue;
-      float* q = base + r * G * 4;
-      const float o0 = q[0], o1 = q[1], o2 = q[2], o3 = q[3];
-      q[0] = o0 + acc[r].x, q[1] = o1 + acc[r].y, q[2] = o2 + acc[r].z, q[3] = o3 + acc[r].w;
+      const int c0 = gl * 4 + r * G * 4;
+      if (c0 < feat) old[r] = ld4(base + chunk_offset(c0, feat));
+    }
+#pragma unroll
+    for (int r = 0; r < REP; ++r) {
+      const int c0 = gl * 4 + r * G * 4;
+      if (c0 >= feat) continue;  // feat below 4*G*REP: this lane's chunk is padding
+      float* q = base + chunk_offset(c0, feat);
+      q[0] = old[r].x + acc[r].x, q[1] = old[r].y + acc[r].y;
+      q[2] = old[r].z + acc[r].z, q[3] = old[r].w + acc[r].w;
     }
     return;
   }
   if (!atomic) {
-    float* base = C + row * feat + gl * 4;
+    float* base = C + row * feat;
 #pragma unroll
     for (int r = 0; r < REP; ++r) {
-      if (gl * 4 + r * G * 4 >= feat) continue;  // feat below 4*G*REP: this lane's float4 is padding
-      float* q = base + r * G * 4;
+      const int c0 = gl * 4 + r * G * 4;
+      if (c0 >= feat) continue;
+      float* q = base + chunk_offset(c0, feat);
       __builtin_nontemporal_store(acc[r].x, q);
       __builtin_nontemporal_store(acc[r].y, q + 1);
       __builtin_nontemporal_store(acc[r].z, q + 2);
@@ -107,7 +135,14 @@ __device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int l
   }
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int r = 0; r < REP; ++r) *reinterpret_cast<float4*>(stage + (r * kWave + lane) * 4) = acc[r];
+  for (int r = 0; r < REP; ++r) {
+    float4 v = acc[r];
+    if (feat & 3) {  // uniform
+      const int over = gl * 4 + r * G * 4 + 4 - feat;
+      if (over > 0 && over < 4) v = tail_chunk(v, over);
+    }
+    *reinterpret_cast<float4*>(stage + (r * kWave + lane) * 4) = v;
+  }
   __builtin_amdgcn_wave_barrier();
   float* base = C + row * feat + gl;
 #pragma unroll
@@ -152,11 +187,13 @@ __device__ __forceinline__ void csr_accumulate(float4 (&acc)[REP], int start, in
         const int j = j0 + u * NG + g;  // < 64 because NG*UNROLL divides 64
         const int col = __shfl(my_col, j, kWave);
         v[u] = __shfl(my_val, j, kWave);
-        const float* bp = B + (int64_t)col * feat + gl * 4;
+        const float* bp = B + (int64_t)col * feat;
 #pragma unroll
-        for (int r = 0; r < REP; ++r)
-          x[u][r] = (j < cnt && gl * 4 + r * G * 4 < feat && (!INDIRECT || v[u] != 0.f)) ? ld4(bp + r * G * 4)
-                                                                                          : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int r = 0; r < REP; ++r) {
+          const int c0 = gl * 4 + r * G * 4;
+          x[u][r] = (j < cnt && c0 < feat && (!INDIRECT || v[u] != 0.f)) ? ld4(bp + chunk_offset(c0, feat))
+                                                                         : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
       }
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
@@ -233,7 +270,7 @@ __global__ __launch_bounds__(256) void csr_spmm_rows_kernel(int m, int feat, int
   const bool alone = end - start <= kGroupRow;
   const int my_end = alone ? end : start;
   const bool chunk_live = gl * 4 < feat;
-  const float* Bl = B + gl * 4;
+  const float* Bl = B + chunk_offset(gl * 4, feat);
   float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int base = start; base < my_end; base += G) {
     const int p = base + gl;
@@ -255,12 +292,9 @@ __global__ __launch_bounds__(256) void csr_spmm_rows_kernel(int m, int feat, int
       for (int u = 0; u < CH; ++u) fma4(acc, v[u], x[u]);
     }
   }
-  if (row < m && alone && chunk_live) {
-    float* q = C + row * feat + gl * 4;
-    __builtin_nontemporal_store(acc.x, q);
-    __builtin_nontemporal_store(acc.y, q + 1);
-    __builtin_nontemporal_store(acc.z, q + 2);
-    __builtin_nontemporal_store(acc.w, q + 3);
+  if (row < m && alone) {
+    const float4 sum[1] = {acc};
+    write_row<G, 1>(C, row, feat, lane, sum, 0, nullptr);
   }
   // the longer rows, one after the other, by the whole wavefront
   uint64_t todo = __ballot(row < m && !alone && gl == 0);
@@ -316,7 +350,7 @@ __global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int
   }
 }
 
-// Any feature width: one wavefront per row, lane l owns features l, l+64, ...
+// Widths without a vector class: one wavefront per row, lane l owns features l, l+64, ...
 __global__ __launch_bounds__(256) void csr_spmm_generic_kernel(int m, int feat, const float* __restrict__ A,
                                                                const float* __restrict__ B,
                                                                float* __restrict__ C,
@@ -369,12 +403,13 @@ __device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, in
       const int sl = g * G + c + u;
       const int col = __shfl(my_col, sl, kWave);
       v[u] = __shfl(my_val, sl, kWave);
-      const float* bp = B + (int64_t)col * feat + gl * 4;
+      const float* bp = B + (int64_t)col * feat;
       // a slot of weight zero (padding) adds nothing: its row of B is not fetched
 #pragma unroll
-      for (int r = 0; r < REP; ++r)
-        x[u][r] = (v[u] != 0.f && gl * 4 + r * G * 4 < feat) ? ld4(bp + r * G * 4)
-                                                             : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int r = 0; r < REP; ++r) {
+        const int c0 = gl * 4 + r * G * 4;
+        x[u][r] = (v[u] != 0.f && c0 < feat) ? ld4(bp + chunk_offset(c0, feat)) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
@@ -430,11 +465,12 @@ __device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int
         const int sl = g * G + c + u;
         const int col = __shfl(my_col, sl, kWave);
         v[u] = __shfl(my_val, sl, kWave);  // zero beyond s_end and on padding
-        const float* bp = B + (int64_t)col * feat + gl * 4;
+        const float* bp = B + (int64_t)col * feat;
 #pragma unroll
-        for (int r = 0; r < REP; ++r)
-          x[u][r] = (v[u] != 0.f && gl * 4 + r * G * 4 < feat) ? ld4(bp + r * G * 4)
-                                                             : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int r = 0; r < REP; ++r) {
+          const int c0 = gl * 4 + r * G * 4;
+          x[u][r] = (v[u] != 0.f && c0 < feat) ? ld4(bp + chunk_offset(c0, feat)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
       }
 #pragma unroll
       for (int u = 0; u < CH; ++u)
@@ -485,7 +521,7 @@ __global__ __launch_bounds__(256) void hyb_spmm_kernel(const HybBucket* __restri
   }
 }
 
-// Any feature width: one wavefront per ELL row, lane l owns features l, l+64, ...
+// Widths without a vector class: one wavefront per ELL row, lane l owns features l, l+64, ...
 __global__ __launch_bounds__(256) void hyb_spmm_generic_kernel(const HybBucket* __restrict__ table,
                                                                int nb, int64_t total_rows, int feat,
                                                                const float* __restrict__ B,
@@ -586,9 +622,12 @@ __global__ __launch_bounds__(256) void hyb_table_fill_kernel(HybTableChunk chunk
   for (int i = threadIdx.x; i < count * kWords; i += 256) out[i] = src[i];
 }
 
-// 0..5: lane groups of 4, 8, 16, 32, 64 lanes and 64 lanes x 2 float4 cover feat; -1: generic kernel
+// 0..5: lane groups of 4, 8, 16, 32, 64 lanes and 64 lanes x 2 float4 cover feat; -1: the kernel of
+// one lane per feature (a row narrower than one float4, or wider than two per lane).  Widths that are
+// no multiple of 4 take the same kernels (chunk_offset): 169 k nodes, 1.17 M edges with hubs on both
+// sides, 47 features: 1750 us with one lane per feature (the chain of the hub row), 52 us with these.
 int vector_class(int feat) {
-  if (feat % 4 != 0 || feat > 512) return -1;
+  if (feat < 4 || feat > 512) return -1;
   int c = 0;
   while ((16 << c) < feat) ++c;
   return c;
@@ -934,8 +973,7 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
       hipLaunchKernelGGL((csr_long_rows_kernel<G, REP>), pieces, block, 0, st, m, feat, (int64_t)0, nnz, d_A,   \
                          d_B, d_C, d_indptr, d_indices);                                                   \
   }
-  // feature widths that are a multiple of 4 take the vectorised kernel with the smallest lane
-  // group that covers them (lanes beyond feat / 4 idle); anything else the generic one
+  // the smallest lane group that covers the feature width (lanes beyond feat / 4 idle)
   // lane groups narrower than the wavefront: a lane group per row (csr_spmm_rows_kernel)
 #define STIR_CSR_ROWS(G)                                                                                   \
   {                                                                                                        \

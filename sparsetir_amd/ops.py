@@ -31,7 +31,7 @@ import operator
 
 import torch
 
-from . import _lib
+from . import _host, _lib
 
 
 def _ptr(t):
@@ -51,8 +51,9 @@ class _PlanCache:
     while a plan made from them exists."""
     capacity = 8
 
-    def __init__(self, destroy):
+    def __init__(self, destroy, forget):
         self._destroy = destroy
+        self._forget = forget  # tells the launcher of the operator that a plan (None: every plan) goes
         self._plans = collections.OrderedDict()  # key -> (plan, arrays kept alive)
         self.builds = 0
 
@@ -65,12 +66,14 @@ class _PlanCache:
 
     def put(self, key, plan, keep):
         while len(self._plans) >= self.capacity:
-            _, (old, _) = self._plans.popitem(last=False)
+            gone, (old, _) = self._plans.popitem(last=False)
+            self._forget(gone)
             self._destroy(old)
         self._plans[key] = (plan, keep)
         self.builds += 1
 
     def clear(self):
+        self._forget(None)
         while self._plans:
             _, (old, _) = self._plans.popitem()
             self._destroy(old)
@@ -89,13 +92,36 @@ _data_ptrs = torch.Tensor.data_ptr
 _version_of = operator.attrgetter("_version")
 
 
-def _same_objects(a, b):
-    return b is not None and len(a) == len(b) and all(map(operator.is_, a, b))
+# operand descriptions of _host.Launcher: (type, length, what of the tensor a plan depends on)
+_CODE = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2, torch.int32: 3}
+_FREE, _ADDRESS, _CONTENT = 0, 1, 3  # nothing; where it lives; where it lives and torch's version counter
 
 
 class _Operator:
+    """A call goes to the native launcher first (``_launch``, csrc/bindings/host.cpp), which takes it
+    when every argument is as expected and the plan it needs is known.  Everything else -- a wrong
+    argument, the first call of a plan, tensors on a device that is not the current one -- is the
+    business of ``_call`` of the operator."""
     name = "main"
     entry_name = "main"
+
+    def __call__(self, *args):
+        rc = self._launch(args)
+        if rc == 0:
+            return
+        if rc == 1:
+            self._call(*args)
+        elif rc == -1:
+            _lib.check(rc)
+        else:  # launched, with a plan that was not the one used last
+            self._plans.get(rc)
+
+    def _bind(self, kind, sizes, spec, key=None):
+        """Makes the launcher: ``spec`` as for :meth:`_check`, ``key`` what a plan depends on."""
+        # (an element type that no operator takes: the type code of no tensor, so that _call refuses it)
+        self._host = _host.Launcher(kind, sizes, [(_CODE.get(t, -1), length, key[k] if key else _FREE)
+                                                  for k, (_, t, length) in enumerate(spec)])
+        self._launch = self._host.launch
 
     def _check(self, args, spec):
         """spec: list of (label, dtype, length).  Returns the device all arrays live on."""
@@ -158,12 +184,13 @@ class CsrMM(_Operator):
     def __init__(self, m, n, feat, nnz):
         self.m, self.n, self.feat, self.nnz = int(m), int(n), int(feat), int(nnz)
         self.L = _lib.lib()
-
-    def __call__(self, *args):
         f32, i32 = torch.float32, torch.int32
-        dev = self._check(args, [("A", f32, self.nnz), ("B", f32, self.n * self.feat),
-                                 ("C", f32, self.m * self.feat), ("indptr", i32, self.m + 1),
-                                 ("indices", i32, self.nnz)])
+        self._operands = [("A", f32, self.nnz), ("B", f32, self.n * self.feat), ("C", f32, self.m * self.feat),
+                          ("indptr", i32, self.m + 1), ("indices", i32, self.nnz)]
+        self._bind(_host.CSR, (self.m, self.n, self.feat, self.nnz), self._operands)
+
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, b, c, indptr, indices = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_csr_spmm_f32(self.m, self.n, self.feat, self.nnz, _ptr(a),
@@ -193,9 +220,10 @@ class HybCsrMM(_Operator):
         if len(self.nrows) != self.parts * len(self.buckets):
             raise _lib.SparseTIRError("hyb_csrmm: nrows must have num_col_parts*len(buckets) entries")
         self.L = _lib.lib()
-        self._plans = _PlanCache(self.L.stir_hyb_plan_destroy)
+        self._host = _host.Launcher.hyb(self.n, self.m, self.feat, self.buckets, self.nrows)
+        self._launch = self._host.launch
+        self._plans = _PlanCache(self.L.stir_hyb_plan_destroy, self._host.forget)
         self._spec_cache = None
-        self._last_args, self._last_dev = None, None
 
     @property
     def plan_builds(self):
@@ -214,7 +242,6 @@ class HybCsrMM(_Operator):
     def invalidate(self):
         """Forget every plan made from the arrays of earlier calls."""
         self._plans.clear()
-        self._last_args = None
 
     def __del__(self):
         try:
@@ -222,27 +249,14 @@ class HybCsrMM(_Operator):
         except Exception:
             pass
 
-    def __call__(self, *args):
+    def _call(self, *args):
         if self._spec_cache is None:
             self._spec_cache = self._spec()
+        dev = self._check(args, self._spec_cache)
         b, c, triples = args[0], args[1], args[2:]
         # addresses of all arrays; torch's count of in-place changes for the row and column arrays
-        try:
-            key = (tuple(map(_data_ptrs, triples)), tuple(map(_version_of, triples[1::3])),
-                   tuple(map(_version_of, triples[2::3])))
-        except (TypeError, AttributeError):  # an argument that is no tensor: the check says which
-            self._check(args, self._spec_cache)
-            raise
-        if _same_objects(triples, self._last_args) and self._plans.get((self._last_dev,) + key) is not None:
-            # the tensor objects of the last, checked call, unchanged (and kept alive by their plan):
-            # only B and C are new
-            dev = self._check(args[:2], self._spec_cache[:2])
-            if dev != self._last_dev:
-                raise _lib.SparseTIRError(f"{self.name}: all arrays must be on one device")
-        else:
-            dev = self._check(args, self._spec_cache)
-            self._last_args, self._last_dev = triples, dev
-        key = (dev,) + key
+        key = (dev, tuple(map(_data_ptrs, triples)), tuple(map(_version_of, triples[1::3])),
+               tuple(map(_version_of, triples[2::3])))
         with torch.cuda.device(dev):
             plan = self._plans.get(key)
             if plan is None:
@@ -257,6 +271,7 @@ class HybCsrMM(_Operator):
                                                        len(self.buckets), widths, nrows, A, R, Cc))
                 self._plans.put(key, plan, triples)  # the plan stores pointers into these arrays
             _lib.check(self.L.stir_hyb_spmm_f32(plan, self.feat, _ptr(b), _ptr(c), _stream()))
+            self._host.remember(args, plan.value, key)
 
 
 class SddmmPreproc(_Operator):
@@ -265,6 +280,10 @@ class SddmmPreproc(_Operator):
     def __init__(self, m, n, feat, nnz):
         self.m, self.n, self.feat, self.nnz = int(m), int(n), int(feat), int(nnz)
         self.L = _lib.lib()
+        self._operands = self._spec()
+        self._bind(self._kind, (self.m, self.n, self.feat, self.nnz), self._operands)
+
+    _kind = _host.SDDMM_PREPROC
 
     def _spec(self):
         f32, i32 = torch.float32, torch.int32
@@ -272,8 +291,8 @@ class SddmmPreproc(_Operator):
                 ("C", f32, self.nnz), ("indptr", i32, self.m + 1), ("indices", i32, self.nnz),
                 ("mid", i32, self.nnz)]
 
-    def __call__(self, *args):
-        dev = self._check(args, self._spec())
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, b, c, indptr, indices, mid = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_sddmm_preproc(self.m, self.nnz, _ptr(indptr), _ptr(mid), _stream()))
@@ -281,9 +300,10 @@ class SddmmPreproc(_Operator):
 
 class Sddmm(SddmmPreproc):
     name = "sddmm"
+    _kind = _host.SDDMM
 
-    def __call__(self, *args):
-        dev = self._check(args, self._spec())
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, b, c, indptr, indices, mid = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_sddmm_f32(self.m, self.n, self.feat, self.nnz, _ptr(a), _ptr(b),
@@ -294,9 +314,13 @@ class Sddmm(SddmmPreproc):
 class SddmmScaled(SddmmPreproc):
     """C[e] = E[e] * <A[mid[e], :], B[indices[e], :]>: f(A, B, C, indptr, indices, mid, E)."""
     name = "sddmm_scaled"
+    _kind = _host.SDDMM_SCALED
 
-    def __call__(self, *args):
-        dev = self._check(args, self._spec() + [("E", torch.float32, self.nnz)])
+    def _spec(self):
+        return super()._spec() + [("E", torch.float32, self.nnz)]
+
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, b, c, indptr, indices, mid, e = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_sddmm_scaled_f32(self.m, self.n, self.feat, self.nnz, _ptr(a), _ptr(b),
@@ -317,13 +341,16 @@ class BsrMM(_Operator):
         if dtype not in (torch.float16, torch.bfloat16):
             raise _lib.SparseTIRError("bsrmm: inputs must be float16 or bfloat16")
         self.L = _lib.lib()
-
-    def __call__(self, *args):
         i32 = torch.int32
-        dev = self._check(args, [("A", self.dtype, self.nnzb * self.blk * self.blk),
-                                 ("X", self.dtype, self.nb * self.blk * self.feat),
-                                 ("Y", self.out_dtype, self.mb * self.blk * self.feat),
-                                 ("indptr", i32, self.mb + 1), ("indices", i32, self.nnzb)])
+        self._operands = [("A", self.dtype, self.nnzb * self.blk * self.blk),
+                          ("X", self.dtype, self.nb * self.blk * self.feat),
+                          ("Y", self.out_dtype, self.mb * self.blk * self.feat),
+                          ("indptr", i32, self.mb + 1), ("indices", i32, self.nnzb)]
+        self._bind(_host.BSR, (_DT[self.dtype], _DT.get(self.out_dtype, -1), self.mb, self.nb, self.blk, self.feat, self.nnzb),
+                   self._operands)
+
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, x, y, indptr, indices = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_bsr_spmm(_DT[self.dtype], _DT[self.out_dtype], self.mb, self.nb,
@@ -341,14 +368,17 @@ class DBsrMM(_Operator):
         self.dtype = dtype
         self.out_dtype = dtype if out_dtype is None else out_dtype
         self.L = _lib.lib()
-
-    def __call__(self, *args):
         i32 = torch.int32
-        dev = self._check(args, [("A", self.dtype, self.nnzb * self.blk * self.blk),
-                                 ("X", self.dtype, self.nb * self.blk * self.feat),
-                                 ("Y", self.out_dtype, self.mb * self.blk * self.feat),
-                                 ("indptr_0", i32, 2), ("indices_0", i32, self.nr),
-                                 ("indptr_1", i32, self.nr + 1), ("indices_1", i32, self.nnzb)])
+        self._operands = [("A", self.dtype, self.nnzb * self.blk * self.blk),
+                          ("X", self.dtype, self.nb * self.blk * self.feat),
+                          ("Y", self.out_dtype, self.mb * self.blk * self.feat),
+                          ("indptr_0", i32, 2), ("indices_0", i32, self.nr),
+                          ("indptr_1", i32, self.nr + 1), ("indices_1", i32, self.nnzb)]
+        self._bind(_host.DBSR, (_DT.get(self.dtype, -1), _DT.get(self.out_dtype, -1), self.nr, self.nb, self.blk, self.feat, self.nnzb),
+                   self._operands)
+
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, x, y, _, rows, indptr, indices = args
         with torch.cuda.device(dev):
             _lib.check(self.L.stir_dbsr_spmm(_DT[self.dtype], _DT[self.out_dtype], self.nr, self.nb, self.blk,
@@ -374,7 +404,13 @@ class TcSpMM(_Operator):
         self.t, self.g, self.brows = int(tile_size), int(group_size), int(num_b_rows)
         self.out_dtype = out_dtype
         self.L = _lib.lib()
-        self._plans = _PlanCache(self.L.stir_tc_plan_destroy)
+        f16, i32 = torch.float16, torch.int32
+        self._operands = [("A", f16, self.nnzb * self.t * self.g), ("B", f16, self.brows * self.feat),
+                          ("C", self.out_dtype, self.mb * self.t * self.feat),
+                          ("indptr", i32, self.mb + 1), ("indices", i32, self.nnzb * self.g)]
+        self._bind(_host.TC, (_DT.get(out_dtype, -1), self.mb, self.t, self.g, self.feat, self.nnzb), self._operands,
+                   (_FREE, _FREE, _FREE, _CONTENT, _FREE))
+        self._plans = _PlanCache(self.L.stir_tc_plan_destroy, self._host.forget)
 
     @property
     def plan_builds(self):
@@ -390,11 +426,8 @@ class TcSpMM(_Operator):
         except Exception:
             pass
 
-    def __call__(self, *args):
-        f16, i32 = torch.float16, torch.int32
-        dev = self._check(args, [("A", f16, self.nnzb * self.t * self.g), ("B", f16, self.brows * self.feat),
-                                 ("C", self.out_dtype, self.mb * self.t * self.feat),
-                                 ("indptr", i32, self.mb + 1), ("indices", i32, self.nnzb * self.g)])
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, b, c, indptr, indices = args
         with torch.cuda.device(dev):
             if self.t not in (8, 16, 32) or self.g != 16:  # refused by the library with its own message
@@ -415,6 +448,7 @@ class TcSpMM(_Operator):
                                                        self.feat, self.nnzb,
                                                        _ptr(a), _ptr(b), _ptr(c), _ptr(indptr), _ptr(indices),
                                                        _stream()))
+            self._host.remember(args, plan.value, key)
 
 
 class Rgms(_Operator):
@@ -459,9 +493,15 @@ class Rgms(_Operator):
         self.rb, self.cb = [int(v) for v in rows_bkt], [int(v) for v in cols_bkt]
         self.groups = [int(v) for v in groups]
         self.L = _lib.lib()
-        self._plans = _PlanCache(getattr(self.L, self._fns[2]))
-        self._spec_cache = None
-        self._last_args, self._last_dev = None, None
+        # index arrays: address and torch's count of in-place changes; weights: address only, unless the
+        # plan keeps them inside its index
+        nb = len(self.groups)
+        key = [_FREE] * 3 + [_CONTENT if self._static else _ADDRESS, _CONTENT, _CONTENT] * nb + [_CONTENT] * nb
+        form = 2 if self._in_dtype is torch.bfloat16 else 1 if self._out_dtype is torch.float16 else 0
+        self._operands = self._spec()
+        self._bind(_host.RGMS_F32 if self._in_dtype is torch.float32 else _host.RGMS,
+                   (self.m, self.n, self.R, self.fin, self.fout, form), self._operands, key)
+        self._plans = _PlanCache(getattr(self.L, self._fns[2]), self._host.forget)
 
     @property
     def plan_builds(self):
@@ -481,7 +521,6 @@ class Rgms(_Operator):
     def invalidate(self):
         """Forget the plans (and edge indices) made from the arrays of earlier calls."""
         self._plans.clear()
-        self._last_args = None
 
     def __del__(self):
         try:
@@ -489,31 +528,14 @@ class Rgms(_Operator):
         except Exception:
             pass
 
-    def __call__(self, *args):
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         w, x, y, rest = args[0], args[1], args[2], args[3:]
         nb = len(self.groups)
         triples, mids = rest[:3 * nb], rest[3 * nb:]
-        # index arrays: address and torch's count of in-place changes; weights: address only, unless
-        # the plan keeps them inside its index
-        if self._spec_cache is None:
-            self._spec_cache = self._spec()
-        try:
-            key = (tuple(map(_data_ptrs, rest)), tuple(map(_version_of, triples[1::3])),
-                   tuple(map(_version_of, triples[2::3])), tuple(map(_version_of, mids)),
-                   tuple(map(_version_of, triples[0::3])) if self._static else ())
-        except (TypeError, AttributeError):  # an argument that is no tensor: the check says which
-            self._check(args, self._spec_cache)
-            raise
-        if _same_objects(rest, self._last_args) and self._plans.get((self._last_dev,) + key) is not None:
-            # the tensor objects of the last, checked call, unchanged (and kept alive by their plan):
-            # only W, X and Y are new
-            dev = self._check(args[:3], self._spec_cache[:3])
-            if dev != self._last_dev:
-                raise _lib.SparseTIRError(f"{self.name}: all arrays must be on one device")
-        else:
-            dev = self._check(args, self._spec_cache)
-            self._last_args, self._last_dev = rest, dev
-        key = (dev,) + key
+        key = (dev, tuple(map(_data_ptrs, rest)), tuple(map(_version_of, triples[1::3])),
+               tuple(map(_version_of, triples[2::3])), tuple(map(_version_of, mids)),
+               tuple(map(_version_of, triples[0::3])) if self._static else ())
         with torch.cuda.device(dev):
             plan = self._plans.get(key)
             if plan is None:
@@ -532,6 +554,7 @@ class Rgms(_Operator):
                     _lib.check(self.L.stir_rgms_f32_plan_set_deterministic(plan, 1))
             _lib.check(getattr(self.L, self._fns[1])(plan, self.m, self.n, self.R, self.fin, self.fout,
                                                      _ptr(w), _ptr(x), _ptr(y), _stream()))
+            self._host.remember(args, plan.value, key)
 
 
 class RgmsF32(Rgms):
@@ -569,7 +592,14 @@ class RgmsCsf(_Operator):
         self.fin, self.fout, self.nnz_i, self.nnz_j = int(feat_in), int(feat_out), int(nnz_i), int(nnz_j)
         self.deterministic = bool(deterministic)
         self.L = _lib.lib()
-        self._plans = _PlanCache(self.L.stir_rgms_csf_f32_plan_destroy)
+        f32, i32 = torch.float32, torch.int32
+        self._operands = [("A", f32, self.nnz_j), ("W", f32, self.R * self.fout * self.fin),
+                          ("X", f32, self.n * self.fin), ("Y", f32, self.m * self.fout),
+                          ("indptr_i", i32, self.R + 1), ("indices_i", i32, self.nnz_i),
+                          ("indptr_j", i32, self.nnz_i + 1), ("indices_j", i32, self.nnz_j)]
+        self._bind(_host.RGMS_CSF, (self.m, self.n, self.R, self.fin, self.fout), self._operands,
+                   (_ADDRESS, _FREE, _FREE, _FREE, _CONTENT, _CONTENT, _CONTENT, _CONTENT))
+        self._plans = _PlanCache(self.L.stir_rgms_csf_f32_plan_destroy, self._host.forget)
 
     @property
     def plan_builds(self):
@@ -585,12 +615,8 @@ class RgmsCsf(_Operator):
         except Exception:
             pass
 
-    def __call__(self, *args):
-        f32, i32 = torch.float32, torch.int32
-        dev = self._check(args, [("A", f32, self.nnz_j), ("W", f32, self.R * self.fout * self.fin),
-                                 ("X", f32, self.n * self.fin), ("Y", f32, self.m * self.fout),
-                                 ("indptr_i", i32, self.R + 1), ("indices_i", i32, self.nnz_i),
-                                 ("indptr_j", i32, self.nnz_i + 1), ("indices_j", i32, self.nnz_j)])
+    def _call(self, *args):
+        dev = self._check(args, self._operands)
         a, w, x, y, pi, ii, pj, ij = args
         if not self.deterministic:
             with torch.cuda.device(dev):
@@ -609,6 +635,7 @@ class RgmsCsf(_Operator):
                 self._plans.put(key, plan, graph)
             _lib.check(self.L.stir_rgms_csf_f32_planned(plan, self.m, self.n, self.R, self.fin, self.fout, _ptr(w),
                                                         _ptr(x), _ptr(y), _stream()))
+            self._host.remember(args, plan.value, key)
 
 
 def build_csrmm(m, n, feat, nnz):

@@ -1,0 +1,69 @@
+"""The native host path of the operators: which plan a call uses, and when it leaves a call to Python."""
+import numpy as np
+import pytest
+import torch
+
+from sparsetir_amd import ops
+from sparsetir_amd._lib import SparseTIRError
+
+pytestmark = pytest.mark.gpu
+
+
+def _graphs(dev, count, m=200, w=4, feat=32):
+    """Matrices of one hyb bucket that differ in their columns only, and their products with x."""
+    g = torch.Generator(device=dev).manual_seed(count)
+    x = torch.randn(m, feat, device=dev, generator=g)
+    rows = torch.arange(m, dtype=torch.int32, device=dev)
+    out = []
+    for _ in range(count):
+        cols = torch.randint(m, (m, w), dtype=torch.int32, device=dev, generator=g)
+        a = torch.rand(m, w, device=dev, generator=g)
+        want = (a.double()[:, :, None] * x.double()[cols.long()]).sum(1)
+        out.append((a.reshape(-1), rows.clone(), cols.reshape(-1), want))
+    return x, out, ops.build_hyb_csrmm(m, m, feat, 1, [w, 2 * w], [m, 0])
+
+
+@pytest.mark.parametrize("count", [1, 2, 8, 9])
+def test_plans_of_several_matrices(dev, count):
+    """Up to eight matrices in turn keep their plans; a ninth evicts the one used longest ago, and a
+    call with that one makes it anew instead of using what was destroyed."""
+    x, mats, f = _graphs(dev, count)
+    z = torch.zeros(0, device=dev)
+    zi = torch.zeros(0, dtype=torch.int32, device=dev)
+    for _ in range(3):
+        for a, r, c, want in mats:
+            y = torch.zeros_like(x)
+            f(x.reshape(-1), y.reshape(-1), a, r, c, z, zi, zi)
+            assert torch.allclose(y.double(), want, rtol=1e-5, atol=1e-5)
+    assert f.plan_builds == (count if count <= 8 else 3 * count)
+
+
+def test_falls_back_to_python(dev):
+    """Arguments the launcher does not take get the same answer, or the same error, as before."""
+    x, mats, f = _graphs(dev, 1)
+    a, r, c, want = mats[0]
+    z, zi = torch.zeros(0, device=dev), torch.zeros(0, dtype=torch.int32, device=dev)
+    y = torch.zeros(x.numel(), device=dev)
+    args = [x.reshape(-1), y, a, r, c, z, zi, zi]
+    f(*args)
+    builds = f.plan_builds
+    with pytest.raises(SparseTIRError, match="shape"):
+        f(x.reshape(-1)[:-1], *args[1:])
+    with pytest.raises(SparseTIRError, match="dtype"):
+        f(args[0].double(), *args[1:])
+    with pytest.raises(SparseTIRError, match="compact"):
+        f(torch.zeros(2 * x.numel(), device=dev)[::2], *args[1:])
+    with pytest.raises(SparseTIRError, match="num_args"):
+        f(*args[:-1])
+    f.invalidate()
+    y.zero_()
+    f(*args)
+    assert f.plan_builds == builds + 1
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):  # the stream that is current when the call is made
+        y2 = torch.zeros_like(y)
+        f(args[0], y2, *args[2:])
+    side.synchronize()
+    for got in (y, y2):
+        assert np.allclose(got.cpu().numpy().reshape(want.shape), want.cpu().numpy(), rtol=1e-5, atol=1e-5)

@@ -161,12 +161,11 @@ __device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int l
 // groups take the nonzeros round-robin; the caller combines the groups.
 // INDIRECT: A is an array of addresses of the values (the merged rows of a hyb plan, whose values
 // stay in the caller's bucket arrays), and nonzeros whose value is 0 -- ELL padding -- fetch no row.
-template <int G, int REP, bool INDIRECT = false>
+template <int G, int REP, bool INDIRECT = false, int UNROLL = 4>
 __device__ __forceinline__ void csr_accumulate(float4 (&acc)[REP], int start, int end, int feat,
                                                const float* __restrict__ A, const float* __restrict__ B,
                                                const int32_t* __restrict__ indices, int lane) {
   constexpr int NG = kWave / G;
-  constexpr int UNROLL = 4;
   const int g = lane / G, gl = lane % G;
   for (int base = start; base < end; base += kWave) {
     const int p = base + lane;
@@ -205,39 +204,106 @@ __device__ __forceinline__ void csr_accumulate(float4 (&acc)[REP], int start, in
 
 // Rows with more nonzeros than this are not left to a single wavefront (a 17k-entry hub row
 // costs one wavefront milliseconds): the row kernel only clears them and csr_long_rows_kernel,
-// launched after it, adds them up in pieces of kLongPiece nonzeros.  64 rather than 256: the
+// launched after it, adds them up in pieces (long_piece()).  64 rather than 256: the
 // piece kernel keeps every lane busy whatever the row, a wavefront on a row of its own does not
 // (169 k-node power-law graph, half of its nonzeros in rows above 256: 46 -> 41 us at 32 features,
 // 223 -> 203 us at 256; 2.45 M-node graph, 128 features: 5.05 -> 5.01 ms; 32 is slower again).
 constexpr int kLongRow = 64;
-constexpr int kLongPiece = 256;
+// Nonzeros per piece: short ones where whole pieces would leave the chip idle or end it on a few
+// (240 k nonzeros, 100 features: 40 / 32 / 31 us with 256 / 128 / 64; 600 k: 59 / 52 / 54; 1.19 M:
+// 106 / 110 / 111).
+inline int long_piece(int64_t nnz) { return nnz < (1 << 18) ? 64 : nnz < (1 << 20) ? 128 : 256; }
 
-// One wavefront per row.  With split_long the rows above kLongRow are zero-filled here.
-template <int G, int REP, bool INDIRECT = false>
-__global__ __launch_bounds__(256) void csr_spmm_kernel(int m, int feat, int split_long,
-                                                       const float* __restrict__ A,
-                                                       const float* __restrict__ B,
-                                                       float* __restrict__ C,
-                                                       const int32_t* __restrict__ indptr,
-                                                       const int32_t* __restrict__ indices) {
+// Small products are one launch: rows above kBlockRow nonzeros are left until the workgroup has done
+// its other rows and takes them together, each wavefront a stretch of the row, the sums meeting in
+// LDS.  Left to one wavefront a row of 1024 nonzeros was 16 round trips to memory one after the other
+// and set the time of a 4096-row launch (70 k nonzeros, 32 features: 17 us, now 7 us).
+// The line lies at nnz * feat because what a compute unit can read sets how long a hub row takes it:
+// 80 k nonzeros with a row of 2000 cost the same either way at 64 features (13.3 us, split 13.9), at
+// 16 features 10.2 us (12.4), at 100 features 21.5 us (19.5).
+constexpr int64_t kSmallProduct = 6000000;
+constexpr int kBlockRow = 128;
+constexpr int kSmallWaves = 8;      // 16 are slower (10 us for the launch above)
+constexpr int kWavePerRow = 20000;  // small products with more rows: a lane group per row
+
+struct BlockRow {
+  int row, start, end;
+};
+
+// The rows of `list` by all WAVES wavefronts of the workgroup; part: WAVES * 4 * G * REP floats.
+template <int G, int REP, int WAVES>
+__device__ __forceinline__ void block_rows(const BlockRow* list, int count, float* part, int feat,
+                                           const float* __restrict__ A, const float* __restrict__ B,
+                                           float* __restrict__ C, const int32_t* __restrict__ indices, int lane,
+                                           int wave) {
+  const int g = lane / G, gl = lane % G;
+  for (int k = 0; k < count; ++k) {
+    const BlockRow b = list[k];
+    const int per = ((b.end - b.start + WAVES - 1) / WAVES + 3) & ~3;
+    const int s = min(b.end, b.start + wave * per), e = min(b.end, s + per);
+    float4 acc[REP];
+#pragma unroll
+    for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+    csr_accumulate<G, REP, false, (G >= 64 ? 4 : 8) / REP>(acc, s, e, feat, A, B, indices, lane);
+    reduce_groups<G, REP>(acc, kWave);
+    if (g == 0)
+#pragma unroll
+      for (int r = 0; r < REP; ++r) *reinterpret_cast<float4*>(part + ((wave * REP + r) * G + gl) * 4) = acc[r];
+    __syncthreads();
+    if (wave == 0 && g == 0) {
+      for (int w = 1; w < WAVES; ++w)
+#pragma unroll
+        for (int r = 0; r < REP; ++r) {
+          const float4 o = *reinterpret_cast<const float4*>(part + ((w * REP + r) * G + gl) * 4);
+          acc[r].x += o.x, acc[r].y += o.y, acc[r].z += o.z, acc[r].w += o.w;
+        }
+      write_row<G, REP>(C, b.row, feat, lane, acc, 0, nullptr);
+    }
+    __syncthreads();
+  }
+}
+
+// One wavefront per row, WAVES rows per workgroup.  With WAVES = 4 the matrix is split: rows above
+// kLongRow are zero-filled here and added by csr_long_rows_kernel.
+template <int G, int REP, int WAVES, bool INDIRECT = false>
+__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat, const float* __restrict__ A,
+                                                                 const float* __restrict__ B,
+                                                                 float* __restrict__ C,
+                                                                 const int32_t* __restrict__ indptr,
+                                                                 const int32_t* __restrict__ indices) {
+  constexpr bool SPLIT = WAVES == 4;
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= m) return;
+  const int wave = threadIdx.x >> 6;
+  const int row = blockIdx.x * WAVES + wave;
   const int g = lane / G;
-  const int start = indptr[row], end = indptr[row + 1];
+  int start = 0, end = 0;
+  if (row < m) start = indptr[row], end = indptr[row + 1];
+  if constexpr (SPLIT) {
+    if (row >= m) return;
+  }
   float4 acc[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (!(split_long && end - start > kLongRow))
-    csr_accumulate<G, REP, INDIRECT>(acc, start, end, feat, A, B, indices, lane);
+  const bool later = end - start > (SPLIT ? kLongRow : kBlockRow);
+  if (!later) csr_accumulate<G, REP, INDIRECT>(acc, start, end, feat, A, B, indices, lane);
   reduce_groups<G, REP>(acc, kWave);
   if constexpr (INDIRECT) {
     // merged rows of a hyb plan: the operator adds to C, as its buckets do; this wavefront is the
     // row's only writer in this launch, long rows are left to csr_long_rows_kernel altogether
-    if (end - start > kLongRow) return;
+    if (later) return;
     if (g == 0) write_row<G, REP>(C, row, feat, lane, acc, 2, nullptr);
-  } else {
+  } else if constexpr (SPLIT) {
     if (g == 0) write_row<G, REP>(C, row, feat, lane, acc, 0, nullptr);
+  } else {
+    __shared__ BlockRow list[WAVES];
+    __shared__ __attribute__((aligned(16))) float part[WAVES * 4 * G * REP];
+    if (row < m && !later && g == 0) write_row<G, REP>(C, row, feat, lane, acc, 0, nullptr);
+    if (!__syncthreads_or(later)) return;
+    if (lane == 0) list[wave] = BlockRow{row, start, end};
+    __syncthreads();
+    for (int w = 0; w < WAVES; ++w)
+      if (list[w].end - list[w].start > kBlockRow)  // uniform
+        block_rows<G, REP, WAVES>(list + w, 1, part, feat, A, B, C, indices, lane, wave);
   }
 }
 
@@ -248,22 +314,23 @@ __global__ __launch_bounds__(256) void csr_spmm_kernel(int m, int feat, int spli
 // row of seven nonzeros at 32 features keeps one lane group in eight busy for one step and still
 // pays the index round trip, the cross-lane sum and the store.  Rows of more than 2 * G nonzeros
 // would hold the other groups up: the wavefront takes those one by one afterwards, all groups
-// sharing the row as in the kernel above (and leaves rows above kLongRow zero-filled for
-// csr_long_rows_kernel when split_long is set).
-template <int G>
-__global__ __launch_bounds__(256) void csr_spmm_rows_kernel(int m, int feat, int split_long,
-                                                            const float* __restrict__ A,
-                                                            const float* __restrict__ B,
-                                                            float* __restrict__ C,
-                                                            const int32_t* __restrict__ indptr,
-                                                            const int32_t* __restrict__ indices) {
+// sharing the row as in the kernel above, up to the length that is left to csr_long_rows_kernel
+// (WAVES = 4, the matrix is split: zero-filled here) or to the workgroup.
+template <int G, int WAVES>
+__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int feat,
+                                                                      const float* __restrict__ A,
+                                                                      const float* __restrict__ B,
+                                                                      float* __restrict__ C,
+                                                                      const int32_t* __restrict__ indptr,
+                                                                      const int32_t* __restrict__ indices) {
+  constexpr bool SPLIT = WAVES == 4;
   constexpr int NG = kWave / G;
   constexpr int CH = G < 8 ? G : 8;  // gathers in flight per lane
   constexpr int kGroupRow = 2 * G;   // longest row a lane group takes alone (1 to 4 * G measure the same)
   const int lane = threadIdx.x & 63;
   const int g = lane / G, gl = lane % G;
-  const int64_t row0 = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * NG;
-  if (row0 >= m) return;
+  const int64_t row0 = ((int64_t)blockIdx.x * WAVES + (threadIdx.x >> 6)) * NG;
+  if (SPLIT && row0 >= m) return;
   const int64_t row = row0 + g;
   int start = 0, end = 0;
   if (row < m) start = indptr[row], end = indptr[row + 1];
@@ -297,23 +364,35 @@ __global__ __launch_bounds__(256) void csr_spmm_rows_kernel(int m, int feat, int
     write_row<G, 1>(C, row, feat, lane, sum, 0, nullptr);
   }
   // the longer rows, one after the other, by the whole wavefront
-  uint64_t todo = __ballot(row < m && !alone && gl == 0);
+  const bool later = end - start > (SPLIT ? kLongRow : kBlockRow);
+  uint64_t todo = __ballot(row < m && !alone && gl == 0 && (SPLIT || !later));
   while (todo) {
     const int src = __ffsll((long long)todo) - 1;
     todo &= todo - 1;
     const int s = __shfl(start, src, kWave), e = __shfl(end, src, kWave);
     float4 sum[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
-    if (!(split_long && e - s > kLongRow)) csr_accumulate<G, 1>(sum, s, e, feat, A, B, indices, lane);
+    if (!(SPLIT && e - s > kLongRow)) csr_accumulate<G, 1>(sum, s, e, feat, A, B, indices, lane);
     reduce_groups<G, 1>(sum, kWave);
     if (g == 0) write_row<G, 1>(C, row0 + src / G, feat, lane, sum, 0, nullptr);
   }
+  if constexpr (!SPLIT) {
+    __shared__ BlockRow list[WAVES * NG];
+    __shared__ int count;
+    __shared__ __attribute__((aligned(16))) float part[WAVES * 4 * G];
+    if (!__syncthreads_or(later)) return;
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    if (later && gl == 0) list[atomicAdd(&count, 1)] = BlockRow{(int)row, start, end};
+    __syncthreads();
+    block_rows<G, 1, WAVES>(list, count, part, feat, A, B, C, indices, lane, threadIdx.x >> 6);
+  }
 }
 
-// One wavefront per kLongPiece consecutive nonzeros: the parts of rows longer than kLongRow that
-// fall into the piece are summed and added to C (cleared by csr_spmm_kernel) with atomics.
+// One wavefront per `piece` consecutive nonzeros: the parts of rows longer than kLongRow that fall
+// into the piece are summed and added to C (cleared by csr_spmm_kernel) with atomics.
 // Pieces that touch no long row -- nearly all of them -- end after looking at their rows.
 template <int G, int REP, bool INDIRECT = false>
-__global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int64_t first, int64_t nnz,
+__global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int64_t nnz, int piece,
                                                             const float* __restrict__ A,
                                                             const float* __restrict__ B,
                                                             float* __restrict__ C,
@@ -322,18 +401,18 @@ __global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int
   __shared__ float stage_all[4][kWave * 4 * REP];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t p0 = first + ((int64_t)blockIdx.x * 4 + wave) * kLongPiece;
-  const int64_t end_all = first + nnz;
-  if (p0 >= end_all) return;
-  const int64_t p1 = min(end_all, p0 + kLongPiece);
+  const int64_t p0 = ((int64_t)blockIdx.x * 4 + wave) * piece;
+  if (p0 >= nnz) return;
+  const int64_t p1 = min(nnz, p0 + piece);
   const int ra = stir::wave_last_row(indptr, m, p0, lane);
-  const int rb = stir::wave_last_row(indptr, m, p1 - 1, lane);
   const int g = lane / G;
-  for (int r0 = ra; r0 <= rb; r0 += kWave) {
+  // 64 rows at a time, until one of them reaches the end of the piece
+  for (int r0 = ra, more = 1; more; r0 += kWave) {
     const int r = r0 + lane;
     int rs = 0, re = 0;
-    if (r <= rb && r < m) rs = indptr[r], re = indptr[r + 1];
-    uint64_t todo = __ballot(re - rs > kLongRow);
+    if (r < m) rs = indptr[r], re = indptr[r + 1];
+    more = !__any(r >= m || re >= p1);
+    uint64_t todo = __ballot(rs < p1 && re - rs > kLongRow);
     while (todo) {
       const int src = __ffsll((long long)todo) - 1;
       todo &= todo - 1;
@@ -862,13 +941,14 @@ int build_merged_rows(int32_t m, int total_buckets, int num_buckets, const int32
 // Launches the CSR row kernels over the merged rows.  feat must have a vector class.
 int launch_merged(const MergedRows& mr, int32_t m, int32_t feat, const float* d_B, float* d_C, hipStream_t st) {
   dim3 grid((unsigned)stir::ceil_div(m, 4)), block(256);
-  dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(mr.slots, kLongPiece), 4));
+  const int piece = long_piece(mr.slots);
+  dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(mr.slots, piece), 4));
   const float* vals = reinterpret_cast<const float*>(mr.vals);
 #define STIR_MERGED(G, REP)                                                                                   \
   {                                                                                                           \
-    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, true>), grid, block, 0, st, m, feat, 1, vals, d_B, d_C,       \
+    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4, true>), grid, block, 0, st, m, feat, vals, d_B, d_C,       \
                        mr.slot_ptr, mr.cols);                                                                 \
-    hipLaunchKernelGGL((csr_long_rows_kernel<G, REP, true>), pieces, block, 0, st, m, feat, (int64_t)0, mr.slots, \
+    hipLaunchKernelGGL((csr_long_rows_kernel<G, REP, true>), pieces, block, 0, st, m, feat, mr.slots, piece,   \
                        vals, d_B, d_C, mr.slot_ptr, mr.cols);                                                 \
   }
   switch (vector_class(feat)) {
@@ -960,30 +1040,43 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
   if (m == 0) return 0;
   STIR_REQUIRE(d_B && d_C && d_indptr && (nnz == 0 || (d_A && d_indices)), "csr_spmm: null pointer argument");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  dim3 grid((unsigned)stir::ceil_div(m, 4)), block(256);
-  // Hub rows are split over many wavefronts by a second launch; a matrix this small cannot hold
-  // a row long enough to matter against the extra launch.
-  const int split_long = nnz >= (int64_t(1) << 18) ? 1 : 0;
-  dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(nnz, kLongPiece), 4));
+  // Hub rows are split over many wavefronts by a second launch, or shared by a workgroup
+  const bool split = nnz * feat >= kSmallProduct;
+  const int waves = split ? 4 : kSmallWaves;
+  dim3 grid((unsigned)stir::ceil_div(m, waves)), block(waves * kWave);
+  const int piece = long_piece(nnz);
+  dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(nnz, piece), 4));
+#define STIR_CSR_LONG(G, REP)                                                                              \
+  hipLaunchKernelGGL((csr_long_rows_kernel<G, REP>), pieces, dim3(256), 0, st, m, feat, nnz, piece, d_A, d_B, d_C, \
+                     d_indptr, d_indices)
+  // one wavefront per row
 #define STIR_CSR(G, REP)                                                                                   \
   {                                                                                                        \
-    hipLaunchKernelGGL((csr_spmm_kernel<G, REP>), grid, block, 0, st, m, feat, split_long, d_A, d_B, d_C,  \
-                       d_indptr, d_indices);                                                               \
-    if (split_long)                                                                                        \
-      hipLaunchKernelGGL((csr_long_rows_kernel<G, REP>), pieces, block, 0, st, m, feat, (int64_t)0, nnz, d_A,   \
-                         d_B, d_C, d_indptr, d_indices);                                                   \
+    if (split) {                                                                                           \
+      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4>), grid, block, 0, st, m, feat, d_A, d_B, d_C, d_indptr, \
+                         d_indices);                                                                       \
+      STIR_CSR_LONG(G, REP);                                                                               \
+    } else {                                                                                               \
+      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, kSmallWaves>), grid, block, 0, st, m, feat, d_A, d_B, d_C, \
+                         d_indptr, d_indices);                                                             \
+    }                                                                                                      \
   }
-  // the smallest lane group that covers the feature width (lanes beyond feat / 4 idle)
   // lane groups narrower than the wavefront: a lane group per row (csr_spmm_rows_kernel)
 #define STIR_CSR_ROWS(G)                                                                                   \
   {                                                                                                        \
-    const dim3 row_grid((unsigned)stir::ceil_div(m, 4 * (kWave / G)));                                     \
-    hipLaunchKernelGGL((csr_spmm_rows_kernel<G>), row_grid, block, 0, st, m, feat, split_long, d_A, d_B,   \
-                       d_C, d_indptr, d_indices);                                                          \
-    if (split_long)                                                                                        \
-      hipLaunchKernelGGL((csr_long_rows_kernel<G, 1>), pieces, block, 0, st, m, feat, (int64_t)0, nnz, d_A, \
-                         d_B, d_C, d_indptr, d_indices);                                                   \
+    const dim3 row_grid((unsigned)stir::ceil_div(m, waves * (kWave / G)));                                 \
+    if (split) {                                                                                           \
+      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, 4>), row_grid, block, 0, st, m, feat, d_A, d_B, d_C,     \
+                         d_indptr, d_indices);                                                             \
+      STIR_CSR_LONG(G, 1);                                                                                 \
+    } else if (m <= kWavePerRow) {                                                                         \
+      STIR_CSR(G, 1)                                                                                       \
+    } else {                                                                                               \
+      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, kSmallWaves>), row_grid, block, 0, st, m, feat, d_A, d_B, d_C, \
+                         d_indptr, d_indices);                                                             \
+    }                                                                                                      \
   }
+  // the smallest lane group that covers the feature width (lanes beyond feat / 4 idle)
   switch (vector_class(feat)) {
     case 0: STIR_CSR_ROWS(4); break;
     case 1: STIR_CSR_ROWS(8); break;
@@ -996,10 +1089,12 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
     case 4: STIR_CSR(64, 1); break;
     case 5: STIR_CSR(64, 2); break;
     default:
-      hipLaunchKernelGGL(csr_spmm_generic_kernel, grid, block, 0, st, m, feat, d_A, d_B, d_C, d_indptr, d_indices);
+      hipLaunchKernelGGL(csr_spmm_generic_kernel, dim3((unsigned)stir::ceil_div(m, 4)), dim3(256), 0, st, m, feat, d_A,
+                         d_B, d_C, d_indptr, d_indices);
   }
 #undef STIR_CSR_ROWS
 #undef STIR_CSR
+#undef STIR_CSR_LONG
   STIR_LAUNCH_CHECK();
   return 0;
 }

@@ -120,6 +120,21 @@ int stir_column_part_hyb_device_values(int32_t num_rows, int32_t num_cols, const
                                        float* const* d_A, void* stream);
 
 /*
+ * The same pass for one column partition and at most 32 buckets, shorter where the matrix is small
+ * (a fresh matrix per mini-batch): max_nnz is the length of d_indices, checked against d_indptr on
+ * the device; _sizes synchronises the stream once, _fill does not, and with d_values / d_A (both or
+ * neither null) it writes the value arrays too.  Same workspace size as above, untouched in between.
+ */
+int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr,
+                                   const int32_t* d_indices, int64_t max_nnz, const int32_t* buckets,
+                                   int32_t num_buckets, void* d_workspace, int64_t* nrows, void* stream);
+int stir_column_part_hyb_one_fill(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr,
+                                  const int32_t* d_indices, int64_t max_nnz, const float* d_values,
+                                  int32_t num_buckets, void* d_workspace, int32_t* const* d_row_indices,
+                                  int32_t* const* d_col_indices, int32_t* const* d_mask, float* const* d_A,
+                                  void* stream);
+
+/*
  * CSFToELL3D on the GPU, bit-exact with stir_csf_to_ell3d_sizes / _fill above (the reference runs
  * this on the CPU only, src/sparse/format.cc:195-202).  num_stored_rows is the length of
  * csf_indices_0, nnz that of csf_indices_1.  The row ids of every relation must ascend strictly

@@ -29,6 +29,8 @@ SIGNATURES = {
     "stir_column_part_hyb_device_sizes": (I32, [I32, I32, VP, VP, I32, VP, I32, VP, VP, VP]),
     "stir_column_part_hyb_device_fill": (I32, [I32, I32, VP, VP, I32, VP, I32, VP, VP, VP, VP, VP]),
     "stir_column_part_hyb_device_values": (I32, [I32, I32, VP, VP, VP, I32, VP, I32, VP, VP, VP, VP]),
+    "stir_column_part_hyb_one_sizes": (I32, [I32, I32, VP, VP, I64, VP, I32, VP, VP, VP]),
+    "stir_column_part_hyb_one_fill": (I32, [I32, I32, VP, VP, I64, VP, I32, VP, VP, VP, VP, VP, VP]),
     "stir_csf_to_ell3d_device_workspace_bytes": (SZ, [I32, I64, I32]),
     "stir_csf_to_ell3d_device_sizes": (I32, [I32, I64, I64, VP, VP, VP, VP, VP, VP, I32, VP, VP, VP]),
     "stir_csf_to_ell3d_device_fill": (I32, [I32, I64, I64, VP, VP, VP, VP, VP, VP, I32, VP, VP, VP, VP, VP, VP, VP]),

@@ -9,8 +9,14 @@
 // tensor of the expected type and length on the current device and, for operators with plans, the
 // arrays those of a plan it was told of (same addresses, same torch version counters).  Anything else
 // is left to the Python code, which words the errors, makes the plans and keeps them.
+//
+// column_part_hyb() is the decomposition of one column partition for tensors on the current device: its
+// launches, its one wait and the tensors it returns (40 of them with ten buckets and values, 3 us each
+// when sliced and reshaped from Python).
+#define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/ops/empty.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -193,6 +199,47 @@ PyObject* forget(PyObject* self, PyObject* name) {
   Py_RETURN_NONE;
 }
 
+// new_hyb_plan(args) -> (name, plan) for arguments launch() did not know, None when they are not the
+// ordinary ones, -1 when the C ABI refused.  The name is the properties the plan depends on.
+PyObject* new_hyb_plan(PyObject* self, PyObject* args) {
+  Launcher* l = reinterpret_cast<Launcher*>(self);
+  stir_hyb_plan* plan = nullptr;
+  try {
+    if (l->kind != kHyb) Py_RETURN_NONE;
+    const int64_t device = c10::hip::current_device();
+    void* p[kPassed];
+    std::vector<int64_t>& key = *l->key;
+    key.assign(1, device);
+    if (!walk(l, args, (int)device, p, [&](int64_t v) { return key.push_back(v), true; })) Py_RETURN_NONE;
+    // key: device, then per bucket the address of A, address and version of rows, of cols
+    const size_t nk = (l->operands->size() - 2) / 3;
+    const std::vector<int64_t>& n = *l->sizes;  // feat, m, n, parts, widths ...
+    const size_t nb = n.size() - 4;
+    std::vector<int32_t> widths(n.begin() + 4, n.end());
+    std::vector<int64_t> nrows(nk + 1);
+    std::vector<const float*> A(nk + 1);
+    std::vector<const int32_t*> rows(nk + 1), cols(nk + 1);
+    for (size_t k = 0; k < nk; ++k) {
+      const int64_t* q = key.data() + 1 + 5 * k;
+      A[k] = reinterpret_cast<const float*>(q[0]);
+      rows[k] = reinterpret_cast<const int32_t*>(q[1]);
+      cols[k] = reinterpret_cast<const int32_t*>(q[3]);
+      nrows[k] = (*l->operands)[2 + 3 * k + 1].length;
+    }
+    if (nb == 0 || nk != nb * (size_t)n[3]) Py_RETURN_NONE;
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = stir_hyb_plan_create(&plan, (int32_t)n[1], (int32_t)n[2], (int32_t)n[3], (int32_t)nb, widths.data(),
+                              nrows.data(), A.data(), rows.data(), cols.data());
+    Py_END_ALLOW_THREADS
+    if (rc != 0) return PyLong_FromLong(kFailed);
+  } catch (...) {
+    Py_RETURN_NONE;
+  }
+  return Py_BuildValue("(y#K)", reinterpret_cast<const char*>(l->key->data()),
+                       (Py_ssize_t)(l->key->size() * sizeof(int64_t)), reinterpret_cast<unsigned long long>(plan));
+}
+
 bool scalar_type(long code, c10::ScalarType* out) {
   switch (code) {
     case 0: *out = c10::ScalarType::Half; return true;
@@ -230,12 +277,12 @@ bool ints_of(PyObject* o, std::vector<int64_t>* out) {
   return !PyErr_Occurred();
 }
 
-// Launcher.hyb(n, m, feat, buckets, nrows): the operands of the hyb operator, B and C followed by
+// Launcher.hyb(n, m, feat, parts, buckets, nrows): the operands of the hyb operator, B and C followed by
 // (A_k, rows_k, cols_k) of every bucket of every partition
 PyObject* launcher_hyb(PyObject*, PyObject* args) {
-  long long n, m, feat;
+  long long n, m, feat, parts;
   PyObject *buckets, *nrows;
-  if (!PyArg_ParseTuple(args, "LLLOO", &n, &m, &feat, &buckets, &nrows)) return nullptr;
+  if (!PyArg_ParseTuple(args, "LLLLOO", &n, &m, &feat, &parts, &buckets, &nrows)) return nullptr;
   std::vector<int64_t> w, r;
   if (!ints_of(buckets, &w) || !ints_of(nrows, &r)) return nullptr;
   if (w.empty() && !r.empty()) {
@@ -244,7 +291,8 @@ PyObject* launcher_hyb(PyObject*, PyObject* args) {
   }
   Launcher* l = make(kHyb);
   if (!l) return nullptr;
-  l->sizes->push_back(feat);
+  *l->sizes = {feat, m, n, parts};
+  l->sizes->insert(l->sizes->end(), w.begin(), w.end());
   l->operands->push_back({c10::ScalarType::Float, n * feat, 0});
   l->operands->push_back({c10::ScalarType::Float, m * feat, 0});
   for (size_t k = 0; k < r.size(); ++k) {
@@ -301,11 +349,118 @@ void launcher_dealloc(PyObject* self) {
 PyMethodDef launcher_methods[] = {
     {"launch", launch, METH_O, "launch(args) -> 0: launched, -1: refused, 1: not taken, or the name of the plan"},
     {"remember", remember, METH_VARARGS, "remember(args, plan, name): a plan made from these arguments"},
+    {"new_hyb_plan", new_hyb_plan, METH_O, "new_hyb_plan(args) -> (name, plan), None: not taken, -1: refused"},
     {"forget", forget, METH_O, "forget(name): the plan is no more; None: all of them"},
-    {"hyb", launcher_hyb, METH_VARARGS | METH_STATIC, "hyb(n, m, feat, buckets, nrows): launcher of the hyb operator"},
+    {"hyb", launcher_hyb, METH_VARARGS | METH_STATIC, "hyb(n, m, feat, parts, buckets, nrows): launcher of the hyb operator"},
     {nullptr, nullptr, 0, nullptr}};
 
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "host path of the operators", -1, nullptr};
+// ---- decomposition
+
+// A tensor over `sizes` elements of the pool from `offset` on.
+PyObject* piece(const at::Tensor& pool, int64_t offset, c10::IntArrayRef sizes) {
+  at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(pool.storage()), pool.key_set(), pool.dtype());
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+  t.unsafeGetTensorImpl()->set_storage_offset(offset);
+  return THPVariable_Wrap(std::move(t));
+}
+
+// Appends the buckets' pieces of a pool to `list` (256-byte aligned pieces, as their addresses say).
+bool append_pieces(PyObject* list, const at::Tensor& pool, const std::vector<int64_t>& offsets,
+                   const std::vector<int64_t>& nrows, const std::vector<int64_t>* widths) {
+  for (size_t k = 0; k < nrows.size(); ++k) {
+    const int64_t both[2] = {nrows[k], widths ? (*widths)[k] : 0};
+    PyObject* t = piece(pool, offsets[k], c10::IntArrayRef(both, widths ? 2 : 1));
+    if (!t || PyList_Append(list, t) < 0) {
+      Py_XDECREF(t);
+      return false;
+    }
+    Py_DECREF(t);
+  }
+  return true;
+}
+
+// column_part_hyb(num_rows, num_cols, indptr, indices, buckets, values or None) for one column partition
+// -> (rows, cols, mask, values) lists over the buckets, values None without; None: not taken; -1: refused
+PyObject* column_part_hyb(PyObject*, PyObject* args) {
+  int m, n;
+  PyObject *o_ptr, *o_idx, *o_buckets, *o_values;
+  if (!PyArg_ParseTuple(args, "iiOOOO", &m, &n, &o_ptr, &o_idx, &o_buckets, &o_values)) return nullptr;
+  std::vector<int64_t> widths;
+  if (!ints_of(o_buckets, &widths)) return nullptr;
+  PyObject* lists[4] = {nullptr, nullptr, nullptr, nullptr};
+  bool ok = true;
+  try {
+    const int device = (int)c10::hip::current_device();
+    const size_t nb = widths.size();
+    if (m < 0 || nb == 0 || nb > 32 || !THPVariable_Check(o_idx)) Py_RETURN_NONE;
+    const int64_t nnz = THPVariable_Unpack(o_idx).numel();
+    const at::Tensor* ptr = take(o_ptr, {c10::ScalarType::Int, (int64_t)m + 1, 0}, device);
+    const at::Tensor* idx = take(o_idx, {c10::ScalarType::Int, nnz, 0}, device);
+    const bool with_values = o_values != Py_None;
+    const at::Tensor* val = with_values ? take(o_values, {c10::ScalarType::Float, nnz, 0}, device) : nullptr;
+    if (!ptr || !idx || (with_values && !val)) Py_RETURN_NONE;
+    void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    const int32_t* d_ptr = static_cast<const int32_t*>(ptr->data_ptr());
+    const int32_t* d_idx = static_cast<const int32_t*>(idx->data_ptr());
+    const float* d_val = val ? static_cast<const float*>(val->data_ptr()) : nullptr;
+    std::vector<int32_t> w32(widths.begin(), widths.end());
+    std::vector<int64_t> nrows(nb), row_at(nb), slot_at(nb);
+    const at::TensorOptions on = ptr->options();
+    const int64_t ws_bytes = (int64_t)stir_column_part_hyb_device_workspace_bytes(m, 1, (int32_t)nb, nnz);
+    // freed to the allocator of this stream when the call returns: what uses it next runs after the
+    // kernels below
+    const at::Tensor ws = at::empty({std::max<int64_t>(ws_bytes, 256)}, on.dtype(c10::ScalarType::Byte));
+    int rc;
+    Py_BEGIN_ALLOW_THREADS
+    rc = stir_column_part_hyb_one_sizes(m, n, d_ptr, d_idx, nnz, w32.data(), (int32_t)nb, ws.data_ptr(), nrows.data(), st);
+    Py_END_ALLOW_THREADS
+    if (rc != 0) return PyLong_FromLong(kFailed);
+    int64_t rows = 0, slots = 0;
+    for (size_t k = 0; k < nb; ++k) {
+      row_at[k] = rows, slot_at[k] = slots;
+      rows += (nrows[k] + 63) / 64 * 64;
+      slots += (nrows[k] * widths[k] + 63) / 64 * 64;
+    }
+    const at::Tensor pool_rows = at::empty({std::max<int64_t>(rows, 1)}, on);
+    const at::Tensor pool_cols = at::empty({std::max<int64_t>(slots, 1)}, on);
+    const at::Tensor pool_mask = at::empty({std::max<int64_t>(slots, 1)}, on);
+    const at::Tensor pool_vals =
+        val ? at::empty({std::max<int64_t>(slots, 1)}, on.dtype(c10::ScalarType::Float)) : at::Tensor();
+    std::vector<int32_t*> r(nb), c(nb), k01(nb);
+    std::vector<float*> a(nb);
+    for (size_t k = 0; k < nb; ++k) {
+      r[k] = static_cast<int32_t*>(pool_rows.data_ptr()) + row_at[k];
+      c[k] = static_cast<int32_t*>(pool_cols.data_ptr()) + slot_at[k];
+      k01[k] = static_cast<int32_t*>(pool_mask.data_ptr()) + slot_at[k];
+      if (val) a[k] = static_cast<float*>(pool_vals.data_ptr()) + slot_at[k];
+    }
+    rc = stir_column_part_hyb_one_fill(m, n, d_ptr, d_idx, nnz, d_val, (int32_t)nb, ws.data_ptr(), r.data(), c.data(),
+                                       k01.data(), val ? a.data() : nullptr, st);
+    if (rc != 0) return PyLong_FromLong(kFailed);
+    for (PyObject*& list : lists) ok = (list = PyList_New(0)) != nullptr && ok;
+    ok = ok && append_pieces(lists[0], pool_rows, row_at, nrows, nullptr) &&
+         append_pieces(lists[1], pool_cols, slot_at, nrows, &widths) &&
+         append_pieces(lists[2], pool_mask, slot_at, nrows, &widths) &&
+         (!val || append_pieces(lists[3], pool_vals, slot_at, nrows, &widths));
+    if (ok && !val) {
+      Py_INCREF(Py_None);
+      Py_SETREF(lists[3], Py_None);
+    }
+  } catch (const std::exception& e) {  // out of memory, in torch's words
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
+    ok = false;
+  }
+  PyObject* out = ok ? PyTuple_Pack(4, lists[0], lists[1], lists[2], lists[3]) : nullptr;
+  for (PyObject* list : lists) Py_XDECREF(list);
+  return out;
+}
+
+PyMethodDef module_methods[] = {
+    {"column_part_hyb", column_part_hyb, METH_VARARGS,
+     "column_part_hyb(num_rows, num_cols, indptr, indices, buckets, values) -> (rows, cols, mask, values)"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "host path of the operators", -1, module_methods};
 
 }  // namespace
 

@@ -561,8 +561,21 @@ __device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int
   if (g == 0) write_row<G, REP>(C, bk.rows[row], feat, lane, acc, bk.atomic, stage);
 }
 
-__device__ __forceinline__ int find_bucket(const HybBucket* __restrict__ table, int nb,
-                                           int64_t tile) {
+// The descriptors of a launch: a table in device memory, or, up to kInlineBuckets of them, the kernel
+// argument itself.  A plan of that size needs no device memory at all, so making, using and dropping it
+// costs a mini-batch neither an allocation nor a copy nor the wait of hipFree.
+constexpr int kInlineBuckets = 32;
+struct HybInline {
+  HybBucket b[kInlineBuckets];
+  __device__ __forceinline__ const HybBucket& operator[](int k) const { return b[k]; }
+};
+struct HybTable {
+  const HybBucket* b;
+  __device__ __forceinline__ const HybBucket& operator[](int k) const { return b[k]; }
+};
+
+template <class TABLE>
+__device__ __forceinline__ int find_bucket(const TABLE& table, int nb, int64_t tile) {
   int lo = 0, hi = nb - 1;  // largest k with tile_begin[k] <= tile
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
@@ -574,8 +587,8 @@ __device__ __forceinline__ int find_bucket(const HybBucket* __restrict__ table, 
   return lo;
 }
 
-template <int G, int REP>
-__global__ __launch_bounds__(256) void hyb_spmm_kernel(const HybBucket* __restrict__ table, int nb,
+template <int G, int REP, class TABLE>
+__global__ __launch_bounds__(256) void hyb_spmm_kernel(const TABLE table, int nb,
                                                        int64_t tile_base, int64_t tile_end, int feat,
                                                        const float* __restrict__ B,
                                                        float* __restrict__ C) {
@@ -601,12 +614,12 @@ __global__ __launch_bounds__(256) void hyb_spmm_kernel(const HybBucket* __restri
 }
 
 // Widths without a vector class: one wavefront per ELL row, lane l owns features l, l+64, ...
-__global__ __launch_bounds__(256) void hyb_spmm_generic_kernel(const HybBucket* __restrict__ table,
-                                                               int nb, int64_t total_rows, int feat,
+template <class TABLE>
+__global__ __launch_bounds__(256) void hyb_spmm_generic_kernel(const TABLE table, int nb, int64_t total_rows, int feat,
                                                                const float* __restrict__ B,
                                                                float* __restrict__ C) {
   const int lane = threadIdx.x & 63;
-  const int64_t tile = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t tile = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (tile >= total_rows) return;
   const int k = find_bucket(table, nb, tile);
   const HybBucket bk = table[k];
@@ -965,7 +978,14 @@ int launch_merged(const MergedRows& mr, int32_t m, int32_t feat, const float* d_
   return 0;
 }
 
-// Launches the kernels of a hyb operator whose descriptor tables are at d_tiles / d_rows.
+HybInline inline_table(const HybBucket* first, int count) {
+  HybInline t = {};
+  std::copy(first, first + count, t.b);
+  return t;
+}
+
+// Launches the kernels of a hyb operator whose descriptor tables are at d_tiles / d_rows (null: handed
+// over as kernel arguments, at most kInlineBuckets).
 int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_rows, int32_t feat,
                const float* d_B, float* d_C, hipStream_t st) {
   const int nk = (int)t.tiles.size();
@@ -977,9 +997,14 @@ int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_
   for (size_t ph = 0; ph + 1 < t.phase_bucket.size(); ++ph) {                                               \
     const int64_t t0 = t.phase_tile[ph], t1 = t.phase_tile[ph + 1];                                          \
     if (t1 == t0) continue;                                                                                 \
-    hipLaunchKernelGGL((hyb_spmm_kernel<G, REP>), dim3((unsigned)stir::ceil_div(t1 - t0, 4)), block, 0, st,  \
-                       d_tiles + t.phase_bucket[ph], t.phase_bucket[ph + 1] - t.phase_bucket[ph], t0, t1,   \
-                       feat, d_B, d_C);                                                                     \
+    const int b0 = t.phase_bucket[ph], count = t.phase_bucket[ph + 1] - b0;                                  \
+    const dim3 grid((unsigned)stir::ceil_div(t1 - t0, 4));                                                  \
+    if (d_tiles)                                                                                            \
+      hipLaunchKernelGGL((hyb_spmm_kernel<G, REP, HybTable>), grid, block, 0, st, HybTable{d_tiles + b0},    \
+                         count, t0, t1, feat, d_B, d_C);                                                    \
+    else                                                                                                    \
+      hipLaunchKernelGGL((hyb_spmm_kernel<G, REP, HybInline>), grid, block, 0, st,                           \
+                         inline_table(t.tiles.data() + b0, count), count, t0, t1, feat, d_B, d_C);          \
   }
   switch (vector_class(feat)) {
     case 0: STIR_HYB(4, 1); break;
@@ -991,8 +1016,12 @@ int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_
     default: {
       const int64_t rb = stir::ceil_div(t.total_rows, 4);
       STIR_REQUIRE(rb < (int64_t(1) << 31), "hyb_spmm: %lld rows exceed one launch", (long long)t.total_rows);
-      hipLaunchKernelGGL(hyb_spmm_generic_kernel, dim3((unsigned)rb), block, 0, st, d_rows, nk, t.total_rows,
-                         feat, d_B, d_C);
+      if (d_rows)
+        hipLaunchKernelGGL(hyb_spmm_generic_kernel<HybTable>, dim3((unsigned)rb), block, 0, st, HybTable{d_rows}, nk,
+                           t.total_rows, feat, d_B, d_C);
+      else
+        hipLaunchKernelGGL(hyb_spmm_generic_kernel<HybInline>, dim3((unsigned)rb), block, 0, st,
+                           inline_table(t.rows.data(), nk), nk, t.total_rows, feat, d_B, d_C);
     }
   }
 #undef STIR_HYB
@@ -1026,7 +1055,7 @@ struct stir_hyb_plan {
   int32_t m, n, num_col_parts, num_buckets;
   int device;
   HybTables tables;
-  HybBucket* d_tables;  // tables.tiles followed by tables.rows
+  HybBucket* d_tables;  // tables.tiles followed by tables.rows; null up to kInlineBuckets buckets with rows
   bool merged;          // more partitions than run as phases: launches go over `rows`
   MergedRows rows;
 };
@@ -1142,7 +1171,7 @@ int stir_hyb_plan_create_ex(stir_hyb_plan** plan, int32_t m, int32_t n, int32_t 
   make_hyb_tables(num_col_parts, num_buckets, bucket_widths, nrows, d_A, d_rows, d_cols, phased, &p->tables);
   const size_t nk = p->tables.tiles.size();
   hipError_t e = hipGetDevice(&p->device);
-  if (e == hipSuccess && nk > 0) {
+  if (e == hipSuccess && nk > kInlineBuckets) {
     e = hipMalloc(reinterpret_cast<void**>(&p->d_tables), sizeof(HybBucket) * 2 * nk);
     if (e == hipSuccess)
       e = hipMemcpy(p->d_tables, p->tables.tiles.data(), sizeof(HybBucket) * nk, hipMemcpyHostToDevice);
@@ -1168,8 +1197,8 @@ int stir_hyb_spmm_f32(const stir_hyb_plan* plan, int32_t feat, const float* d_B,
   STIR_REQUIRE(d_B && d_C, "hyb_spmm: null pointer argument");
   if (plan->merged && vector_class(feat) >= 0 && (plan->num_col_parts > kMaxPhases || feat >= kMergedFromFeat))
     return launch_merged(plan->rows, plan->m, feat, d_B, d_C, static_cast<hipStream_t>(stream));
-  return launch_hyb(plan->tables, plan->d_tables, plan->d_tables + nk, feat, d_B, d_C,
-                    static_cast<hipStream_t>(stream));
+  const HybBucket* d_rows = plan->d_tables ? plan->d_tables + nk : nullptr;
+  return launch_hyb(plan->tables, plan->d_tables, d_rows, feat, d_B, d_C, static_cast<hipStream_t>(stream));
 }
 
 int stir_hyb_spmm_f32_noalloc(int32_t m, int32_t n, int32_t num_col_parts, int32_t num_buckets,
@@ -1190,9 +1219,10 @@ int stir_hyb_spmm_f32_noalloc(int32_t m, int32_t n, int32_t num_col_parts, int32
   STIR_REQUIRE(nk <= kStaticBuckets, "hyb_spmm_noalloc: %d non-empty buckets, at most %d are supported", nk,
                kStaticBuckets);
   STIR_REQUIRE(d_B && d_C, "hyb_spmm_noalloc: null pointer argument");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (nk <= kInlineBuckets) return launch_hyb(tables, nullptr, nullptr, feat, d_B, d_C, st);
   HybBucket* d_tables = nullptr;
   if (static_scratch(&d_tables) != 0) return -1;
-  hipStream_t st = static_cast<hipStream_t>(stream);
   // only the table the kernel for this feature width reads is written
   const bool generic = vector_class(feat) < 0;
   const std::vector<HybBucket>& src = generic ? tables.rows : tables.tiles;

@@ -89,6 +89,14 @@ def _column_part_hyb_device(num_rows, num_cols, indptr, indices, num_col_parts, 
     if indptr.shape[0] != num_rows + 1:
         raise _lib.SparseTIRError("ColumnPartHyb: indptr must have num_rows + 1 entries")
     dev = indptr.device
+    if num_col_parts == 1:
+        from . import _host
+
+        out = _host.column_part_hyb(num_rows, num_cols, indptr, indices, buckets, values)
+        if out == -1:
+            _lib.check(out)
+        if out is not None:
+            return tuple([lists] for lists in out if lists is not None)
     widths = np.ascontiguousarray(np.asarray(list(buckets), dtype=np.int32))
     nb = len(widths)
     nk = num_col_parts * nb

@@ -220,7 +220,7 @@ class HybCsrMM(_Operator):
         if len(self.nrows) != self.parts * len(self.buckets):
             raise _lib.SparseTIRError("hyb_csrmm: nrows must have num_col_parts*len(buckets) entries")
         self.L = _lib.lib()
-        self._host = _host.Launcher.hyb(self.n, self.m, self.feat, self.buckets, self.nrows)
+        self._host = _host.Launcher.hyb(self.n, self.m, self.feat, self.parts, self.buckets, self.nrows)
         self._launch = self._host.launch
         self._plans = _PlanCache(self.L.stir_hyb_plan_destroy, self._host.forget)
         self._spec_cache = None
@@ -250,6 +250,15 @@ class HybCsrMM(_Operator):
             pass
 
     def _call(self, *args):
+        made = self._host.new_hyb_plan(args)
+        if made is not None:
+            if made == -1:
+                _lib.check(made)
+            name, plan = made
+            self._plans.put(name, ctypes.c_void_p(plan), args[2:])  # the plan stores pointers into these arrays
+            self._host.remember(args, plan, name)
+            _lib.check(self._launch(args))
+            return
         if self._spec_cache is None:
             self._spec_cache = self._spec()
         dev = self._check(args, self._spec_cache)

@@ -212,6 +212,18 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
                       const int32_t* d_indices, void* stream);
 
 /*
+ * The same product by workgroups of equal work, for callers that keep a workspace: device memory of
+ * stir_csr_spmm_workspace_bytes() bytes, aligned to 16, that holds zeros before the first call and is
+ * left to this operator (same m, feat and nnz) between calls.  Calls that may overlap in time need
+ * workspaces of their own; the same bits come out every time.  0 bytes: no workspace is needed, it may
+ * be null and the call is stir_csr_spmm_f32.
+ */
+size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t feat, int64_t nnz);
+int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A,
+                                const float* d_B, float* d_C, const int32_t* d_indptr,
+                                const int32_t* d_indices, void* d_workspace, void* stream);
+
+/*
  * hyb SpMM fp32: all ELL buckets of all column partitions in one launch.
  * The reference specialises and builds one fused kernel per (graph, bucket list)
  * (examples/spmm/bench_spmm.py:116-199); the plan is that built object.  Bucket k =

@@ -17,7 +17,9 @@
 #include <Python.h>
 
 #include <ATen/ops/empty.h>
+#include <ATen/ops/zeros.h>
 #include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -47,6 +49,13 @@ struct Plan {
   PyObject* name;
 };
 
+// Zeroed once, then left to the calls on one stream, which run one after the other
+struct Workspace {
+  c10::hip::HIPStream stream;
+  at::Tensor memory;
+};
+constexpr size_t kWorkspaces = 4;  // streams an operator keeps one for
+
 struct Launcher {
   PyObject_HEAD
   Kind kind;
@@ -54,6 +63,8 @@ struct Launcher {
   std::vector<Operand>* operands;
   std::vector<Plan>* plans;     // as many as the operator keeps, the one used last in front
   std::vector<int64_t>* key;    // of the call in hand (filled and read under the GIL)
+  size_t workspace_bytes;       // of a call (CSR SpMM)
+  std::vector<Workspace>* workspaces;  // one per stream the operator runs on, the one used last in front
 };
 
 // The tensor behind `o` when it is what the operand wants, else null.
@@ -68,13 +79,34 @@ const at::Tensor* take(PyObject* o, const Operand& want, int device) {
 
 int64_t version_of(const at::Tensor& t) { return (int64_t)t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
-int call(const Launcher* l, void* const* p, void* plan, void* st) {
+// The workspace of a call on `st`.  A call that is being captured gets one of its own, cleared by the
+// graph itself: the graph may be replayed on any stream.  `held` keeps it until the call is recorded.
+void* workspace(Launcher* l, const c10::hip::HIPStream& st, at::Tensor* held) {
+  std::vector<Workspace>& all = *l->workspaces;
+  if (!all.empty() && all.front().stream == st && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
+    return all.front().memory.data_ptr();
+  const at::TensorOptions on = at::TensorOptions(c10::ScalarType::Byte).device(c10::DeviceType::CUDA, st.device_index());
+  if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
+    *held = at::zeros({(int64_t)l->workspace_bytes}, on);
+    return held->data_ptr();
+  }
+  size_t at = 0;
+  while (at < all.size() && all[at].stream != st) ++at;
+  if (at == all.size()) {
+    if (at == kWorkspaces) all.pop_back(), --at;  // back to the allocator of its stream
+    all.push_back({st, at::zeros({(int64_t)l->workspace_bytes}, on)});
+  }
+  std::rotate(all.begin(), all.begin() + at, all.begin() + at + 1);
+  return all.front().memory.data_ptr();
+}
+
+int call(const Launcher* l, void* const* p, void* plan, void* ws, void* st) {
   const std::vector<int64_t>& n = *l->sizes;
   auto i = [&](int k) { return (int32_t)n[k]; };
   auto f = [&](int k) { return static_cast<float*>(p[k]); };
   auto x = [&](int k) { return static_cast<int32_t*>(p[k]); };
   switch (l->kind) {
-    case kCsr: return stir_csr_spmm_f32(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), st);
+    case kCsr: return stir_csr_spmm_f32_workspace(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), ws, st);
     case kSddmmPreproc: return stir_sddmm_preproc(i(0), n[3], x(3), x(5), st);
     case kSddmm: return stir_sddmm_f32(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), x(5), st);
     case kSddmmScaled:
@@ -151,9 +183,12 @@ PyObject* launch(PyObject* self, PyObject* args) {
     } else if (!walk(l, args, device, p, [](int64_t) { return true; })) {
       return PyLong_FromLong(kNotTaken);
     }
-    void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device);
+    at::Tensor held;
+    void* ws = l->workspace_bytes ? workspace(l, stream, &held) : nullptr;
+    void* st = stream.stream();
     Py_BEGIN_ALLOW_THREADS  // a launch waits when the queue is full
-    rc = call(l, p, plan, st);
+    rc = call(l, p, plan, ws, st);
     Py_END_ALLOW_THREADS
   } catch (...) {  // a tensor without storage: the Python code says what is wrong with it
     rc = kNotTaken;
@@ -261,7 +296,8 @@ Launcher* make(Kind kind) {
   l->operands = new (std::nothrow) std::vector<Operand>();
   l->plans = new (std::nothrow) std::vector<Plan>();
   l->key = new (std::nothrow) std::vector<int64_t>();
-  if (l->sizes && l->operands && l->plans && l->key) return l;
+  l->workspaces = new (std::nothrow) std::vector<Workspace>();
+  if (l->sizes && l->operands && l->plans && l->key && l->workspaces) return l;
   Py_DECREF(l);
   PyErr_NoMemory();
   return nullptr;
@@ -333,6 +369,10 @@ PyObject* launcher_new(PyTypeObject*, PyObject* args, PyObject*) {
     Py_DECREF(l);
     return nullptr;
   }
+  if (l->kind == kCsr && l->sizes->size() == 4) {
+    const std::vector<int64_t>& n = *l->sizes;
+    l->workspace_bytes = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[2], n[3]);
+  }
   return reinterpret_cast<PyObject*>(l);
 }
 
@@ -343,6 +383,7 @@ void launcher_dealloc(PyObject* self) {
   if (l->plans) drop(l, nullptr);
   delete l->plans;
   delete l->key;
+  delete l->workspaces;
   Py_TYPE(self)->tp_free(self);
 }
 

@@ -1,0 +1,331 @@
+// CSR SpMM fp32 in one launch whose workgroups do equal work whatever the row lengths.
+//
+// The rows and the nonzeros are one list -- every row's mark, followed by its nonzeros -- and a workgroup
+// takes `items` consecutive entries of it.  Inside, every lane group takes an equal stretch of the
+// nonzeros, eight rows of B in flight, and writes a row of C when it meets the row's last nonzero; what
+// is left of a row at either end of a stretch meets in LDS.  A row cut by the end of a workgroup leaves
+// partial rows in memory; the workgroup that finishes last among those of the row -- a counter in device
+// memory, set back to zero by that workgroup -- adds them up in order.  So C is written once, without
+// atomics, and the same bits every time.
+//
+// Bound by the gather of rows of B (1.17 M nonzeros, 47 features: 38 us, 9.6 TB/s of the 128-byte lines
+// that its rows touch).  With a launch over rows and a second one for what is long among them (spmm.hip) the
+// same product pays a second launch, a search of every piece for long rows that mostly are not there, and
+// wavefronts whose rows differ in length (51 us).
+#include <algorithm>
+
+#include "common.h"
+#include "lane_group.h"
+#include "../../include/sparsetir_amd.h"
+
+namespace {
+
+using stir::chunk_offset;
+using stir::fma4;
+using stir::kWave;
+using stir::ld4;
+
+constexpr int kBlock = 256;
+constexpr int kSlots = 768;     // nonzeros a workgroup holds in LDS: eight workgroups per compute unit
+// A row of at most this many nonzeros is not cut: it is left whole to the workgroup that has its mark.
+constexpr int kWhole = 128;
+constexpr int kMaxItems = 512;
+static_assert(kMaxItems + kWhole <= kSlots, "the last row of a workgroup may lie behind its entries");
+constexpr int kFlight = 8;      // rows of B requested at a time by a lane group
+
+// Last row r with indptr[r] + r <= q: q is a place in the list (indptr[0] added) and indptr[r] + r that of
+// the row's mark (q >= indptr[0], m >= 1).  The whole wavefront looks, 64 places at a time; four times as
+// many make the chain of round trips no shorter at these sizes and keep the texture addresser busy for
+// 0.6 us a workgroup (64 cache lines per load).
+__device__ __forceinline__ int last_mark(const int32_t* __restrict__ indptr, int m, int64_t q, int lane) {
+  int lo = 0, hi = m - 1;
+  while (hi > lo) {
+    const int64_t span = hi - lo;
+    const int base = lo;
+    const int pos = base + (int)((span * (lane + 1) + kWave - 1) / kWave);  // in (lo, hi], ascending
+    const int cnt = __popcll(__ballot((int64_t)indptr[pos] + pos <= q));
+    if (cnt) lo = base + (int)((span * cnt + kWave - 1) / kWave);
+    if (cnt < kWave) hi = base + (int)((span * (cnt + 1) + kWave - 1) / kWave) - 1;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ void coherent_store(float* p, const float4& v) {
+  __hip_atomic_store(p + 0, v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(p + 1, v.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(p + 2, v.z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(p + 3, v.w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ float4 coherent_load(const float* p) {
+  float4 v;
+  v.x = __hip_atomic_load(p + 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  v.y = __hip_atomic_load(p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  v.z = __hip_atomic_load(p + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  v.w = __hip_atomic_load(p + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return v;
+}
+
+__device__ __forceinline__ void add4(float4& a, const float4& b) { a.x += b.x, a.y += b.y, a.z += b.z, a.w += b.w; }
+
+__device__ __forceinline__ void store4(float* q, const float4& v) {
+  __builtin_nontemporal_store(v.x, q);
+  __builtin_nontemporal_store(v.y, q + 1);
+  __builtin_nontemporal_store(v.z, q + 2);
+  __builtin_nontemporal_store(v.w, q + 3);
+}
+
+template <int G, int REP>
+__global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(int m, int feat, int64_t nnz, int items,
+                                                              const float* __restrict__ A,
+                                                              const float* __restrict__ B, float* __restrict__ C,
+                                                              const int32_t* __restrict__ indptr,
+                                                              const int32_t* __restrict__ indices,
+                                                              uint32_t* __restrict__ counters,
+                                                              float* __restrict__ partials) {
+  constexpr int NG = kBlock / G;
+  constexpr int CH = kFlight / REP;
+  constexpr int kPad = 4 * G * REP;  // floats of a partial row
+  __shared__ int2 nz[kSlots];     // column, value
+  __shared__ int ends[kSlots];    // row + 1 at the row's last nonzero, else 0
+  __shared__ float4 head[NG * G * REP], tail[NG * G * REP];
+  __shared__ int open_all[NG];
+  __shared__ int row_at[2], nz_at[2], cut[2];
+  __shared__ int last[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int base = indptr[0];
+  const int64_t total = m + min(nnz, (int64_t)indptr[m]) - base;
+  const int64_t d0 = (int64_t)blockIdx.x * items, d1 = min(total, d0 + items);
+  if (d0 >= total) return;
+  if (wave < 2) {
+    const int64_t d = wave ? d1 : d0;
+    int i = 0, j = base, c = 0;
+    if (d > 0) {
+      const int r = last_mark(indptr, m, d - 1 + base, lane);
+      const int s = indptr[r], e = indptr[r + 1];
+      i = r + 1, j = (int)(d - i + base);
+      if (e > j) {
+        c = e - s > kWhole;
+        if (c) c = s < j; else j = e;
+      }
+    }
+    if (lane == 0) row_at[wave] = i, nz_at[wave] = j, cut[wave] = c;
+  }
+  for (int t = tid; t < kSlots; t += kBlock) ends[t] = 0;
+  __syncthreads();
+  // rows [i0, i1) have their marks here, the nonzeros [j0, j1) belong to them and, cut_before, to row i0 - 1
+  const int i0 = __builtin_amdgcn_readfirstlane(row_at[0]), i1 = __builtin_amdgcn_readfirstlane(row_at[1]);
+  const int j0 = __builtin_amdgcn_readfirstlane(nz_at[0]), j1 = __builtin_amdgcn_readfirstlane(nz_at[1]);
+  const bool cut_before = __builtin_amdgcn_readfirstlane(cut[0]), cut_after = __builtin_amdgcn_readfirstlane(cut[1]);
+  const int cnt = j1 - j0;
+  for (int t = tid; t < cnt; t += kBlock)
+    nz[t] = make_int2(__builtin_nontemporal_load(indices + j0 + t),
+                      __float_as_int(__builtin_nontemporal_load(A + j0 + t)));
+  const int first = max(i0 - 1, 0);
+  for (int r0 = first; r0 < i1; r0 += kBlock) {
+    const int r = r0 + tid;
+    int s = 0, e = 0;
+    if (r < i1) s = indptr[r], e = indptr[r + 1];
+    if (e > j0 && e > s && e <= j1) ends[e - 1 - j0] = r + 1;
+    uint64_t empty = __ballot(r >= i0 && r < i1 && s == e);
+    while (empty) {
+      const int k = __ffsll((long long)empty) - 1;
+      empty &= empty - 1;
+      float* row = C + (int64_t)(r0 + wave * kWave + k) * feat;
+      for (int f = lane; f < feat; f += kWave) __builtin_nontemporal_store(0.f, row + f);
+    }
+  }
+  __syncthreads();
+
+  const int grp = tid / G, gl = tid % G;
+  const int per = max(CH, (cnt + NG - 1) / NG);
+  const int a = min(cnt, grp * per), b = min(cnt, a + per);
+  const bool mid = a < b ? (a > 0 ? ends[a - 1] == 0 : cut_before) : true;  // begins inside a row
+  bool flushed = false;
+  int head_row = 0;
+  float4 acc[REP];
+#pragma unroll
+  for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k0 = 0; k0 < per; k0 += CH) {
+    float4 x[CH][REP];
+    float v[CH];
+    int f[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int p = a + k0 + u;
+      const bool live = p < b;
+      const int2 q = nz[min(p, kSlots - 1)];
+      f[u] = live ? ends[min(p, kSlots - 1)] : 0;
+      v[u] = live ? __int_as_float(q.y) : 0.f;
+      const float* bp = B + (int64_t)q.x * feat;
+#pragma unroll
+      for (int r = 0; r < REP; ++r) {
+        const int c0 = gl * 4 + r * G * 4;
+        x[u][r] = live && c0 < feat ? ld4(bp + chunk_offset(c0, feat)) : make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+#pragma unroll
+      for (int r = 0; r < REP; ++r) fma4(acc[r], v[u], x[u][r]);
+      if (f[u]) {
+        const bool keep = mid && !flushed;
+        float* row = C + (int64_t)(f[u] - 1) * feat;
+#pragma unroll
+        for (int r = 0; r < REP; ++r) {
+          const int c0 = gl * 4 + r * G * 4;
+          if (keep)
+            head[(grp * REP + r) * G + gl] = acc[r];
+          else if (c0 < feat)
+            store4(row + chunk_offset(c0, feat), acc[r]);
+          acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        if (keep) head_row = f[u];
+        flushed = true;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < REP; ++r) tail[(grp * REP + r) * G + gl] = acc[r];
+  if (gl == 0) open_all[grp] = mid && !flushed;
+  __syncthreads();
+
+  // pieces of rows: what the groups before a head left of its row, and of the row the workgroup ends in
+  const uint64_t open_groups = __ballot(lane < NG && open_all[lane % NG]);
+  const bool through = cut_after && cut_before && i0 == i1;
+  for (int which = 0; which < 2; ++which) {
+    const bool mine = which == 0 ? head_row != 0 : cut_after && grp == NG - 1;
+    if (!mine) continue;
+    // the row began in group k, -1: in a workgroup before this one
+    const uint64_t closed = ~open_groups & ((uint64_t(1) << (which == 0 ? grp : NG - 1) << (which == 0 ? 0 : 1)) - 1);
+    const int k = closed ? 63 - __clzll((long long)closed) : -1;
+    float4 sum[REP];
+#pragma unroll
+    for (int r = 0; r < REP; ++r)
+      sum[r] = which == 0 ? head[(grp * REP + r) * G + gl] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+    for (int q = max(k, 0); q < (which == 0 ? grp : NG); ++q)
+#pragma unroll
+      for (int r = 0; r < REP; ++r) add4(sum[r], tail[(q * REP + r) * G + gl]);
+#pragma unroll
+    for (int r = 0; r < REP; ++r) {
+      const int c0 = gl * 4 + r * G * 4;
+      if (which == 0 && k >= 0) {
+        if (c0 < feat) store4(C + (int64_t)(head_row - 1) * feat + chunk_offset(c0, feat), sum[r]);
+      } else {
+        coherent_store(partials + ((int64_t)blockIdx.x * 2 + which) * kPad + c0, sum[r]);
+      }
+    }
+  }
+  // a row that goes through the whole workgroup counts as the one it ends in
+  const bool has_head = cut_before && !through;
+  if (!has_head && !cut_after) return;  // uniform
+  // every store above has to have reached memory before the workgroup counts itself in
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid < 2) {
+    const bool mine = tid == 0 ? has_head : cut_after;
+    int before_last = 0;
+    if (mine) {
+      const int64_t r = tid == 0 ? i0 - 1 : i1 - 1;
+      const int64_t b0 = (indptr[r] - base + r + 1) / items, b1 = (indptr[r + 1] - base + r) / items;
+      before_last = __hip_atomic_fetch_add(counters + b0, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)(b1 - b0);
+      if (before_last) __hip_atomic_store(counters + b0, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    last[tid] = before_last;
+  }
+  __syncthreads();
+  for (int which = 0; which < 2; ++which) {
+    if (!last[which]) continue;  // uniform
+    const int r = which == 0 ? i0 - 1 : i1 - 1;
+    const int64_t b0 = ((int64_t)indptr[r] - base + r + 1) / items, b1 = ((int64_t)indptr[r + 1] - base + r) / items;
+    const int64_t count = b1 - b0 + 1, share = (count + NG - 1) / NG;
+    float4 sum[REP];
+#pragma unroll
+    for (int q = 0; q < REP; ++q) sum[q] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int64_t p = b0 + grp * share; p < min(b1 + 1, b0 + (grp + 1) * share); ++p)
+#pragma unroll
+      for (int q = 0; q < REP; ++q)
+        add4(sum[q], coherent_load(partials + (p * 2 + (p == b1 ? 0 : 1)) * kPad + gl * 4 + q * G * 4));
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < REP; ++q) tail[(grp * REP + q) * G + gl] = sum[q];
+    __syncthreads();
+    if (grp == 0) {
+      const int used = (int)min((int64_t)NG, count);
+      for (int k = 1; k < used; ++k)
+#pragma unroll
+        for (int q = 0; q < REP; ++q) add4(sum[q], tail[(k * REP + q) * G + gl]);
+#pragma unroll
+      for (int q = 0; q < REP; ++q) {
+        const int c0 = gl * 4 + q * G * 4;
+        if (c0 < feat) store4(C + (int64_t)r * feat + chunk_offset(c0, feat), sum[q]);
+      }
+    }
+  }
+}
+
+// About 1100 workgroups, four per compute unit, as long as that gives each a few stretches of nonzeros and
+// what it holds fits: 50 k rows, 450 k nonzeros, 64 features: 34.8 us with 64 entries, 22.9 with 288 or 480.
+int entries_per_workgroup(int32_t m, int64_t nnz) {
+  const int64_t items = (m + nnz) / 1100;
+  return (int)(std::max<int64_t>(64, std::min<int64_t>(items, kMaxItems)) + 31) / 32 * 32;
+}
+
+int64_t workgroups(int32_t m, int64_t nnz) {
+  return stir::ceil_div(m + nnz, entries_per_workgroup(m, nnz));
+}
+
+// Below, the search for its entries costs a workgroup more than it gains (4096 rows, 65 k nonzeros, 32
+// features: 8.6 us against 6.9); above, two launches over rows read B as fast and leave no partial rows
+// (2.4 M rows, 61.9 M nonzeros, 128 features: 5.49 ms against 4.98).  Between (old / new, us):
+// 6 k rows, 90 k nonzeros, 128 features 15.5 / 10.0; 24 k, 360 k, 33: 19.4 / 13.1; 50 k, 450 k, 8: 24.3 / 11.6;
+// 169 k, 1.17 M, 47: 50.7 / 38.2; 115 k, 2.3 M, 64: 92 / 85; 100 k, 1.5 M, 128: 121 / 117.
+bool balanced(int32_t m, int32_t feat, int64_t nnz) {
+  if (stir::vector_class(feat) < 0 || nnz * feat >= 500000000) return false;
+  return m >= 8192 || nnz * feat >= 3000000;
+}
+
+size_t padded(int feat) { return size_t(16) << stir::vector_class(feat); }
+
+}  // namespace
+
+extern "C" {
+
+size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t feat, int64_t nnz) {
+  if (m < 0 || feat <= 0 || nnz < 0 || !balanced(m, feat, nnz)) return 0;
+  const size_t wgs = (size_t)workgroups(m, nnz);
+  return (wgs * 4 + 15) / 16 * 16 + wgs * 2 * padded(feat) * 4;
+}
+
+int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A, const float* d_B,
+                                float* d_C, const int32_t* d_indptr, const int32_t* d_indices, void* d_workspace,
+                                void* stream) {
+  STIR_REQUIRE(m >= 0 && n >= 0 && feat > 0 && nnz >= 0, "csr_spmm: bad sizes m=%d n=%d feat=%d", m, n, feat);
+  if (!balanced(m, feat, nnz))
+    return stir_csr_spmm_f32(m, n, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, stream);
+  STIR_REQUIRE(d_B && d_C && d_indptr && d_workspace && (nnz == 0 || (d_A && d_indices)),
+               "csr_spmm: null pointer argument");
+  const int64_t wgs = workgroups(m, nnz);
+  STIR_REQUIRE(wgs < (int64_t(1) << 31), "csr_spmm: %lld workgroups exceed one launch", (long long)wgs);
+  const int items = entries_per_workgroup(m, nnz);
+  uint32_t* counters = static_cast<uint32_t*>(d_workspace);
+  float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + (size_t(wgs) * 4 + 15) / 16 * 16);
+#define STIR_BALANCED(G, REP)                                                                                    \
+  hipLaunchKernelGGL((csr_balanced_kernel<G, REP>), dim3((unsigned)wgs), dim3(kBlock), 0,                         \
+                     static_cast<hipStream_t>(stream), m, feat, nnz, items, d_A, d_B, d_C, d_indptr, d_indices,   \
+                     counters, partials)
+  switch (stir::vector_class(feat)) {
+    case 0: STIR_BALANCED(4, 1); break;
+    case 1: STIR_BALANCED(8, 1); break;
+    case 2: STIR_BALANCED(16, 1); break;
+    case 3: STIR_BALANCED(32, 1); break;
+    case 4: STIR_BALANCED(64, 1); break;
+    default: STIR_BALANCED(64, 2); break;
+  }
+#undef STIR_BALANCED
+  STIR_LAUNCH_CHECK();
+  return 0;
+}
+
+}  // extern "C"

@@ -13,6 +13,7 @@
 #include <vector>
 
 #include "common.h"
+#include "lane_group.h"
 #include "row_lookup.h"
 #include "../../include/sparsetir_amd.h"
 
@@ -25,7 +26,12 @@ static __device__ __align__(256) unsigned char scratch[2 * kStaticBuckets * 64];
 
 namespace {
 
+using stir::chunk_offset;
+using stir::fma4;
 using stir::kWave;
+using stir::ld4;
+using stir::tail_chunk;
+using stir::vector_class;
 
 struct alignas(16) HybBucket {
   const float* A;
@@ -42,34 +48,6 @@ struct alignas(16) HybBucket {
 // Row mode splits an ELL row of an accumulating bucket into chunks of this many slots, one
 // wavefront each, so that a hub row does not serialise on a single wavefront.
 constexpr int kRowChunk = 256;
-
-// four consecutive floats; a row of B whose width is no multiple of four starts at any float, and a
-// 16-byte load only needs its address to be a multiple of four bytes
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ float4 ld4(const float* p) {
-  const f32x4u v = *reinterpret_cast<const f32x4u*>(p);
-  return make_float4(v[0], v[1], v[2], v[3]);
-}
-
-// Feature widths: a lane's chunk number r is the four features from c0 = 4 * (lane in group + r * G)
-// on.  In a row whose width is no multiple of four the last chunk would reach into the next row (or
-// past the end of B): it is loaded from feat - 4 instead, four features of this row again; a store
-// writes the shared ones twice with the same value, an addition moves the ones that are not shared to
-// the front first (tail_chunk).
-__device__ __forceinline__ int chunk_offset(int c0, int feat) { return min(c0, feat - 4); }
-
-__device__ __forceinline__ float4 tail_chunk(float4 a, int over) {  // over: features of `a` before c0
-  if (over & 1) a = make_float4(a.y, a.z, a.w, 0.f);
-  if (over & 2) a = make_float4(a.z, a.w, 0.f, 0.f);
-  return a;
-}
-
-__device__ __forceinline__ void fma4(float4& acc, float a, const float4& x) {
-  acc.x = fmaf(a, x.x, acc.x);
-  acc.y = fmaf(a, x.y, acc.y);
-  acc.z = fmaf(a, x.z, acc.z);
-  acc.w = fmaf(a, x.w, acc.w);
-}
 
 // Sum `acc` over the lane groups whose group index differs in the bits [G, limit).
 template <int G, int REP>
@@ -712,17 +690,6 @@ __global__ __launch_bounds__(256) void hyb_table_fill_kernel(HybTableChunk chunk
   const uint32_t* src = reinterpret_cast<const uint32_t*>(&chunk);
   uint32_t* out = reinterpret_cast<uint32_t*>(dst);
   for (int i = threadIdx.x; i < count * kWords; i += 256) out[i] = src[i];
-}
-
-// 0..5: lane groups of 4, 8, 16, 32, 64 lanes and 64 lanes x 2 float4 cover feat; -1: the kernel of
-// one lane per feature (a row narrower than one float4, or wider than two per lane).  Widths that are
-// no multiple of 4 take the same kernels (chunk_offset): 169 k nodes, 1.17 M edges with hubs on both
-// sides, 47 features: 1750 us with one lane per feature (the chain of the hub row), 52 us with these.
-int vector_class(int feat) {
-  if (feat < 4 || feat > 512) return -1;
-  int c = 0;
-  while ((16 << c) < feat) ++c;
-  return c;
 }
 
 int log2_exact(int64_t x) {

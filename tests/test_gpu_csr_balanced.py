@@ -1,0 +1,57 @@
+"""CSR products by workgroups of equal work: one launch, rows cut between workgroups and lane groups."""
+import numpy as np
+import pytest
+import torch
+
+from sparsetir_amd import ops
+from test_gpu_spmm import _check
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(rng, m, n, lengths, most):
+    """Row degrees 0 to `most` with the given lengths at the front, in the middle and at the end."""
+    deg = rng.integers(0, most + 1, m)
+    deg[m // 4:m // 3] = 0  # a run of empty rows
+    for k, d in enumerate(lengths):
+        deg[k] = deg[m // 2 + 3 * k] = deg[m - 1 - 2 * k] = d
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    return deg, indptr, rng.integers(0, n, indptr[-1]).astype(np.int32)
+
+
+@pytest.mark.parametrize("feat", [4, 13, 16, 32, 47, 64, 100, 128, 256, 300, 512])
+@pytest.mark.parametrize("m,most", [(8192, 3), (9001, 24), (40003, 14)])
+def test_rows_across_workgroups(dev, feat, m, most):
+    """Rows around the length that is never cut, rows over many workgroups next to each other, empty
+    rows, arrays longer than the last row pointer; the same bits again, on another stream and recorded."""
+    rng = np.random.default_rng(feat + m)
+    n = 5000
+    deg, indptr, indices = _matrix(rng, m, n, [0, 128, 129, 127, 1, 4000, 3000, 512, 640, 0, 257, 130], most)
+    spare = 7
+    indices = np.concatenate([indices, np.zeros(spare, np.int32)])
+    vals = rng.random(len(indices), dtype=np.float32) - 0.4
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    args = (t(vals), t(x.ravel()))
+    tail = (t(indptr), t(indices))
+    f = ops.build_csrmm(m, n, feat, len(indices))
+    c = [torch.full((m * feat,), float("nan"), device=dev) for _ in range(3)]
+    f(*args, c[0], *tail)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        f(*args, c[1], *tail)
+        f(*args, c[1], *tail)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        f(*args, c[2], *tail)
+    for _ in range(3):
+        c[2].fill_(float("nan"))
+        graph.replay()
+        f(*args, c[1], *tail)
+        torch.cuda.synchronize()
+        assert torch.equal(c[0], c[1]) and torch.equal(c[0], c[2])
+    got = c[0].cpu().numpy().reshape(m, feat)
+    assert np.all(got[deg == 0] == 0.0)
+    _check(got, indptr, indices[:-spare], vals[:-spare], x, f"m={m} feat={feat}")

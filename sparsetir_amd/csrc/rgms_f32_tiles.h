@@ -1,13 +1,14 @@
-// Destination-tiled fp32 RGMS: every 64-row tile of Y is summed on chip and written once, without
+// Destination-tiled fp32 RGMS: every 128-row tile of Y is summed on chip and written once, without
 // atomics.  Serves both fp32 front ends (ELL3D buckets and the CSF arrays).
 //
 // The edges (slots) of the operator are re-indexed once per plan, sorted by (destination tile of
-// 64 rows, relation, destination row); runs of equal key are the (relation, row) pairs, whose
-// weighted sums of X rows meet the relation's W on the matrix cores 16 pairs at a time
-// (v_mfma_f32_16x16x4_f32), and the products are added into a partial tile in LDS.  Tiles with
-// many more edges than the average are cut into pieces, and so are the few tiles beyond whole
-// rounds of resident workgroups; the piece of a tile that finishes last adds the pieces' partial
-// tiles in a fixed order: the result does not depend on the order in which wavefronts run.
+// 128 rows, relation, destination row); runs of equal key are the (relation, row) pairs, whose
+// weighted sums of X rows meet the relation's W on the matrix cores 16 pairs at a time, both split into
+// three bf16 terms, and the products are added into a partial tile in LDS.  Tiles are cut into pieces
+// where whole ones would not give every compute unit an equal part; the piece of a tile that finishes last
+// adds the pieces' partial tiles in a fixed order: the result does not depend on the order in which
+// wavefronts run.
+// (The split keeps 24 bits of finite values below 3.38e38; an infinite sum or weight gives NaN.)
 #pragma once
 #include <cstdint>
 #include <vector>
@@ -37,17 +38,22 @@ struct F32Source {
   int64_t nnz_i = 0, nnz_j = 0;
 };
 
+// What a launch's workgroups take, longest first: tiles or pieces of tiles, as ranges of batches.
+struct F32Units {
+  int64_t count = 0, partial_tiles = 0;
+  void* d_units = nullptr;     // count x 32 bytes
+  void* d_arrived = nullptr;   // a counter per tile cut into several units, zero between launches
+  void* d_partials = nullptr;  // their partial tiles, rewritten by every launch
+  size_t partial_bytes = 0;
+};
+
 struct F32TileIndex {
   int32_t m = -1, n = -1, num_rels = -1, emax = 0;  // what the index was built for (emax: edges per batch)
   int64_t edges = 0, pairs = 0, batches = 0, tiles = 0;
-  int64_t units = 0, multi = 0, partial_tiles = 0;
-  void* d_edges = nullptr;     // edges x 16 bytes, sorted
-  void* d_pairs = nullptr;     // pairs x 4 bytes, sorted: row in tile | edges << 8 | first edge in its batch << 16
-  void* d_batches = nullptr;   // batches x 16 bytes: up to 16 pairs and emax edges of one (tile, relation) each
-  void* d_units = nullptr;     // units x 32 bytes: a tile or a piece of one, as a range of batches; longest first
-  void* d_arrived = nullptr;   // a counter per tile cut into several units (`multi` of them), zero between launches
-  void* d_partials = nullptr;  // their partial tiles, rewritten by every launch
-  size_t partial_bytes = 0;
+  F32Units units[2];           // for feat_out up to 32, and above
+  void* d_edges = nullptr;     // places x 12 bytes: an edge each, or none
+  void* d_pairs = nullptr;     // batches x 16 x 4 bytes: a word per pair
+  void* d_batches = nullptr;   // batches x 16 bytes: up to 16 pairs and emax places of one (tile, relation) each
   void* d_wpack = nullptr;     // W in the multiply's operand order, rewritten by every launch
   size_t wpack_bytes = 0;
 };

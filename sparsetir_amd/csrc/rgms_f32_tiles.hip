@@ -1,36 +1,38 @@
 // Destination-tiled fp32 RGMS declared in rgms_f32_tiles.h: index construction and the kernels.
 //
 // Index (once per plan): every slot of the ELL3D buckets -- or every stored column of the CSF
-// arrays -- is an edge with the key (destination row / 64, relation, destination row % 64).  One
+// arrays -- is an edge with the key (destination row / 128, relation, destination row % 128).  One
 // stable radix sort orders the edges by key; runs of equal key are the (relation, row) pairs, cut
 // into pieces of at most EMAX = 32 / KS edges (a second key: key << 20 | position in the run /
 // EMAX, run-length encoded).  The pairs of one (tile, relation) run are cut into batches of at
-// most 16 pairs and at most EMAX edges, listed per tile; a tile with many more batches than the
-// average is cut into several units, whose partial tiles go to memory of the plan; the unit of a
-// tile that finishes last adds them up, in the order of the units.
-// An edge record holds the source row and the address of the edge's weight (weights are read at
-// every launch); a pair is one word: row inside the tile, edges, first edge inside its batch.
+// most 16 pairs and at most EMAX places, listed per tile.  The places of a batch are columns of four: the
+// edges of a pair stand in them one below the other, as chains of at most four.
+// An edge record holds the source row, the address of the edge's weight (weights are read at
+// every launch) and its part in a chain; a pair is one word: row inside the tile, chains, first chain.
 //
-// Kernel: one workgroup of four wavefronts per unit; wavefront w takes the unit's batches w,
-// w + 4, ... and sums into a partial tile of its own in LDS.  Per batch:
-//   1. the rows of X of the batch's edges, times their weights, go to a tile of LDS, eight rows
-//      (128 bytes each) per load instruction: every lane useful whatever the pairs look like;
-//   2. lane (i = l % 16, q = l / 16) adds up the rows of pair i from that tile: inputs 8q .. 8q+7
+// Kernel: one workgroup per unit -- a tile, or a piece of one; wavefront w takes the unit's batches w,
+// w + WAVES, ... and all of them sum into one partial tile in LDS, in turn.  Per batch:
+//   1. the rows of X of the batch's edges are gathered eight rows (128 bytes each) per load instruction,
+//      a column of places per lane group, which weights and adds up its chains in registers and writes
+//      each to a row of a tile of LDS;
+//   2. lane (i = l % 16, q = l / 16) adds up the chains of pair i, mostly one: inputs 8q .. 8q+7
 //      (+32 per further 32 inputs) of S[i, :] = sum over the edges e of pair i of w_e X[src_e, :];
-//   3. P = S @ W[rel]^T on v_mfma_f32_16x16x4_f32.  The instruction's k index is lane / 16; the
-//      t-th instruction takes input 8q + t from lane (., q) in both operands, so S needs no
-//      rearrangement and a lane's W operands are 32 contiguous bytes of a row of W[rel];
-//   4. row i of P is added to row (destination row % 64) of the wavefront's partial tile with a
+//   3. P = S @ W[rel]^T on v_mfma_f32_16x16x32_bf16, S and W split into three bf16 terms each: a lane's
+//      eight inputs are its operand as they stand;
+//   4. row i of P is added to row (destination row % 128) of the partial tile with a
 //      plain LDS read-modify-write: the pairs of a batch end in different rows or in pieces of
-//      one row that this lane order adds one after the other, and no other wavefront touches
-//      this partial tile (LDS float atomics run at a third of a lane per clock and compute unit
+//      one row that this lane order adds one after the other, and the wavefronts take turns, in the order
+//      of the batches (LDS float atomics run at a third of a lane per clock and compute unit
 //      on this chip, slower than atomics in memory).
-// A batch is a chain of dependent loads (batch record -> edge records -> rows of X and weights),
-// so everything is requested two of the wavefront's batches before the step of the chain that
-// needs it, into registers that are never copied while a load is in flight (two sets, a loop
-// unrolled by two); the loop body has no branch around a load.
-// At the end the four partial tiles are added up: into the tile's rows of Y, each element once,
-// or -- for a unit that is a piece of a tile -- into the plan's memory for partial tiles, with
+// A batch is a chain of dependent loads (batch record -> edge records -> rows of X and weights), each step
+// of it requested one batch ahead of the next.
+//
+// Bound by the vector unit: 165 instructions per batch, busy 61 % of the kernel's clocks (100 k nodes, 65
+// relations, 2 M edges, 32 -> 32: 112 k batches, 67 us, 78 per call; 129 before, when each wavefront had a
+// partial tile of 64 rows to itself -- 146 k batches -- and three wavefronts per SIMD in the place of four
+// waited on v_mfma_f32_16x16x4_f32, during which the vector unit stands still).
+// At the end the partial tile is added to the tile's rows of Y, each element once,
+// or -- for a unit that is a piece of a tile -- goes to the plan's memory for partial tiles, with
 // device-coherent stores.  Such a unit then counts itself in (a counter per cut tile); the one
 // that counts last reads the partial tiles of all, coherently, adds them in unit order into Y and
 // sets the counter back to zero: no second launch, no fence that writes back or invalidates a
@@ -38,6 +40,7 @@
 #include "rgms_f32_tiles.h"
 
 #include <algorithm>
+#include <type_traits>
 
 #include <hipcub/hipcub.hpp>
 
@@ -45,17 +48,19 @@ namespace stir {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 
-constexpr int kTileRows = 64;
-constexpr int kTileShift = 6;
+constexpr int kTileRows = 128;
+constexpr int kTileShift = 7;
 constexpr int kBatch = 16;    // pairs per matrix-core product
+constexpr int kChain = 4;     // edges of a pair that a lane group adds up one after the other
 constexpr int kSubBits = 20;  // pieces of one (relation, row) run in the second sort key
 
 struct alignas(16) BatchF32 {
-  int32_t pair_begin;  // first pair word
-  int32_t edge_begin;  // first sorted edge
-  uint32_t counts;     // pairs (at most kBatch) | edges << 8 (at most EMAX) | most edges of a pair << 16
+  uint32_t place_begin;  // first place of its edges
+  uint32_t counts;       // pairs (at most kBatch) | most chains of a pair << 8 | places (at most EMAX) << 16
   int32_t rel;
+  int32_t pad;
 };
 
 struct alignas(16) UnitF32 {
@@ -85,12 +90,18 @@ struct CsfArrays {
   int64_t nnz_i;
 };
 
-struct alignas(16) EdgeF32 {
-  int32_t src;  // row of X
-  int32_t pad;
-  const float* w;  // the edge's weight
+struct EdgeF32 {  // 12 bytes
+  uint32_t src;   // row of X; kUnused: no edge
+  uint32_t w_lo;  // address of the edge's weight,
+  uint32_t w_hi;  // 48 bits of it | chain << 16: the row of the chain tile the sum goes to after this edge (the
+                  // row behind the row of zeros unless the edge ends a chain) | 256 when the edge before it in
+                  // the column belongs to the same chain
 };
-
+constexpr uint32_t kBehindX = 0xffff0000u;  // X is shorter: no row begins here, and 16 bytes per lane do not wrap
+constexpr uint32_t kUnused = (1u << 28) - 1;  // rows of X are fewer: X has less than 2^32 bytes
+// pair word: row in the tile | chains << 8 | byte offset of the first chain's row in the chain tile << 16;
+// 16 words per batch, for a place without a pair the row behind the tile and the row of zeros
+__host__ __device__ constexpr uint32_t chain_row_bytes(int emax) { return emax == 32 ? 36 * 4 : 68 * 4; }
 
 __device__ __forceinline__ int bucket_of(const DevBucketF32* __restrict__ tab, int nb, int64_t q) {
   int lo = 0, hi = nb - 1;
@@ -154,21 +165,42 @@ __global__ __launch_bounds__(256) void f32_edge_keys_kernel(const DevBucketF32* 
   vals[q] = (int32_t)q;
 }
 
+// Places without an edge: nothing is fetched for them but a weight that exists.
+__global__ __launch_bounds__(256) void f32_clear_places_kernel(EdgeF32* __restrict__ places, int64_t count, int emax,
+                                                               const float* w, uint32_t* __restrict__ pinfo,
+                                                               int64_t words) {
+  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const uint64_t at = reinterpret_cast<uintptr_t>(w);
+  if (p < count) places[p] = EdgeF32{kUnused, (uint32_t)at, (uint32_t)(at >> 32) | ((uint32_t)(emax + 1) << 16)};
+  if (p < words) pinfo[p] = (uint32_t)kTileRows | ((uint32_t)emax * chain_row_bytes(emax) << 16);
+}
+
+// Sorted edge i, number t of its pair, goes to the pair's place number t: the last pair whose first
+// edge is not behind i.
 template <bool CSF>
 __global__ __launch_bounds__(256) void f32_edge_records_kernel(const DevBucketF32* __restrict__ tab, int nb,
-                                                               CsfArrays csf, int64_t slots, int num_rels,
+                                                               CsfArrays csf, int64_t slots, int num_rels, int emax,
                                                                const int32_t* __restrict__ vals,
-                                                               EdgeF32* __restrict__ edges) {
-  const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= slots) return;
+                                                               const int32_t* __restrict__ pair_first,
+                                                               const int32_t* __restrict__ pair_edges,
+                                                               const int64_t* __restrict__ pair_place, int64_t pairs,
+                                                               EdgeF32* __restrict__ places) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= slots) return;
+  int64_t lo = 0, hi = pairs - 1;
+  while (lo < hi) {
+    const int64_t mid = (lo + hi + 1) >> 1;
+    if ((int64_t)pair_first[mid] <= i) lo = mid; else hi = mid - 1;
+  }
+  const int t = (int)(i - pair_first[lo]);
   int dest, rel, src;
   const float* w;
-  edge_of<CSF>(tab, nb, csf, num_rels, vals[p], dest, rel, src, w);
-  EdgeF32 e;
-  e.src = src;
-  e.pad = 0;
-  e.w = w;
-  edges[p] = e;
+  edge_of<CSF>(tab, nb, csf, num_rels, vals[i], dest, rel, src, w);
+  const uint64_t at = reinterpret_cast<uintptr_t>(w);
+  const int64_t place = pair_place[lo];  // place << 8 | first chain
+  const bool last = t == pair_edges[lo] - 1 || t % kChain == kChain - 1;
+  const uint32_t chain = (last ? (uint32_t)(place & 255) + t / kChain : emax + 1) | (t % kChain ? 256u : 0u);
+  places[(place >> 8) + t] = EdgeF32{(uint32_t)src, (uint32_t)at, (uint32_t)(at >> 32) | (chain << 16)};
 }
 
 // key2[i] = key[i] << kSubBits | (position of sorted edge i in its run of equal key) / emax; `first`
@@ -199,9 +231,10 @@ __global__ __launch_bounds__(256) void f32_shift_keys_kernel(const uint64_t* __r
 }
 
 // Run i is a (tile, relation) run of run_pairs[i] pairs starting at pair run_first_pair[i]: its
-// pairs, in order, fill batches of at most kBatch pairs and at most emax edges.  Counts the
-// batches (FILL = false) or writes them and the pairs' words (FILL = true).  A pair has at most
-// emax edges (f32_subkeys_kernel), so every batch takes at least one.
+// pairs, in order, fill batches of at most kBatch pairs and emax places.  The places are columns of kChain,
+// one column per lane group: a pair of up to kChain edges lies inside a column, a longer one (at most emax
+// edges, f32_subkeys_kernel) begins a column and goes on in the next.  Counts the batches (FILL = false) or
+// writes them, the pairs' words and first places (FILL = true).
 template <bool FILL>
 __global__ __launch_bounds__(256) void f32_batches_kernel(const uint64_t* __restrict__ run_keys,
                                                           const int32_t* __restrict__ run_pairs,
@@ -209,37 +242,45 @@ __global__ __launch_bounds__(256) void f32_batches_kernel(const uint64_t* __rest
                                                           const int32_t* __restrict__ run_first_batch, int64_t runs,
                                                           int num_rels, int emax, const uint64_t* __restrict__ pair_keys,
                                                           const int32_t* __restrict__ pair_edges,
-                                                          const int32_t* __restrict__ pair_first,
                                                           int32_t* __restrict__ run_batches,
-                                                          BatchF32* __restrict__ batches, uint32_t* __restrict__ pinfo) {
+                                                          int64_t* __restrict__ run_places,
+                                                          const int64_t* __restrict__ run_first_place,
+                                                          BatchF32* __restrict__ batches, uint32_t* __restrict__ pinfo,
+                                                          int64_t* __restrict__ pair_place) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= runs) return;
   const int np = run_pairs[i], fp = run_first_pair[i];
   const int rel = (int)(run_keys[i] % (uint64_t)num_rels);
   int nb = 0;
+  int64_t base = FILL ? run_first_place[i] : 0;
   for (int j = 0; j < np;) {
     const int pb = j;
-    int ne = 0, most = 0;
+    int place = 0, chains = 0, most = 0;
     do {
       const int c = min(pair_edges[fp + j], emax);
-      if (j > pb && (j - pb == kBatch || ne + c > emax)) break;
+      int at = place;
+      if (at % kChain + c > kChain) at = (at + kChain - 1) / kChain * kChain;
+      if (j > pb && (j - pb == kBatch || at + c > emax)) break;
+      const int mine = (c + kChain - 1) / kChain;
       if (FILL) {
         const uint32_t dl = (uint32_t)((pair_keys[fp + j] >> kSubBits) & (kTileRows - 1));
-        pinfo[fp + j] = dl | ((uint32_t)c << 8) | ((uint32_t)ne << 16);
+        pinfo[((int64_t)run_first_batch[i] + nb) * kBatch + (j - pb)] =
+            dl | ((uint32_t)mine << 8) | ((uint32_t)chains * chain_row_bytes(emax) << 16);
+        pair_place[fp + j] = ((base + at) << 8) | chains;
       }
-      ne += c, most = max(most, c), ++j;
+      place = at + c, chains += mine, most = max(most, mine), ++j;
     } while (j < np);
     if (FILL) {
       BatchF32 b;
-      b.pair_begin = fp + pb;
-      b.edge_begin = pair_first[fp + pb];
-      b.counts = (uint32_t)(j - pb) | ((uint32_t)ne << 8) | ((uint32_t)most << 16);
+      b.place_begin = (uint32_t)base;
+      b.counts = (uint32_t)(j - pb) | ((uint32_t)most << 8) | ((uint32_t)place << 16);
       b.rel = rel;
+      b.pad = 0;
       batches[run_first_batch[i] + nb] = b;
     }
-    ++nb;
+    base += place, ++nb;
   }
-  if (!FILL) run_batches[i] = nb;
+  if (!FILL) run_batches[i] = nb, run_places[i] = base;
 }
 
 // begin[t] = first batch of tile t (t = tiles gives the batch count): the first run whose key
@@ -261,27 +302,71 @@ __global__ __launch_bounds__(256) void f32_tile_batches_kernel(const uint64_t* _
 
 typedef __attribute__((address_space(1))) const float GlobalF32;  // a global-memory load, not a flat one
 
-// W[rel][16 nt + i][32 s + 8 q + 4 c .. + 3] -> Wp[((rel * NT + nt) * KS + s) * 2 + c][lane (i, q)]: the
-// B operands of a batch as four-float words in lane order, so that the kernel's loads of W are
-// contiguous (a lane of the multiply owns one row of W per output tile: read in place, the 64
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+// Eight floats as sums of three bf16 each: v = t[0] + t[1] + t[2], exactly as long as nothing underflows (each
+// term is what the ones before it leave, rounded to nearest: 8 + 8 + 8 bits of a 24-bit significand).
+__device__ __forceinline__ void split3(const float (&v)[8], bf16x8 (&t)[3]) {
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    f32x2 r = {v[j], v[j + 1]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const bf16x2 h = __builtin_convertvector(r, bf16x2);
+      t[k][j] = h[0], t[k][j + 1] = h[1];
+      if (k < 2) {
+        const uint32_t both = __builtin_bit_cast(uint32_t, h);
+        r[0] -= __uint_as_float(both << 16), r[1] -= __uint_as_float(both & 0xffff0000u);
+      }
+    }
+  }
+}
+
+// W[rel][16 nt + i][32 s + 8 q .. + 7] -> Wp[((rel * NT + nt) * KS + s) * 3 + term][lane (i, q)]: the B
+// operands of a batch, split into three bf16 terms, as 16-byte words in lane order, so that the kernel's loads
+// of W are contiguous (a lane of the multiply owns one row of W per output tile: read in place, the 64
 // lanes of a load would touch 16 different lines four times over).  Zero beyond feat_in and
-// feat_out.  One thread per word.
-__global__ __launch_bounds__(256) void f32_pack_w_kernel(const float* __restrict__ W, float4* __restrict__ Wp,
-                                                         int64_t words, int nt_count, int ks_count, int fin, int fout) {
+// feat_out.  One thread per lane of a fragment.
+__global__ __launch_bounds__(256) void f32_pack_w_kernel(const float* __restrict__ W, bf16x8* __restrict__ Wp,
+                                                         int64_t fragments, int nt_count, int ks_count, int fin, int fout) {
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (t >= words) return;
+  if (t >= fragments) return;
   const int lane = (int)(t & 63), i = lane & 15, q = lane >> 4;
-  int64_t f = t >> 6;
-  const int c = (int)(f & 1);
-  f >>= 1;
+  const int64_t f = t >> 6;
   const int s = (int)(f % ks_count);
-  f /= ks_count;
-  const int nt = (int)(f % nt_count);
-  const int64_t rel = f / nt_count;
-  const int out = 16 * nt + i, k = 32 * s + 8 * q + 4 * c;
-  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (out < fout && k < fin) v = *reinterpret_cast<const float4*>(W + (rel * fout + out) * fin + k);
-  Wp[t] = v;
+  const int nt = (int)(f / ks_count % nt_count);
+  const int64_t rel = f / ks_count / nt_count;
+  const int out = 16 * nt + i;
+  float v[8];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int k = 32 * s + 8 * q + 4 * c;  // fin is a multiple of 4
+    float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (out < fout && k < fin) w = *reinterpret_cast<const float4*>(W + (rel * fout + out) * fin + k);
+    v[4 * c] = w.x, v[4 * c + 1] = w.y, v[4 * c + 2] = w.z, v[4 * c + 3] = w.w;
+  }
+  bf16x8 term[3];
+  split3(v, term);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) Wp[(f * 3 + k) * 64 + lane] = term[k];
+}
+
+// The value that the lane of place K of the lane's own column holds (see my_place in the kernel).
+template <int KS, int K>
+__device__ __forceinline__ int at_place(int v) {
+  const int a = __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, false);  // lane K of the row of 16
+  if constexpr (KS == 1) return __builtin_amdgcn_update_dpp(a, v, 0x150 + kChain + K, 0xf, 0xc, false);
+  return a;
+}
+
+template <class F>
+__device__ __forceinline__ void static_for_chain(F f) {
+  f(std::integral_constant<int, 0>());
+  f(std::integral_constant<int, 1>());
+  f(std::integral_constant<int, 2>());
+  f(std::integral_constant<int, 3>());
 }
 
 // KS: feat_in <= 32 * KS; NT: feat_out <= 16 * NT.
@@ -290,242 +375,243 @@ __global__ __launch_bounds__(256) void f32_pack_w_kernel(const float* __restrict
 // neighbouring lanes, four floats each, so that a load instruction reads 64 / CPR whole rows and
 // the texture addresser sees whole lines per quad of lanes; the four load instructions of a batch
 // cover its EMAX = 32 / KS edges in order.  Multiplying: lane (i = l % 16, q = l / 16) holds
-// inputs 8q .. 8q+7 of pair i.  The weighted rows change layout through an EMAX x 32 KS tile of
-// LDS per wavefront: written once per edge, read once per edge by the lanes of the edge's pair.
+// inputs 8q .. 8q+7 of pair i.  The rows change layout through an EMAX x 32 KS tile of LDS per
+// wavefront: written once per edge, read once per edge by the lanes of the edge's pair.
 //
-// The loads of the batch loop are unconditional -- indices are clamped to records that exist and
-// what must not count is multiplied by zero afterwards -- so that the loop body is one basic
-// block.  Offsets into X and the edge records are 32-bit byte offsets from scalar bases (the
-// launch checks that they fit).
+// The loads of the batch loop are unconditional, so that the loop body has no branch around a load:
+// edge records are clamped to ones that exist, and a row of X that no edge asks for is read behind the
+// end of the buffer, which returns zeros and fetches nothing.  Offsets into X and the edge records are
+// 32-bit byte offsets (the launch checks that they fit).
 template <int KS, int NT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KS == 1 && NT == 2 ? 3 : 1, 3)))
-void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches,
-                                                            const UnitF32* __restrict__ units,
-                                                            const BatchF32* __restrict__ batches,
-                                                            const uint32_t* __restrict__ pinfo,
-                                                            const EdgeF32* __restrict__ edges,
-                                                            const float4* __restrict__ Wp,
-                                                            const float* __restrict__ X, float* __restrict__ Y,
-                                                            float* partials, uint32_t* arrived) {
-  constexpr int FO = 16 * NT;      // floats per row of a partial tile
+struct TileShape {
+  // as many wavefronts as registers and LDS allow per compute unit: 20, 16, 16, 12 (4, 2, 4, 2 workgroups)
+  static constexpr int kWaves = KS == 1 ? (NT == 4 ? 8 : 4) : (NT == 4 ? 6 : 4);
+  static constexpr int kPerSimd = KS == 1 ? (NT == 4 ? 4 : 4) : (NT == 4 ? 3 : 4);
+};
+
+template <int KS, int NT>
+__global__ __launch_bounds__((64 * TileShape<KS, NT>::kWaves))
+__attribute__((amdgpu_waves_per_eu(TileShape<KS, NT>::kPerSimd, TileShape<KS, NT>::kPerSimd)))
+void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t x_bytes,
+                          const UnitF32* __restrict__ units, const BatchF32* __restrict__ batches,
+                          const uint32_t* __restrict__ pinfo, const EdgeF32* __restrict__ edges,
+                          const bf16x8* __restrict__ Wp, const float* __restrict__ X, float* __restrict__ Y,
+                          float* partials, uint32_t* arrived) {
+  constexpr int WAVES = TileShape<KS, NT>::kWaves;
+  constexpr int THREADS = 64 * WAVES;
+  constexpr int FO = 16 * NT;      // floats per row of the partial tile
   constexpr int CPR = 8 * KS;      // lanes (16-byte chunks) per gathered row
   constexpr int RPI = 64 / CPR;    // rows per load instruction
-  constexpr int EMAX = 32 / KS;    // edges per batch
-  constexpr int NLOAD = EMAX / RPI;
-  constexpr int SS = 32 * KS + 4;  // floats per row of the edge tile: 16 lanes reading 32 bytes each hit 64 banks
-  static_assert(NLOAD == 4, "four load instructions per batch");
-  static_assert(NT == 2 || NT == 4, "a lane's outputs are one 8- or 16-byte word of the partial tile");
-  __shared__ __attribute__((aligned(16))) float ytile[4][kTileRows * FO];
-  __shared__ __attribute__((aligned(16))) float etile[4][(EMAX + 1) * SS];  // the last row stays zero
-  __shared__ int last_of_tile;
+  constexpr int EMAX = 32 / KS;    // places per batch
+  constexpr int SS = 32 * KS + 4;  // floats per row of the chain tile: 16 lanes reading 32 bytes each hit 64 banks
+  static_assert(EMAX == RPI * kChain, "a lane group has a column of places");
+  static_assert(NT == 1 || NT == 2 || NT == 4, "a lane's outputs are one word of the partial tile");
+  __shared__ __attribute__((aligned(16))) float yt[(kTileRows + 1) * FO];
+  // a row per chain; row EMAX stays zero, row EMAX + 1 takes what ends no chain
+  __shared__ __attribute__((aligned(16))) float etile[WAVES][(EMAX + 2) * SS - 4];
+  __shared__ int turn, last_of_tile;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i = lane & 15, q = lane >> 4;      // multiplying
-  const int gr = lane / CPR, gc = lane % CPR;  // gathering
+  const int gc = lane % CPR;                   // gathering
   const UnitF32 u = units[blockIdx.x];
-  float* yt = ytile[wave];
   float* et = etile[wave];
-  for (int e = lane; e < kTileRows * FO; e += 64) yt[e] = 0.f;
-  for (int e = lane; e < (EMAX + 1) * SS; e += 64) et[e] = 0.f;
-
+  for (int e = tid; e < kTileRows * FO; e += THREADS) yt[e] = 0.f;
+  for (int e = lane; e < SS; e += 64) et[EMAX * SS + e] = 0.f;
+  if (tid == 0) turn = u.batch_begin;
   const int b_end = u.batch_end;
   int b = u.batch_begin + wave;
   const bool chunk_live = 4 * gc < fin;  // fin is a multiple of 4: chunks are whole
-  const uint32_t x_off = chunk_live ? 16u * gc : 0u;
   const uint32_t row_bytes = 4u * (uint32_t)fin;
-  const char* Xb = reinterpret_cast<const char*>(X);
-  const char* Eb = reinterpret_cast<const char*>(edges);
+  const __amdgpu_buffer_rsrc_t Xr =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(X), 0, x_bytes, 0x00027000);
 
   struct Batch {  // the same in every lane
-    uint32_t pair_begin, edge_off;  // edge_off in bytes
-    int npairs, nedges, most, rel;
+    uint32_t place_begin;
+    int npairs, most, places, rel;
   };
-  auto raw_batch = [&](int bi) { return batches[min(bi, total_batches - 1)]; };
-  auto scalars = [&](const BatchF32& t, int bi) {  // a batch beyond the unit's last one: no pairs, no edges
+  // A vector load although every lane wants the same 16 bytes: a scalar load in flight makes every wait for
+  // LDS a wait for memory (both count in lgkmcnt, and scalar loads return in any order).
+  int no_scalar = 0;
+  asm("" : "+v"(no_scalar));
+  auto raw_batch = [&](int bi) { return batches[min(bi, total_batches - 1) + no_scalar]; };
+  auto scalars = [&](const BatchF32& t, int bi) {  // a batch beyond the unit's last one: no pairs
     Batch r;
     const uint32_t c = bi < b_end ? __builtin_amdgcn_readfirstlane(t.counts) : 0u;
-    r.pair_begin = __builtin_amdgcn_readfirstlane((uint32_t)t.pair_begin);
-    r.edge_off = __builtin_amdgcn_readfirstlane((uint32_t)t.edge_begin) * 16u;
-    r.npairs = (int)(c & 255u), r.nedges = (int)((c >> 8) & 255u), r.most = (int)((c >> 16) & 255u);
+    r.place_begin = __builtin_amdgcn_readfirstlane(t.place_begin);
+    r.npairs = (int)(c & 255u), r.most = (int)((c >> 8) & 255u), r.places = (int)((c >> 16) & 255u);
     r.rel = __builtin_amdgcn_readfirstlane(t.rel);
     return r;
   };
-  struct EdgesG {  // gathering layout: load instruction k serves edge k * RPI + gr of the batch
-    int32_t src[NLOAD];
-    const float* w[NLOAD];
+  // Lane j of a row of 16 lanes holds the places of the lane groups in that row: two columns (KS = 1, lanes
+  // 8 ... 15 as lanes 0 ... 7) or one (KS = 2).  at_place<k> hands a lane the value of place k of its own
+  // column, by DPP broadcasts inside the row: no trip through LDS.
+  const int my_place = (lane >> 4) * (KS == 1 ? 2 * kChain : kChain) + (lane & (KS == 1 ? 2 * kChain - 1 : kChain - 1));
+  auto load_record = [&](const Batch& bt) {
+    return *reinterpret_cast<const u32x3*>(edges + (int64_t)bt.place_begin + min(my_place, max(bt.places - 1, 0)));
   };
-  auto load_edges = [&](const Batch& bt) {  // beyond the batch's last edge: that one again
-    EdgesG r;
-#pragma unroll
-    for (int k = 0; k < NLOAD; ++k) {
-      const int e = k * RPI + gr;
-      // (one 16-byte load; taken apart field by field it becomes two)
-      const uint4 rec = *reinterpret_cast<const uint4*>(Eb + (bt.edge_off + 16u * (uint32_t)min(e, max(bt.nedges - 1, 0))));
-      r.src[k] = (int32_t)rec.x;
-      r.w[k] = reinterpret_cast<const float*>((uintptr_t)rec.z | ((uintptr_t)rec.w << 32));
-    }
+  struct Rows {
+    f32x4 x[kChain];  // place k of the lane group's column
+    float w;          // of the lane's own place
+    uint32_t chain;   // of the lane's own place
+  };
+  const uint32_t no_chunk = chunk_live ? 0u : 0xfffffff0u;
+  auto load_rows = [&](const u32x3& rec, int places) {  // rec: {src, w_lo, w_hi} of EdgeF32
+    Rows r;
+    r.w = *reinterpret_cast<GlobalF32*>((uintptr_t)rec.y | ((uintptr_t)(rec.z & 0xffffu) << 32));
+    const bool live = my_place < places;
+    r.chain = live ? rec.z >> 16 : (uint32_t)(EMAX + 1);
+    // no edge or no such inputs: behind the end of X, which reads as zeros
+    const uint32_t off = live && rec.x != kUnused ? rec.x * row_bytes : kBehindX;
+    static_for_chain([&](auto K) {
+      const uint32_t at = (uint32_t)at_place<KS, decltype(K)::value>((int)off);
+      r.x[K] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(Xr, (at + 16u * gc) | no_chunk, 0, 0));
+    });
     return r;
   };
-  struct RowsG {
-    float w[NLOAD];
-    float4 x[NLOAD];
-  };
-  auto load_rows = [&](const EdgesG& eg) {
-    RowsG r;
-#pragma unroll
-    for (int k = 0; k < NLOAD; ++k) {
-      r.w[k] = *reinterpret_cast<GlobalF32*>(reinterpret_cast<uintptr_t>(eg.w[k]));
-      r.x[k] = *reinterpret_cast<const float4*>(Xb + ((uint32_t)eg.src[k] * row_bytes + x_off));
-    }
-    return r;
-  };
-  auto load_pair = [&](const Batch& bt) { return pinfo[bt.pair_begin + (i < bt.npairs ? (uint32_t)i : 0u)]; };
-
-  auto load_w = [&](float4 (&wq)[NT][KS][2], int rel) {  // B operands of `rel`, in lane order
-    const float4* wrel = Wp + (int64_t)rel * (NT * KS * 2 * 64) + lane;
+  // lane (i, q): the word of pair i, and, i < 4, the word of pair 4 q + i
+  auto load_pair = [&](int bi) { return pinfo[(int64_t)min(bi, total_batches - 1) * kBatch + i]; };
+  auto load_row = [&](int bi) { return pinfo[(int64_t)min(bi, total_batches - 1) * kBatch + (4 * q + (i & 3))]; };
+  bf16x8 wq[NT][KS][3];  // W operands of the batch, three terms each
+  auto load_w = [&](int rel) {
+    const bf16x8* wrel = Wp + (int64_t)rel * (NT * KS * 3 * 64) + lane;
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) wq[nt][s][c] = wrel[((nt * KS + s) * 2 + c) * 64];
+        for (int k = 0; k < 3; ++k) wq[nt][s][k] = wrel[((nt * KS + s) * 3 + k) * 64];
   };
 
-  // The pipeline.  Everything a batch needs is requested two of the wavefront's batches ahead of
-  // its use -- the record of batch j + 6 (so that its scalars exist at j + 4), the edge records of
-  // j + 4 (so that the rows of X of j + 2 can be requested at j), the rows, pair words and W
-  // operands of j + 2 -- into two sets of registers, one for the even and one for the odd batches:
-  // a set's registers are reloaded right after their last use, nothing in flight is ever copied,
-  // and the loop is unrolled by two.
-  struct Stage {
-    RowsG rw;              // rows of X and weights of batch j
-    EdgesG eg;             // edge records of batch j + 2
-    BatchF32 raw;          // record of batch j + 4
-    uint32_t pw;           // pair word of batch j
-    float4 wq[NT][KS][2];  // W operands of batch j
-  };
-  Batch bt0 = scalars(raw_batch(b), b), bt1 = scalars(raw_batch(b + 4), b + 4);
-  Batch bt2 = scalars(raw_batch(b + 8), b + 8), bt3 = scalars(raw_batch(b + 12), b + 12);
-  Stage even, odd;
-  even.raw = raw_batch(b + 16), odd.raw = raw_batch(b + 20);
-  even.eg = load_edges(bt2), odd.eg = load_edges(bt3);
-  even.pw = load_pair(bt0), odd.pw = load_pair(bt1);
-  load_w(even.wq, bt0.rel);
-  load_w(odd.wq, bt1.rel);
-  {
-    const EdgesG eg0 = load_edges(bt0), eg1 = load_edges(bt1);
-    even.rw = load_rows(eg0), odd.rw = load_rows(eg1);
-  }
+  // The pipeline: at batch j the record of batch j + 3 is requested, the edge records of j + 2, the rows of
+  // X, weights, pair words and W operands of j + 1.  One set of registers: what a batch holds is used up
+  // before the next one's is requested into it, and the other wavefronts of the SIMD cover the rest.
+  Batch bt0 = scalars(raw_batch(b), b), bt1 = scalars(raw_batch(b + WAVES), b + WAVES);
+  BatchF32 raw = raw_batch(b + 2 * WAVES);
+  Rows rw = load_rows(load_record(bt0), bt0.places);
+  u32x3 rec = load_record(bt1);
+  uint32_t pw = load_pair(b), pr = load_row(b);
+  load_w(bt0.rel);
+  __syncthreads();
 
-  auto batch = [&](Stage& st) {
-    // 1. the weighted rows of this batch, into the edge tile.  Places behind the batch's last edge
-    // get whatever was read: no pair reads them.  Chunks beyond feat_in are never written and stay
-    // zero.
-    if (chunk_live) {
+  while (bt0.npairs > 0) {  // the same for every lane
+    // 1. the chains of this batch: a lane group adds up its column of weighted rows, and writes a row of the
+    // chain tile wherever a chain ends
+    f32x4 run = {0.f, 0.f, 0.f, 0.f};
+    static_for_chain([&](auto K) {
+      const float w = __int_as_float(at_place<KS, decltype(K)::value>(__float_as_int(rw.w)));
+      const uint32_t chain = (uint32_t)at_place<KS, decltype(K)::value>((int)rw.chain);
 #pragma unroll
-      for (int k = 0; k < NLOAD; ++k) {
-        const float w = st.rw.w[k];
-        float4 v = st.rw.x[k];
-        v.x *= w, v.y *= w, v.z *= w, v.w *= w;
-        *reinterpret_cast<float4*>(et + (k * RPI + gr) * SS + 4 * gc) = v;
+      for (int c = 0; c < 4; ++c) {
+        if constexpr (K == 0)
+          run[c] = w * rw.x[K][c];
+        else
+          run[c] = fmaf(w, rw.x[K][c], chain >= 256 ? run[c] : 0.f);
       }
-    }
+      *reinterpret_cast<f32x4*>(et + __umul24(chain & 255, SS) + 4 * gc) = run;
+    });
     // requests for the batches to come
-    st.rw = load_rows(st.eg);
-    const Batch bt4 = scalars(st.raw, b + 16);
-    st.eg = load_edges(bt4);
-    st.raw = raw_batch(b + 24);
-    // 2. the sums of the pairs, multiplying layout: lane (i, q) walks the edges of pair i; a lane
-    // whose pair has fewer edges than the batch's longest reads the tile's row of zeros meanwhile
-    const uint32_t pw = st.pw;
-    const int my_first = (int)((pw >> 16) & 255u), my_count = i < bt0.npairs ? (int)((pw >> 8) & 255u) : 0;
-    const int my_dl = (int)(pw & (kTileRows - 1));
-    float4 sq[KS][2];
-    {  // every pair has a first edge; a lane without a pair takes the row of zeros
-      const float* row = et + (my_count > 0 ? my_first : EMAX) * SS + 8 * q;
+    rw = load_rows(rec, bt1.places);
+    const Batch bt2 = scalars(raw, b + 2 * WAVES);
+    rec = load_record(bt2);
+    raw = raw_batch(b + 3 * WAVES);
+    // 2. the sums of the pairs, multiplying layout: lane (i, q) adds the chains of pair i, mostly one; a lane
+    // whose pair has fewer than the batch's longest reads the tile's row of zeros meanwhile
+    const int my_count = (int)((pw >> 8) & 255u);
+    const uint32_t next_pw = load_pair(b + WAVES), next_pr = load_row(b + WAVES);
+    const char* first = reinterpret_cast<const char*>(et + 8 * q) + (pw >> 16);
+    float sum[KS][8];
 #pragma unroll
-      for (int s = 0; s < KS; ++s)
+    for (int s = 0; s < KS; ++s)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) sq[s][c] = *reinterpret_cast<const float4*>(row + 32 * s + 4 * c);
-    }
+      for (int c = 0; c < 2; ++c) {
+        const float4 v = reinterpret_cast<const float4*>(first)[8 * s + c];
+        sum[s][4 * c] = v.x, sum[s][4 * c + 1] = v.y, sum[s][4 * c + 2] = v.z, sum[s][4 * c + 3] = v.w;
+      }
+#pragma unroll 1
     for (int t = 1; t < bt0.most; ++t) {  // the same for every lane
-      const float* row = et + (t < my_count ? my_first + t : EMAX) * SS + 8 * q;
+      const char* row = t < my_count ? first + t * (4 * SS) : reinterpret_cast<const char*>(et + EMAX * SS + 8 * q);
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-          const float4 v = *reinterpret_cast<const float4*>(row + 32 * s + 4 * c);
-          sq[s][c].x += v.x, sq[s][c].y += v.y, sq[s][c].z += v.z, sq[s][c].w += v.w;
+          const float4 v = reinterpret_cast<const float4*>(row)[8 * s + c];
+          sum[s][4 * c] += v.x, sum[s][4 * c + 1] += v.y, sum[s][4 * c + 2] += v.z, sum[s][4 * c + 3] += v.w;
         }
     }
-    // 3. times W[rel]^T
+    // 3. times W[rel]^T, on the bf16 matrix cores: both factors are three terms, and of the nine products the
+    // six above 2^-24 of the whole are added, small ones first.  v_mfma_f32_16x16x4_f32 would keep the vector
+    // unit waiting for its 32 clocks (measured: the two add up, a bf16 product of twice the size costs it 9),
+    // and this loop needs the vector unit most of the time.
     f32x4 acc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s = 0; s < KS; ++s)
+    for (int s = 0; s < KS; ++s) {
+      bf16x8 a[3];
+      split3(sum[s], a);
+      constexpr int kTerms[6][2] = {{0, 2}, {2, 0}, {1, 1}, {0, 1}, {1, 0}, {0, 0}};
 #pragma unroll
-      for (int c = 0; c < 2; ++c)
+      for (int p = 0; p < 6; ++p)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const float4 wk = st.wq[nt][s][c], sk = sq[s][c];
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk.x, wk.x, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk.y, wk.y, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk.z, wk.z, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(sk.w, wk.w, acc[nt], 0, 0, 0);
-        }
-    load_w(st.wq, bt2.rel);
+        for (int nt = 0; nt < NT; ++nt)
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kTerms[p][0]], wq[nt][s][kTerms[p][1]], acc[nt], 0, 0, 0);
+    }
+    load_w(bt1.rel);
     // 4. acc[nt][v]: pair 4 q + v of the batch, output 16 nt + i, which lives at float NT i + nt of
     // its row of the partial tile: a lane's NT outputs are neighbours, one read and one write.
     // The pairs of a batch end in different rows (a row cut into pieces has at most its last,
     // shorter piece in a batch with other pairs: a full piece fills a batch), so no two lanes
-    // update the same float.
+    // update the same float; the wavefronts take turns, in the order of the batches.  (LDS
+    // instructions of a wavefront execute in order: the turn goes on after the tile is written.)
+    while (__hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != b) __builtin_amdgcn_s_sleep(1);
+    asm volatile("" ::: "memory");
+    float* at[4];
+    static_for_chain([&](auto V) {
+      at[V] = yt + (__builtin_amdgcn_mov_dpp((int)pr, 0x150 + decltype(V)::value, 0xf, 0xf, false) & 255) * FO + NT * i;
+    });
+    float old[4][NT];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int dl = __shfl(my_dl, 4 * q + v, 64);
-      if (4 * q + v < bt0.npairs) {
-        float* at = yt + dl * FO + NT * i;
-        if constexpr (NT == 2) {
-          float2 o = *reinterpret_cast<float2*>(at);
-          o.x += acc[0][v], o.y += acc[1][v];
-          *reinterpret_cast<float2*>(at) = o;
-        } else {
-          float4 o = *reinterpret_cast<float4*>(at);
-          o.x += acc[0][v], o.y += acc[1][v], o.z += acc[2][v], o.w += acc[3][v];
-          *reinterpret_cast<float4*>(at) = o;
-        }
-      }
-    }
-    st.pw = load_pair(bt2);  // last: the old word's row number was in use until here
-    b += 4;
-    bt0 = bt1, bt1 = bt2, bt2 = bt3, bt3 = bt4;  // scalars: copies wait for nothing
-  };
-  // (With the way out between the two halves, the compiler's wait counts at the top of a round are
-  // "everything requested in the round before has arrived".  Without it -- both batches run
-  // whether the second exists or not, and the requests of the prologue waited for once before the
-  // loop -- the counts leave two batches' worth of loads in flight, and the launch is slower: 139
-  // against 130 us on 100k nodes / 65 relations / 2M edges.  The loop is bound by instruction
-  // issue, not by the latency of its loads.)
-  while (bt0.npairs > 0) {  // the same for every lane
-    batch(even);
-    if (bt0.npairs == 0) break;
-    batch(odd);
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) old[v][nt] = at[v][nt];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) at[v][nt] = old[v][nt] + acc[nt][v];
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(&turn, b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    pw = next_pw, pr = next_pr;
+    b += WAVES;
+    bt0 = bt1, bt1 = bt2;
   }
 
   __syncthreads();
+  // The tile's rows of Y are one stretch of memory.  A thread requests all it is about to add to before it
+  // waits for any of it: one element at a time this end of a unit took 13 round trips to memory.
   const int64_t row0 = (int64_t)u.tile * kTileRows;
   const int64_t stride = (int64_t)kTileRows * fout;
-  for (int e = tid; e < kTileRows * fout; e += 256) {
-    const int r = e / fout, c = e - r * fout;
-    if (row0 + r >= m) break;
-    const int at = r * FO + NT * (c & 15) + (c >> 4);
-    const float sum = (ytile[0][at] + ytile[1][at]) + (ytile[2][at] + ytile[3][at]);
-    if (u.partial < 0)
-      Y[(row0 + r) * fout + c] += sum;
-    else
-      __hip_atomic_store(partials + u.partial * stride + e, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const int count = (int)min((int64_t)kTileRows, m - row0) * fout;
+  float* Yt = Y + row0 * fout;
+  constexpr int AHEAD = 8;
+  const uint32_t inverse = (uint32_t)((0x100000000ull + fout - 1) / fout);  // exact quotients for these e
+  auto sum_at = [&](int e) {
+    const int r = fout > 1 ? (int)__umulhi((uint32_t)e, inverse) : e, c = e - r * fout;
+    return yt[r * FO + NT * (c & 15) + (c >> 4)];
+  };
+  if (u.partial < 0) {
+    for (int e0 = tid; e0 < count; e0 += AHEAD * THREADS) {
+      float old[AHEAD];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k) old[k] = Yt[min(e0 + k * THREADS, count - 1)];
+#pragma unroll
+      for (int k = 0; k < AHEAD; ++k)
+        if (e0 + k * THREADS < count) Yt[e0 + k * THREADS] = old[k] + sum_at(e0 + k * THREADS);
+    }
+    return;
   }
-  if (u.partial < 0) return;
+  for (int e = tid; e < count; e += THREADS)
+    __hip_atomic_store(partials + u.partial * stride + e, sum_at(e), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   // A piece of a tile.  Every wavefront waits until its stores have arrived, then one thread
   // counts the unit in; the unit that counts last finds the partial tiles of all the others in
   // memory (stores and loads of partial tiles pass the L2 of their XCD).
@@ -540,12 +626,27 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches,
   }
   __syncthreads();
   if (!last_of_tile) return;
-  for (int e = tid; e < kTileRows * fout; e += 256) {
-    if (row0 + e / fout >= m) break;
-    float sum = 0.f;
-    for (int p = 0; p < u.pieces; ++p)
-      sum += __hip_atomic_load(partials + (u.first_partial + p) * stride + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    Y[row0 * fout + e] += sum;
+  const float* all = partials + u.first_partial * stride;
+  for (int e0 = tid; e0 < count; e0 += AHEAD * THREADS) {
+    float old[AHEAD], sum[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) old[k] = Yt[min(e0 + k * THREADS, count - 1)], sum[k] = 0.f;
+    for (int p0 = 0; p0 < u.pieces; p0 += 4) {  // the pieces add up in their order
+      float v[4][AHEAD];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+          v[j][k] = __hip_atomic_load(all + min(p0 + j, u.pieces - 1) * stride + min(e0 + k * THREADS, count - 1),
+                                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) sum[k] += p0 + j < u.pieces ? v[j][k] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k)
+      if (e0 + k * THREADS < count) Yt[e0 + k * THREADS] = old[k] + sum[k];
   }
 }
 
@@ -576,16 +677,18 @@ bool f32_tiles_serves(int32_t feat_in, int32_t feat_out) {
 }
 
 bool f32_tiles_fits(int32_t n, int32_t feat_in, int64_t edges) {
-  return (int64_t)n * feat_in * 4 < (int64_t(1) << 32) && edges * 16 < (int64_t(1) << 32);
+  return (int64_t)n * feat_in * 4 <= (int64_t)kBehindX && edges < (int64_t(1) << 31);
 }
 
 void f32_tiles_free(F32TileIndex& idx) {
   if (idx.d_edges) (void)hipFree(idx.d_edges);
   if (idx.d_pairs) (void)hipFree(idx.d_pairs);
   if (idx.d_batches) (void)hipFree(idx.d_batches);
-  if (idx.d_units) (void)hipFree(idx.d_units);
-  if (idx.d_arrived) (void)hipFree(idx.d_arrived);
-  if (idx.d_partials) (void)hipFree(idx.d_partials);
+  for (F32Units& u : idx.units) {
+    if (u.d_units) (void)hipFree(u.d_units);
+    if (u.d_arrived) (void)hipFree(u.d_arrived);
+    if (u.d_partials) (void)hipFree(u.d_partials);
+  }
   if (idx.d_wpack) (void)hipFree(idx.d_wpack);
   idx = F32TileIndex();
 }
@@ -606,6 +709,58 @@ int f32_tiles_prepare(F32TileIndex& idx, const F32Source& src, int32_t m, int32_
 }
 
 namespace {
+// The units of a launch: whole tiles, or pieces of tiles of at most `cap` batches, longest first.  As many as
+// run at the same time: 4 workgroups per compute unit, 2 when feat_out is above 32 (wide), so that each takes
+// an equal part of the whole.  Fewer when there are few tiles -- most of them would be cut, and the last
+// piece of a tile adds up what all of them wrote (24 k nodes, 65 relations, 299 k edges: 26.8 us with 768
+// units, 30.0 with 1024, 36.8 uncut) -- and no pieces so short that filling the pipeline and the partial
+// tile cost more than they bring.  Wide launches with many tiles: two rounds (110 k nodes, 130
+// relations, 2 M edges, 64 -> 64: 334 us with 1024 units, 371 with 860 whole tiles).
+int make_units(F32Units& out, const std::vector<int64_t>& tile_begin, bool wide, hipStream_t stream) {
+  const int64_t tiles = (int64_t)tile_begin.size() - 1, cus = compute_units();
+  STIR_REQUIRE(cus > 0, "rgms_f32: no device");
+  const int64_t target = tiles > 2 * cus ? 4 * cus : (wide ? 2 : 3) * cus;
+  auto count_with = [&](int64_t cap) {
+    int64_t count = 0;
+    for (int64_t t = 0; t < tiles; ++t) count += ceil_div(tile_begin[(size_t)t + 1] - tile_begin[(size_t)t], cap);
+    return count;
+  };
+  int64_t cap = wide ? 48 : 24, top = std::max(tile_begin[(size_t)tiles], cap);
+  while (cap < top) {  // the shortest pieces that are not too many
+    const int64_t mid = (cap + top) / 2;
+    if (count_with(mid) <= target) top = mid; else cap = mid + 1;
+  }
+  std::vector<UnitF32> units;
+  int64_t partial_tiles = 0, cut_tiles = 0;
+  for (int64_t t = 0; t < tiles; ++t) {
+    const int64_t lo = tile_begin[(size_t)t], hi = tile_begin[(size_t)t + 1];
+    if (hi <= lo) continue;
+    if (hi - lo <= cap) {
+      units.push_back(UnitF32{(int32_t)t, (int32_t)lo, (int32_t)hi, -1, 0, 0, 0, 0});
+      continue;
+    }
+    const int64_t pieces = ceil_div(hi - lo, cap);
+    STIR_REQUIRE(partial_tiles + pieces < (int64_t(1) << 31), "rgms_f32: too many partial tiles");
+    for (int64_t p = 0; p < pieces; ++p)
+      units.push_back(UnitF32{(int32_t)t, (int32_t)(lo + (hi - lo) * p / pieces), (int32_t)(lo + (hi - lo) * (p + 1) / pieces),
+                              (int32_t)(partial_tiles + p), (int32_t)partial_tiles, (int32_t)pieces,
+                              (int32_t)cut_tiles, 0});
+    partial_tiles += pieces, ++cut_tiles;
+  }
+  std::stable_sort(units.begin(), units.end(), [](const UnitF32& a, const UnitF32& b) {
+    return a.batch_end - a.batch_begin > b.batch_end - b.batch_begin;
+  });
+  out.count = (int64_t)units.size(), out.partial_tiles = partial_tiles;
+  STIR_HIP(hipMalloc(&out.d_units, sizeof(UnitF32) * std::max<size_t>(units.size(), 1)));
+  STIR_HIP(hipMemcpy(out.d_units, units.data(), sizeof(UnitF32) * units.size(), hipMemcpyHostToDevice));
+  if (cut_tiles > 0) {  // the counters of the cut tiles: zero between launches
+    STIR_HIP(hipMalloc(&out.d_arrived, sizeof(uint32_t) * (size_t)cut_tiles));
+    STIR_HIP(hipMemsetAsync(out.d_arrived, 0, sizeof(uint32_t) * (size_t)cut_tiles, stream));
+    STIR_HIP(hipStreamSynchronize(stream));  // done before a launch on any stream
+  }
+  return 0;
+}
+
 int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, int32_t num_rels, int32_t emax,
                 hipStream_t stream) {
   STIR_REQUIRE(m > 0 && n > 0 && num_rels > 0, "rgms_f32: m, n and num_rels must be positive");
@@ -648,8 +803,8 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   const dim3 grid((unsigned)ceil_div(slots, 256)), block(256);
   const int nb = (int)tab.size();
   if (src.csf)
-    hipLaunchKernelGGL(f32_edge_keys_kernel<true>, grid, block, 0, stream, d_tab, nb, csf, slots, m, n, num_rels, keys_in,
-                       vals_in, flags);
+    hipLaunchKernelGGL(f32_edge_keys_kernel<true>, grid, block, 0, stream, d_tab, nb, csf, slots, m, n, num_rels,
+                       keys_in, vals_in, flags);
   else
     hipLaunchKernelGGL(f32_edge_keys_kernel<false>, grid, block, 0, stream, d_tab, nb, csf, slots, m, n, num_rels,
                        keys_in, vals_in, flags);
@@ -666,14 +821,6 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   size_t bytes = sort_bytes;
   STIR_HIP(hipcub::DeviceRadixSort::SortPairs(cub_tmp, bytes, keys_in, keys_out, vals_in, vals_out, (int)slots, 0,
                                               key_bits, stream));
-  STIR_HIP(hipMalloc(&idx.d_edges, sizeof(EdgeF32) * (size_t)slots));
-  if (src.csf)
-    hipLaunchKernelGGL(f32_edge_records_kernel<true>, grid, block, 0, stream, d_tab, nb, csf, slots, num_rels, vals_out,
-                       static_cast<EdgeF32*>(idx.d_edges));
-  else
-    hipLaunchKernelGGL(f32_edge_records_kernel<false>, grid, block, 0, stream, d_tab, nb, csf, slots, num_rels,
-                       vals_out, static_cast<EdgeF32*>(idx.d_edges));
-  STIR_LAUNCH_CHECK();
   // runs of equal key, cut into pieces of at most emax edges by a second key
   bytes = rle_bytes;
   STIR_HIP(hipcub::DeviceRunLengthEncode::Encode(cub_tmp, bytes, keys_out, unique, counts, flags + 1, (int)slots,
@@ -700,13 +847,16 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   idx.pairs = pairs;
   bytes = scan_bytes;
   STIR_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, bytes, counts, first, (int)pairs, stream));
-  // the (tile, relation) runs of pairs.  keys_out / vals_in / vals_out are free again; keys_in is
+  // the (tile, relation) runs of pairs.  keys_out and vals_in are free again; keys_in is
   // once the run-length encoding above has read it (same stream)
   uint64_t* run_of_pair = keys_out;
   uint64_t* run_keys = keys_in;
-  int32_t *run_pairs = vals_in, *run_first_pair = vals_out;
+  int32_t *run_pairs = vals_in, *run_first_pair = nullptr;
   int32_t *run_batches = nullptr, *run_first_batch = nullptr;
-  if (tmp.get(&run_batches, pairs + 1) || tmp.get(&run_first_batch, pairs + 1)) return -1;
+  int64_t *pair_place = nullptr, *run_places = nullptr, *run_first_place = nullptr;
+  if (tmp.get(&run_batches, pairs + 1) || tmp.get(&run_first_batch, pairs + 1) || tmp.get(&run_first_pair, pairs + 1) ||
+      tmp.get(&pair_place, pairs) || tmp.get(&run_places, pairs + 1) || tmp.get(&run_first_place, pairs + 1))
+    return -1;
   hipLaunchKernelGGL(f32_shift_keys_kernel, dim3((unsigned)ceil_div(pairs, 256)), block, 0, stream, unique, pairs,
                      run_of_pair);
   STIR_LAUNCH_CHECK();
@@ -725,97 +875,53 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   STIR_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, bytes, run_pairs, run_first_pair, (int)runs, stream));
   const dim3 run_grid((unsigned)ceil_div(runs, 256));
   hipLaunchKernelGGL(f32_batches_kernel<false>, run_grid, block, 0, stream, run_keys, run_pairs, run_first_pair,
-                     (const int32_t*)nullptr, runs, num_rels, (int)emax, unique, counts, first, run_batches,
-                     (BatchF32*)nullptr, (uint32_t*)nullptr);
+                     (const int32_t*)nullptr, runs, num_rels, (int)emax, unique, counts, run_batches, run_places,
+                     (const int64_t*)nullptr, (BatchF32*)nullptr, (uint32_t*)nullptr, (int64_t*)nullptr);
   STIR_LAUNCH_CHECK();
   // one entry more than runs: the last one is the batch count (run_batches[runs] is not read as an addend)
   STIR_HIP(hipMemsetAsync(run_batches + runs, 0, sizeof(int32_t), stream));
   bytes = scan2;
   STIR_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, bytes, run_batches, run_first_batch, (int)runs + 1, stream));
+  STIR_HIP(hipMemsetAsync(run_places + runs, 0, sizeof(int64_t), stream));
+  size_t scan3 = 0;
+  STIR_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan3, run_places, run_first_place, (int)runs + 1, stream));
+  STIR_REQUIRE(scan3 <= cub_bytes, "rgms_f32: scratch of the index build is too small");
+  STIR_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, scan3, run_places, run_first_place, (int)runs + 1, stream));
   int32_t total_batches = 0;
+  int64_t places = 0;
+  STIR_HIP(hipMemcpyAsync(&places, run_first_place + runs, sizeof(int64_t), hipMemcpyDeviceToHost, stream));
   STIR_HIP(hipMemcpyAsync(&total_batches, run_first_batch + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
   STIR_HIP(hipStreamSynchronize(stream));
   idx.batches = total_batches;
   STIR_HIP(hipMalloc(&idx.d_batches, sizeof(BatchF32) * (size_t)std::max<int64_t>(total_batches, 1)));
-  STIR_HIP(hipMalloc(&idx.d_pairs, sizeof(uint32_t) * (size_t)std::max<int64_t>(pairs, 1)));
+  const int64_t words = (int64_t)total_batches * kBatch;
+  STIR_HIP(hipMalloc(&idx.d_pairs, sizeof(uint32_t) * (size_t)std::max<int64_t>(words, 1)));
+  STIR_REQUIRE(places < (int64_t(1) << 32), "rgms_f32: too many edges");
+  STIR_HIP(hipMalloc(&idx.d_edges, sizeof(EdgeF32) * (size_t)std::max<int64_t>(places, 1)));
+  EdgeF32* d_places = static_cast<EdgeF32*>(idx.d_edges);
+  const float* some_weight = src.csf ? src.A : tab[0].A;
+  hipLaunchKernelGGL(f32_clear_places_kernel, dim3((unsigned)ceil_div(std::max(places, words), 256)), block, 0, stream,
+                     d_places, places, (int)emax, some_weight, static_cast<uint32_t*>(idx.d_pairs), words);
+  STIR_LAUNCH_CHECK();
   hipLaunchKernelGGL(f32_batches_kernel<true>, run_grid, block, 0, stream, run_keys, run_pairs, run_first_pair,
-                     run_first_batch, runs, num_rels, (int)emax, unique, counts, first, (int32_t*)nullptr,
-                     static_cast<BatchF32*>(idx.d_batches), static_cast<uint32_t*>(idx.d_pairs));
+                     run_first_batch, runs, num_rels, (int)emax, unique, counts, (int32_t*)nullptr,
+                     (int64_t*)nullptr, run_first_place, static_cast<BatchF32*>(idx.d_batches), static_cast<uint32_t*>(idx.d_pairs), pair_place);
+  STIR_LAUNCH_CHECK();
+  if (src.csf)
+    hipLaunchKernelGGL(f32_edge_records_kernel<true>, grid, block, 0, stream, d_tab, nb, csf, slots, num_rels,
+                       (int)emax, vals_out, first, counts, pair_place, pairs, d_places);
+  else
+    hipLaunchKernelGGL(f32_edge_records_kernel<false>, grid, block, 0, stream, d_tab, nb, csf, slots, num_rels,
+                       (int)emax, vals_out, first, counts, pair_place, pairs, d_places);
   STIR_LAUNCH_CHECK();
   hipLaunchKernelGGL(f32_tile_batches_kernel, dim3((unsigned)ceil_div(tiles + 1, 256)), block, 0, stream, run_keys,
                      run_first_batch, runs, (int64_t)total_batches, tiles, num_rels, tile_begin);
   STIR_LAUNCH_CHECK();
-  // units: a tile, or -- for a tile with more than 1.5 times `cap` batches -- pieces of at most
-  // `cap` batches, cap = twice the average of the tiles that have batches (at least 32)
   std::vector<int64_t> tb((size_t)tiles + 1);
   STIR_HIP(hipMemcpyAsync(tb.data(), tile_begin, sizeof(int64_t) * tb.size(), hipMemcpyDeviceToHost, stream));
   STIR_HIP(hipStreamSynchronize(stream));  // also: the scratch arrays go away
-  int64_t busy = 0;
-  for (int64_t t = 0; t < tiles; ++t) busy += tb[(size_t)t + 1] > tb[(size_t)t];
-  const int64_t cap = std::max<int64_t>(32, busy ? 2 * ceil_div((int64_t)total_batches, busy) : 32);
-  std::vector<UnitF32> units;
-  int64_t partial_tiles = 0, cut_tiles = 0;
-  for (int64_t t = 0; t < tiles; ++t) {
-    const int64_t lo = tb[(size_t)t], hi = tb[(size_t)t + 1];
-    if (hi <= lo) continue;
-    if (2 * (hi - lo) <= 3 * cap) {
-      units.push_back(UnitF32{(int32_t)t, (int32_t)lo, (int32_t)hi, -1, 0, 0, 0, 0});
-      continue;
-    }
-    const int64_t pieces = ceil_div(hi - lo, cap), len = ceil_div(hi - lo, pieces);
-    STIR_REQUIRE(partial_tiles + pieces < (int64_t(1) << 31), "rgms_f32: too many partial tiles");
-    for (int64_t p = 0; p < pieces; ++p)
-      units.push_back(UnitF32{(int32_t)t, (int32_t)(lo + p * len), (int32_t)std::min(hi, lo + (p + 1) * len),
-                              (int32_t)(partial_tiles + p), (int32_t)partial_tiles, (int32_t)pieces,
-                              (int32_t)cut_tiles, 0});
-    partial_tiles += pieces, ++cut_tiles;
-  }
-  // the longest units first
-  std::stable_sort(units.begin(), units.end(), [](const UnitF32& a, const UnitF32& b) {
-    return a.batch_end - a.batch_begin > b.batch_end - b.batch_begin;
-  });
-  // A few units beyond whole rounds of resident workgroups (three per CU) would run when the
-  // others are done, each as slowly as a unit alone: those are cut into four pieces that run side
-  // by side (100k nodes, 65 relations, 2M edges: 1563 units on 768 resident workgroups, 27 beyond
-  // two rounds; 133 -> 127 us).  Only when they are few and of ordinary length.
-  {
-    int dev = 0, cus = 0;
-    STIR_HIP(hipGetDevice(&dev));
-    STIR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const int64_t resident = 3 * (int64_t)cus, count = (int64_t)units.size();
-    const int64_t beyond = resident > 0 ? count % resident : 0;
-    constexpr int64_t kPieces = 4;  // 3 to 4 measured best; 6 and 8 give the gain back
-    if (count > resident && beyond > 0 && 8 * beyond <= resident) {
-      const int64_t ordinary = total_batches / (2 * count);  // half the average length
-      std::vector<UnitF32> cut;
-      int64_t kept = 0;
-      for (int64_t k = count - beyond; k < count; ++k) {
-        const UnitF32 whole = units[(size_t)k];
-        const int64_t lo = whole.batch_begin, hi = whole.batch_end;
-        if (whole.partial >= 0 || hi - lo < std::max<int64_t>(ordinary, 2 * kPieces) ||
-            partial_tiles + kPieces >= (int64_t(1) << 31)) {
-          units[(size_t)(count - beyond + kept++)] = whole;
-          continue;
-        }
-        const int64_t len = ceil_div(hi - lo, kPieces);
-        for (int64_t p = 0; p < kPieces; ++p)
-          cut.push_back(UnitF32{whole.tile, (int32_t)(lo + p * len), (int32_t)std::min(hi, lo + (p + 1) * len),
-                                (int32_t)(partial_tiles + p), (int32_t)partial_tiles, (int32_t)kPieces,
-                                (int32_t)cut_tiles, 0});
-        partial_tiles += kPieces, ++cut_tiles;
-      }
-      units.resize((size_t)(count - beyond + kept));
-      units.insert(units.end(), cut.begin(), cut.end());
-    }
-  }
-  idx.units = (int64_t)units.size(), idx.multi = cut_tiles, idx.partial_tiles = partial_tiles;
-  STIR_HIP(hipMalloc(&idx.d_units, sizeof(UnitF32) * std::max<size_t>(units.size(), 1)));
-  STIR_HIP(hipMemcpy(idx.d_units, units.data(), sizeof(UnitF32) * units.size(), hipMemcpyHostToDevice));
-  if (cut_tiles > 0) {  // the counters of the cut tiles: zero between launches
-    STIR_HIP(hipMalloc(&idx.d_arrived, sizeof(uint32_t) * (size_t)cut_tiles));
-    STIR_HIP(hipMemsetAsync(idx.d_arrived, 0, sizeof(uint32_t) * (size_t)cut_tiles, stream));
-    STIR_HIP(hipStreamSynchronize(stream));  // done before a launch on any stream
-  }
+  for (int wide = 0; wide < 2; ++wide)
+    if (make_units(idx.units[wide], tb, wide != 0, stream)) return -1;
   return 0;
 }
 }  // namespace
@@ -825,46 +931,50 @@ int f32_tiles_launch(F32TileIndex& idx, int32_t feat_in, int32_t feat_out, const
   STIR_REQUIRE(f32_tiles_serves(feat_in, feat_out), "rgms_f32: feature sizes %d -> %d are not served by the tiled kernel",
                feat_in, feat_out);
   STIR_REQUIRE(idx.emax == (feat_in <= 32 ? 32 : 16), "rgms_f32: the edge index was built for another feat_in");
-  if (idx.units == 0) return 0;
-  STIR_REQUIRE(idx.units < (int64_t(1) << 31), "rgms_f32: too many units for one launch");
+  F32Units& u = idx.units[feat_out > 32];
+  if (u.count == 0) return 0;
+  STIR_REQUIRE(u.count < (int64_t(1) << 31), "rgms_f32: too many units for one launch");
   // the kernel's 32-bit byte offsets
   STIR_REQUIRE(f32_tiles_fits(idx.n, feat_in, idx.edges),
                "rgms_f32: the tiled kernel addresses X and its index with 32-bit offsets");
-  const int ks = feat_in <= 32 ? 1 : 2, nt = feat_out <= 32 ? 2 : 4;
+  const int ks = feat_in <= 32 ? 1 : 2, nt = feat_out <= 16 ? 1 : feat_out <= 32 ? 2 : 4;
   // W in operand order, rewritten by every launch (W may change between launches)
-  const int64_t words = (int64_t)idx.num_rels * nt * ks * 2 * 64;
-  const size_t need = sizeof(float4) * (size_t)words;
+  const int64_t fragments = (int64_t)idx.num_rels * nt * ks * 64;
+  const size_t need = 3 * sizeof(bf16x8) * (size_t)fragments;
   if (need > idx.wpack_bytes) {
     if (idx.d_wpack) STIR_HIP(hipFree(idx.d_wpack));
     idx.d_wpack = nullptr, idx.wpack_bytes = 0;
     STIR_HIP(hipMalloc(&idx.d_wpack, need));
     idx.wpack_bytes = need;
   }
-  const size_t partial_need = sizeof(float) * (size_t)idx.partial_tiles * kTileRows * (size_t)feat_out;
-  if (partial_need > idx.partial_bytes) {
-    if (idx.d_partials) STIR_HIP(hipFree(idx.d_partials));
-    idx.d_partials = nullptr, idx.partial_bytes = 0;
-    STIR_HIP(hipMalloc(&idx.d_partials, partial_need));
-    idx.partial_bytes = partial_need;
+  const size_t partial_need = sizeof(float) * (size_t)u.partial_tiles * kTileRows * (size_t)feat_out;
+  if (partial_need > u.partial_bytes) {
+    if (u.d_partials) STIR_HIP(hipFree(u.d_partials));
+    u.d_partials = nullptr, u.partial_bytes = 0;
+    STIR_HIP(hipMalloc(&u.d_partials, partial_need));
+    u.partial_bytes = partial_need;
   }
-  float4* wp = static_cast<float4*>(idx.d_wpack);
-  hipLaunchKernelGGL(f32_pack_w_kernel, dim3((unsigned)ceil_div(words, 256)), dim3(256), 0, stream, d_W, wp, words, nt, ks,
+  bf16x8* wp = static_cast<bf16x8*>(idx.d_wpack);
+  hipLaunchKernelGGL(f32_pack_w_kernel, dim3((unsigned)ceil_div(fragments, 256)), dim3(256), 0, stream, d_W, wp, fragments, nt, ks,
                      feat_in, feat_out);
   STIR_LAUNCH_CHECK();
-  const dim3 grid((unsigned)idx.units), block(256);  // longest units first: they go to whichever slot is free
-  const UnitF32* units = static_cast<const UnitF32*>(idx.d_units);
+  const dim3 grid((unsigned)u.count);  // longest units first: they go to whichever slot is free
+  const UnitF32* units = static_cast<const UnitF32*>(u.d_units);
   const BatchF32* bts = static_cast<const BatchF32*>(idx.d_batches);
   const uint32_t* pinfo = static_cast<const uint32_t*>(idx.d_pairs);
   const EdgeF32* edges = static_cast<const EdgeF32*>(idx.d_edges);
-  float* partials = static_cast<float*>(idx.d_partials);
+  float* partials = static_cast<float*>(u.d_partials);
 #define STIR_F32_TILE(KS, NT)                                                                                   \
-  hipLaunchKernelGGL((rgms_f32_tile_kernel<KS, NT>), grid, block, 0, stream, idx.m, feat_in, feat_out,          \
-                     (int)idx.batches, units, bts, pinfo, edges, wp, d_X, d_Y, partials,                        \
-                     static_cast<uint32_t*>(idx.d_arrived))
-  if (ks == 1) {
-    if (nt == 2) STIR_F32_TILE(1, 2); else STIR_F32_TILE(1, 4);
-  } else {
-    if (nt == 2) STIR_F32_TILE(2, 2); else STIR_F32_TILE(2, 4);
+  hipLaunchKernelGGL((rgms_f32_tile_kernel<KS, NT>), grid, dim3((64 * TileShape<KS, NT>::kWaves)), 0, stream, idx.m, \
+                     feat_in, feat_out, (int)idx.batches, (uint32_t)((int64_t)idx.n * feat_in * 4), units, bts,  \
+                     pinfo, edges, wp, d_X, d_Y, partials, static_cast<uint32_t*>(u.d_arrived))
+  switch (ks * 10 + nt) {
+    case 11: STIR_F32_TILE(1, 1); break;
+    case 12: STIR_F32_TILE(1, 2); break;
+    case 14: STIR_F32_TILE(1, 4); break;
+    case 21: STIR_F32_TILE(2, 1); break;
+    case 22: STIR_F32_TILE(2, 2); break;
+    default: STIR_F32_TILE(2, 4); break;
   }
 #undef STIR_F32_TILE
   STIR_LAUNCH_CHECK();

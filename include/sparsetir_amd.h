@@ -383,7 +383,7 @@ int stir_tc_plan_destroy(stir_tc_plan* plan);
  * launch with given feature sizes a work list for them (both allocate and synchronise the
  * stream; later launches do neither).  W is read anew at every launch.  W that does not fit the
  * LDS of a compute unit beside the kernel's tiles (about 130 KB: 65 relations of 32 x 32) is
- * served as up to three ranges of relations, each with an index and a launch of its own.  With
+ * served as two ranges of relations (when there are edges enough), each with an index and a launch of its own.  With
  * more relations than that, with feat_in above 64 or a d_W that is not 16-byte aligned, every
  * launch rewrites a packed copy of W held by the plan; a plan therefore serves one call at a
  * time.

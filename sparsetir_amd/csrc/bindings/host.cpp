@@ -234,9 +234,10 @@ PyObject* forget(PyObject* self, PyObject* name) {
   Py_RETURN_NONE;
 }
 
-// new_hyb_plan(args) -> (name, plan) for arguments launch() did not know, None when they are not the
-// ordinary ones, -1 when the C ABI refused.  The name is the properties the plan depends on.
-PyObject* new_hyb_plan(PyObject* self, PyObject* args) {
+// launch_new_hyb(args) -> (name, plan) of a new plan for arguments launch() did not know, remembered and
+// launched; None when they are not the ordinary ones, -1 when the C ABI refused.  The name is the properties the
+// plan depends on.
+PyObject* launch_new_hyb(PyObject* self, PyObject* args) {
   Launcher* l = reinterpret_cast<Launcher*>(self);
   stir_hyb_plan* plan = nullptr;
   try {
@@ -268,11 +269,27 @@ PyObject* new_hyb_plan(PyObject* self, PyObject* args) {
                               nrows.data(), A.data(), rows.data(), cols.data());
     Py_END_ALLOW_THREADS
     if (rc != 0) return PyLong_FromLong(kFailed);
+    l->plans->insert(l->plans->begin(), Plan{plan, (int)device, std::vector<int64_t>(key.begin() + 1, key.end()), nullptr});
+    void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    Py_BEGIN_ALLOW_THREADS
+    rc = call(l, p, plan, nullptr, st);
+    Py_END_ALLOW_THREADS
+    Plan& made = l->plans->front();
+    if (rc == 0)
+      made.name = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key.data()),
+                                            (Py_ssize_t)(key.size() * sizeof(int64_t)));
+    PyObject* out = made.name ? Py_BuildValue("(OK)", made.name, reinterpret_cast<unsigned long long>(plan)) : nullptr;
+    if (!out) {  // nobody would own the plan
+      Py_XDECREF(made.name);
+      l->plans->erase(l->plans->begin());
+      stir_hyb_plan_destroy(plan);
+      return rc == 0 ? nullptr : PyLong_FromLong(kFailed);
+    }
+    return out;
   } catch (...) {
+    if (plan) stir_hyb_plan_destroy(plan);
     Py_RETURN_NONE;
   }
-  return Py_BuildValue("(y#K)", reinterpret_cast<const char*>(l->key->data()),
-                       (Py_ssize_t)(l->key->size() * sizeof(int64_t)), reinterpret_cast<unsigned long long>(plan));
 }
 
 bool scalar_type(long code, c10::ScalarType* out) {
@@ -390,7 +407,7 @@ void launcher_dealloc(PyObject* self) {
 PyMethodDef launcher_methods[] = {
     {"launch", launch, METH_O, "launch(args) -> 0: launched, -1: refused, 1: not taken, or the name of the plan"},
     {"remember", remember, METH_VARARGS, "remember(args, plan, name): a plan made from these arguments"},
-    {"new_hyb_plan", new_hyb_plan, METH_O, "new_hyb_plan(args) -> (name, plan), None: not taken, -1: refused"},
+    {"launch_new_hyb", launch_new_hyb, METH_O, "launch_new_hyb(args) -> (name, plan), None: not taken, -1: refused"},
     {"forget", forget, METH_O, "forget(name): the plan is no more; None: all of them"},
     {"hyb", launcher_hyb, METH_VARARGS | METH_STATIC, "hyb(n, m, feat, parts, buckets, nrows): launcher of the hyb operator"},
     {nullptr, nullptr, 0, nullptr}};

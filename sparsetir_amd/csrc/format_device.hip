@@ -16,6 +16,7 @@
 // histogram plus the rank inside the wavefront, write row ids and padding; (4) scatter the
 // column ids and the mask, eight consecutive nonzeros per thread.
 #include <cstring>
+#include <utility>
 #include <mutex>
 #include <vector>
 
@@ -749,11 +750,22 @@ struct OneOutputs {
   int32_t* mask[kOneBuckets];
   float* a[kOneBuckets];  // null without values
 };
-// In host memory, written by the kernels.
+// In host memory, written by the kernels.  rows[b]: the ELL rows of bucket b below the number of the call, one
+// 8-byte store that needs no order with another.  The host watches for it: waiting for the stream takes 5 us
+// more, from the end of the kernel to the wake-up.
 struct OneAnswer {
-  int64_t nrows[kOneBuckets];
-  int32_t bad_range, bad_indptr;
+  uint64_t rows[kOneBuckets];
+  int32_t bad_range, bad_indptr;  // there before the rows
 };
+constexpr int kCallShift = 40;  // rows of a bucket are fewer
+__device__ __forceinline__ void answer_rows(OneAnswer* answer, int b, int64_t nrows, uint32_t number) {
+  __hip_atomic_store(&answer->rows[b], (uint64_t)nrows | ((uint64_t)number << kCallShift), __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// (a plain store would stay in the L2 of the XCD until the end of the kernel)
+__device__ __forceinline__ void answer_bad(int32_t* what) {
+  __hip_atomic_store(what, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // The nonzeros [first, first + nnz) as indptr has them; none when it contradicts itself or the length
 // of `indices` (reported as bad_indptr).
@@ -771,13 +783,66 @@ __device__ __forceinline__ OneEnds one_ends(const int32_t* __restrict__ indptr, 
 }
 __device__ __forceinline__ int64_t one_stride(int64_t nnz) { return nnz > kCoarse ? (nnz + kCoarse - 1) / kCoarse : 1; }
 
+// Exclusive scan of hist[b][0 .. W) by one wavefront, W at most 4 * 64, for a workgroup of four wavefronts; the
+// counts were written by other workgroups of the same launch.
+__device__ __forceinline__ void scan_few(int64_t W, int NB, int32_t* __restrict__ hist, OneAnswer* answer,
+                                         uint32_t number) {
+  constexpr int kMost = kOneBuckets / 4;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int32_t v[kMost][4];
+#pragma unroll
+  for (int k = 0; k < kMost; ++k)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t w = lane * 4 + j;
+      v[k][j] = wave + 4 * k < NB && w < W
+                    ? __hip_atomic_load(hist + (wave + 4 * k) * W + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                    : 0;
+    }
+#pragma unroll
+  for (int k = 0; k < kMost; ++k) {
+    const int b = wave + 4 * k;
+    if (b >= NB) break;
+    const int sum = v[k][0] + v[k][1] + v[k][2] + v[k][3];
+    int incl = sum;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int up = __shfl_up(incl, off, kWave);
+      if (lane >= off) incl += up;
+    }
+    int run = incl - sum;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (lane * 4 + j < W) hist[b * W + lane * 4 + j] = run;
+      run += v[k][j];
+    }
+    if (lane == kWave - 1) answer_rows(answer, b, incl, number);
+  }
+}
+constexpr int64_t kFewCounts = 256;  // entries per bucket (16 384 rows) that the last workgroup scans itself
+
 // Workgroups below count_blocks count the rows (as count_kernel), the others check that columns lie in
-// range, kValidatePerThread per thread.
+// range, kValidatePerThread per thread.  arrived: null, or a counter that is zero between launches; the
+// workgroup that finishes last then scans the counts (at most kFewCounts per bucket): a launch less, 4 us.
 __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int NB, int64_t W, int64_t max_nnz,
                                                         int count_blocks, OneWidths widths, Workspace ws,
                                                         const int32_t* __restrict__ indptr,
                                                         const int32_t* __restrict__ indices,
-                                                        OneAnswer* __restrict__ answer) {
+                                                        OneAnswer* __restrict__ answer,
+                                                        uint32_t* __restrict__ arrived, uint32_t number) {
+  auto finish = [&]() {  // by every thread of the workgroup
+    if (!arrived) return;
+    __shared__ int last;
+    // the counts have passed the L2 of this XCD, and the host has what was wrong
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      last = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == gridDim.x;
+      if (last) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (last) scan_few(W, NB, ws.hist, answer, number);
+  };
   const OneEnds ends = one_ends(indptr, m, max_nnz);
   const int64_t end = ends.first + ends.nnz;
   if ((int)blockIdx.x >= count_blocks) {
@@ -797,23 +862,23 @@ __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int
       for (int j = 0; j < N; ++j)
         if (e0 + j < end) bad |= (uint32_t)indices[e0 + j] >= (uint32_t)num_cols;
     }
-    if (bad) answer->bad_range = 1;
+    if (bad) answer_bad(&answer->bad_range);
+    finish();
     return;
   }
   if (blockIdx.x == 0) {
-    if (threadIdx.x == 0 && ends.bad) answer->bad_indptr = 1;
+    if (threadIdx.x == 0 && ends.bad) answer_bad(&answer->bad_indptr);
     if ((int)threadIdx.x < NB) ws.widths[threadIdx.x] = widths.w[threadIdx.x];
   }
   const int i = blockIdx.x * 256 + threadIdx.x;
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wave >= W) return;
   const int64_t stride = one_stride(ends.nnz);
   int d = 0;
   if (i < m) {
     int rs = indptr[i], re = indptr[i + 1];
     if (re < rs || rs < ends.first || re > end) {
-      if (!ends.bad) answer->bad_indptr = 1;
+      if (!ends.bad) answer_bad(&answer->bad_indptr);
       rs = re = ends.first;
     }
     for (int64_t q = (rs - ends.first + stride - 1) / stride; ends.first + q * stride < re; ++q) ws.coarse[q] = i;
@@ -823,19 +888,23 @@ __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int
   const int beta = bucket_of_dev(widths.w, NB, d);
   const int rho = d == 0 ? 0 : (d + widths.w[beta] - 1) / widths.w[beta];
   int32_t* h = ws.hist + wave;  // [b][W]
+  auto put = [&](int b, int32_t v) {
+    if (lane == 0 && wave < W) __hip_atomic_store(h + b * W, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
   for (int b = 0; b < NB - 1; ++b) {
     const unsigned long long bal = __ballot(d > 0 && beta == b);
-    if (lane == 0) h[b * W] = __popcll(bal);
+    put(b, __popcll(bal));
   }
   int tot = beta == NB - 1 ? rho : 0;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off, kWave);
-  if (lane == 0) h[(NB - 1) * W] = tot;
+  put(NB - 1, tot);
+  finish();
 }
 
 // Exclusive scan of hist[b][.] by one workgroup per bucket, a tile after the other.
 __global__ __launch_bounds__(256) void one_scan_kernel(int64_t W, int32_t* __restrict__ hist,
-                                                       OneAnswer* __restrict__ answer) {
+                                                       OneAnswer* __restrict__ answer, uint32_t number) {
   __shared__ int64_t red[4];
   int32_t* h = hist + (int64_t)blockIdx.x * W;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -868,12 +937,13 @@ __global__ __launch_bounds__(256) void one_scan_kernel(int64_t W, int32_t* __res
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) answer->nrows[blockIdx.x] = carry;
+  if (threadIdx.x == 0) answer_rows(answer, blockIdx.x, carry, number);
 }
 constexpr int64_t kOneScanMax = 16384;  // entries per bucket (a million rows); beyond, the three scan kernels
 
-__global__ void one_totals_kernel(int NB, const int64_t* __restrict__ totals, OneAnswer* __restrict__ answer) {
-  if ((int)threadIdx.x < NB) answer->nrows[threadIdx.x] = totals[threadIdx.x];
+__global__ void one_totals_kernel(int NB, const int64_t* __restrict__ totals, OneAnswer* __restrict__ answer,
+                                  uint32_t number) {
+  if ((int)threadIdx.x < NB) answer_rows(answer, threadIdx.x, totals[threadIdx.x], number);
 }
 
 __global__ __launch_bounds__(256) void one_rows_kernel(int m, int NB, int64_t W, Workspace ws, OneOutputs out,
@@ -917,18 +987,21 @@ __global__ __launch_bounds__(256) void one_place_kernel(int m, int num_cols, int
       });
 }
 
-// Host memory the kernels write their answer to: one block per thread, which waits for the answer
-// before it returns.
+// Host memory the kernels write their answer to and, per GPU, the counter of their workgroups: one of each per
+// thread, which waits for the answer before it returns.
 struct AnswerBox {
   OneAnswer* host = nullptr;
   OneAnswer* device = nullptr;
+  uint32_t number = 0;
+  std::vector<std::pair<int, uint32_t*>> arrived;
   ~AnswerBox() {
     if (host) (void)hipHostFree(host);
+    for (auto& a : arrived) (void)hipFree(a.second);
   }
 };
 thread_local AnswerBox t_answer;
 
-int answer_box(const char* who, AnswerBox** out) {
+int answer_box(const char* who, AnswerBox** out, uint32_t** arrived) {
   if (!t_answer.host) {
     void *h = nullptr, *d = nullptr;
     STIR_HIP(hipHostMalloc(&h, sizeof(OneAnswer), hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent));
@@ -939,8 +1012,35 @@ int answer_box(const char* who, AnswerBox** out) {
     }
     t_answer.host = static_cast<OneAnswer*>(h);
     t_answer.device = static_cast<OneAnswer*>(d);
+    std::memset(h, 0, sizeof(OneAnswer));
+  }
+  int device = -1;
+  STIR_HIP(hipGetDevice(&device));
+  *arrived = nullptr;
+  for (const auto& a : t_answer.arrived)
+    if (a.first == device) *arrived = a.second;
+  if (!*arrived) {
+    void* p = nullptr;
+    STIR_HIP(hipMalloc(&p, sizeof(uint32_t)));
+    t_answer.arrived.emplace_back(device, static_cast<uint32_t*>(p));
+    STIR_HIP(hipMemset(p, 0, sizeof(uint32_t)));
+    STIR_HIP(hipDeviceSynchronize());
+    *arrived = static_cast<uint32_t*>(p);
   }
   *out = &t_answer;
+  return 0;
+}
+
+// Until the answer for `buckets` buckets is there: at most some 100 us of watching, then the stream's own wait
+// (which also reports what went wrong with it).
+int wait_for_answer(const AnswerBox& box, int buckets, hipStream_t st) {
+  int b = 0;
+  for (int turn = 0; turn < 20000; ++turn) {
+    while (b < buckets && (__atomic_load_n(&box.host->rows[b], __ATOMIC_ACQUIRE) >> kCallShift) == box.number) ++b;
+    if (b == buckets) return 0;
+    __builtin_ia32_pause();
+  }
+  STIR_HIP(hipStreamSynchronize(st));
   return 0;
 }
 
@@ -1265,27 +1365,31 @@ int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int
   const Workspace ws = carve(d_workspace, m, 1, NB);
   const int64_t W = stir::ceil_div(m, kWave);
   AnswerBox* box = nullptr;
-  if (answer_box(who, &box)) return -1;
+  uint32_t* arrived = nullptr;
+  if (answer_box(who, &box, &arrived)) return -1;
   box->host->bad_range = box->host->bad_indptr = 0;
+  const uint32_t number = box->number = (box->number + 1) & ((1u << (64 - kCallShift)) - 1);
+  const bool few = W <= kFewCounts;
   OneWidths widths = {};
   std::copy(buckets, buckets + NB, widths.w);
   const int64_t count_blocks = stir::ceil_div(m, 256);
   const int64_t check_blocks = stir::ceil_div(max_nnz, 256 * kValidatePerThread);
   STIR_REQUIRE(count_blocks + check_blocks < (int64_t(1) << 31), "%s: too many nonzeros for one launch", who);
   hipLaunchKernelGGL(one_count_kernel, dim3((unsigned)(count_blocks + check_blocks)), dim3(256), 0, st, m, num_cols,
-                     NB, W, max_nnz, (int)count_blocks, widths, ws, d_indptr, d_indices, box->device);
+                     NB, W, max_nnz, (int)count_blocks, widths, ws, d_indptr, d_indices, box->device, few ? arrived : nullptr, number);
   STIR_LAUNCH_CHECK();
-  if (W <= kOneScanMax) {
-    hipLaunchKernelGGL(one_scan_kernel, dim3((unsigned)NB), dim3(256), 0, st, W, ws.hist, box->device);
-  } else {
+  if (!few && W <= kOneScanMax) {
+    hipLaunchKernelGGL(one_scan_kernel, dim3((unsigned)NB), dim3(256), 0, st, W, ws.hist, box->device, number);
+  } else if (!few) {
     if (scan_hist(ws, 1, NB, W, st)) return -1;
-    hipLaunchKernelGGL(one_totals_kernel, dim3(1), dim3(kWave), 0, st, NB, ws.totals, box->device);
+    hipLaunchKernelGGL(one_totals_kernel, dim3(1), dim3(kWave), 0, st, NB, ws.totals, box->device,
+                       number);
   }
   STIR_LAUNCH_CHECK();
-  STIR_HIP(hipStreamSynchronize(st));
+  if (wait_for_answer(*box, NB, st)) return -1;
   STIR_REQUIRE(!box->host->bad_indptr, "%s: indptr is not a CSR row pointer of %lld nonzeros", who, (long long)max_nnz);
   STIR_REQUIRE(!box->host->bad_range, "%s: a column index lies outside [0, %d)", who, num_cols);
-  std::copy(box->host->nrows, box->host->nrows + NB, nrows);
+  for (int k = 0; k < NB; ++k) nrows[k] = (int64_t)(box->host->rows[k] & ((uint64_t(1) << kCallShift) - 1));
   for (int k = 0; k < NB; ++k)
     STIR_REQUIRE(nrows[k] < kMaxSlots / buckets[k], "%s: bucket %d holds too many slots", who, k);
   return 0;

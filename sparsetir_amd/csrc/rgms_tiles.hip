@@ -752,9 +752,14 @@ int bit_length(uint64_t x) {
 // LDS beside W).  16 would leave 128 registers per wavefront, which the kernel only just fits or
 // spills, and measured no faster where W left the room (60 relations of 32 x 32).
 constexpr int kResidentMaxQuads = 3;
-// W beyond the LDS: at most this many ranges of relations, each with a launch of its own; more
-// relations than that read W from memory in one launch
-constexpr int kMaxRelationParts = 3;
+// W beyond the LDS: two ranges of relations with a launch each when the edges make up for the second launch
+// and its fill of the LDS, else W is read from memory in one launch.  Two launches / one, us:
+//   40 k nodes, 280 k edges, 50 relations 32 -> 64: 64 / 39; 720 k edges, 90 relations 32 -> 32: 35.6 / 31.6;
+//   110 k nodes, 880 k edges, 24 relations 64 -> 64: 81 / 88; 1.98 M edges, 90 relations 32 -> 32: 57 / 65.
+// Three launches are never the faster form (65 relations 32 -> 64: 77 / 22 at 144 k edges, 116 / 111 at 1.98 M).
+constexpr int kMaxRelationParts = 2;
+// (fewer edges suffice where a relation's W is large, 64 -> 32 and up: every run of a step fetches it)
+inline int64_t relation_parts_slots(int feat_in, int feat_out) { return feat_in * feat_out >= 2048 ? 850000 : 1300000; }
 
 // Launches the resident kernel with `quads` x 4 wavefronts per workgroup.
 template <int KK, bool BF16, typename Rec, typename YT>
@@ -1116,6 +1121,8 @@ int tile_set_prepare(TileIndexSet& set, const std::vector<TileBucket>& buckets, 
   // Relations per part: all of them, unless W is too large for the LDS of a compute unit and a few
   // ranges of relations are not -- then every range gets an index and a launch of its own.
   int32_t per_part = num_rels;
+  int64_t slots = 0;
+  for (const TileBucket& b : buckets) slots += b.groups * b.rb * b.cb;
   if (feat_in % 16 == 0 && feat_in / 16 <= kLdsMaxKK && feat_out % 32 == 0 &&
       (int64_t)n * feat_in * 2 < (int64_t(1) << 32)) {
     const size_t rel_bytes = size_t(feat_out / 32) * (feat_in / 16) * 64 * sizeof(u32x4);
@@ -1123,7 +1130,8 @@ int tile_set_prepare(TileIndexSet& set, const std::vector<TileBucket>& buckets, 
     auto fit = [&](int quads) { return (int64_t)((lds_limit - size_t(quads) * 4 * kSBytes) / rel_bytes); };
     if (num_rels > fit(2) && fit(kResidentMaxQuads) > 0) {
       const int64_t parts = ceil_div((int64_t)num_rels, fit(kResidentMaxQuads));
-      if (parts <= kMaxRelationParts) per_part = (int32_t)ceil_div((int64_t)num_rels, parts);
+      if (parts <= kMaxRelationParts && slots >= relation_parts_slots(feat_in, feat_out))
+        per_part = (int32_t)ceil_div((int64_t)num_rels, parts);
     }
   }
   if (set.m == m && set.n == n && set.num_rels == num_rels && set.rels_per_part == per_part) return 0;

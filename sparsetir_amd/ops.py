@@ -250,14 +250,12 @@ class HybCsrMM(_Operator):
             pass
 
     def _call(self, *args):
-        made = self._host.new_hyb_plan(args)
+        made = self._host.launch_new_hyb(args)
         if made is not None:
             if made == -1:
                 _lib.check(made)
             name, plan = made
             self._plans.put(name, ctypes.c_void_p(plan), args[2:])  # the plan stores pointers into these arrays
-            self._host.remember(args, plan, name)
-            _lib.check(self._launch(args))
             return
         if self._spec_cache is None:
             self._spec_cache = self._spec()

@@ -41,10 +41,12 @@ struct F32Source {
 // What a launch's workgroups take, longest first: tiles or pieces of tiles, as ranges of batches.
 struct F32Units {
   int64_t count = 0, partial_tiles = 0;
-  void* d_units = nullptr;     // count x 32 bytes, and behind them
-  void* d_arrived = nullptr;   // a counter per tile cut into several units, zero between launches
-  void* d_partials = nullptr;  // their partial tiles, rewritten by every launch
-  size_t partial_bytes = 0;
+  void* d_units = nullptr;     // count x 32 bytes; the allocation goes on with
+  void* d_arrived = nullptr;   // a counter per tile cut into several units, zero between launches,
+  void* d_wpack = nullptr;     // W in the multiply's operand order, rewritten by every launch,
+  void* d_partials = nullptr;  // and the partial tiles of the cut tiles, rewritten by every launch
+  size_t wpack_bytes = 0;      // what they have room for
+  int32_t feat_out = 0;
 };
 
 struct F32TileIndex {
@@ -52,11 +54,10 @@ struct F32TileIndex {
   int64_t edges = 0, pairs = 0, batches = 0, tiles = 0;
   std::vector<int64_t> tile_begin;  // first batch of every tile, and the end
   F32Units units[2];           // for feat_out up to 32, and above; made by the first launch that needs them
-  void* d_edges = nullptr;     // places x 12 bytes: an edge each, or none
-  void* d_pairs = nullptr;     // batches x 16 x 4 bytes: a word per pair
-  void* d_batches = nullptr;   // batches x 16 bytes: up to 16 pairs and emax places of one (tile, relation) each
-  void* d_wpack = nullptr;     // W in the multiply's operand order, rewritten by every launch
-  size_t wpack_bytes = 0;
+  void* d_batches = nullptr;   // batches x 16 bytes: up to 16 pairs and emax places of one (tile, relation) each;
+                               // the allocation goes on with
+  void* d_pairs = nullptr;     // batches x 16 x 4 bytes: a word per pair,
+  void* d_edges = nullptr;     // and places x 12 bytes: an edge each, or none
 };
 
 // True when the kernel serves these feature sizes (else the caller keeps its other kernel).

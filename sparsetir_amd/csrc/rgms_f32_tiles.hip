@@ -247,40 +247,46 @@ __global__ __launch_bounds__(256) void f32_batches_kernel(const uint64_t* __rest
                                                           const int64_t* __restrict__ run_first_place,
                                                           BatchF32* __restrict__ batches, uint32_t* __restrict__ pinfo,
                                                           int64_t* __restrict__ pair_place) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int64_t i = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (i >= runs) return;
   const int np = run_pairs[i], fp = run_first_pair[i];
   const int rel = (int)(run_keys[i] % (uint64_t)num_rels);
-  int nb = 0;
-  int64_t base = FILL ? run_first_place[i] : 0;
-  for (int j = 0; j < np;) {
-    const int pb = j;
-    int place = 0, chains = 0, most = 0;
-    do {
-      const int c = min(pair_edges[fp + j], emax);
+  int64_t base = FILL ? run_first_place[i] : 0;  // first place of the batch in hand
+  int64_t number = FILL ? run_first_batch[i] : 0;
+  int nb = 0, pairs = 0, place = 0, chains = 0, most = 0;
+  auto close = [&]() {
+    if (FILL && lane == 0)
+      batches[number] = BatchF32{(uint32_t)base, (uint32_t)pairs | ((uint32_t)most << 8) | ((uint32_t)place << 16), rel, 0};
+    base += place, ++number, ++nb;
+    pairs = place = chains = most = 0;
+  };
+  // 64 pairs at a time, one per lane: the wavefront goes through them together (one thread per run would wait
+  // for memory at every pair), lane k keeps what came out for pair k
+  for (int j0 = 0; j0 < np; j0 += 64) {
+    const int count = min(64, np - j0);
+    const int mine = lane < count ? min(pair_edges[fp + j0 + lane], emax) : 0;
+    int my_pair = 0, my_place = 0, my_chain = 0;
+    int64_t my_number = 0, my_base = 0;
+    for (int k = 0; k < count; ++k) {
+      const int c = __builtin_amdgcn_readlane(mine, k);
       int at = place;
       if (at % kChain + c > kChain) at = (at + kChain - 1) / kChain * kChain;
-      if (j > pb && (j - pb == kBatch || at + c > emax)) break;
-      const int mine = (c + kChain - 1) / kChain;
-      if (FILL) {
-        const uint32_t dl = (uint32_t)((pair_keys[fp + j] >> kSubBits) & (kTileRows - 1));
-        pinfo[((int64_t)run_first_batch[i] + nb) * kBatch + (j - pb)] =
-            dl | ((uint32_t)mine << 8) | ((uint32_t)chains * chain_row_bytes(emax) << 16);
-        pair_place[fp + j] = ((base + at) << 8) | chains;
-      }
-      place = at + c, chains += mine, most = max(most, mine), ++j;
-    } while (j < np);
-    if (FILL) {
-      BatchF32 b;
-      b.place_begin = (uint32_t)base;
-      b.counts = (uint32_t)(j - pb) | ((uint32_t)most << 8) | ((uint32_t)place << 16);
-      b.rel = rel;
-      b.pad = 0;
-      batches[run_first_batch[i] + nb] = b;
+      if (pairs > 0 && (pairs == kBatch || at + c > emax)) close(), at = 0;
+      if (FILL && lane == k) my_pair = pairs, my_place = at, my_chain = chains, my_number = number, my_base = base;
+      const int own = (c + kChain - 1) / kChain;
+      place = at + c, chains += own, most = max(most, own), ++pairs;
     }
-    base += place, ++nb;
+    if (FILL && lane < count) {
+      const int j = fp + j0 + lane;
+      const uint32_t dl = (uint32_t)((pair_keys[j] >> kSubBits) & (kTileRows - 1));
+      pinfo[my_number * kBatch + my_pair] =
+          dl | ((uint32_t)((mine + kChain - 1) / kChain) << 8) | ((uint32_t)my_chain * chain_row_bytes(emax) << 16);
+      pair_place[j] = ((my_base + my_place) << 8) | my_chain;
+    }
   }
-  if (!FILL) run_batches[i] = nb, run_places[i] = base;
+  close();
+  if (!FILL && lane == 0) run_batches[i] = nb, run_places[i] = base;
 }
 
 // begin[t] = first batch of tile t (t = tiles gives the batch count): the first run whose key
@@ -690,14 +696,10 @@ bool f32_tiles_fits(int32_t n, int32_t feat_in, int64_t edges) {
 }
 
 void f32_tiles_free(F32TileIndex& idx) {
-  if (idx.d_edges) (void)hipFree(idx.d_edges);
-  if (idx.d_pairs) (void)hipFree(idx.d_pairs);
   if (idx.d_batches) (void)hipFree(idx.d_batches);
   for (F32Units& u : idx.units) {
     if (u.d_units) (void)hipFree(u.d_units);
-    if (u.d_partials) (void)hipFree(u.d_partials);
   }
-  if (idx.d_wpack) (void)hipFree(idx.d_wpack);
   idx = F32TileIndex();
 }
 
@@ -724,7 +726,8 @@ namespace {
 // units, 30.0 with 1024, 36.8 uncut) -- and no pieces so short that filling the pipeline and the partial
 // tile cost more than they bring.  Wide launches with many tiles: two rounds (110 k nodes, 130
 // relations, 2 M edges, 64 -> 64: 334 us with 1024 units, 371 with 860 whole tiles).
-int make_units(F32Units& out, const std::vector<int64_t>& tile_begin, bool wide, hipStream_t stream) {
+int make_units(F32Units& out, const std::vector<int64_t>& tile_begin, bool wide, int32_t feat_out, size_t wpack_bytes,
+               hipStream_t stream) {
   const int64_t tiles = (int64_t)tile_begin.size() - 1, cus = compute_units();
   STIR_REQUIRE(cus > 0, "rgms_f32: no device");
   const int64_t target = tiles > 2 * cus ? 4 * cus : (wide ? 2 : 3) * cus;
@@ -759,12 +762,18 @@ int make_units(F32Units& out, const std::vector<int64_t>& tile_begin, bool wide,
     return a.batch_end - a.batch_begin > b.batch_end - b.batch_begin;
   });
   out.count = (int64_t)units.size(), out.partial_tiles = partial_tiles;
-  // the units and behind them the counters of the cut tiles, zero between launches
+  // one allocation: the units, the counters of the cut tiles (zero between launches), W in operand order, the
+  // partial tiles
   const size_t unit_bytes = sizeof(UnitF32) * units.size();
-  std::vector<char> image(unit_bytes + sizeof(uint32_t) * (size_t)cut_tiles + 16);
+  std::vector<char> image(Scratch::rounded(unit_bytes + sizeof(uint32_t) * (size_t)cut_tiles));
   std::copy_n(reinterpret_cast<const char*>(units.data()), unit_bytes, image.data());
-  STIR_HIP(hipMalloc(&out.d_units, image.size()));
-  out.d_arrived = static_cast<char*>(out.d_units) + unit_bytes;
+  const size_t partial_bytes = sizeof(float) * (size_t)partial_tiles * kTileRows * (size_t)feat_out;
+  STIR_HIP(hipMalloc(&out.d_units, image.size() + Scratch::rounded(wpack_bytes) + partial_bytes));
+  char* base = static_cast<char*>(out.d_units);
+  out.d_arrived = base + unit_bytes;
+  out.d_wpack = base + image.size();
+  out.d_partials = base + image.size() + Scratch::rounded(wpack_bytes);
+  out.wpack_bytes = wpack_bytes, out.feat_out = feat_out;
   STIR_HIP(hipMemcpyAsync(out.d_units, image.data(), image.size(), hipMemcpyHostToDevice, stream));
   STIR_HIP(hipStreamSynchronize(stream));  // there before a launch on any stream
   return 0;
@@ -891,7 +900,7 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   const int64_t runs = host_flags[1];
   bytes = scan2;
   STIR_HIP(hipcub::DeviceScan::ExclusiveSum(cub_tmp, bytes, run_pairs, run_first_pair, (int)runs, stream));
-  const dim3 run_grid((unsigned)ceil_div(runs, 256));
+  const dim3 run_grid((unsigned)ceil_div(runs, 4));
   hipLaunchKernelGGL(f32_batches_kernel<false>, run_grid, block, 0, stream, run_keys, run_pairs, run_first_pair,
                      (const int32_t*)nullptr, runs, num_rels, (int)emax, unique, counts, run_batches, run_places,
                      (const int64_t*)nullptr, (BatchF32*)nullptr, (uint32_t*)nullptr, (int64_t*)nullptr);
@@ -911,11 +920,13 @@ int build_index(F32TileIndex& idx, const F32Source& src, int32_t m, int32_t n, i
   STIR_HIP(hipMemcpyAsync(&total_batches, run_first_batch + runs, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
   STIR_HIP(hipStreamSynchronize(stream));
   idx.batches = total_batches;
-  STIR_HIP(hipMalloc(&idx.d_batches, sizeof(BatchF32) * (size_t)std::max<int64_t>(total_batches, 1)));
   const int64_t words = (int64_t)total_batches * kBatch;
-  STIR_HIP(hipMalloc(&idx.d_pairs, sizeof(uint32_t) * (size_t)std::max<int64_t>(words, 1)));
   STIR_REQUIRE(places < (int64_t(1) << 32), "rgms_f32: too many edges");
-  STIR_HIP(hipMalloc(&idx.d_edges, sizeof(EdgeF32) * (size_t)std::max<int64_t>(places, 1)));
+  const size_t batch_bytes = Scratch::rounded(sizeof(BatchF32) * (size_t)total_batches);
+  const size_t word_bytes = Scratch::rounded(sizeof(uint32_t) * (size_t)words);
+  STIR_HIP(hipMalloc(&idx.d_batches, batch_bytes + word_bytes + Scratch::rounded(sizeof(EdgeF32) * (size_t)places)));
+  idx.d_pairs = static_cast<char*>(idx.d_batches) + batch_bytes;
+  idx.d_edges = static_cast<char*>(idx.d_batches) + batch_bytes + word_bytes;
   EdgeF32* d_places = static_cast<EdgeF32*>(idx.d_edges);
   const float* some_weight = src.csf ? src.A : tab[0].A;
   hipLaunchKernelGGL(f32_clear_places_kernel, dim3((unsigned)ceil_div(std::max(places, words), 256)), block, 0, stream,
@@ -949,32 +960,23 @@ int f32_tiles_launch(F32TileIndex& idx, int32_t feat_in, int32_t feat_out, const
                feat_in, feat_out);
   STIR_REQUIRE(idx.emax == (feat_in <= 32 ? 32 : 16), "rgms_f32: the edge index was built for another feat_in");
   if (idx.edges == 0) return 0;
-  const bool wide = feat_out > 32;
-  F32Units& u = idx.units[wide];
-  if (!u.d_units && make_units(u, idx.tile_begin, wide, stream)) return -1;
-  if (u.count == 0) return 0;
-  STIR_REQUIRE(u.count < (int64_t(1) << 31), "rgms_f32: too many units for one launch");
   // the kernel's 32-bit byte offsets
   STIR_REQUIRE(f32_tiles_fits(idx.n, feat_in, idx.edges),
                "rgms_f32: the tiled kernel addresses X and its index with 32-bit offsets");
   const int ks = feat_in <= 32 ? 1 : 2, nt = feat_out <= 16 ? 1 : feat_out <= 32 ? 2 : 4;
   // W in operand order, rewritten by every launch (W may change between launches)
   const int64_t fragments = (int64_t)idx.num_rels * nt * ks * 64;
-  const size_t need = 3 * sizeof(bf16x8) * (size_t)fragments;
-  if (need > idx.wpack_bytes) {
-    if (idx.d_wpack) STIR_HIP(hipFree(idx.d_wpack));
-    idx.d_wpack = nullptr, idx.wpack_bytes = 0;
-    STIR_HIP(hipMalloc(&idx.d_wpack, need));
-    idx.wpack_bytes = need;
+  const size_t wpack_bytes = 3 * sizeof(bf16x8) * (size_t)fragments;
+  const bool wide = feat_out > 32;
+  F32Units& u = idx.units[wide];
+  if (!u.d_units || wpack_bytes > u.wpack_bytes || feat_out > u.feat_out) {
+    if (u.d_units) STIR_HIP(hipFree(u.d_units));
+    u = F32Units();
+    if (make_units(u, idx.tile_begin, wide, feat_out, wpack_bytes, stream)) return -1;
   }
-  const size_t partial_need = sizeof(float) * (size_t)u.partial_tiles * kTileRows * (size_t)feat_out;
-  if (partial_need > u.partial_bytes) {
-    if (u.d_partials) STIR_HIP(hipFree(u.d_partials));
-    u.d_partials = nullptr, u.partial_bytes = 0;
-    STIR_HIP(hipMalloc(&u.d_partials, partial_need));
-    u.partial_bytes = partial_need;
-  }
-  bf16x8* wp = static_cast<bf16x8*>(idx.d_wpack);
+  if (u.count == 0) return 0;
+  STIR_REQUIRE(u.count < (int64_t(1) << 31), "rgms_f32: too many units for one launch");
+  bf16x8* wp = static_cast<bf16x8*>(u.d_wpack);
   hipLaunchKernelGGL(f32_pack_w_kernel, dim3((unsigned)ceil_div(fragments, 256)), dim3(256), 0, stream, d_W, wp, fragments, nt, ks,
                      feat_in, feat_out);
   STIR_LAUNCH_CHECK();

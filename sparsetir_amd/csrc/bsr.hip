@@ -5,10 +5,12 @@
 // feature axis; a wavefront owns NT 32-feature tiles per 32 rows, each a 32x32 fp32 accumulator
 // fed by v_mfma_f32_32x32x16_{f16,bf16}.  Both operands go through LDS: the MFMA B operand wants
 // 8 consecutive k for one feature per lane while X is feature-contiguous, and the A fragment is
-// shared by the four wavefronts (see bsr_tile).  Small launches use bsr_spmm_ksplit_kernel.
+// shared by the four wavefronts (see bsr_tile).  Blocks of 16 k + 16 rows use bsr16_spmm_kernel, small
+// launches bsr_split_kernel.
 #include <hip/hip_fp16.h>
 
 #include <numeric>
+#include <type_traits>
 
 #include "common.h"
 #include "../../include/sparsetir_amd.h"
@@ -417,140 +419,10 @@ __global__ __launch_bounds__(256) void bsr_spmm_sweep_kernel(int blk, int feat, 
   }
 }
 
-// Small launches (at most a couple of workgroups per CU): a workgroup's run time is the serial
-// chain of its block row's steps, each a memory round trip, and nothing else is resident to hide
-// it.  Here the four wavefronts of a workgroup split the steps of the block row instead of the
-// feature axis: wavefront w takes steps w, w + 4, ... for all 128 features (four accumulators),
-// stages its own X tile in its own piece of LDS (no workgroup barrier in the loop: the LDS
-// operations of one wavefront execute in order) and the four partial results are added through
-// LDS at the end.  Same tile and the same global traffic as bsr_spmm_kernel, a chain four times
-// shorter.
-constexpr int kSplitLdsWords = 4 * 4 * 16 * 64;  // reduction: [wavefront][feature tile][register][lane]
-
-template <bool BF16, int OUT>
-__global__ __launch_bounds__(256) void bsr_spmm_ksplit_kernel(int blk, int feat, int64_t slices, int f_tiles,
-                                                              const uint16_t* __restrict__ A,
-                                                              const uint16_t* __restrict__ X, void* __restrict__ Y,
-                                                              const int32_t* __restrict__ indptr,
-                                                              const int32_t* __restrict__ indices,
-                                                              const int32_t* __restrict__ row_ids) {
-  __shared__ __attribute__((aligned(16))) uint32_t lds[kSplitLdsWords];  // 64 KB
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = lane & 31, h = lane >> 5;
-  const int f_tile = (int)(blockIdx.x % f_tiles);
-  const int64_t slice = blockIdx.x / f_tiles;
-  const int sub = blk / 32;
-  const int i = (int)(slice / sub), bi0 = (int)(slice % sub) * 32;
-  const int f0 = f_tile * kTileF;
-  // staging role of a lane: k pairs kp, kp + 4, kp + 8, kp + 12; 8-feature chunk fc
-  const int kp = lane >> 4, fc = lane & 15;
-  const bool stage_live = f0 + fc * 8 < feat;
-  uint32_t(*xs)[kTileF] = reinterpret_cast<uint32_t(*)[kTileF]>(lds + wave * (16 * kTileF));  // [k pair][feature]
-
-  f32x16 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
-
-  const int i_out = row_ids ? row_ids[i] : i;
-  const int p_begin = indptr[i];
-  const int ksteps = blk / kTileK;
-  const int steps = (indptr[i + 1] - p_begin) * ksteps;
-
-  // The block columns of the row's first 64 blocks are fetched once, one per lane: looking them up
-  // step by step would put a second memory round trip in front of every step's loads of X.
-  const int nblk = indptr[i + 1] - p_begin;
-  const int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
-  u32x4 r0[4], r1[4], areg[2];
-  auto fetch = [&](int it) {
-    const int b = it / ksteps, k0 = (it % ksteps) * kTileK;
-    const int p = p_begin + b;
-    const int64_t j = b < kWave ? __shfl(j_lane, b, kWave) : indices[p];
-    const uint16_t* ablk = A + (int64_t)p * blk * blk + (int64_t)(bi0 + n) * blk + k0;
-    areg[0] = *reinterpret_cast<const u32x4*>(ablk + 8 * h);
-    areg[1] = *reinterpret_cast<const u32x4*>(ablk + 16 + 8 * h);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      r0[q] = r1[q] = u32x4{0, 0, 0, 0};
-      if (stage_live) {
-        const uint16_t* xp = X + ((int64_t)j * blk + k0 + 2 * (kp + 4 * q)) * feat + f0 + fc * 8;
-        r0[q] = *reinterpret_cast<const u32x4*>(xp);
-        r1[q] = *reinterpret_cast<const u32x4*>(xp + feat);
-      }
-    }
-  };
-
-  if (wave < steps) fetch(wave);
-  for (int it = wave; it < steps; it += 4) {
-    const u32x4 a0 = areg[0], a1 = areg[1];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      u32x4 lo, hi;
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        lo[2 * d] = __builtin_amdgcn_perm(r1[q][d], r0[q][d], 0x05040100);
-        lo[2 * d + 1] = __builtin_amdgcn_perm(r1[q][d], r0[q][d], 0x07060302);
-        hi[2 * d] = __builtin_amdgcn_perm(r1[q][d + 2], r0[q][d + 2], 0x05040100);
-        hi[2 * d + 1] = __builtin_amdgcn_perm(r1[q][d + 2], r0[q][d + 2], 0x07060302);
-      }
-      *reinterpret_cast<u32x4*>(&xs[kp + 4 * q][fc * 8]) = lo;
-      *reinterpret_cast<u32x4*>(&xs[kp + 4 * q][fc * 8 + 4]) = hi;
-    }
-    if (it + 4 < steps) fetch(it + 4);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int col = t * 32 + n;
-      u32x4 b0, b1;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        b0[d] = xs[4 * h + d][col];
-        b1[d] = xs[8 + 4 * h + d][col];
-      }
-      acc[t] = mfma32<BF16>(a0, b0, acc[t]);
-      acc[t] = mfma32<BF16>(a1, b1, acc[t]);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
-  }
-
-  // ---- add the four partial results: wavefront w ends up with feature tile w
-  __syncthreads();  // every wavefront is done with its staging piece
-  float* red = reinterpret_cast<float*>(lds);
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) red[((wave * 4 + t) * 16 + v) * 64 + lane] = acc[t][v];
-  __syncthreads();
-  const int fcol = f0 + wave * 32;
-  if (fcol >= feat) return;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    float sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) sum += red[((w * 4 + wave) * 16 + v) * 64 + lane];
-    const int row = (v & 3) + 4 * h + 8 * (v >> 2);
-    const int64_t off = ((int64_t)i_out * blk + bi0 + row) * feat + fcol + n;
-    if constexpr (OUT == 1)
-      static_cast<float*>(Y)[off] = sum;
-    else
-      static_cast<uint16_t*>(Y)[off] = to16<BF16>(sum);
-  }
-}
-
 // ------------------------------------------------------------------ blocks of 16 k+16 rows
 // Block sides that are a multiple of 16 but not of 32 (the reference's schedule splits both block
 // axes by 16, examples/blocksparse/bsr_spmm.py:379-380): 16-row slices on v_mfma_f32_16x16x32,
-// whose k extent of 32 is two 16-column chunks of the block row's blocks in storage order.  A
-// workgroup of four wavefronts owns (block row, 16-row slice, 128 features), a wavefront 16 rows
-// x 32 features (two accumulators of four registers).  The A operand -- 8 consecutive k of one row
-// per lane -- is one 16-byte load from the block; the 32 rows of X of a step go through LDS as
-// (k, k+1) pairs, double-buffered, the next step's loads in flight during the multiply.  Rows of
-// the staged image are rotated by 16 (k pair / 4) words so that the four k groups a multiply
-// reads lie on different banks.
+// whose k extent of 32 is two 16-column chunks of the block row's blocks in storage order.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <bool BF16>
@@ -563,100 +435,284 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                   0, 0);
 }
 
-template <bool BF16, int OUT>
+// 8 consecutive k of one feature per lane, from a feature-contiguous image: two transposing reads `next`
+// bytes (four rows of k) apart
+__device__ __forceinline__ u32x4 read_b(const char* at, int next) {
+  const tr16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at));
+  const tr16x4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at + next));
+  const u32x2 lo = __builtin_bit_cast(u32x2, t0), hi = __builtin_bit_cast(u32x2, t1);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// A chunk of 16 columns: number `number` of a block row's chunks, columns 16 * col of block `block`
+struct Chunk {
+  int number, block, col;
+  __device__ __forceinline__ void advance(int by, int sub) {
+    number += by, col += by;
+    while (col >= sub) col -= sub, ++block;
+  }
+};
+
+// A workgroup of four wavefronts owns (block row, 16-row slice, 128 * NT features), a wavefront 16 rows x
+// 32 * NT features.  Per step the 32 rows of X of two chunks go through LDS as in bsr_tile (two stages, one
+// barrier per step, the next step's loads in flight), the image's XOR extended by 2 * (k / 8 % 2): the two
+// blocks of 16 lanes that a transposing read serves together ask for the same units of k groups eight rows
+// apart here.  The A operand is one 16-byte load per lane from the block.
+// Bound by the rows of X that come out of L2: a 16-row slice uses each of them for 16 rows only (318 x 284
+// blocks of 16, 20 %, 3328 features: 1.9 GB of X in 221 us with 128 features per workgroup and X transposed on
+// the way into LDS by 2-byte stores, in 118 us with this image and in 110 us with 256 features; 1006 x 599,
+// 544 features: 262 -> 155 us).
+template <bool BF16, int OUT, int NT>
 __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int64_t slices, int f_tiles,
                                                          const uint16_t* __restrict__ A,
                                                          const uint16_t* __restrict__ X, void* __restrict__ Y,
                                                          const int32_t* __restrict__ indptr,
                                                          const int32_t* __restrict__ indices,
                                                          const int32_t* __restrict__ row_ids) {
-  __shared__ __attribute__((aligned(16))) uint32_t xs[2][16 * kTileF];  // [buffer][k pair][feature]
+  constexpr int TF = kTileF * NT;
+  constexpr int FCN = TF / 8;          // 16-byte units per row of X
+  constexpr int XB = kTileK * TF * 2;  // bytes per stage
+  __shared__ __attribute__((aligned(16))) char xs[2 * XB];
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int f_tile = (int)(blockIdx.x % f_tiles);
-  const int64_t slice = blockIdx.x / f_tiles;
-  if (slice >= slices) return;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int64_t slice;
+  int f_tile;
+  if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) return;
   const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
   const int i = (int)(slice / sub), s = (int)(slice % sub);
   const int i_out = row_ids ? row_ids[i] : i;
-  const int f0 = f_tile * kTileF;
-  // staging role: k pair kp (rows 2kp, 2kp+1 of the step's 32), 8-feature chunk fc
-  const int kp = tid >> 4, fc = tid & 15;
-  const bool stage_live = f0 + fc * 8 < feat;
-  const int stage_at = kp * kTileF + ((fc * 8 + 16 * (kp >> 2)) & (kTileF - 1));
+  const int f0 = f_tile * TF;
+  // staging role: 2 * NT units of the wavefront's chunk (wavefronts 0, 1: the step's first; 2, 3: its second)
+  uint32_t xoff[2 * NT], xdst[2 * NT];
+#pragma unroll
+  for (int u = 0; u < 2 * NT; ++u) {
+    const int idx = 64 * (wave * 2 * NT + u) + lane, c = idx % FCN, k = idx / FCN;
+    xoff[u] = (uint32_t)((k & 15) * feat + 8 * c);
+    xdst[u] = (uint32_t)(((k >> 2) * 4 * FCN + (k & 3) * FCN + (c ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)))) * 16);
+  }
+  static_assert(64 % FCN == 0, "a lane's units share their feature column");
+  const bool xlive = f0 + 8 * (lane % FCN) < feat;
   // operand role: row ii of the slice, k group q (8 of the step's 32 k)
   const int ii = lane & 15, q = lane >> 4;
+  const uint32_t aoff = (uint32_t)((s * 16 + ii) * blk + 8 * (q & 1));
+  uint32_t bread[2 * NT];
+#pragma unroll
+  for (int t = 0; t < 2 * NT; ++t) {
+    const int kr = ii >> 2, c = wave * NT * 4 + 2 * t + ((ii & 3) >> 1);
+    bread[t] = (uint32_t)(((2 * q) * 4 * FCN + kr * FCN + (c ^ (4 * kr) ^ (2 * (q & 1)))) * 16 + (ii & 1) * 8);
+  }
 
   const int p_begin = indptr[i];
   const int chunks = (indptr[i + 1] - p_begin) * sub;
   const int steps = (chunks + 1) / 2;
 
-  f32x4 acc[2];
+  f32x4 acc[2 * NT];
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < 2 * NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // the block column of a step's chunk is requested one step before its rows of X
-  int j_stage = 0;
-  auto fetch_ids = [&](int it) {
-    const int c = 2 * it + (kp >> 3);
-    j_stage = c < chunks ? indices[p_begin + c / sub] : 0;
-  };
-  u32x4 r0, r1, a_next;
-  auto fetch = [&](int it) {
-    a_next = r0 = r1 = u32x4{0, 0, 0, 0};
-    const int ca = 2 * it + (q >> 1);
-    if (ca < chunks)
-      a_next = *reinterpret_cast<const u32x4*>(A + ((int64_t)(p_begin + ca / sub) * blk + s * 16 + ii) * blk +
-                                               (ca % sub) * 16 + 8 * (q & 1));
-    const int c = 2 * it + (kp >> 3);
-    if (stage_live && c < chunks) {
-      const uint16_t* xp = X + ((int64_t)j_stage * blk + (c % sub) * 16 + 2 * (kp & 7)) * feat + f0 + fc * 8;
-      r0 = *reinterpret_cast<const u32x4*>(xp);
-      r1 = *reinterpret_cast<const u32x4*>(xp + feat);
+  // the chunks of the step to fetch next: of the wavefront's rows of X, and of the lane's piece of A; the block
+  // column is requested one step before the rows of X
+  Chunk mx{0, 0, 0}, ma{0, 0, 0};
+  mx.advance(wave >> 1, sub);
+  ma.advance(q >> 1, sub);
+  int j = mx.number < chunks ? indices[p_begin + mx.block] : 0;
+  u32x4 xr[2 * NT], a_next;
+  auto fetch = [&]() {
+    a_next = u32x4{0, 0, 0, 0};
+    if (ma.number < chunks)
+      a_next = *reinterpret_cast<const u32x4*>(A + (int64_t)(p_begin + ma.block) * blk * blk + aoff + 16 * ma.col);
+    const bool live = xlive && mx.number < chunks;
+    const uint16_t* xb = X + ((int64_t)j * blk + 16 * mx.col) * feat + f0;
+#pragma unroll
+    for (int u = 0; u < 2 * NT; ++u) {
+      xr[u] = u32x4{0, 0, 0, 0};
+      if (live) xr[u] = *reinterpret_cast<const u32x4*>(xb + xoff[u]);
     }
-    if (it + 1 < steps) fetch_ids(it + 1);
+    ma.advance(2, sub);
+    mx.advance(2, sub);
+    if (mx.number < chunks) j = indices[p_begin + mx.block];
   };
 
-  if (steps > 0) {
-    fetch_ids(0);
-    fetch(0);
-  }
+  if (steps > 0) fetch();
   for (int it = 0; it < steps; ++it) {
-    const int buf = it & 1;
-    const u32x4 a_now = a_next;
-    u32x4 lo, hi;
+    char* stage = xs + (it & 1) * XB;
+    const u32x4 a = a_next;
 #pragma unroll
-    for (int d = 0; d < 2; ++d) {
-      lo[2 * d] = __builtin_amdgcn_perm(r1[d], r0[d], 0x05040100);
-      lo[2 * d + 1] = __builtin_amdgcn_perm(r1[d], r0[d], 0x07060302);
-      hi[2 * d] = __builtin_amdgcn_perm(r1[d + 2], r0[d + 2], 0x05040100);
-      hi[2 * d + 1] = __builtin_amdgcn_perm(r1[d + 2], r0[d + 2], 0x07060302);
-    }
-    *reinterpret_cast<u32x4*>(&xs[buf][stage_at]) = lo;
-    *reinterpret_cast<u32x4*>(&xs[buf][stage_at + 4]) = hi;
-    if (it + 1 < steps) fetch(it + 1);
+    for (int u = 0; u < 2 * NT; ++u) *reinterpret_cast<u32x4*>(stage + xdst[u]) = xr[u];
+    if (it + 1 < steps) fetch();
     __syncthreads();
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      const int c = ((wave * 32 + 16 * nt + 16 * q) & (kTileF - 1)) + ii;
-      u32x4 b;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) b[d] = xs[buf][(4 * q + d) * kTileF + c];  // rows 8q .. 8q+7 of the step
-      acc[nt] = mfma16<BF16>(a_now, b, acc[nt]);
-    }
+    for (int t = 0; t < 2 * NT; ++t) acc[t] = mfma16<BF16>(a, read_b(stage + bread[t], FCN * 64), acc[t]);
   }
-  const int fcol = f0 + wave * 32;
-  if (fcol >= feat) return;
 #pragma unroll
-  for (int nt = 0; nt < 2; ++nt)
+  for (int t = 0; t < 2 * NT; ++t) {
+    const int fcol = f0 + wave * 32 * NT + 16 * t;
+    if (fcol >= feat) continue;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      const int64_t off = ((int64_t)i_out * blk + s * 16 + 4 * q + v) * feat + fcol + 16 * nt + ii;
+      const int64_t off = ((int64_t)i_out * blk + s * 16 + 4 * q + v) * feat + fcol + ii;
       if constexpr (OUT == 1)
-        static_cast<float*>(Y)[off] = acc[nt][v];
+        static_cast<float*>(Y)[off] = acc[t][v];
       else
-        static_cast<uint16_t*>(Y)[off] = to16<BF16>(acc[nt][v]);
+        static_cast<uint16_t*>(Y)[off] = to16<BF16>(acc[t][v]);
     }
+  }
+}
+
+// ------------------------------------------------------------------ small launches
+// With a few workgroups per CU the run time is the chain of steps of the longest block row, each a memory
+// round trip.  Here the eight wavefronts of a workgroup take the steps of a block row (ROWS = 32 or 16 of its
+// rows, 64 features) in turn: wavefront w the steps w, w + 8, ..., each with an X tile of its own in LDS (no
+// workgroup barrier in the loop: the LDS operations of one wavefront execute in order); the eight partial
+// results are added through LDS at the end.
+// The X tile is 32 rows of 8 units of 16 bytes; unit (k, c) sits at place c ^ 4 * (k / 2 % 2) of its row -- two
+// rows fill the 64 banks -- and, ROWS = 16, ^ 2 * (k / 8 % 2) (see bsr16_spmm_kernel).
+// Against four wavefronts that took the k halves of each step: 40 x 510 blocks of 32, 18 %, 288 features
+// 27.4 -> 15.9 us; 50 x 63 blocks of 128, 128 features 27.6 -> 17.2 us; 358 x 998 blocks of 16, 64 features
+// (which had no such form) 39 -> 11.8 us.
+constexpr int kSplitWaves = 8;
+constexpr int kSplitF = 64;
+
+template <bool BF16, int OUT, int ROWS>
+__global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, int feat, int64_t slices, int f_tiles,
+                                                                     const uint16_t* __restrict__ A,
+                                                                     const uint16_t* __restrict__ X,
+                                                                     void* __restrict__ Y,
+                                                                     const int32_t* __restrict__ indptr,
+                                                                     const int32_t* __restrict__ indices,
+                                                                     const int32_t* __restrict__ row_ids) {
+  constexpr int FCN = kSplitF / 8;
+  constexpr int XB = kTileK * kSplitF * 2;          // bytes of a wavefront's X tile
+  constexpr int TILES = ROWS == 32 ? 2 : 4;         // 32- or 16-feature tiles
+  constexpr int REGS = ROWS == 32 ? 16 : 4;         // accumulator registers of one
+  constexpr int ELEMS = TILES * REGS * kWave;       // floats of a partial result
+  __shared__ __attribute__((aligned(16))) char lds[kSplitWaves * (XB > ELEMS * 4 ? XB : ELEMS * 4)];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int64_t slice;
+  int f_tile;
+  if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) return;
+  const int sub = blk / ROWS;
+  const int i = (int)(slice / sub), bi0 = (int)(slice % sub) * ROWS;
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = f_tile * kSplitF;
+  char* stage = lds + wave * XB;
+  // staging role: unit xc of the rows k = 8 u + kq
+  const int xc = lane & 7, kq = lane >> 3;
+  const bool xlive = f0 + 8 * xc < feat;
+  const uint32_t xoff = (uint32_t)(kq * feat + 8 * xc);
+  uint32_t xdst[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    xdst[u] = (uint32_t)(((8 * u + kq) * FCN + (xc ^ (4 * ((kq >> 1) & 1)) ^ (ROWS == 16 ? 2 * (u & 1) : 0))) * 16);
+  // operand role
+  const int n = ROWS == 32 ? lane & 31 : lane & 15, h = ROWS == 32 ? lane >> 5 : lane >> 4;
+  const int sl = lane & 15, kr = sl >> 2;
+  uint32_t bread[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t) {
+    const int c = ROWS == 32 ? 4 * t + 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1) : 2 * t + ((sl & 3) >> 1);
+    const int place = c ^ (4 * (kr >> 1)) ^ (ROWS == 16 ? 2 * (h & 1) : 0);
+    bread[t] = (uint32_t)(((8 * h + kr) * FCN + place) * 16 + (sl & 1) * 8);
+  }
+
+  const int p_begin = indptr[i];
+  const int nblk = indptr[i + 1] - p_begin;
+  const int ksteps = blk / kTileK;                       // ROWS = 32: steps per block
+  const int chunks = nblk * sub;                         // ROWS = 16: two per step
+  const int steps = ROWS == 32 ? nblk * ksteps : (chunks + 1) / 2;
+  // The block columns of the row's first 64 blocks are fetched once, one per lane: looking them up
+  // step by step would put a second memory round trip in front of every step's loads of X.
+  const int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
+  auto column = [&](int b) -> int64_t {
+    return b < kWave ? __builtin_amdgcn_readlane(j_lane, b) : indices[p_begin + b];
+  };
+
+  u32x4 xr[4], ar[2];
+  auto fetch = [&](int it) {
+    if constexpr (ROWS == 32) {
+      const int b = it / ksteps, k0 = (it - b * ksteps) * kTileK;
+      const uint16_t* ab = A + (int64_t)(p_begin + b) * blk * blk + (int64_t)(bi0 + n) * blk + k0 + 8 * h;
+      ar[0] = *reinterpret_cast<const u32x4*>(ab);
+      ar[1] = *reinterpret_cast<const u32x4*>(ab + 16);
+      const uint16_t* xb = X + (column(b) * blk + k0) * feat + f0 + xoff;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        xr[u] = u32x4{0, 0, 0, 0};
+        if (xlive) xr[u] = *reinterpret_cast<const u32x4*>(xb + (int64_t)(8 * u) * feat);
+      }
+    } else {
+      const int c0 = 2 * it, b0 = c0 / sub, b1 = (c0 + 1) / sub;
+      const bool two = c0 + 1 < chunks;
+      const int ba = h >> 1 ? b1 : b0, ca = c0 + (h >> 1) - ba * sub;
+      ar[0] = u32x4{0, 0, 0, 0};
+      if (h < 2 || two)
+        ar[0] = *reinterpret_cast<const u32x4*>(A + (int64_t)(p_begin + ba) * blk * blk + (int64_t)(bi0 + n) * blk +
+                                                16 * ca + 8 * (h & 1));
+      const uint16_t* x0 = X + (column(b0) * blk + 16 * (c0 - b0 * sub)) * feat + f0 + xoff;
+      const uint16_t* x1 = X + (column(two ? b1 : b0) * blk + 16 * (two ? c0 + 1 - b1 * sub : 0)) * feat + f0 + xoff;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        xr[u] = u32x4{0, 0, 0, 0};
+        if (xlive && (u < 2 || two))
+          xr[u] = *reinterpret_cast<const u32x4*>((u < 2 ? x0 : x1) + (int64_t)(8 * (u & 1)) * feat);
+      }
+    }
+  };
+
+  typename std::conditional<ROWS == 32, f32x16, f32x4>::type acc[TILES];
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int v = 0; v < REGS; ++v) acc[t][v] = 0.f;
+
+  if (wave < steps) fetch(wave);
+  for (int it = wave; it < steps; it += kSplitWaves) {
+    const u32x4 a0 = ar[0], a1 = ar[1];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) *reinterpret_cast<u32x4*>(stage + xdst[u]) = xr[u];
+    if (it + kSplitWaves < steps) fetch(it + kSplitWaves);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < TILES; ++t) {
+      if constexpr (ROWS == 32) {
+        acc[t] = mfma32<BF16>(a0, read_b(stage + bread[t], 4 * FCN * 16), acc[t]);
+        acc[t] = mfma32<BF16>(a1, read_b(stage + bread[t] + 16 * FCN * 16, 4 * FCN * 16), acc[t]);
+      } else {
+        acc[t] = mfma16<BF16>(a0, read_b(stage + bread[t], 4 * FCN * 16), acc[t]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+  }
+
+  // ---- add the partial results
+  __syncthreads();  // every wavefront is done with its tile
+  float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+  for (int t = 0; t < TILES; ++t)
+#pragma unroll
+    for (int v = 0; v < REGS; ++v) red[wave * ELEMS + (t * REGS + v) * kWave + lane] = acc[t][v];
+  __syncthreads();
+  const int used = min(steps, kSplitWaves);
+#pragma unroll
+  for (int e0 = 0; e0 < ELEMS; e0 += 64 * kSplitWaves) {
+    const int e = e0 + tid, l = e & 63, v = (e >> 6) % REGS, t = (e >> 6) / REGS;
+    float sum = 0.f;
+    for (int w = 0; w < used; ++w) sum += red[w * ELEMS + e];
+    int row, col;
+    if constexpr (ROWS == 32)
+      row = (v & 3) + 4 * (l >> 5) + 8 * (v >> 2), col = f0 + 32 * t + (l & 31);
+    else
+      row = 4 * (l >> 4) + v, col = f0 + 16 * t + (l & 15);
+    if (col >= feat) continue;
+    const int64_t off = ((int64_t)i_out * blk + bi0 + row) * feat + col;
+    if constexpr (OUT == 1)
+      static_cast<float*>(Y)[off] = sum;
+    else
+      static_cast<uint16_t*>(Y)[off] = to16<BF16>(sum);
+  }
 }
 
 }  // namespace
@@ -671,21 +727,58 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   STIR_REQUIRE(feat > 0 && feat % 32 == 0, "bsr_spmm: feat=%d must be a multiple of 32", feat);
   if (mb == 0) return 0;
   STIR_REQUIRE(d_X && d_Y && d_indptr && (nnzb == 0 || (d_A && d_indices)), "bsr_spmm: null pointer argument");
-  hipStream_t st16 = static_cast<hipStream_t>(stream);
-  if (blk % 32 != 0) {
-    const int f_tiles16 = (int)stir::ceil_div(feat, kTileF);
-    const int64_t slices16 = (int64_t)mb * (blk / 16);
-    STIR_REQUIRE(slices16 * f_tiles16 < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-    dim3 grid16((unsigned)(slices16 * f_tiles16)), block16(256);
-#define STIR_BSR_16(BF, OUT)                                                                                    \
-  hipLaunchKernelGGL((bsr16_spmm_kernel<BF, OUT>), grid16, block16, 0, st16, blk, feat, slices16, f_tiles16,     \
-                     static_cast<const uint16_t*>(d_A), static_cast<const uint16_t*>(d_X), d_Y, d_indptr, d_indices, \
-                     d_row_ids)
-    if (dtype == STIR_BF16) {
-      if (out_dtype == STIR_F32) STIR_BSR_16(true, 1); else STIR_BSR_16(true, 0);
-    } else {
-      if (out_dtype == STIR_F32) STIR_BSR_16(false, 1); else STIR_BSR_16(false, 0);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint16_t* A = static_cast<const uint16_t*>(d_A);
+  const uint16_t* X = static_cast<const uint16_t*>(d_X);
+  const int cus = stir::compute_units();
+  const int unit = blk % 32 != 0 ? 16 : 32;  // rows of a slice
+  const int64_t unit_slices = (int64_t)mb * (blk / unit);
+  auto grid_of = [](int64_t n, int tiles) { return 8 * stir::ceil_div(n * tiles, 8); };  // see decode_tile
+#define STIR_BSR_TYPES(LAUNCH)                                        \
+  if (dtype == STIR_BF16) {                                           \
+    if (out_dtype == STIR_F32) LAUNCH(true, 1); else LAUNCH(true, 0); \
+  } else {                                                            \
+    if (out_dtype == STIR_F32) LAUNCH(false, 1); else LAUNCH(false, 0); \
+  }
+  // The split form wins as long as its workgroups are resident at once (64 KB of LDS with 32-row slices: two per
+  // CU; four with 16-row slices), and up to twice as many where block rows have enough steps to pay for the
+  // second turn.  Measured with 256 features, split against not: 32-row slices, 500 workgroups of 16 steps 7.8
+  // against 10.2 us, 1000 of 16 steps 14.1 against 10.8 us, of 32 steps 19.4 against 21.0 us; 16-row slices,
+  // 1000 of 4 steps 7.3 against 7.3 us, 2000 of 16 steps 16.9 against 16.2 us, of 24 steps 20.2 against 21.3 us.
+  {
+    const int f_tiles = (int)stir::ceil_div(feat, kSplitF);
+    const int64_t blocks = grid_of(unit_slices, f_tiles);
+    const int64_t at_once = (unit == 16 ? 4 : 2) * (int64_t)cus;
+    const int64_t row_steps = nnzb * (blk / 16) / 2 / mb;  // steps of a block row, on average
+    if (blocks <= at_once || (blocks <= 2 * at_once && row_steps >= (unit == 16 ? 24 : 32))) {
+      const dim3 grid((unsigned)blocks), block(kWave * kSplitWaves);
+#define STIR_BSR_S(BF, OUT)                                                                                  \
+  if (unit == 16)                                                                                            \
+    hipLaunchKernelGGL((bsr_split_kernel<BF, OUT, 16>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
+                       d_Y, d_indptr, d_indices, d_row_ids);                                                 \
+  else                                                                                                       \
+    hipLaunchKernelGGL((bsr_split_kernel<BF, OUT, 32>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
+                       d_Y, d_indptr, d_indices, d_row_ids)
+      STIR_BSR_TYPES(STIR_BSR_S)
+#undef STIR_BSR_S
+      STIR_LAUNCH_CHECK();
+      return 0;
     }
+  }
+  if (unit == 16) {
+    const int nt16 = feat >= 256 ? 2 : 1;
+    const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt16);
+    const int64_t blocks = grid_of(unit_slices, f_tiles);
+    STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
+    const dim3 grid((unsigned)blocks), block(256);
+#define STIR_BSR_16(BF, OUT)                                                                                  \
+  if (nt16 == 2)                                                                                              \
+    hipLaunchKernelGGL((bsr16_spmm_kernel<BF, OUT, 2>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
+                       d_Y, d_indptr, d_indices, d_row_ids);                                                  \
+  else                                                                                                        \
+    hipLaunchKernelGGL((bsr16_spmm_kernel<BF, OUT, 1>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
+                       d_Y, d_indptr, d_indices, d_row_ids)
+    STIR_BSR_TYPES(STIR_BSR_16)
 #undef STIR_BSR_16
     STIR_LAUNCH_CHECK();
     return 0;
@@ -693,30 +786,6 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // two 32-row slices per workgroup when the block height allows it
   const int rs = (blk % 64 == 0) ? 2 : 1;
   const int64_t slices = (int64_t)mb * (blk / (32 * rs));
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const uint16_t* A = static_cast<const uint16_t*>(d_A);
-  const uint16_t* X = static_cast<const uint16_t*>(d_X);
-  // A launch of at most two workgroups per CU is bound by the chain of steps of its longest block
-  // row: the four wavefronts of a workgroup then split the steps instead of the features.
-  {
-    const int f_tiles_s = (int)stir::ceil_div(feat, kTileF);
-    const int64_t blocks_s = (int64_t)mb * (blk / 32) * f_tiles_s;
-    if (blocks_s <= 2 * (int64_t)stir::compute_units()) {
-      const int64_t slices_s = (int64_t)mb * (blk / 32);
-      dim3 grid_s((unsigned)blocks_s), block_s(256);
-#define STIR_BSR_S(BF, OUT)                                                                                  \
-  hipLaunchKernelGGL((bsr_spmm_ksplit_kernel<BF, OUT>), grid_s, block_s, 0, st, blk, feat, slices_s, f_tiles_s, \
-                     A, X, d_Y, d_indptr, d_indices, d_row_ids)
-      if (dtype == STIR_BF16) {
-        if (out_dtype == STIR_F32) STIR_BSR_S(true, 1); else STIR_BSR_S(true, 0);
-      } else {
-        if (out_dtype == STIR_F32) STIR_BSR_S(false, 1); else STIR_BSR_S(false, 0);
-      }
-#undef STIR_BSR_S
-      STIR_LAUNCH_CHECK();
-      return 0;
-    }
-  }
   // Two 32-wide accumulators per wavefront once the feature axis is wide enough to still yield
   // several workgroups per CU.  One prefetched step is enough: measured on MI355X, deeper
   // register rings (2-6 steps) change nothing, the kernel is not bound by latency.
@@ -725,7 +794,6 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   dim3 block(256);
   // Launches whose X rows per feature tile do not fit a per-XCD L2 and that give every resident
   // workgroup several tiles are swept in step (bsr_spmm_sweep_kernel).
-  const int cus = stir::compute_units();
   const int64_t x_tile_bytes = (int64_t)nb * blk * kTileF * nt * 2;
   const int parts = 8 / std::gcd(f_tiles, 8);
 #define STIR_BSR_SWEEP(BF, OUT, NTV, RSV)                                                                     \
@@ -756,12 +824,12 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int sub_rows = blk / (32 * rs);
   const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2) ? 1 : 0;
   const int64_t blocks = by_rows ? 8 * stir::ceil_div((int64_t)mb, 8) * sub_rows * f_tiles
-                         : 8 * stir::ceil_div(slices * f_tiles, 8);
+                                 : grid_of(slices, f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   dim3 grid((unsigned)blocks);
 #define STIR_BSR_L(BF, OUT, NTV, RSV)                                                                      \
   {                                                                                                        \
-    if (sweep && !by_rows) STIR_BSR_SWEEP(BF, OUT, NTV, RSV);                                                        \
+    if (sweep && !by_rows) STIR_BSR_SWEEP(BF, OUT, NTV, RSV);                                              \
     hipLaunchKernelGGL((bsr_spmm_kernel<BF, OUT, NTV, RSV>), grid, block, 0, st, blk, feat, slices, f_tiles, \
                        by_rows, A, X, d_Y, d_indptr, d_indices, d_row_ids);                                \
   }
@@ -773,11 +841,8 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       if (rs == 2) STIR_BSR_L(BF, OUT, 1, 2) else STIR_BSR_L(BF, OUT, 1, 1)        \
     }                                                                              \
   } while (0)
-  if (dtype == STIR_BF16) {
-    if (out_dtype == STIR_F32) STIR_BSR(true, 1); else STIR_BSR(true, 0);
-  } else {
-    if (out_dtype == STIR_F32) STIR_BSR(false, 1); else STIR_BSR(false, 0);
-  }
+  STIR_BSR_TYPES(STIR_BSR)
+#undef STIR_BSR_TYPES
 #undef STIR_BSR
 #undef STIR_BSR_L
 #undef STIR_BSR_SWEEP

@@ -44,4 +44,27 @@ inline int vector_class(int feat) {
   return c;
 }
 
+// Feature slices: workgroup L of slice_grid(slices, blocks) takes block `block` (which may lie behind the last:
+// nothing to do) of slice `slice`.  Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2:
+// an XCD works on an eighth of the slices, so it gathers from that much of B.  A slice is dealt out in
+// ceil(8 / slices) interleaved pieces, so that an XCD with a part of one has blocks of all its kinds.
+constexpr int kXcds = 8;
+inline int64_t slice_grid(int slices, int64_t blocks) {
+  if (slices == 1) return blocks;
+  const int pieces = (kXcds + slices - 1) / slices;
+  return kXcds * ceil_div(slices * pieces * ceil_div(blocks, pieces), kXcds);
+}
+__device__ __forceinline__ void slice_block(int64_t L, int slices, int64_t blocks, int& slice, int64_t& block) {
+  const int pieces = (kXcds + slices - 1) / slices;
+  const int64_t piece = (blocks + pieces - 1) / pieces, all = slices * pieces * piece;
+  const int64_t per = (all + kXcds - 1) / kXcds, t = (L & (kXcds - 1)) * per + L / kXcds;
+  if (t >= all || L / kXcds >= per) {
+    slice = 0, block = blocks;
+    return;
+  }
+  slice = (int)(t / (pieces * piece));
+  const int64_t p = t - slice * (pieces * piece);
+  block = p % piece * pieces + p / piece;
+}
+
 }  // namespace stir

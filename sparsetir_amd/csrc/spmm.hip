@@ -67,20 +67,20 @@ __device__ __forceinline__ void reduce_groups(float4 (&acc)[REP], int limit) {
 }
 
 // Store, or accumulate with atomics, the 4*G*REP features a lane group holds for output row
-// `row`.  A lane owns 4 consecutive floats, so issuing the atomics straight from the registers
+// `row` (feat of them are there; rows are `stride` floats apart).  A lane owns 4 consecutive floats, so issuing the atomics straight from the registers
 // would make every atomic instruction touch G addresses 16 bytes apart (4 cache lines per 32
 // lanes, 4 times over).  Instead the group's floats go through the wavefront's piece of LDS
 // (`stage`, 256*REP floats) and come back with lane l holding float k*G + l, so each atomic
 // instruction covers G consecutive floats.  LDS instructions of one wavefront execute in order,
 // no workgroup barrier is involved.
 template <int G, int REP>
-__device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int lane,
+__device__ __forceinline__ void write_row(float* C, int64_t row, int stride, int feat, int lane,
                                           const float4 (&acc)[REP], int atomic, float* stage) {
   const int g = lane / G, gl = lane % G;
   if (atomic == 2) {
     // the only writer of this row in this launch: no atomics needed to add.  All of the row is read
     // before any of it is written: of a width that is no multiple of four, two chunks share features.
-    float* base = C + row * feat;
+    float* base = C + row * stride;
     float4 old[REP];
 #pragma unroll
     for (int r = 0; r < REP; ++r) {
@@ -98,7 +98,7 @@ __device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int l
     return;
   }
   if (!atomic) {
-    float* base = C + row * feat;
+    float* base = C + row * stride;
 #pragma unroll
     for (int r = 0; r < REP; ++r) {
       const int c0 = gl * 4 + r * G * 4;
@@ -122,7 +122,7 @@ __device__ __forceinline__ void write_row(float* C, int64_t row, int feat, int l
     *reinterpret_cast<float4*>(stage + (r * kWave + lane) * 4) = v;
   }
   __builtin_amdgcn_wave_barrier();
-  float* base = C + row * feat + gl;
+  float* base = C + row * stride + gl;
 #pragma unroll
   for (int r = 0; r < REP; ++r) {
 #pragma unroll
@@ -235,7 +235,7 @@ __device__ __forceinline__ void block_rows(const BlockRow* list, int count, floa
           const float4 o = *reinterpret_cast<const float4*>(part + ((w * REP + r) * G + gl) * 4);
           acc[r].x += o.x, acc[r].y += o.y, acc[r].z += o.z, acc[r].w += o.w;
         }
-      write_row<G, REP>(C, b.row, feat, lane, acc, 0, nullptr);
+      write_row<G, REP>(C, b.row, feat, feat, lane, acc, 0, nullptr);
     }
     __syncthreads();
   }
@@ -269,13 +269,13 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat
     // merged rows of a hyb plan: the operator adds to C, as its buckets do; this wavefront is the
     // row's only writer in this launch, long rows are left to csr_long_rows_kernel altogether
     if (later) return;
-    if (g == 0) write_row<G, REP>(C, row, feat, lane, acc, 2, nullptr);
+    if (g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 2, nullptr);
   } else if constexpr (SPLIT) {
-    if (g == 0) write_row<G, REP>(C, row, feat, lane, acc, 0, nullptr);
+    if (g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 0, nullptr);
   } else {
     __shared__ BlockRow list[WAVES];
     __shared__ __attribute__((aligned(16))) float part[WAVES * 4 * G * REP];
-    if (row < m && !later && g == 0) write_row<G, REP>(C, row, feat, lane, acc, 0, nullptr);
+    if (row < m && !later && g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 0, nullptr);
     if (!__syncthreads_or(later)) return;
     if (lane == 0) list[wave] = BlockRow{row, start, end};
     __syncthreads();
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int
   }
   if (row < m && alone) {
     const float4 sum[1] = {acc};
-    write_row<G, 1>(C, row, feat, lane, sum, 0, nullptr);
+    write_row<G, 1>(C, row, feat, feat, lane, sum, 0, nullptr);
   }
   // the longer rows, one after the other, by the whole wavefront
   const bool later = end - start > (SPLIT ? kLongRow : kBlockRow);
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int
     float4 sum[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
     if (!(SPLIT && e - s > kLongRow)) csr_accumulate<G, 1>(sum, s, e, feat, A, B, indices, lane);
     reduce_groups<G, 1>(sum, kWave);
-    if (g == 0) write_row<G, 1>(C, row0 + src / G, feat, lane, sum, 0, nullptr);
+    if (g == 0) write_row<G, 1>(C, row0 + src / G, feat, feat, lane, sum, 0, nullptr);
   }
   if constexpr (!SPLIT) {
     __shared__ BlockRow list[WAVES * NG];
@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int
       for (int q = 0; q < REP; ++q) acc[q] = make_float4(0.f, 0.f, 0.f, 0.f);
       csr_accumulate<G, REP, INDIRECT>(acc, (int)s, (int)e, feat, A, B, indices, lane);
       reduce_groups<G, REP>(acc, kWave);
-      if (g == 0) write_row<G, REP>(C, row, feat, lane, acc, true, stage_all[wave]);
+      if (g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, true, stage_all[wave]);
     }
   }
 }
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256) void csr_spmm_generic_kernel(int m, int feat, 
 // Slot-tile mode (power-of-two width <= 64): a wavefront owns 64 consecutive ELL slots,
 // i.e. 64/width whole ELL rows.  Lane group g owns slots [g*G, g*G+G) of the tile.
 template <int G, int REP, int LOG2W>
-__device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, int feat,
+__device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, int stride, int feat,
                                               const float* __restrict__ B, float* __restrict__ C,
                                               int lane, float* stage) {
   constexpr int W = 1 << LOG2W;
@@ -460,7 +460,7 @@ __device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, in
       const int sl = g * G + c + u;
       const int col = __shfl(my_col, sl, kWave);
       v[u] = __shfl(my_val, sl, kWave);
-      const float* bp = B + (int64_t)col * feat;
+      const float* bp = B + (int64_t)col * stride;
       // a slot of weight zero (padding) adds nothing: its row of B is not fetched
 #pragma unroll
       for (int r = 0; r < REP; ++r) {
@@ -476,7 +476,7 @@ __device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, in
         // end of an ELL row inside this lane group; for W <= CH this folds to a constant
         if (((c + u + 1) & (W - 1)) == 0) {
           const int out_row = __shfl(my_row, (g * G + c + u) >> LOG2W, kWave);
-          if (out_row >= 0) write_row<G, REP>(C, out_row, feat, lane, acc, atomic, stage);
+          if (out_row >= 0) write_row<G, REP>(C, out_row, stride, feat, lane, acc, atomic, stage);
 #pragma unroll
           for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
@@ -488,14 +488,14 @@ __device__ __forceinline__ void hyb_slot_tile(const HybBucket& bk, int64_t t, in
     reduce_groups<G, REP>(acc, W);
     const int out_row = __shfl(my_row, (g * G) >> LOG2W, kWave);
     if (((g * G) & (W - 1)) == 0 && out_row >= 0)
-      write_row<G, REP>(C, out_row, feat, lane, acc, atomic, stage);
+      write_row<G, REP>(C, out_row, stride, feat, lane, acc, atomic, stage);
   }
 }
 
 // Row mode (any width): a wavefront owns one ELL row, or one kRowChunk-slot piece of it when
 // the bucket accumulates, and walks it 64 slots at a time.
 template <int G, int REP>
-__device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int feat,
+__device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int stride, int feat,
                                              const float* __restrict__ B, float* __restrict__ C,
                                              int lane, float* stage) {
   constexpr int CH = G < 8 ? G : 8;
@@ -522,7 +522,7 @@ __device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int
         const int sl = g * G + c + u;
         const int col = __shfl(my_col, sl, kWave);
         v[u] = __shfl(my_val, sl, kWave);  // zero beyond s_end and on padding
-        const float* bp = B + (int64_t)col * feat;
+        const float* bp = B + (int64_t)col * stride;
 #pragma unroll
         for (int r = 0; r < REP; ++r) {
           const int c0 = gl * 4 + r * G * 4;
@@ -536,7 +536,7 @@ __device__ __forceinline__ void hyb_row_tile(const HybBucket& bk, int64_t t, int
     }
   }
   reduce_groups<G, REP>(acc, kWave);
-  if (g == 0) write_row<G, REP>(C, bk.rows[row], feat, lane, acc, bk.atomic, stage);
+  if (g == 0) write_row<G, REP>(C, bk.rows[row], stride, feat, lane, acc, bk.atomic, stage);
 }
 
 // The descriptors of a launch: a table in device memory, or, up to kInlineBuckets of them, the kernel
@@ -567,27 +567,35 @@ __device__ __forceinline__ int find_bucket(const TABLE& table, int nb, int64_t t
 
 template <int G, int REP, class TABLE>
 __global__ __launch_bounds__(256) void hyb_spmm_kernel(const TABLE table, int nb,
-                                                       int64_t tile_base, int64_t tile_end, int feat,
+                                                       int64_t tile_base, int64_t tile_end, int slices, int stride,
                                                        const float* __restrict__ B,
                                                        float* __restrict__ C) {
   __shared__ float stage_all[4][kWave * 4 * REP];  // per-wavefront staging for atomic rows
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   float* stage = stage_all[wave];
-  const int64_t tile = tile_base + (int64_t)blockIdx.x * 4 + wave;
+  int64_t block = blockIdx.x;
+  int feat = stride;
+  if (slices > 1) {
+    int slice;
+    stir::slice_block(blockIdx.x, slices, (tile_end - tile_base + 3) / 4, slice, block);
+    const int f0 = slice * 4 * G * REP;
+    B += f0, C += f0, feat -= f0;
+  }
+  const int64_t tile = tile_base + block * 4 + wave;
   if (tile >= tile_end) return;
   const int k = find_bucket(table, nb, tile);
   const HybBucket bk = table[k];
   const int64_t t = tile - bk.tile_begin;
   switch (bk.log2w) {
-    case 0: hyb_slot_tile<G, REP, 0>(bk, t, feat, B, C, lane, stage); break;
-    case 1: hyb_slot_tile<G, REP, 1>(bk, t, feat, B, C, lane, stage); break;
-    case 2: hyb_slot_tile<G, REP, 2>(bk, t, feat, B, C, lane, stage); break;
-    case 3: hyb_slot_tile<G, REP, 3>(bk, t, feat, B, C, lane, stage); break;
-    case 4: hyb_slot_tile<G, REP, 4>(bk, t, feat, B, C, lane, stage); break;
-    case 5: hyb_slot_tile<G, REP, 5>(bk, t, feat, B, C, lane, stage); break;
-    case 6: hyb_slot_tile<G, REP, 6>(bk, t, feat, B, C, lane, stage); break;
-    default: hyb_row_tile<G, REP>(bk, t, feat, B, C, lane, stage); break;
+    case 0: hyb_slot_tile<G, REP, 0>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 1: hyb_slot_tile<G, REP, 1>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 2: hyb_slot_tile<G, REP, 2>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 3: hyb_slot_tile<G, REP, 3>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 4: hyb_slot_tile<G, REP, 4>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 5: hyb_slot_tile<G, REP, 5>(bk, t, stride, feat, B, C, lane, stage); break;
+    case 6: hyb_slot_tile<G, REP, 6>(bk, t, stride, feat, B, C, lane, stage); break;
+    default: hyb_row_tile<G, REP>(bk, t, stride, feat, B, C, lane, stage); break;
   }
 }
 
@@ -945,6 +953,31 @@ int launch_merged(const MergedRows& mr, int32_t m, int32_t feat, const float* d_
   return 0;
 }
 
+// The lane groups (vector_class) of a hyb launch: those of feat, or narrower ones and several feature slices
+// (slice_block).  Two reasons to cut:
+// - an XCD's L2 (4 MB) holds more rows of B when they are a slice wide.  64 features are the narrowest slice that
+//   costs the gather nothing, as long as every one begins on a 256-byte boundary (the interleave of memory
+//   channels: 96 features of 150 k nodes 84 -> 102 us, 120 features of 127 k nodes 215 -> 247 us).  With two or
+//   four slices it pays or is even up to 160 MB of B, uniform / skewed columns: 25 k nodes, 1 M nonzeros, 128
+//   features 58 -> 44 / 39 -> 41 us, 256 features 132 -> 86 / 80 -> 78 us; 60 k, 720 k, 256: 123 -> 104 / 81 -> 75;
+//   150 k, 1.8 M, 128: 147 -> 145 / 99 -> 92; 300 k, 3 M, 256 (307 MB): 518 -> 539 / 404 -> 384.  With three up to
+//   50 MB: 60 k, 720 k, 192: 91 -> 85 / 61 -> 62; 150 k, 1.2 M, 192 (115 MB): 163 -> 173 / 111 -> 112.
+// - a launch of fewer wavefronts than the card holds (8192) lasts as long as one of them takes for its 64 slots:
+//   10 k nodes, 120 k nonzeros, 256 features: 36.7 us in one piece, 19.3 in slices of 64, 16.9 of 32, 22.0 of 16.
+int slice_class(int32_t feat, int32_t n, int64_t tiles) {
+  constexpr int kNarrowest = 1;              // 32 features, a line of B
+  constexpr int64_t kWavefronts = 8192;
+  const int whole = vector_class(feat);
+  auto slices = [&](int c) { return stir::ceil_div(feat, 16 << c); };
+  // a slice of a chunk that reaches back into its neighbour (chunk_offset) would write what that one writes
+  auto allowed = [&](int c) { return feat % (16 << c) == 0 || feat % (16 << c) >= 4; };
+  int c = whole;
+  if (whole > 2 && feat % 64 == 0 && (int64_t)n * feat * 4 <= (feat % 128 == 0 ? 160000000 : 50000000)) c = 2;
+  while (c > kNarrowest && tiles * slices(c) < kWavefronts) --c;
+  while (c < whole && !allowed(c)) ++c;
+  return c;
+}
+
 HybInline inline_table(const HybBucket* first, int count) {
   HybInline t = {};
   std::copy(first, first + count, t.b);
@@ -953,7 +986,7 @@ HybInline inline_table(const HybBucket* first, int count) {
 
 // Launches the kernels of a hyb operator whose descriptor tables are at d_tiles / d_rows (null: handed
 // over as kernel arguments, at most kInlineBuckets).
-int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_rows, int32_t feat,
+int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_rows, int32_t n, int32_t feat,
                const float* d_B, float* d_C, hipStream_t st) {
   const int nk = (int)t.tiles.size();
   dim3 block(256);
@@ -965,15 +998,17 @@ int launch_hyb(const HybTables& t, const HybBucket* d_tiles, const HybBucket* d_
     const int64_t t0 = t.phase_tile[ph], t1 = t.phase_tile[ph + 1];                                          \
     if (t1 == t0) continue;                                                                                 \
     const int b0 = t.phase_bucket[ph], count = t.phase_bucket[ph + 1] - b0;                                  \
-    const dim3 grid((unsigned)stir::ceil_div(t1 - t0, 4));                                                  \
+    const dim3 grid((unsigned)stir::slice_grid(slices, stir::ceil_div(t1 - t0, 4)));                        \
     if (d_tiles)                                                                                            \
       hipLaunchKernelGGL((hyb_spmm_kernel<G, REP, HybTable>), grid, block, 0, st, HybTable{d_tiles + b0},    \
-                         count, t0, t1, feat, d_B, d_C);                                                    \
+                         count, t0, t1, slices, feat, d_B, d_C);                                            \
     else                                                                                                    \
       hipLaunchKernelGGL((hyb_spmm_kernel<G, REP, HybInline>), grid, block, 0, st,                           \
-                         inline_table(t.tiles.data() + b0, count), count, t0, t1, feat, d_B, d_C);          \
+                         inline_table(t.tiles.data() + b0, count), count, t0, t1, slices, feat, d_B, d_C);  \
   }
-  switch (vector_class(feat)) {
+  const int vclass = slice_class(feat, n, t.total_tiles / std::max<int64_t>(1, t.phase_tile.size() - 1));
+  const int slices = vclass < 0 ? 1 : (int)stir::ceil_div(feat, 16 << vclass);
+  switch (vclass) {
     case 0: STIR_HYB(4, 1); break;
     case 1: STIR_HYB(8, 1); break;
     case 2: STIR_HYB(16, 1); break;
@@ -1165,7 +1200,7 @@ int stir_hyb_spmm_f32(const stir_hyb_plan* plan, int32_t feat, const float* d_B,
   if (plan->merged && vector_class(feat) >= 0 && (plan->num_col_parts > kMaxPhases || feat >= kMergedFromFeat))
     return launch_merged(plan->rows, plan->m, feat, d_B, d_C, static_cast<hipStream_t>(stream));
   const HybBucket* d_rows = plan->d_tables ? plan->d_tables + nk : nullptr;
-  return launch_hyb(plan->tables, plan->d_tables, d_rows, feat, d_B, d_C, static_cast<hipStream_t>(stream));
+  return launch_hyb(plan->tables, plan->d_tables, d_rows, plan->n, feat, d_B, d_C, static_cast<hipStream_t>(stream));
 }
 
 int stir_hyb_spmm_f32_noalloc(int32_t m, int32_t n, int32_t num_col_parts, int32_t num_buckets,
@@ -1187,7 +1222,7 @@ int stir_hyb_spmm_f32_noalloc(int32_t m, int32_t n, int32_t num_col_parts, int32
                kStaticBuckets);
   STIR_REQUIRE(d_B && d_C, "hyb_spmm_noalloc: null pointer argument");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (nk <= kInlineBuckets) return launch_hyb(tables, nullptr, nullptr, feat, d_B, d_C, st);
+  if (nk <= kInlineBuckets) return launch_hyb(tables, nullptr, nullptr, n, feat, d_B, d_C, st);
   HybBucket* d_tables = nullptr;
   if (static_scratch(&d_tables) != 0) return -1;
   // only the table the kernel for this feature width reads is written
@@ -1201,7 +1236,7 @@ int stir_hyb_spmm_f32_noalloc(int32_t m, int32_t n, int32_t num_col_parts, int32
     hipLaunchKernelGGL(hyb_table_fill_kernel, dim3(1), dim3(256), 0, st, chunk, count, dst + first);
   }
   STIR_LAUNCH_CHECK();
-  return launch_hyb(tables, d_tables, d_tables + kStaticBuckets, feat, d_B, d_C, st);
+  return launch_hyb(tables, d_tables, d_tables + kStaticBuckets, n, feat, d_B, d_C, st);
 }
 
 int stir_hyb_plan_destroy(stir_hyb_plan* plan) {

@@ -218,7 +218,7 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
  * workspaces of their own; the same bits come out every time.  0 bytes: no workspace is needed, it may
  * be null and the call is stir_csr_spmm_f32.
  */
-size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t feat, int64_t nnz);
+size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz);
 int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A,
                                 const float* d_B, float* d_C, const int32_t* d_indptr,
                                 const int32_t* d_indices, void* d_workspace, void* stream);

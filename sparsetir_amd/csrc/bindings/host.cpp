@@ -388,7 +388,7 @@ PyObject* launcher_new(PyTypeObject*, PyObject* args, PyObject*) {
   }
   if (l->kind == kCsr && l->sizes->size() == 4) {
     const std::vector<int64_t>& n = *l->sizes;
-    l->workspace_bytes = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[2], n[3]);
+    l->workspace_bytes = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
   }
   return reinterpret_cast<PyObject*>(l);
 }

@@ -76,7 +76,7 @@ __device__ __forceinline__ void store4(float* q, const float4& v) {
 }
 
 template <int G, int REP>
-__global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(int m, int feat, int64_t nnz, int items,
+__global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(int m, int stride, int slices, int64_t nnz, int items,
                                                               const float* __restrict__ A,
                                                               const float* __restrict__ B, float* __restrict__ C,
                                                               const int32_t* __restrict__ indptr,
@@ -95,7 +95,17 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int base = indptr[0];
   const int64_t total = m + min(nnz, (int64_t)indptr[m]) - base;
-  const int64_t d0 = (int64_t)blockIdx.x * items, d1 = min(total, d0 + items);
+  int feat = stride;
+  int64_t wg = blockIdx.x;
+  if (slices > 1) {  // see slice_block
+    const int64_t wgs = (m + nnz + items - 1) / items;
+    int slice;
+    stir::slice_block(blockIdx.x, slices, wgs, slice, wg);
+    const int f0 = slice * kPad;
+    B += f0, C += f0, feat -= f0;
+    counters += slice * wgs, partials += slice * wgs * 2 * kPad;
+  }
+  const int64_t d0 = wg * items, d1 = min(total, d0 + items);
   if (d0 >= total) return;
   if (wave < 2) {
     const int64_t d = wave ? d1 : d0;
@@ -131,8 +141,8 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
     while (empty) {
       const int k = __ffsll((long long)empty) - 1;
       empty &= empty - 1;
-      float* row = C + (int64_t)(r0 + wave * kWave + k) * feat;
-      for (int f = lane; f < feat; f += kWave) __builtin_nontemporal_store(0.f, row + f);
+      float* row = C + (int64_t)(r0 + wave * kWave + k) * stride;
+      for (int f = lane; f < min(feat, kPad); f += kWave) __builtin_nontemporal_store(0.f, row + f);
     }
   }
   __syncthreads();
@@ -157,7 +167,7 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
       const int2 q = nz[min(p, kSlots - 1)];
       f[u] = live ? ends[min(p, kSlots - 1)] : 0;
       v[u] = live ? __int_as_float(q.y) : 0.f;
-      const float* bp = B + (int64_t)q.x * feat;
+      const float* bp = B + (int64_t)q.x * stride;
 #pragma unroll
       for (int r = 0; r < REP; ++r) {
         const int c0 = gl * 4 + r * G * 4;
@@ -170,7 +180,7 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
       for (int r = 0; r < REP; ++r) fma4(acc[r], v[u], x[u][r]);
       if (f[u]) {
         const bool keep = mid && !flushed;
-        float* row = C + (int64_t)(f[u] - 1) * feat;
+        float* row = C + (int64_t)(f[u] - 1) * stride;
 #pragma unroll
         for (int r = 0; r < REP; ++r) {
           const int c0 = gl * 4 + r * G * 4;
@@ -211,9 +221,9 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
     for (int r = 0; r < REP; ++r) {
       const int c0 = gl * 4 + r * G * 4;
       if (which == 0 && k >= 0) {
-        if (c0 < feat) store4(C + (int64_t)(head_row - 1) * feat + chunk_offset(c0, feat), sum[r]);
+        if (c0 < feat) store4(C + (int64_t)(head_row - 1) * stride + chunk_offset(c0, feat), sum[r]);
       } else {
-        coherent_store(partials + ((int64_t)blockIdx.x * 2 + which) * kPad + c0, sum[r]);
+        coherent_store(partials + (wg * 2 + which) * kPad + c0, sum[r]);
       }
     }
   }
@@ -259,7 +269,7 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
 #pragma unroll
       for (int q = 0; q < REP; ++q) {
         const int c0 = gl * 4 + q * G * 4;
-        if (c0 < feat) store4(C + (int64_t)r * feat + chunk_offset(c0, feat), sum[q]);
+        if (c0 < feat) store4(C + (int64_t)r * stride + chunk_offset(c0, feat), sum[q]);
       }
     }
   }
@@ -276,46 +286,66 @@ int64_t workgroups(int32_t m, int64_t nnz) {
   return stir::ceil_div(m + nnz, entries_per_workgroup(m, nnz));
 }
 
-// Below, the search for its entries costs a workgroup more than it gains (4096 rows, 65 k nonzeros, 32
-// features: 8.6 us against 6.9); above, two launches over rows read B as fast and leave no partial rows
-// (2.4 M rows, 61.9 M nonzeros, 128 features: 5.49 ms against 4.98).  Between (old / new, us):
-// 6 k rows, 90 k nonzeros, 128 features 15.5 / 10.0; 24 k, 360 k, 33: 19.4 / 13.1; 50 k, 450 k, 8: 24.3 / 11.6;
-// 169 k, 1.17 M, 47: 50.7 / 38.2; 115 k, 2.3 M, 64: 92 / 85; 100 k, 1.5 M, 128: 121 / 117.
-bool balanced(int32_t m, int32_t feat, int64_t nnz) {
-  if (stir::vector_class(feat) < 0 || nnz * feat >= 500000000) return false;
-  return m >= 8192 || nnz * feat >= 3000000;
+// Lane groups as wide as feat, or of 64 features and several feature slices (slice_block): an XCD's L2 holds
+// more rows of B a slice wide, which pays for looking for the entries once per slice from 1.5e8 multiplications
+// on, as long as slices begin on 256-byte boundaries and B is not far beyond what the last level holds.
+// In one piece / in slices, uniform and skewed columns, us:
+//   25 k rows, 1 M nonzeros, 256 features 136 / 87, 84 / 81 (300 k nonzeros 49 / 40, 31 / 38);
+//   60 k, 720 k, 256: 118 / 97, 71 / 72 (128: 58 / 54, 36 / 39); 150 k, 1.2 M, 192: 154 / 142, 102 / 90;
+//   300 k, 7.8 M, 128: 573 / 563, 434 / 377; the same, 256 (307 MB): 1161 / 1167, 1016 / 797;
+//   600 k, 6 M, 256 (614 MB): 932 / 1012, 786 / 757.
+// The upper end of the products is that of the measurements (and bounds the workspace).
+int slice_class(int32_t n, int32_t feat, int64_t nnz) {
+  const int whole = stir::vector_class(feat);
+  const int64_t work = nnz * feat;
+  const bool cut = whole > 2 && feat % 64 == 0 && work >= 150000000 && work <= 2500000000 &&
+                   (int64_t)n * feat * 4 <= 320000000;
+  return cut ? 2 : whole;
 }
 
-size_t padded(int feat) { return size_t(16) << stir::vector_class(feat); }
+// Below, the search for its entries costs a workgroup more than it gains (4096 rows, 65 k nonzeros, 32
+// features: 8.6 us against 6.9); above, if not in slices, two launches over rows read B as fast and leave no
+// partial rows (2.4 M rows, 61.9 M nonzeros, 128 features: 5.49 ms against 4.98).  Between (old / new, us):
+// 6 k rows, 90 k nonzeros, 128 features 15.5 / 10.0; 24 k, 360 k, 33: 19.4 / 13.1; 50 k, 450 k, 8: 24.3 / 11.6;
+// 169 k, 1.17 M, 47: 50.7 / 38.2; 115 k, 2.3 M, 64: 92 / 85; 100 k, 1.5 M, 128: 121 / 117.
+bool balanced(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
+  const int c = stir::vector_class(feat);
+  if (c < 0 || (nnz * feat >= 500000000 && slice_class(n, feat, nnz) == c)) return false;
+  return m >= 8192 || nnz * feat >= 3000000;
+}
 
 }  // namespace
 
 extern "C" {
 
-size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t feat, int64_t nnz) {
-  if (m < 0 || feat <= 0 || nnz < 0 || !balanced(m, feat, nnz)) return 0;
+size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
+  if (m < 0 || n < 0 || feat <= 0 || nnz < 0 || !balanced(m, n, feat, nnz)) return 0;
   const size_t wgs = (size_t)workgroups(m, nnz);
-  return (wgs * 4 + 15) / 16 * 16 + wgs * 2 * padded(feat) * 4;
+  const int c = slice_class(n, feat, nnz);
+  const size_t parts = wgs * stir::ceil_div(feat, 16 << c);
+  return (parts * 4 + 15) / 16 * 16 + parts * 2 * (size_t(16) << c) * 4;
 }
 
 int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A, const float* d_B,
                                 float* d_C, const int32_t* d_indptr, const int32_t* d_indices, void* d_workspace,
                                 void* stream) {
   STIR_REQUIRE(m >= 0 && n >= 0 && feat > 0 && nnz >= 0, "csr_spmm: bad sizes m=%d n=%d feat=%d", m, n, feat);
-  if (!balanced(m, feat, nnz))
+  if (!balanced(m, n, feat, nnz))
     return stir_csr_spmm_f32(m, n, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, stream);
   STIR_REQUIRE(d_B && d_C && d_indptr && d_workspace && (nnz == 0 || (d_A && d_indices)),
                "csr_spmm: null pointer argument");
   const int64_t wgs = workgroups(m, nnz);
-  STIR_REQUIRE(wgs < (int64_t(1) << 31), "csr_spmm: %lld workgroups exceed one launch", (long long)wgs);
+  const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c);
+  const int64_t grid = stir::slice_grid(slices, wgs);
+  STIR_REQUIRE(grid < (int64_t(1) << 31), "csr_spmm: %lld workgroups exceed one launch", (long long)grid);
   const int items = entries_per_workgroup(m, nnz);
   uint32_t* counters = static_cast<uint32_t*>(d_workspace);
-  float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + (size_t(wgs) * 4 + 15) / 16 * 16);
+  float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + (size_t(wgs) * slices * 4 + 15) / 16 * 16);
 #define STIR_BALANCED(G, REP)                                                                                    \
-  hipLaunchKernelGGL((csr_balanced_kernel<G, REP>), dim3((unsigned)wgs), dim3(kBlock), 0,                         \
-                     static_cast<hipStream_t>(stream), m, feat, nnz, items, d_A, d_B, d_C, d_indptr, d_indices,   \
+  hipLaunchKernelGGL((csr_balanced_kernel<G, REP>), dim3((unsigned)grid), dim3(kBlock), 0,                         \
+                     static_cast<hipStream_t>(stream), m, feat, slices, nnz, items, d_A, d_B, d_C, d_indptr, d_indices,   \
                      counters, partials)
-  switch (stir::vector_class(feat)) {
+  switch (c) {
     case 0: STIR_BALANCED(4, 1); break;
     case 1: STIR_BALANCED(8, 1); break;
     case 2: STIR_BALANCED(16, 1); break;

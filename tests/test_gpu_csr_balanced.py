@@ -55,3 +55,10 @@ def test_rows_across_workgroups(dev, feat, m, most):
     got = c[0].cpu().numpy().reshape(m, feat)
     assert np.all(got[deg == 0] == 0.0)
     _check(got, indptr, indices[:-spare], vals[:-spare], x, f"m={m} feat={feat}")
+
+
+@pytest.mark.parametrize("feat,m,most", [(128, 9001, 300), (192, 9001, 200), (256, 40003, 34), (320, 9001, 120),
+                                         (512, 9001, 80)])
+def test_feature_slices(dev, feat, m, most):
+    """Products large enough for slices of 64 features, two to eight of them."""
+    test_rows_across_workgroups(dev, feat, m, most)

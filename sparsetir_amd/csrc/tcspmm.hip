@@ -6,14 +6,20 @@
 //   C[io*t + ii, f] = sum over groups jo of tile io, ji < 16:  A[jo, ii, ji] * B[indices[jo, ji], f]
 // fp16 inputs, fp32 accumulation, fp16 or fp32 output.
 //
-// Same tiling as the BSR kernel: a workgroup of four wavefronts owns (row tile, 128 features),
-// a wavefront t rows x 32 features.  A step covers two groups (32 gathered rows of B): A[jo] is
-// already in MFMA A-operand order (a lane's 8 k values are contiguous), the 32 gathered rows of
-// B go through LDS, interleaved into (k, k+1) pairs on the way, double-buffered, with the next
-// step's gathers in flight during the multiply.  Tiles of 32 rows multiply with two
-// v_mfma_f32_32x32x16_f16 per step (one per group); tiles of 16 rows with v_mfma_f32_16x16x32_f16,
-// whose k extent of 32 is the step's two groups, once per 16 features; tiles of 8 rows are the
-// upper half of a 16-row operand whose other rows are zero.
+// With a plan (stir_tc_plan: the long tiles listed once, longest first, in pieces) a product is one launch of
+// tcspmm_units_kernel.  Bound by the gather of rows of B where there are tiles enough (179 k rows, 4.5 M
+// nonzeros, 64 features: 5.8 TB/s), else by the chain id -> row of B -> product of the longest unit.  Before, the
+// tiles of up to 16 steps went as below and the pieces of the others in a second launch, a workgroup of 16
+// wavefronts each; us: 25.9 k rows, 626 k nonzeros, 32 features 23.4 -> 9.4; 167 k, 3.8 M, 32: 81 -> 46; 24 k,
+// 244 k, 64: 22.4 -> 12.5; 200 k, 4 M, 64: 92 -> 58; 33 k, 648 k, 224: 49 -> 41.5; 169 k, 1.17 M, 128: 50.8 -> 48.3.
+//
+// Without a plan: a workgroup of four wavefronts owns (row tile, 128 features), a wavefront t rows x 32 features.
+// A step covers two groups (32 gathered rows of B): A[jo] is already in MFMA A-operand order (a lane's 8 k values
+// are contiguous), the 32 gathered rows of B go through LDS, interleaved into (k, k+1) pairs on the way,
+// double-buffered, with the next step's gathers in flight during the multiply.  Tiles of 32 rows multiply with
+// two v_mfma_f32_32x32x16_f16 per step (one per group); tiles of 16 rows with v_mfma_f32_16x16x32_f16, whose k
+// extent of 32 is the step's two groups, once per 16 features; tiles of 8 rows are the upper half of a 16-row
+// operand whose other rows are zero.
 //
 // A row tile that touches thousands of distinct columns (a hub row of a power-law graph) would be
 // one long serial chain in one workgroup.  With fp32 output such tiles are cut into up to kSplit
@@ -21,13 +27,7 @@
 // of those tiles.  With fp16 output partial sums would be rounded once per unit; there, tiles of
 // more than kLongSteps steps are left to a second launch (tcspmm_long_kernel) whose workgroups
 // have 16 wavefronts that split the steps of the tile among them and add their fp32 partial sums
-// through LDS before the one write of the tile.  (For fp32 output that launch is the slower of the
-// two ways: the launches run in turn.  Running them side by side on two streams was tried for
-// fp16 output and lost: workgroups of 16 wavefronts wait for room beside the other launch, and
-// the hub tile's chain runs slower on a shared compute unit than the overlap gains.)
-// With a plan (stir_tc_plan: the long tiles listed once, longest first, in pieces of at most
-// kPieceSteps steps) the second launch has a workgroup per piece and the hub tiles are spread
-// over many compute units; fp32 partial tiles in the plan's memory, one rounding at the end.
+// through LDS before the one write of the tile.
 #include <algorithm>
 #include <vector>
 
@@ -161,7 +161,7 @@ __global__ __launch_bounds__(256) void tcspmm_clear_long_kernel(int tile, int fe
 
 // OUT: 0 = fp16 output, 1 = fp32 output.  SPLIT: grid is (mb * f_tiles, kSplit); the units of a
 // long tile take equal shares of its steps and add with atomics, unit 0 of a short tile stores.
-template <int T, int OUT, bool SPLIT, bool SKIP_LONG = (OUT == 0)>
+template <int T, int OUT, bool SPLIT>
 __global__ __launch_bounds__(256) void tcspmm_kernel(int feat, int64_t mb, int f_tiles,
                                                      const uint16_t* __restrict__ A,
                                                      const uint16_t* __restrict__ B, void* __restrict__ C,
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(256) void tcspmm_kernel(int feat, int64_t mb, int f
   const int64_t rows_total = (g_end - g_begin) * kGroup;  // gathered rows of B for this tile
   const int steps = (int)((rows_total + 31) / 32);
   const int32_t* rowlist = indices + g_begin * kGroup;
-  if constexpr (SKIP_LONG) {
+  if constexpr (OUT == 0) {
     if (steps > kLongSteps) return;  // left to the launch for long tiles; uniform over the workgroup
   }
   int it_begin = 0, it_end = steps;
@@ -416,25 +416,28 @@ __global__ __launch_bounds__(64 * (32 / NTL)) void tcspmm_long_kernel(int feat, 
   }
 }
 
-// ---- fp16 output with a plan (stir_tc_plan): the long tiles are listed once, longest first, and
-// cut into pieces of at most kPieceSteps steps, a workgroup of 16 wavefronts each, so that the
-// hub tiles of a power-law graph are spread over many compute units from the start of the launch
-// and no workgroup is started only to find its tile short.  A tile that is one piece is written
-// as fp16 by its workgroup; the pieces of a longer tile leave fp32 partial tiles in the plan's
-// scratch memory, and the workgroup that finishes last among the pieces of a tile (per feature
-// tile: a counter in device memory, which that workgroup sets back to zero) adds them up in piece
-// order and rounds once -- no launch of its own for the sums, and the same bits whichever
-// workgroup comes last.  The partial tiles are written and read with device-coherent accesses
-// (they pass the XCD's L2), so that no workgroup has to write back or invalidate a whole L2 --
-// which a release or acquire at device scope does, and which costs more than the extra launch.
-constexpr int kPieceSteps = 128;
+// ---- with a plan (stir_tc_plan): one launch of units, each a whole row tile of at most kPieceSteps steps or a
+// piece of that many of a longer one.  The pieces are listed once by the plan, the longest tiles first, and come
+// before the whole tiles in the launch.  A unit is a workgroup of W wavefronts for (T rows) x (32 * NTL
+// features) that take its steps in turn: wavefront w the steps w, w + W, ..., each with an image of its step's 32
+// gathered rows of B in its own LDS -- no workgroup barrier in the loop, the LDS operations of one wavefront
+// execute in order -- and the partial results meet in LDS at the end.  The image is the rows as they are, 16-byte
+// unit c of row k at place c ^ swizzle(k), and comes out in MFMA operand order through the transposing read
+// ds_read_b64_tr_b16 (see bsr_tile in bsr.hip; the XOR keeps the two blocks of 16 lanes that the LDS serves
+// together on distinct banks).
+// The pieces of a long tile leave fp32 partial tiles in the plan's scratch memory, and the workgroup that
+// finishes last among the pieces of a tile (per feature tile: a counter in device memory, which that workgroup
+// sets back to zero) adds them up in piece order and rounds once: the same bits whichever workgroup comes last.
+// The partial tiles are written and read with device-coherent accesses (they pass the XCD's L2), so that no
+// workgroup has to write back or invalidate a whole L2, as a release or acquire at device scope does.
+constexpr int kPieceSteps = 32;
 
 struct TcPiece {
   int32_t tile, step_begin, step_end;
-  int32_t slot;        // partial tile in the scratch memory, or -1: the piece is the whole tile
+  int32_t slot;        // partial tile in the scratch memory
   int32_t first_slot;  // of the tile's pieces
   int32_t pieces;      // of the tile
-  int32_t multi;       // number of the tile among the tiles of several pieces
+  int32_t multi;       // number of the tile among the long tiles
   int32_t pad;
 };
 
@@ -445,46 +448,206 @@ __device__ __forceinline__ float coherent_load(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int T, int NTL, int OUT>
-__global__ __launch_bounds__(64 * (32 / NTL)) void tcspmm_pieces_kernel(int feat, int f_tiles,
-                                                                        const TcPiece* __restrict__ pieces,
-                                                                        const uint16_t* __restrict__ A,
-                                                                        const uint16_t* __restrict__ B,
-                                                                        void* __restrict__ C,
-                                                                        float* scratch, uint32_t* arrived,
-                                                                        const int32_t* __restrict__ indptr,
-                                                                        const int32_t* __restrict__ indices) {
-  extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
-  __shared__ int last_of_tile;
-  constexpr int TF = 32 * NTL;
-  const TcPiece pc = pieces[blockIdx.x / f_tiles];
-  const int f_tile = (int)(blockIdx.x % f_tiles);
-  const int f0 = f_tile * TF;
-  const int64_t io = pc.tile;
-  // a plan made from other contents of indptr: stay inside the tile as it is now
-  const int s_end = min(pc.step_end, tile_steps(indptr, io));
-  if (pc.slot < 0) {
-    tcspmm_long_steps<T, NTL>(lds, feat, io, f0, pc.step_begin, s_end, A, B, indptr, indices,
-                              [&](int row, int fcol, float sum) {
-                                const int64_t off = (io * T + row) * feat + fcol;
-                                if constexpr (OUT == 1) {
-                                  static_cast<float*>(C)[off] = sum;
-                                } else {
-                                  const _Float16 hv = (_Float16)sum;
-                                  static_cast<uint16_t*>(C)[off] = __builtin_bit_cast(uint16_t, hv);
-                                }
-                              });
-    return;
+typedef __fp16 tr16x4 __attribute__((__vector_size__(4 * sizeof(__fp16))));  // result type of the transposing LDS read
+#define STIR_LDS __attribute__((address_space(3)))
+
+// 8 consecutive k of one feature per lane: two transposing reads `next` bytes (four rows of k) apart
+__device__ __forceinline__ f16x8 tc_read_b(const char* at, int next) {
+  union {
+    tr16x4 t[2];
+    f16x8 v;
+  } u;
+  u.t[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at));
+  u.t[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at + next));
+  return u.v;
+}
+
+// four consecutive features of a row of C; aligned: as one store
+template <int OUT>
+__device__ __forceinline__ void tc_store4(void* C, int64_t off, const float4& v, bool aligned) {
+  if constexpr (OUT == 1) {
+    float* q = static_cast<float*>(C) + off;
+    if (aligned)
+      *reinterpret_cast<float4*>(q) = v;
+    else
+      q[0] = v.x, q[1] = v.y, q[2] = v.z, q[3] = v.w;
+  } else {
+    const _Float16 h[4] = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+    uint16_t* q = static_cast<uint16_t*>(C) + off;
+    if (aligned) {
+      uint2 out;
+      out.x = (uint32_t)__builtin_bit_cast(uint16_t, h[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, h[1]) << 16);
+      out.y = (uint32_t)__builtin_bit_cast(uint16_t, h[2]) | ((uint32_t)__builtin_bit_cast(uint16_t, h[3]) << 16);
+      *reinterpret_cast<uint2*>(q) = out;
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) q[u] = __builtin_bit_cast(uint16_t, h[u]);
+    }
   }
+}
+
+template <int T, int NTL, int W, int OUT>
+__global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t mb, int f_tiles, int64_t n_pieces,
+                                                              const TcPiece* __restrict__ pieces,
+                                                              const uint16_t* __restrict__ A,
+                                                              const uint16_t* __restrict__ B, void* __restrict__ C,
+                                                              int aligned, float* scratch, uint32_t* arrived,
+                                                              const int32_t* __restrict__ indptr,
+                                                              const int32_t* __restrict__ indices) {
+  using Acc = TcAcc<T == 32>;
+  constexpr int TF = 32 * NTL;
+  constexpr int FCN = TF / 8;             // 16-byte units of a staged row
+  constexpr int LOADS = FCN / 2;          // ... of a step's 32 rows per lane
+  constexpr int XB = 32 * TF * 2;         // bytes of a wavefront's image
+  constexpr int REGS = Acc::kRegs;
+  constexpr int ATONCE = NTL * 8 / REGS ? NTL * 8 / REGS : 1;  // 32-feature tiles summed at a time: what fits
+  constexpr int RB = ATONCE * REGS * 64 * 4;                   // bytes per wavefront of a sum
+  __shared__ __attribute__((aligned(16))) char lds[W * (XB > RB ? XB : RB)];
+  __shared__ int last_of_tile;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int f_tile = (int)(blockIdx.x % f_tiles);
+  const int64_t unit = blockIdx.x / f_tiles;
+  const int f0 = f_tile * TF;
+  TcPiece pc;
+  pc.slot = -1;
+  int64_t io = unit - n_pieces;
+  int s_begin = 0, s_end = 0;
+  if (unit < n_pieces) {
+    pc = pieces[unit];
+    io = pc.tile;
+    // a plan made from other contents of indptr: stay inside the tile as it is now
+    s_begin = pc.step_begin, s_end = min(pc.step_end, tile_steps(indptr, io));
+  } else {
+    if (io >= mb) return;
+    s_end = tile_steps(indptr, io);
+    if (s_end > kPieceSteps) return;  // in pieces
+  }
+  const int64_t g_begin = indptr[io], g_end = indptr[io + 1];
+  const int64_t rows_total = (g_end - g_begin) * kGroup;
+  const int32_t* rowlist = indices + g_begin * kGroup;
+  char* image = lds + wave * XB;
+
+  auto swizzle = [](int k) {
+    return (FCN == 4 ? 0 : FCN == 8 ? 4 * ((k >> 1) & 1) : 4 * (k & 3)) ^ (T == 32 ? 0 : 2 * ((k >> 3) & 1));
+  };
+  // staging role: unit c of the rows k0 + u * (64 / FCN)
+  const int c = lane % FCN, k0 = lane / FCN;
+  const bool live = f0 + 8 * c < feat;
+  uint32_t put[LOADS];
+#pragma unroll
+  for (int u = 0; u < LOADS; ++u) {
+    const int k = k0 + u * (64 / FCN);
+    put[u] = (uint32_t)((k * FCN + (c ^ swizzle(k))) * 16);
+  }
+  // operand role: a block of 16 lanes reads four rows of two units
+  const int sl = lane & 15, kr = sl >> 2;
+  uint32_t get[NTL][T == 32 ? 1 : 2];
+#pragma unroll
+  for (int t = 0; t < NTL; ++t) {
+    if constexpr (T == 32) {
+      const int k = 8 * (lane >> 5) + kr, cc = 4 * t + 2 * ((lane >> 4) & 1) + ((sl & 3) >> 1);
+      get[t][0] = (uint32_t)((k * FCN + (cc ^ swizzle(k))) * 16 + (sl & 1) * 8);
+    } else {
+      const int k = 8 * (lane >> 4) + kr;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        const int cc = 4 * t + 2 * nt + ((sl & 3) >> 1);
+        get[t][nt] = (uint32_t)((k * FCN + (cc ^ swizzle(k))) * 16 + (sl & 1) * 8);
+      }
+    }
+  }
+
+  Acc acc[NTL];
+#pragma unroll
+  for (int t = 0; t < NTL; ++t) acc[t].clear();
+
+  // The row ids of a step are requested a step (of this wavefront) before its rows of B, so that a step costs
+  // one memory round trip, not two in a row.
+  int id = 0;
+  auto fetch_ids = [&](int it) {
+    const int64_t k = (int64_t)it * 32 + (lane & 31);
+    id = k < rows_total ? rowlist[k] : -1;  // the second group of a tile's last step may not exist
+  };
+  u32x4 x[LOADS], a_next[2];
+  auto fetch = [&](int it) {
+    tc_load_a<T>(a_next, A, g_begin + 2 * it, g_end, lane);
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) {
+      const int row = __shfl(id, k0 + u * (64 / FCN), 64);
+      x[u] = u32x4{0, 0, 0, 0};
+      if (live && row >= 0) x[u] = *reinterpret_cast<const u32x4*>(B + (int64_t)row * feat + f0 + 8 * c);
+    }
+    if (it + W < s_end) fetch_ids(it + W);
+  };
+  if (s_begin + wave < s_end) {
+    fetch_ids(s_begin + wave);
+    fetch(s_begin + wave);
+  }
+  for (int it = s_begin + wave; it < s_end; it += W) {
+    const u32x4 a[2] = {a_next[0], a_next[1]};
+#pragma unroll
+    for (int u = 0; u < LOADS; ++u) *reinterpret_cast<u32x4*>(image + put[u]) = x[u];
+    if (it + W < s_end) fetch(it + W);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < NTL; ++t) {
+      if constexpr (T == 32) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d)
+          acc[t].r = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              __builtin_bit_cast(f16x8, a[d]), tc_read_b(image + get[t][0] + 16 * d * FCN * 16, 4 * FCN * 16),
+              acc[t].r, 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt)
+          acc[t].r[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(f16x8, a[0]), tc_read_b(image + get[t][nt], 4 * FCN * 16), acc[t].r[nt], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+  }
+
+  // ---- the sums over the wavefronts, four consecutive features per thread
+  const int used = min(W, s_end - s_begin);
   const int64_t elems = (int64_t)T * feat;
-  float* part = scratch + (int64_t)pc.slot * elems;
-  tcspmm_long_steps<T, NTL>(lds, feat, io, f0, pc.step_begin, s_end, A, B, indptr, indices,
-                            [&](int row, int fcol, float sum) { coherent_store(part + (int64_t)row * feat + fcol, sum); });
+  float* red = reinterpret_cast<float*>(lds);  // [wavefront][tile][register][lane]
+  float* part = pc.slot < 0 ? nullptr : scratch + (int64_t)pc.slot * elems;
+#pragma unroll
+  for (int t0 = 0; t0 < NTL; t0 += ATONCE) {
+    __syncthreads();  // images, or the sums before, are done with
+#pragma unroll
+    for (int t = 0; t < ATONCE; ++t)
+#pragma unroll
+      for (int v = 0; v < REGS; ++v) red[((wave * ATONCE + t) * REGS + v) * 64 + lane] = acc[t0 + t].get(v);
+    __syncthreads();
+    for (int e = tid; e < T * ATONCE * 8; e += 64 * W) {
+      const int row = e / (ATONCE * 8), t = e % (ATONCE * 8) / 8, col = e % 8 * 4;
+      const int v = T == 32 ? (row & 3) + 4 * (row >> 3) : (row & 3) + 4 * (col >> 4);
+      const int l = T == 32 ? col + 32 * ((row >> 2) & 1) : (col & 15) + 16 * (row >> 2);
+      float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int w = 0; w < used; ++w) {
+        const float4 o = *reinterpret_cast<const float4*>(red + ((w * ATONCE + t) * REGS + v) * 64 + l);
+        sum.x += o.x, sum.y += o.y, sum.z += o.z, sum.w += o.w;
+      }
+      const int fcol = f0 + (t0 + t) * 32 + col;
+      if (fcol >= feat) continue;
+      if (!part) {
+        tc_store4<OUT>(C, (io * T + row) * feat + fcol, sum, aligned);
+      } else {
+        float* q = part + (int64_t)row * feat + fcol;
+        coherent_store(q, sum.x), coherent_store(q + 1, sum.y), coherent_store(q + 2, sum.z), coherent_store(q + 3, sum.w);
+      }
+    }
+  }
+  if (!part) return;
   // Every wavefront waits until its stores have arrived, then one thread counts the workgroup
   // in: whoever counts last finds the partial tiles of all the others in memory.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     uint32_t* counter = arrived + (int64_t)pc.multi * f_tiles + f_tile;
     const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const bool last = before + 1 == (uint32_t)pc.pieces;
@@ -493,36 +656,27 @@ __global__ __launch_bounds__(64 * (32 / NTL)) void tcspmm_pieces_kernel(int feat
   }
   __syncthreads();
   if (!last_of_tile) return;
-  // C[tile, f0 .. f0 + TF) = the partial tiles added in piece order, rounded once; four
-  // consecutive features per thread (feat is a multiple of 32)
+  // C[tile, f0 .. f0 + TF) = the partial tiles added in piece order, rounded once
   const float* first = scratch + (int64_t)pc.first_slot * elems;
-  for (int w = threadIdx.x; w < T * (TF / 4); w += 64 * (32 / NTL)) {
+  for (int w = tid; w < T * (TF / 4); w += 64 * W) {
     const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
     if (fcol >= feat) continue;
     const int64_t e = (int64_t)row * feat + fcol;
     float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int p0 = 0; p0 < pc.pieces; p0 += 4) {
-      float4 x[4];
+      float4 y[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        y[u] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (p0 + u < pc.pieces) {
           const float* at = first + (p0 + u) * elems + e;
-          x[u] = make_float4(coherent_load(at), coherent_load(at + 1), coherent_load(at + 2), coherent_load(at + 3));
+          y[u] = make_float4(coherent_load(at), coherent_load(at + 1), coherent_load(at + 2), coherent_load(at + 3));
         }
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sum.x += x[u].x, sum.y += x[u].y, sum.z += x[u].z, sum.w += x[u].w;
+      for (int u = 0; u < 4; ++u) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
     }
-    if constexpr (OUT == 1) {
-      *reinterpret_cast<float4*>(static_cast<float*>(C) + io * elems + e) = sum;
-    } else {
-      const _Float16 h0 = (_Float16)sum.x, h1 = (_Float16)sum.y, h2 = (_Float16)sum.z, h3 = (_Float16)sum.w;
-      uint2 out;
-      out.x = (uint32_t)__builtin_bit_cast(uint16_t, h0) | ((uint32_t)__builtin_bit_cast(uint16_t, h1) << 16);
-      out.y = (uint32_t)__builtin_bit_cast(uint16_t, h2) | ((uint32_t)__builtin_bit_cast(uint16_t, h3) << 16);
-      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(C) + io * elems + e) = out;
-    }
+    tc_store4<OUT>(C, io * elems + e, sum, aligned);
   }
 }
 
@@ -570,32 +724,35 @@ int launch_unplanned(bool out32, int32_t mb, int32_t feat, const uint16_t* A, co
 }
 
 template <int T>
-int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t n_pieces, const TcPiece* d_pieces, float* d_scratch,
+int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n_pieces, const TcPiece* d_pieces, float* d_scratch,
                    uint32_t* d_arrived, const uint16_t* A, const uint16_t* B, void* d_C, const int32_t* d_indptr,
                    const int32_t* d_indices, hipStream_t st) {
-  const int f_tiles = (int)stir::ceil_div(feat, kTileF);
-  const int64_t blocks = (int64_t)mb * f_tiles;
+  // Wide units (128 features) fetch A and the row ids once for all of them, narrow ones are more and finer: 128
+  // features of 8401 tiles of 16 rows 58.6 against 63.3 us, of 1250 tiles 16.9 against 14.3 us; 192 features, whose
+  // last wide unit is half empty, 56.4 against 45.6 us.
+  // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
+  // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
+  // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
+  const int past = feat % 128;
+  const bool wide = feat > 64 && (past == 0 || past > 64) && mb * stir::ceil_div(feat, 128) >= 3000;
+  const int ntl = feat <= 32 ? 1 : wide ? 4 : 2;
+  const int f_tiles = (int)stir::ceil_div(feat, 32 * ntl);
+  const int64_t blocks = (mb + n_pieces) * f_tiles;
+  const bool pairs = blocks >= 8000 && (ntl > 1 || nnzb < 4 * (int64_t)mb);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "tc_spmm: too many tiles for one launch");
-  // the tiles of up to kLongSteps steps
-  if (out32)
-    hipLaunchKernelGGL((tcspmm_kernel<T, 1, false, true>), dim3((unsigned)blocks), dim3(256), 0, st, feat,
-                       (int64_t)mb, f_tiles, A, B, d_C, d_indptr, d_indices);
-  else
-    hipLaunchKernelGGL((tcspmm_kernel<T, 0, false, true>), dim3((unsigned)blocks), dim3(256), 0, st, feat,
-                       (int64_t)mb, f_tiles, A, B, d_C, d_indptr, d_indices);
-  STIR_LAUNCH_CHECK();
-  if (n_pieces == 0) return 0;
-  const int long_f_tiles = (int)stir::ceil_div(feat, kLongTF);
-  const int64_t long_blocks = n_pieces * long_f_tiles;
-  STIR_REQUIRE(long_blocks < (int64_t(1) << 31), "tc_spmm: too many pieces for one launch");
-  if (out32)
-    hipLaunchKernelGGL((tcspmm_pieces_kernel<T, kLongNT, 1>), dim3((unsigned)long_blocks), dim3(64 * kLongWaves),
-                       kLongLds, st, feat, long_f_tiles, d_pieces, A, B, d_C, d_scratch, d_arrived, d_indptr,
-                       d_indices);
-  else
-    hipLaunchKernelGGL((tcspmm_pieces_kernel<T, kLongNT, 0>), dim3((unsigned)long_blocks), dim3(64 * kLongWaves),
-                       kLongLds, st, feat, long_f_tiles, d_pieces, A, B, d_C, d_scratch, d_arrived, d_indptr,
-                       d_indices);
+  const int aligned = reinterpret_cast<uintptr_t>(d_C) % (out32 ? 16 : 8) == 0;
+#define STIR_TC(NTL, W, OUT)                                                                                        \
+  hipLaunchKernelGGL((tcspmm_units_kernel<T, NTL, W, OUT>), dim3((unsigned)blocks), dim3(64 * W), 0, st, feat,       \
+                     (int64_t)mb, f_tiles, n_pieces, d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr,   \
+                     d_indices)
+#define STIR_TC_W(NTL, W) if (out32) STIR_TC(NTL, W, 1); else STIR_TC(NTL, W, 0);
+  if (pairs) {
+    if (ntl == 1) { STIR_TC_W(1, 2) } else if (ntl == 2) { STIR_TC_W(2, 2) } else { STIR_TC_W(4, 2) }
+  } else {
+    if (ntl == 1) { STIR_TC_W(1, 4) } else if (ntl == 2) { STIR_TC_W(2, 4) } else { STIR_TC_W(4, 4) }
+  }
+#undef STIR_TC_W
+#undef STIR_TC
   STIR_LAUNCH_CHECK();
   return 0;
 }
@@ -654,7 +811,7 @@ extern "C" int stir_tc_plan_create(stir_tc_plan** plan, int32_t mb, const int32_
   for (int32_t io = 0; io < mb; ++io) {
     STIR_REQUIRE(ptr[io] <= ptr[io + 1], "tc_plan_create: indptr decreases at tile %d", io);
     const int64_t steps = ((int64_t)(ptr[io + 1] - ptr[io]) * kGroup + 31) / 32;
-    if (steps > kLongSteps) longs.emplace_back((int32_t)steps, io);
+    if (steps > kPieceSteps) longs.emplace_back((int32_t)steps, io);
   }
   std::stable_sort(longs.begin(), longs.end(),
                    [](const std::pair<int32_t, int32_t>& a, const std::pair<int32_t, int32_t>& b) { return a.first > b.first; });
@@ -666,9 +823,9 @@ extern "C" int stir_tc_plan_create(stir_tc_plan** plan, int32_t mb, const int32_
     const int32_t len = (steps + n - 1) / n;
     STIR_REQUIRE(slots + n < (int64_t(1) << 31), "tc_plan_create: too many pieces");
     for (int32_t p = 0; p < n; ++p)
-      pieces.push_back(TcPiece{io, p * len, std::min(steps, (p + 1) * len), n > 1 ? (int32_t)(slots + p) : -1,
-                               (int32_t)slots, n, (int32_t)n_multi, 0});
-    if (n > 1) slots += n, ++n_multi;
+      pieces.push_back(TcPiece{io, p * len, std::min(steps, (p + 1) * len), (int32_t)(slots + p), (int32_t)slots, n,
+                               (int32_t)n_multi, 0});
+    slots += n, ++n_multi;
   }
   stir_tc_plan* p = new stir_tc_plan();
   p->mb = mb;
@@ -705,10 +862,7 @@ extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, i
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* A = static_cast<const uint16_t*>(d_A);
   const uint16_t* B = static_cast<const uint16_t*>(d_B);
-  // the sums of the partial tiles leave four to a thread, as one 8- or 16-byte store
   const bool out32 = out_dtype == STIR_F32;
-  STIR_REQUIRE(plan->n_multi == 0 || reinterpret_cast<uintptr_t>(d_C) % (out32 ? 16 : 8) == 0,
-               "tc_spmm: C must be %d-byte aligned", out32 ? 16 : 8);
   // the partial tiles of this tile size and feature width
   const size_t need = size_t(plan->slots) * size_t(tile_size) * size_t(feat) * sizeof(float);
   if (need > plan->scratch_bytes) {
@@ -718,7 +872,7 @@ extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, i
     STIR_HIP(hipMalloc(reinterpret_cast<void**>(&plan->d_scratch), need));
     plan->scratch_bytes = need;
   }
-  const size_t counters = size_t(plan->n_multi) * size_t(stir::ceil_div(feat, kLongTF));
+  const size_t counters = size_t(plan->n_multi) * size_t(stir::ceil_div(feat, 32));
   if (counters > plan->arrived_count) {
     if (plan->d_arrived) STIR_HIP(hipFree(plan->d_arrived));
     plan->d_arrived = nullptr;
@@ -729,13 +883,13 @@ extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, i
   }
   switch (tile_size) {
     case 8:
-      return launch_planned<8>(out32, mb, feat, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A, B,
+      return launch_planned<8>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A, B,
                                d_C, d_indptr, d_indices, st);
     case 16:
-      return launch_planned<16>(out32, mb, feat, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
+      return launch_planned<16>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
                                 B, d_C, d_indptr, d_indices, st);
     default:
-      return launch_planned<32>(out32, mb, feat, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
+      return launch_planned<32>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
                                 B, d_C, d_indptr, d_indices, st);
   }
 }

@@ -75,7 +75,30 @@ __device__ __forceinline__ void store4(float* q, const float4& v) {
   __builtin_nontemporal_store(v.w, q + 3);
 }
 
+// C[row] += acc by the only lane group that adds to the row in this launch.  All of the row is read before any of
+// it is written: of a width that is no multiple of four, two chunks share features.
 template <int G, int REP>
+__device__ __forceinline__ void add_row(float* row, int feat, int gl, const float4 (&acc)[REP]) {
+  float4 old[REP];
+#pragma unroll
+  for (int r = 0; r < REP; ++r) {
+    const int c0 = gl * 4 + r * G * 4;
+    if (c0 < feat) old[r] = ld4(row + chunk_offset(c0, feat));
+  }
+#pragma unroll
+  for (int r = 0; r < REP; ++r) {
+    const int c0 = gl * 4 + r * G * 4;
+    if (c0 >= feat) continue;
+    add4(old[r], acc[r]);
+    float* q = row + chunk_offset(c0, feat);
+    q[0] = old[r].x, q[1] = old[r].y, q[2] = old[r].z, q[3] = old[r].w;
+  }
+}
+
+// MERGED: the merged rows of a hyb plan (spmm.hip).  A holds addresses of the values, slots of value 0 (padding)
+// fetch no row of B, and the product is added to C: what a workgroup has of a row that it shares with others goes
+// there by atomics, so there are no partial rows to be added up.
+template <int G, int REP, bool MERGED = false>
 __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(int m, int stride, int slices, int64_t nnz, int items,
                                                               const float* __restrict__ A,
                                                               const float* __restrict__ B, float* __restrict__ C,
@@ -103,7 +126,7 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
     stir::slice_block(blockIdx.x, slices, wgs, slice, wg);
     const int f0 = slice * kPad;
     B += f0, C += f0, feat -= f0;
-    counters += slice * wgs, partials += slice * wgs * 2 * kPad;
+    if (!MERGED) counters += slice * wgs, partials += slice * wgs * 2 * kPad;
   }
   const int64_t d0 = wg * items, d1 = min(total, d0 + items);
   if (d0 >= total) return;
@@ -128,15 +151,21 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
   const int j0 = __builtin_amdgcn_readfirstlane(nz_at[0]), j1 = __builtin_amdgcn_readfirstlane(nz_at[1]);
   const bool cut_before = __builtin_amdgcn_readfirstlane(cut[0]), cut_after = __builtin_amdgcn_readfirstlane(cut[1]);
   const int cnt = j1 - j0;
-  for (int t = tid; t < cnt; t += kBlock)
-    nz[t] = make_int2(__builtin_nontemporal_load(indices + j0 + t),
-                      __float_as_int(__builtin_nontemporal_load(A + j0 + t)));
+  for (int t = tid; t < cnt; t += kBlock) {
+    float value;
+    if constexpr (MERGED)
+      value = *reinterpret_cast<const float* const*>(A)[j0 + t];
+    else
+      value = __builtin_nontemporal_load(A + j0 + t);
+    nz[t] = make_int2(__builtin_nontemporal_load(indices + j0 + t), __float_as_int(value));
+  }
   const int first = max(i0 - 1, 0);
   for (int r0 = first; r0 < i1; r0 += kBlock) {
     const int r = r0 + tid;
     int s = 0, e = 0;
     if (r < i1) s = indptr[r], e = indptr[r + 1];
     if (e > j0 && e > s && e <= j1) ends[e - 1 - j0] = r + 1;
+    if constexpr (MERGED) continue;
     uint64_t empty = __ballot(r >= i0 && r < i1 && s == e);
     while (empty) {
       const int k = __ffsll((long long)empty) - 1;
@@ -163,10 +192,11 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const int p = a + k0 + u;
-      const bool live = p < b;
+      bool live = p < b;
       const int2 q = nz[min(p, kSlots - 1)];
       f[u] = live ? ends[min(p, kSlots - 1)] : 0;
       v[u] = live ? __int_as_float(q.y) : 0.f;
+      if constexpr (MERGED) live = live && v[u] != 0.f;
       const float* bp = B + (int64_t)q.x * stride;
 #pragma unroll
       for (int r = 0; r < REP; ++r) {
@@ -186,10 +216,14 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
           const int c0 = gl * 4 + r * G * 4;
           if (keep)
             head[(grp * REP + r) * G + gl] = acc[r];
-          else if (c0 < feat)
+          else if (!MERGED && c0 < feat)
             store4(row + chunk_offset(c0, feat), acc[r]);
-          acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
+        if constexpr (MERGED) {
+          if (!keep) add_row<G, REP>(row, feat, gl, acc);
+        }
+#pragma unroll
+        for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (keep) head_row = f[u];
         flushed = true;
       }
@@ -217,9 +251,26 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
     for (int q = max(k, 0); q < (which == 0 ? grp : NG); ++q)
 #pragma unroll
       for (int r = 0; r < REP; ++r) add4(sum[r], tail[(q * REP + r) * G + gl]);
+    if constexpr (MERGED) {
+      if (which == 0 && k >= 0) {
+        add_row<G, REP>(C + (int64_t)(head_row - 1) * stride, feat, gl, sum);
+        continue;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < REP; ++r) {
       const int c0 = gl * 4 + r * G * 4;
+      if constexpr (MERGED) {
+        if (c0 >= feat) continue;
+        const int over = c0 + 4 - feat;
+        const float4 v = over > 0 ? stir::tail_chunk(sum[r], over) : sum[r];
+        float* q = C + (int64_t)((which == 0 ? i0 : i1) - 1) * stride + c0;
+        const float part[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int f = 0; f < 4; ++f)
+          if (c0 + f < feat) __hip_atomic_fetch_add(q + f, part[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        continue;
+      }
       if (which == 0 && k >= 0) {
         if (c0 < feat) store4(C + (int64_t)(head_row - 1) * stride + chunk_offset(c0, feat), sum[r]);
       } else {
@@ -227,6 +278,7 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
       }
     }
   }
+  if constexpr (MERGED) return;
   // a row that goes through the whole workgroup counts as the one it ends in
   const bool has_head = cut_before && !through;
   if (!has_head && !cut_after) return;  // uniform
@@ -314,7 +366,43 @@ bool balanced(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   return m >= 8192 || nnz * feat >= 3000000;
 }
 
+template <bool MERGED>
+int launch(int c, int64_t grid, int slices, int items, int32_t m, int32_t feat, int64_t nnz, const float* d_A,
+           const float* d_B, float* d_C, const int32_t* d_indptr, const int32_t* d_indices, uint32_t* counters,
+           float* partials, hipStream_t st) {
+#define STIR_BALANCED(G, REP)                                                                                        \
+  hipLaunchKernelGGL((csr_balanced_kernel<G, REP, MERGED>), dim3((unsigned)grid), dim3(kBlock), 0, st, m, feat,       \
+                     slices, nnz, items, d_A, d_B, d_C, d_indptr, d_indices, counters, partials)
+  switch (c) {
+    case 0: STIR_BALANCED(4, 1); break;
+    case 1: STIR_BALANCED(8, 1); break;
+    case 2: STIR_BALANCED(16, 1); break;
+    case 3: STIR_BALANCED(32, 1); break;
+    case 4: STIR_BALANCED(64, 1); break;
+    default: STIR_BALANCED(64, 2); break;
+  }
+#undef STIR_BALANCED
+  STIR_LAUNCH_CHECK();
+  return 0;
+}
+
 }  // namespace
+
+namespace stir {
+
+bool merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots) { return balanced(m, n, feat, slots); }
+
+int launch_merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots, const float* const* d_vals,
+                           const float* d_B, float* d_C, const int32_t* d_slot_ptr, const int32_t* d_cols,
+                           hipStream_t st) {
+  const int c = slice_class(n, feat, slots), slices = (int)ceil_div(feat, 16 << c);
+  const int64_t grid = slice_grid(slices, workgroups(m, slots));
+  STIR_REQUIRE(grid < (int64_t(1) << 31), "hyb_spmm: %lld workgroups exceed one launch", (long long)grid);
+  return launch<true>(c, grid, slices, entries_per_workgroup(m, slots), m, feat, slots,
+                      reinterpret_cast<const float*>(d_vals), d_B, d_C, d_slot_ptr, d_cols, nullptr, nullptr, st);
+}
+
+}  // namespace stir
 
 extern "C" {
 
@@ -341,21 +429,8 @@ int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz,
   const int items = entries_per_workgroup(m, nnz);
   uint32_t* counters = static_cast<uint32_t*>(d_workspace);
   float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + (size_t(wgs) * slices * 4 + 15) / 16 * 16);
-#define STIR_BALANCED(G, REP)                                                                                    \
-  hipLaunchKernelGGL((csr_balanced_kernel<G, REP>), dim3((unsigned)grid), dim3(kBlock), 0,                         \
-                     static_cast<hipStream_t>(stream), m, feat, slices, nnz, items, d_A, d_B, d_C, d_indptr, d_indices,   \
-                     counters, partials)
-  switch (c) {
-    case 0: STIR_BALANCED(4, 1); break;
-    case 1: STIR_BALANCED(8, 1); break;
-    case 2: STIR_BALANCED(16, 1); break;
-    case 3: STIR_BALANCED(32, 1); break;
-    case 4: STIR_BALANCED(64, 1); break;
-    default: STIR_BALANCED(64, 2); break;
-  }
-#undef STIR_BALANCED
-  STIR_LAUNCH_CHECK();
-  return 0;
+  return launch<false>(c, grid, slices, items, m, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, counters, partials,
+                       static_cast<hipStream_t>(stream));
 }
 
 }  // extern "C"

@@ -67,4 +67,11 @@ __device__ __forceinline__ void slice_block(int64_t L, int slices, int64_t block
   block = p % piece * pieces + p / piece;
 }
 
+// csr_balanced.hip: the product of merged rows (see spmm.hip) by workgroups of equal work, added to C, where
+// merged_balanced says that this is the better way.
+bool merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots);
+int launch_merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots, const float* const* d_vals,
+                           const float* d_B, float* d_C, const int32_t* d_slot_ptr, const int32_t* d_cols,
+                           hipStream_t st);
+
 }  // namespace stir

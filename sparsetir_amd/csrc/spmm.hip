@@ -754,6 +754,11 @@ constexpr int kMaxPhases = 4;
 // 44 / 60 / 119 / 254 us, merged rows 81 / 98 / 136 / 235 us -- a phase reads and writes C once
 // more, which at 256 features (173 MB each way) costs more than the merged list's indirect loads.
 constexpr int kMergedFromFeat = 256;
+// ... or where a launch per phase is what it costs: merged rows in one launch of equal workgroups
+// (csr_balanced.hip) up to this many slots per phase beyond the first.  Two partitions, phases / merged, us: 13.6 k
+// rows, 162 k nonzeros, 59 features 24.2 / 16.1; 22.5 k, 524 k, 144: 62 / 52, 128: 48 / 33; 60 k, 1 M, 32: 29.7 / 31.5,
+// 64: 49.0 / 50.3, 128: 72.6 / 71.6; 400 k, 4 M, 16: 69 / 87.  Four: 169 k, 1.17 M, 32: 53.5 / 40.3.
+constexpr int64_t kMergedSlotsPerPhase = 1000000;
 constexpr size_t kMergedOptionalBytes = size_t(1) << 30;  // ... when the slot list stays below this
 
 namespace {
@@ -927,7 +932,10 @@ int build_merged_rows(int32_t m, int total_buckets, int num_buckets, const int32
 }
 
 // Launches the CSR row kernels over the merged rows.  feat must have a vector class.
-int launch_merged(const MergedRows& mr, int32_t m, int32_t feat, const float* d_B, float* d_C, hipStream_t st) {
+int launch_merged(const MergedRows& mr, int32_t m, int32_t n, int32_t feat, const float* d_B, float* d_C,
+                  hipStream_t st) {
+  if (stir::merged_balanced(m, n, feat, mr.slots))
+    return stir::launch_merged_balanced(m, n, feat, mr.slots, mr.vals, d_B, d_C, mr.slot_ptr, mr.cols, st);
   dim3 grid((unsigned)stir::ceil_div(m, 4)), block(256);
   const int piece = long_piece(mr.slots);
   dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(mr.slots, piece), 4));
@@ -1197,8 +1205,12 @@ int stir_hyb_spmm_f32(const stir_hyb_plan* plan, int32_t feat, const float* d_B,
   const size_t nk = plan->tables.tiles.size();
   if (nk == 0) return 0;
   STIR_REQUIRE(d_B && d_C, "hyb_spmm: null pointer argument");
-  if (plan->merged && vector_class(feat) >= 0 && (plan->num_col_parts > kMaxPhases || feat >= kMergedFromFeat))
-    return launch_merged(plan->rows, plan->m, feat, d_B, d_C, static_cast<hipStream_t>(stream));
+  const int parts = plan->num_col_parts;
+  if (plan->merged && vector_class(feat) >= 0 &&
+      (parts > kMaxPhases || feat >= kMergedFromFeat ||
+       (plan->rows.slots <= kMergedSlotsPerPhase * (parts - 1) &&
+        stir::merged_balanced(plan->m, plan->n, feat, plan->rows.slots))))
+    return launch_merged(plan->rows, plan->m, plan->n, feat, d_B, d_C, static_cast<hipStream_t>(stream));
   const HybBucket* d_rows = plan->d_tables ? plan->d_tables + nk : nullptr;
   return launch_hyb(plan->tables, plan->d_tables, d_rows, plan->n, feat, d_B, d_C, static_cast<hipStream_t>(stream));
 }

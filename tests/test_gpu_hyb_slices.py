@@ -4,6 +4,7 @@ Checked against the fp64 product as in test_gpu_spmm.py; one partition stores, t
 import numpy as np
 import pytest
 import scipy.sparse as sp
+import torch
 
 from helpers import random_csr
 from test_gpu_spmm import RTOL, _hyb_as_coo, _hyb_setup, _run_hyb
@@ -25,3 +26,27 @@ def test_hyb_feature_slices(dev, nnz, feat, parts, buckets):
     r, c, v = _hyb_as_coo(triples)
     a = sp.csr_matrix((v.astype(np.float64), (r, c)), shape=(m, n))
     assert np.all(np.abs(got - a @ x.astype(np.float64)) <= RTOL * (a @ np.abs(x).astype(np.float64)) + 1e-30)
+
+
+@pytest.mark.parametrize("feat", [8, 31, 67, 129, 192, 255, 300])
+@pytest.mark.parametrize("parts", [2, 5])
+def test_hyb_merged_rows_of_equal_work(dev, feat, parts):
+    """Column partitions whose rows run merged, a row over many workgroups among them; the product is added."""
+    m, n = 8500, 4000
+    rng = np.random.default_rng(feat + parts)
+    deg = rng.integers(0, 30, m)
+    deg[[0, 77, m - 1]] = [3900, 129, 700]
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(n, d, replace=False)) for d in deg]).astype(np.int32)
+    buckets = [1, 2, 4, 8, 16, 32]
+    triples = _hyb_setup(dev, indptr, indices, m, n, parts, buckets, weighted=True, seed=feat)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    got, (f, args) = _run_hyb(dev, m, n, feat, parts, buckets, triples, x)
+    r, c, v = _hyb_as_coo(triples)
+    a = sp.csr_matrix((v.astype(np.float64), (r, c)), shape=(m, n))
+    want, bound = a @ x.astype(np.float64), RTOL * (a @ np.abs(x).astype(np.float64)) + 1e-30
+    assert np.all(np.abs(got - want) <= bound)
+    y = torch.from_numpy(got.ravel().copy()).to(dev)
+    f(torch.from_numpy(x.ravel()).to(dev), y, *args)  # the operator adds to what is there
+    torch.cuda.synchronize()
+    assert np.all(np.abs(y.cpu().numpy().reshape(m, feat) - 2 * want) <= 3 * bound)

@@ -441,11 +441,21 @@ struct TcPiece {
   int32_t pad;
 };
 
-__device__ __forceinline__ void coherent_store(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Sixteen bytes through to the memory that all XCDs see, and from there (a load: after arrived_all(), which waits for
+// every load of the wavefront).  As four-byte atomics a partial tile took four masked writes per 16 bytes.
+__device__ __forceinline__ void coherent_store(float* p, const f32x4& v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
 }
-__device__ __forceinline__ float coherent_load(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ f32x4 coherent_load(const float* p) {
+  f32x4 v;
+  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
+  return v;
+}
+template <int N>
+__device__ __forceinline__ void arrived_all(f32x4 (&v)[N]) {
+  asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]) : : "memory");
+#pragma unroll
+  for (int u = 1; u < N; ++u) asm volatile("" : "+v"(v[u]));
 }
 
 typedef __fp16 tr16x4 __attribute__((__vector_size__(4 * sizeof(__fp16))));  // result type of the transposing LDS read
@@ -637,8 +647,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
       if (!part) {
         tc_store4<OUT>(C, (io * T + row) * feat + fcol, sum, aligned);
       } else {
-        float* q = part + (int64_t)row * feat + fcol;
-        coherent_store(q, sum.x), coherent_store(q + 1, sum.y), coherent_store(q + 2, sum.z), coherent_store(q + 3, sum.w);
+        coherent_store(part + (int64_t)row * feat + fcol, f32x4{sum.x, sum.y, sum.z, sum.w});
       }
     }
   }
@@ -662,21 +671,17 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
     const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
     if (fcol >= feat) continue;
     const int64_t e = (int64_t)row * feat + fcol;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int p0 = 0; p0 < pc.pieces; p0 += 4) {
-      float4 y[4];
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (int p0 = 0; p0 < pc.pieces; p0 += 8) {
+      f32x4 y[8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        y[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (p0 + u < pc.pieces) {
-          const float* at = first + (p0 + u) * elems + e;
-          y[u] = make_float4(coherent_load(at), coherent_load(at + 1), coherent_load(at + 2), coherent_load(at + 3));
-        }
-      }
+      for (int u = 0; u < 8; ++u) y[u] = coherent_load(first + min(p0 + u, pc.pieces - 1) * elems + e);
+      arrived_all(y);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u < pc.pieces) sum += y[u];
     }
-    tc_store4<OUT>(C, io * elems + e, sum, aligned);
+    tc_store4<OUT>(C, io * elems + e, make_float4(sum[0], sum[1], sum[2], sum[3]), aligned);
   }
 }
 
@@ -729,16 +734,18 @@ int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n
                    const int32_t* d_indices, hipStream_t st) {
   // Wide units (128 features) fetch A and the row ids once for all of them, narrow ones are more and finer: 128
   // features of 8401 tiles of 16 rows 58.6 against 63.3 us, of 1250 tiles 16.9 against 14.3 us; 192 features, whose
-  // last wide unit is half empty, 56.4 against 45.6 us.
+  // last wide unit is half empty, 56.4 against 45.6 us; 128 features of 21 k tiles of 8 rows, with little of A
+  // to fetch, 68.3 against 62.7 us, 256 of 12.5 k 86.2 against 91.4.
   // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
   // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
-  // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
+  // 35.5 against 38.3 us; wide units, 5292 tiles of 7 steps 61.0 against 54.2, 3125 of 10 steps 50.7 against 53.0
+  // us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
   const int past = feat % 128;
-  const bool wide = feat > 64 && (past == 0 || past > 64) && mb * stir::ceil_div(feat, 128) >= 3000;
+  const bool wide = (T > 8 || feat >= 256) && feat > 64 && (past == 0 || past > 64) && mb * stir::ceil_div(feat, 128) >= 3000;
   const int ntl = feat <= 32 ? 1 : wide ? 4 : 2;
   const int f_tiles = (int)stir::ceil_div(feat, 32 * ntl);
   const int64_t blocks = (mb + n_pieces) * f_tiles;
-  const bool pairs = blocks >= 8000 && (ntl > 1 || nnzb < 4 * (int64_t)mb);
+  const bool pairs = blocks >= (wide ? 5000 : 8000) && (ntl > 1 || nnzb < 4 * (int64_t)mb);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "tc_spmm: too many tiles for one launch");
   const int aligned = reinterpret_cast<uintptr_t>(d_C) % (out32 ? 16 : 8) == 0;
 #define STIR_TC(NTL, W, OUT)                                                                                        \

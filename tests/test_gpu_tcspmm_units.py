@@ -30,7 +30,7 @@ def test_tile_lengths(dev, t, feat, out_dtype):
     _run(dev, indptr, indices, n, feat, False, out_dtype, t=t)
 
 
-@pytest.mark.parametrize("t,tiles,feat", [(8, 8200, 32), (8, 8200, 64), (16, 3100, 128), (8, 8200, 96), (32, 2700, 192)])
+@pytest.mark.parametrize("t,tiles,feat", [(8, 8200, 32), (8, 8200, 64), (16, 3100, 128), (16, 8200, 96), (32, 2700, 192), (16, 5100, 128)])
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
 def test_many_tiles(dev, t, tiles, feat, out_dtype):
     rng = np.random.default_rng(feat)

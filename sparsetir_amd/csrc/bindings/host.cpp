@@ -23,6 +23,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <sched.h>
+
 #include <algorithm>
 #include <new>
 #include <vector>
@@ -62,7 +64,8 @@ struct Launcher {
   std::vector<int64_t>* sizes;
   std::vector<Operand>* operands;
   std::vector<Plan>* plans;     // as many as the operator keeps, the one used last in front
-  std::vector<int64_t>* key;    // of the call in hand (filled and read under the GIL)
+  std::vector<int64_t>* key;    // of the call in hand, for as long as it holds the GIL
+  std::vector<void*>* in_use;   // a plan per launch that is under way without the GIL
   size_t workspace_bytes;       // of a call (CSR SpMM)
   std::vector<Workspace>* workspaces;  // one per stream the operator runs on, the one used last in front
 };
@@ -135,6 +138,27 @@ int call(const Launcher* l, void* const* p, void* plan, void* ws, void* st) {
 
 bool planned(Kind k) { return k >= kTc; }
 
+// call() without the GIL (a launch waits when the queue is full).  Other threads may use the launcher meanwhile, so
+// nothing of it is read here but its kind and sizes, and nobody destroys `plan` before the call is done with it.
+int call_unlocked(Launcher* l, void* const* p, void* plan, void* ws, void* st) {
+  int rc;
+  if (plan) l->in_use->push_back(plan);
+  Py_BEGIN_ALLOW_THREADS
+  rc = call(l, p, plan, ws, st);
+  Py_END_ALLOW_THREADS
+  if (plan) l->in_use->erase(std::find(l->in_use->begin(), l->in_use->end(), plan));
+  return rc;
+}
+
+// Lets go of the GIL until no launch uses `plan`, which is in the launcher's list no more.
+void wait_until_unused(Launcher* l, void* plan) {
+  while (std::find(l->in_use->begin(), l->in_use->end(), plan) != l->in_use->end()) {
+    Py_BEGIN_ALLOW_THREADS
+    sched_yield();
+    Py_END_ALLOW_THREADS
+  }
+}
+
 constexpr size_t kPassed = 8;  // a C entry point takes at most this many of the leading arguments
 
 // Looks at the whole argument tuple and fills p with the addresses of the leading arguments.
@@ -186,10 +210,7 @@ PyObject* launch(PyObject* self, PyObject* args) {
     const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device);
     at::Tensor held;
     void* ws = l->workspace_bytes ? workspace(l, stream, &held) : nullptr;
-    void* st = stream.stream();
-    Py_BEGIN_ALLOW_THREADS  // a launch waits when the queue is full
-    rc = call(l, p, plan, ws, st);
-    Py_END_ALLOW_THREADS
+    rc = call_unlocked(l, p, plan, ws, stream.stream());
   } catch (...) {  // a tensor without storage: the Python code says what is wrong with it
     rc = kNotTaken;
   }
@@ -198,14 +219,19 @@ PyObject* launch(PyObject* self, PyObject* args) {
   return PyLong_FromLong(rc);
 }
 
-void drop(Launcher* l, PyObject* name) {  // null: all of them
+// Takes the plan of that name (null: every plan) off the list; the caller may destroy it then.
+void drop(Launcher* l, PyObject* name) {
+  std::vector<Plan> gone;
   for (size_t k = l->plans->size(); k-- > 0;) {
-    PyObject* n = (*l->plans)[k].name;
-    const int same = name ? PyObject_RichCompareBool(n, name, Py_EQ) : 1;
+    const int same = name ? PyObject_RichCompareBool((*l->plans)[k].name, name, Py_EQ) : 1;
     if (same < 0) PyErr_Clear();
     if (same == 0) continue;
+    gone.push_back(std::move((*l->plans)[k]));
     l->plans->erase(l->plans->begin() + k);
-    Py_DECREF(n);
+  }
+  for (Plan& g : gone) {
+    wait_until_unused(l, g.plan);
+    Py_DECREF(g.name);
   }
 }
 
@@ -235,17 +261,19 @@ PyObject* forget(PyObject* self, PyObject* name) {
 }
 
 // launch_new_hyb(args) -> (name, plan) of a new plan for arguments launch() did not know, remembered and
-// launched; None when they are not the ordinary ones, -1 when the C ABI refused.  The name is the properties the
-// plan depends on.
+// launched; 0 when another thread made the plan meanwhile (launched with it); None when they are not the ordinary
+// ones, -1 when the C ABI refused.  The name is the properties the plan depends on.  Other threads run while the
+// plan is made: everything about this call is its own until the plan is put into the list, whole.
 PyObject* launch_new_hyb(PyObject* self, PyObject* args) {
   Launcher* l = reinterpret_cast<Launcher*>(self);
   stir_hyb_plan* plan = nullptr;
+  PyObject* out = nullptr;
+  Plan made{nullptr, 0, {}, nullptr};
   try {
     if (l->kind != kHyb) Py_RETURN_NONE;
     const int64_t device = c10::hip::current_device();
     void* p[kPassed];
-    std::vector<int64_t>& key = *l->key;
-    key.assign(1, device);
+    std::vector<int64_t> key(1, device);
     if (!walk(l, args, (int)device, p, [&](int64_t v) { return key.push_back(v), true; })) Py_RETURN_NONE;
     // key: device, then per bucket the address of A, address and version of rows, of cols
     const size_t nk = (l->operands->size() - 2) / 3;
@@ -263,33 +291,34 @@ PyObject* launch_new_hyb(PyObject* self, PyObject* args) {
       nrows[k] = (*l->operands)[2 + 3 * k + 1].length;
     }
     if (nb == 0 || nk != nb * (size_t)n[3]) Py_RETURN_NONE;
+    void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
+    made.device = (int)device;
+    made.key.assign(key.begin() + 1, key.end());
+    for (const Plan& q : *l->plans)
+      if (q.device == made.device && q.key == made.key) return PyLong_FromLong(call_unlocked(l, p, q.plan, nullptr, st));
+    made.name = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key.data()),
+                                          (Py_ssize_t)(key.size() * sizeof(int64_t)));
+    if (!made.name) return nullptr;
     int rc;
     Py_BEGIN_ALLOW_THREADS
     rc = stir_hyb_plan_create(&plan, (int32_t)n[1], (int32_t)n[2], (int32_t)n[3], (int32_t)nb, widths.data(),
                               nrows.data(), A.data(), rows.data(), cols.data());
+    if (rc == 0) rc = call(l, p, plan, nullptr, st);
     Py_END_ALLOW_THREADS
-    if (rc != 0) return PyLong_FromLong(kFailed);
-    l->plans->insert(l->plans->begin(), Plan{plan, (int)device, std::vector<int64_t>(key.begin() + 1, key.end()), nullptr});
-    void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-    Py_BEGIN_ALLOW_THREADS
-    rc = call(l, p, plan, nullptr, st);
-    Py_END_ALLOW_THREADS
-    Plan& made = l->plans->front();
-    if (rc == 0)
-      made.name = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key.data()),
-                                            (Py_ssize_t)(key.size() * sizeof(int64_t)));
-    PyObject* out = made.name ? Py_BuildValue("(OK)", made.name, reinterpret_cast<unsigned long long>(plan)) : nullptr;
-    if (!out) {  // nobody would own the plan
-      Py_XDECREF(made.name);
-      l->plans->erase(l->plans->begin());
-      stir_hyb_plan_destroy(plan);
-      return rc == 0 ? nullptr : PyLong_FromLong(kFailed);
+    made.plan = plan;
+    out = rc == 0 ? Py_BuildValue("(OK)", made.name, reinterpret_cast<unsigned long long>(plan)) : PyLong_FromLong(kFailed);
+    if (rc == 0 && out) {
+      l->plans->insert(l->plans->begin(), std::move(made));
+      return out;
     }
-    return out;
-  } catch (...) {
-    if (plan) stir_hyb_plan_destroy(plan);
-    Py_RETURN_NONE;
+  } catch (...) {  // out of memory: the Python code makes the plan, or says so
+    Py_CLEAR(out);
+    Py_INCREF(Py_None);
+    out = Py_None;
   }
+  Py_XDECREF(made.name);  // nobody would own the plan
+  if (plan) stir_hyb_plan_destroy(plan);
+  return out;
 }
 
 bool scalar_type(long code, c10::ScalarType* out) {
@@ -313,8 +342,9 @@ Launcher* make(Kind kind) {
   l->operands = new (std::nothrow) std::vector<Operand>();
   l->plans = new (std::nothrow) std::vector<Plan>();
   l->key = new (std::nothrow) std::vector<int64_t>();
+  l->in_use = new (std::nothrow) std::vector<void*>();
   l->workspaces = new (std::nothrow) std::vector<Workspace>();
-  if (l->sizes && l->operands && l->plans && l->key && l->workspaces) return l;
+  if (l->sizes && l->operands && l->plans && l->key && l->in_use && l->workspaces) return l;
   Py_DECREF(l);
   PyErr_NoMemory();
   return nullptr;
@@ -400,6 +430,7 @@ void launcher_dealloc(PyObject* self) {
   if (l->plans) drop(l, nullptr);
   delete l->plans;
   delete l->key;
+  delete l->in_use;
   delete l->workspaces;
   Py_TYPE(self)->tp_free(self);
 }
@@ -407,7 +438,7 @@ void launcher_dealloc(PyObject* self) {
 PyMethodDef launcher_methods[] = {
     {"launch", launch, METH_O, "launch(args) -> 0: launched, -1: refused, 1: not taken, or the name of the plan"},
     {"remember", remember, METH_VARARGS, "remember(args, plan, name): a plan made from these arguments"},
-    {"launch_new_hyb", launch_new_hyb, METH_O, "launch_new_hyb(args) -> (name, plan), None: not taken, -1: refused"},
+    {"launch_new_hyb", launch_new_hyb, METH_O, "launch_new_hyb(args) -> (name, plan), 0: launched, None: not taken, -1: refused"},
     {"forget", forget, METH_O, "forget(name): the plan is no more; None: all of them"},
     {"hyb", launcher_hyb, METH_VARARGS | METH_STATIC, "hyb(n, m, feat, parts, buckets, nrows): launcher of the hyb operator"},
     {nullptr, nullptr, 0, nullptr}};

@@ -28,6 +28,7 @@ mean of ``number`` back-to-back launches between device events
 import collections
 import ctypes
 import operator
+import threading
 
 import torch
 
@@ -48,7 +49,9 @@ class _PlanCache:
     whose last use lies furthest back, so a caller that alternates between a few graphs
     (mini-batches, training and validation sets) builds each plan once.  ``builds`` counts the
     plans made.  An entry keeps its arrays alive: their addresses cannot be handed to other arrays
-    while a plan made from them exists."""
+    while a plan made from them exists.  ``lock`` is held by whoever makes, uses or drops plans in
+    Python, so that threads that share an operator do not destroy a plan another one is about to
+    launch (the launcher keeps the plans of its own launches from being destroyed)."""
     capacity = 8
 
     def __init__(self, destroy, forget):
@@ -56,27 +59,31 @@ class _PlanCache:
         self._forget = forget  # tells the launcher of the operator that a plan (None: every plan) goes
         self._plans = collections.OrderedDict()  # key -> (plan, arrays kept alive)
         self.builds = 0
+        self.lock = threading.RLock()
 
     def get(self, key):
-        hit = self._plans.get(key)
-        if hit is None:
-            return None
-        self._plans.move_to_end(key)
-        return hit[0]
+        with self.lock:
+            hit = self._plans.get(key)
+            if hit is None:
+                return None
+            self._plans.move_to_end(key)
+            return hit[0]
 
     def put(self, key, plan, keep):
-        while len(self._plans) >= self.capacity:
-            gone, (old, _) = self._plans.popitem(last=False)
-            self._forget(gone)
-            self._destroy(old)
-        self._plans[key] = (plan, keep)
-        self.builds += 1
+        with self.lock:
+            while len(self._plans) >= self.capacity:
+                gone, (old, _) = self._plans.popitem(last=False)
+                self._forget(gone)
+                self._destroy(old)
+            self._plans[key] = (plan, keep)
+            self.builds += 1
 
     def clear(self):
-        self._forget(None)
-        while self._plans:
-            _, (old, _) = self._plans.popitem()
-            self._destroy(old)
+        with self.lock:
+            self._forget(None)
+            while self._plans:
+                _, (old, _) = self._plans.popitem()
+                self._destroy(old)
 
     def __len__(self):
         return len(self._plans)
@@ -104,13 +111,18 @@ class _Operator:
     business of ``_call`` of the operator."""
     name = "main"
     entry_name = "main"
+    _plans = None  # of the operators that keep plans
 
     def __call__(self, *args):
         rc = self._launch(args)
         if rc == 0:
             return
         if rc == 1:
-            self._call(*args)
+            if self._plans is None:
+                self._call(*args)
+            else:
+                with self._plans.lock:
+                    self._call(*args)
         elif rc == -1:
             _lib.check(rc)
         else:  # launched, with a plan that was not the one used last
@@ -254,6 +266,8 @@ class HybCsrMM(_Operator):
         if made is not None:
             if made == -1:
                 _lib.check(made)
+            if made == 0:  # another thread made the plan meanwhile
+                return
             name, plan = made
             self._plans.put(name, ctypes.c_void_p(plan), args[2:])  # the plan stores pointers into these arrays
             return

@@ -1,4 +1,7 @@
 """The native host path of the operators: which plan a call uses, and when it leaves a call to Python."""
+import sys
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -67,3 +70,42 @@ def test_falls_back_to_python(dev):
     side.synchronize()
     for got in (y, y2):
         assert np.allclose(got.cpu().numpy().reshape(want.shape), want.cpu().numpy(), rtol=1e-5, atol=1e-5)
+
+
+def test_threads_share_an_operator(dev):
+    """Four threads with three matrices each use one operator, more matrices than it keeps plans: every product is
+    that of the arrays handed in, during the calls and afterwards (a plan filed under another thread's arrays would
+    multiply the wrong matrix from then on)."""
+    x, mats, f = _graphs(dev, 12)
+    z, zi = torch.zeros(0, device=dev), torch.zeros(0, dtype=torch.int32, device=dev)
+
+    def product(k):
+        a, r, c, want = mats[k]
+        y = torch.zeros_like(x)
+        f(x.reshape(-1), y.reshape(-1), a, r, c, z, zi, zi)
+        assert torch.allclose(y.double(), want, rtol=1e-5, atol=1e-5), f"matrix {k}"
+
+    failed = []
+
+    def work(first):
+        try:
+            for _ in range(25):
+                for k in range(first, 12, 4):
+                    product(k)
+        except BaseException as e:  # noqa: B036 (reported by the test)
+            failed.append(e)
+
+    before = sys.getswitchinterval()
+    sys.setswitchinterval(1e-5)
+    try:
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(before)
+    assert not failed, failed[0]
+    assert len(f._plans) == f._plans.capacity
+    for k in range(12):
+        product(k)

@@ -8,7 +8,8 @@
 // where whole ones would not give every compute unit an equal part; the piece of a tile that finishes last
 // adds the pieces' partial tiles in a fixed order: the result does not depend on the order in which
 // wavefronts run.
-// (The split keeps 24 bits of finite values below 3.38e38; an infinite sum or weight gives NaN.)
+// The split keeps all 24 bits of every fp32 value, subnormal ones too; a unit in which something overflows or is
+// infinite is done again with fp32 products, so the results are those of fp32 arithmetic over all of its range.
 #pragma once
 #include <cstdint>
 #include <vector>

@@ -312,8 +312,13 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// Eight floats as sums of three bf16 each: v = t[0] + t[1] + t[2], exactly as long as nothing underflows (each
-// term is what the ones before it leave, rounded to nearest: 8 + 8 + 8 bits of a 24-bit significand).
+// Eight floats as sums of three bf16 each: v = t[0] + t[1] + t[2], exactly as long as nothing underflows or
+// overflows (each term is what the ones before it leave, rounded to nearest: 8 + 8 + 8 bits of a 24-bit significand).
+// So that nothing underflows, whatever fp32 numbers come in, both factors of the product are taken times kScale: the
+// last bit of the smallest subnormal number is a normal bf16 then, and the sums come out times kScale^2.  What
+// overflows on the way (sums and weights from 2^104 on, products from 2^80, infinities) leaves an infinity or NaN in
+// the partial tile, and the unit is done again without terms (exact_unit).
+constexpr float kScale = 0x1p24f;
 __device__ __forceinline__ void split3(const float (&v)[8], bf16x8 (&t)[3]) {
 #pragma unroll
   for (int j = 0; j < 8; j += 2) {
@@ -351,7 +356,7 @@ __global__ __launch_bounds__(256) void f32_pack_w_kernel(const float* __restrict
     const int k = 32 * s + 8 * q + 4 * c;  // fin is a multiple of 4
     float4 w = make_float4(0.f, 0.f, 0.f, 0.f);
     if (out < fout && k < fin) w = *reinterpret_cast<const float4*>(W + (rel * fout + out) * fin + k);
-    v[4 * c] = w.x, v[4 * c + 1] = w.y, v[4 * c + 2] = w.z, v[4 * c + 3] = w.w;
+    v[4 * c] = kScale * w.x, v[4 * c + 1] = kScale * w.y, v[4 * c + 2] = kScale * w.z, v[4 * c + 3] = kScale * w.w;
   }
   bf16x8 term[3];
   split3(v, term);
@@ -395,14 +400,91 @@ struct TileShape {
   static constexpr int kPerSimd = KS == 1 ? (NT == 4 ? 4 : 4) : (NT == 4 ? 3 : 4);
 };
 
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef __attribute__((address_space(3))) float LdsF32;
+typedef __attribute__((address_space(3))) int LdsInt;
+
+// All of a unit once more into its partial tile, with fp32 products.  A function of its own: in the kernel it took
+// registers from the loop, as a branch inside or behind it (110 k nodes, 130 relations, 2 M edges, 64 -> 64: 333 us,
+// 422 and 458 with it).  A unit that comes here takes about six times as long.
+template <int KS, int NT>
+__device__ __attribute__((noinline)) void exact_unit(int b_begin, int b_end, int fin, int fout, const BatchF32* batches,
+                                                     const uint32_t* pinfo, const EdgeF32* edges, const float* W,
+                                                     const float* X, LdsF32* yt, LdsF32* et, LdsInt* turn) {
+  constexpr int WAVES = TileShape<KS, NT>::kWaves, THREADS = 64 * WAVES, FO = 16 * NT, CPR = 8 * KS, EMAX = 32 / KS;
+  constexpr int SS = 32 * KS + 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int i = lane & 15, q = lane >> 4, g = lane / CPR, gc = lane % CPR;
+  for (int e = tid; e < kTileRows * FO; e += THREADS) yt[e] = 0.f;
+  if (tid == 0) *turn = b_begin;
+  __syncthreads();
+#pragma unroll 1
+  for (int b = b_begin + wave; b < b_end; b += WAVES) {
+    const BatchF32 bt = batches[b];
+    const int places = (int)((bt.counts >> 16) & 255u);
+    // the places of a lane group's column, one after the other
+    f32x4 run = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int k = 0; k < kChain; ++k) {
+      const int place = g * kChain + k;
+      uint32_t chain = (uint32_t)(EMAX + 1);
+      f32x4 x = {0.f, 0.f, 0.f, 0.f};
+      float w = 0.f;
+      if (place < places) {
+        const EdgeF32 rec = edges[(int64_t)bt.place_begin + place];
+        chain = rec.w_hi >> 16;
+        if (rec.src != kUnused) {
+          w = *reinterpret_cast<GlobalF32*>((uintptr_t)rec.w_lo | ((uintptr_t)(rec.w_hi & 0xffffu) << 32));
+          if (4 * gc < fin) x = *reinterpret_cast<const f32x4u*>(X + (int64_t)rec.src * fin + 4 * gc);
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) run[c] = k == 0 ? w * x[c] : fmaf(w, x[c], chain >= 256 ? run[c] : 0.f);
+      LdsF32* row = et + (chain & 255) * SS + 4 * gc;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) row[c] = run[c];
+    }
+    const uint32_t pair = pinfo[(int64_t)b * kBatch + i];
+    const LdsF32* first = et + 8 * q + (pair >> 16) / 4;
+    const int chains = (int)((pair >> 8) & 255u);
+    const float* wrel = W + (int64_t)bt.rel * fout * fin;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int j = 0; j < 8 * KS; ++j) {  // product number j of four inputs takes input 8 q + j of each lane
+      const int k = 32 * (j >> 3) + 8 * q + (j & 7), at = 32 * (j >> 3) + (j & 7);
+      float x = first[at];
+      for (int t = 1; t < chains; ++t) x += first[t * SS + at];
+      x = k < fin ? x : 0.f;  // what lies beyond feat_in is no input
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const int out = 16 * nt + i;
+        acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(x, out < fout && k < fin ? wrel[out * fin + k] : 0.f, acc[nt], 0, 0, 0);
+      }
+    }
+    while (__hip_atomic_load(turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != b) __builtin_amdgcn_s_sleep(1);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      LdsF32* row = yt + (pinfo[(int64_t)b * kBatch + 4 * q + v] & 255u) * FO + NT * i;
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) row[nt] += acc[nt][v];
+    }
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(turn, b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __syncthreads();
+}
+
 template <int KS, int NT>
 __global__ __launch_bounds__((64 * TileShape<KS, NT>::kWaves))
 __attribute__((amdgpu_waves_per_eu(TileShape<KS, NT>::kPerSimd, TileShape<KS, NT>::kPerSimd)))
 void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t x_bytes,
                           const UnitF32* __restrict__ units, const BatchF32* __restrict__ batches,
                           const uint32_t* __restrict__ pinfo, const EdgeF32* __restrict__ edges,
-                          const bf16x8* __restrict__ Wp, const float* __restrict__ X, float* __restrict__ Y,
-                          float* partials, uint32_t* arrived) {
+                          const bf16x8* __restrict__ Wp, const float* __restrict__ W,
+                          const float* __restrict__ X, float* __restrict__ Y, float* partials, uint32_t* arrived) {
   constexpr int WAVES = TileShape<KS, NT>::kWaves;
   constexpr int THREADS = 64 * WAVES;
   constexpr int FO = 16 * NT;      // floats per row of the partial tile
@@ -504,8 +586,9 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     // 1. the chains of this batch: a lane group adds up its column of weighted rows, and writes a row of the
     // chain tile wherever a chain ends
     f32x4 run = {0.f, 0.f, 0.f, 0.f};
+    const float own = kScale * rw.w;
     static_for_chain([&](auto K) {
-      const float w = __int_as_float(at_place<KS, decltype(K)::value>(__float_as_int(rw.w)));
+      const float w = __int_as_float(at_place<KS, decltype(K)::value>(__float_as_int(own)));
       const uint32_t chain = (uint32_t)at_place<KS, decltype(K)::value>((int)rw.chain);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
@@ -593,6 +676,17 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
   }
 
   __syncthreads();
+  // a unit in which something overflowed is done again, with fp32 products
+  float unscale = 1.f / (kScale * kScale), all_finite = 0.f;  // all_finite: or NaN
+  for (int e = tid; e < kTileRows * FO / 4; e += THREADS) {
+    const float4 v = reinterpret_cast<const float4*>(yt)[e];
+    all_finite = fmaf(v.x, 0.f, all_finite), all_finite = fmaf(v.y, 0.f, all_finite);
+    all_finite = fmaf(v.z, 0.f, all_finite), all_finite = fmaf(v.w, 0.f, all_finite);
+  }
+  if (__syncthreads_or(!(all_finite == 0.f))) {
+    exact_unit<KS, NT>(u.batch_begin, b_end, fin, fout, batches, pinfo, edges, W, X, (LdsF32*)yt, (LdsF32*)et, (LdsInt*)&turn);
+    unscale = 1.f;
+  }
   // The tile's rows of Y are one stretch of memory.  A thread requests all it is about to add to before it
   // waits for any of it: one element at a time this end of a unit took 13 round trips to memory.
   const int64_t row0 = (int64_t)u.tile * kTileRows;
@@ -603,7 +697,7 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
   const uint32_t inverse = (uint32_t)((0x100000000ull + fout - 1) / fout);  // exact quotients for these e
   auto sum_at = [&](int e) {
     const int r = fout > 1 ? (int)__umulhi((uint32_t)e, inverse) : e, c = e - r * fout;
-    return yt[r * FO + NT * (c & 15) + (c >> 4)];
+    return unscale * yt[r * FO + NT * (c & 15) + (c >> 4)];
   };
   if (u.partial < 0) {
     for (int e0 = tid; e0 < count; e0 += AHEAD * THREADS) {
@@ -989,7 +1083,7 @@ int f32_tiles_launch(F32TileIndex& idx, int32_t feat_in, int32_t feat_out, const
 #define STIR_F32_TILE(KS, NT)                                                                                   \
   hipLaunchKernelGGL((rgms_f32_tile_kernel<KS, NT>), grid, dim3((64 * TileShape<KS, NT>::kWaves)), 0, stream, idx.m, \
                      feat_in, feat_out, (int)idx.batches, (uint32_t)((int64_t)idx.n * feat_in * 4), units, bts,  \
-                     pinfo, edges, wp, d_X, d_Y, partials, static_cast<uint32_t*>(u.d_arrived))
+                     pinfo, edges, wp, d_W, d_X, d_Y, partials, static_cast<uint32_t*>(u.d_arrived))
   switch (ks * 10 + nt) {
     case 11: STIR_F32_TILE(1, 1); break;
     case 12: STIR_F32_TILE(1, 2); break;

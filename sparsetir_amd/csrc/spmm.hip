@@ -187,6 +187,12 @@ __device__ __forceinline__ void csr_accumulate(float4 (&acc)[REP], int start, in
 // (169 k-node power-law graph, half of its nonzeros in rows above 256: 46 -> 41 us at 32 features,
 // 223 -> 203 us at 256; 2.45 M-node graph, 128 features: 5.05 -> 5.01 ms; 32 is slower again).
 constexpr int kLongRow = 64;
+// Fewer nonzeros: rows of up to four times the average, 256 at most, are ordinary ones and stay with their wavefront
+// (5 k rows of 50, 128 features: 14.3 -> 9.8 us).
+inline int long_row(int64_t m, int64_t nnz) {
+  return nnz < (1 << 18) ? (int)std::min<int64_t>(256, std::max<int64_t>(kLongRow, 4 * nnz / std::max<int64_t>(m, 1)))
+                         : kLongRow;
+}
 // Nonzeros per piece: short ones where whole pieces would leave the chip idle or end it on a few
 // (240 k nonzeros, 100 features: 40 / 32 / 31 us with 256 / 128 / 64; 600 k: 59 / 52 / 54; 1.19 M:
 // 106 / 110 / 111).
@@ -200,6 +206,15 @@ inline int long_piece(int64_t nnz) { return nnz < (1 << 18) ? 64 : nnz < (1 << 2
 // 80 k nonzeros with a row of 2000 cost the same either way at 64 features (13.3 us, split 13.9), at
 // 16 features 10.2 us (12.4), at 100 features 21.5 us (19.5).
 constexpr int64_t kSmallProduct = 6000000;
+// With fewer than 2^18 nonzeros the line lies higher.  The second launch costs 3 us also where it finds no long rows,
+// and nothing but the row pointers tells: us, in one launch / two / in one whose wavefronts keep their hub rows:
+//   100 k rows, 200 k nonzeros, 32 features, no long rows 8.4 / 10.5 / 7.6, a row of 1000 8.4 / 12.3 / 26,
+//     a row of 8000 27 / 15 / 185; 64 features 15.3 / 17.3 / 14.4, 15.4 / 20.5 / 47, 43 / 23 / 317;
+//   60 k, 240 k, 128 (31 M): 23.1 / 25.1 / 22.4, 22.9 / 30.0 / 80, 72 / 32 / 562.
+constexpr int64_t kSmallProductFew = 20000000;
+inline bool long_rows_apart(int64_t nnz, int32_t feat) {
+  return nnz * feat >= (nnz < (1 << 18) ? kSmallProductFew : kSmallProduct);
+}
 constexpr int kBlockRow = 128;
 constexpr int kSmallWaves = 8;      // 16 are slower (10 us for the launch above)
 constexpr int kWavePerRow = 20000;  // small products with more rows: a lane group per row
@@ -244,7 +259,7 @@ __device__ __forceinline__ void block_rows(const BlockRow* list, int count, floa
 // One wavefront per row, WAVES rows per workgroup.  With WAVES = 4 the matrix is split: rows above
 // kLongRow are zero-filled here and added by csr_long_rows_kernel.
 template <int G, int REP, int WAVES, bool INDIRECT = false>
-__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat, const float* __restrict__ A,
+__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat, int long_row, const float* __restrict__ A,
                                                                  const float* __restrict__ B,
                                                                  float* __restrict__ C,
                                                                  const int32_t* __restrict__ indptr,
@@ -262,7 +277,7 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat
   float4 acc[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool later = end - start > (SPLIT ? kLongRow : kBlockRow);
+  const bool later = end - start > (SPLIT ? long_row : kBlockRow);
   if (!later) csr_accumulate<G, REP, INDIRECT>(acc, start, end, feat, A, B, indices, lane);
   reduce_groups<G, REP>(acc, kWave);
   if constexpr (INDIRECT) {
@@ -295,7 +310,7 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat
 // sharing the row as in the kernel above, up to the length that is left to csr_long_rows_kernel
 // (WAVES = 4, the matrix is split: zero-filled here) or to the workgroup.
 template <int G, int WAVES>
-__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int feat,
+__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int feat, int long_row,
                                                                       const float* __restrict__ A,
                                                                       const float* __restrict__ B,
                                                                       float* __restrict__ C,
@@ -342,14 +357,14 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int
     write_row<G, 1>(C, row, feat, feat, lane, sum, 0, nullptr);
   }
   // the longer rows, one after the other, by the whole wavefront
-  const bool later = end - start > (SPLIT ? kLongRow : kBlockRow);
+  const bool later = end - start > (SPLIT ? long_row : kBlockRow);
   uint64_t todo = __ballot(row < m && !alone && gl == 0 && (SPLIT || !later));
   while (todo) {
     const int src = __ffsll((long long)todo) - 1;
     todo &= todo - 1;
     const int s = __shfl(start, src, kWave), e = __shfl(end, src, kWave);
     float4 sum[1] = {make_float4(0.f, 0.f, 0.f, 0.f)};
-    if (!(SPLIT && e - s > kLongRow)) csr_accumulate<G, 1>(sum, s, e, feat, A, B, indices, lane);
+    if (!(SPLIT && e - s > long_row)) csr_accumulate<G, 1>(sum, s, e, feat, A, B, indices, lane);
     reduce_groups<G, 1>(sum, kWave);
     if (g == 0) write_row<G, 1>(C, row0 + src / G, feat, feat, lane, sum, 0, nullptr);
   }
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int
 // into the piece are summed and added to C (cleared by csr_spmm_kernel) with atomics.
 // Pieces that touch no long row -- nearly all of them -- end after looking at their rows.
 template <int G, int REP, bool INDIRECT = false>
-__global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int64_t nnz, int piece,
+__global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int64_t nnz, int piece, int long_row,
                                                             const float* __restrict__ A,
                                                             const float* __restrict__ B,
                                                             float* __restrict__ C,
@@ -390,7 +405,7 @@ __global__ __launch_bounds__(256) void csr_long_rows_kernel(int m, int feat, int
     int rs = 0, re = 0;
     if (r < m) rs = indptr[r], re = indptr[r + 1];
     more = !__any(r >= m || re >= p1);
-    uint64_t todo = __ballot(rs < p1 && re - rs > kLongRow);
+    uint64_t todo = __ballot(rs < p1 && re - rs > long_row);
     while (todo) {
       const int src = __ffsll((long long)todo) - 1;
       todo &= todo - 1;
@@ -942,9 +957,9 @@ int launch_merged(const MergedRows& mr, int32_t m, int32_t n, int32_t feat, cons
   const float* vals = reinterpret_cast<const float*>(mr.vals);
 #define STIR_MERGED(G, REP)                                                                                   \
   {                                                                                                           \
-    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4, true>), grid, block, 0, st, m, feat, vals, d_B, d_C,       \
+    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4, true>), grid, block, 0, st, m, feat, kLongRow, vals, d_B, d_C,       \
                        mr.slot_ptr, mr.cols);                                                                 \
-    hipLaunchKernelGGL((csr_long_rows_kernel<G, REP, true>), pieces, block, 0, st, m, feat, mr.slots, piece,   \
+    hipLaunchKernelGGL((csr_long_rows_kernel<G, REP, true>), pieces, block, 0, st, m, feat, mr.slots, piece, kLongRow,   \
                        vals, d_B, d_C, mr.slot_ptr, mr.cols);                                                 \
   }
   switch (vector_class(feat)) {
@@ -1080,23 +1095,24 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
   STIR_REQUIRE(d_B && d_C && d_indptr && (nnz == 0 || (d_A && d_indices)), "csr_spmm: null pointer argument");
   hipStream_t st = static_cast<hipStream_t>(stream);
   // Hub rows are split over many wavefronts by a second launch, or shared by a workgroup
-  const bool split = nnz * feat >= kSmallProduct;
+  const bool split = long_rows_apart(nnz, feat);
+  const int longest = long_row(m, nnz);
   const int waves = split ? 4 : kSmallWaves;
   dim3 grid((unsigned)stir::ceil_div(m, waves)), block(waves * kWave);
   const int piece = long_piece(nnz);
   dim3 pieces((unsigned)stir::ceil_div(stir::ceil_div(nnz, piece), 4));
 #define STIR_CSR_LONG(G, REP)                                                                              \
-  hipLaunchKernelGGL((csr_long_rows_kernel<G, REP>), pieces, dim3(256), 0, st, m, feat, nnz, piece, d_A, d_B, d_C, \
+  hipLaunchKernelGGL((csr_long_rows_kernel<G, REP>), pieces, dim3(256), 0, st, m, feat, nnz, piece, longest, d_A, d_B, d_C, \
                      d_indptr, d_indices)
   // one wavefront per row
 #define STIR_CSR(G, REP)                                                                                   \
   {                                                                                                        \
     if (split) {                                                                                           \
-      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4>), grid, block, 0, st, m, feat, d_A, d_B, d_C, d_indptr, \
+      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4>), grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, d_indptr, \
                          d_indices);                                                                       \
       STIR_CSR_LONG(G, REP);                                                                               \
     } else {                                                                                               \
-      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, kSmallWaves>), grid, block, 0, st, m, feat, d_A, d_B, d_C, \
+      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, kSmallWaves>), grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, \
                          d_indptr, d_indices);                                                             \
     }                                                                                                      \
   }
@@ -1105,13 +1121,13 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
   {                                                                                                        \
     const dim3 row_grid((unsigned)stir::ceil_div(m, waves * (kWave / G)));                                 \
     if (split) {                                                                                           \
-      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, 4>), row_grid, block, 0, st, m, feat, d_A, d_B, d_C,     \
+      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, 4>), row_grid, block, 0, st, m, feat, longest, d_A, d_B, d_C,     \
                          d_indptr, d_indices);                                                             \
       STIR_CSR_LONG(G, 1);                                                                                 \
     } else if (m <= kWavePerRow) {                                                                         \
       STIR_CSR(G, 1)                                                                                       \
     } else {                                                                                               \
-      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, kSmallWaves>), row_grid, block, 0, st, m, feat, d_A, d_B, d_C, \
+      hipLaunchKernelGGL((csr_spmm_rows_kernel<G, kSmallWaves>), row_grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, \
                          d_indptr, d_indices);                                                             \
     }                                                                                                      \
   }

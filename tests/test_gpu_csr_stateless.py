@@ -1,0 +1,48 @@
+"""The CSR product without a workspace: one launch below a size, a second one for long rows above it."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from sparsetir_amd import _lib
+from test_gpu_spmm import _check
+
+pytestmark = pytest.mark.gpu
+
+FEW = 1 << 18  # nonzeros; below, two launches from 20 M products on, from there on from 6 M
+
+
+def _run(dev, m, n, feat, indptr, indices, vals, x):
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    p = lambda a: ctypes.c_void_p(a.data_ptr())
+    arrays = [t(vals), t(x.ravel()), torch.full((m * feat,), float("nan"), device=dev), t(indptr), t(indices)]
+    _lib.check(_lib.lib().stir_csr_spmm_f32(m, n, feat, len(indices), *[p(a) for a in arrays],
+                                            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    return arrays[2].cpu().numpy().reshape(m, feat)
+
+
+@pytest.mark.parametrize("feat,nnz", [(77, 20_000_000 // 77), (77, 20_000_000 // 77 + 1), (100, 199_999), (100, 200_000),
+                                      (512, 39_063), (24, FEW - 1), (24, FEW), (23, FEW), (128, FEW)])
+@pytest.mark.parametrize("m", [90, 3000, 60000])
+def test_both_sides_of_the_lines(dev, m, feat, nnz):
+    """Row lengths around the longest that stays with a wavefront (64 to 256, by the average row), empty rows and
+    rows of many pieces, at sizes next to where the second launch begins."""
+    n = 5000
+    rng = np.random.default_rng(feat + nnz + m)
+    average = nnz // m
+    ordinary = min(256, max(64, 4 * average)) if nnz < FEW else 64
+    deg = np.zeros(m, np.int64)
+    for k, d in enumerate([ordinary, ordinary + 1, 64, 65, 0, 128, 129, 4000, 257, 0, 2049]):
+        deg[m - 1 - 2 * k] = d
+    free = np.flatnonzero(deg == 0)[:-3]
+    deg += np.bincount(rng.choice(free, nnz - deg.sum()), minlength=m)
+    assert deg.sum() == nnz
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    indices = rng.integers(0, n, nnz).astype(np.int32)
+    vals = rng.random(nnz, dtype=np.float32) - np.float32(0.4)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    got = _run(dev, m, n, feat, indptr, indices, vals, x)
+    assert np.all(got[deg == 0] == 0.0)
+    _check(got, indptr, indices, vals, x, f"m={m} feat={feat} nnz={nnz}")

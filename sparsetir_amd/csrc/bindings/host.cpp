@@ -75,7 +75,8 @@ const at::Tensor* take(PyObject* o, const Operand& want, int device) {
   if (!THPVariable_Check(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
   if (!t.defined() || !t.is_cuda() || t.scalar_type() != want.dtype || t.layout() != c10::kStrided || t.dim() != 1 ||
-      t.size(0) != want.length || !t.is_contiguous() || t.get_device() != device || t.is_inference())
+      t.size(0) != want.length || !t.is_contiguous() || t.get_device() != device ||
+      ((want.key & kKeyVersion) && t.is_inference()))  // an inference tensor counts no versions
     return nullptr;
   return &t;
 }
@@ -483,10 +484,10 @@ PyObject* column_part_hyb(PyObject*, PyObject* args) {
     const size_t nb = widths.size();
     if (m < 0 || nb == 0 || nb > 32 || !THPVariable_Check(o_idx)) Py_RETURN_NONE;
     const int64_t nnz = THPVariable_Unpack(o_idx).numel();
-    const at::Tensor* ptr = take(o_ptr, {c10::ScalarType::Int, (int64_t)m + 1, 0}, device);
-    const at::Tensor* idx = take(o_idx, {c10::ScalarType::Int, nnz, 0}, device);
+    const at::Tensor* ptr = take(o_ptr, {c10::ScalarType::Int, (int64_t)m + 1, kKeyVersion}, device);
+    const at::Tensor* idx = take(o_idx, {c10::ScalarType::Int, nnz, kKeyVersion}, device);
     const bool with_values = o_values != Py_None;
-    const at::Tensor* val = with_values ? take(o_values, {c10::ScalarType::Float, nnz, 0}, device) : nullptr;
+    const at::Tensor* val = with_values ? take(o_values, {c10::ScalarType::Float, nnz, kKeyVersion}, device) : nullptr;
     if (!ptr || !idx || (with_values && !val)) Py_RETURN_NONE;
     void* st = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
     const int32_t* d_ptr = static_cast<const int32_t*>(ptr->data_ptr());

@@ -205,6 +205,11 @@ class CsrMM(_Operator):
         dev = self._check(args, self._operands)
         a, b, c, indptr, indices = args
         with torch.cuda.device(dev):
+            # the launcher has the workspace, and takes tensors of the device that is current
+            rc = self._launch(args)
+            if rc != 1:
+                _lib.check(rc)
+                return
             _lib.check(self.L.stir_csr_spmm_f32(self.m, self.n, self.feat, self.nnz, _ptr(a),
                                                 _ptr(b), _ptr(c), _ptr(indptr), _ptr(indices),
                                                 _stream()))

@@ -109,3 +109,41 @@ def test_threads_share_an_operator(dev):
     assert len(f._plans) == f._plans.capacity
     for k in range(12):
         product(k)
+
+
+def test_inference_tensors_get_the_same_bits(dev):
+    """Tensors made under inference_mode count no versions, which only what a plan depends on has to: a CSR product
+    and the features of a planned operator take the same way as under no_grad, to the same bits."""
+    rng = np.random.default_rng(3)
+    m, n, feat = 9001, 3000, 64
+    deg = rng.integers(0, 12, m)
+    deg[[0, 5, m // 2, m - 1]] = [3000, 129, 1000, 400]
+    indptr = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)).to(dev)
+    nnz = int(deg.sum())
+    indices = torch.from_numpy(rng.integers(0, n, nnz).astype(np.int32)).to(dev)
+    a, x = torch.rand(nnz, device=dev), torch.randn(n * feat, device=dev)
+    f = ops.build_csrmm(m, n, feat, nnz)
+    want = torch.empty(m * feat, device=dev)
+    f(a, x, want, indptr, indices)
+    with torch.inference_mode():
+        args = [t.clone() for t in (a, x, want, indptr, indices)]
+        assert all(t.is_inference() for t in args)
+        args[2].fill_(float("nan"))
+        f(*args)
+        assert torch.equal(args[2], want)
+    args = [a, x, torch.empty_like(want), indptr, indices]
+    f._call(*args)  # the way of a call that the launcher did not take, on another device than the current one say
+    assert torch.equal(args[2], want)
+
+    x, mats, f = _graphs(dev, 1)
+    a, r, c, want = mats[0]
+    z, zi = torch.zeros(0, device=dev), torch.zeros(0, dtype=torch.int32, device=dev)
+    y = torch.zeros_like(x)
+    f(x.reshape(-1), y.reshape(-1), a, r, c, z, zi, zi)
+    builds, slow = f.plan_builds, f._call
+    f._call = None  # not needed
+    with torch.inference_mode():
+        x2, y2 = x.clone().reshape(-1), torch.zeros_like(x).reshape(-1)
+        f(x2, y2, a, r, c, z, zi, zi)
+        assert torch.equal(y2, y.reshape(-1)) and f.plan_builds == builds
+    f._call = slow

@@ -213,12 +213,13 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
 
 /*
  * The same product by workgroups of equal work, for callers that keep a workspace: device memory of
- * stir_csr_spmm_workspace_bytes() bytes, aligned to 16, that holds zeros before the first call and is
- * left to this operator (same m, feat and nnz) between calls.  Calls that may overlap in time need
+ * stir_csr_spmm_workspace_bytes() bytes, aligned to 16, whose first stir_csr_spmm_workspace_clear_bytes()
+ * are zero before the first call and which is left to this operator (same m, feat and nnz) between calls.  Calls that may overlap in time need
  * workspaces of their own; the same bits come out every time.  0 bytes: no workspace is needed, it may
  * be null and the call is stir_csr_spmm_f32.
  */
 size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz);
+size_t stir_csr_spmm_workspace_clear_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz);
 int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A,
                                 const float* d_B, float* d_C, const int32_t* d_indptr,
                                 const int32_t* d_indices, void* d_workspace, void* stream);

@@ -42,6 +42,7 @@ SIGNATURES = {
     "stir_csr_to_bsr_fill": (I32, [I32, I32, I32, VP, VP, VP, VP, VP, VP, VP, I32, I64, VP]),
     "stir_csr_spmm_f32": (I32, [I32, I32, I32, I64, VP, VP, VP, VP, VP, VP]),
     "stir_csr_spmm_workspace_bytes": (SZ, [I32, I32, I32, I64]),
+    "stir_csr_spmm_workspace_clear_bytes": (SZ, [I32, I32, I32, I64]),
     "stir_csr_spmm_f32_workspace": (I32, [I32, I32, I32, I64, VP, VP, VP, VP, VP, VP, VP]),
     "stir_hyb_plan_create": (I32, [VP, I32, I32, I32, I32, VP, VP, VP, VP, VP]),
     "stir_hyb_plan_create_ex": (I32, [VP, I32, I32, I32, I32, VP, VP, VP, VP, VP, ctypes.c_uint32]),

@@ -16,8 +16,8 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
-#include <ATen/ops/zeros.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
@@ -51,7 +51,7 @@ struct Plan {
   PyObject* name;
 };
 
-// Zeroed once, then left to the calls on one stream, which run one after the other
+// Counters at the front, zeroed once; then left to the calls on one stream, which run one after the other
 struct Workspace {
   c10::hip::HIPStream stream;
   at::Tensor memory;
@@ -66,7 +66,7 @@ struct Launcher {
   std::vector<Plan>* plans;     // as many as the operator keeps, the one used last in front
   std::vector<int64_t>* key;    // of the call in hand, for as long as it holds the GIL
   std::vector<void*>* in_use;   // a plan per launch that is under way without the GIL
-  size_t workspace_bytes;       // of a call (CSR SpMM)
+  size_t workspace_bytes, counter_bytes;  // of a call (CSR SpMM)
   std::vector<Workspace>* workspaces;  // one per stream the operator runs on, the one used last in front
 };
 
@@ -83,22 +83,28 @@ const at::Tensor* take(PyObject* o, const Operand& want, int device) {
 
 int64_t version_of(const at::Tensor& t) { return (int64_t)t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
-// The workspace of a call on `st`.  A call that is being captured gets one of its own, cleared by the
-// graph itself: the graph may be replayed on any stream.  `held` keeps it until the call is recorded.
+at::Tensor new_workspace(const Launcher* l, const at::TensorOptions& on) {
+  at::Tensor t = at::empty({(int64_t)l->workspace_bytes}, on);
+  t.narrow(0, 0, (int64_t)l->counter_bytes).zero_();
+  return t;
+}
+
+// The workspace of a call on `st`.  A call that is being captured gets one of its own, its counters cleared by
+// the graph itself: the graph may be replayed on any stream.  `held` keeps it until the call is recorded.
 void* workspace(Launcher* l, const c10::hip::HIPStream& st, at::Tensor* held) {
   std::vector<Workspace>& all = *l->workspaces;
   if (!all.empty() && all.front().stream == st && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
     return all.front().memory.data_ptr();
   const at::TensorOptions on = at::TensorOptions(c10::ScalarType::Byte).device(c10::DeviceType::CUDA, st.device_index());
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
-    *held = at::zeros({(int64_t)l->workspace_bytes}, on);
+    *held = new_workspace(l, on);
     return held->data_ptr();
   }
   size_t at = 0;
   while (at < all.size() && all[at].stream != st) ++at;
   if (at == all.size()) {
     if (at == kWorkspaces) all.pop_back(), --at;  // back to the allocator of its stream
-    all.push_back({st, at::zeros({(int64_t)l->workspace_bytes}, on)});
+    all.push_back({st, new_workspace(l, on)});
   }
   std::rotate(all.begin(), all.begin() + at, all.begin() + at + 1);
   return all.front().memory.data_ptr();
@@ -420,6 +426,7 @@ PyObject* launcher_new(PyTypeObject*, PyObject* args, PyObject*) {
   if (l->kind == kCsr && l->sizes->size() == 4) {
     const std::vector<int64_t>& n = *l->sizes;
     l->workspace_bytes = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
+    l->counter_bytes = stir_csr_spmm_workspace_clear_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
   }
   return reinterpret_cast<PyObject*>(l);
 }

@@ -406,12 +406,18 @@ int launch_merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots, co
 
 extern "C" {
 
+// the counters, one per workgroup; behind them two partial rows per workgroup
+size_t stir_csr_spmm_workspace_clear_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
+  if (m < 0 || n < 0 || feat <= 0 || nnz < 0 || !balanced(m, n, feat, nnz)) return 0;
+  const size_t parts = size_t(workgroups(m, nnz)) * stir::ceil_div(feat, 16 << slice_class(n, feat, nnz));
+  return (parts * 4 + 15) / 16 * 16;
+}
+
 size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   if (m < 0 || n < 0 || feat <= 0 || nnz < 0 || !balanced(m, n, feat, nnz)) return 0;
-  const size_t wgs = (size_t)workgroups(m, nnz);
   const int c = slice_class(n, feat, nnz);
-  const size_t parts = wgs * stir::ceil_div(feat, 16 << c);
-  return (parts * 4 + 15) / 16 * 16 + parts * 2 * (size_t(16) << c) * 4;
+  const size_t parts = size_t(workgroups(m, nnz)) * stir::ceil_div(feat, 16 << c);
+  return stir_csr_spmm_workspace_clear_bytes(m, n, feat, nnz) + parts * 2 * (size_t(16) << c) * 4;
 }
 
 int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz, const float* d_A, const float* d_B,
@@ -428,7 +434,8 @@ int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz,
   STIR_REQUIRE(grid < (int64_t(1) << 31), "csr_spmm: %lld workgroups exceed one launch", (long long)grid);
   const int items = entries_per_workgroup(m, nnz);
   uint32_t* counters = static_cast<uint32_t*>(d_workspace);
-  float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) + (size_t(wgs) * slices * 4 + 15) / 16 * 16);
+  float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) +
+                                             stir_csr_spmm_workspace_clear_bytes(m, n, feat, nnz));
   return launch<false>(c, grid, slices, items, m, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, counters, partials,
                        static_cast<hipStream_t>(stream));
 }

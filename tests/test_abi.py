@@ -65,3 +65,15 @@ def test_probe_library_exports_its_entry_points():
     lib = ctypes.CDLL(path)
     for name in ("bench_probe_copy", "bench_probe_gather", "bench_probe_mfma_f16", "bench_probe_atomic_rows"):
         assert hasattr(lib, name), name
+
+
+def test_csr_workspace_needs_few_zeros():
+    """Of the workspace of a CSR product only the counters have to be zero: one word per workgroup, next to two
+    partial rows each."""
+    L.lib()
+    total, clear = L.lib().stir_csr_spmm_workspace_bytes, L.lib().stir_csr_spmm_workspace_clear_bytes
+    for m, n, feat, nnz in [(169343, 169343, 47, 1166243), (9001, 3000, 4, 100000), (300000, 300000, 256, 7800000)]:
+        row = 16 << max(0, (feat - 1).bit_length() - 4)
+        assert 0 < clear(m, n, feat, nnz) <= total(m, n, feat, nnz) / min(row, 64)
+        assert clear(m, n, feat, nnz) % 16 == 0
+    assert total(100, 100, 32, 500) == clear(100, 100, 32, 500) == 0  # none is needed

@@ -1,9 +1,11 @@
 """CSR products by workgroups of equal work: one launch, rows cut between workgroups and lane groups."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from sparsetir_amd import ops
+from sparsetir_amd import _lib, ops
 from test_gpu_spmm import _check
 
 pytestmark = pytest.mark.gpu
@@ -62,3 +64,27 @@ def test_rows_across_workgroups(dev, feat, m, most):
 def test_feature_slices(dev, feat, m, most):
     """Products large enough for slices of 64 features, two to eight of them."""
     test_rows_across_workgroups(dev, feat, m, most)
+
+
+@pytest.mark.parametrize("feat", [4, 47, 64, 256])
+def test_only_the_counters_are_cleared(dev, feat):
+    """What is in the workspace behind the counters does not matter, and the counters are zero again afterwards."""
+    rng = np.random.default_rng(feat)
+    m, n = 9001, 3000
+    deg, indptr, indices = _matrix(rng, m, n, [129, 4000, 1000], 30)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    p = lambda a: ctypes.c_void_p(a.data_ptr())
+    vals = rng.random(len(indices), dtype=np.float32) - np.float32(0.4)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    lib = _lib.lib()
+    size = (m, n, feat, len(indices))
+    clear = lib.stir_csr_spmm_workspace_clear_bytes(*size)
+    ws = torch.full((lib.stir_csr_spmm_workspace_bytes(*size),), 255, dtype=torch.uint8, device=dev)
+    ws[:clear] = 0
+    args = [t(vals), t(x.ravel()), torch.full((m * feat,), float("nan"), device=dev), t(indptr), t(indices), ws]
+    for _ in range(2):
+        _lib.check(lib.stir_csr_spmm_f32_workspace(*size, *[p(a) for a in args],
+                                                   ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        assert not ws[:clear].any()
+        _check(args[2].cpu().numpy().reshape(m, feat), indptr, indices, vals, x, f"feat={feat}")

@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "coherent.h"
 #include "common.h"
 #include "../../include/sparsetir_amd.h"
 
@@ -441,23 +442,6 @@ struct TcPiece {
   int32_t pad;
 };
 
-// Sixteen bytes through to the memory that all XCDs see, and from there (a load: after arrived_all(), which waits for
-// every load of the wavefront).  As four-byte atomics a partial tile took four masked writes per 16 bytes.
-__device__ __forceinline__ void coherent_store(float* p, const f32x4& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-}
-__device__ __forceinline__ f32x4 coherent_load(const float* p) {
-  f32x4 v;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=v"(v) : "v"(p) : "memory");
-  return v;
-}
-template <int N>
-__device__ __forceinline__ void arrived_all(f32x4 (&v)[N]) {
-  asm volatile("s_waitcnt vmcnt(0)" : "+v"(v[0]) : : "memory");
-#pragma unroll
-  for (int u = 1; u < N; ++u) asm volatile("" : "+v"(v[u]));
-}
-
 typedef __fp16 tr16x4 __attribute__((__vector_size__(4 * sizeof(__fp16))));  // result type of the transposing LDS read
 #define STIR_LDS __attribute__((address_space(3)))
 
@@ -647,7 +631,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
       if (!part) {
         tc_store4<OUT>(C, (io * T + row) * feat + fcol, sum, aligned);
       } else {
-        coherent_store(part + (int64_t)row * feat + fcol, f32x4{sum.x, sum.y, sum.z, sum.w});
+        stir::coherent_store(part + (int64_t)row * feat + fcol, stir::f32x4c{sum.x, sum.y, sum.z, sum.w});
       }
     }
   }
@@ -671,12 +655,13 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
     const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
     if (fcol >= feat) continue;
     const int64_t e = (int64_t)row * feat + fcol;
-    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    stir::f32x4c sum = {0.f, 0.f, 0.f, 0.f};
     for (int p0 = 0; p0 < pc.pieces; p0 += 8) {
-      f32x4 y[8];
+      stir::f32x4c y[8];
+      const float* at[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) y[u] = coherent_load(first + min(p0 + u, pc.pieces - 1) * elems + e);
-      arrived_all(y);
+      for (int u = 0; u < 8; ++u) at[u] = first + min(p0 + u, pc.pieces - 1) * elems + e;
+      stir::coherent_load(y, at);
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         if (p0 + u < pc.pieces) sum += y[u];

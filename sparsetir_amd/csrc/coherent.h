@@ -6,29 +6,26 @@
 
 namespace stir {
 
-typedef float f32x4c __attribute__((ext_vector_type(4)));
+// Buffer instructions with the bit that a device-wide atomic load or store sets (sc1), rather than inline assembly:
+// the compiler knows when the result of a load is there and which registers a store still reads.
+class CoherentPiece {
+ public:
+  typedef uint32_t Four __attribute__((ext_vector_type(4)));
+  // `bytes` (below 2^32) from a 16-byte aligned address that is the same for all lanes
+  __device__ __forceinline__ CoherentPiece(float* base, uint32_t bytes)
+      : r_(__builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00027000)) {}
+  // offsets in floats, a multiple of four
+  __device__ __forceinline__ float4 load(uint32_t at) const {
+    return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r_, 4 * at, 0, kSc1));
+  }
+  // has arrived when the wavefront's vmcnt is zero
+  __device__ __forceinline__ void store(uint32_t at, const float4& v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Four, v), r_, 4 * at, 0, kSc1);
+  }
 
-// Has arrived when the wavefront's vmcnt is zero.
-__device__ __forceinline__ void coherent_store(float* p, const f32x4c& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-}
-
-// v[u] = the four floats at p[u], all eight in flight together.  One statement, the wait included: to the compiler
-// the result of a load it does not know of is there at once, and it may move it before a wait that stands apart.
-__device__ __forceinline__ void coherent_load(f32x4c (&v)[8], const float* const (&p)[8]) {
-  asm volatile(
-      "global_load_dwordx4 %0, %8, off sc1\n\t"
-      "global_load_dwordx4 %1, %9, off sc1\n\t"
-      "global_load_dwordx4 %2, %10, off sc1\n\t"
-      "global_load_dwordx4 %3, %11, off sc1\n\t"
-      "global_load_dwordx4 %4, %12, off sc1\n\t"
-      "global_load_dwordx4 %5, %13, off sc1\n\t"
-      "global_load_dwordx4 %6, %14, off sc1\n\t"
-      "global_load_dwordx4 %7, %15, off sc1\n\t"
-      "s_waitcnt vmcnt(0)"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7])
-      : "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7])
-      : "memory");
-}
+ private:
+  static constexpr int kSc1 = 16;
+  __amdgpu_buffer_rsrc_t r_;
+};
 
 }  // namespace stir

@@ -608,7 +608,8 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
   const int used = min(W, s_end - s_begin);
   const int64_t elems = (int64_t)T * feat;
   float* red = reinterpret_cast<float*>(lds);  // [wavefront][tile][register][lane]
-  float* part = pc.slot < 0 ? nullptr : scratch + (int64_t)pc.slot * elems;
+  const bool part = pc.slot >= 0;
+  const stir::CoherentPiece partial(scratch + (part ? (int64_t)pc.slot * elems : 0), part ? (uint32_t)(elems * 4) : 0u);
 #pragma unroll
   for (int t0 = 0; t0 < NTL; t0 += ATONCE) {
     __syncthreads();  // images, or the sums before, are done with
@@ -631,7 +632,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
       if (!part) {
         tc_store4<OUT>(C, (io * T + row) * feat + fcol, sum, aligned);
       } else {
-        stir::coherent_store(part + (int64_t)row * feat + fcol, stir::f32x4c{sum.x, sum.y, sum.z, sum.w});
+        partial.store((uint32_t)(row * feat + fcol), sum);
       }
     }
   }
@@ -650,23 +651,23 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
   __syncthreads();
   if (!last_of_tile) return;
   // C[tile, f0 .. f0 + TF) = the partial tiles added in piece order, rounded once
-  const float* first = scratch + (int64_t)pc.first_slot * elems;
+  float* first = scratch + (int64_t)pc.first_slot * elems;
   for (int w = tid; w < T * (TF / 4); w += 64 * W) {
     const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
     if (fcol >= feat) continue;
     const int64_t e = (int64_t)row * feat + fcol;
-    stir::f32x4c sum = {0.f, 0.f, 0.f, 0.f};
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int p0 = 0; p0 < pc.pieces; p0 += 8) {
-      stir::f32x4c y[8];
-      const float* at[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) at[u] = first + min(p0 + u, pc.pieces - 1) * elems + e;
-      stir::coherent_load(y, at);
+      float4 y[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (p0 + u < pc.pieces) sum += y[u];
+        y[u] = stir::CoherentPiece(first + min(p0 + u, pc.pieces - 1) * elems, (uint32_t)(elems * 4)).load((uint32_t)e);
+        __builtin_amdgcn_sched_barrier(0);  // all eight, then the sums
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u < pc.pieces) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
     }
-    tc_store4<OUT>(C, io * elems + e, make_float4(sum[0], sum[1], sum[2], sum[3]), aligned);
+    tc_store4<OUT>(C, io * elems + e, sum, aligned);
   }
 }
 

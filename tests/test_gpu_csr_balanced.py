@@ -88,3 +88,26 @@ def test_only_the_counters_are_cleared(dev, feat):
         torch.cuda.synchronize()
         assert not ws[:clear].any()
         _check(args[2].cpu().numpy().reshape(m, feat), indptr, indices, vals, x, f"feat={feat}")
+
+
+@pytest.mark.parametrize("feat,hub", [(4, 1_200_000), (16, 1_000_003), (256, 400_001), (300, 300_000)])
+def test_a_row_over_thousands_of_workgroups(dev, feat, hub):
+    """The workgroup that finishes last adds hundreds of partial rows per lane group, a number that is no multiple of
+    those it requests at a time; the same bits again."""
+    rng = np.random.default_rng(feat)
+    m, n = 12000, 20000
+    deg = rng.integers(0, 4, m)
+    deg[m // 3] = hub
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    indices = rng.integers(0, n, indptr[-1]).astype(np.int32)
+    vals = rng.random(len(indices), dtype=np.float32) - np.float32(0.4)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    f = ops.build_csrmm(m, n, feat, len(indices))
+    c = [torch.full((m * feat,), float("nan"), device=dev) for _ in range(2)]
+    args = [t(vals), t(x.ravel())], [t(indptr), t(indices)]
+    for y in c:
+        f(*args[0], y, *args[1])
+    torch.cuda.synchronize()
+    assert torch.equal(*c)
+    _check(c[0].cpu().numpy().reshape(m, feat), indptr, indices, vals, x, f"feat={feat} hub={hub}")

@@ -22,6 +22,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include "call_answer.h"
 #include "common.h"
 #include "row_lookup.h"
 #include "../../include/sparsetir_amd.h"
@@ -750,14 +751,13 @@ struct OneOutputs {
   int32_t* mask[kOneBuckets];
   float* a[kOneBuckets];  // null without values
 };
-// In host memory, written by the kernels.  rows[b]: the ELL rows of bucket b below the number of the call, one
-// 8-byte store that needs no order with another.  The host watches for it: waiting for the stream takes 5 us
-// more, from the end of the kernel to the wake-up.
+// In host memory, written by the kernels.  rows[b]: the answer for bucket b (call_answer.h).  The host watches for
+// it: waiting for the stream takes 5 us more, from the end of the kernel to the wake-up.
 struct OneAnswer {
   uint64_t rows[kOneBuckets];
   int32_t bad_range, bad_indptr;  // there before the rows
 };
-constexpr int kCallShift = 40;  // rows of a bucket are fewer
+using stir::kCallShift;
 __device__ __forceinline__ void answer_rows(OneAnswer* answer, int b, int64_t nrows, uint32_t number) {
   __hip_atomic_store(&answer->rows[b], (uint64_t)nrows | ((uint64_t)number << kCallShift), __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1036,7 +1036,7 @@ int answer_box(const char* who, AnswerBox** out, uint32_t** arrived) {
 int wait_for_answer(const AnswerBox& box, int buckets, hipStream_t st) {
   int b = 0;
   for (int turn = 0; turn < 20000; ++turn) {
-    while (b < buckets && (__atomic_load_n(&box.host->rows[b], __ATOMIC_ACQUIRE) >> kCallShift) == box.number) ++b;
+    while (b < buckets && stir::answered(&box.host->rows[b], box.number)) ++b;
     if (b == buckets) return 0;
     __builtin_ia32_pause();
   }
@@ -1368,7 +1368,8 @@ int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int
   uint32_t* arrived = nullptr;
   if (answer_box(who, &box, &arrived)) return -1;
   box->host->bad_range = box->host->bad_indptr = 0;
-  const uint32_t number = box->number = (box->number + 1) & ((1u << (64 - kCallShift)) - 1);
+  const uint32_t number = box->number = stir::next_call(box->number);
+  stir::forget_answers(box->host->rows, NB);
   const bool few = W <= kFewCounts;
   OneWidths widths = {};
   std::copy(buckets, buckets + NB, widths.w);
@@ -1389,7 +1390,7 @@ int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int
   if (wait_for_answer(*box, NB, st)) return -1;
   STIR_REQUIRE(!box->host->bad_indptr, "%s: indptr is not a CSR row pointer of %lld nonzeros", who, (long long)max_nnz);
   STIR_REQUIRE(!box->host->bad_range, "%s: a column index lies outside [0, %d)", who, num_cols);
-  for (int k = 0; k < NB; ++k) nrows[k] = (int64_t)(box->host->rows[k] & ((uint64_t(1) << kCallShift) - 1));
+  for (int k = 0; k < NB; ++k) nrows[k] = stir::answered_rows(box->host->rows[k]);
   for (int k = 0; k < NB; ++k)
     STIR_REQUIRE(nrows[k] < kMaxSlots / buckets[k], "%s: bucket %d holds too many slots", who, k);
   return 0;

@@ -417,9 +417,9 @@ __global__ __launch_bounds__(64 * (32 / NTL)) void tcspmm_long_kernel(int feat, 
   }
 }
 
-// ---- with a plan (stir_tc_plan): one launch of units, each a whole row tile of at most kPieceSteps steps or a
-// piece of that many of a longer one.  The pieces are listed once by the plan, the longest tiles first, and come
-// before the whole tiles in the launch.  A unit is a workgroup of W wavefronts for (T rows) x (32 * NTL
+// ---- with a plan (stir_tc_plan): one launch of units, each a whole row tile or a piece of a long one.  Tiles of more
+// than kWholeSteps steps are listed once by the plan, the longest first, and come before the others in the launch;
+// those that the launch would end on are cut into pieces.  A unit is a workgroup of W wavefronts for (T rows) x (32 * NTL
 // features) that take its steps in turn: wavefront w the steps w, w + W, ..., each with an image of its step's 32
 // gathered rows of B in its own LDS -- no workgroup barrier in the loop, the LDS operations of one wavefront
 // execute in order -- and the partial results meet in LDS at the end.  The image is the rows as they are, 16-byte
@@ -431,11 +431,18 @@ __global__ __launch_bounds__(64 * (32 / NTL)) void tcspmm_long_kernel(int feat, 
 // sets back to zero) adds them up in piece order and rounds once: the same bits whichever workgroup comes last.
 // The partial tiles are written and read with device-coherent accesses (they pass the XCD's L2), so that no
 // workgroup has to write back or invalidate a whole L2, as a release or acquire at device scope does.
-constexpr int kPieceSteps = 32;
+constexpr int kWholeSteps = 32;
+// A tile of more than this part of all steps is cut: about the units that run at a time, so that what is left whole
+// ends with the others.  Pieces cost memory for partial tiles, at most 2 * kShares of them.  us with every tile above
+// 32 steps cut / with parts of 4096 / 2048 / 1024 / 512 / 128: 169 k rows, 1.17 M nonzeros with hubs, 128 features, 16
+// rows 62.1 / 62.0 / 61.9 / 61.3 / 63.2 / 166; 200 k, 4 M, 64, 32 rows 118 / 118 / 108 / 107 / 115 / 204; the same,
+// skewed columns, 16 rows 57.3 / 57.2 / 56.7 / 62.8 / 80.2 / 80.4; 40 k, 1 M, 128, 32 rows 45.6 / 45.1 / 45.2 / 45.1 /
+// 42.8 / 58.9.
+constexpr int kShares = 2048;
 
 struct TcPiece {
   int32_t tile, step_begin, step_end;
-  int32_t slot;        // partial tile in the scratch memory
+  int32_t slot;        // partial tile in the scratch memory; -1: the whole tile
   int32_t first_slot;  // of the tile's pieces
   int32_t pieces;      // of the tile
   int32_t multi;       // number of the tile among the long tiles
@@ -515,7 +522,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
   } else {
     if (io >= mb) return;
     s_end = tile_steps(indptr, io);
-    if (s_end > kPieceSteps) return;  // in pieces
+    if (s_end > kWholeSteps) return;  // in the list
   }
   const int64_t g_begin = indptr[io], g_end = indptr[io + 1];
   const int64_t rows_total = (g_end - g_begin) * kGroup;
@@ -773,19 +780,17 @@ struct stir_tc_plan {
   int device = 0;
   int64_t n_pieces = 0, n_multi = 0, slots = 0;
   TcPiece* d_pieces = nullptr;
-  float* d_scratch = nullptr;  // slots x 32 x feat floats, grown by the launch that needs more
-  size_t scratch_bytes = 0;
-  // per tile of several pieces and feature tile: the pieces that have finished in the running
-  // launch; zero between launches (the workgroup that counts last clears its counter)
+  // Counters, and behind them the partial tiles, made anew by the launch that needs more.  A counter per cut tile and
+  // feature tile: the pieces that have finished in the running launch; zero between launches (the workgroup that
+  // counts last clears its counter).
   uint32_t* d_arrived = nullptr;
-  size_t arrived_count = 0;
+  size_t arrived_bytes = 0, scratch_bytes = 0;
 };
 
 extern "C" int stir_tc_plan_destroy(stir_tc_plan* plan) {
   if (!plan) return 0;
   if (plan->d_pieces) (void)hipFree(plan->d_pieces);
   if (plan->d_arrived) (void)hipFree(plan->d_arrived);
-  if (plan->d_scratch) (void)hipFree(plan->d_scratch);
   delete plan;
   return 0;
 }
@@ -801,24 +806,27 @@ extern "C" int stir_tc_plan_create(stir_tc_plan** plan, int32_t mb, const int32_
   }
   // the long tiles, longest first (ties in tile order)
   std::vector<std::pair<int32_t, int32_t>> longs;  // (steps, tile)
+  int64_t all_steps = 0;
   for (int32_t io = 0; io < mb; ++io) {
     STIR_REQUIRE(ptr[io] <= ptr[io + 1], "tc_plan_create: indptr decreases at tile %d", io);
     const int64_t steps = ((int64_t)(ptr[io + 1] - ptr[io]) * kGroup + 31) / 32;
-    if (steps > kPieceSteps) longs.emplace_back((int32_t)steps, io);
+    if (steps > kWholeSteps) longs.emplace_back((int32_t)steps, io);
+    all_steps += steps;
   }
+  const int64_t most = std::max<int64_t>(kWholeSteps, all_steps / kShares);
   std::stable_sort(longs.begin(), longs.end(),
                    [](const std::pair<int32_t, int32_t>& a, const std::pair<int32_t, int32_t>& b) { return a.first > b.first; });
   std::vector<TcPiece> pieces;
   int64_t slots = 0, n_multi = 0;
   for (const auto& lt : longs) {
     const int32_t steps = lt.first, io = lt.second;
-    const int32_t n = (steps + kPieceSteps - 1) / kPieceSteps;  // pieces of equal length
+    const int32_t n = (int32_t)((steps + most - 1) / most);  // pieces of equal length
     const int32_t len = (steps + n - 1) / n;
     STIR_REQUIRE(slots + n < (int64_t(1) << 31), "tc_plan_create: too many pieces");
     for (int32_t p = 0; p < n; ++p)
-      pieces.push_back(TcPiece{io, p * len, std::min(steps, (p + 1) * len), (int32_t)(slots + p), (int32_t)slots, n,
-                               (int32_t)n_multi, 0});
-    slots += n, ++n_multi;
+      pieces.push_back(TcPiece{io, p * len, std::min(steps, (p + 1) * len), n > 1 ? (int32_t)(slots + p) : -1,
+                               (int32_t)slots, n, (int32_t)n_multi, 0});
+    if (n > 1) slots += n, ++n_multi;
   }
   stir_tc_plan* p = new stir_tc_plan();
   p->mb = mb;
@@ -856,33 +864,29 @@ extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, i
   const uint16_t* A = static_cast<const uint16_t*>(d_A);
   const uint16_t* B = static_cast<const uint16_t*>(d_B);
   const bool out32 = out_dtype == STIR_F32;
-  // the partial tiles of this tile size and feature width
-  const size_t need = size_t(plan->slots) * size_t(tile_size) * size_t(feat) * sizeof(float);
-  if (need > plan->scratch_bytes) {
-    if (plan->d_scratch) STIR_HIP(hipFree(plan->d_scratch));
-    plan->d_scratch = nullptr;
-    plan->scratch_bytes = 0;
-    STIR_HIP(hipMalloc(reinterpret_cast<void**>(&plan->d_scratch), need));
-    plan->scratch_bytes = need;
-  }
-  const size_t counters = size_t(plan->n_multi) * size_t(stir::ceil_div(feat, 32));
-  if (counters > plan->arrived_count) {
+  // the counters and partial tiles of this tile size and feature width
+  const size_t counters = (size_t(plan->n_multi) * size_t(stir::ceil_div(feat, 32)) * sizeof(uint32_t) + 255) / 256 * 256;
+  const size_t partials = size_t(plan->slots) * size_t(tile_size) * size_t(feat) * sizeof(float);
+  if (counters > plan->arrived_bytes || partials > plan->scratch_bytes) {
+    const size_t more_counters = std::max(counters, plan->arrived_bytes);
+    const size_t more_partials = std::max(partials, plan->scratch_bytes);
     if (plan->d_arrived) STIR_HIP(hipFree(plan->d_arrived));
     plan->d_arrived = nullptr;
-    plan->arrived_count = 0;
-    STIR_HIP(hipMalloc(reinterpret_cast<void**>(&plan->d_arrived), counters * sizeof(uint32_t)));
-    STIR_HIP(hipMemsetAsync(plan->d_arrived, 0, counters * sizeof(uint32_t), st));
-    plan->arrived_count = counters;
+    plan->arrived_bytes = plan->scratch_bytes = 0;
+    STIR_HIP(hipMalloc(reinterpret_cast<void**>(&plan->d_arrived), more_counters + more_partials));
+    STIR_HIP(hipMemsetAsync(plan->d_arrived, 0, more_counters, st));
+    plan->arrived_bytes = more_counters, plan->scratch_bytes = more_partials;
   }
+  float* scratch = reinterpret_cast<float*>(reinterpret_cast<char*>(plan->d_arrived) + plan->arrived_bytes);
   switch (tile_size) {
     case 8:
-      return launch_planned<8>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A, B,
+      return launch_planned<8>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A, B,
                                d_C, d_indptr, d_indices, st);
     case 16:
-      return launch_planned<16>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
+      return launch_planned<16>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A,
                                 B, d_C, d_indptr, d_indices, st);
     default:
-      return launch_planned<32>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, plan->d_scratch, plan->d_arrived, A,
+      return launch_planned<32>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A,
                                 B, d_C, d_indptr, d_indices, st);
   }
 }

@@ -59,3 +59,19 @@ def test_output_between_boundaries(dev, out_dtype):
     f(*args, shifted[1:], *tail)
     torch.cuda.synchronize()
     assert torch.equal(c, shifted[1:])
+
+
+@pytest.mark.parametrize("t,feat,out_dtype", [(8, 32, torch.float32), (16, 96, torch.float16), (32, 64, torch.float16)])
+def test_long_tiles_left_whole(dev, t, feat, out_dtype):
+    """Enough steps in all for tiles of more than 32 to stay whole: around that length and around the one from which
+    they are cut, the 2048th part of all steps."""
+    rng = np.random.default_rng(t)
+    steps = np.array([32, 33, 40, 51, 52, 102, 103, 66, 129, 200, 1, 0] * 130)
+    assert steps.sum() // 2048 == 51
+    rng.shuffle(steps)
+    deg = np.zeros(len(steps) * t, np.int64)
+    deg[np.arange(len(steps)) * t + rng.integers(0, t, len(steps))] = steps * 32 - rng.integers(0, 16, len(steps)) * (steps > 0)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    n = 9001
+    indices = ((np.arange(indptr[-1]) * 7 + 3) % n).astype(np.int32)  # distinct in a row: 7 * 6400 steps, n is no multiple of 7
+    _run(dev, indptr, indices, n, feat, False, out_dtype, t=t)

@@ -351,12 +351,11 @@ int stir_tc_spmm_f16(int32_t out_dtype, int32_t mb, int32_t tile_size, int32_t g
  * The same operator with a plan made once from the group counts (the reference
  * has no counterpart: its built operator, examples/spmm/bench_tc_spmm.py:650-656, reads nothing
  * ahead of the launch).  stir_tc_plan_create reads d_indptr (mb+1 entries) on `stream`,
- * synchronises it, and lists the row tiles of more than 16 steps (32 gathered rows each), longest
- * first, cut into pieces of at most 128 steps.  stir_tc_spmm_f16_planned then takes the arguments
- * of stir_tc_spmm_f16: the short tiles as there, then one workgroup per
- * piece -- none is started only to find its tile short, and the hub tiles of a power-law graph
- * are spread over many compute units from the start of the launch.  The pieces of a tile leave
- * fp32 partial tiles, and the workgroup that finishes last among them (a counter per tile and
+ * synchronises it, and lists the row tiles of more than 32 steps (32 gathered rows each), longest
+ * first, those of more than the 2048th part of all steps cut into pieces.  stir_tc_spmm_f16_planned then takes the arguments
+ * of stir_tc_spmm_f16: one launch, a workgroup per tile or piece and 32 to 128 features, the listed ones
+ * first, so that the hub tiles of a power-law graph are spread over many compute units from the start.
+ * The pieces of a tile leave fp32 partial tiles, and the workgroup that finishes last among them (a counter per tile and
  * feature tile, which it sets back to zero) adds them in piece order and rounds once: no atomics
  * on C, the same bits on every run (the sums are those of stir_tc_spmm_f16 up to the order of
  * the fp32 additions).  The partial tiles and counters live in memory the plan owns, sized by the
@@ -370,6 +369,18 @@ int stir_tc_plan_create(stir_tc_plan** plan, int32_t mb, const int32_t* d_indptr
 int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, int32_t mb, int32_t tile_size,
                              int32_t group_size, int32_t feat, int64_t nnzb, const void* d_A, const void* d_B,
                              void* d_C, const int32_t* d_indptr, const int32_t* d_indices, void* stream);
+/*
+ * The same launch with counters and partial tiles in the caller's memory, aligned to 16: stir_tc_plan_counter_bytes()
+ * bytes that are zero before the first call, and stir_tc_plan_partial_bytes() bytes.  Both are left to this operator
+ * between calls -- larger pieces, and other plans' calls in between, are fine -- and calls that may overlap in time
+ * need their own.  0 bytes: null will do.  Nothing is allocated.
+ */
+size_t stir_tc_plan_counter_bytes(const stir_tc_plan* plan, int32_t feat);
+size_t stir_tc_plan_partial_bytes(const stir_tc_plan* plan, int32_t tile_size, int32_t feat);
+int stir_tc_spmm_f16_workspace(const stir_tc_plan* plan, int32_t out_dtype, int32_t mb, int32_t tile_size,
+                               int32_t group_size, int32_t feat, int64_t nnzb, const void* d_A, const void* d_B,
+                               void* d_C, const int32_t* d_indptr, const int32_t* d_indices, void* d_counters,
+                               void* d_partials, void* stream);
 int stir_tc_plan_destroy(stir_tc_plan* plan);
 
 /*

@@ -51,9 +51,15 @@ struct Plan {
   PyObject* name;
 };
 
+// What a call needs of its stream's workspace: counters, which are zero between launches, and the rest.
+struct Need {
+  size_t counters, rest;
+};
+
 // Counters at the front, zeroed once; then left to the calls on one stream, which run one after the other
 struct Workspace {
   c10::hip::HIPStream stream;
+  Need has;
   at::Tensor memory;
 };
 constexpr size_t kWorkspaces = 4;  // streams an operator keeps one for
@@ -66,7 +72,7 @@ struct Launcher {
   std::vector<Plan>* plans;     // as many as the operator keeps, the one used last in front
   std::vector<int64_t>* key;    // of the call in hand, for as long as it holds the GIL
   std::vector<void*>* in_use;   // a plan per launch that is under way without the GIL
-  size_t workspace_bytes, counter_bytes;  // of a call (CSR SpMM)
+  Need csr;                     // of a CSR product
   std::vector<Workspace>* workspaces;  // one per stream the operator runs on, the one used last in front
 };
 
@@ -83,40 +89,58 @@ const at::Tensor* take(PyObject* o, const Operand& want, int device) {
 
 int64_t version_of(const at::Tensor& t) { return (int64_t)t.unsafeGetTensorImpl()->version_counter().current_version(); }
 
-at::Tensor new_workspace(const Launcher* l, const at::TensorOptions& on) {
-  at::Tensor t = at::empty({(int64_t)l->workspace_bytes}, on);
-  t.narrow(0, 0, (int64_t)l->counter_bytes).zero_();
-  return t;
+Need need_of(const Launcher* l, const void* plan) {
+  if (l->kind == kCsr) return l->csr;
+  if (l->kind != kTc) return {0, 0};
+  const stir_tc_plan* q = static_cast<const stir_tc_plan*>(plan);
+  const int32_t tile = (int32_t)(*l->sizes)[2], feat = (int32_t)(*l->sizes)[4];
+  return {stir_tc_plan_counter_bytes(q, feat), stir_tc_plan_partial_bytes(q, tile, feat)};
+}
+
+Workspace new_workspace(const c10::hip::HIPStream& st, const Need& need) {
+  const at::TensorOptions on = at::TensorOptions(c10::ScalarType::Byte).device(c10::DeviceType::CUDA, st.device_index());
+  Workspace w{st, need, at::empty({(int64_t)(need.counters + need.rest)}, on)};
+  w.memory.narrow(0, 0, (int64_t)need.counters).zero_();
+  return w;
+}
+
+// Where the two parts of a call's workspace are.
+struct Scratch {
+  char *counters = nullptr, *rest = nullptr;
+};
+Scratch scratch_of(const Workspace& w) {
+  char* p = static_cast<char*>(w.memory.data_ptr());
+  return {p, p + w.has.counters};
 }
 
 // The workspace of a call on `st`.  A call that is being captured gets one of its own, its counters cleared by
 // the graph itself: the graph may be replayed on any stream.  `held` keeps it until the call is recorded.
-void* workspace(Launcher* l, const c10::hip::HIPStream& st, at::Tensor* held) {
+Scratch workspace(Launcher* l, const c10::hip::HIPStream& st, const Need& need, at::Tensor* held) {
   std::vector<Workspace>& all = *l->workspaces;
-  if (!all.empty() && all.front().stream == st && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None)
-    return all.front().memory.data_ptr();
-  const at::TensorOptions on = at::TensorOptions(c10::ScalarType::Byte).device(c10::DeviceType::CUDA, st.device_index());
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
-    *held = new_workspace(l, on);
-    return held->data_ptr();
+    const Workspace w = new_workspace(st, need);
+    *held = w.memory;
+    return scratch_of(w);
   }
   size_t at = 0;
   while (at < all.size() && all[at].stream != st) ++at;
   if (at == all.size()) {
     if (at == kWorkspaces) all.pop_back(), --at;  // back to the allocator of its stream
-    all.push_back({st, new_workspace(l, on)});
+    all.push_back(new_workspace(st, need));
+  } else if (all[at].has.counters < need.counters || all[at].has.rest < need.rest) {  // another plan's call
+    all[at] = new_workspace(st, {std::max(all[at].has.counters, need.counters), std::max(all[at].has.rest, need.rest)});
   }
-  std::rotate(all.begin(), all.begin() + at, all.begin() + at + 1);
-  return all.front().memory.data_ptr();
+  if (at > 0) std::rotate(all.begin(), all.begin() + at, all.begin() + at + 1);
+  return scratch_of(all.front());
 }
 
-int call(const Launcher* l, void* const* p, void* plan, void* ws, void* st) {
+int call(const Launcher* l, void* const* p, void* plan, const Scratch& ws, void* st) {
   const std::vector<int64_t>& n = *l->sizes;
   auto i = [&](int k) { return (int32_t)n[k]; };
   auto f = [&](int k) { return static_cast<float*>(p[k]); };
   auto x = [&](int k) { return static_cast<int32_t*>(p[k]); };
   switch (l->kind) {
-    case kCsr: return stir_csr_spmm_f32_workspace(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), ws, st);
+    case kCsr: return stir_csr_spmm_f32_workspace(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), ws.counters, st);
     case kSddmmPreproc: return stir_sddmm_preproc(i(0), n[3], x(3), x(5), st);
     case kSddmm: return stir_sddmm_f32(i(0), i(1), i(2), n[3], f(0), f(1), f(2), x(3), x(4), x(5), st);
     case kSddmmScaled:
@@ -125,8 +149,8 @@ int call(const Launcher* l, void* const* p, void* plan, void* ws, void* st) {
     case kDbsr:
       return stir_dbsr_spmm(i(0), i(1), i(2), i(3), i(4), i(5), n[6], p[0], p[1], p[2], x(4), x(5), x(6), st);
     case kTc:
-      return stir_tc_spmm_f16_planned(static_cast<stir_tc_plan*>(plan), i(0), i(1), i(2), i(3), i(4), n[5], p[0],
-                                      p[1], p[2], x(3), x(4), st);
+      return stir_tc_spmm_f16_workspace(static_cast<const stir_tc_plan*>(plan), i(0), i(1), i(2), i(3), i(4), n[5], p[0],
+                                        p[1], p[2], x(3), x(4), ws.counters, ws.rest, st);
     case kRgms: {
       stir_rgms_plan* q = static_cast<stir_rgms_plan*>(plan);
       if (n[5] == 2) return stir_rgms_bf16(q, i(0), i(1), i(2), i(3), i(4), p[0], p[1], f(2), st);
@@ -147,7 +171,7 @@ bool planned(Kind k) { return k >= kTc; }
 
 // call() without the GIL (a launch waits when the queue is full).  Other threads may use the launcher meanwhile, so
 // nothing of it is read here but its kind and sizes, and nobody destroys `plan` before the call is done with it.
-int call_unlocked(Launcher* l, void* const* p, void* plan, void* ws, void* st) {
+int call_unlocked(Launcher* l, void* const* p, void* plan, const Scratch& ws, void* st) {
   int rc;
   if (plan) l->in_use->push_back(plan);
   Py_BEGIN_ALLOW_THREADS
@@ -216,7 +240,8 @@ PyObject* launch(PyObject* self, PyObject* args) {
     }
     const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device);
     at::Tensor held;
-    void* ws = l->workspace_bytes ? workspace(l, stream, &held) : nullptr;
+    const Need need = need_of(l, plan);
+    const Scratch ws = need.counters ? workspace(l, stream, need, &held) : Scratch();
     rc = call_unlocked(l, p, plan, ws, stream.stream());
   } catch (...) {  // a tensor without storage: the Python code says what is wrong with it
     rc = kNotTaken;
@@ -302,7 +327,7 @@ PyObject* launch_new_hyb(PyObject* self, PyObject* args) {
     made.device = (int)device;
     made.key.assign(key.begin() + 1, key.end());
     for (const Plan& q : *l->plans)
-      if (q.device == made.device && q.key == made.key) return PyLong_FromLong(call_unlocked(l, p, q.plan, nullptr, st));
+      if (q.device == made.device && q.key == made.key) return PyLong_FromLong(call_unlocked(l, p, q.plan, Scratch(), st));
     made.name = PyBytes_FromStringAndSize(reinterpret_cast<const char*>(key.data()),
                                           (Py_ssize_t)(key.size() * sizeof(int64_t)));
     if (!made.name) return nullptr;
@@ -310,7 +335,7 @@ PyObject* launch_new_hyb(PyObject* self, PyObject* args) {
     Py_BEGIN_ALLOW_THREADS
     rc = stir_hyb_plan_create(&plan, (int32_t)n[1], (int32_t)n[2], (int32_t)n[3], (int32_t)nb, widths.data(),
                               nrows.data(), A.data(), rows.data(), cols.data());
-    if (rc == 0) rc = call(l, p, plan, nullptr, st);
+    if (rc == 0) rc = call(l, p, plan, Scratch(), st);
     Py_END_ALLOW_THREADS
     made.plan = plan;
     out = rc == 0 ? Py_BuildValue("(OK)", made.name, reinterpret_cast<unsigned long long>(plan)) : PyLong_FromLong(kFailed);
@@ -425,8 +450,8 @@ PyObject* launcher_new(PyTypeObject*, PyObject* args, PyObject*) {
   }
   if (l->kind == kCsr && l->sizes->size() == 4) {
     const std::vector<int64_t>& n = *l->sizes;
-    l->workspace_bytes = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
-    l->counter_bytes = stir_csr_spmm_workspace_clear_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
+    l->csr.counters = stir_csr_spmm_workspace_clear_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]);
+    l->csr.rest = stir_csr_spmm_workspace_bytes((int32_t)n[0], (int32_t)n[1], (int32_t)n[2], n[3]) - l->csr.counters;
   }
   return reinterpret_cast<PyObject*>(l);
 }

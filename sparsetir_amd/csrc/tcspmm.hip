@@ -669,7 +669,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         y[u] = stir::CoherentPiece(first + min(p0 + u, pc.pieces - 1) * elems, (uint32_t)(elems * 4)).load((uint32_t)e);
-        __builtin_amdgcn_sched_barrier(0);  // all eight, then the sums
+      __builtin_amdgcn_sched_barrier(0);  // all eight, then the sums
 #pragma unroll
       for (int u = 0; u < 8; ++u)
         if (p0 + u < pc.pieces) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
@@ -848,10 +848,20 @@ extern "C" int stir_tc_plan_create(stir_tc_plan** plan, int32_t mb, const int32_
   return 0;
 }
 
-extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, int32_t mb, int32_t tile_size,
-                                        int32_t group_size, int32_t feat, int64_t nnzb, const void* d_A,
-                                        const void* d_B, void* d_C, const int32_t* d_indptr,
-                                        const int32_t* d_indices, void* stream) {
+extern "C" size_t stir_tc_plan_counter_bytes(const stir_tc_plan* plan, int32_t feat) {
+  if (!plan || feat <= 0) return 0;
+  return (size_t(plan->n_multi) * size_t(stir::ceil_div(feat, 32)) * sizeof(uint32_t) + 255) / 256 * 256;
+}
+
+extern "C" size_t stir_tc_plan_partial_bytes(const stir_tc_plan* plan, int32_t tile_size, int32_t feat) {
+  if (!plan || tile_size <= 0 || feat <= 0) return 0;
+  return size_t(plan->slots) * size_t(tile_size) * size_t(feat) * sizeof(float);
+}
+
+extern "C" int stir_tc_spmm_f16_workspace(const stir_tc_plan* plan, int32_t out_dtype, int32_t mb, int32_t tile_size,
+                                          int32_t group_size, int32_t feat, int64_t nnzb, const void* d_A,
+                                          const void* d_B, void* d_C, const int32_t* d_indptr, const int32_t* d_indices,
+                                          void* d_counters, void* d_partials, void* stream) {
   STIR_REQUIRE(plan, "tc_spmm_planned: plan is null");
   if (check_args(out_dtype, mb, tile_size, group_size, feat, nnzb, d_A, d_B, d_C, d_indptr, d_indices)) return -1;
   STIR_REQUIRE(plan->mb == mb, "tc_spmm_planned: the plan was made for %d row tiles, not %d", plan->mb, mb);
@@ -859,34 +869,49 @@ extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, i
   STIR_HIP(hipGetDevice(&device));
   STIR_REQUIRE(device == plan->device, "tc_spmm_planned: the plan lives on device %d, the current device is %d",
                plan->device, device);
+  STIR_REQUIRE(plan->n_multi == 0 || (d_counters && d_partials), "tc_spmm_planned: null workspace");
   if (mb == 0) return 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* A = static_cast<const uint16_t*>(d_A);
   const uint16_t* B = static_cast<const uint16_t*>(d_B);
   const bool out32 = out_dtype == STIR_F32;
-  // the counters and partial tiles of this tile size and feature width
-  const size_t counters = (size_t(plan->n_multi) * size_t(stir::ceil_div(feat, 32)) * sizeof(uint32_t) + 255) / 256 * 256;
-  const size_t partials = size_t(plan->slots) * size_t(tile_size) * size_t(feat) * sizeof(float);
-  if (counters > plan->arrived_bytes || partials > plan->scratch_bytes) {
+  float* partials = static_cast<float*>(d_partials);
+  uint32_t* counters = static_cast<uint32_t*>(d_counters);
+  switch (tile_size) {
+    case 8:
+      return launch_planned<8>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, partials, counters, A, B, d_C,
+                               d_indptr, d_indices, st);
+    case 16:
+      return launch_planned<16>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, partials, counters, A, B, d_C,
+                                d_indptr, d_indices, st);
+    default:
+      return launch_planned<32>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, partials, counters, A, B, d_C,
+                                d_indptr, d_indices, st);
+  }
+}
+
+extern "C" int stir_tc_spmm_f16_planned(stir_tc_plan* plan, int32_t out_dtype, int32_t mb, int32_t tile_size,
+                                        int32_t group_size, int32_t feat, int64_t nnzb, const void* d_A,
+                                        const void* d_B, void* d_C, const int32_t* d_indptr,
+                                        const int32_t* d_indices, void* stream) {
+  STIR_REQUIRE(plan, "tc_spmm_planned: plan is null");
+  // memory of the plan is made only for a call that goes on to launch
+  if (check_args(out_dtype, mb, tile_size, group_size, feat, nnzb, d_A, d_B, d_C, d_indptr, d_indices)) return -1;
+  int device = 0;
+  STIR_HIP(hipGetDevice(&device));
+  const size_t counters = stir_tc_plan_counter_bytes(plan, feat), partials = stir_tc_plan_partial_bytes(plan, tile_size, feat);
+  if (plan->mb == mb && plan->device == device && mb > 0 &&
+      (counters > plan->arrived_bytes || partials > plan->scratch_bytes)) {
     const size_t more_counters = std::max(counters, plan->arrived_bytes);
     const size_t more_partials = std::max(partials, plan->scratch_bytes);
     if (plan->d_arrived) STIR_HIP(hipFree(plan->d_arrived));
     plan->d_arrived = nullptr;
     plan->arrived_bytes = plan->scratch_bytes = 0;
     STIR_HIP(hipMalloc(reinterpret_cast<void**>(&plan->d_arrived), more_counters + more_partials));
-    STIR_HIP(hipMemsetAsync(plan->d_arrived, 0, more_counters, st));
+    STIR_HIP(hipMemsetAsync(plan->d_arrived, 0, more_counters, static_cast<hipStream_t>(stream)));
     plan->arrived_bytes = more_counters, plan->scratch_bytes = more_partials;
   }
-  float* scratch = reinterpret_cast<float*>(reinterpret_cast<char*>(plan->d_arrived) + plan->arrived_bytes);
-  switch (tile_size) {
-    case 8:
-      return launch_planned<8>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A, B,
-                               d_C, d_indptr, d_indices, st);
-    case 16:
-      return launch_planned<16>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A,
-                                B, d_C, d_indptr, d_indices, st);
-    default:
-      return launch_planned<32>(out32, mb, feat, nnzb, plan->n_pieces, plan->d_pieces, scratch, plan->d_arrived, A,
-                                B, d_C, d_indptr, d_indices, st);
-  }
+  char* scratch = reinterpret_cast<char*>(plan->d_arrived);
+  return stir_tc_spmm_f16_workspace(plan, out_dtype, mb, tile_size, group_size, feat, nnzb, d_A, d_B, d_C, d_indptr, d_indices,
+                                    scratch, scratch ? scratch + plan->arrived_bytes : nullptr, stream);
 }

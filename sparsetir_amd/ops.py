@@ -207,8 +207,9 @@ class CsrMM(_Operator):
         with torch.cuda.device(dev):
             # the launcher has the workspace, and takes tensors of the device that is current
             rc = self._launch(args)
-            if rc != 1:
+            if rc == -1:
                 _lib.check(rc)
+            if rc != 1:
                 return
             _lib.check(self.L.stir_csr_spmm_f32(self.m, self.n, self.feat, self.nnz, _ptr(a),
                                                 _ptr(b), _ptr(c), _ptr(indptr), _ptr(indices),
@@ -420,7 +421,8 @@ class TcSpMM(_Operator):
     that are summed in fp32 and rounded once.  In-place changes of ``indptr`` made through torch
     are noticed (its version counter is part of the key); after rewriting it by other means (a
     kernel of the caller's, another library) call :meth:`invalidate` -- the reference's operator
-    reads the array on every call.  The first call
+    reads the array on every call.  The memory for the pieces is kept per stream, so calls on several
+    streams may overlap; a recorded call has its own.  The first call
     of a plan allocates and synchronises the stream, so it cannot be part of a captured graph;
     later calls can."""
     name = "tcspmm"
@@ -470,11 +472,17 @@ class TcSpMM(_Operator):
                 # the array stays alive with the plan: its address cannot be handed to another
                 # indptr array (same size, version 0) that the key would take for this one
                 self._plans.put(key, plan, indptr)
+            # the launcher has the memory for partial tiles, one piece per stream
+            self._host.remember(args, plan.value, key)
+            rc = self._launch(args)
+            if rc == -1:
+                _lib.check(rc)
+            if rc != 1:
+                return
             _lib.check(self.L.stir_tc_spmm_f16_planned(plan, _DT[self.out_dtype], self.mb, self.t, self.g,
                                                        self.feat, self.nnzb,
                                                        _ptr(a), _ptr(b), _ptr(c), _ptr(indptr), _ptr(indices),
                                                        _stream()))
-            self._host.remember(args, plan.value, key)
 
 
 class Rgms(_Operator):

@@ -513,7 +513,7 @@ def side_kernels(torch, dev, ops, st, datasets, time_steps):
     for k in range(len(buckets)):
         triples += [t(mask[k].astype(np.float32).ravel()), t(rows[k].ravel()), t(cols[k].ravel())]
         mids.append(t(np.repeat(np.arange(R, dtype=np.int32), np.diff(ptr[k]))))
-    # the operator's default: every 64-row tile of Y summed on chip from an edge index, no atomics
+    # the operator's default: every 128-row tile of Y summed on chip from an edge index, no atomics
     f32 = ops.build_rgms_f32(n, n, R, fin, fout, rb32, buckets, [c.shape[0] for c in cols])
     f32(w32, x32, y, *triples, *mids)  # builds its edge index
     tm = time_small(lambda: f32(w32, x32, y, *triples, *mids), 20, 2, torch)

@@ -467,11 +467,12 @@ int stir_rgms_f32(const stir_rgms_f32_plan* plan, int32_t m, int32_t n, int32_t 
  * Optional (no counterpart in the reference): sums that come out the same, bit for bit, on every
  * run, and faster.  From 8192 slots on, with feat_in and feat_out of at most 64, the first launch
  * of a plan switched to this mode builds an edge index from the three index arrays (sorted by
- * 64-row tile of Y, relation, row; it allocates and synchronises the stream, later launches only
+ * 128-row tile of Y, relation, row; it allocates and synchronises the stream, later launches only
  * rewrite a packed copy of W held by the plan; the index arrays must not change afterwards, the
  * weights may) and every tile of Y is summed on chip in a fixed order and written once, without
- * atomics: 134 us against 159 us on 100k nodes, 65 relations, 2M edges.  Inputs outside these
- * limits, or whose index would not fit its 64-bit sort keys, run the atomic kernels.
+ * atomics: 79 us against 156 us on 100k nodes, 65 relations, 2M edges.  The products with W are those
+ * of fp32 arithmetic over all of its range, infinities included; sums or weights from 2^104 on and
+ * products from 2^80 on cost a tile about six times its time.  Inputs outside these limits, or whose index would not fit its 64-bit sort keys, run the atomic kernels.
  * A plan in this mode serves one call at a time.
  */
 int stir_rgms_f32_plan_set_deterministic(stir_rgms_f32_plan* plan, int32_t on);
@@ -493,11 +494,11 @@ int stir_rgms_csf_f32(int32_t m, int32_t n, int32_t num_rels, int32_t feat_in, i
 
 /*
  * The same operator without atomics (no counterpart in the reference): sums that come out the
- * same, bit for bit, on every run, and faster than stir_rgms_csf_f32 (122 against 159 us on 100k
+ * same, bit for bit, on every run, and faster than stir_rgms_csf_f32 (75 against 159 us on 100k
  * nodes, 65 relations, 2M edges).  The plan keeps the pointers of the five arrays; from 8192 edges
  * on, with feat_in and feat_out of at most 64, its first launch builds the edge index described
  * at stir_rgms_f32_plan_set_deterministic from the four index arrays (they must not change
- * afterwards, the edge values may) and every 64-row tile of Y is written once.  Other inputs run
+ * afterwards, the edge values may) and every 128-row tile of Y is written once.  Other inputs run
  * stir_rgms_csf_f32.  A plan serves one call at a time.
  */
 typedef struct stir_rgms_csf_f32_plan stir_rgms_csf_f32_plan;

@@ -27,10 +27,11 @@
 // A batch is a chain of dependent loads (batch record -> edge records -> rows of X and weights), each step
 // of it requested one batch ahead of the next.
 //
-// Bound by the vector unit: 165 instructions per batch, busy 61 % of the kernel's clocks (100 k nodes, 65
-// relations, 2 M edges, 32 -> 32: 112 k batches, 67 us, 78 per call; 129 before, when each wavefront had a
-// partial tile of 64 rows to itself -- 146 k batches -- and three wavefronts per SIMD in the place of four
-// waited on v_mfma_f32_16x16x4_f32, during which the vector unit stands still).
+// Bound by the vector unit: 200 instructions per batch, what a unit costs besides included, busy 57 % of the
+// kernel's clocks, the matrix cores 13 % (100 k nodes, 65 relations, 2 M edges, 32 -> 32: 117 k batches, 68 us, 75
+// per call; 122 before, when each wavefront had a partial tile of 64 rows to itself -- 146 k batches -- and three
+// wavefronts per SIMD in the place of four waited on v_mfma_f32_16x16x4_f32, during which the vector unit stands
+// still).
 // At the end the partial tile is added to the tile's rows of Y, each element once,
 // or -- for a unit that is a piece of a tile -- goes to the plan's memory for partial tiles, with
 // device-coherent stores.  Such a unit then counts itself in (a counter per cut tile); the one

@@ -7,11 +7,12 @@
 // fp16 inputs, fp32 accumulation, fp16 or fp32 output.
 //
 // With a plan (stir_tc_plan: the long tiles listed once, longest first, in pieces) a product is one launch of
-// tcspmm_units_kernel.  Bound by the gather of rows of B where there are tiles enough (179 k rows, 4.5 M
-// nonzeros, 64 features: 5.8 TB/s), else by the chain id -> row of B -> product of the longest unit.  Before, the
-// tiles of up to 16 steps went as below and the pieces of the others in a second launch, a workgroup of 16
-// wavefronts each; us: 25.9 k rows, 626 k nonzeros, 32 features 23.4 -> 9.4; 167 k, 3.8 M, 32: 81 -> 46; 24 k,
-// 244 k, 64: 22.4 -> 12.5; 200 k, 4 M, 64: 92 -> 58; 33 k, 648 k, 224: 49 -> 41.5; 169 k, 1.17 M, 128: 50.8 -> 48.3.
+// tcspmm_units_kernel.  Bound by the gather of rows of B where there are tiles enough, else by the chain id -> row of B
+// -> product of the longest unit.  Before, the tiles of up to 16 steps went as below and the pieces of the others in a
+// second launch, a workgroup of 16 wavefronts each.  Tiles of 16 rows, power-law rows of up to 500 to 17.5 k nonzeros,
+// uniform columns, us: 25.9 k rows, 626 k nonzeros, 32 features 22.4 -> 10.8; 167 k, 3.8 M, 32: 83 -> 66; 24 k, 244 k,
+// 64: 22.2 -> 10.8; 200 k, 4 M, 64: 101 -> 90; 33 k, 648 k, 224: 61 -> 48; 169 k, 1.17 M, 128: 62.1 -> 62.7 over the
+// same arrays again and again, 70.3 -> 63.4 where other arrays are used in between (skewed columns 47 -> 49).
 //
 // Without a plan: a workgroup of four wavefronts owns (row tile, 128 features), a wavefront t rows x 32 features.
 // A step covers two groups (32 gathered rows of B): A[jo] is already in MFMA A-operand order (a lane's 8 k values

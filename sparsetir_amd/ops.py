@@ -595,8 +595,8 @@ class RgmsF32(Rgms):
     """fp32 RGMS on ELL3D buckets with W laid out [R, feat_out, feat_in]: the composable operator of
     examples/rgms/rgcn/bench_rgcn_composable.py:208-221, same argument order as :class:`Rgms`.
     From 8192 slots on (and for feature sizes up to 64) a plan builds, at its first call, an edge
-    index by 64-row tile of Y, and every tile is summed on chip in a fixed order and written once:
-    no atomics, the same bits on every run, and about a tenth faster than the form with atomics
+    index by 128-row tile of Y, and every tile is summed on chip in a fixed order and written once:
+    no atomics, the same bits on every run, and in half the time of the form with atomics
     (no counterpart in the reference, whose operator adds with atomics).  ``deterministic=False``
     keeps the atomic form at every size: nothing is derived from what the index arrays hold."""
     name = "rgms_f32"
@@ -614,9 +614,9 @@ class RgmsCsf(_Operator):
 
     By default the operator keeps plans, keyed by the addresses of the five graph arrays and torch's
     version counters of the four index arrays; from 8192 edges on (feature sizes up to 64) a plan
-    holds an edge index by 64-row tile of Y (built by the first call: it allocates and synchronises)
+    holds an edge index by 128-row tile of Y (built by the first call: it allocates and synchronises)
     and Y is accumulated into without atomics: sums that come out the same, bit for bit, on every
-    run, about a sixth faster than with atomics (no counterpart in the reference).
+    run, in half the time of the form with atomics (no counterpart in the reference).
     ``deterministic=False`` is the stateless form, like the reference's operator: every call reads
     the arrays and adds to Y with atomics.  The edge values ``A`` are read on every call either way."""
     name = "rgms_csf"

@@ -111,3 +111,25 @@ def test_a_row_over_thousands_of_workgroups(dev, feat, hub):
     torch.cuda.synchronize()
     assert torch.equal(*c)
     _check(c[0].cpu().numpy().reshape(m, feat), indptr, indices, vals, x, f"feat={feat} hub={hub}")
+
+
+def test_more_streams_than_workspaces(dev):
+    """An operator keeps workspaces for four streams: a fifth takes the place of the one used longest ago, whose
+    kernels may still be running."""
+    rng = np.random.default_rng(6)
+    m, n, feat = 20000, 5000, 64
+    deg, indptr, indices = _matrix(rng, m, n, [3000, 700, 129], 20)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(dev)
+    args = [t(rng.random(len(indices), dtype=np.float32)), t(rng.standard_normal(n * feat).astype(np.float32))]
+    tail = [t(indptr), t(indices)]
+    f = ops.build_csrmm(m, n, feat, len(indices))
+    want = torch.empty(m * feat, device=dev)
+    f(*args, want, *tail)
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    out = [torch.full((m * feat,), float("nan"), device=dev) for _ in range(60)]
+    torch.cuda.synchronize()
+    for k, c in enumerate(out):
+        with torch.cuda.stream(streams[(k * 5 + k // 7) % 6]):
+            f(*args, c, *tail)
+    torch.cuda.synchronize()
+    assert all(torch.equal(c, want) for c in out)

@@ -114,7 +114,9 @@ Scratch scratch_of(const Workspace& w) {
 }
 
 // The workspace of a call on `st`.  A call that is being captured gets one of its own, its counters cleared by
-// the graph itself: the graph may be replayed on any stream.  `held` keeps it until the call is recorded.
+// the graph itself: the graph may be replayed on any stream.  `held` keeps the memory until the call is recorded or
+// in its queue: while it has let go of the GIL another thread may take the workspace off the list, and what the
+// allocator gave out then would be used before the kernel that is yet to come.
 Scratch workspace(Launcher* l, const c10::hip::HIPStream& st, const Need& need, at::Tensor* held) {
   std::vector<Workspace>& all = *l->workspaces;
   if (c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None) {
@@ -131,6 +133,7 @@ Scratch workspace(Launcher* l, const c10::hip::HIPStream& st, const Need& need, 
     all[at] = new_workspace(st, {std::max(all[at].has.counters, need.counters), std::max(all[at].has.rest, need.rest)});
   }
   if (at > 0) std::rotate(all.begin(), all.begin() + at, all.begin() + at + 1);
+  *held = all.front().memory;
   return scratch_of(all.front());
 }
 

@@ -425,7 +425,7 @@ int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz,
                                 float* d_C, const int32_t* d_indptr, const int32_t* d_indices, void* d_workspace,
                                 void* stream) {
   STIR_REQUIRE(m >= 0 && n >= 0 && feat > 0 && nnz >= 0, "csr_spmm: bad sizes m=%d n=%d feat=%d", m, n, feat);
-  if (!balanced(m, n, feat, nnz))
+  if (m == 0 || !balanced(m, n, feat, nnz))
     return stir_csr_spmm_f32(m, n, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, stream);
   STIR_REQUIRE(d_B && d_C && d_indptr && d_workspace && (nnz == 0 || (d_A && d_indices)),
                "csr_spmm: null pointer argument");

@@ -77,3 +77,11 @@ def test_csr_workspace_needs_few_zeros():
         assert 0 < clear(m, n, feat, nnz) <= total(m, n, feat, nnz) / min(row, 64)
         assert clear(m, n, feat, nnz) % 16 == 0
     assert total(100, 100, 32, 500) == clear(100, 100, 32, 500) == 0  # none is needed
+
+
+def test_csr_product_without_rows_needs_nothing():
+    """No rows: nothing is written or read, whatever else the arguments say (arrays of no elements have no address)."""
+    lib = L.lib()
+    for nnz in (0, 10_000_000):
+        assert lib.stir_csr_spmm_f32(0, 100, 64, nnz, None, None, None, None, None, None) == 0
+        assert lib.stir_csr_spmm_f32_workspace(0, 100, 64, nnz, None, None, None, None, None, None, None) == 0

@@ -5,6 +5,8 @@ import numpy as np
 import pytest
 import torch
 
+import test_gpu_odd_widths
+import test_gpu_spmm
 from sparsetir_amd import _lib
 from test_gpu_spmm import _check
 
@@ -46,3 +48,51 @@ def test_both_sides_of_the_lines(dev, m, feat, nnz):
     got = _run(dev, m, n, feat, indptr, indices, vals, x)
     assert np.all(got[deg == 0] == 0.0)
     _check(got, indptr, indices, vals, x, f"m={m} feat={feat} nnz={nnz}")
+
+
+@pytest.mark.parametrize("feat", [3, 4, 16, 47, 64, 128, 200, 512, 600])
+@pytest.mark.parametrize("m", [1, 9, 1003, 20001])
+def test_one_launch(dev, feat, m):
+    """Every lane group width with a wavefront per row and (above 20000 rows) a lane group per row; hub rows that the
+    workgroup shares, several of them in one workgroup, at lengths around the limit of 128 and far above it."""
+    n = 3000
+    rng = np.random.default_rng(feat + m)
+    deg = rng.integers(0, 3, m) if m * feat < 2_000_000 else (rng.random(m) < 0.1).astype(np.int64)
+    for k, d in enumerate([129, 128, 0, 2049, 127, 256, 135, 1, 700]):
+        deg[m - 1 - k if k < m else 0] = d
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    assert indptr[-1] * feat < 20_000_000 and indptr[-1] < FEW
+    indices = np.concatenate([np.sort(rng.choice(n, d, replace=False)) for d in deg]).astype(np.int32)
+    vals = rng.random(len(indices), dtype=np.float32) - np.float32(0.4)
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    got = _run(dev, m, n, feat, indptr, indices, vals, x)
+    assert np.all(got[deg == 0] == 0.0)
+    _check(got, indptr, indices, vals, x, f"m={m} feat={feat}")
+
+
+# The operator takes the products of these tests through its workspace: here they go the way without one that they
+# were written for.
+@pytest.fixture
+def stateless(monkeypatch):
+    def run_csr(dev, indptr, indices, vals, x, feat):
+        return _run(dev, len(indptr) - 1, x.shape[0], feat, indptr, indices, vals, x)
+
+    monkeypatch.setattr(test_gpu_spmm, "_run_csr", run_csr)
+    monkeypatch.setattr(test_gpu_odd_widths, "_run_csr", run_csr)
+
+
+@pytest.mark.parametrize("feat", [32, 128, 512, 96])
+def test_hub_rows_in_pieces(dev, stateless, feat):
+    test_gpu_spmm.test_csr_spmm_hub_rows_are_split(dev, feat)
+
+
+@pytest.mark.parametrize("feat", [4, 8, 12, 32, 40, 64, 128])
+@pytest.mark.parametrize("split", [False, True])
+def test_lane_group_per_row(dev, stateless, feat, split):
+    test_gpu_spmm.test_csr_spmm_lane_group_per_row(dev, feat, split)
+
+
+@pytest.mark.parametrize("feat", test_gpu_odd_widths.WIDTHS)
+@pytest.mark.parametrize("hubs", [False, True])
+def test_odd_widths(dev, stateless, feat, hubs):
+    test_gpu_odd_widths.test_csr_odd_width(dev, feat, hubs)

@@ -680,7 +680,7 @@ def main():
     check = {"hyb_vs_csr_max_abs_diff": max_diff, "hyb_vs_csr_ok": hyb_vs_csr_ok}
     cpu = None
     if not args.no_cpu:
-        import oracle  # checker and cpu_baseline only
+        import oracle  # for the check of the result and cpu_baseline only
         r_hi = min(m, args.cpu_rows)
         sub_ptr = indptr[: r_hi + 1].copy()
         sub_idx = indices[: sub_ptr[-1]]

@@ -6,10 +6,9 @@
 // fed by v_mfma_f32_32x32x16_{f16,bf16}.  Both operands go through LDS: the MFMA B operand wants
 // 8 consecutive k for one feature per lane while X is feature-contiguous, and the A fragment is
 // shared by the four wavefronts (see bsr_tile).  Blocks of 16 k + 16 rows use bsr16_spmm_kernel, small
-// launches bsr_split_kernel.
+// launches bsr_split_kernel, large ones of 32-row blocks bsr_wave_kernel.
 #include <hip/hip_fp16.h>
 
-#include <numeric>
 #include <type_traits>
 
 #include "common.h"
@@ -43,10 +42,7 @@ __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
 template <bool BF16>
 __device__ __forceinline__ uint16_t to16(float v) {
   if constexpr (BF16) {
-    uint32_t u = __float_as_uint(v);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return uint16_t((u >> 16) | 0x40);  // quiet NaN
-    u += 0x7fffu + ((u >> 16) & 1u);                                          // nearest even
-    return uint16_t(u >> 16);
+    return __builtin_bit_cast(uint16_t, (__bf16)v);  // v_cvt_pk_bf16_f32: nearest even, NaN stays a (quiet) NaN
   } else {
     _Float16 h = (_Float16)v;
     return __builtin_bit_cast(uint16_t, h);
@@ -67,6 +63,118 @@ __device__ __forceinline__ bool decode_tile(int64_t L, int64_t slices, int f_til
   f_tile = (int)(t / slices);
   slice = t % slices;
   return (L >> 3) < per && t < total;
+}
+
+// The same when the slices are numbered by rank (row_of_rank): where XCDs share a feature tile, each takes ranks from
+// the whole range in proportion to its share, so that none has the long ones.  With n of them here and m at another
+// XCD, the k-th here comes after those there whose (2 k' + 1) / m is smaller than (2 k + 1) / n.
+__device__ __forceinline__ bool decode_ranked(int64_t L, int64_t slices, int f_tiles, int64_t& slice, int& f_tile) {
+  const int64_t total = slices * f_tiles, per = (total + 7) >> 3;
+  const int x = (int)(L & 7);
+  const int64_t t = x * per + (L >> 3);
+  if ((L >> 3) >= per || t >= total) return false;
+  f_tile = (int)(t / slices);
+  const int64_t lo = f_tile * slices, hi = lo + slices;
+  const int64_t first = max(x * per, lo), n = min((x + 1) * per, hi) - first, k = t - first;
+  slice = k;
+  for (int y = (int)(lo / per); y < 8 && y * per < hi; ++y) {
+    if (y == x) continue;
+    const int64_t m = min((y + 1) * per, hi) - max(y * per, lo);
+    slice += ((2 * k + 1) * m + n - (y > x)) / (2 * n);
+  }
+  return true;
+}
+
+// The block row of rank `rank` when the block rows are ordered by their number of blocks, longest first, equal ones
+// by number.  Workgroups of a launch that walk block rows of equal length side by side move through X together (block
+// columns ascend in a block row) and share a window of it in L2, one turn of resident workgroups after the other:
+// nothing synchronises them, the order only decides what L2 holds.  Every wavefront finds the row from indptr by
+// itself, the length of that rank by halving, then the place among the rows of that length.
+constexpr int kRankChunks = 16;
+constexpr int kRankRows = kRankChunks * kWave;  // block rows whose lengths a wavefront can hold
+__device__ __forceinline__ int row_of_rank(const int32_t* __restrict__ indptr, int rows, int rank) {
+  const int lane = threadIdx.x & 63;
+  int len[kRankChunks], most = 0, least = INT32_MAX;
+#pragma unroll
+  for (int q = 0; q < kRankChunks; ++q) {
+    const int i = q * kWave + lane;
+    len[q] = -1;
+    if (i < rows) {
+      len[q] = indptr[i + 1] - indptr[i];
+      most = max(most, len[q]), least = min(least, len[q]);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    most = max(most, __shfl_xor(most, off, kWave));
+    least = min(least, __shfl_xor(least, off, kWave));
+  }
+  auto reach = [&](int at_least) {  // rows of that length or longer
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < kRankChunks; ++q)
+      if (q * kWave < rows) n += __popcll(__ballot(len[q] >= at_least));
+    return n;
+  };
+  // the longest length that more than `rank` rows reach
+  int lo = __builtin_amdgcn_readfirstlane(least), hi = __builtin_amdgcn_readfirstlane(most) + 1;
+  while (hi - lo > 1) {
+    const int mid = lo + ((hi - lo) >> 1);
+    if (reach(mid) > rank) lo = mid; else hi = mid;
+  }
+  int left = rank - reach(lo + 1), row = 0;  // rows of that length before the one wanted
+#pragma unroll
+  for (int q = 0; q < kRankChunks; ++q) {
+    if (q * kWave >= rows) continue;
+    const uint64_t same = __ballot(len[q] == lo);
+    const int n = __popcll(same);
+    if (left >= 0 && left < n) {
+      const bool wanted = ((same >> lane) & 1) && __popcll(same & ((uint64_t(1) << lane) - 1)) == left;
+      row = q * kWave + __ffsll((unsigned long long)__ballot(wanted)) - 1;
+    }
+    left -= n;
+  }
+  return row;
+}
+
+// 32 rows of Y from row `row0`, features f0 .. f0 + 32 T, from a wavefront's accumulators: acc[t][v] is row (v%4) + 4h +
+// 8(v/4), column n of the t-th 32x32 tile.  16-bit results go through 2048 T bytes of LDS of the wavefront's own into
+// 16-byte stores (2-byte stores take eight times the instructions: 73 of 605 us at 16384 x 16384, 10 %, 4096
+// features), fp32 results as they are, a line per 32 lanes.
+template <bool BF16, int OUT, int T>
+__device__ __forceinline__ void store_rows(char* __restrict__ own, const f32x16 (&acc)[T], void* __restrict__ Y,
+                                           int64_t row0, int feat, int f0) {
+  const int lane = threadIdx.x & 63, n = lane & 31, h = lane >> 5;
+  if constexpr (OUT == 1) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (f0 + 32 * t >= feat) continue;
+      float* first = static_cast<float*>(Y) + (row0 + 4 * h) * feat + f0 + 32 * t + n;
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        __builtin_nontemporal_store(acc[t][v], first + (int64_t)((v & 3) + 8 * (v >> 2)) * feat);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        *reinterpret_cast<uint16_t*>(own + (((v & 3) + 4 * h + 8 * (v >> 2)) * 32 * T + 32 * t + n) * 2) =
+            to16<BF16>(acc[t][v]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    constexpr int UN = 4 * T;  // 16-byte units per row
+#pragma unroll
+    for (int q = 0; q < 2 * T; ++q) {
+      const int at = kWave * q + lane, row = at / UN, u = at % UN;
+      const u32x4 w = *reinterpret_cast<const u32x4*>(own + at * 16);
+      if (f0 + 8 * u < feat)
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row0 + row) * feat + f0 +
+                                                                8 * u));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
 }
 
 // One tile of the output: the 32*RS rows [bi0, bi0 + 32*RS) of stored block row i times the
@@ -209,29 +317,11 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
       }
     }
   }
-  // acc[rs][t][v] is row 32 rs + (v%4) + 4h + 8(v/4), column n of the t-th 32x32 tile.
-  // The row stride is made opaque here: when this function is inlined into a loop over tiles,
-  // the sixteen row offsets would otherwise be computed once before that loop and held in
-  // registers throughout it (60 registers, halving the resident workgroups).
-  int row_stride = feat;
-  asm volatile("" : "+s"(row_stride));
+  if constexpr (OUT == 0) __syncthreads();  // the stages are free
 #pragma unroll
-  for (int rs = 0; rs < RS; ++rs) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int fcol = f0 + (wave * NT + t) * 32;
-      if (fcol >= feat) continue;
-      const int64_t first = ((int64_t)i_out * blk + bi0 + 32 * rs + 4 * h) * row_stride + fcol + n;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t off = first + (int64_t)((v & 3) + 8 * (v >> 2)) * row_stride;
-        if constexpr (OUT == 1)
-          __builtin_nontemporal_store(acc[rs][t][v], static_cast<float*>(Y) + off);
-        else
-          __builtin_nontemporal_store(to16<BF16>(acc[rs][t][v]), static_cast<uint16_t*>(Y) + off);
-      }
-    }
-  }
+  for (int rs = 0; rs < RS; ++rs)
+    store_rows<BF16, OUT>(lds + wave * 2048 * NT, acc[rs], Y, (int64_t)i_out * blk + bi0 + 32 * rs, feat,
+                          f0 + wave * NT * 32);
 }
 
 // The other order, for tall blocks (by_rows): XCD x owns the block rows i = x, x + 8, ... and
@@ -252,6 +342,7 @@ __device__ __forceinline__ bool decode_tile_by_rows(int64_t L, int64_t block_row
 // One workgroup per tile, 1-D grid (see decode_tile).
 template <bool BF16, int OUT, int NT, int RS>
 __global__ __launch_bounds__(256) void bsr_spmm_kernel(int blk, int feat, int64_t slices, int f_tiles, int by_rows,
+                                                       int ranked,
                                                        const uint16_t* __restrict__ A,
                                                        const uint16_t* __restrict__ X, void* __restrict__ Y,
                                                        const int32_t* __restrict__ indptr,
@@ -264,159 +355,16 @@ __global__ __launch_bounds__(256) void bsr_spmm_kernel(int blk, int feat, int64_
   const int sub = blk / (32 * RS);  // slices of 32*RS rows per block row
   if (by_rows) {
     if (!decode_tile_by_rows(blockIdx.x, slices / sub, sub, f_tiles, slice, f_tile)) return;
-  } else if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
+  } else if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+                    : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
     return;
   }
-  const int i = (int)(slice / sub), bi0 = (int)(slice % sub) * (32 * RS);
+  int i = (int)(slice / sub);
+  const int bi0 = (int)(slice % sub) * (32 * RS);
+  if (ranked) i = row_of_rank(indptr, (int)(slices / sub), i);
   // doubly-compressed form: stored block row i is block row row_ids[i] of the output
   const int i_out = row_ids ? row_ids[i] : i;
   bsr_tile<BF16, OUT, NT, RS>(xs, blk, feat, i, i_out, bi0, f_tile * TF, A, X, Y, indptr, indices);
-}
-
-// ------------------------------------------------------------------ large launches, swept in step
-// When the X rows of one feature tile (nb*blk rows of 256*NT bytes) exceed a per-XCD L2 (4 MB),
-// workgroups that walk their block rows at unrelated times miss L2 on about half of their X
-// tiles.  Block columns are ascending inside a block row, so workgroups that start together on
-// block rows of equal length move through X together and share a narrow window of it.  This
-// kernel arranges that: exactly as many workgroups as are resident at once (gridDim.x = 8 * G,
-// workgroup b runs on XCD b % 8, the dispatch order of the hardware), each a loop over tiles; all
-// workgroups of an XCD work on the same feature tile, and in round r workgroup w of the XCD takes
-// the slice of rank r*G + w when slices are ordered by their number of blocks, longest first.  A
-// round's slices have (nearly) the same length, so no workgroup has to wait for another and the
-// workgroups still stay in step; nothing here synchronises workgroups, the order only decides
-// what L2 holds.  The ranking is computed by every workgroup from indptr before its first tile
-// (a stable counting sort in LDS: every workgroup gets the same permutation).
-constexpr int kSweepMaxSlices = 8192;  // permutation entries are 16 bits wide and live in LDS
-constexpr int kSweepBins = 1024;       // block rows with more blocks than this share the last bin
-constexpr int kSweepMaxItems = 128;    // tiles per workgroup and feature tile
-
-// Calls f(value, lanes holding it) once per distinct value among the lanes with valid = true.
-template <typename F>
-__device__ __forceinline__ void for_each_distinct(int value, bool valid, F f) {
-  uint64_t todo = __ballot(valid);
-  while (todo) {
-    const int src = __ffsll((long long)todo) - 1;
-    const int v = __shfl(value, src, kWave);
-    const uint64_t same = __ballot(valid && value == v);
-    f(v, same);
-    todo &= ~same;
-  }
-}
-
-// Fills items[0 .. count) with the slices this workgroup takes, one per round, for subset
-// `part` of `parts`: ranks (r*G + w)*parts + part.  lds: at least 4*kSweepBins + kSweepMaxSlices/2
-// words, free again when the call returns.
-__device__ __forceinline__ int sweep_my_slices(uint32_t* __restrict__ lds, uint16_t* __restrict__ items,
-                                               const int32_t* __restrict__ indptr, int slices, int sub,
-                                               int G, int w, int parts, int part) {
-  uint32_t* hist = lds;                                                       // [bin][wavefront]
-  uint16_t* perm = reinterpret_cast<uint16_t*>(lds + 4 * kSweepBins);         // [rank] -> slice
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  for (int b = tid; b < 4 * kSweepBins; b += 256) hist[b] = 0;
-  __syncthreads();
-  // wavefront `wave` ranks the contiguous quarter [s_begin, s_end) of the slices
-  const int quarter = ((slices + 3) / 4 + kWave - 1) / kWave * kWave;
-  const int s_begin = wave * quarter, s_end = min(slices, s_begin + quarter);
-  auto bin_of = [&](int s) {
-    const int i = s / sub;
-    const int len = indptr[i + 1] - indptr[i];
-    return kSweepBins - 1 - min(len, kSweepBins - 1);  // longest first
-  };
-  for (int s0 = s_begin; s0 < s_end; s0 += kWave) {
-    const int s = s0 + lane;
-    const bool valid = s < s_end;
-    const int bin = valid ? bin_of(s) : 0;
-    for_each_distinct(bin, valid, [&](int v, uint64_t same) {
-      if (lane == 0) hist[v * 4 + wave] += (uint32_t)__popcll(same);
-    });
-  }
-  __syncthreads();
-  // exclusive scan over hist in (bin, wavefront) order: 16 consecutive entries per thread, read
-  // twice rather than held in registers (the tile loop decides the kernel's register count)
-  {
-    uint32_t sum = 0;
-#pragma unroll 1
-    for (int q = 0; q < 16; ++q) sum += hist[tid * 16 + q];
-    uint32_t incl = sum;
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const uint32_t up = __shfl_up(incl, off, kWave);
-      if (lane >= off) incl += up;
-    }
-    __shared__ uint32_t wave_total[4];
-    if (lane == kWave - 1) wave_total[wave] = incl;
-    __syncthreads();
-    uint32_t base = incl - sum;
-    for (int q = 0; q < wave; ++q) base += wave_total[q];
-#pragma unroll 1
-    for (int q = 0; q < 16; ++q) {
-      const uint32_t v = hist[tid * 16 + q];
-      hist[tid * 16 + q] = base;
-      base += v;
-    }
-  }
-  __syncthreads();
-  // placement, in slice order inside every (bin, wavefront) run: stable
-  for (int s0 = s_begin; s0 < s_end; s0 += kWave) {
-    const int s = s0 + lane;
-    const bool valid = s < s_end;
-    const int bin = valid ? bin_of(s) : 0;
-    for_each_distinct(bin, valid, [&](int v, uint64_t same) {
-      const uint32_t first = hist[v * 4 + wave];
-      if (valid && bin == v) perm[first + __popcll(same & ((uint64_t(1) << lane) - 1))] = (uint16_t)s;
-      __builtin_amdgcn_wave_barrier();
-      if (lane == 0) hist[v * 4 + wave] = first + (uint32_t)__popcll(same);
-      __builtin_amdgcn_wave_barrier();
-    });
-  }
-  __syncthreads();
-  int count = 0;
-  for (int r = 0;; ++r) {
-    const int64_t rank = ((int64_t)r * G + w) * parts + part;
-    if (rank >= slices || r >= kSweepMaxItems) break;
-    if (tid == 0) items[r] = perm[rank];
-    ++count;
-  }
-  __syncthreads();
-  return count;
-}
-
-template <bool BF16, int OUT, int NT, int RS>
-__global__ __launch_bounds__(256) void bsr_spmm_sweep_kernel(int blk, int feat, int slices, int f_tiles, int parts,
-                                                             const uint16_t* __restrict__ A,
-                                                             const uint16_t* __restrict__ X, void* __restrict__ Y,
-                                                             const int32_t* __restrict__ indptr,
-                                                             const int32_t* __restrict__ indices,
-                                                             const int32_t* __restrict__ row_ids) {
-  constexpr int TF = kTileF * NT;
-  constexpr int kXsWords = 2 * (kTileK * TF * 2 + 2048 * RS) / 4;
-  constexpr int kSortWords = 4 * kSweepBins + kSweepMaxSlices / 2;
-  __shared__ __attribute__((aligned(16))) uint32_t lds[kXsWords > kSortWords ? kXsWords : kSortWords];
-  __shared__ uint16_t items[kSweepMaxItems];
-  const int xcd = blockIdx.x & 7, w = blockIdx.x >> 3, G = gridDim.x >> 3;
-  const int sub = blk / (32 * RS);
-  // unit u = f_tile + f_tiles * part (part: every parts-th slice by rank); XCD x takes units x, x + 8, ...
-  const int units = f_tiles * parts;
-  int part_of_items = -1, count = 0;
-#pragma unroll 1
-  for (int u = xcd; u < units; u += 8) {
-    const int f_tile = u % f_tiles, part = u / f_tiles;
-    if (part != part_of_items) {
-      __syncthreads();  // the last tile's LDS reads are over
-      count = sweep_my_slices(lds, items, indptr, slices, sub, G, w, parts, part);
-      part_of_items = part;
-    }
-#pragma unroll 1
-    for (int r = 0; r < count; ++r) {
-      const int slice = items[r];
-      const int i = slice / sub, bi0 = (slice % sub) * (32 * RS);
-      const int i_out = row_ids ? row_ids[i] : i;
-      __syncthreads();  // the previous tile's readers are done with both LDS buffers
-      bsr_tile<BF16, OUT, NT, RS>(reinterpret_cast<char*>(lds), blk, feat, i, i_out, bi0, f_tile * TF, A, X, Y,
-                                  indptr, indices);
-    }
-  }
 }
 
 // ------------------------------------------------------------------ blocks of 16 k+16 rows
@@ -557,6 +505,117 @@ __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int6
         static_cast<uint16_t*>(Y)[off] = to16<BF16>(acc[t][v]);
     }
   }
+}
+
+// ------------------------------------------------------------------ large launches: a wavefront per tile
+// A wavefront owns 32 rows of a block row and 256 features: eight 32x32 accumulators.  Its X tile has 16 KB of LDS of
+// its own (image as in bsr_tile), filled from registers that were loaded a step before, so that 8 wavefronts per CU
+// have 144 KB on their way and none waits for another; the A operand is loaded straight into registers.  The first
+// half of a step's operands is read before its first MFMA, the second half as the first is used.
+// With the ranked order (row_of_rank) the wavefronts of an XCD stay within reach of each other in X: 16384 x 16384,
+// 10 % blocks of 32, 4096 features 595 us with workgroups of four wavefronts, 590 with this kernel in plain order
+// (3.97 GB through the L2s, 31 M misses), 377 with both; 300 x 450 blocks, 3232 features 290 -> 217 us; 1024 x 512,
+// 5 % 706 -> 454.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
+constexpr int kWaveF = 256;
+
+// `bytes` from an address that is the same for all lanes; a lane that asks for what lies beyond gets zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t window(const uint16_t* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
+}
+
+template <bool BF16, int OUT>
+__global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
+                                                            const uint16_t* __restrict__ A,
+                                                            const uint16_t* __restrict__ X, void* __restrict__ Y,
+                                                            const int32_t* __restrict__ indptr,
+                                                            const int32_t* __restrict__ indices,
+                                                            const int32_t* __restrict__ row_ids) {
+  constexpr int FT = kWaveF / 32;  // accumulators
+  constexpr int FCN = kWaveF / 8;  // 16-byte units per row of X
+  constexpr int XQ = 16;           // units per lane and step, two rows of X per load
+  __shared__ __attribute__((aligned(16))) char stage[kTileK * kWaveF * 2];
+  int64_t slice;
+  int f_tile;
+  if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+             : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
+    return;
+  const int lane = threadIdx.x, n = lane & 31, h = lane >> 5;
+  const int sub = blk / 32;
+  int i = (int)(slice / sub);
+  const int bi0 = (int)(slice % sub) * 32;
+  if (ranked) i = row_of_rank(indptr, (int)(slices / sub), i);
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = f_tile * kWaveF;
+  // staging: unit c of the rows 2 q + kq.  Units beyond feat repeat the last one: features nobody stores.
+  const int c = lane % FCN, kq = lane / FCN;
+  const uint32_t xoff = (uint32_t)(kq * feat + min(8 * c, feat - f0 - 8)) * 2;
+  uint32_t xdst[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) xdst[q] = (uint32_t)(((2 * q + kq) * FCN + (c ^ (4 * (2 * q + kq)))) * 16);
+  const uint32_t aoff = (uint32_t)((bi0 + n) * blk + 8 * h) * 2;
+  // operand reads: tile t is 256 bytes behind tile t - 4
+  const int sl = lane & 15, kr = sl >> 2, half16 = (lane >> 4) & 1;
+  uint32_t bread[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int u = 4 * t + 2 * half16 + ((sl & 3) >> 1);
+    bread[t] = (uint32_t)(((2 * h) * 4 * FCN + kr * FCN + (u ^ (4 * kr))) * 16 + (sl & 1) * 8);
+  }
+  auto operand = [&](int m, int t) {
+    return read_b(stage + bread[t % 4] + (t / 4) * 256 + m * 4 * FCN * 64, FCN * 64);
+  };
+
+  f32x16 acc[FT];
+#pragma unroll
+  for (int t = 0; t < FT; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
+
+  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
+  const int steps = nblk * (blk / kTileK);
+  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;  // block columns of 64 blocks
+  int pb = 0, k0 = 0;
+  u32x4 xr[XQ], ar[2];
+  auto fetch = [&]() {  // the next step's; nothing beyond the last
+    const int j = __builtin_amdgcn_readlane(j_lane, pb & 63);
+    const bool live = pb < nblk;
+    const auto ra = window(A + (int64_t)(p_begin + pb) * blk * blk + k0, live ? (uint32_t)(blk * blk - k0) * 2 : 0);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + 32 * m, 0, 0);
+    const auto rx = window(X + ((int64_t)j * blk + k0) * feat + f0, live ? 64u * feat : 0);
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) xr[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * 4 * feat, 0);
+    k0 += kTileK;
+    if (k0 == blk) {
+      k0 = 0, ++pb;
+      if ((pb & 63) == 0 && pb < nblk) j_lane = pb + lane < nblk ? indices[p_begin + pb + lane] : 0;
+    }
+  };
+  if (steps > 0) fetch();
+#pragma unroll 1
+  for (int it = 0; it < steps; ++it) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + xdst[q & 1] + (q / 2) * 4 * FCN * 16) = xr[q];
+    const u32x4 a0 = ar[0], a1 = ar[1];
+    fetch();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    u32x4 b[FT];
+#pragma unroll
+    for (int t = 0; t < FT; ++t) b[t] = operand(0, t);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < FT; ++t) {
+      acc[t] = mfma32<BF16>(a0, b[t], acc[t]);
+      b[t] = operand(1, t);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int t = 0; t < FT; ++t) acc[t] = mfma32<BF16>(a1, b[t], acc[t]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+  }
+  store_rows<BF16, OUT>(stage, acc, Y, (int64_t)i_out * blk + bi0, feat, f0);
 }
 
 // ------------------------------------------------------------------ small launches
@@ -792,35 +851,32 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int nt = (feat >= 1024) ? 2 : 1;
   const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
   dim3 block(256);
-  // Launches whose X rows per feature tile do not fit a per-XCD L2 and that give every resident
-  // workgroup several tiles are swept in step (bsr_spmm_sweep_kernel).
-  const int64_t x_tile_bytes = (int64_t)nb * blk * kTileF * nt * 2;
-  const int parts = 8 / std::gcd(f_tiles, 8);
-#define STIR_BSR_SWEEP(BF, OUT, NTV, RSV)                                                                     \
-  {                                                                                                           \
-    static int occupancy = 0; /* workgroups of this kernel per CU; the same on every gfx950 device */        \
-    if (occupancy == 0) {                                                                                     \
-      int o = 0;                                                                                              \
-      STIR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, bsr_spmm_sweep_kernel<BF, OUT, NTV, RSV>, 256, 0)); \
-      occupancy = o > 0 ? o : 1;                                                                              \
-    }                                                                                                         \
-    const int G = occupancy * (cus / 8);                                                                      \
-    const int64_t rounds = stir::ceil_div(stir::ceil_div(slices, parts), G);                                  \
-    if (rounds <= kSweepMaxItems && slices * f_tiles >= 4 * 8 * (int64_t)G) {                                 \
-      hipLaunchKernelGGL((bsr_spmm_sweep_kernel<BF, OUT, NTV, RSV>), dim3(8 * G), block, 0, st, blk, feat,    \
-                         (int)slices, f_tiles, parts, A, X, d_Y, d_indptr, d_indices, d_row_ids);             \
-      STIR_LAUNCH_CHECK();                                                                                    \
-      return 0;                                                                                               \
-    }                                                                                                         \
+  // Where the X rows of a feature tile are more than an XCD's L2 holds beside A (x_tile_bytes), the slices are taken in
+  // order of their length (row_of_rank), and those of 32 rows by one wavefront each once there are enough of them:
+  // 219 x 201 blocks, 1504 features (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 456 x 309, 352 features (912, of which
+  // half have 96 features) 66.4 -> 69.4.  Below 3 MB finding the row (2-3 us a tile) is lost: 359 x 71, 3488 features
+  // 69 -> 83 us ranked, 430 x 120, 1120 features 62 -> 67.
+  auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
+  constexpr int64_t kMuchX = 3 << 20;
+  const int rankable = mb <= kRankRows ? 1 : 0;
+  const int wf_tiles = (int)stir::ceil_div(feat, kWaveF);
+  if (rs == 1 && x_tile_bytes(kWaveF) > kMuchX && slices * wf_tiles >= 4 * cus && feat < (1 << 25) && blk <= 4096) {
+    const int64_t blocks = grid_of(slices, wf_tiles);
+    STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
+#define STIR_BSR_W(BF, OUT)                                                                                       \
+  hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices,     \
+                     wf_tiles, rankable, A, X, d_Y, d_indptr, d_indices, d_row_ids)
+    STIR_BSR_TYPES(STIR_BSR_W)
+#undef STIR_BSR_W
+    STIR_LAUNCH_CHECK();
+    return 0;
   }
-  // (measured: 16384^2, 32x32 blocks, 10 %, 4096 features 650 -> 590 us, L2 hit rate 46 -> 57 %;
-  // with fewer than 8 feature tiles or two slices per workgroup the plain order is faster)
-  const bool sweep = cus >= 8 && cus % 8 == 0 && rs == 1 && f_tiles >= 8 && x_tile_bytes > (3 << 20) &&
-                     slices <= kSweepMaxSlices;
+  // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
+  const int ranked = x_tile_bytes(kTileF * nt) > kMuchX ? rankable : 0;
   // Blocks of 128 rows and more: block rows dealt to XCDs (decode_tile_by_rows).  Measured at
   // 16384^2, 10 %, 4096 features: 128 x 128 blocks 387 -> 365 us; 64 x 64 blocks (one slice per
-  // block row, so only A is shared) 443 -> 514 us and 32 x 32 blocks 600 -> 950 us: there the
-  // feature tile per XCD, which keeps an XCD on one slice of X, is worth more.
+  // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an
+  // XCD on one slice of X, is worth more.
   const int sub_rows = blk / (32 * rs);
   const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2) ? 1 : 0;
   const int64_t blocks = by_rows ? 8 * stir::ceil_div((int64_t)mb, 8) * sub_rows * f_tiles
@@ -828,24 +884,20 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   dim3 grid((unsigned)blocks);
 #define STIR_BSR_L(BF, OUT, NTV, RSV)                                                                      \
-  {                                                                                                        \
-    if (sweep && !by_rows) STIR_BSR_SWEEP(BF, OUT, NTV, RSV);                                              \
-    hipLaunchKernelGGL((bsr_spmm_kernel<BF, OUT, NTV, RSV>), grid, block, 0, st, blk, feat, slices, f_tiles, \
-                       by_rows, A, X, d_Y, d_indptr, d_indices, d_row_ids);                                \
-  }
+  hipLaunchKernelGGL((bsr_spmm_kernel<BF, OUT, NTV, RSV>), grid, block, 0, st, blk, feat, slices, f_tiles, \
+                     by_rows, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
 #define STIR_BSR(BF, OUT)                                                          \
   do {                                                                             \
     if (nt == 2) {                                                                 \
-      if (rs == 2) STIR_BSR_L(BF, OUT, 2, 2) else STIR_BSR_L(BF, OUT, 2, 1)        \
+      if (rs == 2) STIR_BSR_L(BF, OUT, 2, 2); else STIR_BSR_L(BF, OUT, 2, 1);      \
     } else {                                                                       \
-      if (rs == 2) STIR_BSR_L(BF, OUT, 1, 2) else STIR_BSR_L(BF, OUT, 1, 1)        \
+      if (rs == 2) STIR_BSR_L(BF, OUT, 1, 2); else STIR_BSR_L(BF, OUT, 1, 1);      \
     }                                                                              \
   } while (0)
   STIR_BSR_TYPES(STIR_BSR)
 #undef STIR_BSR_TYPES
 #undef STIR_BSR
 #undef STIR_BSR_L
-#undef STIR_BSR_SWEEP
   STIR_LAUNCH_CHECK();
   return 0;
 }

@@ -1,0 +1,56 @@
+"""BSR SpMM where X does not fit an L2: slices taken in order of their length, 32-row slices by a wavefront each.
+Empty block rows, a few with more blocks than a wavefront has lanes, block columns in any order, ragged feature
+tiles, arrays that start at an odd element.  Checked against the fp64 oracle as in test_gpu_bsr.py."""
+import numpy as np
+import pytest
+import torch
+
+from sparsetir_amd import datasets, ops
+from test_gpu_bsr import _check
+
+pytestmark = pytest.mark.gpu
+
+
+def _config(mb, nb, blk, density, feat, seed):
+    """config4 with two long block rows and the columns of every row shuffled."""
+    cfg = datasets.config4(seed=seed, mb=mb, nb=nb, blk=blk, density=density, feat=feat)
+    rng = np.random.default_rng(seed)
+    rows = [rng.permutation(cfg["indices"][cfg["indptr"][i]:cfg["indptr"][i + 1]]) for i in range(mb)]
+    for i in (1, mb - 2):
+        rows[i] = rng.permutation(nb)[:max(nb // 2, 1)].astype(np.int32)
+    cfg["indptr"] = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cfg["indices"] = np.concatenate(rows).astype(np.int32)
+    cfg["data"] = rng.standard_normal((len(cfg["indices"]), blk, blk)).astype(np.float32) * 0.1
+    return cfg
+
+
+@pytest.mark.parametrize("mb,nb,blk,density,feat", [
+    (1024, 193, 32, 0.004, 224),   # as many block rows as are ranked
+    (1030, 200, 32, 0.004, 256),   # more: plain order
+    (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles
+    (343, 200, 32, 0.01, 736),
+    (20, 200, 64, 0.03, 96),       # four wavefronts per 64 rows
+    (12, 100, 128, 0.05, 160),     # block rows dealt to XCDs
+    (1, 6200, 32, 0.001, 64),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("start", [0, 1])
+def test_bsr_ranked_edges(dev, mb, nb, blk, density, feat, dtype, start):
+    cfg = _config(mb, nb, blk, density, feat, seed=mb + feat) if mb > 2 else datasets.config4(
+        seed=1, mb=mb, nb=nb, blk=blk, density=density, feat=feat)
+    out = torch.float32 if start and dtype is torch.float16 else dtype
+
+    def place(values, dt):
+        t = torch.empty(values.size + start, dtype=dt, device=dev)[start:]
+        t.copy_(torch.from_numpy(values.reshape(-1)))
+        return t
+
+    a, x = place(cfg["data"], dtype), place(cfg["x"], dtype)
+    y = torch.full((mb * blk * feat + start,), float("nan"), dtype=out, device=dev)[start:]
+    f = ops.build_bsrmm(mb, nb, len(cfg["indices"]), blk, feat, dtype, out)
+    f(a, x, y, torch.from_numpy(cfg["indptr"]).to(dev), torch.from_numpy(cfg["indices"]).to(dev))
+    torch.cuda.synchronize()
+    a32 = a.float().cpu().numpy().reshape(-1, blk, blk)
+    x32 = x.float().cpu().numpy().reshape(nb * blk, feat)
+    _check(y.float().cpu().numpy().reshape(mb * blk, feat), cfg, a32, x32, out is not torch.float32,
+           f"{mb}x{nb} blk {blk} feat {feat} {dtype} start {start}")

@@ -137,6 +137,20 @@ __device__ __forceinline__ int row_of_rank(const int32_t* __restrict__ indptr, i
   return row;
 }
 
+// 8 consecutive k of one feature per lane, from a feature-contiguous image: two transposing reads `next`
+// bytes (four rows of k) apart
+__device__ __forceinline__ u32x4 read_b(const char* at, int next) {
+  const tr16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at));
+  const tr16x4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at + next));
+  const u32x2 lo = __builtin_bit_cast(u32x2, t0), hi = __builtin_bit_cast(u32x2, t1);
+  return u32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
+// `bytes` from an address that is the same for all lanes; a lane that asks for what lies beyond gets zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t window(const uint16_t* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
+}
+
 // 32 rows of Y from row `row0`, features f0 .. f0 + 32 T, from a wavefront's accumulators: acc[t][v] is row (v%4) + 4h +
 // 8(v/4), column n of the t-th 32x32 tile.  16-bit results go through 2048 T bytes of LDS of the wavefront's own into
 // 16-byte stores (2-byte stores take eight times the instructions: 73 of 605 us at 16384 x 16384, 10 %, 4096
@@ -213,26 +227,22 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, h = lane >> 5;
 
-  // staging role: 2*NT chunks of X per thread
+  // staging role: 2*NT chunks of X per thread, of the eight rows from 8 * wave on; a chunk beyond feat reads as zero
   uint32_t xoff[2 * NT], xdst[2 * NT];
 #pragma unroll
   for (int q = 0; q < 2 * NT; ++q) {
-    const int idx = 64 * (wave * 2 * NT + q) + lane, c = idx % FCN, k = idx / FCN;
-    xoff[q] = (uint32_t)(k * feat + 8 * c);  // in elements, from the tile's first element
+    const int idx = 64 * q + lane, c = idx % FCN, kw = idx / FCN, k = 8 * wave + kw;
+    xoff[q] = f0 + 8 * c < feat ? (uint32_t)(kw * feat + 8 * c) * 2 : ~15u;  // bytes from the wavefront's first
     xdst[q] = (uint32_t)(((k >> 2) * 4 * FCN + (k & 3) * FCN + (c ^ (4 * (k & 3)))) * 16);
   }
-  // a lane's chunks all lie in the same feature column (FCN divides 64): one test for all of
-  // them; feat is a multiple of 32, so chunks are whole.  A lane beyond feat never loads and
-  // keeps staging the zeros its registers start with.
-  static_assert(64 % FCN == 0, "a lane's chunks share their feature column");
-  const bool xlive = f0 + 8 * (lane % FCN) < feat;
+  const uint16_t* Xw = X + (int64_t)(8 * wave) * feat + f0;
   // ... and 8*RS bytes of the block: RS = 1: half of the unit (chunk tid/64, row (tid/2)%32);
   // RS = 2: the unit (slice tid/128, chunk (tid/32)%4, row tid%32)
   uint32_t aoff;
   if constexpr (RS == 1)
-    aoff = (uint32_t)(((tid >> 1) & 31) * blk + (tid >> 6) * 8 + (tid & 1) * 4);
+    aoff = (uint32_t)(((tid >> 1) & 31) * blk + (tid >> 6) * 8 + (tid & 1) * 4) * 2;
   else
-    aoff = (uint32_t)((32 * (tid >> 7) + (tid & 31)) * blk + ((tid >> 5) & 3) * 8);
+    aoff = (uint32_t)((32 * (tid >> 7) + (tid & 31)) * blk + ((tid >> 5) & 3) * 8) * 2;
   // operand reads, bytes inside a stage
   const int sl = lane & 15, half16 = (lane >> 4) & 1;
   uint32_t bread[NT];
@@ -255,39 +265,39 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
   const int nblk = indptr[i + 1] - p_begin;
   const int steps = nblk * (blk / kTileK);
 
-  // The step to fetch next: block pb of the row, k offset k0.  The block column of the block after
-  // the current one is requested a whole block ahead, so that no step waits for an index before
-  // it can ask for its rows of X.
+  // The step to fetch next: block pb of the row, k offset k0; nothing beyond the last, so that no load depends on a
+  // branch.  The block columns of the 64 blocks in hand and of the next 64 are in registers, one per lane: asked for
+  // one by one, each block waited for a scalar load (128 x 128 blocks of 32, 512 features 11.7 -> 11.3 us; 60 x 60 of
+  // 64, 512 features 13.0 -> 11.9; 430 x 120 of 32, 1120 features 62.5 -> 59.3).  Two to four steps in registers at a
+  // time gain on the first two (11.0 and 10.7 with four) and lose 3 to 15 % on larger ones.
   int pb = 0, k0 = 0;
-  int j_cur = nblk > 0 ? indices[p_begin] : 0;
-  int j_nxt = nblk > 1 ? indices[p_begin + 1] : 0;
-  u32x4 xr[2 * NT];
-#pragma unroll
-  for (int q = 0; q < 2 * NT; ++q) xr[q] = u32x4{0, 0, 0, 0};
-  u32x4 ar;  // RS = 1 uses the first two words
+  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
+  int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
+  u32x4 xr[2 * NT], ar;  // RS = 1 uses the first two words of ar
   auto fetch = [&]() {
-    const uint16_t* xb = X + ((int64_t)j_cur * blk + k0) * feat + f0;
-    const uint16_t* ab = A + (int64_t)(p_begin + pb) * blk * blk + (int64_t)bi0 * blk + k0;
-    if (xlive) {
+    const bool live = pb < nblk;
+    const int j = __builtin_amdgcn_readlane(j_lane, pb & (kWave - 1));
+    const auto rx = window(Xw + ((int64_t)j * blk + k0) * feat, live ? 16u * feat : 0);
+    const auto ra =
+        window(A + (int64_t)(p_begin + pb) * blk * blk + (int64_t)bi0 * blk + k0, live ? 64u * RS * blk : 0);
 #pragma unroll
-      for (int q = 0; q < 2 * NT; ++q) xr[q] = *reinterpret_cast<const u32x4*>(xb + xoff[q]);
-    }
+    for (int q = 0; q < 2 * NT; ++q) xr[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[q], 0, 0);
     if constexpr (RS == 1) {
-      const u32x2 v = *reinterpret_cast<const u32x2*>(ab + aoff);
+      const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(ra, aoff, 0, 0);
       ar[0] = v[0], ar[1] = v[1];
     } else {
-      ar = *reinterpret_cast<const u32x4*>(ab + aoff);
+      ar = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff, 0, 0);
     }
     k0 += kTileK;
     if (k0 == blk) {
-      k0 = 0;
-      ++pb;
-      j_cur = j_nxt;
-      if (pb + 1 < nblk) j_nxt = indices[p_begin + pb + 1];
+      k0 = 0, ++pb;
+      if ((pb & (kWave - 1)) == 0) {
+        j_lane = j_more;
+        j_more = pb + kWave + lane < nblk ? indices[p_begin + pb + kWave + lane] : 0;
+      }
     }
   };
-
-  if (steps > 0) fetch();
+  fetch();
   for (int it = 0; it < steps; ++it) {
     char* stage = lds + (it & 1) * SB;
 #pragma unroll
@@ -296,7 +306,7 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
       *reinterpret_cast<u32x2*>(stage + XB + tid * 8) = u32x2{ar[0], ar[1]};
     else
       *reinterpret_cast<u32x4*>(stage + XB + tid * 16) = ar;
-    if (it + 1 < steps) fetch();
+    fetch();
     __syncthreads();  // stage `it` is complete; the other stage's readers passed the previous barrier
     u32x4 a[RS][2];
 #pragma unroll
@@ -307,11 +317,7 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const char* bp = stage + bread[t] + (4 * m) * FCN * 64;
-        const tr16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(bp));
-        const tr16x4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(bp + FCN * 64));
-        const u32x2 lo = __builtin_bit_cast(u32x2, t0), hi = __builtin_bit_cast(u32x2, t1);
-        const u32x4 b = {lo[0], lo[1], hi[0], hi[1]};
+        const u32x4 b = read_b(stage + bread[t] + (4 * m) * FCN * 64, FCN * 64);
 #pragma unroll
         for (int rs = 0; rs < RS; ++rs) acc[rs][t] = mfma32<BF16>(a[rs][m], b, acc[rs][t]);
       }
@@ -359,9 +365,11 @@ __global__ __launch_bounds__(256) void bsr_spmm_kernel(int blk, int feat, int64_
                     : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
     return;
   }
-  int i = (int)(slice / sub);
-  const int bi0 = (int)(slice % sub) * (32 * RS);
-  if (ranked) i = row_of_rank(indptr, (int)(slices / sub), i);
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  int i = (int)slice / sub;
+  const int bi0 = ((int)slice % sub) * (32 * RS);
+  if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
   // doubly-compressed form: stored block row i is block row row_ids[i] of the output
   const int i_out = row_ids ? row_ids[i] : i;
   bsr_tile<BF16, OUT, NT, RS>(xs, blk, feat, i, i_out, bi0, f_tile * TF, A, X, Y, indptr, indices);
@@ -381,15 +389,6 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
   else
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0,
                                                   0, 0);
-}
-
-// 8 consecutive k of one feature per lane, from a feature-contiguous image: two transposing reads `next`
-// bytes (four rows of k) apart
-__device__ __forceinline__ u32x4 read_b(const char* at, int next) {
-  const tr16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at));
-  const tr16x4 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16((STIR_LDS tr16x4*)(at + next));
-  const u32x2 lo = __builtin_bit_cast(u32x2, t0), hi = __builtin_bit_cast(u32x2, t1);
-  return u32x4{lo[0], lo[1], hi[0], hi[1]};
 }
 
 // A chunk of 16 columns: number `number` of a block row's chunks, columns 16 * col of block `block`
@@ -518,11 +517,6 @@ __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int6
 // 5 % 706 -> 454.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
 constexpr int kWaveF = 256;
 
-// `bytes` from an address that is the same for all lanes; a lane that asks for what lies beyond gets zeros
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t window(const uint16_t* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(base), 0, bytes, 0x00020000);
-}
-
 template <bool BF16, int OUT>
 __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
                                                             const uint16_t* __restrict__ A,
@@ -541,9 +535,11 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
     return;
   const int lane = threadIdx.x, n = lane & 31, h = lane >> 5;
   const int sub = blk / 32;
-  int i = (int)(slice / sub);
-  const int bi0 = (int)(slice % sub) * 32;
-  if (ranked) i = row_of_rank(indptr, (int)(slices / sub), i);
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  int i = (int)slice / sub;
+  const int bi0 = ((int)slice % sub) * 32;
+  if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
   const int i_out = row_ids ? row_ids[i] : i;
   const int f0 = f_tile * kWaveF;
   // staging: unit c of the rows 2 q + kq.  Units beyond feat repeat the last one: features nobody stores.
@@ -573,12 +569,13 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
 
   const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
   const int steps = nblk * (blk / kTileK);
-  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;  // block columns of 64 blocks
   int pb = 0, k0 = 0;
+  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;  // block columns of 128 blocks (see bsr_tile)
+  int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
   u32x4 xr[XQ], ar[2];
   auto fetch = [&]() {  // the next step's; nothing beyond the last
-    const int j = __builtin_amdgcn_readlane(j_lane, pb & 63);
     const bool live = pb < nblk;
+    const int j = __builtin_amdgcn_readlane(j_lane, pb & (kWave - 1));
     const auto ra = window(A + (int64_t)(p_begin + pb) * blk * blk + k0, live ? (uint32_t)(blk * blk - k0) * 2 : 0);
 #pragma unroll
     for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + 32 * m, 0, 0);
@@ -588,7 +585,10 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
     k0 += kTileK;
     if (k0 == blk) {
       k0 = 0, ++pb;
-      if ((pb & 63) == 0 && pb < nblk) j_lane = pb + lane < nblk ? indices[p_begin + pb + lane] : 0;
+      if ((pb & (kWave - 1)) == 0) {
+        j_lane = j_more;
+        j_more = pb + kWave + lane < nblk ? indices[p_begin + pb + kWave + lane] : 0;
+      }
     }
   };
   if (steps > 0) fetch();

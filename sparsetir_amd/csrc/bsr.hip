@@ -28,6 +28,7 @@ typedef __fp16 tr16x4 __attribute__((__vector_size__(4 * sizeof(__fp16))));  // 
 
 constexpr int kTileF = 128;  // features per workgroup
 constexpr int kTileK = 32;   // k rows staged per step
+constexpr int kWaveF = 256;  // features per wavefront where a wavefront owns a tile
 
 template <bool BF16>
 __device__ __forceinline__ f32x16 mfma32(u32x4 a, u32x4 b, f32x16 c) {
@@ -400,15 +401,12 @@ struct Chunk {
   }
 };
 
-// A workgroup of four wavefronts owns (block row, 16-row slice, 128 * NT features), a wavefront 16 rows x
+// Few slices: a workgroup of four wavefronts owns (block row, 16-row slice, 128 * NT features), a wavefront 16 rows x
 // 32 * NT features.  Per step the 32 rows of X of two chunks go through LDS as in bsr_tile (two stages, one
 // barrier per step, the next step's loads in flight), the image's XOR extended by 2 * (k / 8 % 2): the two
 // blocks of 16 lanes that a transposing read serves together ask for the same units of k groups eight rows
 // apart here.  The A operand is one 16-byte load per lane from the block.
-// Bound by the rows of X that come out of L2: a 16-row slice uses each of them for 16 rows only (318 x 284
-// blocks of 16, 20 %, 3328 features: 1.9 GB of X in 221 us with 128 features per workgroup and X transposed on
-// the way into LDS by 2-byte stores, in 118 us with this image and in 110 us with 256 features; 1006 x 599,
-// 544 features: 262 -> 155 us).
+// 60 x 200 blocks of 48, 10 %, 1024 features: 31 us.
 template <bool BF16, int OUT, int NT>
 __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int64_t slices, int f_tiles,
                                                          const uint16_t* __restrict__ A,
@@ -506,6 +504,135 @@ __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int6
   }
 }
 
+// A wavefront owns a 16-row slice and TF features (TF / 16 accumulators) and takes two chunks of 16 columns of the block
+// row per step: their 32 rows of X go through LDS of its own (image as in bsr_tile, the XOR extended by 2 * (k / 8 %
+// 2): the two blocks of 16 lanes that a transposing read serves together ask for the same units of k groups eight rows
+// apart here), the next step's loads in flight; no wavefront waits for another.  The A operand is one 16-byte load per
+// lane.  Bound by the rows of X that come out of L2: a slice uses each of them for 16 rows only.  Against four
+// wavefronts that shared 256 features and met at a barrier per step: 318 x 284 blocks of 16, 20 %, 3328 features 108
+// -> 95 us; 732 x 74, 14 %, 320 features 15.3 -> 10.6; 1024 x 1024, 10 %, 4096 features 1081 -> 614 with 256 features
+// in ranked order (722 with 128; 975 with 256 in plain order).
+template <bool BF16, int OUT, int TF, bool ONE>  // ONE: blk == 16, a chunk is a block
+__global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(int blk, int feat, int64_t slices,
+                                                                              int f_tiles, int ranked,
+                                                                              const uint16_t* __restrict__ A,
+                                                                              const uint16_t* __restrict__ X,
+                                                                              void* __restrict__ Y,
+                                                                              const int32_t* __restrict__ indptr,
+                                                                              const int32_t* __restrict__ indices,
+                                                                              const int32_t* __restrict__ row_ids) {
+  constexpr int FT = TF / 16;   // accumulators
+  constexpr int FCN = TF / 8;   // 16-byte units per row of X
+  constexpr int KQ = 64 / FCN;  // rows of X per load
+  constexpr int XQ = 16 / KQ;   // loads per chunk
+  __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
+  int64_t slice;
+  int f_tile;
+  if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+             : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
+    return;
+  const int lane = threadIdx.x, ii = lane & 15, g = lane >> 4;
+  if (ONE) blk = 16;
+  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  int i = (int)slice / sub;
+  const int bi0 = (int)slice % sub * 16;
+  if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = f_tile * TF;
+  // staging: unit c of the rows KQ * q + kq of a chunk.  Units beyond feat repeat the last one: features nobody stores.
+  const int c = lane % FCN, kq = lane / FCN;
+  const uint32_t xoff = (uint32_t)(kq * feat + min(8 * c, feat - f0 - 8)) * 2;
+  auto place = [&](int k) {
+    return (uint32_t)(((k >> 2) * 4 * FCN + (k & 3) * FCN + (c ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)))) * 16);
+  };
+  // operands: row ii of the slice, k group g (8 of the step's 32); tile t of X is where its bits 5 ... say
+  const uint32_t aoff = (uint32_t)((bi0 + ii) * blk + 8 * (g & 1)) * 2;
+  const int kr = ii >> 2;
+  const uint32_t bread = (uint32_t)(((2 * g) * 4 * FCN + kr * FCN + (((ii & 3) >> 1) ^ (4 * kr) ^ (2 * (g & 1)))) * 16 +
+                                    (ii & 1) * 8);
+
+  f32x4 acc[FT];
+#pragma unroll
+  for (int t = 0; t < FT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
+  const int steps = (nblk * sub + 1) / 2;
+  // block columns of the 64 blocks from `base` on and of the next 64
+  int base = 0;
+  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
+  int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
+  int block = 0, col = 0;  // the next chunk to fetch
+  u32x4 xr[2][XQ], ar;
+  auto fetch = [&]() {
+    const int first = block;
+    uint32_t a_at[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const bool live = block < nblk;
+      const int of = block & (kWave - 1);
+      const int j = ONE || block < base + kWave ? __builtin_amdgcn_readlane(j_lane, of) : __builtin_amdgcn_readlane(j_more, of);
+      const auto rx = window(X + ((int64_t)j * blk + 16 * col) * feat + f0, live ? 32u * feat : 0);
+#pragma unroll
+      for (int q = 0; q < XQ; ++q)
+        xr[b][q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * KQ * 2 * feat, 0);
+      a_at[b] = live ? (uint32_t)((block - first) * blk * blk + 16 * col) * 2 + aoff : ~15u;
+      if (ONE || ++col == sub) col = 0, ++block;
+    }
+    const auto ra = window(A + (int64_t)(p_begin + first) * blk * blk, ONE ? 512u * max(min(nblk - first, 2), 0) : 4u * blk * blk);
+    ar = __builtin_amdgcn_raw_buffer_load_b128(ra, ONE ? aoff + 512 * (g >> 1) : g < 2 ? a_at[0] : a_at[1], 0, 0);
+    if (block >= base + kWave) {
+      base += kWave;
+      j_lane = j_more;
+      j_more = base + kWave + lane < nblk ? indices[p_begin + base + kWave + lane] : 0;
+    }
+  };
+  fetch();
+#pragma unroll 1
+  for (int it = 0; it < steps; ++it) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + place(16 * b + KQ * q + kq)) = xr[b][q];
+    const u32x4 a = ar;
+    fetch();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < FT; ++t) acc[t] = mfma16<BF16>(a, read_b(stage + (bread ^ (32 * t)), FCN * 64), acc[t]);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+  }
+  // acc[t][v] is row 4 g + v, column 16 t + ii; 16-bit results through LDS into 16-byte stores (see store_rows)
+  const int64_t row0 = (int64_t)i_out * blk + bi0;
+  if constexpr (OUT == 1) {
+#pragma unroll
+    for (int t = 0; t < FT; ++t) {
+      if (f0 + 16 * t >= feat) continue;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        static_cast<float*>(Y)[(row0 + 4 * g + v) * feat + f0 + 16 * t + ii] = acc[t][v];
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < FT; ++t)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        *reinterpret_cast<uint16_t*>(stage + ((4 * g + v) * TF + 16 * t + ii) * 2) = to16<BF16>(acc[t][v]);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int q = 0; q < 16 * FCN / kWave; ++q) {
+      const int at = kWave * q + lane, row = at / FCN, u = at % FCN;
+      const u32x4 w = *reinterpret_cast<const u32x4*>(stage + at * 16);
+      if (f0 + 8 * u < feat)
+        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row0 + row) * feat + f0 +
+                                                                8 * u));
+    }
+  }
+}
+
 // ------------------------------------------------------------------ large launches: a wavefront per tile
 // A wavefront owns 32 rows of a block row and 256 features: eight 32x32 accumulators.  Its X tile has 16 KB of LDS of
 // its own (image as in bsr_tile), filled from registers that were loaded a step before, so that 8 wavefronts per CU
@@ -515,8 +642,6 @@ __global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int6
 // 10 % blocks of 32, 4096 features 595 us with workgroups of four wavefronts, 590 with this kernel in plain order
 // (3.97 GB through the L2s, 31 M misses), 377 with both; 300 x 450 blocks, 3232 features 290 -> 217 us; 1024 x 512,
 // 5 % 706 -> 454.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
-constexpr int kWaveF = 256;
-
 template <bool BF16, int OUT>
 __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
                                                             const uint16_t* __restrict__ A,
@@ -824,7 +949,40 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       return 0;
     }
   }
+  auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
+  constexpr int64_t kMuchX = 3 << 20;
+  const int rankable = mb <= kRankRows ? 1 : 0;
   if (unit == 16) {
+    // Ranked order as below.  256 features per wavefront then, unless the last tile would be mostly empty or wavefronts
+    // few: 1024 x 1024 blocks of 16, 1024 features 158 us (171 with 128), 1006 x 599, 544 features 155 (140).
+    const bool much = x_tile_bytes(kWaveF) > kMuchX;
+    const bool wide = much && unit_slices * stir::ceil_div(feat, kWaveF) >= 8 * cus &&
+                      (kWaveF - 1 - (feat - 1) % kWaveF) * 8 <= feat;
+    const int ranked = much ? rankable : 0;
+    // A wavefront per slice once eight per CU have one: 60 x 200 blocks of 48, 1024 features (1440) 33.1 us against 31.0
+    // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
+    if (unit_slices * stir::ceil_div(feat, kTileF) >= 8 * cus && feat < (1 << 25) && blk <= 4096) {
+      const int f_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
+      const int64_t blocks = grid_of(unit_slices, f_tiles);
+      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
+      const dim3 grid((unsigned)blocks), block(kWave);
+#define STIR_BSR_16W(BF, OUT, TF, ONE)                                                                             \
+  hipLaunchKernelGGL((bsr16_wave_kernel<BF, OUT, TF, ONE>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, ranked, \
+                     A, X, d_Y, d_indptr, d_indices, d_row_ids)
+#define STIR_BSR_16(BF, OUT)                                                                                   \
+  do {                                                                                                         \
+    if (wide) {                                                                                                \
+      if (blk == 16) STIR_BSR_16W(BF, OUT, kWaveF, true); else STIR_BSR_16W(BF, OUT, kWaveF, false);           \
+    } else {                                                                                                   \
+      if (blk == 16) STIR_BSR_16W(BF, OUT, kTileF, true); else STIR_BSR_16W(BF, OUT, kTileF, false);           \
+    }                                                                                                          \
+  } while (0)
+      STIR_BSR_TYPES(STIR_BSR_16)
+#undef STIR_BSR_16
+#undef STIR_BSR_16W
+      STIR_LAUNCH_CHECK();
+      return 0;
+    }
     const int nt16 = feat >= 256 ? 2 : 1;
     const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt16);
     const int64_t blocks = grid_of(unit_slices, f_tiles);
@@ -856,9 +1014,6 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // 219 x 201 blocks, 1504 features (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 456 x 309, 352 features (912, of which
   // half have 96 features) 66.4 -> 69.4.  Below 3 MB finding the row (2-3 us a tile) is lost: 359 x 71, 3488 features
   // 69 -> 83 us ranked, 430 x 120, 1120 features 62 -> 67.
-  auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
-  constexpr int64_t kMuchX = 3 << 20;
-  const int rankable = mb <= kRankRows ? 1 : 0;
   const int wf_tiles = (int)stir::ceil_div(feat, kWaveF);
   if (rs == 1 && x_tile_bytes(kWaveF) > kMuchX && slices * wf_tiles >= 4 * cus && feat < (1 << 25) && blk <= 4096) {
     const int64_t blocks = grid_of(slices, wf_tiles);

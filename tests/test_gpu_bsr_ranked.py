@@ -32,6 +32,10 @@ def _config(mb, nb, blk, density, feat, seed):
     (20, 200, 64, 0.03, 96),       # four wavefronts per 64 rows
     (12, 100, 128, 0.05, 160),     # block rows dealt to XCDs
     (1, 6200, 32, 0.001, 64),
+    (1030, 90, 16, 0.02, 224),     # 16-row slices by a wavefront each: plain order
+    (1024, 400, 16, 0.004, 512),   # ranked, 256 features
+    (700, 400, 16, 0.004, 320),    # ranked, 128 features, an odd number of blocks
+    (230, 50, 48, 0.05, 352),      # chunks of two blocks in one step
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("start", [0, 1])

@@ -8,7 +8,7 @@
 // memory, set back to zero by that workgroup -- adds them up in order.  So C is written once, without
 // atomics, and the same bits every time.
 //
-// Bound by the gather of rows of B (1.17 M nonzeros, 47 features: 38 us, 9.6 TB/s of the 128-byte lines
+// Bound by the gather of rows of B (1.17 M nonzeros, 47 features: 36 us, 10 TB/s of the 128-byte lines
 // that its rows touch).  With a launch over rows and a second one for what is long among them (spmm.hip) the
 // same product pays a second launch, a search of every piece for long rows that mostly are not there, and
 // wavefronts whose rows differ in length (51 us).
@@ -27,10 +27,10 @@ using stir::kWave;
 using stir::ld4;
 
 constexpr int kBlock = 256;
-constexpr int kSlots = 768;     // nonzeros a workgroup holds in LDS: eight workgroups per compute unit
+constexpr int kSlots = 1152;    // nonzeros a workgroup holds in LDS: seven workgroups per compute unit
 // A row of at most this many nonzeros is not cut: it is left whole to the workgroup that has its mark.
 constexpr int kWhole = 128;
-constexpr int kMaxItems = 512;
+constexpr int kMaxItems = 1024;
 static_assert(kMaxItems + kWhole <= kSlots, "the last row of a workgroup may lie behind its entries");
 constexpr int kFlight = 8;      // rows of B requested at a time by a lane group
 
@@ -328,17 +328,6 @@ __global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(
   }
 }
 
-// About 1100 workgroups, four per compute unit, as long as that gives each a few stretches of nonzeros and
-// what it holds fits: 50 k rows, 450 k nonzeros, 64 features: 34.8 us with 64 entries, 22.9 with 288 or 480.
-int entries_per_workgroup(int32_t m, int64_t nnz) {
-  const int64_t items = (m + nnz) / 1100;
-  return (int)(std::max<int64_t>(64, std::min<int64_t>(items, kMaxItems)) + 31) / 32 * 32;
-}
-
-int64_t workgroups(int32_t m, int64_t nnz) {
-  return stir::ceil_div(m + nnz, entries_per_workgroup(m, nnz));
-}
-
 // Lane groups as wide as feat, or of 64 features and several feature slices (slice_block): an XCD's L2 holds
 // more rows of B a slice wide, which pays for looking for the entries once per slice from 1.5e8 multiplications
 // on, as long as slices begin on 256-byte boundaries and B is not far beyond what the last level holds.
@@ -354,6 +343,31 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
   const bool cut = whole > 2 && feat % 64 == 0 && work >= 150000000 && work <= 2500000000 &&
                    (int64_t)n * feat * 4 <= 320000000;
   return cut ? 2 : whole;
+}
+
+// As many workgroups as are resident at once, so that all end together: seven per compute unit where that leaves them
+// a few hundred entries each, else five; of several slices of features five or four (their workgroups take turns
+// anyhow, and each looks for its entries once per slice).  us with 4 / 5 / 6 / 7 / 8 per compute unit, and with 512
+// entries each:
+//   169 k rows, 1.17 M nonzeros, 64 features 35.2 / 35.3 / 33.0 / 32.2 / 36.2, 35.6; 47: 39.3 / 39.4 / 37.1 / 36.1 / 39.8, 39.7;
+//   108 k, 1.2 M, 64: 33.4 / 33.3 / 31.8 / 31.4 / 35.2, 34.4; 17 k, 288 k, 12: 10.3 / 10.1 / 10.6 / 11.3 / 13.7, 10.2;
+//   54 k, 521 k, 100: 27.6 / 28.1 / 27.8 / 28.1 / 30.8, 29.2; 9 k, 146 k, 64: 10.3 / 9.8 / 10.1 / 10.4 / 12.9, 10.3;
+//   25 k, 1 M, 256 (four slices): 85.3 / 85.8 / 87.0 / 87.5 / 87.8, 90.4; 30 k, 500 k, 512 (eight): 97 / 100 / 102 / 107 / 109, 98.
+// The other way: 100 k rows, 1.5 M nonzeros of uniform columns, 128 features 111.4 against 109.3 (skewed: 69.6, 73.0).
+// From several turns of the largest workgroups on, 512 entries: 199 k rows, 4.9 M nonzeros, 44 features 167.8 / 163.4.
+int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
+  const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c);
+  constexpr int64_t kUnits = 256;  // compute units
+  const int64_t entries = m + nnz;
+  int64_t per_unit = c == 5 ? 6 : 7;
+  if (entries > 2 * kUnits * per_unit * kMaxItems) return 512;
+  if (slices > 2 || entries < kUnits * per_unit * 400) per_unit = slices > 5 ? 4 : 5;
+  const int64_t items = stir::ceil_div(entries, kUnits * per_unit);
+  return (int)(std::max<int64_t>(64, std::min<int64_t>(items, kMaxItems)) + 3) / 4 * 4;
+}
+
+int64_t workgroups(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
+  return stir::ceil_div(m + nnz, entries_per_workgroup(m, n, feat, nnz));
 }
 
 // Below, the search for its entries costs a workgroup more than it gains (4096 rows, 65 k nonzeros, 32
@@ -397,9 +411,9 @@ int launch_merged_balanced(int32_t m, int32_t n, int32_t feat, int64_t slots, co
                            const float* d_B, float* d_C, const int32_t* d_slot_ptr, const int32_t* d_cols,
                            hipStream_t st) {
   const int c = slice_class(n, feat, slots), slices = (int)ceil_div(feat, 16 << c);
-  const int64_t grid = slice_grid(slices, workgroups(m, slots));
+  const int64_t grid = slice_grid(slices, workgroups(m, n, feat, slots));
   STIR_REQUIRE(grid < (int64_t(1) << 31), "hyb_spmm: %lld workgroups exceed one launch", (long long)grid);
-  return launch<true>(c, grid, slices, entries_per_workgroup(m, slots), m, feat, slots,
+  return launch<true>(c, grid, slices, entries_per_workgroup(m, n, feat, slots), m, feat, slots,
                       reinterpret_cast<const float*>(d_vals), d_B, d_C, d_slot_ptr, d_cols, nullptr, nullptr, st);
 }
 
@@ -410,14 +424,14 @@ extern "C" {
 // the counters, one per workgroup; behind them two partial rows per workgroup
 size_t stir_csr_spmm_workspace_clear_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   if (m < 0 || n < 0 || feat <= 0 || nnz < 0 || !balanced(m, n, feat, nnz)) return 0;
-  const size_t parts = size_t(workgroups(m, nnz)) * stir::ceil_div(feat, 16 << slice_class(n, feat, nnz));
+  const size_t parts = size_t(workgroups(m, n, feat, nnz)) * stir::ceil_div(feat, 16 << slice_class(n, feat, nnz));
   return (parts * 4 + 15) / 16 * 16;
 }
 
 size_t stir_csr_spmm_workspace_bytes(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   if (m < 0 || n < 0 || feat <= 0 || nnz < 0 || !balanced(m, n, feat, nnz)) return 0;
   const int c = slice_class(n, feat, nnz);
-  const size_t parts = size_t(workgroups(m, nnz)) * stir::ceil_div(feat, 16 << c);
+  const size_t parts = size_t(workgroups(m, n, feat, nnz)) * stir::ceil_div(feat, 16 << c);
   return stir_csr_spmm_workspace_clear_bytes(m, n, feat, nnz) + parts * 2 * (size_t(16) << c) * 4;
 }
 
@@ -429,11 +443,11 @@ int stir_csr_spmm_f32_workspace(int32_t m, int32_t n, int32_t feat, int64_t nnz,
     return stir_csr_spmm_f32(m, n, feat, nnz, d_A, d_B, d_C, d_indptr, d_indices, stream);
   STIR_REQUIRE(d_B && d_C && d_indptr && d_workspace && (nnz == 0 || (d_A && d_indices)),
                "csr_spmm: null pointer argument");
-  const int64_t wgs = workgroups(m, nnz);
+  const int64_t wgs = workgroups(m, n, feat, nnz);
   const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c);
   const int64_t grid = stir::slice_grid(slices, wgs);
   STIR_REQUIRE(grid < (int64_t(1) << 31), "csr_spmm: %lld workgroups exceed one launch", (long long)grid);
-  const int items = entries_per_workgroup(m, nnz);
+  const int items = entries_per_workgroup(m, n, feat, nnz);
   uint32_t* counters = static_cast<uint32_t*>(d_workspace);
   float* partials = reinterpret_cast<float*>(static_cast<char*>(d_workspace) +
                                              stir_csr_spmm_workspace_clear_bytes(m, n, feat, nnz));

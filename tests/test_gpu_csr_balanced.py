@@ -66,6 +66,12 @@ def test_feature_slices(dev, feat, m, most):
     test_rows_across_workgroups(dev, feat, m, most)
 
 
+@pytest.mark.parametrize("feat,m,most", [(8, 25001, 40), (13, 60003, 62), (8, 120001, 64)])
+def test_workgroups_by_size(dev, feat, m, most):
+    """Hundreds of entries a workgroup, as many as it holds, and several turns of fewer."""
+    test_rows_across_workgroups(dev, feat, m, most)
+
+
 @pytest.mark.parametrize("feat", [4, 47, 64, 256])
 def test_only_the_counters_are_cleared(dev, feat):
     """What is in the workspace behind the counters does not matter, and the counters are zero again afterwards."""

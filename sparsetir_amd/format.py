@@ -75,7 +75,22 @@ def column_part_hyb(num_rows, num_cols, indptr_nd, indices_nd, num_col_parts, bu
     return nest(rows), nest(cols), nest(mask)
 
 
+def _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values):
+    """One column partition of tensors as they should be, on the current device; None: not taken."""
+    if num_col_parts != 1:
+        return None
+    from . import _host
+
+    out = _host.column_part_hyb(num_rows, num_cols, indptr, indices, buckets, values)
+    if out == -1:
+        _lib.check(out)
+    return None if out is None else tuple([lists] for lists in out if lists is not None)
+
+
 def _column_part_hyb_device(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values=None):
+    out = _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values)
+    if out is not None:
+        return out
     import torch
 
     L = _lib.lib()
@@ -89,14 +104,9 @@ def _column_part_hyb_device(num_rows, num_cols, indptr, indices, num_col_parts, 
     if indptr.shape[0] != num_rows + 1:
         raise _lib.SparseTIRError("ColumnPartHyb: indptr must have num_rows + 1 entries")
     dev = indptr.device
-    if num_col_parts == 1:
-        from . import _host
-
-        out = _host.column_part_hyb(num_rows, num_cols, indptr, indices, buckets, values)
-        if out == -1:
-            _lib.check(out)
-        if out is not None:
-            return tuple([lists] for lists in out if lists is not None)
+    out = _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values)
+    if out is not None:
+        return out
     widths = np.ascontiguousarray(np.asarray(list(buckets), dtype=np.int32))
     nb = len(widths)
     nk = num_col_parts * nb

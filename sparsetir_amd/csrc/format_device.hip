@@ -484,7 +484,18 @@ struct EntryArgs {
   const int32_t* permuted;
   const int32_t* idx2;
   const int32_t* perm;
+  // one partition: where not null, instead of slot0_in the ELL rows that the row's bucket has in front of the row's
+  // group of 64 rows ([bucket][groups]) and, of those, in the group
+  const int32_t* __restrict__ group_base;
+  const int32_t* __restrict__ rank_in;
+  int64_t groups;
 };
+
+// Slot of entry e of the row is this + e; lo: the row's first entry.
+__device__ __forceinline__ int64_t first_slot(const EntryArgs& g, int row, int beta, int lo) {
+  if (!g.rank_in) return g.slot0_in[row];
+  return (int64_t)(g.group_base[beta * g.groups + row / kWave] + g.rank_in[row]) * g.widths[beta] - lo;
+}
 
 // The view of the matrix the placement kernels walk: the caller's arrays, or the regrouped ones.
 __device__ __forceinline__ EntryArgs effective(EntryArgs g) {
@@ -562,8 +573,12 @@ __device__ __forceinline__ void place_general(const EntryArgs& g, EntryStage& st
       const int p = col[j] / g.psize;
       if (p != cur_p) {
         cur_p = p;
-        k = p * NB + g.kb_in[(int64_t)p * m + r];
-        slot0 = g.slot0_in[(int64_t)p * m + r];
+        const int beta = g.kb_in[(int64_t)p * m + r];
+        k = p * NB + beta;
+        if constexpr (SINGLE)
+          slot0 = first_slot(g, r, beta, (int)ptr_at(r));
+        else
+          slot0 = g.slot0_in[(int64_t)p * m + r];
       }
       const int64_t slot = slot0 + e;
       st.kh[at] = k * 256 + (int32_t)(slot >> 32);
@@ -619,7 +634,7 @@ __device__ __forceinline__ void place_single(const EntryArgs& g, RowStage& rs, i
     if (x < nr) {
       const int lo = g.indptr[ra + x], hi = g.indptr[ra + x + 1];
       const int beta = g.kb_in[ra + x];
-      const int64_t slot0 = g.slot0_in[ra + x];
+      const int64_t slot0 = first_slot(g, ra + x, beta, lo);
       const int d = hi - lo;
       const int w = g.widths[beta];
       rs.ptr[x] = lo;
@@ -737,9 +752,9 @@ __global__ __launch_bounds__(256) void place_values_kernel(EntryArgs g_in, const
 // chain of small launches and of calls between them, so the host reads nothing before it launches (the
 // kernels take the ends of indptr from device memory), sizes and status come back through host memory
 // that the kernels write themselves, bucket widths and output addresses travel as kernel arguments, and
-// columns, mask and values are placed by one kernel: 4 launches and one wait instead of 17 launches and
-// copies and 4 waits.  With values: 20 k rows, 200 k nonzeros 449 -> 85 us per call from Python, 169 k rows,
-// 1.17 M nonzeros 417 -> 57 us, 2.45 M rows, 61.8 M nonzeros 1053 -> 524 us.
+// columns, mask, values and row ids are placed by one kernel: 2 or 3 launches and one wait instead of 17 launches
+// and copies and 4 waits.  With values, and a kernel for the row ids still: 20 k rows, 200 k nonzeros 449 -> 85 us
+// per call from Python, 169 k rows, 1.17 M nonzeros 417 -> 57 us, 2.45 M rows, 61.8 M nonzeros 1053 -> 524 us.
 constexpr int kOneBuckets = 32;
 
 struct OneWidths {
@@ -781,6 +796,14 @@ __device__ __forceinline__ OneEnds one_ends(const int32_t* __restrict__ indptr, 
   if (e.bad) e.first = 0, e.nnz = 0;
   return e;
 }
+// the ELL rows of its bucket before a row in its group of 64, in the place of the slots of other paths
+__device__ __forceinline__ int32_t* ranks(const Workspace& ws) { return reinterpret_cast<int32_t*>(ws.slot0); }
+// Row ids and the rows' first slots by a kernel of their own?  Without, the placement finds a row's first slot from
+// its rank and its group's place in the bucket, a load behind a load, and the row ids ride in its launch.  Per call
+// from Python with / without that kernel: 1 k rows, 8 k nonzeros 35.6 / 31.6 us, 200 k, 3.2 M 47 / 41 us, 1 M, 4 M
+// 79 / 69 us, 1 M, 27 M 172 / 169 us, but 2.45 M, 66 M 394 / 407 us: there the chain costs more than the launch.
+constexpr int kRowsApart = 1 << 20;
+__host__ __device__ __forceinline__ bool rows_apart(int m) { return m > kRowsApart; }
 __device__ __forceinline__ int64_t one_stride(int64_t nnz) { return nnz > kCoarse ? (nnz + kCoarse - 1) / kCoarse : 1; }
 
 // Exclusive scan of hist[b][0 .. W) by one wavefront, W at most 4 * 64, for a workgroup of four wavefronts; the
@@ -874,31 +897,47 @@ __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t stride = one_stride(ends.nnz);
-  int d = 0;
+  int d = 0, rs = 0;
   if (i < m) {
-    int rs = indptr[i], re = indptr[i + 1];
+    rs = indptr[i];
+    int re = indptr[i + 1];
     if (re < rs || rs < ends.first || re > end) {
       if (!ends.bad) answer_bad(&answer->bad_indptr);
       rs = re = ends.first;
     }
     for (int64_t q = (rs - ends.first + stride - 1) / stride; ends.first + q * stride < re; ++q) ws.coarse[q] = i;
-    ws.lo[i] = rs;
     d = re - rs;
   }
-  const int beta = bucket_of_dev(widths.w, NB, d);
-  const int rho = d == 0 ? 0 : (d + widths.w[beta] - 1) / widths.w[beta];
   int32_t* h = ws.hist + wave;  // [b][W]
   auto put = [&](int b, int32_t v) {
     if (lane == 0 && wave < W) __hip_atomic_store(h + b * W, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
+  const int beta = bucket_of_dev(widths.w, NB, d);
+  int rank = 0;
   for (int b = 0; b < NB - 1; ++b) {
     const unsigned long long bal = __ballot(d > 0 && beta == b);
+    if (beta == b) rank = __popcll(bal & ((1ull << lane) - 1ull));
     put(b, __popcll(bal));
   }
-  int tot = beta == NB - 1 ? rho : 0;
+  int tot = 0;
+  if (__ballot(beta == NB - 1)) {  // rows of several ELL rows
+    const int rho = beta == NB - 1 ? (d + widths.w[beta] - 1) / widths.w[beta] : 0;
+    tot = rho;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off, kWave);
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int up = __shfl_up(tot, off, kWave);
+      if (lane >= off) tot += up;
+    }
+    if (beta == NB - 1) rank = tot - rho;
+    tot = __shfl(tot, kWave - 1, kWave);
+  }
   put(NB - 1, tot);
+  if (i < m) {
+    if (rows_apart(m))
+      ws.lo[i] = rs;
+    else
+      ws.kb[i] = beta, ranks(ws)[i] = rank;
+  }
   finish();
 }
 
@@ -956,15 +995,36 @@ struct OneCarried {
   float value;
 };
 
-// Columns, mask and -- VALUES -- values of every nonzero, and the padding behind every row.
-template <bool VALUES>
-__global__ __launch_bounds__(256) void one_place_kernel(int m, int num_cols, int NB, int64_t max_nnz, Workspace ws,
-                                                        OneOutputs out, const int32_t* __restrict__ indptr,
+// Columns, mask and -- VALUES -- values of every nonzero, and the padding behind every row; unless they were written
+// APART, the row ids, by the workgroups from place_blocks on.  (Row ids by the wavefront that places the row's first
+// nonzero instead: registers and stores in the placement's way, 24 against 20.6 us at 200 k rows, 3.2 M nonzeros.)
+template <bool VALUES, bool APART>
+__global__ __launch_bounds__(256) void one_place_kernel(int m, int num_cols, int NB, int64_t W, int64_t max_nnz,
+                                                        int place_blocks, Workspace ws, OneOutputs out,
+                                                        const int32_t* __restrict__ indptr,
                                                         const int32_t* __restrict__ indices,
                                                         const float* __restrict__ values) {
   const OneEnds ends = one_ends(indptr, m, max_nnz);
+  if (!APART && (int)blockIdx.x >= place_blocks) {
+    const int i = ((int)blockIdx.x - place_blocks) * 256 + threadIdx.x, lane = threadIdx.x & 63;
+    int beta = 0, rho = 0, base = 0;
+    if (i < m) {
+      const int d = indptr[i + 1] - indptr[i];
+      beta = ws.kb[i];
+      if (d > 0) {
+        base = ws.hist[beta * W + i / kWave] + ranks(ws)[i];
+        rho = beta < NB - 1 ? 1 : (d + ws.widths[beta] - 1) / ws.widths[beta];
+      }
+    }
+    wave_fill(rho, lane, [&](int owner, int off, bool active) {
+      const int k = __shfl(beta, owner, kWave), at = __shfl(base, owner, kWave) + off, row = __shfl(i, owner, kWave);
+      if (active) out.rows[k][at] = row;
+    });
+    return;
+  }
   const EntryArgs g{m, 1, num_cols, NB, ends.nnz, ends.first, indptr, indices, ws.widths, ws.slot0, ws.kb, ws.coarse,
-                    one_stride(ends.nnz), nullptr, nullptr, nullptr};
+                    one_stride(ends.nnz), nullptr, nullptr, nullptr, ws.hist,
+                    APART ? nullptr : ranks(ws), W};
   __shared__ int32_t *cols[kOneBuckets], *mask[kOneBuckets];
   __shared__ float* a[kOneBuckets];
   if ((int)threadIdx.x < NB) {
@@ -1294,7 +1354,7 @@ int stir_column_part_hyb_device_fill(int32_t num_rows, int32_t num_cols, const i
   const PermutedTail tail = permuted_tail(d_workspace, ws, nnz);
   const EntryArgs ea{m, P, psize, NB, nnz, ends[0], d_indptr, d_indices, ws.widths, ws.slot0, ws.kb, ws.coarse,
                      coarse_stride(nnz), P > 1 ? ws.status + kPermutedAt : nullptr,
-                     P > 1 ? tail.idx2 - ends[0] : nullptr, P > 1 ? tail.perm - ends[0] : nullptr};
+                     P > 1 ? tail.idx2 - ends[0] : nullptr, P > 1 ? tail.perm - ends[0] : nullptr, nullptr, nullptr, 0};
   if (P == 1)
     hipLaunchKernelGGL(place_entries_kernel<true>, dim3((unsigned)stir::ceil_div(nnz, 4 * kSingleTile)), dim3(256), 0,
                        st, ea, ws.cols_tab, ws.mask_tab);
@@ -1339,7 +1399,7 @@ int stir_column_part_hyb_device_values(int32_t num_rows, int32_t num_cols, const
   const PermutedTail tail = permuted_tail(d_workspace, ws, nnz);
   const EntryArgs ea{m, P, psize, NB, nnz, ends[0], d_indptr, d_indices, ws.widths, ws.slot0, ws.kb, ws.coarse,
                      coarse_stride(nnz), P > 1 ? ws.status + kPermutedAt : nullptr,
-                     P > 1 ? tail.idx2 - ends[0] : nullptr, P > 1 ? tail.perm - ends[0] : nullptr};
+                     P > 1 ? tail.idx2 - ends[0] : nullptr, P > 1 ? tail.perm - ends[0] : nullptr, nullptr, nullptr, 0};
   if (P == 1)
     hipLaunchKernelGGL(place_values_kernel<true>, dim3((unsigned)stir::ceil_div(nnz, 4 * kSingleTile)), dim3(256), 0,
                        st, ea, d_values, a_tab);
@@ -1416,16 +1476,16 @@ int stir_column_part_hyb_one_fill(int32_t num_rows, int32_t num_cols, const int3
   std::copy(d_col_indices, d_col_indices + NB, out.cols);
   std::copy(d_mask, d_mask + NB, out.mask);
   if (d_A) std::copy(d_A, d_A + NB, out.a);
-  hipLaunchKernelGGL(one_rows_kernel, dim3((unsigned)stir::ceil_div(m, 256)), dim3(256), 0, st, m, NB, W, ws, out,
-                     d_indptr);
-  STIR_LAUNCH_CHECK();
-  const dim3 grid((unsigned)stir::ceil_div(max_nnz, 4 * kSingleTile));
-  if (d_A)
-    hipLaunchKernelGGL(one_place_kernel<true>, grid, dim3(256), 0, st, m, num_cols, NB, max_nnz, ws, out, d_indptr,
-                       d_indices, d_values);
-  else
-    hipLaunchKernelGGL(one_place_kernel<false>, grid, dim3(256), 0, st, m, num_cols, NB, max_nnz, ws, out, d_indptr,
-                       d_indices, d_values);
+  const bool apart = rows_apart(m);
+  const int64_t place_blocks = stir::ceil_div(max_nnz, 4 * kSingleTile), row_blocks = stir::ceil_div(m, 256);
+  if (apart) {
+    hipLaunchKernelGGL(one_rows_kernel, dim3((unsigned)row_blocks), dim3(256), 0, st, m, NB, W, ws, out, d_indptr);
+    STIR_LAUNCH_CHECK();
+  }
+  const auto kernel = d_A ? apart ? one_place_kernel<true, true> : one_place_kernel<true, false>
+                          : apart ? one_place_kernel<false, true> : one_place_kernel<false, false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(place_blocks + (apart ? 0 : row_blocks))), dim3(256), 0, st, m, num_cols,
+                     NB, W, max_nnz, (int)place_blocks, ws, out, d_indptr, d_indices, d_values);
   STIR_LAUNCH_CHECK();
   return 0;
 }

@@ -47,6 +47,17 @@ def test_matches_host(dev, m, buckets):
     _compare(dev, m, 900, *_csr(m, 900, deg, m), buckets)
 
 
+@pytest.mark.parametrize("m", [64 * 256, 64 * 256 + 1, 1 << 20, (1 << 20) + 1])
+def test_around_the_changes_of_kernel(dev, m):
+    """The most rows whose counts the counting kernel scans itself, the most whose ids are written with the columns,
+    and one more; rows of many ELL rows and runs of empty ones."""
+    rng = np.random.default_rng(m)
+    deg = rng.integers(0, 9 if m < 1 << 20 else 3, m)
+    deg[[0, m // 3, m - 1]] = [700, 20000, 40]
+    deg[m // 2:m // 2 + 300] = 0
+    _compare(dev, m, 5000, *_csr(m, 5000, deg, m), [1, 2, 4, 8, 16, 32])
+
+
 def test_long_runs_of_empty_rows(dev):
     """More rows around a tile's nonzeros than the row window holds: the per-nonzero search."""
     deg = np.zeros(5000, np.int64)
@@ -78,5 +89,15 @@ def test_refuses_what_the_arrays_cannot_mean(dev):
                                  ([0, 1, 1, 2], [3, -1], "outside")):
         with pytest.raises(SparseTIRError, match=msg):
             st.column_part_hyb(3, 4, t(indptr), t(indices), 1, [1, 2])
+    m = 9000  # what is wrong lies with a later group of rows, a later workgroup of the check
+    indptr = torch.arange(0, 10 * m + 1, 10, dtype=torch.int32, device=dev)
+    indices = torch.zeros(10 * m, dtype=torch.int32, device=dev)
+    indices[70001] = 4
+    with pytest.raises(SparseTIRError, match="outside"):
+        st.column_part_hyb(m, 4, indptr, indices, 1, [1, 2])
+    indices[70001] = 0
+    indptr[8500] = 0
+    with pytest.raises(SparseTIRError, match="row pointer"):
+        st.column_part_hyb(m, 4, indptr, indices, 1, [1, 2])
     empty = st.column_part_hyb(2, 4, t([0, 0, 0]), t([]), 1, [1, 2])
     assert [x.numel() for x in empty[0][0]] == [0, 0]

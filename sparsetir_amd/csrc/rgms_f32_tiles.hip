@@ -10,8 +10,11 @@
 // An edge record holds the source row, the address of the edge's weight (weights are read at
 // every launch) and its part in a chain; a pair is one word: row inside the tile, chains, first chain.
 //
-// Kernel: one workgroup per unit -- a tile, or a piece of one; wavefront w takes the unit's batches w,
-// w + WAVES, ... and all of them sum into one partial tile in LDS, in turn.  Per batch:
+// Kernel: one workgroup per unit -- a tile, or a piece of one; each wavefront takes an equal stretch of the unit's
+// batches, which are in order of their relations, and all of them sum into one partial tile in LDS, in turn.  W is
+// read when the relation changes: with batches dealt out one by one it was read for each, 12 KB at 64 -> 32, and
+// half the time went there (2 M edges, 65 relations, us per call: 32 -> 32 73 / 63, 64 -> 32 132 / 107, 32 -> 64 107 / 97;
+// 342 k edges, 130 relations, hardly two batches of each in a tile: 29.5 / 28.9, 42 / 40, 38 / 37).  Per batch:
 //   1. the rows of X of the batch's edges are gathered eight rows (128 bytes each) per load instruction,
 //      a column of places per lane group, which weights and adds up its chains in registers and writes
 //      each to a row of a tile of LDS;
@@ -21,9 +24,9 @@
 //      eight inputs are its operand as they stand;
 //   4. row i of P is added to row (destination row % 128) of the partial tile with a
 //      plain LDS read-modify-write: the pairs of a batch end in different rows or in pieces of
-//      one row that this lane order adds one after the other, and the wavefronts take turns, in the order
-//      of the batches (LDS float atomics run at a third of a lane per clock and compute unit
-//      on this chip, slower than atomics in memory).
+//      one row that this lane order adds one after the other, and the wavefronts take turns (LDS float
+//      atomics run at a third of a lane per clock and compute unit on this chip, slower than atomics in
+//      memory).
 // A batch is a chain of dependent loads (batch record -> edge records -> rows of X and weights), each step
 // of it requested one batch ahead of the next.
 //
@@ -396,9 +399,11 @@ __device__ __forceinline__ void static_for_chain(F f) {
 // 32-bit byte offsets (the launch checks that they fit).
 template <int KS, int NT>
 struct TileShape {
-  // as many wavefronts as registers and LDS allow per compute unit: 20, 16, 16, 12 (4, 2, 4, 2 workgroups)
-  static constexpr int kWaves = KS == 1 ? (NT == 4 ? 8 : 4) : (NT == 4 ? 6 : 4);
-  static constexpr int kPerSimd = KS == 1 ? (NT == 4 ? 4 : 4) : (NT == 4 ? 3 : 4);
+  // as many wavefronts as registers and LDS allow per compute unit: 16, and 8 above 32 inputs and outputs (4 workgroups,
+  // 2 above 32 outputs).  Twelve there left ten registers of W in memory, and waiting for them was waiting for
+  // everything in flight (2 M edges, 65 relations, 64 -> 64: 291 / 166 us; 342 k edges, 8 relations: 63 / 43).
+  static constexpr int kWaves = KS == 1 && NT == 4 ? 8 : 4;
+  static constexpr int kPerSimd = KS == 2 && NT == 4 ? 2 : 4;
 };
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
@@ -507,9 +512,12 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
   float* et = etile[wave];
   for (int e = tid; e < kTileRows * FO; e += THREADS) yt[e] = 0.f;
   for (int e = lane; e < SS; e += 64) et[EMAX * SS + e] = 0.f;
-  if (tid == 0) turn = u.batch_begin;
-  const int b_end = u.batch_end;
-  int b = u.batch_begin + wave;
+  if (tid == 0) turn = 0;
+  // a stretch of batches for each wavefront, its k-th one in turn k * WAVES + wave
+  const int fewest = (u.batch_end - u.batch_begin) / WAVES, more = (u.batch_end - u.batch_begin) % WAVES;
+  int b = u.batch_begin + wave * fewest + min(wave, more);
+  const int b_end = b + fewest + (wave < more ? 1 : 0);
+  int my_turn = wave;
   const bool chunk_live = 4 * gc < fin;  // fin is a multiple of 4: chunks are whole
   const uint32_t row_bytes = 4u * (uint32_t)fin;
   const __amdgpu_buffer_rsrc_t Xr =
@@ -574,9 +582,11 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
 
   // The pipeline: at batch j the record of batch j + 3 is requested, the edge records of j + 2, the rows of
   // X, weights, pair words and W operands of j + 1.  One set of registers: what a batch holds is used up
-  // before the next one's is requested into it, and the other wavefronts of the SIMD cover the rest.
-  Batch bt0 = scalars(raw_batch(b), b), bt1 = scalars(raw_batch(b + WAVES), b + WAVES);
-  BatchF32 raw = raw_batch(b + 2 * WAVES);
+  // before the next one's is requested into it, and the other wavefronts of the SIMD cover the rest.  All but the
+  // pair words behind the products, where fewer registers are in use, and W last, so that only what needs W waits
+  // for it (requests before the products: 3 to 5 % slower above 32 outputs, else the same).
+  Batch bt0 = scalars(raw_batch(b), b), bt1 = scalars(raw_batch(b + 1), b + 1);
+  BatchF32 raw = raw_batch(b + 2);
   Rows rw = load_rows(load_record(bt0), bt0.places);
   u32x3 rec = load_record(bt1);
   uint32_t pw = load_pair(b), pr = load_row(b);
@@ -600,15 +610,10 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
       }
       *reinterpret_cast<f32x4*>(et + __umul24(chain & 255, SS) + 4 * gc) = run;
     });
-    // requests for the batches to come
-    rw = load_rows(rec, bt1.places);
-    const Batch bt2 = scalars(raw, b + 2 * WAVES);
-    rec = load_record(bt2);
-    raw = raw_batch(b + 3 * WAVES);
     // 2. the sums of the pairs, multiplying layout: lane (i, q) adds the chains of pair i, mostly one; a lane
     // whose pair has fewer than the batch's longest reads the tile's row of zeros meanwhile
     const int my_count = (int)((pw >> 8) & 255u);
-    const uint32_t next_pw = load_pair(b + WAVES), next_pr = load_row(b + WAVES);
+    const uint32_t next_pw = load_pair(b + 1), next_pr = load_row(b + 1);
     const char* first = reinterpret_cast<const char*>(et + 8 * q) + (pw >> 16);
     float sum[KS][8];
 #pragma unroll
@@ -647,14 +652,19 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
         for (int nt = 0; nt < NT; ++nt)
           acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kTerms[p][0]], wq[nt][s][kTerms[p][1]], acc[nt], 0, 0, 0);
     }
-    load_w(bt1.rel);
+    // requests for the batches to come
+    rw = load_rows(rec, bt1.places);
+    const Batch bt2 = scalars(raw, b + 2);
+    rec = load_record(bt2);
+    raw = raw_batch(b + 3);
+    if (bt1.rel != bt0.rel) load_w(bt1.rel);
     // 4. acc[nt][v]: pair 4 q + v of the batch, output 16 nt + i, which lives at float NT i + nt of
     // its row of the partial tile: a lane's NT outputs are neighbours, one read and one write.
     // The pairs of a batch end in different rows (a row cut into pieces has at most its last,
     // shorter piece in a batch with other pairs: a full piece fills a batch), so no two lanes
-    // update the same float; the wavefronts take turns, in the order of the batches.  (LDS
-    // instructions of a wavefront execute in order: the turn goes on after the tile is written.)
-    while (__hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != b) __builtin_amdgcn_s_sleep(1);
+    // update the same float; the wavefronts take turns.  (LDS instructions of a wavefront execute in
+    // order: the turn goes on after the tile is written.)
+    while (__hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != my_turn) __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");
     float* at[4];
     static_for_chain([&](auto V) {
@@ -670,9 +680,9 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) at[v][nt] = old[v][nt] + acc[nt][v];
     asm volatile("" ::: "memory");
-    __hip_atomic_store(&turn, b + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_store(&turn, my_turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     pw = next_pw, pr = next_pr;
-    b += WAVES;
+    ++b, my_turn += WAVES;
     bt0 = bt1, bt1 = bt2;
   }
 
@@ -685,7 +695,7 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     all_finite = fmaf(v.z, 0.f, all_finite), all_finite = fmaf(v.w, 0.f, all_finite);
   }
   if (__syncthreads_or(!(all_finite == 0.f))) {
-    exact_unit<KS, NT>(u.batch_begin, b_end, fin, fout, batches, pinfo, edges, W, X, (LdsF32*)yt, (LdsF32*)et, (LdsInt*)&turn);
+    exact_unit<KS, NT>(u.batch_begin, u.batch_end, fin, fout, batches, pinfo, edges, W, X, (LdsF32*)yt, (LdsF32*)et, (LdsInt*)&turn);
     unscale = 1.f;
   }
   // The tile's rows of Y are one stretch of memory.  A thread requests all it is about to add to before it

@@ -67,3 +67,41 @@ def test_chains_and_batches(dev, fin, fout, n):
     err = np.abs(got - want)
     assert np.all(err <= 1e-5 * np.abs(want) + 1e-5 * scale + 1e-6), f"worst {err.max():.3e}"
     assert np.linalg.norm(err) <= 1e-6 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("fin,fout", [(32, 32), (32, 64), (64, 32), (64, 64)])
+def test_stretches_of_batches(dev, fin, fout):
+    """Tiles of 1 to 20 batches, each of another relation or with two in a row of one, for workgroups of 4 and 8
+    wavefronts: fewer batches than wavefronts, as many, and every remainder."""
+    rng = np.random.default_rng(fin + fout)
+    tiles, R = 20, 20
+    n = 128 * (tiles + 1)
+
+    def lengths_of(r):
+        pick = {}
+        for t in range(r, tiles):  # tile t: relations 0 ... t
+            if t % 2 == 0 and r == t:
+                continue  # instead of the last relation a second batch of the one before
+            pairs = 17 if t % 2 == 0 and r == t - 1 else 1 + (r + t) % 16
+            for k in rng.choice(128, pairs, replace=False):
+                pick[128 * t + int(k)] = 1
+        if r < 10:  # a tile of many batches, and edges enough for the tile form
+            for k in range(128):
+                pick[128 * tiles + k] = 7
+        return pick
+
+    csf = _csf(rng, n, R, lengths_of)
+    assert len(csf[3]) >= 8192
+    a = rng.random(len(csf[3]), dtype=np.float32) - 0.3
+    x = rng.standard_normal((n, fin), dtype=np.float32)
+    w = rng.standard_normal((R, fout, fin), dtype=np.float32) * 0.1
+    t = lambda v: torch.from_numpy(np.ascontiguousarray(v)).to(dev)
+    f = ops.build_rgms_csf(n, n, R, fin, fout, len(csf[1]), len(csf[3]))
+    y = torch.full((n * fout,), 0.5, dtype=torch.float32, device=dev)
+    f(t(a), t(w.ravel()), t(x.ravel()), y, *[t(c) for c in csf])
+    got = y.cpu().numpy().reshape(n, fout) - np.float32(0.5)
+    wt = np.ascontiguousarray(w.transpose(0, 2, 1))
+    want = rgms_f64(*csf, a, x, wt, n)
+    scale = rgms_f64(*csf, np.abs(a), np.abs(x), np.abs(wt), n)
+    err = np.abs(got - want)
+    assert np.all(err <= 1e-5 * np.abs(want) + 1e-5 * scale + 1e-6), f"worst {err.max():.3e}"

@@ -368,12 +368,12 @@ __global__ __launch_bounds__(256) void f32_pack_w_kernel(const float* __restrict
   for (int k = 0; k < 3; ++k) Wp[(f * 3 + k) * 64 + lane] = term[k];
 }
 
-// The value that the lane of place K of the lane's own column holds (see my_place in the kernel).
-template <int KS, int K>
-__device__ __forceinline__ int at_place(int v) {
-  const int a = __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xf, 0xf, false);  // lane K of the row of 16
-  if constexpr (KS == 1) return __builtin_amdgcn_update_dpp(a, v, 0x150 + kChain + K, 0xf, 0xc, false);
-  return a;
+// The value of lane K of the lane's own four, which the compiler makes an operand of the instruction that takes it.
+// Broadcasts over eight lanes, as two instructions of their own, were a sixth of the loop's vector instructions
+// (2 M edges, 65 relations, us per call: 32 -> 8 52 / 50, 32 -> 32 63 / 61, 64 -> 32 107 / 104, 32 -> 64 97 / 95).
+template <int K>
+__device__ __forceinline__ uint32_t of_four(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, K * 0x55, 0xf, 0xf, true);
 }
 
 template <class F>
@@ -540,10 +540,8 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     r.rel = __builtin_amdgcn_readfirstlane(t.rel);
     return r;
   };
-  // Lane j of a row of 16 lanes holds the places of the lane groups in that row: two columns (KS = 1, lanes
-  // 8 ... 15 as lanes 0 ... 7) or one (KS = 2).  at_place<k> hands a lane the value of place k of its own
-  // column, by DPP broadcasts inside the row: no trip through LDS.
-  const int my_place = (lane >> 4) * (KS == 1 ? 2 * kChain : kChain) + (lane & (KS == 1 ? 2 * kChain - 1 : kChain - 1));
+  // Each four lanes hold the four places of their lane group's column, and a lane gets at them by DPP.
+  const int my_place = lane / CPR * kChain + (lane & (kChain - 1));
   auto load_record = [&](const Batch& bt) {
     return *reinterpret_cast<const u32x3*>(edges + (int64_t)bt.place_begin + min(my_place, max(bt.places - 1, 0)));
   };
@@ -561,8 +559,8 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     // no edge or no such inputs: behind the end of X, which reads as zeros
     const uint32_t off = live && rec.x != kUnused ? rec.x * row_bytes : kBehindX;
     static_for_chain([&](auto K) {
-      const uint32_t at = (uint32_t)at_place<KS, decltype(K)::value>((int)off);
-      r.x[K] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(Xr, (at + 16u * gc) | no_chunk, 0, 0));
+      const uint32_t at = of_four<decltype(K)::value>(off) + 16u * gc;
+      r.x[K] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(Xr, at | no_chunk, 0, 0));
     });
     return r;
   };
@@ -597,18 +595,20 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     // 1. the chains of this batch: a lane group adds up its column of weighted rows, and writes a row of the
     // chain tile wherever a chain ends
     f32x4 run = {0.f, 0.f, 0.f, 0.f};
-    const float own = kScale * rw.w;
+    const uint32_t own = __float_as_uint(kScale * rw.w);
+    const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)rw.chain, 8, 1);  // all bits: the sum goes on
+    const uint32_t to = 4u * __umul24(rw.chain & 255, SS);
     static_for_chain([&](auto K) {
-      const float w = __int_as_float(at_place<KS, decltype(K)::value>(__float_as_int(own)));
-      const uint32_t chain = (uint32_t)at_place<KS, decltype(K)::value>((int)rw.chain);
+      constexpr int k = decltype(K)::value;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        if constexpr (K == 0)
+        const float w = __uint_as_float(of_four<k>(own));
+        if constexpr (k == 0)
           run[c] = w * rw.x[K][c];
         else
-          run[c] = fmaf(w, rw.x[K][c], chain >= 256 ? run[c] : 0.f);
+          run[c] = fmaf(w, rw.x[K][c], __uint_as_float(of_four<k>(keep) & __float_as_uint(run[c])));
       }
-      *reinterpret_cast<f32x4*>(et + __umul24(chain & 255, SS) + 4 * gc) = run;
+      *reinterpret_cast<f32x4*>(reinterpret_cast<char*>(et + 4 * gc) + of_four<k>(to)) = run;
     });
     // 2. the sums of the pairs, multiplying layout: lane (i, q) adds the chains of pair i, mostly one; a lane
     // whose pair has fewer than the batch's longest reads the tile's row of zeros meanwhile
@@ -666,19 +666,22 @@ void rgms_f32_tile_kernel(int m, int fin, int fout, int total_batches, uint32_t 
     // order: the turn goes on after the tile is written.)
     while (__hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != my_turn) __builtin_amdgcn_s_sleep(1);
     asm volatile("" ::: "memory");
-    float* at[4];
+    struct alignas(4 * NT) Outs {
+      float v[NT];
+    };
+    Outs *at[4], sums[4];
+    const uint32_t row = 4 * FO * (pr & 255);
     static_for_chain([&](auto V) {
-      at[V] = yt + (__builtin_amdgcn_mov_dpp((int)pr, 0x150 + decltype(V)::value, 0xf, 0xf, false) & 255) * FO + NT * i;
+      at[V] = reinterpret_cast<Outs*>(reinterpret_cast<char*>(yt + NT * i) + of_four<decltype(V)::value>(row));
     });
-    float old[4][NT];
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+    for (int v = 0; v < 4; ++v) sums[v] = *at[v];
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) old[v][nt] = at[v][nt];
+    for (int v = 0; v < 4; ++v) {
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) at[v][nt] = old[v][nt] + acc[nt][v];
+      for (int nt = 0; nt < NT; ++nt) sums[v].v[nt] += acc[nt][v];
+      *at[v] = sums[v];
+    }
     asm volatile("" ::: "memory");
     __hip_atomic_store(&turn, my_turn + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     pw = next_pw, pr = next_pr;

@@ -36,11 +36,13 @@ struct TileIndex {
   size_t wpack_bytes = 0;
   // For the launch whose workgroups stay resident (W in LDS): the sorted edges cut into equal
   // shares of steps, one per team of wavefronts, each share a list of units.  Built at the first
-  // such launch and again when the number of teams changes.
+  // such launch with workgroups of 8 and at the first with 12 wavefronts.
   std::vector<int64_t> tile_begin;  // host copy: first sorted edge of every tile, then the edge count
-  int64_t share_teams = 0;
-  void* d_share_ptr = nullptr;    // share_teams + 1 offsets into d_share_units
-  void* d_share_units = nullptr;  // units x 16 bytes, grouped by team
+  struct Shares {
+    int64_t wgs = 0;          // workgroups of the launch
+    void* d_units = nullptr;  // units x 16 bytes, grouped by team; the allocation goes on with
+    void* d_ptr = nullptr;    // teams + 1 offsets into the units
+  } shares[2];
 };
 
 // The indices of a plan: one for all relations, or -- when W does not fit the LDS of a compute unit

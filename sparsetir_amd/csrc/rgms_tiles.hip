@@ -14,6 +14,7 @@
 #include "rgms_out.h"
 
 #include <hipcub/hipcub.hpp>
+#include <algorithm>
 #include <type_traits>
 
 
@@ -278,9 +279,9 @@ constexpr int kSStride = 40;  // 16-bit elements per row of the S tile (32 used;
 // (dl, jcol) of the wavefront's all-zero S tile, every lane reads its operand row, and the entry
 // is cleared again; LDS operations of one wavefront execute in order, so no barrier is needed.
 // Steps of at most 16 edges skip the second half of k.
-template <bool BF16, bool ONE_TERM>
-__device__ __forceinline__ f32x16 scatter_step(uint16_t* S, int dl, int jcol, int mrow, int h, uint16_t weight,
-                                               int left, const f32x16& acc1, f32x16 acc2) {
+template <bool BF16, bool ONE_TERM, int NT>
+__device__ __forceinline__ void scatter_step(uint16_t* S, int dl, int jcol, int mrow, int h, uint16_t weight, int left,
+                                             const f32x16 (&acc1)[NT], f32x16 (&acc2)[NT]) {
   if (h == 0) S[dl * kSStride + jcol] = weight;
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -290,26 +291,28 @@ __device__ __forceinline__ f32x16 scatter_step(uint16_t* S, int dl, int jcol, in
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   if (h == 0) S[dl * kSStride + jcol] = 0;
-  float t[16];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) t[v] = acc1[v];
-  acc2 = stage2<BF16, ONE_TERM>(sa0, t, acc2);
-  if (left > 16) acc2 = stage2<BF16, ONE_TERM>(sa1, t + 8, acc2);
-  return acc2;
+  for (int nt = 0; nt < NT; ++nt) {
+    float t[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) t[v] = acc1[nt][v];
+    acc2[nt] = stage2<BF16, ONE_TERM>(sa0, t, acc2[nt]);
+    if (left > 16) acc2[nt] = stage2<BF16, ONE_TERM>(sa1, t + 8, acc2[nt]);
+  }
 }
 
 // One workgroup per unit.  Its four wavefronts take the unit's steps in turn (wavefront w the
 // steps w, w + 4, ...: more wavefronts in flight per tile, since a step costs a full memory
 // round trip), each with its own accumulator tile; the four tiles are added through LDS and the
-// workgroup writes the 32 rows of Y once.  KK = feat_in / 16.
-template <int KK, bool BF16, typename Rec, typename YT>
+// workgroup writes the 32 rows of Y once.  KK = feat_in / 16; a pass is over NT tiles of 32 output features.
+template <int KK, int NT, bool BF16, typename Rec, typename YT>
 __global__ __launch_bounds__(64 * kUnitWaves) void rgms_tile_kernel(const Unit* __restrict__ units,
                                                         const Rec* __restrict__ edges, int m, int feat_out,
                                                         const u32x4* __restrict__ Wp, const uint16_t* __restrict__ X,
                                                         YT* __restrict__ Y) {
   constexpr int FIN = KK * 16;
   constexpr bool kPacked = sizeof(Rec) == sizeof(PackedEdge);
-  constexpr int PW = KK <= 4 ? 2 : 1;  // relations whose W fragments are requested together
+  constexpr int PW = KK * NT <= 4 ? 2 : 1;  // relations whose W fragments are requested together
   constexpr int kThreads = 64 * kUnitWaves, kSumIters = kTileRows * 32 / kThreads;
   __shared__ __attribute__((aligned(16))) uint16_t s_all[kUnitWaves][kTileRows * kSStride];
   __shared__ float partial[kUnitWaves][16 * 64];  // [wavefront][accumulator register][lane]
@@ -332,10 +335,12 @@ __global__ __launch_bounds__(64 * kUnitWaves) void rgms_tile_kernel(const Unit* 
   const int64_t e_end = u.edge_begin + u.edge_count;
   const int tile = u.tile_flag >> 1;
 
-  for (int nti = 0; nti < ntiles; ++nti) {
-    f32x16 acc2;
+  for (int nti = 0; nti < ntiles; nti += NT) {
+    f32x16 acc2[NT];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc2[v] = 0.f;
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc2[nt][v] = 0.f;
     // lanes past the last edge repeat it with weight zero
     constexpr int64_t kStride = kUnitWaves * kStepEdges;  // edges between a wavefront's steps
     Rec next = edges[min(u.edge_begin + wave * kStepEdges + mrow, e_end - 1)];
@@ -364,7 +369,7 @@ __global__ __launch_bounds__(64 * kUnitWaves) void rgms_tile_kernel(const Unit* 
       // every load of the step is requested here; the records of the step after the next go
       // last, so that waiting for the operands leaves them in flight (loads retire in order, so
       // they have until the next step's operands are waited for)
-      u32x4 xa[KK], wf[PW][KK];
+      u32x4 xa[KK], wf[PW][NT * KK];
       const uint16_t* xp = X + (int64_t)cur.src * FIN + 8 * h;
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) xa[kk] = *reinterpret_cast<const u32x4*>(xp + 16 * kk);
@@ -378,81 +383,90 @@ __global__ __launch_bounds__(64 * kUnitWaves) void rgms_tile_kernel(const Unit* 
         if (r[q] >= 0) {
           const u32x4* w = Wp + (uint32_t)((r[q] * ntiles + nti) * (KK * 64) + lane);
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) wf[q][kk] = w[kk * 64];
+          for (int f = 0; f < NT * KK; ++f) wf[q][f] = w[f * 64];
         }
       }
       after = edges[min(e0 + 2 * kStride + mrow, e_end - 1)];  // past the end: the last record again
 
       // ---- stage 1
-      f32x16 acc1;
+      f32x16 acc1[NT];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc1[v] = 0.f;  // a constant operand of the first MFMA, not 16 moves
-      auto add_run = [&](int rq, const u32x4* w, f32x16 c) {
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc1[nt][v] = 0.f;  // a constant operand of the first MFMA, not 16 moves
+      auto add_run = [&](int rq, const u32x4* w) {
         const bool sel = rel == rq;
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
           u32x4 a;
 #pragma unroll
           for (int d = 0; d < 4; ++d) a[d] = sel ? xa[kk][d] : 0u;
-          c = mfma32<BF16>(a, w[kk], c);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc1[nt] = mfma32<BF16>(a, w[nt * KK + kk], acc1[nt]);
         }
-        return c;
       };
       bool single = pos >= kStepEdges;  // the requested runs cover the step ...
       if constexpr (PW > 1) single = single && r[1] < 0;  // ... and the first one does so alone
       if (single) {
         // one relation in the whole step: nothing to mask
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) acc1 = mfma32<BF16>(xa[kk], wf[0][kk], acc1);
+        for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc1[nt] = mfma32<BF16>(xa[kk], wf[0][nt * KK + kk], acc1[nt]);
       } else {
-        acc1 = add_run(r[0], wf[0], acc1);
+        add_run(r[0], wf[0]);
 #pragma unroll
         for (int q = 1; q < PW; ++q)
-          if (r[q] >= 0) acc1 = add_run(r[q], wf[q], acc1);
+          if (r[q] >= 0) add_run(r[q], wf[q]);
       }
       while (pos < kStepEdges) {  // steps with more than PW relations: one at a time
         const int rq = __builtin_amdgcn_readlane(rel, pos);
         pos += __popcll(__ballot(rel == rq) & 0xffffffffull);
         const u32x4* w = Wp + (uint32_t)((rq * ntiles + nti) * (KK * 64) + lane);
-        u32x4 wl[KK];
+        u32x4 wl[NT * KK];
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) wl[kk] = w[kk * 64];
-        acc1 = add_run(rq, wl, acc1);
+        for (int f = 0; f < NT * KK; ++f) wl[f] = w[f * 64];
+        add_run(rq, wl);
       }
 
       // ---- stage 2
-      acc2 = scatter_step<BF16, std::is_same<YT, _Float16>::value>(S, dl, jcol, mrow, h, live ? wbits : (uint16_t)0, left, acc1, acc2);
+      scatter_step<BF16, std::is_same<YT, _Float16>::value>(S, dl, jcol, mrow, h, live ? wbits : (uint16_t)0, left, acc1, acc2);
     }
 
-    // ---- add the four tiles and write back.  acc2[v] of lane (n, h) is row (v%4) + 4h + 8(v/4)
-    // of the tile, output feature 32 nti + n.
-#pragma unroll
-    for (int v = 0; v < 16; ++v) partial[wave][v * 64 + lane] = acc2[v];
+    // ---- add the four tiles and write back.  acc2[nt][v] of lane (n, h) is row (v%4) + 4h + 8(v/4)
+    // of the tile, output feature 32 (nti + nt) + n.
     const bool atomic = u.tile_flag & 1;
-    float yold[kSumIters];  // requested before the barrier
+    float yold[NT][kSumIters];  // requested before the barriers
 #pragma unroll
-    for (int k = 0; k < kSumIters; ++k) {
-      const int elem = threadIdx.x + kThreads * k;
-      const int64_t yrow = (int64_t)tile * kTileRows + (elem >> 5);
-      yold[k] = (!atomic && yrow < m) ? y_load(Y + yrow * feat_out + 32 * nti + (elem & 31)) : 0.f;
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int k = 0; k < kSumIters; ++k) {
+        const int elem = threadIdx.x + kThreads * k;
+        const int64_t yrow = (int64_t)tile * kTileRows + (elem >> 5);
+        yold[nt][k] = (!atomic && yrow < m) ? y_load(Y + yrow * feat_out + 32 * (nti + nt) + (elem & 31)) : 0.f;
+      }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) partial[wave][v * 64 + lane] = acc2[nt][v];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kSumIters; ++k) {
+        const int elem = threadIdx.x + kThreads * k, row = elem >> 5, col = elem & 31;
+        const int at = ((row & 3) + 4 * (row >> 3)) * 64 + col + 32 * ((row >> 2) & 1);
+        float sum = partial[0][at];
+#pragma unroll
+        for (int w = 1; w < kUnitWaves; ++w) sum += partial[w][at];
+        const int64_t yrow = (int64_t)tile * kTileRows + row;
+        // (a row belongs to 32 consecutive threads: the two lanes of a pair share `yrow`)
+        YT* y = Y + yrow * feat_out + 32 * (nti + nt) + col;
+        if (atomic)  // uniform over the workgroup
+          y_atomic_add(y, sum, yrow < m, threadIdx.x);
+        else if (yrow < m)
+          y_store(y, yold[nt][k] + sum);
+      }
+      if (nt + 1 < NT || nti + NT < ntiles) __syncthreads();  // the partial sums are rewritten
     }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kSumIters; ++k) {
-      const int elem = threadIdx.x + kThreads * k, row = elem >> 5, col = elem & 31;
-      const int at = ((row & 3) + 4 * (row >> 3)) * 64 + col + 32 * ((row >> 2) & 1);
-      float sum = partial[0][at];
-#pragma unroll
-      for (int w = 1; w < kUnitWaves; ++w) sum += partial[w][at];
-      const int64_t yrow = (int64_t)tile * kTileRows + row;
-      // (a row belongs to 32 consecutive threads: the two lanes of a pair share `yrow`)
-      YT* y = Y + yrow * feat_out + 32 * nti + col;
-      if (atomic)  // uniform over the workgroup
-        y_atomic_add(y, sum, yrow < m, threadIdx.x);
-      else if (yrow < m)
-        y_store(y, yold[k] + sum);
-    }
-    if (nti + 1 < ntiles) __syncthreads();  // the partial sums are rewritten by the next pass
   }
 }
 
@@ -478,7 +492,7 @@ constexpr int kTeamWaves = 2;  // wavefronts that share a unit in the resident k
 // distinct banks, and so do the eight writers of one column phase (see the fill loop)
 __device__ __forceinline__ int w_slot(int lane) { return lane ^ ((lane >> 3) & 7); }
 
-template <int KK, bool BF16, typename Rec, int T, typename YT>
+template <int KK, int NT, bool BF16, typename Rec, int T, typename YT>
 __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
     const int32_t* __restrict__ share_ptr, const Unit* __restrict__ share_units, const Rec* __restrict__ edges, int m,
     int feat_out, int num_rels, const uint16_t* __restrict__ W, const uint16_t* __restrict__ X,
@@ -516,7 +530,7 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
       x[kk] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const unsigned char*>(X) + at + 32 * kk);
     wb = weight_of(rec);
   };
-  // What a pass (one unit, one tile of 32 output features) starts from: the records of the
+  // What a pass (one unit, NT tiles of 32 output features) starts from: the records of the
   // wavefront's first three steps and the rows of X of the first.  The records are requested when
   // the pass before begins and the rows when its last step is done, so that a pass does not open
   // with two memory round trips; unit descriptors are read two units ahead for the same reason.
@@ -609,22 +623,26 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
     const int tile = u.tile_flag >> 1;
     const bool atomic = u.tile_flag & 1;
 
-    for (int nti = 0; nti < ntiles; ++nti) {
-      // The next pass: the same unit at the next feature tile, or the next unit.
-      const bool next_pass = nti + 1 < ntiles || more_units;
+    for (int nti = 0; nti < ntiles; nti += NT) {
+      // The next pass: the same unit at the next feature tiles, or the next unit.
+      const bool next_pass = nti + NT < ntiles || more_units;
       Rec p0 = cur, p1 = cur, p2 = cur;
-      if (next_pass) first_records(nti + 1 < ntiles ? u : u1, p0, p1, p2);
+      if (next_pass) first_records(nti + NT < ntiles ? u : u1, p0, p1, p2);
       // What the wavefront's 16 rows of the tile hold now, in accumulator layout (register v of lane
       // (n, h) is row 16 tw + (v%4) + 4h + 8(v/4), feature n); needed at the end only.
-      float yold[8];
+      float yold[NT][8];
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int64_t yrow = (int64_t)tile * kTileRows + 16 * tw + (v & 3) + 4 * h + 8 * (v >> 2);
-        yold[v] = (!atomic && yrow < m) ? y_load(Y + yrow * feat_out + 32 * nti + mrow) : 0.f;
-      }
-      f32x16 acc2;
+      for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc2[v] = 0.f;
+        for (int v = 0; v < 8; ++v) {
+          const int64_t yrow = (int64_t)tile * kTileRows + 16 * tw + (v & 3) + 4 * h + 8 * (v >> 2);
+          yold[nt][v] = (!atomic && yrow < m) ? y_load(Y + yrow * feat_out + 32 * (nti + nt) + mrow) : 0.f;
+        }
+      f32x16 acc2[NT];
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc2[nt][v] = 0.f;
       auto step = [&](const Rec& rec, const u32x4 (&x)[KK], uint16_t wbits, int e0) {
         const int left = min(kStepEdges, e_end - e0);  // uniform
         const bool live = mrow < left;
@@ -635,18 +653,22 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
           rel = (int)(rec.rel_dl >> 5), dl = (int)(rec.rel_dl & 31);
 
         // ---- stage 1: one MFMA chain per run of equal relation (the step is sorted by relation)
-        f32x16 acc1;
+        f32x16 acc1[NT];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc1[v] = 0.f;  // a constant operand of the first MFMA, not 16 moves
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc1[nt][v] = 0.f;  // a constant operand of the first MFMA, not 16 moves
         int rq = __builtin_amdgcn_readlane(rel, 0);
         int pos_e = __popcll(__ballot(rel == rq) & 0xffffffffull);
         if (pos_e >= kStepEdges) {
           // one relation in the whole step: nothing to mask
           const u32x4* w = Wl + (rq * ntiles + nti) * (KK * 64) + slot;
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) acc1 = mfma32<BF16>(x[kk], w[kk * 64], acc1);
+          for (int kk = 0; kk < KK; ++kk)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc1[nt] = mfma32<BF16>(x[kk], w[(nt * KK + kk) * 64], acc1[nt]);
         } else {
-          auto add_run = [&](int r_, f32x16 c) {
+          auto add_run = [&](int r_) {
             const u32x4* w = Wl + (r_ * ntiles + nti) * (KK * 64) + slot;
             const bool sel = rel == r_;
 #pragma unroll
@@ -654,21 +676,21 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
               u32x4 a_;
 #pragma unroll
               for (int d = 0; d < 4; ++d) a_[d] = sel ? x[kk][d] : 0u;
-              c = mfma32<BF16>(a_, w[kk * 64], c);
+#pragma unroll
+              for (int nt = 0; nt < NT; ++nt) acc1[nt] = mfma32<BF16>(a_, w[(nt * KK + kk) * 64], acc1[nt]);
             }
-            return c;
           };
-          acc1 = add_run(rq, acc1);
+          add_run(rq);
           do {
             rq = __builtin_amdgcn_readlane(rel, pos_e);
             pos_e += __popcll(__ballot(rel == rq) & 0xffffffffull);
-            acc1 = add_run(rq, acc1);
+            add_run(rq);
           } while (pos_e < kStepEdges);
         }
 
         // ---- stage 2
         if (e0 == e_first) team_wait();  // the sums of the pass before have been read out of the S tiles
-        acc2 = scatter_step<BF16, std::is_same<YT, _Float16>::value>(S, dl, jcol, mrow, h, live ? wbits : (uint16_t)0, left, acc1, acc2);
+        scatter_step<BF16, std::is_same<YT, _Float16>::value>(S, dl, jcol, mrow, h, live ? wbits : (uint16_t)0, left, acc1, acc2);
       };
       // Two steps per turn of the loop, so that the two sets of X registers swap roles without
       // copies: while a step is computed, the rows of X of the step after it are on their way,
@@ -688,7 +710,9 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
       // Everything requested so far has had the whole pass to arrive.  Naming the old values of
       // Y here settles them, so that the stores below do not wait for the loads that follow.
 #pragma unroll
-      for (int v = 0; v < 8; ++v) asm volatile("" : "+v"(yold[v]));
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int v = 0; v < 8; ++v) asm volatile("" : "+v"(yold[nt][v]));
       if (next_pass) {
         cur = p0, nx1 = p1, nx2 = p2;
         fetch(cur, xa, wa);
@@ -698,32 +722,39 @@ __global__ __launch_bounds__(64 * kTeamWaves * T) void rgms_tile_lds_kernel(
       // ---- teams of two: each wavefront owns 16 rows of the tile (eight accumulator registers),
       // hands the other eight to its partner through LDS and writes its rows back from registers.
       float* theirs = reinterpret_cast<float*>(team_lds + (1 - tw) * kSBytes);
-      if (tw == 0) {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) my_partial[v * 64 + lane] = acc2[8 + v];
-      } else {
+      for (int nt = 0; nt < NT; ++nt) {
+        if (nt > 0) team_barrier();  // the partner has read the tile before
+        if (tw == 0) {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) my_partial[v * 64 + lane] = acc2[v];
-      }
-      team_barrier();
-      float own[8];
-      if (tw == 0) {
+          for (int v = 0; v < 8; ++v) my_partial[v * 64 + lane] = acc2[nt][8 + v];
+        } else {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) own[v] = acc2[v] + theirs[v * 64 + lane];
-      } else {
+          for (int v = 0; v < 8; ++v) my_partial[v * 64 + lane] = acc2[nt][v];
+        }
+        team_barrier();
+        float own[8];
+        if (tw == 0) {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) own[v] = acc2[8 + v] + theirs[v * 64 + lane];
-      }
+          for (int v = 0; v < 8; ++v) own[v] = acc2[nt][v] + theirs[v * 64 + lane];
+        } else {
 #pragma unroll
-      for (int v = 0; v < 8; ++v) theirs[v * 64 + lane] = 0.f;  // the partner's S tile is all zeros again
+          for (int v = 0; v < 8; ++v) own[v] = acc2[nt][8 + v] + theirs[v * 64 + lane];
+        }
+        if (nt + 1 == NT) {
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int64_t yrow = (int64_t)tile * kTileRows + 16 * tw + (v & 3) + 4 * h + 8 * (v >> 2);
-        YT* y = Y + yrow * feat_out + 32 * nti + mrow;  // lanes 2k and 2k + 1: the same row, features 2k, 2k + 1
-        if (atomic)  // uniform over the wavefront
-          y_atomic_add(y, own[v], yrow < m, lane);
-        else if (yrow < m)
-          y_store(y, yold[v] + own[v]);
+          for (int v = 0; v < 8; ++v) theirs[v * 64 + lane] = 0.f;  // the partner's S tile is all zeros again
+        }
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+          const int64_t yrow = (int64_t)tile * kTileRows + 16 * tw + (v & 3) + 4 * h + 8 * (v >> 2);
+          // lanes 2k and 2k + 1: the same row, features 2k, 2k + 1
+          YT* y = Y + yrow * feat_out + 32 * (nti + nt) + mrow;
+          if (atomic)  // uniform over the wavefront
+            y_atomic_add(y, own[v], yrow < m, lane);
+          else if (yrow < m)
+            y_store(y, yold[nt][v] + own[v]);
+        }
       }
       team_arrive();  // waited for where the next pass first writes to its S tile
     }
@@ -752,17 +783,28 @@ int bit_length(uint64_t x) {
 // LDS beside W).  16 would leave 128 registers per wavefront, which the kernel only just fits or
 // spills, and measured no faster where W left the room (60 relations of 32 x 32).
 constexpr int kResidentMaxQuads = 3;
+// Two tiles of 32 output features in a pass (NT = 2) where there is an even number of them: the rows of X, the records,
+// the masks of the runs and the S tiles serve both.  The resident kernel then has 8 wavefronts (12 spill 2 to 29
+// registers), the kernel that reads W from memory keeps to one tile above 48 inputs (registers for two wavefronts per
+// SIMD, 342 k edges, 65 relations, 64 -> 64: 42 / 47 us).  us with one / two tiles, 100 k nodes, 2 M edges:
+// resident, 8 relations 16 -> 64 44 / 41, 32 -> 64 56 / 46, 64 -> 64 80 / 57; W from memory, 130 relations, 16 -> 64
+// 78 / 73, 32 -> 64 127 / 112; 19 k nodes, 342 k edges: 8 relations, 64 -> 64 23.5 / 19.7; 65, 32 -> 64 28.0 / 25.1.
+constexpr int kTwoTilesMaxKK = 3;
+inline bool even_tiles(int feat_out) { return feat_out % 64 == 0; }
+inline int resident_max_quads(int feat_out) { return even_tiles(feat_out) ? 2 : kResidentMaxQuads; }
 // W beyond the LDS: two ranges of relations with a launch each when the edges make up for the second launch
 // and its fill of the LDS, else W is read from memory in one launch.  Two launches / one, us:
-//   40 k nodes, 280 k edges, 50 relations 32 -> 64: 64 / 39; 720 k edges, 90 relations 32 -> 32: 35.6 / 31.6;
-//   110 k nodes, 880 k edges, 24 relations 64 -> 64: 81 / 88; 1.98 M edges, 90 relations 32 -> 32: 57 / 65.
-// Three launches are never the faster form (65 relations 32 -> 64: 77 / 22 at 144 k edges, 116 / 111 at 1.98 M).
+//   40 k nodes, 700 k edges, 65 relations 32 -> 64: 44 / 39; 720 k edges, 90 relations 32 -> 32: 35.6 / 31.6;
+//   60 k, 1 M, 65 relations 32 -> 64: 51 / 54; 24 relations 64 -> 64: 50 / 71; 100 k, 2 M, 65 relations 32 -> 64:
+//   77 / 88; 110 k, 1.98 M edges, 90 relations 32 -> 32: 57 / 65.
+// Three launches were not the faster form (one tile to a pass, 65 relations 32 -> 64: 77 / 22 at 144 k edges, 116 / 111
+// at 1.98 M).
 constexpr int kMaxRelationParts = 2;
 // (fewer edges suffice where a relation's W is large, 64 -> 32 and up: every run of a step fetches it)
 inline int64_t relation_parts_slots(int feat_in, int feat_out) { return feat_in * feat_out >= 2048 ? 850000 : 1300000; }
 
 // Launches the resident kernel with `quads` x 4 wavefronts per workgroup.
-template <int KK, bool BF16, typename Rec, typename YT>
+template <int KK, int NT, bool BF16, typename Rec, typename YT>
 int launch_resident(int quads, dim3 grid, size_t lds, hipStream_t stream, const int32_t* share_ptr,
                     const Unit* share_units, const Rec* edges, int m, int feat_out, int num_rels, const uint16_t* W,
                     const uint16_t* X, YT* Y) {
@@ -773,9 +815,24 @@ int launch_resident(int quads, dim3 grid, size_t lds, hipStream_t stream, const 
     return 0;
   };
   constexpr int kTeamsPerQuad = 4 / kTeamWaves;
-  if (quads == 2) return go(rgms_tile_lds_kernel<KK, BF16, Rec, 2 * kTeamsPerQuad, YT>);
-  if (quads == 3) return go(rgms_tile_lds_kernel<KK, BF16, Rec, 3 * kTeamsPerQuad, YT>);
+  if (quads == 2) return go(rgms_tile_lds_kernel<KK, NT, BF16, Rec, 2 * kTeamsPerQuad, YT>);
+  if constexpr (NT == 1)
+    if (quads == 3) return go(rgms_tile_lds_kernel<KK, NT, BF16, Rec, 3 * kTeamsPerQuad, YT>);
   return fail("rgms: no kernel for %d wavefronts per workgroup", 4 * quads);
+}
+
+template <int KK, bool BF16, typename Rec, typename YT>
+void launch_memory_w(dim3 grid, dim3 block, hipStream_t stream, const Unit* units, const Rec* edges, int m,
+                     int feat_out, const u32x4* Wp, const uint16_t* X, YT* Y) {
+  if constexpr (KK <= kTwoTilesMaxKK) {
+    if (even_tiles(feat_out)) {
+      hipLaunchKernelGGL((rgms_tile_kernel<KK, 2, BF16, Rec, YT>), grid, block, 0, stream, units, edges, m, feat_out,
+                         Wp, X, Y);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((rgms_tile_kernel<KK, 1, BF16, Rec, YT>), grid, block, 0, stream, units, edges, m, feat_out, Wp,
+                     X, Y);
 }
 
 // What a unit costs a team beyond its steps (exchanging half of the tile with the partner, writing
@@ -786,7 +843,12 @@ constexpr int64_t kUnitOverheadSteps = 3;
 // tile is its steps plus the overhead above.  A tile that lies inside one share is a unit that
 // writes its rows of Y alone; the pieces of a tile that is cut by a share boundary all add with
 // atomics.  A boundary that falls into the overhead part of a tile moves to the tile's start.
-int build_shares(TileIndex& ix, int64_t teams, hipStream_t stream) {
+int build_shares(TileIndex& ix, int quads, hipStream_t stream) {
+  const int per_wg = 4 * quads / kTeamWaves;
+  // one workgroup per compute unit, fewer when a team would get less than a handful of steps
+  const int64_t steps_bound = ix.edges / kStepEdges + (int64_t)ix.tile_begin.size();
+  const int64_t wgs = std::min<int64_t>(std::max(1, compute_units()), ceil_div(steps_bound, (int64_t)per_wg * 8));
+  const int64_t teams = wgs * per_wg;
   const int64_t tiles = (int64_t)ix.tile_begin.size() - 1;
   // cost coordinate: tile t occupies [at[t], at[t + 1]), its overhead first, then its steps
   std::vector<int64_t> at(size_t(tiles + 1), 0);
@@ -824,16 +886,15 @@ int build_shares(TileIndex& ix, int64_t teams, hipStream_t stream) {
   }
   ptr[teams] = (int32_t)units.size();
   STIR_REQUIRE(units.size() < (size_t(1) << 31), "rgms: too many units");
-  if (ix.d_share_ptr) STIR_HIP(hipFree(ix.d_share_ptr));
-  if (ix.d_share_units) STIR_HIP(hipFree(ix.d_share_units));
-  ix.d_share_ptr = ix.d_share_units = nullptr;
-  ix.share_teams = 0;
-  STIR_HIP(hipMalloc(&ix.d_share_ptr, sizeof(int32_t) * ptr.size()));
-  STIR_HIP(hipMalloc(&ix.d_share_units, sizeof(Unit) * std::max<size_t>(units.size(), 1)));
-  STIR_HIP(hipMemcpyAsync(ix.d_share_ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice, stream));
-  STIR_HIP(hipMemcpyAsync(ix.d_share_units, units.data(), sizeof(Unit) * units.size(), hipMemcpyHostToDevice, stream));
+  const size_t unit_bytes = sizeof(Unit) * units.size(), ptr_bytes = sizeof(int32_t) * ptr.size();
+  DevBuf mem;
+  STIR_HIP(mem.alloc(unit_bytes + ptr_bytes));
+  char* base = static_cast<char*>(mem.p);
+  STIR_HIP(hipMemcpyAsync(base, units.data(), unit_bytes, hipMemcpyHostToDevice, stream));
+  STIR_HIP(hipMemcpyAsync(base + unit_bytes, ptr.data(), ptr_bytes, hipMemcpyHostToDevice, stream));
   STIR_HIP(hipStreamSynchronize(stream));  // the host vectors go away
-  ix.share_teams = teams;
+  mem.p = nullptr;
+  ix.shares[quads - 2] = {wgs, base, base + unit_bytes};
   return 0;
 }
 
@@ -844,10 +905,11 @@ int tile_index_build(TileIndex& ix, const std::vector<TileBucket>& buckets, int3
   const bool packed = static_weights && num_rels <= kPackedMaxRels;
   if (ix.d_edges) STIR_HIP(hipFree(ix.d_edges));
   if (ix.d_units) STIR_HIP(hipFree(ix.d_units));
-  if (ix.d_share_ptr) STIR_HIP(hipFree(ix.d_share_ptr));
-  if (ix.d_share_units) STIR_HIP(hipFree(ix.d_share_units));
-  ix.d_edges = ix.d_units = ix.d_share_ptr = ix.d_share_units = nullptr;
-  ix.share_teams = 0;
+  for (TileIndex::Shares& sh : ix.shares) {
+    if (sh.d_units) STIR_HIP(hipFree(sh.d_units));
+    sh = {};
+  }
+  ix.d_edges = ix.d_units = nullptr;
   ix.tile_begin.clear();
   ix.m = -1;
   ix.edges = ix.units = 0;
@@ -1005,23 +1067,34 @@ int tile_rgms_launch(bool bf16, bool out16, TileIndex& ix, int32_t feat_in, int3
   if (kk_count <= kLdsMaxKK && reinterpret_cast<uintptr_t>(d_W) % 16 == 0 &&
       (int64_t)ix.n * feat_in * 2 < (int64_t(1) << 32)) {
     const size_t lds_limit = lds_bytes_per_workgroup();
-    for (int q = kResidentMaxQuads; q >= 2 && quads == 0; --q)
+    for (int q = resident_max_quads(feat_out); q >= 2 && quads == 0; --q)
       if (w_bytes + size_t(q) * 4 * kSBytes <= lds_limit) quads = q;
   }
   if (quads) {
-    const int teams = quads * 4 / kTeamWaves;  // per workgroup
+    bool two = even_tiles(feat_out);
+    if (!ix.shares[quads - 2].d_units) {
+      // nothing can be built while the stream is recorded: the other shares then, if there are any, with a kernel
+      // that has both workgroup sizes
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      STIR_HIP(hipStreamIsCapturing(stream, &capture));
+      const int other = 5 - quads;
+      if (capture != hipStreamCaptureStatusNone && ix.shares[other - 2].d_units &&
+          w_bytes + size_t(other) * 4 * kSBytes <= lds_bytes_per_workgroup())
+        quads = other, two = false;
+      else if (int rc = build_shares(ix, quads, stream))
+        return rc;
+    }
     const size_t lds = w_bytes + size_t(quads) * 4 * kSBytes;
-    // one workgroup per compute unit, fewer when a team would get less than a handful of steps
-    const int64_t steps_bound = ix.edges / kStepEdges + (int64_t)ix.tile_begin.size();
-    const int64_t wgs = std::min<int64_t>(std::max(1, compute_units()), ceil_div(steps_bound, (int64_t)teams * 8));
-    if (ix.share_teams != wgs * teams)
-      if (int rc = build_shares(ix, wgs * teams, stream)) return rc;
-    const dim3 grid((unsigned)wgs);
-    const int32_t* share_ptr = static_cast<const int32_t*>(ix.d_share_ptr);
-    const Unit* share_units = static_cast<const Unit*>(ix.d_share_units);
+    const TileIndex::Shares& shares = ix.shares[quads - 2];
+    const dim3 grid((unsigned)shares.wgs);
+    const int32_t* share_ptr = static_cast<const int32_t*>(shares.d_ptr);
+    const Unit* share_units = static_cast<const Unit*>(shares.d_units);
 #define STIR_LDS_R(KKV, BF, REC, PTR, YP)                                                               \
-  if (int rc = launch_resident<KKV, BF, REC>(quads, grid, lds, stream, share_ptr, share_units, PTR, ix.m, feat_out, \
-                                             ix.num_rels, W, X, YP))                                       \
+  if (int rc = two                                                                                             \
+                   ? launch_resident<KKV, 2, BF, REC>(quads, grid, lds, stream, share_ptr, share_units, PTR, ix.m,  \
+                                                      feat_out, ix.num_rels, W, X, YP)                     \
+                   : launch_resident<KKV, 1, BF, REC>(quads, grid, lds, stream, share_ptr, share_units, PTR, ix.m,  \
+                                                      feat_out, ix.num_rels, W, X, YP))                    \
     return rc
 #define STIR_LDS_Y(KKV, REC, PTR)                           \
   if (out16) {                                              \
@@ -1065,8 +1138,8 @@ int tile_rgms_launch(bool bf16, bool out16, TileIndex& ix, int32_t feat_in, int3
                      W, Wp, frags, kk_count, feat_out);
   STIR_LAUNCH_CHECK();
   const dim3 grid((unsigned)ix.units), block(64 * kUnitWaves);
-#define STIR_TILES_R(KKV, BF, REC, PTR, YT, YP) \
-  hipLaunchKernelGGL((rgms_tile_kernel<KKV, BF, REC, YT>), grid, block, 0, stream, units, PTR, ix.m, feat_out, Wp, X, YP)
+#define STIR_TILES_R(KKV, BF, REC, PTR, YT, YP)                                                                     \
+  launch_memory_w<KKV, BF, REC, YT>(grid, block, stream, units, PTR, ix.m, feat_out, Wp, X, YP)
 #define STIR_TILES_Y(KKV, REC, PTR)                       \
   if (out16)                                              \
     STIR_TILES_R(KKV, false, REC, PTR, _Float16, Y16);    \
@@ -1105,8 +1178,8 @@ void tile_index_free(TileIndex& ix) {
   if (ix.d_edges) (void)hipFree(ix.d_edges);
   if (ix.d_units) (void)hipFree(ix.d_units);
   if (ix.d_wpack) (void)hipFree(ix.d_wpack);
-  if (ix.d_share_ptr) (void)hipFree(ix.d_share_ptr);
-  if (ix.d_share_units) (void)hipFree(ix.d_share_units);
+  for (TileIndex::Shares& sh : ix.shares)
+    if (sh.d_units) (void)hipFree(sh.d_units);
   ix = TileIndex();
 }
 
@@ -1128,8 +1201,9 @@ int tile_set_prepare(TileIndexSet& set, const std::vector<TileBucket>& buckets, 
     const size_t rel_bytes = size_t(feat_out / 32) * (feat_in / 16) * 64 * sizeof(u32x4);
     const size_t lds_limit = lds_bytes_per_workgroup();
     auto fit = [&](int quads) { return (int64_t)((lds_limit - size_t(quads) * 4 * kSBytes) / rel_bytes); };
-    if (num_rels > fit(2) && fit(kResidentMaxQuads) > 0) {
-      const int64_t parts = ceil_div((int64_t)num_rels, fit(kResidentMaxQuads));
+    const int quads = resident_max_quads(feat_out);
+    if (num_rels > fit(2) && fit(quads) > 0) {
+      const int64_t parts = ceil_div((int64_t)num_rels, fit(quads));
       if (parts <= kMaxRelationParts && slots >= relation_parts_slots(feat_in, feat_out))
         per_part = (int32_t)ceil_div((int64_t)num_rels, parts);
     }

@@ -1003,10 +1003,12 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // two 32-row slices per workgroup when the block height allows it
   const int rs = (blk % 64 == 0) ? 2 : 1;
   const int64_t slices = (int64_t)mb * (blk / (32 * rs));
-  // Two 32-wide accumulators per wavefront once the feature axis is wide enough to still yield
-  // several workgroups per CU.  One prefetched step is enough: measured on MI355X, deeper
+  // Two 32-wide accumulators per wavefront once the feature axis is wide enough to still yield workgroups for the chip,
+  // 1.6 per CU (us with one / two): 22 x 246 blocks of 64, 2752 features (242 workgroups of two) 56 / 63, 45 x 45 of 128,
+  // 1024 (360) 20.6 / 21.6, 64 x 400 of 32, 1536 (384) 38.0 / 41.1, 60 x 100 of 64, 2048 (480) 26.0 / 24.5, 70 x 60
+  // (560) 34.4 / 29.6, 98 x 90, 2432 (980) 45.8 / 38.6.  One prefetched step is enough: measured on MI355X, deeper
   // register rings (2-6 steps) change nothing, the kernel is not bound by latency.
-  const int nt = (feat >= 1024) ? 2 : 1;
+  const int nt = feat >= 1024 && slices * stir::ceil_div(feat, 2 * kTileF) * 5 >= 8 * (int64_t)cus ? 2 : 1;
   const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
   dim3 block(256);
   // Where the X rows of a feature tile are more than an XCD's L2 holds beside A (x_tile_bytes), the slices are taken in
@@ -1033,7 +1035,10 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an
   // XCD on one slice of X, is worth more.
   const int sub_rows = blk / (32 * rs);
-  const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2) ? 1 : 0;
+  // Few block rows do not go round eight XCDs: 12 block rows (40 x 128 columns, 3008 features) 30.8 us, 26.3 in the
+  // other order; 20 (of 20, 4096) 33.4, 29.1; 45 (of 45, 1024) 21.6, 24.1.
+  const bool rows_go_round = 8 * stir::ceil_div((int64_t)mb, 8) * 7 <= 8 * (int64_t)mb;
+  const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2 && rows_go_round) ? 1 : 0;
   const int64_t blocks = by_rows ? 8 * stir::ceil_div((int64_t)mb, 8) * sub_rows * f_tiles
                                  : grid_of(slices, f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");

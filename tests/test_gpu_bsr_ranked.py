@@ -30,7 +30,10 @@ def _config(mb, nb, blk, density, feat, seed):
     (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles
     (343, 200, 32, 0.01, 736),
     (20, 200, 64, 0.03, 96),       # four wavefronts per 64 rows
-    (12, 100, 128, 0.05, 160),     # block rows dealt to XCDs
+    (12, 100, 128, 0.05, 160),     # too few block rows to deal them to XCDs
+    (14, 100, 128, 0.05, 160),     # block rows dealt to XCDs
+    (40, 20, 64, 0.1, 1056),       # few workgroups: 128 features each
+    (83, 20, 64, 0.1, 1056),       # as many as take 256 features each, the last with 32
     (1, 6200, 32, 0.001, 64),
     (1030, 90, 16, 0.02, 224),     # 16-row slices by a wavefront each: plain order
     (1024, 400, 16, 0.004, 512),   # ranked, 256 features

@@ -774,6 +774,16 @@ constexpr int kMergedFromFeat = 256;
 // rows, 162 k nonzeros, 59 features 24.2 / 16.1; 22.5 k, 524 k, 144: 62 / 52, 128: 48 / 33; 60 k, 1 M, 32: 29.7 / 31.5,
 // 64: 49.0 / 50.3, 128: 72.6 / 71.6; 400 k, 4 M, 16: 69 / 87.  Four: 169 k, 1.17 M, 32: 53.5 / 40.3.
 constexpr int64_t kMergedSlotsPerPhase = 1000000;
+// Of 65 to 127 features up to more of them: 100 k rows, 1.2 M nonzeros, 96 features 97 / 92 (skewed columns 79 / 64),
+// 80: 91 / 87 (76 / 61), but 128: 105 / 114 (84 / 83); 150 k, 1.5 M, 96: 124 / 128 (92 / 101).
+constexpr int64_t kMergedSlotsPerPhaseOdd = 1700000;
+// Above 128 features wherever it is one launch and rows are not long -- a phase more is C read and written once more,
+// and of an X that a partition's share of fits the L2s more is kept when rows are long: 60 k rows, 1 M nonzeros, 144
+// features 167 / 110 (112 / 75), 250 k, 1.5 M, 208: 339 / 310 (286 / 260), 391 k, 2.66 M, 192: 483 / 454 (406 / 415);
+// four partitions, 100 k, 1.2 M, 176: 246 / 174; but 30 k, 1.4 M, 144: 126 / 143, and where the phases run in slices
+// 60 k, 900 k, 192: 109 / 124 (90 / 90).
+constexpr int kMergedWideFeat = 128;
+constexpr int64_t kMergedWideSlotsPerRow = 24;
 constexpr size_t kMergedOptionalBytes = size_t(1) << 30;  // ... when the slot list stays below this
 
 namespace {
@@ -1222,10 +1232,13 @@ int stir_hyb_spmm_f32(const stir_hyb_plan* plan, int32_t feat, const float* d_B,
   if (nk == 0) return 0;
   STIR_REQUIRE(d_B && d_C, "hyb_spmm: null pointer argument");
   const int parts = plan->num_col_parts;
+  const int64_t slots = plan->rows.slots;
+  const bool few = slots <= (feat > 64 && feat < 128 ? kMergedSlotsPerPhaseOdd : kMergedSlotsPerPhase) * (parts - 1) ||
+                   (feat > kMergedWideFeat && slots <= kMergedWideSlotsPerRow * plan->m &&
+                    slice_class(feat, plan->n, INT64_MAX / feat) == vector_class(feat));
   if (plan->merged && vector_class(feat) >= 0 &&
       (parts > kMaxPhases || feat >= kMergedFromFeat ||
-       (plan->rows.slots <= kMergedSlotsPerPhase * (parts - 1) &&
-        stir::merged_balanced(plan->m, plan->n, feat, plan->rows.slots))))
+       (few && stir::merged_balanced(plan->m, plan->n, feat, slots))))
     return launch_merged(plan->rows, plan->m, plan->n, feat, d_B, d_C, static_cast<hipStream_t>(stream));
   const HybBucket* d_rows = plan->d_tables ? plan->d_tables + nk : nullptr;
   return launch_hyb(plan->tables, plan->d_tables, d_rows, plan->n, feat, d_B, d_C, static_cast<hipStream_t>(stream));

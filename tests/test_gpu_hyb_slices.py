@@ -50,3 +50,24 @@ def test_hyb_merged_rows_of_equal_work(dev, feat, parts):
     f(torch.from_numpy(x.ravel()).to(dev), y, *args)  # the operator adds to what is there
     torch.cuda.synchronize()
     assert np.all(np.abs(y.cpu().numpy().reshape(m, feat) - 2 * want) <= 3 * bound)
+
+
+@pytest.mark.parametrize("m,nnz,feat", [
+    (70000, 900000, 96), (70000, 900000, 128), (70000, 900000, 132), (30000, 900000, 132), (70000, 900000, 192),
+    (60000, 900000, 192), (100000, 1500000, 80)])
+def test_hyb_between_phases_and_merged_rows(dev, m, nnz, feat):
+    """Two partitions above a million slots: merged rows up to 127 features (not with more slots) and, above 128, with
+    short rows unless the phases run in slices; phases else."""
+    indptr, indices = random_csr(m, m, nnz, feat, skew=1.0)
+    buckets = [1, 2, 4, 8, 16, 32]
+    triples = _hyb_setup(dev, indptr, indices, m, m, 2, buckets, weighted=True, seed=feat)
+    x = np.random.default_rng(feat).standard_normal((m, feat), dtype=np.float32)
+    got, (f, args) = _run_hyb(dev, m, m, feat, 2, buckets, triples, x)
+    r, c, v = _hyb_as_coo(triples)
+    a = sp.csr_matrix((v.astype(np.float64), (r, c)), shape=(m, m))
+    want, bound = a @ x.astype(np.float64), RTOL * (a @ np.abs(x).astype(np.float64)) + 1e-30
+    assert np.all(np.abs(got - want) <= bound)
+    y = torch.from_numpy(got.ravel().copy()).to(dev)
+    f(torch.from_numpy(x.ravel()).to(dev), y, *args)  # the operator adds to what is there
+    torch.cuda.synchronize()
+    assert np.all(np.abs(y.cpu().numpy().reshape(m, feat) - 2 * want) <= 3 * bound)

@@ -353,7 +353,11 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
 //   108 k, 1.2 M, 64: 33.4 / 33.3 / 31.8 / 31.4 / 35.2, 34.4; 17 k, 288 k, 12: 10.3 / 10.1 / 10.6 / 11.3 / 13.7, 10.2;
 //   54 k, 521 k, 100: 27.6 / 28.1 / 27.8 / 28.1 / 30.8, 29.2; 9 k, 146 k, 64: 10.3 / 9.8 / 10.1 / 10.4 / 12.9, 10.3;
 //   25 k, 1 M, 256 (four slices): 85.3 / 85.8 / 87.0 / 87.5 / 87.8, 90.4; 30 k, 500 k, 512 (eight): 97 / 100 / 102 / 107 / 109, 98.
-// The other way: 100 k rows, 1.5 M nonzeros of uniform columns, 128 features 111.4 against 109.3 (skewed: 69.6, 73.0).
+// Up to 32 features no fewer than 256 entries, eight for each of 32 or more lane groups (us with 64 / 256 as the fewest,
+// 512 entries each): 16 k rows, 121 k nonzeros, 8 features 9.7 / 8.7, 9.2; 10 k, 100 k, 32: 9.3 / 8.7, 8.7; 12 k, 200 k,
+// 16: 9.7 / 9.3, 9.5; but 9 k, 115 k, 84 12.1 / 13.6, 12.2; 9 k, 60 k, 128 11.1 / 13.4, 11.0.
+// The other way, uniform columns only: 100 k rows, 1.5 M nonzeros, 128 features 111.4 against 109.3 (skewed: 69.6,
+// 73.0), 150 k, 1.2 M, 192 in slices 145 against 139 (88, 90).
 // From several turns of the largest workgroups on, 512 entries: 199 k rows, 4.9 M nonzeros, 44 features 167.8 / 163.4.
 int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c);
@@ -363,7 +367,8 @@ int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   if (entries > 2 * kUnits * per_unit * kMaxItems) return 512;
   if (slices > 2 || entries < kUnits * per_unit * 400) per_unit = slices > 5 ? 4 : 5;
   const int64_t items = stir::ceil_div(entries, kUnits * per_unit);
-  return (int)(std::max<int64_t>(64, std::min<int64_t>(items, kMaxItems)) + 3) / 4 * 4;
+  const int64_t fewest = c <= 1 ? 256 : 64;
+  return (int)(std::max(fewest, std::min<int64_t>(items, kMaxItems)) + 3) / 4 * 4;
 }
 
 int64_t workgroups(int32_t m, int32_t n, int32_t feat, int64_t nnz) {

@@ -312,7 +312,10 @@ __global__ __launch_bounds__(64 * kUnitWaves) void rgms_tile_kernel(const Unit* 
                                                         YT* __restrict__ Y) {
   constexpr int FIN = KK * 16;
   constexpr bool kPacked = sizeof(Rec) == sizeof(PackedEdge);
-  constexpr int PW = KK * NT <= 4 ? 2 : 1;  // relations whose W fragments are requested together
+  // Relations whose W fragments are requested together.  One where two cost a wavefront per SIMD: 64 inputs, 2 M edges,
+  // 65 / 130 relations 64 -> 64 162 / 207 us with two, 156 / 197 with one; 64 -> 32 85 / 107, 82 / 102 (three or four
+  // where there is room: the same; 32 -> 64 with three 128 against 112).
+  constexpr int PW = KK * NT < 4 ? 2 : 1;
   constexpr int kThreads = 64 * kUnitWaves, kSumIters = kTileRows * 32 / kThreads;
   __shared__ __attribute__((aligned(16))) uint16_t s_all[kUnitWaves][kTileRows * kSStride];
   __shared__ float partial[kUnitWaves][16 * 64];  // [wavefront][accumulator register][lane]

@@ -897,17 +897,23 @@ __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int64_t stride = one_stride(ends.nnz);
-  int d = 0, rs = 0;
+  int d = 0, rs = 0, re = 0;
   if (i < m) {
-    rs = indptr[i];
-    int re = indptr[i + 1];
+    rs = indptr[i], re = indptr[i + 1];
     if (re < rs || rs < ends.first || re > end) {
       if (!ends.bad) answer_bad(&answer->bad_indptr);
       rs = re = ends.first;
     }
-    for (int64_t q = (rs - ends.first + stride - 1) / stride; ends.first + q * stride < re; ++q) ws.coarse[q] = i;
     d = re - rs;
   }
+  // What only the next kernel reads.  Where this one scans its counts, behind them, so that neither the scan nor the
+  // host waits for these stores: per call from Python 4 k rows, 32 k nonzeros 36.7 -> 29.8 us, 16 k, 160 k 49.4 ->
+  // 43.5.  Where it does not, ahead of them: 20 k, 200 k 44.2, behind them 51.
+  auto keep_places = [&]() {
+    if (i < m)
+      for (int64_t q = (rs - ends.first + stride - 1) / stride; ends.first + q * stride < re; ++q) ws.coarse[q] = i;
+  };
+  if (!arrived) keep_places();
   int32_t* h = ws.hist + wave;  // [b][W]
   auto put = [&](int b, int32_t v) {
     if (lane == 0 && wave < W) __hip_atomic_store(h + b * W, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -932,13 +938,14 @@ __global__ __launch_bounds__(256) void one_count_kernel(int m, int num_cols, int
     tot = __shfl(tot, kWave - 1, kWave);
   }
   put(NB - 1, tot);
+  finish();
+  if (arrived) keep_places();
   if (i < m) {
     if (rows_apart(m))
       ws.lo[i] = rs;
     else
       ws.kb[i] = beta, ranks(ws)[i] = rank;
   }
-  finish();
 }
 
 // Exclusive scan of hist[b][.] by one workgroup per bucket, a tile after the other.

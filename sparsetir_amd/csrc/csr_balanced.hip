@@ -27,11 +27,14 @@ using stir::kWave;
 using stir::ld4;
 
 constexpr int kBlock = 256;
-constexpr int kSlots = 1152;    // nonzeros a workgroup holds in LDS: seven workgroups per compute unit
-// A row of at most this many nonzeros is not cut: it is left whole to the workgroup that has its mark.
+// Workgroups per compute unit and the nonzeros that each then has room for in LDS (REP = 2: rows of more than 256
+// features in one piece, whose partial sums take 8 KB more).
+constexpr int resident(int rep) { return rep == 1 ? 7 : 6; }
+constexpr int slots(int rep) { return rep == 1 ? 1152 : 832; }
+// A row of at most this many nonzeros is not cut: it is left whole to the workgroup that has its mark, and may lie
+// behind the workgroup's entries.
 constexpr int kWhole = 128;
-constexpr int kMaxItems = 1024;
-static_assert(kMaxItems + kWhole <= kSlots, "the last row of a workgroup may lie behind its entries");
+constexpr int max_items(int rep) { return slots(rep) - kWhole; }
 constexpr int kFlight = 8;      // rows of B requested at a time by a lane group
 
 // Last row r with indptr[r] + r <= q: q is a place in the list (indptr[0] added) and indptr[r] + r that of
@@ -84,22 +87,27 @@ __device__ __forceinline__ void add_row(float* row, int feat, int gl, const floa
 // fetch no row of B, and the product is added to C: what a workgroup has of a row that it shares with others goes
 // there by atomics, so there are no partial rows to be added up.
 template <int G, int REP, bool MERGED = false>
-__global__ __launch_bounds__(kBlock, REP == 1 ? 7 : 6) void csr_balanced_kernel(int m, int stride, int slices, int64_t nnz, int items,
-                                                              const float* __restrict__ A,
-                                                              const float* __restrict__ B, float* __restrict__ C,
-                                                              const int32_t* __restrict__ indptr,
-                                                              const int32_t* __restrict__ indices,
-                                                              uint32_t* __restrict__ counters,
-                                                              float* __restrict__ partials) {
+__global__ __launch_bounds__(kBlock, resident(REP)) void csr_balanced_kernel(int m, int stride, int slices, int64_t nnz,
+                                                                             int items, const float* __restrict__ A,
+                                                                             const float* __restrict__ B,
+                                                                             float* __restrict__ C,
+                                                                             const int32_t* __restrict__ indptr,
+                                                                             const int32_t* __restrict__ indices,
+                                                                             uint32_t* __restrict__ counters,
+                                                                             float* __restrict__ partials) {
   constexpr int NG = kBlock / G;
   constexpr int CH = kFlight / REP;
   constexpr int kPad = 4 * G * REP;  // floats of a partial row
+  constexpr int kSlots = slots(REP);
   __shared__ int2 nz[kSlots];     // column, value
   __shared__ int ends[kSlots];    // row + 1 at the row's last nonzero, else 0
   __shared__ float4 head[NG * G * REP], tail[NG * G * REP];
   __shared__ int open_all[NG];
   __shared__ int row_at[2], nz_at[2], cut[2];
   __shared__ int last[2];
+  // all of the above, and what an allocation is rounded up to, in a share of the compute unit's 160 KB
+  static_assert((kSlots * 12 + 2 * NG * G * REP * 16 + NG * 4 + 32 + 1279) / 1280 * 1280 * resident(REP) <= 160 * 1024,
+                "fewer workgroups per compute unit than the number of workgroups is chosen for");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int base = indptr[0];
   const int64_t total = m + min(nnz, (int64_t)indptr[m]) - base;
@@ -345,14 +353,18 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
   return cut ? 2 : whole;
 }
 
-// As many workgroups as are resident at once, so that all end together: seven per compute unit where that leaves them
-// a few hundred entries each, else five; of several slices of features five or four (their workgroups take turns
-// anyhow, and each looks for its entries once per slice).  us with 4 / 5 / 6 / 7 / 8 per compute unit, and with 512
-// entries each:
+// As many workgroups as are resident at once, so that all end together: seven per compute unit (rows of more than 256
+// features in one piece: six) where that leaves them a few hundred entries each, else five; of several slices of
+// features five or four (their workgroups take turns anyhow, and each looks for its entries once per slice).  us with
+// 4 / 5 / 6 / 7 / 8 per compute unit, and with 512 entries each:
 //   169 k rows, 1.17 M nonzeros, 64 features 35.2 / 35.3 / 33.0 / 32.2 / 36.2, 35.6; 47: 39.3 / 39.4 / 37.1 / 36.1 / 39.8, 39.7;
 //   108 k, 1.2 M, 64: 33.4 / 33.3 / 31.8 / 31.4 / 35.2, 34.4; 17 k, 288 k, 12: 10.3 / 10.1 / 10.6 / 11.3 / 13.7, 10.2;
 //   54 k, 521 k, 100: 27.6 / 28.1 / 27.8 / 28.1 / 30.8, 29.2; 9 k, 146 k, 64: 10.3 / 9.8 / 10.1 / 10.4 / 12.9, 10.3;
 //   25 k, 1 M, 256 (four slices): 85.3 / 85.8 / 87.0 / 87.5 / 87.8, 90.4; 30 k, 500 k, 512 (eight): 97 / 100 / 102 / 107 / 109, 98.
+// Six of the wide ones: with room for 1152 nonzeros only five fit, and a sixth each was a turn of its own (uniform /
+// skewed columns, 1152 and 832 nonzeros): 60 k rows, 1 M nonzeros, 260 features 178 / 129, 172 / 114; 100 k, 1.4 M, 300
+// 283 / 204, 281 / 193; merged rows 100 k, 700 k, 300 184 / 139, 176 / 116; 30 k, 500 k, 400 140 / 101, 139 / 87.  Five
+// that ask for five: the same for CSR, but merged rows 100 k, 700 k, 300 177 / 126, 500 278 / 213 against 285 / 192.
 // Up to 32 features no fewer than 256 entries, eight for each of 32 or more lane groups (us with 64 / 256 as the fewest,
 // 512 entries each): 16 k rows, 121 k nonzeros, 8 features 9.7 / 8.7, 9.2; 10 k, 100 k, 32: 9.3 / 8.7, 8.7; 12 k, 200 k,
 // 16: 9.7 / 9.3, 9.5; but 9 k, 115 k, 84 12.1 / 13.6, 12.2; 9 k, 60 k, 128 11.1 / 13.4, 11.0.
@@ -360,15 +372,15 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
 // 73.0), 150 k, 1.2 M, 192 in slices 145 against 139 (88, 90).
 // From several turns of the largest workgroups on, 512 entries: 199 k rows, 4.9 M nonzeros, 44 features 167.8 / 163.4.
 int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
-  const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c);
+  const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c), rep = c == 5 ? 2 : 1;
   constexpr int64_t kUnits = 256;  // compute units
-  const int64_t entries = m + nnz;
-  int64_t per_unit = c == 5 ? 6 : 7;
-  if (entries > 2 * kUnits * per_unit * kMaxItems) return 512;
+  const int64_t entries = m + nnz, most = max_items(rep);
+  int64_t per_unit = resident(rep);
+  if (entries > 2 * kUnits * per_unit * most) return 512;
   if (slices > 2 || entries < kUnits * per_unit * 400) per_unit = slices > 5 ? 4 : 5;
   const int64_t items = stir::ceil_div(entries, kUnits * per_unit);
   const int64_t fewest = c <= 1 ? 256 : 64;
-  return (int)(std::max(fewest, std::min<int64_t>(items, kMaxItems)) + 3) / 4 * 4;
+  return (int)(std::max(fewest, std::min(items, most)) + 3) / 4 * 4;
 }
 
 int64_t workgroups(int32_t m, int32_t n, int32_t feat, int64_t nnz) {

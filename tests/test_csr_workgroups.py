@@ -1,0 +1,32 @@
+"""How many workgroups a CSR product is cut into, as the sizes of its workspace tell (one counter each): no GPU needed."""
+import pytest
+
+from sparsetir_amd import _lib
+
+UNITS = 256  # compute units
+
+
+def _workgroups(m, feat, nnz, n=50000):
+    """Of one slice of features in one piece."""
+    return _lib.lib().stir_csr_spmm_workspace_clear_bytes(m, n, feat, nnz) // 4
+
+
+@pytest.mark.parametrize("feat,resident,room", [(32, 7, 1024), (47, 7, 1024), (100, 7, 1024), (200, 7, 1024),
+                                                (260, 6, 704), (500, 6, 704)])
+def test_one_turn_where_it_holds_the_entries(feat, resident, room):
+    """A launch that fits one turn of resident workgroups asks for no more of them than there are."""
+    m = 60000
+    for share in (0.45, 0.7, 0.9, 1.0):
+        entries = int(UNITS * resident * room * share)
+        if (entries - m) * feat >= 500_000_000:
+            continue
+        wgs = _workgroups(m, feat, entries - m)
+        assert UNITS * 4 < wgs <= UNITS * resident + 3, (feat, entries, wgs)  # sizes are rounded up to four counters
+
+
+@pytest.mark.parametrize("feat,room", [(32, 1024), (200, 1024), (257, 704), (500, 704)])
+def test_no_more_entries_than_there_is_room_for(feat, room):
+    """The room in LDS that lets as many workgroups be resident as are asked for; wide rows have less of it."""
+    m = 60000
+    for entries in range(200_000, min(6_000_000, 500_000_000 // feat + m), 50_000):
+        assert entries <= room * _workgroups(m, feat, entries - m), (feat, entries)

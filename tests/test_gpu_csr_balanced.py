@@ -66,7 +66,8 @@ def test_feature_slices(dev, feat, m, most):
     test_rows_across_workgroups(dev, feat, m, most)
 
 
-@pytest.mark.parametrize("feat,m,most", [(8, 25001, 40), (13, 60003, 62), (8, 120001, 64)])
+@pytest.mark.parametrize("feat,m,most", [(8, 25001, 40), (13, 60003, 62), (8, 120001, 64), (300, 60003, 35),
+                                         (260, 60003, 58)])
 def test_workgroups_by_size(dev, feat, m, most):
     """Hundreds of entries a workgroup, as many as it holds, and several turns of fewer."""
     test_rows_across_workgroups(dev, feat, m, most)

@@ -370,13 +370,30 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
 // 16: 9.7 / 9.3, 9.5; but 9 k, 115 k, 84 12.1 / 13.6, 12.2; 9 k, 60 k, 128 11.1 / 13.4, 11.0.
 // The other way, uniform columns only: 100 k rows, 1.5 M nonzeros, 128 features 111.4 against 109.3 (skewed: 69.6,
 // 73.0), 150 k, 1.2 M, 192 in slices 145 against 139 (88, 90).
-// From several turns of the largest workgroups on, 512 entries: 199 k rows, 4.9 M nonzeros, 44 features 167.8 / 163.4.
+// More than one turn of the largest workgroups (beyond_a_turn), 512 / 768 / 1024 entries, uniform and skewed columns: a
+// last turn that is nearly empty costs wide rows more, finding the entries narrow ones.
+//   170 k rows, 2 M nonzeros, 8 features 34.3 / 32.1 / 30.9, 32.2 / 30.2 / 29.0; 600 k, 20 M, 4: 265 / 245 / 240,
+//   249 / 213 / 197; 170 k, 1.7 M (1.02 turns), 32: 41.6 / 40.9 / 43.5, 32.5 / 30.8 / 31.8; 1.9 M: 44.5 / 43.7 / 45.2,
+//   34.6 / 31.8 / 32.9; 2.7 M: 55.9 / 55.8 / 55.5, 44.1 / 41.1 / 38.7; 500 k, 12 M, 32: 234 / 235 / 236, 169 / 153 / 150;
+//   170 k, 2 M, 64: 81.2 / 83.3 / 84.2, 52.7 / 53.0 / 54.3; 3.5 M: 129.7 / 132.3 / 135.5, 81.5 / 80.6 / 79.5; 50 k, 2.6 M,
+//   47: 74.7 / 74.0 / 75.2, 56.7 / 54.5 / 53.4; 300 k, 4.5 M, 64: 174 / 178 / 177, 112 / 111 / 112;
+//   170 k, 2 M, 150: 221 / 224 / 226, 145 / 149 / 153; 2.8 M, 100: 209 / 214 / 216, 132.5 / 134.8 / 135.2.
+// Turns made equal (two of 560 to 1024 entries each) lie between: 2.4 M, 64 95.7 against 95.2 with 512; 2.4 M, 32 37.4
+// against 36.3 with 1024.
+int64_t beyond_a_turn(int c, int64_t entries, int64_t turn) {
+  if (c == 0) return 1024;
+  if (c == 1) return 4 * entries <= 5 * turn ? 768 : 1024;
+  return c == 2 && entries <= 2 * turn ? 768 : 512;
+}
+
 int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   const int c = slice_class(n, feat, nnz), slices = (int)stir::ceil_div(feat, 16 << c), rep = c == 5 ? 2 : 1;
   constexpr int64_t kUnits = 256;  // compute units
   const int64_t entries = m + nnz, most = max_items(rep);
   int64_t per_unit = resident(rep);
-  if (entries > 2 * kUnits * per_unit * most) return 512;
+  const int64_t turn = kUnits * per_unit * most;
+  if (slices == 1 && entries > turn) return (int)beyond_a_turn(c, entries, turn);
+  if (entries > 2 * turn) return 512;
   if (slices > 2 || entries < kUnits * per_unit * 400) per_unit = slices > 5 ? 4 : 5;
   const int64_t items = stir::ceil_div(entries, kUnits * per_unit);
   const int64_t fewest = c <= 1 ? 256 : 64;

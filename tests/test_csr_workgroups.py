@@ -30,3 +30,13 @@ def test_no_more_entries_than_there_is_room_for(feat, room):
     m = 60000
     for entries in range(200_000, min(6_000_000, 500_000_000 // feat + m), 50_000):
         assert entries <= room * _workgroups(m, feat, entries - m), (feat, entries)
+
+
+@pytest.mark.parametrize("feat,resident,room", [(24, 7, 1024), (47, 7, 1024), (100, 7, 1024), (200, 7, 1024),
+                                                (300, 6, 704)])
+def test_no_nearly_empty_last_turn(feat, resident, room):
+    """A few more entries than one turn of the largest workgroups holds: smaller ones, so that a second turn is worth it."""
+    m = 60000
+    for share in (1.01, 1.05, 1.1):
+        entries = int(UNITS * resident * room * share)
+        assert _workgroups(m, feat, entries - m) > 1.3 * UNITS * resident, (feat, share)

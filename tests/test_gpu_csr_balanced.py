@@ -67,7 +67,7 @@ def test_feature_slices(dev, feat, m, most):
 
 
 @pytest.mark.parametrize("feat,m,most", [(8, 25001, 40), (13, 60003, 62), (8, 120001, 64), (300, 60003, 35),
-                                         (260, 60003, 58)])
+                                         (260, 60003, 58), (32, 60003, 75), (47, 60003, 75), (100, 60003, 75)])
 def test_workgroups_by_size(dev, feat, m, most):
     """Hundreds of entries a workgroup, as many as it holds, and several turns of fewer."""
     test_rows_across_workgroups(dev, feat, m, most)

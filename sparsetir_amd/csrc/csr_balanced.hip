@@ -353,14 +353,19 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
   return cut ? 2 : whole;
 }
 
-// As many workgroups as are resident at once, so that all end together: seven per compute unit (rows of more than 256
-// features in one piece: six) where that leaves them a few hundred entries each, else five; of several slices of
-// features five or four (their workgroups take turns anyhow, and each looks for its entries once per slice).  us with
-// 4 / 5 / 6 / 7 / 8 per compute unit, and with 512 entries each:
+// In one piece, as many workgroups as are resident at once, so that all end together: seven per compute unit (rows of
+// more than 256 features: six) where that leaves them a few hundred entries each, else five.  us with 4 / 5 / 6 / 7 / 8
+// per compute unit, and with 512 entries each:
 //   169 k rows, 1.17 M nonzeros, 64 features 35.2 / 35.3 / 33.0 / 32.2 / 36.2, 35.6; 47: 39.3 / 39.4 / 37.1 / 36.1 / 39.8, 39.7;
 //   108 k, 1.2 M, 64: 33.4 / 33.3 / 31.8 / 31.4 / 35.2, 34.4; 17 k, 288 k, 12: 10.3 / 10.1 / 10.6 / 11.3 / 13.7, 10.2;
-//   54 k, 521 k, 100: 27.6 / 28.1 / 27.8 / 28.1 / 30.8, 29.2; 9 k, 146 k, 64: 10.3 / 9.8 / 10.1 / 10.4 / 12.9, 10.3;
-//   25 k, 1 M, 256 (four slices): 85.3 / 85.8 / 87.0 / 87.5 / 87.8, 90.4; 30 k, 500 k, 512 (eight): 97 / 100 / 102 / 107 / 109, 98.
+//   54 k, 521 k, 100: 27.6 / 28.1 / 27.8 / 28.1 / 30.8, 29.2; 9 k, 146 k, 64: 10.3 / 9.8 / 10.1 / 10.4 / 12.9, 10.3.
+// In slices of features 768 entries: their workgroups take several turns anyhow, each looks for its entries once per
+// slice, and the less of a slice of B comes from memory the more that counts.  512 / 768 / 1024, uniform and skewed
+// columns:
+//   169 k, 1.17 M, 192: 140 / 146 / 147, 92 / 89 / 90; 256: 188 / 189 / 189, 145 / 142 / 142; merged rows of two
+//   partitions 213 / 216 / 223, 172 / 166 / 167; 100 k, 2 M, 256: 279 / 282 / 284, 173 / 168 / 167; 50 k, 2 M, 192: 181 /
+//   183 / 184, 112 / 104 / 102; 400 k, 5 M, 192: 579 / 588 / 592 (896 entries), 385 / 374 / 372; 25 k, 1 M, 256: 88 / 86 /
+//   85, 80 / 76 / 75; 10 k, 300 k, 512: 50 / 48 / 45 (896), 50 / 48 / 46, with five per compute unit and slice 59, 58.
 // Six of the wide ones: with room for 1152 nonzeros only five fit, and a sixth each was a turn of its own (uniform /
 // skewed columns, 1152 and 832 nonzeros): 60 k rows, 1 M nonzeros, 260 features 178 / 129, 172 / 114; 100 k, 1.4 M, 300
 // 283 / 204, 281 / 193; merged rows 100 k, 700 k, 300 184 / 139, 176 / 116; 30 k, 500 k, 400 140 / 101, 139 / 87.  Five
@@ -369,7 +374,7 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
 // 512 entries each): 16 k rows, 121 k nonzeros, 8 features 9.7 / 8.7, 9.2; 10 k, 100 k, 32: 9.3 / 8.7, 8.7; 12 k, 200 k,
 // 16: 9.7 / 9.3, 9.5; but 9 k, 115 k, 84 12.1 / 13.6, 12.2; 9 k, 60 k, 128 11.1 / 13.4, 11.0.
 // The other way, uniform columns only: 100 k rows, 1.5 M nonzeros, 128 features 111.4 against 109.3 (skewed: 69.6,
-// 73.0), 150 k, 1.2 M, 192 in slices 145 against 139 (88, 90).
+// 73.0).
 // More than one turn of the largest workgroups (beyond_a_turn), 512 / 768 / 1024 entries, uniform and skewed columns: a
 // last turn that is nearly empty costs wide rows more, finding the entries narrow ones.
 //   170 k rows, 2 M nonzeros, 8 features 34.3 / 32.1 / 30.9, 32.2 / 30.2 / 29.0; 600 k, 20 M, 4: 265 / 245 / 240,
@@ -391,10 +396,10 @@ int entries_per_workgroup(int32_t m, int32_t n, int32_t feat, int64_t nnz) {
   constexpr int64_t kUnits = 256;  // compute units
   const int64_t entries = m + nnz, most = max_items(rep);
   int64_t per_unit = resident(rep);
+  if (slices > 1) return 768;
   const int64_t turn = kUnits * per_unit * most;
-  if (slices == 1 && entries > turn) return (int)beyond_a_turn(c, entries, turn);
-  if (entries > 2 * turn) return 512;
-  if (slices > 2 || entries < kUnits * per_unit * 400) per_unit = slices > 5 ? 4 : 5;
+  if (entries > turn) return (int)beyond_a_turn(c, entries, turn);
+  if (entries < kUnits * per_unit * 400) per_unit = 5;
   const int64_t items = stir::ceil_div(entries, kUnits * per_unit);
   const int64_t fewest = c <= 1 ? 256 : 64;
   return (int)(std::max(fewest, std::min(items, most)) + 3) / 4 * 4;

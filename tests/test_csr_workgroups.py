@@ -40,3 +40,12 @@ def test_no_nearly_empty_last_turn(feat, resident, room):
     for share in (1.01, 1.05, 1.1):
         entries = int(UNITS * resident * room * share)
         assert _workgroups(m, feat, entries - m) > 1.3 * UNITS * resident, (feat, share)
+
+
+@pytest.mark.parametrize("feat,m,nnz", [(256, 169343, 1166243), (192, 150000, 1200000), (512, 40000, 1500000),
+                                        (128, 300000, 7800000), (512, 10000, 300000)])
+def test_slices_take_several_turns(feat, m, nnz):
+    """In slices of 64 features a workgroup takes 768 entries, whatever the turns: neither what it has room for nor a
+    share of one turn."""
+    slices = feat // 64
+    assert abs(_workgroups(m, feat, nnz, n=m) / slices - (m + nnz) / 768) <= 4

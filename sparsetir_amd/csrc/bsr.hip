@@ -558,7 +558,7 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
   for (int t = 0; t < FT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
-  const int steps = (nblk * sub + 1) / 2;
+  const int chunks = nblk * sub;
   // block columns of the 64 blocks from `base` on and of the next 64
   int base = 0;
   int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
@@ -588,21 +588,30 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
       j_more = base + kWave + lane < nblk ? indices[p_begin + base + kWave + lane] : 0;
     }
   };
-  fetch();
-#pragma unroll 1
-  for (int it = 0; it < steps; ++it) {
+  auto step = [&](bool more) {
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + place(16 * b + KQ * q + kq)) = xr[b][q];
     const u32x4 a = ar;
-    fetch();
+    if (more) fetch();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int t = 0; t < FT; ++t) acc[t] = mfma16<BF16>(a, read_b(stage + (bread ^ (32 * t)), FCN * 64), acc[t]);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+  };
+  fetch();
+#pragma unroll 1
+  for (int it = 0; it < chunks / 2; ++it) step(true);
+  // The second chunk of an odd last step is multiplied by zeros of A and has to be zeros whatever X holds: said here, not
+  // left to an empty window whose loads carry a scalar offset.  (Lane offsets beyond any window cost 1 to 2 %, this
+  // nothing: 1024 x 1024 blocks of 16, 4096 features 607 -> 605 us.)
+  if (chunks & 1) {
+#pragma unroll
+    for (int q = 0; q < XQ; ++q) xr[1][q] = u32x4{0, 0, 0, 0};
+    step(false);
   }
   // acc[t][v] is row 4 g + v, column 16 t + ii; 16-bit results through LDS into 16-byte stores (see store_rows)
   const int64_t row0 = (int64_t)i_out * blk + bi0;

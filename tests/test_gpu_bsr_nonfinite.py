@@ -1,0 +1,69 @@
+"""BSR SpMM with infinities and NaN in X: rows of X that no block names take no part in the result, in any of the kernels
+and for odd numbers of 16-column chunks (whose second half of a step is not there); values that are named reach the
+features they belong to and no others.  Checked against the fp64 oracle as in test_gpu_bsr.py."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import bsr_f64
+from sparsetir_amd import datasets, ops
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [
+    (1024, 60, 16, 0.1, 224),     # a wavefront per 16-row slice, 128 features
+    (1024, 400, 16, 0.01, 512),   # 256 features
+    (230, 50, 48, 0.05, 352),     # three chunks a block
+    (150, 40, 16, 0.2, 1184),     # 16-row slices by four wavefronts
+    (3, 200, 16, 0.5, 64),        # by eight wavefronts
+    (61, 23, 80, 0.3, 480),
+    (9, 90, 32, 0.6, 96),
+    (343, 200, 32, 0.01, 736),    # a wavefront per 32-row slice
+    (520, 200, 32, 0.01, 800),
+    (397, 30, 32, 0.2, 416),      # four wavefronts
+    (147, 13, 64, 0.3, 2400),
+    (14, 100, 128, 0.05, 160),
+]
+
+
+def _without(cfg, cols):
+    """The configuration without the blocks of these block columns, every other block row of an odd length."""
+    rows = [r[~np.isin(r, cols)] for r in np.split(cfg["indices"], cfg["indptr"][1:-1])]
+    rows = [r[:len(r) - 1] if len(r) and (len(r) + i) % 2 == 0 else r for i, r in enumerate(rows)]
+    cfg["indptr"] = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    cfg["indices"] = np.concatenate(rows).astype(np.int32)
+    rng = np.random.default_rng(len(rows))
+    cfg["data"] = (rng.choice([-1.0, 1.0], (len(cfg["indices"]), cfg["blk"], cfg["blk"])) *
+                   rng.uniform(0.01, 0.03, (len(cfg["indices"]), cfg["blk"], cfg["blk"]))).astype(np.float32)
+    return cfg
+
+
+@pytest.mark.parametrize("mb,nb,blk,density,feat", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_non_finite_x(dev, mb, nb, blk, density, feat, dtype):
+    unnamed = np.array([0, 1, nb - 1])
+    cfg = _without(datasets.config4(seed=mb + feat, mb=mb, nb=nb, blk=blk, density=density, feat=feat), unnamed)
+    x = cfg["x"].reshape(nb, blk, feat)
+    x[unnamed[0]], x[unnamed[1]], x[unnamed[2]] = np.inf, np.nan, -np.inf
+    named = int(cfg["indices"][len(cfg["indices"]) // 2])
+    f_inf, f_nan = feat - 1, feat // 2
+    x[named, blk // 2, f_inf], x[named, 3, f_nan] = np.inf, np.nan
+    a = torch.from_numpy(cfg["data"]).to(dev).to(dtype)
+    t = torch.from_numpy(cfg["x"]).to(dev).to(dtype)
+    y = torch.zeros(mb * blk * feat, dtype=torch.float32, device=dev)
+    ops.build_bsrmm(mb, nb, len(cfg["indices"]), blk, feat, dtype, torch.float32)(
+        a.reshape(-1), t.reshape(-1), y, torch.from_numpy(cfg["indptr"]).to(dev), torch.from_numpy(cfg["indices"]).to(dev))
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(mb, blk, feat)
+    a32, x32 = a.float().cpu().numpy(), t.float().cpu().numpy()
+    has = np.array([named in r for r in np.split(cfg["indices"], cfg["indptr"][1:-1])])
+    assert has.any() and not has.all()
+    assert np.isinf(got[has][:, :, f_inf]).all() and np.isnan(got[has][:, :, f_nan]).all()
+    got[np.ix_(has, np.arange(blk), [f_inf, f_nan])] = 0.0
+    assert np.isfinite(got).all()
+    # the finite rest: the same with zeros where the values are not finite
+    x32 = np.where(np.isfinite(x32), x32, 0.0).astype(np.float32)
+    want = bsr_f64(cfg["indptr"], cfg["indices"], a32, x32, mb, nb, blk).reshape(mb, blk, feat)
+    scale = bsr_f64(cfg["indptr"], cfg["indices"], np.abs(a32), np.abs(x32), mb, nb, blk).reshape(mb, blk, feat)
+    want[np.ix_(has, np.arange(blk), [f_inf, f_nan])] = 0.0
+    assert np.all(np.abs(got - want) <= 1e-5 * scale + 1e-30)  # fp32 sums of exact products, as in test_gpu_bsr.py

@@ -959,15 +959,26 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     }
   }
   auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
-  constexpr int64_t kMuchX = 3 << 20;
-  const int rankable = mb <= kRankRows ? 1 : 0;
+  constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000;
+  // Slices in order of their length (row_of_rank) where the rows of X of a feature tile are more than an XCD's L2 holds
+  // beside A, so that what runs side by side reads the same of them.  Finding the row costs 2 to 3 us a tile, which
+  // few feature tiles do not give back: from four on (16-row slices: 512 features).  In order of length / as they come, us:
+  //   wavefronts of 32 x 256 (512 block rows unless noted): 500 columns of blocks, 8 %, 512 features 55.5 / 50.6, 768 77.8 /
+  //   78.3, 832 85.9 / 92.2, 1536 128 / 159, 4096 of 10 % 374 / 662; 260 (4.3 MB of X in a tile), 832 35 / 34 (5 %), 1504
+  //   55 / 59, 4096 116 / 122; 200 (3.3 MB), 832 31.0 / 27.6, 1504 46.5 / 42.3, but with 15 % 95 / 96, 2048 110 / 116:
+  //   there from 16 steps in a block row on;
+  //   four wavefronts: blocks of 64, 256 x 256, 10 %, 256 features 37.5 / 34.7, 384 50.7 / 48.2, 512 58.7 / 61.3;
+  //   16-row slices: 1024 x 1024 blocks, 10 %, 256 features 54 / 47, 384 76 / 68, 512 86 / 85, 1024 157 / 180, 1536 241 /
+  //   319; 1024 x 400 (3.3 MB), 256 30 / 23, 1024 73 / 70, 1536 108 / 100; 700 x 900, 128 features a tile (3.7 MB), 640
+  //   75 / 73; 340 x 340 of 48, 384 82 / 76, 512 101 / 104, 1024 159 / 181.
+  const bool rankable = mb <= kRankRows;
   if (unit == 16) {
-    // Ranked order as below.  256 features per wavefront then, unless the last tile would be mostly empty or wavefronts
-    // few: 1024 x 1024 blocks of 16, 1024 features 158 us (171 with 128), 1006 x 599, 544 features 155 (140).
+    // 256 features per wavefront with much X, unless the last tile would be mostly empty or wavefronts few: 1024 x 1024
+    // blocks of 16, 1024 features 158 us (171 with 128), 1006 x 599, 544 features 155 (140).
     const bool much = x_tile_bytes(kWaveF) > kMuchX;
     const bool wide = much && unit_slices * stir::ceil_div(feat, kWaveF) >= 8 * cus &&
                       (kWaveF - 1 - (feat - 1) % kWaveF) * 8 <= feat;
-    const int ranked = much ? rankable : 0;
+    const int ranked = rankable && feat >= 512 && x_tile_bytes(wide ? kWaveF : kTileF) > kBeyondL2;
     // A wavefront per slice once eight per CU have one: 60 x 200 blocks of 48, 1024 features (1440) 33.1 us against 31.0
     // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
     if (unit_slices * stir::ceil_div(feat, kTileF) >= 8 * cus && feat < (1 << 25) && blk <= 4096) {
@@ -1020,25 +1031,24 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int nt = feat >= 1024 && slices * stir::ceil_div(feat, 2 * kTileF) * 5 >= 8 * (int64_t)cus ? 2 : 1;
   const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
   dim3 block(256);
-  // Where the X rows of a feature tile are more than an XCD's L2 holds beside A (x_tile_bytes), the slices are taken in
-  // order of their length (row_of_rank), and those of 32 rows by one wavefront each once there are enough of them:
-  // 219 x 201 blocks, 1504 features (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 456 x 309, 352 features (912, of which
-  // half have 96 features) 66.4 -> 69.4.  Below 3 MB finding the row (2-3 us a tile) is lost: 359 x 71, 3488 features
-  // 69 -> 83 us ranked, 430 x 120, 1120 features 62 -> 67.
+  // With much X, slices of 32 rows by one wavefront each once there are enough of them: 219 x 201 blocks, 1504 features
+  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 456 x 309, 352 features (912, of which half have 96 features) 66.4 -> 69.4.
   const int wf_tiles = (int)stir::ceil_div(feat, kWaveF);
   if (rs == 1 && x_tile_bytes(kWaveF) > kMuchX && slices * wf_tiles >= 4 * cus && feat < (1 << 25) && blk <= 4096) {
     const int64_t blocks = grid_of(slices, wf_tiles);
     STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
+    const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
+    const int ranked = rankable && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
 #define STIR_BSR_W(BF, OUT)                                                                                       \
   hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices,     \
-                     wf_tiles, rankable, A, X, d_Y, d_indptr, d_indices, d_row_ids)
+                     wf_tiles, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
     STIR_BSR_TYPES(STIR_BSR_W)
 #undef STIR_BSR_W
     STIR_LAUNCH_CHECK();
     return 0;
   }
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
-  const int ranked = x_tile_bytes(kTileF * nt) > kMuchX ? rankable : 0;
+  const int ranked = rankable && f_tiles >= 4 && x_tile_bytes(kTileF * nt) > kMuchX;
   // Blocks of 128 rows and more: block rows dealt to XCDs (decode_tile_by_rows).  Measured at
   // 16384^2, 10 %, 4096 features: 128 x 128 blocks 387 -> 365 us; 64 x 64 blocks (one slice per
   // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an

@@ -1,4 +1,4 @@
-"""BSR SpMM where X does not fit an L2: slices taken in order of their length, 32-row slices by a wavefront each.
+"""BSR SpMM where X does not fit an L2: slices taken in order of their length or as they come, by a wavefront each or not.
 Empty block rows, a few with more blocks than a wavefront has lanes, block columns in any order, ragged feature
 tiles, arrays that start at an odd element.  Checked against the fp64 oracle as in test_gpu_bsr.py."""
 import numpy as np
@@ -25,19 +25,27 @@ def _config(mb, nb, blk, density, feat, seed):
 
 
 @pytest.mark.parametrize("mb,nb,blk,density,feat", [
-    (1024, 193, 32, 0.004, 224),   # as many block rows as are ranked
-    (1030, 200, 32, 0.004, 256),   # more: plain order
-    (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles
+    (1024, 193, 32, 0.004, 224),   # one feature tile: as they come
+    (1030, 200, 32, 0.004, 256),
+    (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles; few steps: as they come
+    (70, 90, 96, 0.04, 1440),      # ranked
+    (257, 250, 32, 0.01, 832),     # ranked, the last of four feature tiles with 64
+    (257, 200, 32, 0.08, 832),     # less of X, 16 steps a slice
     (343, 200, 32, 0.01, 736),
-    (20, 200, 64, 0.03, 96),       # four wavefronts per 64 rows
-    (12, 100, 128, 0.05, 160),     # too few block rows to deal them to XCDs
-    (14, 100, 128, 0.05, 160),     # block rows dealt to XCDs
+    (20, 200, 64, 0.03, 96),       # eight wavefronts
+    (12, 100, 128, 0.05, 160),
+    (14, 100, 128, 0.05, 160),
+    (60, 200, 64, 0.03, 416),      # four wavefronts per 64 rows, ranked
+    (33, 100, 128, 0.05, 544),     # too few block rows to deal them to XCDs
+    (36, 100, 128, 0.05, 544),     # block rows dealt to XCDs
     (40, 20, 64, 0.1, 1056),       # few workgroups: 128 features each
     (83, 20, 64, 0.1, 1056),       # as many as take 256 features each, the last with 32
     (1, 6200, 32, 0.001, 64),
     (1030, 90, 16, 0.02, 224),     # 16-row slices by a wavefront each: plain order
-    (1024, 400, 16, 0.004, 512),   # ranked, 256 features
-    (700, 400, 16, 0.004, 320),    # ranked, 128 features, an odd number of blocks
+    (1024, 400, 16, 0.004, 512),   # 256 features
+    (512, 520, 16, 0.004, 1024),   # ranked, 256 features
+    (700, 400, 16, 0.004, 320),    # 128 features, an odd number of blocks
+    (410, 1000, 16, 0.004, 544),   # ranked, 128 features
     (230, 50, 48, 0.05, 352),      # chunks of two blocks in one step
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

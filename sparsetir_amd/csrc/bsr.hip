@@ -9,6 +9,7 @@
 // launches bsr_split_kernel, large ones of 32-row blocks bsr_wave_kernel.
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -643,25 +644,28 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
 }
 
 // ------------------------------------------------------------------ large launches: a wavefront per tile
-// A wavefront owns 32 rows of a block row and 256 features: eight 32x32 accumulators.  Its X tile has 16 KB of LDS of
-// its own (image as in bsr_tile), filled from registers that were loaded a step before, so that 8 wavefronts per CU
-// have 144 KB on their way and none waits for another; the A operand is loaded straight into registers.  The first
-// half of a step's operands is read before its first MFMA, the second half as the first is used.
+// A wavefront owns 32 rows of a block row and TF = 256 features, eight 32x32 accumulators, or 128 where the launch's rule
+// says so.  Its X tile has 16 (8) KB of LDS of its own (image as in bsr_tile), filled from registers that were loaded a
+// step before, so that 8 (12) wavefronts per CU have 144 (120) KB on their way and none waits for another; the A operand
+// is loaded straight into registers.  The first half of a step's operands is read before its first MFMA, the second half
+// as the first is used.
 // With the ranked order (row_of_rank) the wavefronts of an XCD stay within reach of each other in X: 16384 x 16384,
 // 10 % blocks of 32, 4096 features 595 us with workgroups of four wavefronts, 590 with this kernel in plain order
-// (3.97 GB through the L2s, 31 M misses), 377 with both; 300 x 450 blocks, 3232 features 290 -> 217 us; 1024 x 512,
-// 5 % 706 -> 454.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
-template <bool BF16, int OUT>
-__global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
-                                                            const uint16_t* __restrict__ A,
-                                                            const uint16_t* __restrict__ X, void* __restrict__ Y,
-                                                            const int32_t* __restrict__ indptr,
-                                                            const int32_t* __restrict__ indices,
-                                                            const int32_t* __restrict__ row_ids) {
-  constexpr int FT = kWaveF / 32;  // accumulators
-  constexpr int FCN = kWaveF / 8;  // 16-byte units per row of X
-  constexpr int XQ = 16;           // units per lane and step, two rows of X per load
-  __shared__ __attribute__((aligned(16))) char stage[kTileK * kWaveF * 2];
+// (3.97 GB through the L2s, 31 M misses), 395 with both; 300 x 450 blocks, 3232 features 290 -> 217 us; 1024 x 512,
+// 5 % 702 -> 430.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
+template <bool BF16, int OUT, int TF>
+__global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles,
+                                                                            int ranked, const uint16_t* __restrict__ A,
+                                                                            const uint16_t* __restrict__ X,
+                                                                            void* __restrict__ Y,
+                                                                            const int32_t* __restrict__ indptr,
+                                                                            const int32_t* __restrict__ indices,
+                                                                            const int32_t* __restrict__ row_ids) {
+  constexpr int FT = TF / 32;      // accumulators
+  constexpr int FCN = TF / 8;      // 16-byte units per row of X
+  constexpr int KQ = kWave / FCN;  // rows of X per load
+  constexpr int XQ = kTileK / KQ;  // units per lane and step
+  __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
   int64_t slice;
   int f_tile;
   if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
@@ -675,13 +679,13 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
   const int bi0 = ((int)slice % sub) * 32;
   if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
   const int i_out = row_ids ? row_ids[i] : i;
-  const int f0 = f_tile * kWaveF;
-  // staging: unit c of the rows 2 q + kq.  Units beyond feat repeat the last one: features nobody stores.
+  const int f0 = f_tile * TF;
+  // staging: unit c of the rows KQ q + kq.  Units beyond feat repeat the last one: features nobody stores.
   const int c = lane % FCN, kq = lane / FCN;
   const uint32_t xoff = (uint32_t)(kq * feat + min(8 * c, feat - f0 - 8)) * 2;
-  uint32_t xdst[2];
+  uint32_t xdst[4 / KQ];
 #pragma unroll
-  for (int q = 0; q < 2; ++q) xdst[q] = (uint32_t)(((2 * q + kq) * FCN + (c ^ (4 * (2 * q + kq)))) * 16);
+  for (int q = 0; q < 4 / KQ; ++q) xdst[q] = (uint32_t)(((KQ * q + kq) * FCN + (c ^ (4 * (KQ * q + kq)))) * 16);
   const uint32_t aoff = (uint32_t)((bi0 + n) * blk + 8 * h) * 2;
   // operand reads: tile t is 256 bytes behind tile t - 4
   const int sl = lane & 15, kr = sl >> 2, half16 = (lane >> 4) & 1;
@@ -715,7 +719,7 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
     for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + 32 * m, 0, 0);
     const auto rx = window(X + ((int64_t)j * blk + k0) * feat + f0, live ? 64u * feat : 0);
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) xr[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * 4 * feat, 0);
+    for (int q = 0; q < XQ; ++q) xr[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * KQ * 2 * feat, 0);
     k0 += kTileK;
     if (k0 == blk) {
       k0 = 0, ++pb;
@@ -729,7 +733,7 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
 #pragma unroll 1
   for (int it = 0; it < steps; ++it) {
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + xdst[q & 1] + (q / 2) * 4 * FCN * 16) = xr[q];
+    for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + xdst[q % (4 / KQ)] + q * KQ / 4 * 4 * FCN * 16) = xr[q];
     const u32x4 a0 = ar[0], a1 = ar[1];
     fetch();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1032,20 +1036,37 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
   dim3 block(256);
   // With much X, slices of 32 rows by one wavefront each once there are enough of them: 219 x 201 blocks, 1504 features
-  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 456 x 309, 352 features (912, of which half have 96 features) 66.4 -> 69.4.
-  const int wf_tiles = (int)stir::ceil_div(feat, kWaveF);
-  if (rs == 1 && x_tile_bytes(kWaveF) > kMuchX && slices * wf_tiles >= 4 * cus && feat < (1 << 25) && blk <= 4096) {
-    const int64_t blocks = grid_of(slices, wf_tiles);
-    STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-    const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
-    const int ranked = rankable && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
-#define STIR_BSR_W(BF, OUT)                                                                                       \
-  hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices,     \
+  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 512 x 309, 192 features (1024 of 128) 26.1 against 25.0 by workgroups.
+  // 256 features to a wavefront read A half as often and take the ranked order; up to three such tiles, and for five
+  // where 128 features of X fit an L2, that is less than what empty parts of the last tile, too few wavefronts or a
+  // last turn of a quarter cost, except for one or two full tiles and enough wavefronts.  256 (ranked from four tiles
+  // on) / 128 features, 10 % of 512 x 309 blocks unless noted: 288 42.8 / 33.4, 416 43 / 39.7, 544 60 / 54, 800 68 / 76;
+  // 1024 x 500, 96 features 63 / 39, 384 103 / 85; 512 x 500, 8 %, 640 71 / 68, 768 78 / 74, 1024 84 / 102; 512 x 260, 8 %,
+  // 1152 70 / 60, 1280 69 / 65; 300 x 512, 5 %, 1152 52 / 57; 150 x 200 of 96, 16 %, 512 features 102 / 121; 1500 x 400,
+  // 8 %, 512 113 / 114, 256 55 / 59.  Where 256 leave fewer than four wavefronts per CU, 128 features again: 219 x 300,
+  // 1024 38.2 by workgroups, 35.2; 135 x 512, 5 %, 1536 39.0, 34.1; 85 x 512, 3072 70, 60.
+  if (rs == 1 && x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && feat < (1 << 25) && blk <= 4096) {
+    const int64_t tiles = stir::ceil_div(feat, kWaveF);
+    const bool full = (tiles * kWaveF - feat) * 8 <= feat;
+    const bool narrow = tiles <= 3 || (tiles == 5 && x_tile_bytes(kTileF) <= kMuchX);
+    const bool wide = narrow ? tiles <= 2 && full && slices * tiles >= 5 * (int64_t)cus : slices * tiles >= 4 * (int64_t)cus;
+    const int wf_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
+    if (wide || slices * wf_tiles >= 5 * (int64_t)cus) {
+      const int64_t blocks = grid_of(slices, wf_tiles);
+      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
+      const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
+      const int ranked = rankable && wide && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
+#define STIR_BSR_WT(BF, OUT, TF)                                                                                \
+  hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT, TF>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices, \
                      wf_tiles, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
-    STIR_BSR_TYPES(STIR_BSR_W)
+#define STIR_BSR_W(BF, OUT) \
+  if (wide) STIR_BSR_WT(BF, OUT, kWaveF); else STIR_BSR_WT(BF, OUT, kTileF)
+      STIR_BSR_TYPES(STIR_BSR_W)
 #undef STIR_BSR_W
-    STIR_LAUNCH_CHECK();
-    return 0;
+#undef STIR_BSR_WT
+      STIR_LAUNCH_CHECK();
+      return 0;
+    }
   }
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
   const int ranked = rankable && f_tiles >= 4 && x_tile_bytes(kTileF * nt) > kMuchX;

@@ -25,8 +25,14 @@ def _config(mb, nb, blk, density, feat, seed):
 
 
 @pytest.mark.parametrize("mb,nb,blk,density,feat", [
-    (1024, 193, 32, 0.004, 224),   # one feature tile: as they come
+    (1024, 193, 32, 0.004, 224),   # 32-row slices by a wavefront each, 128 features: as they come
     (1030, 200, 32, 0.004, 256),
+    (430, 200, 32, 0.004, 288),    # the last of three tiles with 32
+    (220, 200, 32, 0.01, 672),
+    (150, 200, 32, 0.02, 1056),    # five tiles of 256 would be
+    (150, 70, 96, 0.04, 352),
+    (170, 260, 32, 0.02, 992),     # too few for 256 features each
+    (650, 200, 32, 0.005, 512),    # two full tiles of 256
     (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles; few steps: as they come
     (70, 90, 96, 0.04, 1440),      # ranked
     (257, 250, 32, 0.01, 832),     # ranked, the last of four feature tiles with 64

@@ -122,8 +122,8 @@ int stir_column_part_hyb_device_values(int32_t num_rows, int32_t num_cols, const
 /*
  * The same pass for one column partition and at most 32 buckets, shorter where the matrix is small
  * (a fresh matrix per mini-batch): max_nnz is the length of d_indices, checked against d_indptr on
- * the device; _sizes synchronises the stream once, _fill does not, and with d_values / d_A (both or
- * neither null) it writes the value arrays too.  Same workspace size as above, untouched in between.
+ * the device; _sizes synchronises the stream once, also when it refuses the matrix, _fill does not,
+ * and with d_values / d_A (both or neither null) it writes the value arrays too.  Same workspace size as above, untouched in between.
  */
 int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr,
                                    const int32_t* d_indices, int64_t max_nnz, const int32_t* buckets,

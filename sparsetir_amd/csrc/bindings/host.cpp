@@ -30,6 +30,7 @@
 #include <vector>
 
 #include "../../../include/sparsetir_amd.h"
+#include "../format_one.h"
 
 namespace {
 
@@ -537,7 +538,7 @@ PyObject* column_part_hyb(PyObject*, PyObject* args) {
     const at::Tensor ws = at::empty({std::max<int64_t>(ws_bytes, 256)}, on.dtype(c10::ScalarType::Byte));
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = stir_column_part_hyb_one_sizes(m, n, d_ptr, d_idx, nnz, w32.data(), (int32_t)nb, ws.data_ptr(), nrows.data(), st);
+    rc = stir::column_part_hyb_one_sizes(m, n, d_ptr, d_idx, nnz, w32.data(), (int32_t)nb, ws.data_ptr(), nrows.data(), st);
     Py_END_ALLOW_THREADS
     if (rc != 0) return PyLong_FromLong(kFailed);
     int64_t rows = 0, slots = 0;

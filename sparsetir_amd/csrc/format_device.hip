@@ -24,6 +24,7 @@
 
 #include "call_answer.h"
 #include "common.h"
+#include "format_one.h"
 #include "row_lookup.h"
 #include "../../include/sparsetir_amd.h"
 
@@ -1248,6 +1249,58 @@ int scan_hist(const Workspace& ws, int P, int NB, int64_t W, hipStream_t st) {
 
 }  // namespace
 
+namespace stir {
+
+// whole: to the end of the kernels; else to the answers (see format_one.h), 5 us less.
+int column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr, const int32_t* d_indices,
+                              int64_t max_nnz, const int32_t* buckets, int32_t num_buckets, void* d_workspace,
+                              int64_t* nrows, void* stream, bool whole) {
+  const char* who = "ColumnPartHyb(device)";
+  if (check_args(who, num_rows, num_cols, 1, buckets, num_buckets)) return -1;
+  STIR_REQUIRE(num_buckets <= kOneBuckets, "%s: %d buckets, at most %d are supported here", who, num_buckets, kOneBuckets);
+  STIR_REQUIRE(nrows && max_nnz >= 0, "%s: bad arguments", who);
+  const int NB = num_buckets, m = num_rows;
+  std::fill(nrows, nrows + NB, int64_t(0));
+  if (m == 0) return 0;
+  STIR_REQUIRE(d_indptr && d_workspace && (max_nnz == 0 || d_indices), "%s: null pointer argument", who);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const Workspace ws = carve(d_workspace, m, 1, NB);
+  const int64_t W = stir::ceil_div(m, kWave);
+  AnswerBox* box = nullptr;
+  uint32_t* arrived = nullptr;
+  if (answer_box(who, &box, &arrived)) return -1;
+  box->host->bad_range = box->host->bad_indptr = 0;
+  const uint32_t number = box->number = stir::next_call(box->number);
+  stir::forget_answers(box->host->rows, NB);
+  const bool few = W <= kFewCounts;
+  OneWidths widths = {};
+  std::copy(buckets, buckets + NB, widths.w);
+  const int64_t count_blocks = stir::ceil_div(m, 256);
+  const int64_t check_blocks = stir::ceil_div(max_nnz, 256 * kValidatePerThread);
+  STIR_REQUIRE(count_blocks + check_blocks < (int64_t(1) << 31), "%s: too many nonzeros for one launch", who);
+  hipLaunchKernelGGL(one_count_kernel, dim3((unsigned)(count_blocks + check_blocks)), dim3(256), 0, st, m, num_cols,
+                     NB, W, max_nnz, (int)count_blocks, widths, ws, d_indptr, d_indices, box->device, few ? arrived : nullptr, number);
+  STIR_LAUNCH_CHECK();
+  if (!few && W <= kOneScanMax) {
+    hipLaunchKernelGGL(one_scan_kernel, dim3((unsigned)NB), dim3(256), 0, st, W, ws.hist, box->device, number);
+  } else if (!few) {
+    if (scan_hist(ws, 1, NB, W, st)) return -1;
+    hipLaunchKernelGGL(one_totals_kernel, dim3(1), dim3(kWave), 0, st, NB, ws.totals, box->device,
+                       number);
+  }
+  STIR_LAUNCH_CHECK();
+  if (!whole && wait_for_answer(*box, NB, st)) return -1;
+  if (whole) STIR_HIP(hipStreamSynchronize(st));
+  STIR_REQUIRE(!box->host->bad_indptr, "%s: indptr is not a CSR row pointer of %lld nonzeros", who, (long long)max_nnz);
+  STIR_REQUIRE(!box->host->bad_range, "%s: a column index lies outside [0, %d)", who, num_cols);
+  for (int k = 0; k < NB; ++k) nrows[k] = stir::answered_rows(box->host->rows[k]);
+  for (int k = 0; k < NB; ++k)
+    STIR_REQUIRE(nrows[k] < kMaxSlots / buckets[k], "%s: bucket %d holds too many slots", who, k);
+  return 0;
+}
+
+}  // namespace stir
+
 extern "C" {
 
 size_t stir_column_part_hyb_device_workspace_bytes(int32_t num_rows, int32_t num_col_parts,
@@ -1417,50 +1470,13 @@ int stir_column_part_hyb_device_values(int32_t num_rows, int32_t num_cols, const
   return 0;
 }
 
+// Programs in C have been promised that the stream is done then: they may fill on another stream, or use the workspace
+// there after an error.
 int stir_column_part_hyb_one_sizes(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr,
                                    const int32_t* d_indices, int64_t max_nnz, const int32_t* buckets,
                                    int32_t num_buckets, void* d_workspace, int64_t* nrows, void* stream) {
-  const char* who = "ColumnPartHyb(device)";
-  if (check_args(who, num_rows, num_cols, 1, buckets, num_buckets)) return -1;
-  STIR_REQUIRE(num_buckets <= kOneBuckets, "%s: %d buckets, at most %d are supported here", who, num_buckets, kOneBuckets);
-  STIR_REQUIRE(nrows && max_nnz >= 0, "%s: bad arguments", who);
-  const int NB = num_buckets, m = num_rows;
-  std::fill(nrows, nrows + NB, int64_t(0));
-  if (m == 0) return 0;
-  STIR_REQUIRE(d_indptr && d_workspace && (max_nnz == 0 || d_indices), "%s: null pointer argument", who);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const Workspace ws = carve(d_workspace, m, 1, NB);
-  const int64_t W = stir::ceil_div(m, kWave);
-  AnswerBox* box = nullptr;
-  uint32_t* arrived = nullptr;
-  if (answer_box(who, &box, &arrived)) return -1;
-  box->host->bad_range = box->host->bad_indptr = 0;
-  const uint32_t number = box->number = stir::next_call(box->number);
-  stir::forget_answers(box->host->rows, NB);
-  const bool few = W <= kFewCounts;
-  OneWidths widths = {};
-  std::copy(buckets, buckets + NB, widths.w);
-  const int64_t count_blocks = stir::ceil_div(m, 256);
-  const int64_t check_blocks = stir::ceil_div(max_nnz, 256 * kValidatePerThread);
-  STIR_REQUIRE(count_blocks + check_blocks < (int64_t(1) << 31), "%s: too many nonzeros for one launch", who);
-  hipLaunchKernelGGL(one_count_kernel, dim3((unsigned)(count_blocks + check_blocks)), dim3(256), 0, st, m, num_cols,
-                     NB, W, max_nnz, (int)count_blocks, widths, ws, d_indptr, d_indices, box->device, few ? arrived : nullptr, number);
-  STIR_LAUNCH_CHECK();
-  if (!few && W <= kOneScanMax) {
-    hipLaunchKernelGGL(one_scan_kernel, dim3((unsigned)NB), dim3(256), 0, st, W, ws.hist, box->device, number);
-  } else if (!few) {
-    if (scan_hist(ws, 1, NB, W, st)) return -1;
-    hipLaunchKernelGGL(one_totals_kernel, dim3(1), dim3(kWave), 0, st, NB, ws.totals, box->device,
-                       number);
-  }
-  STIR_LAUNCH_CHECK();
-  if (wait_for_answer(*box, NB, st)) return -1;
-  STIR_REQUIRE(!box->host->bad_indptr, "%s: indptr is not a CSR row pointer of %lld nonzeros", who, (long long)max_nnz);
-  STIR_REQUIRE(!box->host->bad_range, "%s: a column index lies outside [0, %d)", who, num_cols);
-  for (int k = 0; k < NB; ++k) nrows[k] = stir::answered_rows(box->host->rows[k]);
-  for (int k = 0; k < NB; ++k)
-    STIR_REQUIRE(nrows[k] < kMaxSlots / buckets[k], "%s: bucket %d holds too many slots", who, k);
-  return 0;
+  return stir::column_part_hyb_one_sizes(num_rows, num_cols, d_indptr, d_indices, max_nnz, buckets, num_buckets,
+                                         d_workspace, nrows, stream, /*whole=*/true);
 }
 
 int stir_column_part_hyb_one_fill(int32_t num_rows, int32_t num_cols, const int32_t* d_indptr,

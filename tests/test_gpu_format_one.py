@@ -1,10 +1,13 @@
 """column_part_hyb for one column partition on the device: the short path with its own sizing, scan and
 placement kernels, against the host routine (which is pinned to the oracle)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import sparsetir_amd as st
+from sparsetir_amd import _lib
 from sparsetir_amd._lib import SparseTIRError
 
 pytestmark = pytest.mark.gpu
@@ -101,3 +104,41 @@ def test_refuses_what_the_arrays_cannot_mean(dev):
         st.column_part_hyb(m, 4, indptr, indices, 1, [1, 2])
     empty = st.column_part_hyb(2, 4, t([0, 0, 0]), t([]), 1, [1, 2])
     assert [x.numel() for x in empty[0][0]] == [0, 0]
+
+
+@pytest.mark.parametrize("m", [300, 64 * 256, 64 * 256 + 1])
+def test_sizes_of_the_c_entry_leave_nothing_running(dev, m):
+    """The C entry for the sizes waits for its kernels, whether it takes the matrix or refuses it: another stream may
+    fill, and use the workspace again, at once."""
+    L, buckets = _lib.lib(), [1, 2, 4, 8]
+    deg = np.random.default_rng(m).integers(0, 11, m)
+    indptr, indices = _csr(m, 700, deg, m)
+    want = st.column_part_hyb(m, 700, indptr, indices, 1, buckets)
+    d_ptr, d_idx = torch.from_numpy(indptr).to(dev), torch.from_numpy(indices).to(dev)
+    nnz = len(indices)
+    ws = torch.zeros(L.stir_column_part_hyb_device_workspace_bytes(m, 1, len(buckets), nnz), dtype=torch.uint8, device=dev)
+    out = [[torch.zeros(w[0][b].shape, dtype=torch.int32, device=dev) for b in range(len(buckets))] for w in want]
+    sizing, filling = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    w32 = np.array(buckets, np.int32)
+    nrows = np.zeros(len(buckets), np.int64)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    host = lambda a: ctypes.c_void_p(a.ctypes.data)
+    sizes = lambda p: L.stir_column_part_hyb_one_sizes(m, 700, ptr(p), ptr(d_idx), nnz, host(w32), len(buckets), ptr(ws),
+                                                       host(nrows), ctypes.c_void_p(sizing.cuda_stream))
+    wrong = d_ptr.clone()
+    wrong[m // 2] = nnz + 1
+    torch.cuda.synchronize()
+    for _ in range(8):
+        assert sizes(wrong) == -1
+        assert sizing.query()
+        assert sizes(d_ptr) == 0
+        assert sizing.query()
+    assert nrows.tolist() == [len(r) for r in want[0][0]]
+    tables = [(ctypes.c_void_p * len(buckets))(*[t.data_ptr() for t in o]) for o in out]
+    assert L.stir_column_part_hyb_one_fill(m, 700, ptr(d_ptr), ptr(d_idx), nnz, None, len(buckets), ptr(ws), *tables, None,
+                                           ctypes.c_void_p(filling.cuda_stream)) == 0
+    filling.synchronize()
+    for got, w in zip(out, want):
+        for b in range(len(buckets)):
+            assert np.array_equal(got[b].cpu().numpy(), w[0][b])

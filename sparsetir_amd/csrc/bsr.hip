@@ -67,23 +67,27 @@ __device__ __forceinline__ bool decode_tile(int64_t L, int64_t slices, int f_til
   return (L >> 3) < per && t < total;
 }
 
-// The same when the slices are numbered by rank (row_of_rank): where XCDs share a feature tile, each takes ranks from
-// the whole range in proportion to its share, so that none has the long ones.  With n of them here and m at another
-// XCD, the k-th here comes after those there whose (2 k' + 1) / m is smaller than (2 k + 1) / n.
-__device__ __forceinline__ bool decode_ranked(int64_t L, int64_t slices, int f_tiles, int64_t& slice, int& f_tile) {
-  const int64_t total = slices * f_tiles, per = (total + 7) >> 3;
+// The same when the block rows are numbered by rank (row_of_rank), `sub` slices each that stay together: they read the
+// same X.  Where XCDs share a feature tile, each takes ranks from the whole range in proportion to its share, so that
+// none has the long ones.  With n of them here and m at another XCD, the k-th here comes after those there whose
+// (2 k' + 1) / m is smaller than (2 k + 1) / n.
+__device__ __forceinline__ bool decode_ranked(int64_t L, int64_t slices, int sub, int f_tiles, int64_t& slice,
+                                              int& f_tile) {
+  const int64_t rows = slices / sub, total = rows * f_tiles, per = (total + 7) >> 3;
   const int x = (int)(L & 7);
-  const int64_t t = x * per + (L >> 3);
-  if ((L >> 3) >= per || t >= total) return false;
-  f_tile = (int)(t / slices);
-  const int64_t lo = f_tile * slices, hi = lo + slices;
+  const uint32_t at = (uint32_t)(L >> 3);
+  const int64_t t = x * per + at / sub;
+  if (at / sub >= per || t >= total) return false;
+  f_tile = (int)(t / rows);
+  const int64_t lo = f_tile * rows, hi = lo + rows;
   const int64_t first = max(x * per, lo), n = min((x + 1) * per, hi) - first, k = t - first;
-  slice = k;
+  int64_t rank = k;
   for (int y = (int)(lo / per); y < 8 && y * per < hi; ++y) {
     if (y == x) continue;
     const int64_t m = min((y + 1) * per, hi) - max(y * per, lo);
-    slice += ((2 * k + 1) * m + n - (y > x)) / (2 * n);
+    rank += ((2 * k + 1) * m + n - (y > x)) / (2 * n);
   }
+  slice = rank * sub + at % sub;
   return true;
 }
 
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_kernel(int blk, int feat, int64_
   const int sub = blk / (32 * RS);  // slices of 32*RS rows per block row
   if (by_rows) {
     if (!decode_tile_by_rows(blockIdx.x, slices / sub, sub, f_tiles, slice, f_tile)) return;
-  } else if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+  } else if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
                     : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
     return;
   }
@@ -527,14 +531,14 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
   constexpr int KQ = 64 / FCN;  // rows of X per load
   constexpr int XQ = 16 / KQ;   // loads per chunk
   __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
+  if (ONE) blk = 16;
+  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
   int64_t slice;
   int f_tile;
-  if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+  if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
              : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
     return;
   const int lane = threadIdx.x, ii = lane & 15, g = lane >> 4;
-  if (ONE) blk = 16;
-  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
   // the same for all lanes, which the divisions hide from the compiler
   slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
   int i = (int)slice / sub;
@@ -666,13 +670,13 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int 
   constexpr int KQ = kWave / FCN;  // rows of X per load
   constexpr int XQ = kTileK / KQ;  // units per lane and step
   __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
+  const int sub = blk / 32;
   int64_t slice;
   int f_tile;
-  if (ranked ? !decode_ranked(blockIdx.x, slices, f_tiles, slice, f_tile)
+  if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
              : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
     return;
   const int lane = threadIdx.x, n = lane & 31, h = lane >> 5;
-  const int sub = blk / 32;
   // the same for all lanes, which the divisions hide from the compiler
   slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
   int i = (int)slice / sub;
@@ -931,6 +935,9 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int unit = blk % 32 != 0 ? 16 : 32;  // rows of a slice
   const int64_t unit_slices = (int64_t)mb * (blk / unit);
   auto grid_of = [](int64_t n, int tiles) { return 8 * stir::ceil_div(n * tiles, 8); };  // see decode_tile
+  auto grid_in = [&](bool ranked, int sub, int tiles) {  // `sub` slices a block row; ranked: see decode_ranked
+    return ranked ? sub * grid_of(mb, tiles) : grid_of((int64_t)mb * sub, tiles);
+  };
 #define STIR_BSR_TYPES(LAUNCH)                                        \
   if (dtype == STIR_BF16) {                                           \
     if (out_dtype == STIR_F32) LAUNCH(true, 1); else LAUNCH(true, 0); \
@@ -987,7 +994,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
     if (unit_slices * stir::ceil_div(feat, kTileF) >= 8 * cus && feat < (1 << 25) && blk <= 4096) {
       const int f_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
-      const int64_t blocks = grid_of(unit_slices, f_tiles);
+      const int64_t blocks = grid_in(ranked, blk / 16, f_tiles);
       STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
       const dim3 grid((unsigned)blocks), block(kWave);
 #define STIR_BSR_16W(BF, OUT, TF, ONE)                                                                             \
@@ -1052,10 +1059,10 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     const bool wide = narrow ? tiles <= 2 && full && slices * tiles >= 5 * (int64_t)cus : slices * tiles >= 4 * (int64_t)cus;
     const int wf_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
     if (wide || slices * wf_tiles >= 5 * (int64_t)cus) {
-      const int64_t blocks = grid_of(slices, wf_tiles);
-      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
       const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
       const int ranked = rankable && wide && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
+      const int64_t blocks = grid_in(ranked, blk / 32, wf_tiles);
+      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
 #define STIR_BSR_WT(BF, OUT, TF)                                                                                \
   hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT, TF>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices, \
                      wf_tiles, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
@@ -1080,7 +1087,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const bool rows_go_round = 8 * stir::ceil_div((int64_t)mb, 8) * 7 <= 8 * (int64_t)mb;
   const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2 && rows_go_round) ? 1 : 0;
   const int64_t blocks = by_rows ? 8 * stir::ceil_div((int64_t)mb, 8) * sub_rows * f_tiles
-                                 : grid_of(slices, f_tiles);
+                                 : grid_in(ranked, sub_rows, f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   dim3 grid((unsigned)blocks);
 #define STIR_BSR_L(BF, OUT, NTV, RSV)                                                                      \

@@ -35,6 +35,8 @@ def _config(mb, nb, blk, density, feat, seed):
     (650, 200, 32, 0.005, 512),    # two full tiles of 256
     (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles; few steps: as they come
     (70, 90, 96, 0.04, 1440),      # ranked
+    (250, 270, 48, 0.3, 512),      # 16-row slices of blocks of three, ranked, more than 64 blocks in a row
+    (301, 200, 96, 0.09, 544),     # two feature tiles over eight XCDs: the three slices of a block row on one of them
     (257, 250, 32, 0.01, 832),     # ranked, the last of four feature tiles with 64
     (257, 200, 32, 0.08, 832),     # less of X, 16 steps a slice
     (343, 200, 32, 0.01, 736),

@@ -95,10 +95,15 @@ __device__ __forceinline__ bool decode_ranked(int64_t L, int64_t slices, int sub
 // by number.  Workgroups of a launch that walk block rows of equal length side by side move through X together (block
 // columns ascend in a block row) and share a window of it in L2, one turn of resident workgroups after the other:
 // nothing synchronises them, the order only decides what L2 holds.  Every wavefront finds the row from indptr by
-// itself, the length of that rank by halving, then the place among the rows of that length.
+// itself, the length of that rank by halving, then the place among the rows of that length.  More block rows than a
+// wavefront can hold are ranked in equal groups, one after the other: 2048 x 512 blocks of 32, 10 %, 4096 features 1574 us,
+// 2562 as they come; 1500 x 400, 8 %, 2048 features 354, 498; 2048 x 1024 blocks of 16, 10 %, 1024 features 306, 432.
 constexpr int kRankChunks = 16;
 constexpr int kRankRows = kRankChunks * kWave;  // block rows whose lengths a wavefront can hold
 __device__ __forceinline__ int row_of_rank(const int32_t* __restrict__ indptr, int rows, int rank) {
+  const int groups = (rows + kRankRows - 1) / kRankRows, size = (rows + groups - 1) / groups;
+  const int first = rank / size * size;
+  indptr += first, rank -= first, rows = min(size, rows - first);
   const int lane = threadIdx.x & 63;
   int len[kRankChunks], most = 0, least = INT32_MAX;
 #pragma unroll
@@ -140,7 +145,7 @@ __device__ __forceinline__ int row_of_rank(const int32_t* __restrict__ indptr, i
     }
     left -= n;
   }
-  return row;
+  return first + row;
 }
 
 // 8 consecutive k of one feature per lane, from a feature-contiguous image: two transposing reads `next`
@@ -982,14 +987,13 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   //   16-row slices: 1024 x 1024 blocks, 10 %, 256 features 54 / 47, 384 76 / 68, 512 86 / 85, 1024 157 / 180, 1536 241 /
   //   319; 1024 x 400 (3.3 MB), 256 30 / 23, 1024 73 / 70, 1536 108 / 100; 700 x 900, 128 features a tile (3.7 MB), 640
   //   75 / 73; 340 x 340 of 48, 384 82 / 76, 512 101 / 104, 1024 159 / 181.
-  const bool rankable = mb <= kRankRows;
   if (unit == 16) {
     // 256 features per wavefront with much X, unless the last tile would be mostly empty or wavefronts few: 1024 x 1024
     // blocks of 16, 1024 features 158 us (171 with 128), 1006 x 599, 544 features 155 (140).
     const bool much = x_tile_bytes(kWaveF) > kMuchX;
     const bool wide = much && unit_slices * stir::ceil_div(feat, kWaveF) >= 8 * cus &&
                       (kWaveF - 1 - (feat - 1) % kWaveF) * 8 <= feat;
-    const int ranked = rankable && feat >= 512 && x_tile_bytes(wide ? kWaveF : kTileF) > kBeyondL2;
+    const int ranked = feat >= 512 && x_tile_bytes(wide ? kWaveF : kTileF) > kBeyondL2;
     // A wavefront per slice once eight per CU have one: 60 x 200 blocks of 48, 1024 features (1440) 33.1 us against 31.0
     // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
     if (unit_slices * stir::ceil_div(feat, kTileF) >= 8 * cus && feat < (1 << 25) && blk <= 4096) {
@@ -1060,7 +1064,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     const int wf_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
     if (wide || slices * wf_tiles >= 5 * (int64_t)cus) {
       const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
-      const int ranked = rankable && wide && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
+      const int ranked = wide && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
       const int64_t blocks = grid_in(ranked, blk / 32, wf_tiles);
       STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
 #define STIR_BSR_WT(BF, OUT, TF)                                                                                \
@@ -1076,7 +1080,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     }
   }
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
-  const int ranked = rankable && f_tiles >= 4 && x_tile_bytes(kTileF * nt) > kMuchX;
+  const int ranked = f_tiles >= 4 && x_tile_bytes(kTileF * nt) > kMuchX;
   // Blocks of 128 rows and more: block rows dealt to XCDs (decode_tile_by_rows).  Measured at
   // 16384^2, 10 %, 4096 features: 128 x 128 blocks 387 -> 365 us; 64 x 64 blocks (one slice per
   // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an

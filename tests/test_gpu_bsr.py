@@ -99,30 +99,30 @@ def test_bsr_many_workgroups(dev, mb, nb, blk, feat, dtype):
     _check(got, cfg, a32, x32, True, f"mb={mb} blk={blk} feat={feat} {dtype}")
 
 
-@pytest.mark.parametrize("dtype,out32,varied", [(torch.float16, False, False), (torch.bfloat16, True, True)])
-def test_bsr_launch_swept_in_step(dev, dtype, out32, varied):
-    """A launch large enough for the kernel in which as many workgroups as are resident loop over
-    tiles, every workgroup ranking the block rows by length on its own (X rows of one feature tile
-    beyond 3 MB, at least 8 feature tiles, several tiles per resident workgroup).  Every block row
-    must be computed exactly once: compared on the GPU against the same sum formed block by block in
-    fp32 by torch, for all rows.  `varied`: block rows of very different lengths, empty ones and
-    one beyond the 1024 length classes of the ranking."""
-    mb, nb, blk, feat = 1100, 208, 32, 2048
+@pytest.mark.parametrize("dtype,out32,varied,mb", [(torch.float16, False, False, 1100), (torch.bfloat16, True, True, 1100),
+                                                   (torch.float16, True, True, 1000)])
+def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb):
+    """A launch whose block rows are taken in order of their length (row_of_rank: X rows of a feature tile beyond an L2,
+    rows long enough), found by every wavefront on its own: 1000 rows in one group, 1100 in two.  Every block row must be
+    computed exactly once: compared on the GPU against the same sum formed block by block in fp32 by torch, for all
+    rows.  `varied`: block rows of very different lengths, empty ones and a few much longer than the rest."""
+    nb, blk, feat = 400, 32, 2048
     rng = np.random.default_rng(17)
     if varied:
         nb = 1300
         dens = rng.choice([0.0, 0.002, 0.01, 0.03], size=mb)
         present = rng.random((mb, nb)) < dens[:, None]
-        present[7, :] = True         # 1300 blocks: the last length class
+        present[7, :] = True
         present[8, :1023] = True
         present[9, :1024] = True
     else:
         present = rng.random((mb, nb)) < 0.05
+    assert present.sum() // mb >= 16
     indptr = np.zeros(mb + 1, np.int32)
     np.cumsum(present.sum(axis=1), out=indptr[1:])
     indices = np.nonzero(present)[1].astype(np.int32)
     nnzb = len(indices)
-    assert nb * blk * 256 * 2 > 3 << 20 and feat // 256 >= 8
+    assert nb * blk * 256 * 2 > 4 << 20 and feat // 256 >= 8
     gen = torch.Generator(device=dev).manual_seed(3)
     a = (torch.randn(nnzb * blk * blk, device=dev, generator=gen) * 0.02).to(dtype)
     x = torch.randn(nb * blk * feat, device=dev, generator=gen).to(dtype)

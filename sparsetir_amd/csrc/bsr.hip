@@ -939,6 +939,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int cus = stir::compute_units();
   const int unit = blk % 32 != 0 ? 16 : 32;  // rows of a slice
   const int64_t unit_slices = (int64_t)mb * (blk / unit);
+  const int64_t steps = nnzb * (blk / 16) / 2 / mb;  // of a slice, 32 columns each, on average
   auto grid_of = [](int64_t n, int tiles) { return 8 * stir::ceil_div(n * tiles, 8); };  // see decode_tile
   auto grid_in = [&](bool ranked, int sub, int tiles) {  // `sub` slices a block row; ranked: see decode_ranked
     return ranked ? sub * grid_of(mb, tiles) : grid_of((int64_t)mb * sub, tiles);
@@ -958,8 +959,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     const int f_tiles = (int)stir::ceil_div(feat, kSplitF);
     const int64_t blocks = grid_of(unit_slices, f_tiles);
     const int64_t at_once = (unit == 16 ? 4 : 2) * (int64_t)cus;
-    const int64_t row_steps = nnzb * (blk / 16) / 2 / mb;  // steps of a block row, on average
-    if (blocks <= at_once || (blocks <= 2 * at_once && row_steps >= (unit == 16 ? 24 : 32))) {
+    if (blocks <= at_once || (blocks <= 2 * at_once && steps >= (unit == 16 ? 24 : 32))) {
       const dim3 grid((unsigned)blocks), block(kWave * kSplitWaves);
 #define STIR_BSR_S(BF, OUT)                                                                                  \
   if (unit == 16)                                                                                            \
@@ -975,28 +975,50 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     }
   }
   auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
-  constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000;
-  // Slices in order of their length (row_of_rank) where the rows of X of a feature tile are more than an XCD's L2 holds
-  // beside A, so that what runs side by side reads the same of them.  Finding the row costs 2 to 3 us a tile, which
-  // few feature tiles do not give back: from four on (16-row slices: 512 features).  In order of length / as they come, us:
-  //   wavefronts of 32 x 256 (512 block rows unless noted): 500 columns of blocks, 8 %, 512 features 55.5 / 50.6, 768 77.8 /
-  //   78.3, 832 85.9 / 92.2, 1536 128 / 159, 4096 of 10 % 374 / 662; 260 (4.3 MB of X in a tile), 832 35 / 34 (5 %), 1504
-  //   55 / 59, 4096 116 / 122; 200 (3.3 MB), 832 31.0 / 27.6, 1504 46.5 / 42.3, but with 15 % 95 / 96, 2048 110 / 116:
-  //   there from 16 steps in a block row on;
-  //   four wavefronts: blocks of 64, 256 x 256, 10 %, 256 features 37.5 / 34.7, 384 50.7 / 48.2, 512 58.7 / 61.3;
-  //   16-row slices: 1024 x 1024 blocks, 10 %, 256 features 54 / 47, 384 76 / 68, 512 86 / 85, 1024 157 / 180, 1536 241 /
-  //   319; 1024 x 400 (3.3 MB), 256 30 / 23, 1024 73 / 70, 1536 108 / 100; 700 x 900, 128 features a tile (3.7 MB), 640
-  //   75 / 73; 340 x 340 of 48, 384 82 / 76, 512 101 / 104, 1024 159 / 181.
+  constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kLastLevel = 256 << 20;
+  const int64_t wide_tiles = stir::ceil_div(feat, kWaveF), waste = wide_tiles * kWaveF - feat;
+  // Slices in order of their length (row_of_rank) where that makes up for finding the row, which costs as much as 2 or 3
+  // steps: with the rows of X of a feature tile (x_bytes) more than an XCD's L2 holds beside A, since what runs side by
+  // side then reads the same of them; and with long block rows, since the longest do not come last.  Not with few
+  // workgroups or wavefronts, which are resident at once in any order.  In order of length / as they come, us:
+  //   wavefronts of 32 x 256, 2048 block rows, 512 columns of blocks (8.4 MB of X in a tile), 1024 features: 3 steps 80 / 62,
+  //   10 steps 141 / 148, 16 184 / 218, 32 270 / 389; 305 columns (5 MB) 16 steps 156 / 154, 32 254 / 279; 256 features, 512
+  //   columns, 16 steps 63 / 54;
+  //   four wavefronts, blocks of 64: 1024 rows, 256 columns, 1024 features 12 steps 141 / 119, 24 208 / 209, 48 345 / 387;
+  //   128 features a tile: 256 rows, 512 features 12 steps 24.5 / 22.3, 1024 rows, 24 steps 126 / 132, 48 224 / 246; lengths
+  //   that differ by a factor of ten, 500 rows, 152 columns, 512 features 33 steps 78 / 113;
+  //   16-row slices, 1025 columns (8.4 MB), 1024 features: 1024 rows 10 steps 56 / 56, 18 78 / 85, 40 138 / 156, 4096 rows 10
+  //   steps 197 / 227, 40 523 / 788.
+  // Among those that come as they are, wavefronts of 128 features, whose X an L2 still holds, pass those of 256 then (10
+  // steps of the first and of the last 127 and 165 us).
+  auto rank_pays = [&](int64_t x_bytes, int64_t tiles, int64_t count, int per_cu) {
+    return x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && count >= per_cu * (int64_t)cus &&
+           (steps >= 28 || (steps >= 16 && tiles >= 2 && x_bytes > kBeyondL2));
+  };
   if (unit == 16) {
-    // 256 features per wavefront with much X, unless the last tile would be mostly empty or wavefronts few: 1024 x 1024
-    // blocks of 16, 1024 features 158 us (171 with 128), 1006 x 599, 544 features 155 (140).
-    const bool much = x_tile_bytes(kWaveF) > kMuchX;
-    const bool wide = much && unit_slices * stir::ceil_div(feat, kWaveF) >= 8 * cus &&
-                      (kWaveF - 1 - (feat - 1) % kWaveF) * 8 <= feat;
-    const int ranked = feat >= 512 && x_tile_bytes(wide ? kWaveF : kTileF) > kBeyondL2;
+    // 256 features per wavefront with much X, unless the last tile would be mostly empty, wavefronts few (1024 x 1024
+    // blocks of 16, 1024 features 158 us, 171 with 128; 1006 x 599, 544 features 155, 140) or X as above.  Blocks of
+    // several slices, which read the same X, take 256 whatever X (1100 x 341 of 48, 10 steps, 1024 features 126 us, 136 with
+    // 128; 500 x 37 of 80, 20 steps, 1504 features 283, 334), but for short rows; and whatever the last tile if
+    // A, which every tile reads, is more than the last level holds (3000 x 68 of 80, 20 steps, 800 features 957, 1340).
+    const bool several = blk > 16;
+    const int64_t waves = unit_slices * wide_tiles, narrow_tiles = stir::ceil_div(feat, kTileF);
+    const bool fits = waves >= 8 * cus &&
+                      (waste * 8 <= feat || (several && feat > kTileF && nnzb * blk * blk * 2 > kLastLevel));
+    const bool rank_wide = fits && rank_pays(x_tile_bytes(kWaveF), wide_tiles, waves, 8);
+    const bool wide = rank_wide || (fits && (several ? x_tile_bytes(kWaveF) > kMuchX || steps >= 16
+                                                     : x_tile_bytes(kWaveF) > kMuchX && x_tile_bytes(kWaveF) <= kBeyondL2));
+    const bool ranked =
+        rank_wide || (!fits && rank_pays(x_tile_bytes(kTileF), narrow_tiles, unit_slices * narrow_tiles, 10));
     // A wavefront per slice once eight per CU have one: 60 x 200 blocks of 48, 1024 features (1440) 33.1 us against 31.0
     // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
-    if (unit_slices * stir::ceil_div(feat, kTileF) >= 8 * cus && feat < (1 << 25) && blk <= 4096) {
+    // Nor where blocks of several slices would take 128 features and either have less than a turn (600 x 650 of 48, 7 steps,
+    // 256 features, 3600 wavefronts 37, 28) or far more X than an L2 holds (1214 x 659 of 80, 10 steps, 416 features, 27 MB
+    // 178, 134; but 3693 x 559 of 48, 320 features, 13.7 MB 194, 238).
+    const bool narrow_loses =
+        several && !wide && !ranked && feat >= kWaveF && x_tile_bytes(kWaveF) > kMuchX &&
+        (unit_slices * narrow_tiles < 16 * cus || x_tile_bytes(kWaveF) > 5 * kBeyondL2);
+    if (unit_slices * narrow_tiles >= 8 * cus && !narrow_loses && feat < (1 << 25) && blk <= 4096) {
       const int f_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
       const int64_t blocks = grid_in(ranked, blk / 16, f_tiles);
       STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
@@ -1047,24 +1069,21 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
   dim3 block(256);
   // With much X, slices of 32 rows by one wavefront each once there are enough of them: 219 x 201 blocks, 1504 features
-  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 512 x 309, 192 features (1024 of 128) 26.1 against 25.0 by workgroups.
-  // 256 features to a wavefront read A half as often and take the ranked order; up to three such tiles, and for five
-  // where 128 features of X fit an L2, that is less than what empty parts of the last tile, too few wavefronts or a
-  // last turn of a quarter cost, except for one or two full tiles and enough wavefronts.  256 (ranked from four tiles
-  // on) / 128 features, 10 % of 512 x 309 blocks unless noted: 288 42.8 / 33.4, 416 43 / 39.7, 544 60 / 54, 800 68 / 76;
-  // 1024 x 500, 96 features 63 / 39, 384 103 / 85; 512 x 500, 8 %, 640 71 / 68, 768 78 / 74, 1024 84 / 102; 512 x 260, 8 %,
-  // 1152 70 / 60, 1280 69 / 65; 300 x 512, 5 %, 1152 52 / 57; 150 x 200 of 96, 16 %, 512 features 102 / 121; 1500 x 400,
-  // 8 %, 512 113 / 114, 256 55 / 59.  Where 256 leave fewer than four wavefronts per CU, 128 features again: 219 x 300,
-  // 1024 38.2 by workgroups, 35.2; 135 x 512, 5 %, 1536 39.0, 34.1; 85 x 512, 3072 70, 60.
+  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 512 x 309, 192 features (1024 of 128) 26.1 against 25.0 by workgroups; 135 x
+  // 512, 5 %, 1536 features (1620 of 128) 39.0, 34.1.  256 features to a wavefront in the ranked order, and in the other
+  // one where their X is hardly more than an L2 holds and the last tile is full; else 128 (see above; 10 % of 512 x 309
+  // blocks, 288 features 42.8 / 33.4, 544 60 / 54, 800 in ranked order 68 / 76).  Blocks of several slices, which read the
+  // same X, keep to 256 up to twice as much of it, or are left to the workgroups: 400 x 170 of 96 (8.4 MB), 16 steps,
+  // 512 features 50 us ranked, 60 with 256 as they come, 65 with 128, 64 by workgroups; 1300 x 325 (16 MB), 8 steps, 1504
+  // features 310, 352, 429, 280.
   if (rs == 1 && x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && feat < (1 << 25) && blk <= 4096) {
-    const int64_t tiles = stir::ceil_div(feat, kWaveF);
-    const bool full = (tiles * kWaveF - feat) * 8 <= feat;
-    const bool narrow = tiles <= 3 || (tiles == 5 && x_tile_bytes(kTileF) <= kMuchX);
-    const bool wide = narrow ? tiles <= 2 && full && slices * tiles >= 5 * (int64_t)cus : slices * tiles >= 4 * (int64_t)cus;
+    const bool one = blk == 32;
+    const int64_t waves = slices * wide_tiles, x_bytes = x_tile_bytes(std::min(feat, kWaveF));
+    const bool ranked = waste * 3 <= feat && rank_pays(x_bytes, wide_tiles, waves, 5);
+    const bool wide = ranked || (waste * 8 <= feat && (one ? x_bytes <= kBeyondL2 && waves >= 5 * (int64_t)cus
+                                                          : x_bytes <= 2 * kBeyondL2 && waves >= 8 * (int64_t)cus));
     const int wf_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
-    if (wide || slices * wf_tiles >= 5 * (int64_t)cus) {
-      const int64_t steps = nnzb * (blk / kTileK) / mb;  // of a slice, on average
-      const int ranked = wide && wf_tiles >= 4 && (x_tile_bytes(kWaveF) > kBeyondL2 || steps >= 16);
+    if (wide || (one && slices * wf_tiles >= 5 * (int64_t)cus)) {
       const int64_t blocks = grid_in(ranked, blk / 32, wf_tiles);
       STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
 #define STIR_BSR_WT(BF, OUT, TF)                                                                                \
@@ -1080,7 +1099,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     }
   }
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
-  const int ranked = f_tiles >= 4 && x_tile_bytes(kTileF * nt) > kMuchX;
+  const bool ranked = rs == 2 && rank_pays(x_tile_bytes(std::min(feat, kTileF * nt)), f_tiles, slices * f_tiles, 3);
   // Blocks of 128 rows and more: block rows dealt to XCDs (decode_tile_by_rows).  Measured at
   // 16384^2, 10 %, 4096 features: 128 x 128 blocks 387 -> 365 us; 64 x 64 blocks (one slice per
   // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an

@@ -34,9 +34,7 @@ def _config(mb, nb, blk, density, feat, seed):
     (170, 260, 32, 0.02, 992),     # too few for 256 features each
     (650, 200, 32, 0.005, 512),    # two full tiles of 256
     (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles; few steps: as they come
-    (70, 90, 96, 0.04, 1440),      # ranked
-    (250, 270, 48, 0.3, 512),      # 16-row slices of blocks of three, ranked, more than 64 blocks in a row
-    (301, 200, 96, 0.09, 544),     # two feature tiles over eight XCDs: the three slices of a block row on one of them
+    (72, 90, 96, 0.07, 1440),      # ranked, six feature tiles over eight XCDs: the slices of a block row on one of them
     (257, 250, 32, 0.01, 832),     # ranked, the last of four feature tiles with 64
     (257, 200, 32, 0.08, 832),     # less of X, 16 steps a slice
     (343, 200, 32, 0.01, 736),
@@ -77,3 +75,8 @@ def test_bsr_ranked_edges(dev, mb, nb, blk, density, feat, dtype, start):
     x32 = x.float().cpu().numpy().reshape(nb * blk, feat)
     _check(y.float().cpu().numpy().reshape(mb * blk, feat), cfg, a32, x32, out is not torch.float32,
            f"{mb}x{nb} blk {blk} feat {feat} {dtype} start {start}")
+
+
+def test_bsr_ranked_blocks_of_three(dev):
+    """16-row slices of blocks of 48 in the ranked order, more than 64 blocks in a row, an odd number of chunks in most."""
+    test_bsr_ranked_edges(dev, 171, 170, 48, 0.07, 1024, torch.float16, 1)

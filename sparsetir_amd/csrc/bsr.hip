@@ -5,8 +5,9 @@
 // feature axis; a wavefront owns NT 32-feature tiles per 32 rows, each a 32x32 fp32 accumulator
 // fed by v_mfma_f32_32x32x16_{f16,bf16}.  Both operands go through LDS: the MFMA B operand wants
 // 8 consecutive k for one feature per lane while X is feature-contiguous, and the A fragment is
-// shared by the four wavefronts (see bsr_tile).  Blocks of 16 k + 16 rows use bsr16_spmm_kernel, small
-// launches bsr_split_kernel, large ones of 32-row blocks bsr_wave_kernel.
+// shared by the four wavefronts (see bsr_tile).  Slices of 32 rows by a wavefront each where there are many of them
+// (bsr_wave_kernel); odd multiples of 16 rows by bsr16_wave_kernel, or by bsr16_spmm_kernel where those are few;
+// small launches by bsr_split_kernel.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -569,7 +570,8 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
 
   const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
   const int chunks = nblk * sub;
-  // block columns of the 64 blocks from `base` on and of the next 64
+  // Block columns of the 64 blocks from `base` on and of the next 64.  Two chunks that are fetched together never lie on
+  // both sides: 64 blocks are an even number of chunks.
   int base = 0;
   int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
   int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
@@ -582,7 +584,7 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
     for (int b = 0; b < 2; ++b) {
       const bool live = block < nblk;
       const int of = block & (kWave - 1);
-      const int j = ONE || block < base + kWave ? __builtin_amdgcn_readlane(j_lane, of) : __builtin_amdgcn_readlane(j_more, of);
+      const int j = __builtin_amdgcn_readlane(j_lane, of);
       const auto rx = window(X + ((int64_t)j * blk + 16 * col) * feat + f0, live ? 32u * feat : 0);
 #pragma unroll
       for (int q = 0; q < XQ; ++q)

@@ -923,59 +923,31 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, in
   }
 }
 
-}  // namespace
+// How a product is launched.
+struct BsrForm {
+  enum Kernel { kSplit, kWaves, kGroups } kernel;  // eight wavefronts a slice, slices by a wavefront, by four
+  bool wide;     // tiles of 256 features, else of 128 (kSplit: of kSplitF)
+  bool ranked;   // block rows in order of their length
+  bool by_rows;  // block rows dealt to XCDs
+};
 
-static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, int32_t blk, int32_t feat,
-                      int64_t nnzb, const void* d_A, const void* d_X, void* d_Y, const int32_t* d_indptr,
-                      const int32_t* d_indices, const int32_t* d_row_ids, void* stream) {
-  STIR_REQUIRE(dtype == STIR_F16 || dtype == STIR_BF16, "bsr_spmm: dtype must be STIR_F16 or STIR_BF16");
-  STIR_REQUIRE(out_dtype == dtype || out_dtype == STIR_F32, "bsr_spmm: out_dtype must equal dtype or be STIR_F32");
-  STIR_REQUIRE(mb >= 0 && nb >= 0 && nnzb >= 0, "bsr_spmm: bad sizes mb=%d nb=%d", mb, nb);
-  STIR_REQUIRE(blk > 0 && blk % 16 == 0, "bsr_spmm: blk=%d must be a multiple of 16", blk);
-  STIR_REQUIRE(feat > 0 && feat % 32 == 0, "bsr_spmm: feat=%d must be a multiple of 32", feat);
-  if (mb == 0) return 0;
-  STIR_REQUIRE(d_X && d_Y && d_indptr && (nnzb == 0 || (d_A && d_indices)), "bsr_spmm: null pointer argument");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const uint16_t* A = static_cast<const uint16_t*>(d_A);
-  const uint16_t* X = static_cast<const uint16_t*>(d_X);
-  const int cus = stir::compute_units();
-  const int unit = blk % 32 != 0 ? 16 : 32;  // rows of a slice
+inline int slice_rows(int blk, BsrForm::Kernel kernel) {
+  return blk % 32 != 0 ? 16 : kernel == BsrForm::kGroups && blk % 64 == 0 ? 64 : 32;
+}
+
+BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
+  const int unit = slice_rows(blk, BsrForm::kSplit);
   const int64_t unit_slices = (int64_t)mb * (blk / unit);
   const int64_t steps = nnzb * (blk / 16) / 2 / mb;  // of a slice, 32 columns each, on average
-  auto grid_of = [](int64_t n, int tiles) { return 8 * stir::ceil_div(n * tiles, 8); };  // see decode_tile
-  auto grid_in = [&](bool ranked, int sub, int tiles) {  // `sub` slices a block row; ranked: see decode_ranked
-    return ranked ? sub * grid_of(mb, tiles) : grid_of((int64_t)mb * sub, tiles);
-  };
-#define STIR_BSR_TYPES(LAUNCH)                                        \
-  if (dtype == STIR_BF16) {                                           \
-    if (out_dtype == STIR_F32) LAUNCH(true, 1); else LAUNCH(true, 0); \
-  } else {                                                            \
-    if (out_dtype == STIR_F32) LAUNCH(false, 1); else LAUNCH(false, 0); \
-  }
   // The split form wins as long as its workgroups are resident at once (64 KB of LDS with 32-row slices: two per
   // CU; four with 16-row slices), and up to twice as many where block rows have enough steps to pay for the
   // second turn.  Measured with 256 features, split against not: 32-row slices, 500 workgroups of 16 steps 7.8
   // against 10.2 us, 1000 of 16 steps 14.1 against 10.8 us, of 32 steps 19.4 against 21.0 us; 16-row slices,
   // 1000 of 4 steps 7.3 against 7.3 us, 2000 of 16 steps 16.9 against 16.2 us, of 24 steps 20.2 against 21.3 us.
-  {
-    const int f_tiles = (int)stir::ceil_div(feat, kSplitF);
-    const int64_t blocks = grid_of(unit_slices, f_tiles);
-    const int64_t at_once = (unit == 16 ? 4 : 2) * (int64_t)cus;
-    if (blocks <= at_once || (blocks <= 2 * at_once && steps >= (unit == 16 ? 24 : 32))) {
-      const dim3 grid((unsigned)blocks), block(kWave * kSplitWaves);
-#define STIR_BSR_S(BF, OUT)                                                                                  \
-  if (unit == 16)                                                                                            \
-    hipLaunchKernelGGL((bsr_split_kernel<BF, OUT, 16>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
-                       d_Y, d_indptr, d_indices, d_row_ids);                                                 \
-  else                                                                                                       \
-    hipLaunchKernelGGL((bsr_split_kernel<BF, OUT, 32>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
-                       d_Y, d_indptr, d_indices, d_row_ids)
-      STIR_BSR_TYPES(STIR_BSR_S)
-#undef STIR_BSR_S
-      STIR_LAUNCH_CHECK();
-      return 0;
-    }
-  }
+  const int64_t split = 8 * stir::ceil_div(unit_slices * stir::ceil_div(feat, kSplitF), 8);
+  const int64_t at_once = (unit == 16 ? 4 : 2) * cus;
+  if (split <= at_once || (split <= 2 * at_once && steps >= (unit == 16 ? 24 : 32)))
+    return {BsrForm::kSplit, false, false, false};
   auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
   constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kLastLevel = 256 << 20;
   const int64_t wide_tiles = stir::ceil_div(feat, kWaveF), waste = wide_tiles * kWaveF - feat;
@@ -994,9 +966,10 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // Among those that come as they are, wavefronts of 128 features, whose X an L2 still holds, pass those of 256 then (10
   // steps of the first and of the last 127 and 165 us).
   auto rank_pays = [&](int64_t x_bytes, int64_t tiles, int64_t count, int per_cu) {
-    return x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && count >= per_cu * (int64_t)cus &&
+    return x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && count >= per_cu * cus &&
            (steps >= 28 || (steps >= 16 && tiles >= 2 && x_bytes > kBeyondL2));
   };
+  const bool wavefronts = feat < (1 << 25) && blk <= 4096;  // offsets of a load in 32 bits
   if (unit == 16) {
     // 256 features per wavefront with much X, unless the last tile would be mostly empty, wavefronts few (1024 x 1024
     // blocks of 16, 1024 features 158 us, 171 with 128; 1006 x 599, 544 features 155, 140) or X as above.  Blocks of
@@ -1020,56 +993,18 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     const bool narrow_loses =
         several && !wide && !ranked && feat >= kWaveF && x_tile_bytes(kWaveF) > kMuchX &&
         (unit_slices * narrow_tiles < 16 * cus || x_tile_bytes(kWaveF) > 5 * kBeyondL2);
-    if (unit_slices * narrow_tiles >= 8 * cus && !narrow_loses && feat < (1 << 25) && blk <= 4096) {
-      const int f_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
-      const int64_t blocks = grid_in(ranked, blk / 16, f_tiles);
-      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-      const dim3 grid((unsigned)blocks), block(kWave);
-#define STIR_BSR_16W(BF, OUT, TF, ONE)                                                                             \
-  hipLaunchKernelGGL((bsr16_wave_kernel<BF, OUT, TF, ONE>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, ranked, \
-                     A, X, d_Y, d_indptr, d_indices, d_row_ids)
-#define STIR_BSR_16(BF, OUT)                                                                                   \
-  do {                                                                                                         \
-    if (wide) {                                                                                                \
-      if (blk == 16) STIR_BSR_16W(BF, OUT, kWaveF, true); else STIR_BSR_16W(BF, OUT, kWaveF, false);           \
-    } else {                                                                                                   \
-      if (blk == 16) STIR_BSR_16W(BF, OUT, kTileF, true); else STIR_BSR_16W(BF, OUT, kTileF, false);           \
-    }                                                                                                          \
-  } while (0)
-      STIR_BSR_TYPES(STIR_BSR_16)
-#undef STIR_BSR_16
-#undef STIR_BSR_16W
-      STIR_LAUNCH_CHECK();
-      return 0;
-    }
-    const int nt16 = feat >= 256 ? 2 : 1;
-    const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt16);
-    const int64_t blocks = grid_of(unit_slices, f_tiles);
-    STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-    const dim3 grid((unsigned)blocks), block(256);
-#define STIR_BSR_16(BF, OUT)                                                                                  \
-  if (nt16 == 2)                                                                                              \
-    hipLaunchKernelGGL((bsr16_spmm_kernel<BF, OUT, 2>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
-                       d_Y, d_indptr, d_indices, d_row_ids);                                                  \
-  else                                                                                                        \
-    hipLaunchKernelGGL((bsr16_spmm_kernel<BF, OUT, 1>), grid, block, 0, st, blk, feat, unit_slices, f_tiles, A, X, \
-                       d_Y, d_indptr, d_indices, d_row_ids)
-    STIR_BSR_TYPES(STIR_BSR_16)
-#undef STIR_BSR_16
-    STIR_LAUNCH_CHECK();
-    return 0;
+    if (unit_slices * narrow_tiles >= 8 * cus && !narrow_loses && wavefronts)
+      return {BsrForm::kWaves, wide, ranked, false};
+    return {BsrForm::kGroups, feat >= kWaveF, false, false};
   }
-  // two 32-row slices per workgroup when the block height allows it
-  const int rs = (blk % 64 == 0) ? 2 : 1;
+  const int rs = slice_rows(blk, BsrForm::kGroups) / 32;
   const int64_t slices = (int64_t)mb * (blk / (32 * rs));
   // Two 32-wide accumulators per wavefront once the feature axis is wide enough to still yield workgroups for the chip,
   // 1.6 per CU (us with one / two): 22 x 246 blocks of 64, 2752 features (242 workgroups of two) 56 / 63, 45 x 45 of 128,
   // 1024 (360) 20.6 / 21.6, 64 x 400 of 32, 1536 (384) 38.0 / 41.1, 60 x 100 of 64, 2048 (480) 26.0 / 24.5, 70 x 60
   // (560) 34.4 / 29.6, 98 x 90, 2432 (980) 45.8 / 38.6.  One prefetched step is enough: measured on MI355X, deeper
   // register rings (2-6 steps) change nothing, the kernel is not bound by latency.
-  const int nt = feat >= 1024 && slices * stir::ceil_div(feat, 2 * kTileF) * 5 >= 8 * (int64_t)cus ? 2 : 1;
-  const int f_tiles = (int)stir::ceil_div(feat, kTileF * nt);
-  dim3 block(256);
+  const int nt = feat >= 1024 && slices * stir::ceil_div(feat, 2 * kTileF) * 5 >= 8 * cus ? 2 : 1;
   // With much X, slices of 32 rows by one wavefront each once there are enough of them: 219 x 201 blocks, 1504 features
   // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 512 x 309, 192 features (1024 of 128) 26.1 against 25.0 by workgroups; 135 x
   // 512, 5 %, 1536 features (1620 of 128) 39.0, 34.1.  256 features to a wavefront in the ranked order, and in the other
@@ -1078,63 +1013,99 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   // same X, keep to 256 up to twice as much of it, or are left to the workgroups: 400 x 170 of 96 (8.4 MB), 16 steps,
   // 512 features 50 us ranked, 60 with 256 as they come, 65 with 128, 64 by workgroups; 1300 x 325 (16 MB), 8 steps, 1504
   // features 310, 352, 429, 280.
-  if (rs == 1 && x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && feat < (1 << 25) && blk <= 4096) {
+  if (rs == 1 && x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && wavefronts) {
     const bool one = blk == 32;
     const int64_t waves = slices * wide_tiles, x_bytes = x_tile_bytes(std::min(feat, kWaveF));
     const bool ranked = waste * 3 <= feat && rank_pays(x_bytes, wide_tiles, waves, 5);
-    const bool wide = ranked || (waste * 8 <= feat && (one ? x_bytes <= kBeyondL2 && waves >= 5 * (int64_t)cus
-                                                          : x_bytes <= 2 * kBeyondL2 && waves >= 8 * (int64_t)cus));
-    const int wf_tiles = (int)stir::ceil_div(feat, wide ? kWaveF : kTileF);
-    if (wide || (one && slices * wf_tiles >= 5 * (int64_t)cus)) {
-      const int64_t blocks = grid_in(ranked, blk / 32, wf_tiles);
-      STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-#define STIR_BSR_WT(BF, OUT, TF)                                                                                \
-  hipLaunchKernelGGL((bsr_wave_kernel<BF, OUT, TF>), dim3((unsigned)blocks), dim3(kWave), 0, st, blk, feat, slices, \
-                     wf_tiles, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
-#define STIR_BSR_W(BF, OUT) \
-  if (wide) STIR_BSR_WT(BF, OUT, kWaveF); else STIR_BSR_WT(BF, OUT, kTileF)
-      STIR_BSR_TYPES(STIR_BSR_W)
-#undef STIR_BSR_W
-#undef STIR_BSR_WT
-      STIR_LAUNCH_CHECK();
-      return 0;
-    }
+    const bool wide = ranked || (waste * 8 <= feat && (one ? x_bytes <= kBeyondL2 && waves >= 5 * cus
+                                                          : x_bytes <= 2 * kBeyondL2 && waves >= 8 * cus));
+    if (wide || (one && slices * stir::ceil_div(feat, kTileF) >= 5 * cus)) return {BsrForm::kWaves, wide, ranked, false};
   }
+  const int64_t f_tiles = stir::ceil_div(feat, kTileF * nt);
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
   const bool ranked = rs == 2 && rank_pays(x_tile_bytes(std::min(feat, kTileF * nt)), f_tiles, slices * f_tiles, 3);
   // Blocks of 128 rows and more: block rows dealt to XCDs (decode_tile_by_rows).  Measured at
   // 16384^2, 10 %, 4096 features: 128 x 128 blocks 387 -> 365 us; 64 x 64 blocks (one slice per
   // block row, so only A is shared) 443 -> 514 us: there the feature tile per XCD, which keeps an
   // XCD on one slice of X, is worth more.
-  const int sub_rows = blk / (32 * rs);
   // Few block rows do not go round eight XCDs: 12 block rows (40 x 128 columns, 3008 features) 30.8 us, 26.3 in the
   // other order; 20 (of 20, 4096) 33.4, 29.1; 45 (of 45, 1024) 21.6, 24.1.
   const bool rows_go_round = 8 * stir::ceil_div((int64_t)mb, 8) * 7 <= 8 * (int64_t)mb;
-  const int by_rows = (rs == 2 && sub_rows >= 2 && f_tiles >= 2 && rows_go_round) ? 1 : 0;
-  const int64_t blocks = by_rows ? 8 * stir::ceil_div((int64_t)mb, 8) * sub_rows * f_tiles
-                                 : grid_in(ranked, sub_rows, f_tiles);
+  return {BsrForm::kGroups, nt == 2, ranked, rs == 2 && blk >= 128 && f_tiles >= 2 && rows_go_round};
+}
+
+}  // namespace
+
+static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, int32_t blk, int32_t feat,
+                      int64_t nnzb, const void* d_A, const void* d_X, void* d_Y, const int32_t* d_indptr,
+                      const int32_t* d_indices, const int32_t* d_row_ids, void* stream) {
+  STIR_REQUIRE(dtype == STIR_F16 || dtype == STIR_BF16, "bsr_spmm: dtype must be STIR_F16 or STIR_BF16");
+  STIR_REQUIRE(out_dtype == dtype || out_dtype == STIR_F32, "bsr_spmm: out_dtype must equal dtype or be STIR_F32");
+  STIR_REQUIRE(mb >= 0 && nb >= 0 && nnzb >= 0, "bsr_spmm: bad sizes mb=%d nb=%d", mb, nb);
+  STIR_REQUIRE(blk > 0 && blk % 16 == 0, "bsr_spmm: blk=%d must be a multiple of 16", blk);
+  STIR_REQUIRE(feat > 0 && feat % 32 == 0, "bsr_spmm: feat=%d must be a multiple of 32", feat);
+  if (mb == 0) return 0;
+  STIR_REQUIRE(d_X && d_Y && d_indptr && (nnzb == 0 || (d_A && d_indices)), "bsr_spmm: null pointer argument");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint16_t* A = static_cast<const uint16_t*>(d_A);
+  const uint16_t* X = static_cast<const uint16_t*>(d_X);
+  const BsrForm form = bsr_form(stir::compute_units(), mb, nb, blk, feat, nnzb);
+  const int unit = slice_rows(blk, form.kernel), sub = blk / unit;
+  const int f_tiles = (int)stir::ceil_div(feat, form.kernel == BsrForm::kSplit ? kSplitF : form.wide ? kWaveF : kTileF);
+  const int64_t slices = (int64_t)mb * sub;
+  auto eights = [](int64_t n) { return 8 * stir::ceil_div(n, 8); };  // see decode_tile, decode_ranked
+  const int64_t blocks = form.by_rows  ? eights(mb) * sub * f_tiles
+                         : form.ranked ? eights((int64_t)mb * f_tiles) * sub
+                                       : eights(slices * f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
-  dim3 grid((unsigned)blocks);
-#define STIR_BSR_L(BF, OUT, NTV, RSV)                                                                      \
-  hipLaunchKernelGGL((bsr_spmm_kernel<BF, OUT, NTV, RSV>), grid, block, 0, st, blk, feat, slices, f_tiles, \
-                     by_rows, ranked, A, X, d_Y, d_indptr, d_indices, d_row_ids)
-#define STIR_BSR(BF, OUT)                                                          \
-  do {                                                                             \
-    if (nt == 2) {                                                                 \
-      if (rs == 2) STIR_BSR_L(BF, OUT, 2, 2); else STIR_BSR_L(BF, OUT, 2, 1);      \
-    } else {                                                                       \
-      if (rs == 2) STIR_BSR_L(BF, OUT, 1, 2); else STIR_BSR_L(BF, OUT, 1, 1);      \
-    }                                                                              \
+  const dim3 grid((unsigned)blocks);
+  const int ranked = form.ranked, by_rows = form.by_rows;
+#define STIR_BSR_GO(KERNEL, THREADS, ...)                                                                      \
+  hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, st, blk, feat, slices, f_tiles, ##__VA_ARGS__, A, X, d_Y, \
+                     d_indptr, d_indices, d_row_ids)
+#define STIR_BSR(BF, OUT)                                                                                      \
+  do {                                                                                                         \
+    if (form.kernel == BsrForm::kSplit) {                                                                      \
+      if (unit == 16) STIR_BSR_GO((bsr_split_kernel<BF, OUT, 16>), kWave * kSplitWaves);                       \
+      else STIR_BSR_GO((bsr_split_kernel<BF, OUT, 32>), kWave * kSplitWaves);                                  \
+    } else if (form.kernel == BsrForm::kWaves && unit == 16) {                                                 \
+      if (form.wide && blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kWaveF, true>), kWave, ranked);      \
+      else if (form.wide) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kWaveF, false>), kWave, ranked);             \
+      else if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, true>), kWave, ranked);              \
+      else STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, false>), kWave, ranked);                            \
+    } else if (form.kernel == BsrForm::kWaves) {                                                               \
+      if (form.wide) STIR_BSR_GO((bsr_wave_kernel<BF, OUT, kWaveF>), kWave, ranked);                           \
+      else STIR_BSR_GO((bsr_wave_kernel<BF, OUT, kTileF>), kWave, ranked);                                     \
+    } else if (unit == 16) {                                                                                   \
+      if (form.wide) STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 2>), 256);                                        \
+      else STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 1>), 256);                                                  \
+    } else if (unit == 64) {                                                                                   \
+      if (form.wide) STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 2, 2>), 256, by_rows, ranked);                      \
+      else STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 1, 2>), 256, by_rows, ranked);                                \
+    } else {                                                                                                   \
+      if (form.wide) STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 2, 1>), 256, by_rows, ranked);                      \
+      else STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 1, 1>), 256, by_rows, ranked);                                \
+    }                                                                                                          \
   } while (0)
-  STIR_BSR_TYPES(STIR_BSR)
-#undef STIR_BSR_TYPES
+  if (dtype == STIR_BF16) {
+    if (out_dtype == STIR_F32) STIR_BSR(true, 1); else STIR_BSR(true, 0);
+  } else {
+    if (out_dtype == STIR_F32) STIR_BSR(false, 1); else STIR_BSR(false, 0);
+  }
 #undef STIR_BSR
-#undef STIR_BSR_L
+#undef STIR_BSR_GO
   STIR_LAUNCH_CHECK();
   return 0;
 }
 
 extern "C" {
+
+// The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
+// in order of their length, 16 for block rows dealt to XCDs.  For the tests, which say what they cover.
+int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
+  const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb);
+  return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows;
+}
 
 int stir_bsr_spmm(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, int32_t blk, int32_t feat,
                   int64_t nnzb, const void* d_A, const void* d_X, void* d_Y, const int32_t* d_indptr,

@@ -243,3 +243,17 @@ def assert_close(actual, desired, rtol, atol, what=""):
         raise AssertionError(
             f"{what}: {bad.sum()} of {bad.size} elements out of tolerance (rtol={rtol}, atol={atol}); "
             f"worst at flat index {i}: got {actual.ravel()[i]!r}, want {desired.ravel()[i]!r}")
+
+
+def bsr_form(mb, nb, blk, feat, nnzb, cus=256):
+    """How a BSR product is launched on a device of `cus` compute units: the kernel (eight wavefronts to a slice, slices by
+    a wavefront each or by four), features to a tile, block rows in order of their length, block rows dealt to XCDs."""
+    import ctypes
+
+    from sparsetir_amd import _lib
+
+    code = _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb))
+    kernel = ("split", "waves", "groups")[code % 4]
+    if kernel == "split":
+        return kernel
+    return kernel + (" 256" if code & 4 else " 128") + (" ranked" if code & 8 else "") + (" by rows" if code & 16 else "")

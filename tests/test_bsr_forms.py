@@ -1,0 +1,48 @@
+"""How BSR products are launched, on either side of each line that was measured (256 compute units; no GPU needed)."""
+import pytest
+
+from helpers import bsr_form
+
+
+@pytest.mark.parametrize("mb,nb,blk,steps,feat,form", [
+    # 32-row slices: order of length by the steps, the X of a tile and how many wavefronts there are
+    (2048, 512, 32, 10, 1024, "waves 128"),
+    (2048, 512, 32, 16, 1024, "waves 256 ranked"),
+    (2048, 512, 32, 16, 256, "waves 128"),           # one feature tile
+    (2048, 512, 32, 32, 256, "waves 256 ranked"),
+    (2048, 207, 32, 16, 1024, "waves 256"),          # X in an L2
+    (2048, 207, 32, 32, 1024, "waves 256 ranked"),
+    (250, 512, 32, 16, 1024, "waves 128"),           # few
+    (2048, 512, 32, 16, 544, "waves 128"),           # a last tile mostly empty
+    (512, 512, 32, 51, 4096, "waves 256 ranked"),
+    (400, 170, 96, 6, 512, "groups 128"),
+    (400, 170, 96, 16, 512, "waves 256 ranked"),
+    (1300, 325, 96, 8, 1504, "groups 256"),
+    # 64 rows by four wavefronts
+    (1024, 256, 64, 12, 1024, "groups 256"),
+    (1024, 256, 64, 24, 1024, "groups 256 ranked"),
+    (256, 256, 64, 16, 256, "groups 128"),
+    (128, 128, 128, 51, 4096, "groups 256 ranked by rows"),
+    (12, 40, 128, 30, 3008, "groups 128"),
+    (45, 45, 128, 20, 1024, "groups 128 by rows"),
+    # 16-row slices
+    (4096, 1025, 16, 10, 1024, "waves 128"),
+    (4096, 1025, 16, 18, 1024, "waves 256 ranked"),
+    (1024, 420, 16, 10, 512, "waves 256"),
+    (1100, 341, 48, 10, 1024, "waves 256"),
+    (600, 650, 48, 7, 256, "groups 256"),
+    (3693, 559, 48, 11, 320, "waves 128"),
+    (1214, 659, 80, 10, 416, "groups 256"),
+    (3000, 68, 80, 8, 800, "waves 128"),
+    (3000, 68, 80, 20, 800, "waves 256"),            # A beyond the last level
+])
+def test_form(mb, nb, blk, steps, feat, form):
+    nnzb = -(-steps * mb * 32 // blk)
+    assert bsr_form(mb, nb, blk, feat, nnzb) == form
+
+
+def test_sizes_whose_offsets_do_not_fit():
+    """No wavefront form where a load's offset may not fit 32 bits."""
+    assert bsr_form(4, 4, 32, 1 << 25, 16).startswith("groups")
+    assert bsr_form(64, 4, 4096 + 32, 4096, 64).startswith("groups")
+    assert bsr_form(64, 4, 4096 + 16, 4096, 64).startswith("groups")

@@ -5,24 +5,26 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import bsr_f64
+from helpers import bsr_f64, bsr_form
 from sparsetir_amd import datasets, ops
 
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    (1024, 60, 16, 0.1, 224),     # a wavefront per 16-row slice, 128 features
-    (1024, 400, 16, 0.01, 512),   # 256 features
-    (230, 50, 48, 0.05, 352),     # three chunks a block
-    (150, 40, 16, 0.2, 1184),     # 16-row slices by four wavefronts
-    (3, 200, 16, 0.5, 64),        # by eight wavefronts
-    (61, 23, 80, 0.3, 480),
-    (9, 90, 32, 0.6, 96),
-    (343, 200, 32, 0.01, 736),    # a wavefront per 32-row slice
-    (520, 200, 32, 0.01, 800),
-    (397, 30, 32, 0.2, 416),      # four wavefronts
-    (147, 13, 64, 0.3, 2400),
-    (14, 100, 128, 0.05, 160),
+    (1024, 60, 16, 0.1, 224, "waves 128"),     # 16-row slices by a wavefront each
+    (1024, 400, 16, 0.01, 512, "waves 256"),
+    (230, 50, 48, 0.05, 352, "waves 128"),     # three chunks a block
+    (230, 140, 48, 0.03, 1024, "waves 256"),
+    (150, 40, 16, 0.2, 1184, "groups 256"),    # by four wavefronts
+    (61, 23, 80, 0.3, 480, "groups 256"),
+    (3, 200, 16, 0.5, 64, "split"),            # by eight
+    (9, 90, 32, 0.6, 96, "split"),
+    (343, 200, 32, 0.01, 736, "waves 128"),    # 32-row slices by a wavefront each
+    (520, 200, 32, 0.01, 800, "waves 128"),
+    (650, 200, 32, 0.005, 512, "waves 256"),
+    (397, 30, 32, 0.2, 416, "groups 128"),     # by four
+    (147, 13, 64, 0.3, 2400, "groups 256"),
+    (14, 100, 128, 0.05, 160, "split"),
 ]
 
 
@@ -38,11 +40,13 @@ def _without(cfg, cols):
     return cfg
 
 
-@pytest.mark.parametrize("mb,nb,blk,density,feat", SHAPES)
+@pytest.mark.parametrize("mb,nb,blk,density,feat,form", SHAPES)
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-def test_non_finite_x(dev, mb, nb, blk, density, feat, dtype):
+def test_non_finite_x(dev, mb, nb, blk, density, feat, form, dtype):
     unnamed = np.array([0, 1, nb - 1])
     cfg = _without(datasets.config4(seed=mb + feat, mb=mb, nb=nb, blk=blk, density=density, feat=feat), unnamed)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert bsr_form(mb, nb, blk, feat, len(cfg["indices"]), cus) == form
     x = cfg["x"].reshape(nb, blk, feat)
     x[unnamed[0]], x[unnamed[1]], x[unnamed[2]] = np.inf, np.nan, -np.inf
     named = int(cfg["indices"][len(cfg["indices"]) // 2])

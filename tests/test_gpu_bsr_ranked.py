@@ -6,7 +6,8 @@ import pytest
 import torch
 
 from sparsetir_amd import datasets, ops
-from test_gpu_bsr import _check
+from helpers import bsr_form
+from test_gpu_bsr import RTOL, _check
 
 pytestmark = pytest.mark.gpu
 
@@ -24,41 +25,44 @@ def _config(mb, nb, blk, density, feat, seed):
     return cfg
 
 
-@pytest.mark.parametrize("mb,nb,blk,density,feat", [
-    (1024, 193, 32, 0.004, 224),   # 32-row slices by a wavefront each, 128 features: as they come
-    (1030, 200, 32, 0.004, 256),
-    (430, 200, 32, 0.004, 288),    # the last of three tiles with 32
-    (220, 200, 32, 0.01, 672),
-    (150, 200, 32, 0.02, 1056),    # five tiles of 256 would be
-    (150, 70, 96, 0.04, 352),
-    (170, 260, 32, 0.02, 992),     # too few for 256 features each
-    (650, 200, 32, 0.005, 512),    # two full tiles of 256
-    (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles; few steps: as they come
-    (72, 90, 96, 0.07, 1440),      # ranked, six feature tiles over eight XCDs: the slices of a block row on one of them
-    (257, 250, 32, 0.01, 832),     # ranked, the last of four feature tiles with 64
-    (257, 200, 32, 0.08, 832),     # less of X, 16 steps a slice
-    (343, 200, 32, 0.01, 736),
-    (20, 200, 64, 0.03, 96),       # eight wavefronts
-    (12, 100, 128, 0.05, 160),
-    (14, 100, 128, 0.05, 160),
-    (60, 200, 64, 0.03, 416),      # four wavefronts per 64 rows, ranked
-    (33, 100, 128, 0.05, 544),     # too few block rows to deal them to XCDs
-    (36, 100, 128, 0.05, 544),     # block rows dealt to XCDs
-    (40, 20, 64, 0.1, 1056),       # few workgroups: 128 features each
-    (83, 20, 64, 0.1, 1056),       # as many as take 256 features each, the last with 32
-    (1, 6200, 32, 0.001, 64),
-    (1030, 90, 16, 0.02, 224),     # 16-row slices by a wavefront each: plain order
-    (1024, 400, 16, 0.004, 512),   # 256 features
-    (512, 520, 16, 0.004, 1024),   # ranked, 256 features
-    (700, 400, 16, 0.004, 320),    # 128 features, an odd number of blocks
-    (410, 1000, 16, 0.004, 544),   # ranked, 128 features
-    (230, 50, 48, 0.05, 352),      # chunks of two blocks in one step
+def _cus():
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+@pytest.mark.parametrize("mb,nb,blk,density,feat,form", [
+    (1024, 193, 32, 0.004, 224, "groups 128"),
+    (1030, 200, 32, 0.004, 256, "waves 128"),     # 32-row slices by a wavefront each
+    (430, 200, 32, 0.004, 288, "waves 128"),      # the last of three tiles with 32
+    (220, 200, 32, 0.01, 672, "waves 128"),
+    (150, 200, 32, 0.02, 1056, "waves 128"),
+    (150, 70, 96, 0.04, 352, "groups 128"),
+    (170, 260, 32, 0.02, 992, "waves 128"),
+    (650, 200, 32, 0.005, 512, "waves 256"),      # two full tiles of 256
+    (70, 70, 96, 0.04, 1440, "groups 256"),
+    (257, 250, 32, 0.01, 832, "waves 128"),
+    (343, 200, 32, 0.01, 736, "waves 128"),
+    (20, 200, 64, 0.03, 96, "split"),
+    (12, 100, 128, 0.05, 160, "split"),
+    (14, 100, 128, 0.05, 160, "split"),
+    (60, 200, 64, 0.03, 416, "groups 128"),       # four wavefronts per 64 rows
+    (33, 100, 128, 0.05, 544, "groups 128"),      # too few block rows to deal them to XCDs
+    (36, 100, 128, 0.05, 544, "groups 128 by rows"),
+    (40, 20, 64, 0.1, 1056, "groups 128"),        # few workgroups
+    (83, 20, 64, 0.1, 1056, "groups 256"),        # as many as take 256 features each, the last with 32
+    (1, 6200, 32, 0.001, 64, "split"),
+    (1030, 90, 16, 0.02, 224, "waves 128"),       # 16-row slices by a wavefront each
+    (1024, 400, 16, 0.004, 512, "waves 256"),
+    (512, 520, 16, 0.004, 1024, "waves 128"),
+    (700, 400, 16, 0.004, 320, "waves 128"),      # an odd number of blocks
+    (410, 1000, 16, 0.004, 544, "waves 128"),
+    (230, 50, 48, 0.05, 352, "waves 128"),        # chunks of two blocks in one step
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("start", [0, 1])
-def test_bsr_ranked_edges(dev, mb, nb, blk, density, feat, dtype, start):
+def test_bsr_ranked_edges(dev, mb, nb, blk, density, feat, form, dtype, start):
     cfg = _config(mb, nb, blk, density, feat, seed=mb + feat) if mb > 2 else datasets.config4(
         seed=1, mb=mb, nb=nb, blk=blk, density=density, feat=feat)
+    assert bsr_form(mb, nb, blk, feat, len(cfg["indices"]), _cus()) == form
     out = torch.float32 if start and dtype is torch.float16 else dtype
 
     def place(values, dt):
@@ -77,6 +81,52 @@ def test_bsr_ranked_edges(dev, mb, nb, blk, density, feat, dtype, start):
            f"{mb}x{nb} blk {blk} feat {feat} {dtype} start {start}")
 
 
-def test_bsr_ranked_blocks_of_three(dev):
-    """16-row slices of blocks of 48 in the ranked order, more than 64 blocks in a row, an odd number of chunks in most."""
-    test_bsr_ranked_edges(dev, 171, 170, 48, 0.07, 1024, torch.float16, 1)
+@pytest.mark.parametrize("mb,nb,blk,density,feat,form", [
+    # 32-row slices by a wavefront each, in order of their length: the last of six feature tiles with 32
+    (257, 250, 32, 0.07, 1312, "waves 256 ranked"),
+    (1024, 250, 32, 0.07, 512, "waves 256 ranked"),    # as many block rows as a wavefront ranks
+    (1025, 250, 32, 0.07, 448, "waves 256 ranked"),    # two groups, of 513 and 512
+    (2051, 200, 32, 0.15, 256, "waves 256 ranked"),    # three, one feature tile for all XCDs, X in an L2 but long rows
+    (72, 90, 96, 0.07, 1440, "waves 256 ranked"),      # six tiles over eight XCDs: the slices of a block row on one of them
+    (40, 60, 160, 0.07, 1760, "waves 256 ranked"),
+    (220, 100, 96, 0.02, 1024, "waves 256"),
+    # 64 rows by four wavefronts
+    (200, 250, 64, 0.05, 416, "groups 128 ranked"),
+    (100, 130, 64, 0.08, 2048, "groups 256 ranked"),
+    (1030, 100, 64, 0.15, 256, "groups 128 ranked"),
+    (33, 100, 128, 0.06, 3072, "groups 256 ranked"),   # too few block rows to deal them to XCDs
+    (44, 100, 128, 0.06, 2304, "groups 256 ranked by rows"),
+    (16, 60, 128, 0.05, 2080, "groups 128 by rows"),
+    (16, 30, 192, 0.1, 1056, "groups 128 by rows"),
+    # 16-row slices
+    (1030, 490, 16, 0.07, 512, "waves 256 ranked"),
+    (430, 1000, 16, 0.04, 672, "waves 128 ranked"),
+    (171, 170, 48, 0.07, 1024, "waves 256 ranked"),
+    (200, 330, 48, 0.05, 608, "waves 128 ranked"),
+    (230, 140, 48, 0.03, 1024, "waves 256"),
+    (110, 40, 80, 0.2, 1024, "waves 256"),             # little X, long rows
+    (400, 140, 48, 0.03, 288, "groups 256"),           # wavefronts of 128 features would be few
+])
+def test_bsr_forms(dev, mb, nb, blk, density, feat, form):
+    """Every form of a launch, with long and empty block rows and columns in any order, against the same sums in fp64 by
+    torch, block by block."""
+    cfg = _config(mb, nb, blk, density, feat, seed=mb + feat)
+    nnzb = len(cfg["indices"])
+    assert bsr_form(mb, nb, blk, feat, nnzb, _cus()) == form
+    dtype, out = ((torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16))[mb & 1]
+    a, x = (torch.from_numpy(cfg[k]).to(dev).to(dtype) for k in ("data", "x"))
+    y = torch.full((mb * blk * feat,), float("nan"), dtype=out, device=dev)
+    d_ptr, d_idx = torch.from_numpy(cfg["indptr"]).to(dev), torch.from_numpy(cfg["indices"]).to(dev)
+    ops.build_bsrmm(mb, nb, nnzb, blk, feat, dtype, out)(a.reshape(-1), x.reshape(-1), y, d_ptr, d_idx)
+    torch.cuda.synchronize()
+    rows_of = torch.repeat_interleave(torch.arange(mb, device=dev), torch.from_numpy(np.diff(cfg["indptr"])).to(dev))
+    want = torch.zeros(mb, blk, feat, dtype=torch.float64, device=dev)
+    scale = torch.zeros_like(want)
+    a64, x64 = a.double(), x.view(nb, blk, feat).double()
+    for lo in range(0, nnzb, 2048):
+        xb = x64[d_idx[lo:lo + 2048].long()]
+        want.index_add_(0, rows_of[lo:lo + 2048], torch.bmm(a64[lo:lo + 2048], xb))
+        scale.index_add_(0, rows_of[lo:lo + 2048], torch.bmm(a64[lo:lo + 2048].abs(), xb.abs()))
+    # the bound of test_gpu_bsr.py: fp32 sums of exact products, and a rounding of the result
+    bound = 1e-5 * scale + (0.0 if out is torch.float32 else RTOL * want.abs()) + 1e-30
+    assert bool(((y.view(mb, blk, feat).double() - want).abs() <= bound).all())

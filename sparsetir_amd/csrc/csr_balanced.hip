@@ -373,8 +373,10 @@ int slice_class(int32_t n, int32_t feat, int64_t nnz) {
 // Up to 32 features no fewer than 256 entries, eight for each of 32 or more lane groups (us with 64 / 256 as the fewest,
 // 512 entries each): 16 k rows, 121 k nonzeros, 8 features 9.7 / 8.7, 9.2; 10 k, 100 k, 32: 9.3 / 8.7, 8.7; 12 k, 200 k,
 // 16: 9.7 / 9.3, 9.5; but 9 k, 115 k, 84 12.1 / 13.6, 12.2; 9 k, 60 k, 128 11.1 / 13.4, 11.0.
-// The other way, uniform columns only: 100 k rows, 1.5 M nonzeros, 128 features 111.4 against 109.3 (skewed: 69.6,
-// 73.0).
+// The other way (us, against some 1100 workgroups of 32 k entries): 100 k rows, 1.5 M nonzeros of uniform columns, 128
+// features 111.4, 109.3 (skewed: 69.6, 73.0); 60 k, 400 k, 32 11.4, 9.7; 50 k, 350 k, 20 11.1, 9.8 and 32 10.7, 9.2; 8 k,
+// 150 k, 500 43.4, 41.4.  Up to 32 features a few entries more or less to a lane group move single sizes by 15 % either
+// way (40 k, 300 k, 28 10.2, 10.9; 60 k, 400 k, 12 8.1, 9.4); the mean over 10 sizes each of 12 to 48 features is 2 % less.
 // More than one turn of the largest workgroups (beyond_a_turn), 512 / 768 / 1024 entries, uniform and skewed columns: a
 // last turn that is nearly empty costs wide rows more, finding the entries narrow ones.
 //   170 k rows, 2 M nonzeros, 8 features 34.3 / 32.1 / 30.9, 32.2 / 30.2 / 29.0; 600 k, 20 M, 4: 265 / 245 / 240,

@@ -800,8 +800,9 @@ inline int resident_max_quads(int feat_out) { return even_tiles(feat_out) ? 2 : 
 //   40 k nodes, 700 k edges, 65 relations 32 -> 64: 44 / 39; 720 k edges, 90 relations 32 -> 32: 35.6 / 31.6;
 //   60 k, 1 M, 65 relations 32 -> 64: 51 / 54; 24 relations 64 -> 64: 50 / 71; 100 k, 2 M, 65 relations 32 -> 64:
 //   77 / 88; 110 k, 1.98 M edges, 90 relations 32 -> 32: 57 / 65.
-// Three launches were not the faster form (one tile to a pass, 65 relations 32 -> 64: 77 / 22 at 144 k edges, 116 / 111
-// at 1.98 M).
+// Three and four would gain with very many edges only (one launch / three, or four: 166 k nodes, 2 M edges, 24 relations
+// 64 -> 128 293 / 231; 50, 64 -> 64 192 / 161; 65, 48 -> 64 165 / 161, 64 -> 64 210 / 202; 1 M edges, 24, 64 -> 128 155 / 150).
+// The other way, narrow inputs: 83 k, 1 M, 16 -> 128 50 relations 98 / 86, 65 104 / 93.
 constexpr int kMaxRelationParts = 2;
 // (fewer edges suffice where a relation's W is large, 64 -> 32 and up: every run of a step fetches it)
 inline int64_t relation_parts_slots(int feat_in, int feat_out) { return feat_in * feat_out >= 2048 ? 850000 : 1300000; }

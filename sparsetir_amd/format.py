@@ -88,6 +88,7 @@ def _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, 
 
 
 def _column_part_hyb_device(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values=None):
+    buckets = list(buckets)  # which may be read only once, and is read again where a path does not take the arguments
     out = _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values)
     if out is not None:
         return out
@@ -107,7 +108,7 @@ def _column_part_hyb_device(num_rows, num_cols, indptr, indices, num_col_parts, 
     out = _column_part_hyb_native(num_rows, num_cols, indptr, indices, num_col_parts, buckets, values)
     if out is not None:
         return out
-    widths = np.ascontiguousarray(np.asarray(list(buckets), dtype=np.int32))
+    widths = np.ascontiguousarray(np.asarray(buckets, dtype=np.int32))
     nb = len(widths)
     nk = num_col_parts * nb
     with torch.cuda.device(dev):

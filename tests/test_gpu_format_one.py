@@ -106,6 +106,21 @@ def test_refuses_what_the_arrays_cannot_mean(dev):
     assert [x.numel() for x in empty[0][0]] == [0, 0]
 
 
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("parts,buckets", [(1, [1, 2, 4]), (2, [1, 2, 4]), (1, list(range(1, 41)))])
+def test_buckets_that_can_be_read_once(dev, strided, parts, buckets):
+    """Widths from an iterator, for arrays that the native path takes and for those that it hands on."""
+    rng = np.random.default_rng(parts)
+    indptr, indices = _csr(200, 60, rng.integers(0, 9, 200), parts)
+    d_idx = torch.from_numpy(np.repeat(indices, 2) if strided else indices).to(dev)
+    got = st.column_part_hyb(200, 60, torch.from_numpy(indptr).to(dev), d_idx[::2] if strided else d_idx, parts, iter(buckets))
+    want = st.column_part_hyb(200, 60, indptr, indices, parts, iter(buckets))
+    for g, w in zip(got, want):
+        for p in range(parts):
+            for b in range(len(buckets)):
+                assert np.array_equal(g[p][b].cpu().numpy(), w[p][b])
+
+
 @pytest.mark.parametrize("m", [300, 64 * 256, 64 * 256 + 1])
 def test_sizes_of_the_c_entry_leave_nothing_running(dev, m):
     """The C entry for the sizes waits for its kernels, whether it takes the matrix or refuses it: another stream may

@@ -98,17 +98,20 @@ def test_bsr_many_workgroups(dev, mb, nb, blk, feat, dtype):
     _check(got, cfg, a32, x32, True, f"mb={mb} blk={blk} feat={feat} {dtype}")
 
 
-@pytest.mark.parametrize("dtype,out32,varied,mb", [(torch.float16, False, False, 1100), (torch.bfloat16, True, True, 1100),
-                                                   (torch.float16, True, True, 1000)])
-def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb):
-    """A launch whose block rows are taken in order of their length, found by every wavefront on its own: 1000 rows in one
-    group, 1100 in two.  Every block row must be
-    computed exactly once: compared on the GPU against the same sum formed block by block in fp32 by torch, for all
-    rows.  `varied`: block rows of very different lengths, empty ones and a few much longer than the rest."""
-    nb, blk, feat = 400, 32, 2048
+@pytest.mark.parametrize("dtype,out32,varied,mb,nb,form", [
+    (torch.float16, False, False, 1100, 208, "waves 256"),         # as they come
+    (torch.float16, False, False, 1100, 400, "waves 256 ranked"),
+    (torch.bfloat16, True, True, 1100, 1300, "waves 256 ranked"),
+    (torch.float16, True, True, 1000, 1300, "waves 256 ranked"),
+])
+def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb, nb, form):
+    """Large launches whose block rows are taken in order of their length, found by every wavefront on its own: 1000 rows
+    in one group, 1100 in two.  Every block row must be computed exactly once: compared on the GPU against the same
+    sum formed block by block in fp32 by torch, for all rows.  `varied`: block rows of very different lengths, empty
+    ones and a few much longer than the rest."""
+    blk, feat = 32, 2048
     rng = np.random.default_rng(17)
     if varied:
-        nb = 1300
         dens = rng.choice([0.0, 0.002, 0.01, 0.03], size=mb)
         present = rng.random((mb, nb)) < dens[:, None]
         present[7, :] = True
@@ -121,7 +124,7 @@ def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb):
     indices = np.nonzero(present)[1].astype(np.int32)
     nnzb = len(indices)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert bsr_form(mb, nb, blk, feat, nnzb, cus) == "waves 256 ranked"
+    assert bsr_form(mb, nb, blk, feat, nnzb, cus) == form
     gen = torch.Generator(device=dev).manual_seed(3)
     a = (torch.randn(nnzb * blk * blk, device=dev, generator=gen) * 0.02).to(dtype)
     x = torch.randn(nb * blk * feat, device=dev, generator=gen).to(dtype)

@@ -371,6 +371,7 @@ __global__ __launch_bounds__(256) void bsr_spmm_kernel(int blk, int feat, int64_
   int64_t slice;
   int f_tile;
   const int sub = blk / (32 * RS);  // slices of 32*RS rows per block row
+  if (RS == 1) by_rows = ranked = 0;  // blocks of 64 rows and more only: see bsr_form
   if (by_rows) {
     if (!decode_tile_by_rows(blockIdx.x, slices / sub, sub, f_tiles, slice, f_tile)) return;
   } else if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
@@ -678,6 +679,7 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int 
   constexpr int XQ = kTileK / KQ;  // units per lane and step
   __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
   const int sub = blk / 32;
+  if (TF != kWaveF) ranked = 0;  // see bsr_form
   int64_t slice;
   int f_tile;
   if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)

@@ -1103,8 +1103,10 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
 extern "C" {
 
 // The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
-// in order of their length, 16 for block rows dealt to XCDs.  For the tests, which say what they cover.
+// in order of their length, 16 for block rows dealt to XCDs; -1 for what no product is.  For the tests, which say what
+// they cover.
 int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
+  if (cus <= 0 || mb <= 0 || nb < 0 || nnzb < 0 || blk <= 0 || blk % 16 != 0 || feat <= 0) return -1;
   const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb);
   return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows;
 }

@@ -1,4 +1,6 @@
 """How BSR products are launched, on either side of each line that was measured (256 compute units; no GPU needed)."""
+import ctypes
+
 import pytest
 
 from helpers import bsr_form
@@ -46,3 +48,11 @@ def test_sizes_whose_offsets_do_not_fit():
     assert bsr_form(4, 4, 32, 1 << 25, 16).startswith("groups")
     assert bsr_form(64, 4, 4096 + 32, 4096, 64).startswith("groups")
     assert bsr_form(64, 4, 4096 + 16, 4096, 64).startswith("groups")
+
+
+@pytest.mark.parametrize("mb,nb,blk,feat,nnzb,cus", [(0, 4, 32, 64, 0, 256), (4, 4, 24, 64, 4, 256), (4, 4, 32, 0, 4, 256),
+                                                     (4, 4, 32, 64, -1, 256), (4, 4, 32, 64, 4, 0)])
+def test_what_no_product_is(mb, nb, blk, feat, nnzb, cus):
+    from sparsetir_amd import _lib
+
+    assert _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb)) == -1

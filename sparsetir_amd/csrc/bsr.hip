@@ -1,13 +1,14 @@
 // BSR SpMM on the gfx950 matrix cores: Y[i-th block row] = sum over stored blocks p of
 // A_p (blk x blk) * X[indices[p]-th block of rows], 16-bit inputs, fp32 accumulation.
 //
-// A workgroup of four wavefronts owns 32 or 64 rows of a block row and a 128*NT-wide slice of the
-// feature axis; a wavefront owns NT 32-feature tiles per 32 rows, each a 32x32 fp32 accumulator
-// fed by v_mfma_f32_32x32x16_{f16,bf16}.  Both operands go through LDS: the MFMA B operand wants
-// 8 consecutive k for one feature per lane while X is feature-contiguous, and the A fragment is
-// shared by the four wavefronts (see bsr_tile).  Slices of 32 rows by a wavefront each where there are many of them
-// (bsr_wave_kernel); odd multiples of 16 rows by bsr16_wave_kernel, or by bsr16_spmm_kernel where those are few;
-// small launches by bsr_split_kernel.
+// Slices of 32 rows: a wavefront owns 32 rows x 128 or 256 features, loads the rows of X into registers eight features to
+// a lane and makes the MFMA B operand (8 consecutive k of one feature per lane) out of them with v_perm: no LDS and no
+// other wavefront is in the way (bsr_direct_kernel, bsr_wave_kernel).  In small launches the wavefronts of a workgroup
+// take the steps of one tile in turn.
+// Slices of 64 rows (blocks that are a multiple of 64, where there are many): a workgroup of four wavefronts owns 64 rows
+// and a 128*NT-wide slice of the feature axis; both operands go through LDS (bsr_tile).  Odd multiples of 16 rows by
+// bsr16_wave_kernel, or by bsr16_spmm_kernel where those are few, or, as the smallest launches of long block rows
+// whatever the block, by bsr_split_kernel.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -655,31 +656,198 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
   }
 }
 
-// ------------------------------------------------------------------ large launches: a wavefront per tile
-// A wavefront owns 32 rows of a block row and TF = 256 features, eight 32x32 accumulators, or 128 where the launch's rule
-// says so.  Its X tile has 16 (8) KB of LDS of its own (image as in bsr_tile), filled from registers that were loaded a
-// step before, so that 8 (12) wavefronts per CU have 144 (120) KB on their way and none waits for another; the A operand
-// is loaded straight into registers.  The first half of a step's operands is read before its first MFMA, the second half
-// as the first is used.
+// ------------------------------------------------------------------ 32-row slices, X in registers
+// Lane (c, g) of a wavefront loads 8 features from each of 8 consecutive rows of X, 16 bytes a row.  Word w of the rows 2 d
+// and 2 d + 1 holds features 2 w, 2 w + 1: two v_perm make word d of the B operands of both, whose column is c.  So the
+// operands of eight MFMA, one for each feature of a lane, cost 32 v_perm and no LDS, the loads are whole 256- or 512-byte
+// pieces of a row, and a lane ends up with eight neighbouring features of a row of Y: one 16-byte store.
+// picks word d of the operand of feature 2 w + odd
+template <typename Rows>
+__device__ __forceinline__ u32x4 operand_of(const Rows& x, int w, int odd) {
+  u32x4 b;
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+    b[d] = __builtin_amdgcn_perm(x[2 * d + 1][w], x[2 * d][w], odd ? 0x07060302 : 0x05040100);
+  return b;
+}
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// eight neighbouring features of a row of Y
+template <bool BF16, int OUT>
+__device__ __forceinline__ void store_eight(void* __restrict__ Y, int64_t at, const float (&v)[8]) {
+  if constexpr (OUT == 1) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+      __builtin_nontemporal_store(f32x4u{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]},
+                                  reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + at + 4 * e));
+  } else {
+    u32x4 w;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) w[t] = to16<BF16>(v[2 * t]) | (uint32_t)to16<BF16>(v[2 * t + 1]) << 16;
+    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + at));
+  }
+}
+
+// A tile of 32 rows x 128 features, 16 accumulators of v_mfma_f32_16x16x32, a step of 32 k in eight loads of X and two of A.
+// W wavefronts take the steps of a block row in turn and meet in LDS at the end (W = 1: none does).  GROUP: W = 1, and a
+// workgroup is four wavefronts with neighbouring tiles of one slice, which find each other's A in L1.
+// Two steps are on their way; nothing is asked for beyond the last one: a load outside its window costs as much as another
+// (128 x 128 blocks of 32, 512 features, four wavefronts 9.8 -> 9.1 us).
+// Against four wavefronts that shared 128 features through LDS and met at a barrier per step, us as part of a graph:
+// 128 x 128 blocks of 32, 10 %, 512 features 11.1 -> 9.1 (W = 4); 256 x 256, 512 features 24.0 -> 20.1 (W = 1); 209 x 46, 2
+// steps a row, 1216 features 9.3 -> 7.8 (W = 1); 451 x 87, 160 features 11.5 -> 9.4 (GROUP); against eight wavefronts with 64
+// features through LDS: 197 x 193, 37 steps, 224 features 23.0 -> 16.3 (W = 4), 131 x 322, 78 steps, 128 features 18.7 ->
+// 14.9 (W = 8).  Small launches are bound by the trips to memory one after the other -- indptr, block columns, rows of X,
+// 2.8 us with the launch -- and then by X and A coming through the L2s, which hold neither (config above: 22 MB, 2.7 us).
+template <bool BF16, int OUT, int W, bool GROUP>
+__global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void bsr_direct_kernel(
+    int blk, int feat, int64_t slices, int f_tiles, const uint16_t* __restrict__ A, const uint16_t* __restrict__ X,
+    void* __restrict__ Y, const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
+    const int32_t* __restrict__ row_ids) {
+  static_assert(!GROUP || W == 1, "a group's wavefronts have tiles of their own");
+  constexpr int D = 2;  // steps on their way
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  int64_t slice;
+  int f_tile;
+  if constexpr (GROUP) {  // tiles slice by slice, an eighth of the workgroups to an XCD
+    const int64_t total = slices * f_tiles, per = (((total + 3) >> 2) + 7) >> 3;
+    const int64_t t = ((blockIdx.x & 7) * per + (blockIdx.x >> 3)) * 4 + wave;
+    if ((blockIdx.x >> 3) >= per || t >= total) return;
+    slice = t / f_tiles, f_tile = (int)(t % f_tiles);
+  } else if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
+    return;
+  }
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  const int sub = blk / 32;  // slices per block row = steps per block
+  const int i = (int)slice / sub, bi0 = (int)slice % sub * 32;
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = f_tile * kTileF;
+  // rows 8 g ... 8 g + 7 of a step's 32; features beyond feat repeat the last ones: nobody stores them
+  const uint32_t xoff = (uint32_t)(8 * g * feat + min(8 * c, feat - f0 - 8)) * 2;
+  const uint32_t aoff = (uint32_t)((bi0 + c) * blk + 8 * g) * 2;
+
+  f32x4 acc[2][8];
+#pragma unroll
+  for (int r = 0; r < 2; ++r)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
+  const int steps = nblk * sub, first = W == 1 ? 0 : wave;
+  if (first < steps) {
+    const int32_t* cols = indices + p_begin;
+    int left = (steps - first + W - 1) / W;
+    int block = first / sub, col = first % sub;  // of the step to fetch next
+    u32x4 x[D][8], a[D][2];
+    auto fetch = [&](int s) {
+      const int j = cols[min(block, nblk - 1)];
+      const auto ra = window(A + (int64_t)(p_begin + block) * blk * blk + 32 * col, (uint32_t)(blk * blk - 32 * col) * 2);
+#pragma unroll
+      for (int r = 0; r < 2; ++r) a[s][r] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + 32 * r * blk, 0, 0);
+      const auto rx = window(X + ((int64_t)j * blk + 32 * col) * feat + f0, 64u * feat);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) x[s][q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * 2 * feat, 0);
+      block += W / sub, col += W % sub;
+      if (col >= sub) col -= sub, ++block;
+    };
+    auto multiply = [&](int s) {
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const u32x4 b = operand_of(x[s], t / 2, t % 2);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) acc[r][t] = mfma16<BF16>(a[s][r], b, acc[r][t]);
+      }
+    };
+    fetch(0);
+    if (left > 1) fetch(1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (; left >= 2 * D; left -= D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        multiply(s);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(s);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    multiply(0);  // one to three are left
+    if (left > 2) fetch(0);
+    if (left > 1) multiply(1);
+    if (left > 2) multiply(0);
+  }
+
+  // acc[r][t][v] is row 16 r + 4 g + v, feature 8 c + t
+  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
+  const bool live = f0 + 8 * c < feat;
+  if constexpr (W == 1) {
+    if (!live) return;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float o[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) o[t] = acc[r][t][v];
+        store_eight<BF16, OUT>(Y, (row0 + 16 * r + v) * feat + f0 + 8 * c, o);
+      }
+  } else {
+    // each wavefront adds 8 / W of the eight rows a lane has
+    __shared__ __attribute__((aligned(16))) f32x4 part[W][16][kWave];
+    const int used = min(steps, W);
+    if (wave < used) {
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            part[wave][(4 * r + v) * 2 + e][lane] =
+                f32x4{acc[r][4 * e][v], acc[r][4 * e + 1][v], acc[r][4 * e + 2][v], acc[r][4 * e + 3][v]};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8 / W; ++q) {
+      const int at = wave * (8 / W) + q;
+      float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        if (w >= used) continue;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const f32x4 p = part[w][at * 2 + e][lane];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
+        }
+      }
+      if (live) store_eight<BF16, OUT>(Y, (row0 + 16 * (at >> 2) + (at & 3)) * feat + f0 + 8 * c, o);
+    }
+  }
+}
+
+// A wavefront owns 32 rows x 256 features, eight accumulators of v_mfma_f32_32x32x16: a step of 32 k is two halves of eight
+// loads of X; as soon as the last operand of a half is made, the next step's half is asked for, so that 8 wavefronts per CU
+// have 128 KB on their way.  A comes in 16-byte pieces in memory order, a step ahead, and through 2 KB of LDS of the
+// wavefront's own into operand order: asked for in operand order, a load touches 32 half lines and costs twice as much.
 // With the ranked order (row_of_rank) the wavefronts of an XCD stay within reach of each other in X: 16384 x 16384,
-// 10 % blocks of 32, 4096 features 595 us with workgroups of four wavefronts, 590 with this kernel in plain order
-// (3.97 GB through the L2s, 31 M misses), 395 with both; 300 x 450 blocks, 3232 features 290 -> 217 us; 1024 x 512,
-// 5 % 702 -> 430.  Bound now by LDS and MFMA latency with two wavefronts per SIMD (330 us with no load at all).
-template <bool BF16, int OUT, int TF>
-__global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles,
-                                                                            int ranked, const uint16_t* __restrict__ A,
-                                                                            const uint16_t* __restrict__ X,
-                                                                            void* __restrict__ Y,
-                                                                            const int32_t* __restrict__ indptr,
-                                                                            const int32_t* __restrict__ indices,
-                                                                            const int32_t* __restrict__ row_ids) {
-  constexpr int FT = TF / 32;      // accumulators
-  constexpr int FCN = TF / 8;      // 16-byte units per row of X
-  constexpr int KQ = kWave / FCN;  // rows of X per load
-  constexpr int XQ = kTileK / KQ;  // units per lane and step
-  __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
+// 10 % blocks of 32, 4096 features, fp16: 565 us in plain order, 378 ranked; 416 with X through LDS, 393 with A in operand
+// order.  Bound by the L2s: 7.7 GB through the L1s (233 us at the 33 TB/s that 16 bytes a lane reach) and 1.75 GB of misses,
+// of which 0.86 are A, read once per feature tile: the products alone take 155 us, the loads alone 366, X without A 267, X
+// out of L2 beside A 286.  Not bound by latency: four wavefronts per CU with two or three steps each on their way 410 us.
+// Two feature tiles side by side on an XCD share A but not the window of X (520 us); A past the L2 is slower (465).
+template <bool BF16, int OUT>
+__global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
+                                                            const uint16_t* __restrict__ A,
+                                                            const uint16_t* __restrict__ X, void* __restrict__ Y,
+                                                            const int32_t* __restrict__ indptr,
+                                                            const int32_t* __restrict__ indices,
+                                                            const int32_t* __restrict__ row_ids) {
+  constexpr int FT = kWaveF / 32;  // accumulators
+  __shared__ __attribute__((aligned(16))) u32x4 piece[2 * kWave];
   const int sub = blk / 32;
-  if (TF != kWaveF) ranked = 0;  // see bsr_form
   int64_t slice;
   int f_tile;
   if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
@@ -692,25 +860,10 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int 
   const int bi0 = ((int)slice % sub) * 32;
   if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
   const int i_out = row_ids ? row_ids[i] : i;
-  const int f0 = f_tile * TF;
-  // staging: unit c of the rows KQ q + kq.  Units beyond feat repeat the last one: features nobody stores.
-  const int c = lane % FCN, kq = lane / FCN;
-  const uint32_t xoff = (uint32_t)(kq * feat + min(8 * c, feat - f0 - 8)) * 2;
-  uint32_t xdst[4 / KQ];
-#pragma unroll
-  for (int q = 0; q < 4 / KQ; ++q) xdst[q] = (uint32_t)(((KQ * q + kq) * FCN + (c ^ (4 * (KQ * q + kq)))) * 16);
-  const uint32_t aoff = (uint32_t)((bi0 + n) * blk + 8 * h) * 2;
-  // operand reads: tile t is 256 bytes behind tile t - 4
-  const int sl = lane & 15, kr = sl >> 2, half16 = (lane >> 4) & 1;
-  uint32_t bread[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int u = 4 * t + 2 * half16 + ((sl & 3) >> 1);
-    bread[t] = (uint32_t)(((2 * h) * 4 * FCN + kr * FCN + (u ^ (4 * kr))) * 16 + (sl & 1) * 8);
-  }
-  auto operand = [&](int m, int t) {
-    return read_b(stage + bread[t % 4] + (t / 4) * 256 + m * 4 * FCN * 64, FCN * 64);
-  };
+  const int f0 = f_tile * kWaveF;
+  // rows 16 m + 8 h ... + 7 of a step's 32; features beyond feat repeat the last ones: nobody stores them
+  const uint32_t xoff = (uint32_t)(8 * h * feat + min(8 * n, feat - f0 - 8)) * 2;
+  const uint32_t aoff = (uint32_t)((bi0 + lane / 4) * blk + 8 * (lane % 4)) * 2;
 
   f32x16 acc[FT];
 #pragma unroll
@@ -719,54 +872,68 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 3) void bsr_wave_kernel(int 
     for (int v = 0; v < 16; ++v) acc[t][v] = 0.f;
 
   const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
-  const int steps = nblk * (blk / kTileK);
-  int pb = 0, k0 = 0;
-  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;  // block columns of 128 blocks (see bsr_tile)
-  int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
-  u32x4 xr[XQ], ar[2];
-  auto fetch = [&]() {  // the next step's; nothing beyond the last
-    const bool live = pb < nblk;
-    const int j = __builtin_amdgcn_readlane(j_lane, pb & (kWave - 1));
-    const auto ra = window(A + (int64_t)(p_begin + pb) * blk * blk + k0, live ? (uint32_t)(blk * blk - k0) * 2 : 0);
+  const int steps = nblk * sub;
+  if (steps > 0) {
+    // the step to fetch next: block `block`, k offset k0; nothing beyond the last, so that no load depends on a branch
+    const int32_t* cols = indices + p_begin;
+    int block = 0, k0 = 0, j = cols[0], j_next = cols[min(1, nblk - 1)];
+    u32x4 x[2][8], ar[2], a[2];
+    auto fetch_a = [&]() {
+      const auto ra = window(A + (int64_t)(p_begin + block) * blk * blk + k0, block < nblk ? (uint32_t)(blk * blk - k0) * 2 : 0);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + 32 * m, 0, 0);
-    const auto rx = window(X + ((int64_t)j * blk + k0) * feat + f0, live ? 64u * feat : 0);
+      for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff, m * 32 * blk, 0);
+    };
+    auto fetch_x = [&](int m) {
+      const auto rx = window(X + ((int64_t)j * blk + k0) * feat + f0, block < nblk ? 64u * feat : 0);
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) xr[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * KQ * 2 * feat, 0);
-    k0 += kTileK;
-    if (k0 == blk) {
-      k0 = 0, ++pb;
-      if ((pb & (kWave - 1)) == 0) {
-        j_lane = j_more;
-        j_more = pb + kWave + lane < nblk ? indices[p_begin + pb + kWave + lane] : 0;
-      }
-    }
-  };
-  if (steps > 0) fetch();
+      for (int q = 0; q < 8; ++q) x[m][q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, (16 * m + q) * 2 * feat, 0);
+    };
+    auto advance = [&]() {
+      k0 += 32;
+      const bool over = k0 == blk;
+      k0 = over ? 0 : k0, block += over, j = over ? j_next : j;
+      j_next = cols[min(block + 1, nblk - 1)];
+    };
+    fetch_a(), fetch_x(0), fetch_x(1), advance();
 #pragma unroll 1
-  for (int it = 0; it < steps; ++it) {
+    for (int it = 0; it < steps; ++it) {
+      // piece 64 m + l is row 16 m + l / 4, k 8 (l % 4) ...
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + xdst[q % (4 / KQ)] + q * KQ / 4 * 4 * FCN * 16) = xr[q];
-    const u32x4 a0 = ar[0], a1 = ar[1];
-    fetch();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    u32x4 b[FT];
+      for (int m = 0; m < 2; ++m) piece[(lane % 4) * 32 + 16 * m + lane / 4] = ar[m];
+      fetch_a();
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < FT; ++t) b[t] = operand(0, t);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 0; t < FT; ++t) {
-      acc[t] = mfma32<BF16>(a0, b[t], acc[t]);
-      b[t] = operand(1, t);
+      for (int m = 0; m < 2; ++m) a[m] = piece[(2 * m + h) * 32 + n];
       __builtin_amdgcn_sched_barrier(0);
-    }
 #pragma unroll
-    for (int t = 0; t < FT; ++t) acc[t] = mfma32<BF16>(a1, b[t], acc[t]);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
+      for (int m = 0; m < 2; ++m) {
+        u32x4 b[2][2];
+        auto pick = [&](int w) { b[w % 2][0] = operand_of(x[m], w, 0), b[w % 2][1] = operand_of(x[m], w, 1); };
+        pick(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          if (w < 3) pick(w + 1); else fetch_x(m);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) acc[2 * w + e] = mfma32<BF16>(a[m], b[w % 2][e], acc[2 * w + e]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      advance();
+    }
   }
-  store_rows<BF16, OUT>(stage, acc, Y, (int64_t)i_out * blk + bi0, feat, f0);
+  // acc[t][v] is row (v % 4) + 4 h + 8 (v / 4), feature 8 n + t
+  if (f0 + 8 * n >= feat) return;
+  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * h;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    float o[8];
+#pragma unroll
+    for (int t = 0; t < FT; ++t) o[t] = acc[t][v];
+    store_eight<BF16, OUT>(Y, (row0 + (v & 3) + 8 * (v >> 2)) * feat + f0 + 8 * n, o);
+  }
 }
 
 // ------------------------------------------------------------------ small launches
@@ -927,13 +1094,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, in
 
 // How a product is launched.
 struct BsrForm {
-  enum Kernel { kSplit, kWaves, kGroups } kernel;  // eight wavefronts a slice, slices by a wavefront, by four
-  bool wide;     // tiles of 256 features, else of 128 (kSplit: of kSplitF)
+  enum Kernel { kSplit, kWaves, kGroups } kernel;  // wavefronts take steps in turn, tiles by a wavefront, by workgroups of four
+  bool wide;     // tiles of 256 features, else of 128 (kSplit by bsr_split_kernel: of kSplitF)
   bool ranked;   // block rows in order of their length
   bool by_rows;  // block rows dealt to XCDs
+  int direct = 0;  // bsr_direct_kernel with so many wavefronts to a tile
 };
 
-inline int slice_rows(int blk, BsrForm::Kernel kernel) {
+inline int slice_rows(int blk, BsrForm::Kernel kernel) {  // blocks that are a multiple of 64 are no direct groups
   return blk % 32 != 0 ? 16 : kernel == BsrForm::kGroups && blk % 64 == 0 ? 64 : 32;
 }
 
@@ -941,16 +1109,39 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
   const int unit = slice_rows(blk, BsrForm::kSplit);
   const int64_t unit_slices = (int64_t)mb * (blk / unit);
   const int64_t steps = nnzb * (blk / 16) / 2 / mb;  // of a slice, 32 columns each, on average
-  // The split form wins as long as its workgroups are resident at once (64 KB of LDS with 32-row slices: two per
-  // CU; four with 16-row slices), and up to twice as many where block rows have enough steps to pay for the
-  // second turn.  Measured with 256 features, split against not: 32-row slices, 500 workgroups of 16 steps 7.8
-  // against 10.2 us, 1000 of 16 steps 14.1 against 10.8 us, of 32 steps 19.4 against 21.0 us; 16-row slices,
-  // 1000 of 4 steps 7.3 against 7.3 us, 2000 of 16 steps 16.9 against 16.2 us, of 24 steps 20.2 against 21.3 us.
+  const bool wavefronts = feat < (1 << 25) && blk <= 4096;  // offsets of a load in 32 bits
   const int64_t split = 8 * stir::ceil_div(unit_slices * stir::ceil_div(feat, kSplitF), 8);
-  const int64_t at_once = (unit == 16 ? 4 : 2) * cus;
-  if (split <= at_once || (split <= 2 * at_once && steps >= (unit == 16 ? 24 : 32)))
-    return {BsrForm::kSplit, false, false, false};
+  const int64_t tiles = unit_slices * stir::ceil_div(feat, kTileF);
   auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
+  if (unit == 32 && wavefronts) {
+    // Tiles of 64 features, by eight wavefronts through LDS, where rows are long and tiles of 128 leave CUs without one or,
+    // hardly more than the CUs, with twice as much as the next: 35 x 437 blocks, 97 steps, 96 features 14.6 us, 16.9 with 128;
+    // 42 x 285, 70 steps, 64 10.6, 11.3; 93 x 431, 106 steps, 320 (279 tiles) 26.0, 29.6; but 136 x 333, 67 steps, 256 (272, and
+    // 544 of 64) 24.1, 20.8.
+    if (steps >= 40 && (split * 4 <= (feat % kSplitF ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus)))
+      return {BsrForm::kSplit, false, false, false};
+    // Steps in turn as long as that leaves a CU little more than two workgroups of four wavefronts, or four of two; us with W =
+    // 1 / 2 / 4: 272 x 121 blocks, 25 steps, 224 features (544 tiles) 18.4 / 16.2 / 15.6, 292 x 182, 16 steps, 224 features
+    // (584) 14.2 / 13.8 / 13.9, 57 x 128, 14 steps, 1536 (684) 12.7 / 12.3 / 13.4, 49 x 78, 17 steps, 1952 (784) 14.3 / 14.3 /
+    // 14.3, 77 x 65, 7 steps, 1312 (847) 10.1 / 10.6 / 11.2; sooner not where there are few steps (192 x 51, 2 steps, 160
+    // features 5.1 / 5.5 / 5.2).  Eight where a CU has one tile and many steps: 131 x 322, 78 steps, 128 features 14.9, four 16.2.
+    const bool few = steps < 4;
+    if (tiles <= cus && steps >= 24) return {BsrForm::kSplit, false, false, false, 8};
+    if (tiles * 4 <= (few ? 6 : 9) * cus) return {BsrForm::kSplit, false, false, false, 4};
+    // Two to four tiles to a slice, few steps and X in an L2: neighbours share A (471 x 75, 7 steps, 160 features 8.2, 9.4 with W =
+    // 1; 220 x 66, 5 steps, 288 features 6.9, 7.6; 396 x 27, 5 steps, 416 features 9.7, 10.5; but 166 x 95, 19 steps, 416 17.0, 16)
+    if (blk == 32 && feat > kTileF && feat <= 4 * kTileF && steps <= 8 && x_tile_bytes(kWaveF) <= 2500000)
+      return {BsrForm::kGroups, false, false, false, 1};
+    if (tiles * 4 <= 13 * cus && !few) return {BsrForm::kSplit, false, false, false, 2};
+  } else {
+    // The split form wins as long as its workgroups are resident at once (two per CU with 32-row slices; four with 16-row
+    // slices), and up to twice as many where block rows have enough steps to pay for the second turn.  Split against not, 256
+    // features: 16-row slices, 1000 workgroups of 4 steps 7.3 against 7.3 us, 2000 of 16 steps 16.9 against 16.2 us, of 24
+    // steps 20.2 against 21.3 us.
+    const int64_t at_once = (unit == 16 ? 4 : 2) * cus;
+    if (split <= at_once || (split <= 2 * at_once && steps >= (unit == 16 ? 24 : 32)))
+      return {BsrForm::kSplit, false, false, false};
+  }
   constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kLastLevel = 256 << 20;
   const int64_t wide_tiles = stir::ceil_div(feat, kWaveF), waste = wide_tiles * kWaveF - feat;
   // Slices in order of their length (row_of_rank) where that makes up for finding the row, which costs as much as 2 or 3
@@ -971,7 +1162,6 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     return x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && count >= per_cu * cus &&
            (steps >= 28 || (steps >= 16 && tiles >= 2 && x_bytes > kBeyondL2));
   };
-  const bool wavefronts = feat < (1 << 25) && blk <= 4096;  // offsets of a load in 32 bits
   if (unit == 16) {
     // 256 features per wavefront with much X, unless the last tile would be mostly empty, wavefronts few (1024 x 1024
     // blocks of 16, 1024 features 158 us, 171 with 128; 1006 x 599, 544 features 155, 140) or X as above.  Blocks of
@@ -1003,25 +1193,28 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
   const int64_t slices = (int64_t)mb * (blk / (32 * rs));
   // Two 32-wide accumulators per wavefront once the feature axis is wide enough to still yield workgroups for the chip,
   // 1.6 per CU (us with one / two): 22 x 246 blocks of 64, 2752 features (242 workgroups of two) 56 / 63, 45 x 45 of 128,
-  // 1024 (360) 20.6 / 21.6, 64 x 400 of 32, 1536 (384) 38.0 / 41.1, 60 x 100 of 64, 2048 (480) 26.0 / 24.5, 70 x 60
+  // 1024 (360) 20.6 / 21.6, 60 x 100 of 64, 2048 (480) 26.0 / 24.5, 70 x 60
   // (560) 34.4 / 29.6, 98 x 90, 2432 (980) 45.8 / 38.6.  One prefetched step is enough: measured on MI355X, deeper
   // register rings (2-6 steps) change nothing, the kernel is not bound by latency.
   const int nt = feat >= 1024 && slices * stir::ceil_div(feat, 2 * kTileF) * 5 >= 8 * cus ? 2 : 1;
-  // With much X, slices of 32 rows by one wavefront each once there are enough of them: 219 x 201 blocks, 1504 features
-  // (1314 wavefronts, 3.3 MB) 42.8 -> 40.5 us; 512 x 309, 192 features (1024 of 128) 26.1 against 25.0 by workgroups; 135 x
-  // 512, 5 %, 1536 features (1620 of 128) 39.0, 34.1.  256 features to a wavefront in the ranked order, and in the other
-  // one where their X is hardly more than an L2 holds and the last tile is full; else 128 (see above; 10 % of 512 x 309
-  // blocks, 288 features 42.8 / 33.4, 544 60 / 54, 800 in ranked order 68 / 76).  Blocks of several slices, which read the
-  // same X, keep to 256 up to twice as much of it, or are left to the workgroups: 400 x 170 of 96 (8.4 MB), 16 steps,
-  // 512 features 50 us ranked, 60 with 256 as they come, 65 with 128, 64 by workgroups; 1300 x 325 (16 MB), 8 steps, 1504
-  // features 310, 352, 429, 280.
-  if (rs == 1 && x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && wavefronts) {
+  // Slices of 32 rows, a wavefront to a tile.  256 features to a wavefront take X through the L1s at twice the length of a load
+  // and A half as often; 128 have more wavefronts, and less X in a tile.  us with 128 / 256: 77 x 65 blocks, 7 steps, 1312
+  // features (462 wavefronts of 256) 10.1 / 11.3, 152 x 56, 8 steps, 1056 (760) 13.2 / 12.1, 403 x 191, 40 steps, 512 (806) 42.5
+  // / 36.8, 307 x 92, 21 steps, 2496 (3070) 73 / 65; a last tile mostly empty 344 x 57, 6 steps, 288 features 10.1 / 11.6; with
+  // much X 117 x 257, 20 steps, 2176 (1053, 4.2 MB) 31.6 / 32.5, 109 x 259, 29 steps, 2208 (981) 40.1 / 35.4, 87 x 423, 55
+  // steps, 2784 (957, 6.9 MB) 78 / 69.  Blocks of several slices, which read the same X, with much of it: 256 up to twice
+  // what an L2 holds, or by workgroups: 400 x 170 of 96 (8.4 MB), 16 steps, 512 features 50 ranked, 60 with 256 as they come,
+  // 65 with 128, 64 by workgroups; 1300 x 325 (16 MB), 8 steps, 1504 features 310, 352, 429, 280.
+  if (rs == 1 && wavefronts) {
     const bool one = blk == 32;
     const int64_t waves = slices * wide_tiles, x_bytes = x_tile_bytes(std::min(feat, kWaveF));
-    const bool ranked = waste * 3 <= feat && rank_pays(x_bytes, wide_tiles, waves, 5);
-    const bool wide = ranked || (waste * 8 <= feat && (one ? x_bytes <= kBeyondL2 && waves >= 5 * cus
-                                                          : x_bytes <= 2 * kBeyondL2 && waves >= 8 * cus));
-    if (wide || (one && slices * stir::ceil_div(feat, kTileF) >= 5 * cus)) return {BsrForm::kWaves, wide, ranked, false};
+    const bool ranked = waste * 3 <= feat && rank_pays(x_bytes, wide_tiles, waves, steps >= 64 && wide_tiles >= 4 ? 3 : 5);
+    const bool wide = ranked || (x_bytes <= kMuchX ? waste * 3 <= feat && waves * 10 >= 27 * cus
+                                 : !one            ? waste * 8 <= feat && x_bytes <= 2 * kBeyondL2 && waves >= 8 * cus
+                                 : steps >= 24     ? waste * 4 <= feat && waves >= 3 * cus
+                                                   : waste * 8 <= feat && x_bytes <= kBeyondL2 && waves >= 5 * cus);
+    if (wide) return {BsrForm::kWaves, true, ranked, false};
+    if (one || x_bytes <= kMuchX) return {BsrForm::kWaves, false, false, false, 1};
   }
   const int64_t f_tiles = stir::ceil_div(feat, kTileF * nt);
   // 16384 x 16384, 10 %, 4096 features: 64 x 64 blocks 424 -> 352 us in ranked order, 128 x 128 345 -> 324
@@ -1053,11 +1246,12 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   const uint16_t* X = static_cast<const uint16_t*>(d_X);
   const BsrForm form = bsr_form(stir::compute_units(), mb, nb, blk, feat, nnzb);
   const int unit = slice_rows(blk, form.kernel), sub = blk / unit;
-  const int f_tiles = (int)stir::ceil_div(feat, form.kernel == BsrForm::kSplit ? kSplitF : form.wide ? kWaveF : kTileF);
+  const int f_tiles = (int)stir::ceil_div(feat, form.kernel == BsrForm::kSplit && !form.direct ? kSplitF : form.wide ? kWaveF : kTileF);
   const int64_t slices = (int64_t)mb * sub;
   auto eights = [](int64_t n) { return 8 * stir::ceil_div(n, 8); };  // see decode_tile, decode_ranked
   const int64_t blocks = form.by_rows  ? eights(mb) * sub * f_tiles
                          : form.ranked ? eights((int64_t)mb * f_tiles) * sub
+                         : form.kernel == BsrForm::kGroups && form.direct ? eights(stir::ceil_div(slices * f_tiles, 4))
                                        : eights(slices * f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   const dim3 grid((unsigned)blocks);
@@ -1067,7 +1261,13 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
                      d_indptr, d_indices, d_row_ids)
 #define STIR_BSR(BF, OUT)                                                                                      \
   do {                                                                                                         \
-    if (form.kernel == BsrForm::kSplit) {                                                                      \
+    if (form.direct) {                                                                                         \
+      if (form.kernel == BsrForm::kGroups) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, true>), 4 * kWave);      \
+      else if (form.direct == 1) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false>), kWave);                   \
+      else if (form.direct == 8) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 8, false>), 8 * kWave);               \
+      else if (form.direct == 4) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 4, false>), 4 * kWave);               \
+      else STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 2, false>), 2 * kWave);                                     \
+    } else if (form.kernel == BsrForm::kSplit) {                                                               \
       if (unit == 16) STIR_BSR_GO((bsr_split_kernel<BF, OUT, 16>), kWave * kSplitWaves);                       \
       else STIR_BSR_GO((bsr_split_kernel<BF, OUT, 32>), kWave * kSplitWaves);                                  \
     } else if (form.kernel == BsrForm::kWaves && unit == 16) {                                                 \
@@ -1076,8 +1276,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       else if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, true>), kWave, ranked);              \
       else STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, false>), kWave, ranked);                            \
     } else if (form.kernel == BsrForm::kWaves) {                                                               \
-      if (form.wide) STIR_BSR_GO((bsr_wave_kernel<BF, OUT, kWaveF>), kWave, ranked);                           \
-      else STIR_BSR_GO((bsr_wave_kernel<BF, OUT, kTileF>), kWave, ranked);                                     \
+      STIR_BSR_GO((bsr_wave_kernel<BF, OUT>), kWave, ranked);                                                  \
     } else if (unit == 16) {                                                                                   \
       if (form.wide) STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 2>), 256);                                        \
       else STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 1>), 256);                                                  \
@@ -1103,12 +1302,12 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
 extern "C" {
 
 // The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
-// in order of their length, 16 for block rows dealt to XCDs; -1 for what no product is.  For the tests, which say what
-// they cover.
+// in order of their length, 16 for block rows dealt to XCDs, 32 times the wavefronts that bsr_direct_kernel has at a tile;
+// -1 for what no product is.  For the tests, which say what they cover.
 int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
   if (cus <= 0 || mb <= 0 || nb < 0 || nnzb < 0 || blk <= 0 || blk % 16 != 0 || feat <= 0) return -1;
   const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb);
-  return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows;
+  return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows + 32 * f.direct;
 }
 
 int stir_bsr_spmm(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, int32_t blk, int32_t feat,

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "lane_operand.h"
 #include "../../include/sparsetir_amd.h"
 
 namespace {
@@ -657,30 +658,23 @@ __global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(in
 }
 
 // ------------------------------------------------------------------ 32-row slices, X in registers
-// Lane (c, g) of a wavefront loads 8 features from each of 8 consecutive rows of X, 16 bytes a row.  Word w of the rows 2 d
-// and 2 d + 1 holds features 2 w, 2 w + 1: two v_perm make word d of the B operands of both, whose column is c.  So the
-// operands of eight MFMA, one for each feature of a lane, cost 32 v_perm and no LDS, the loads are whole 256- or 512-byte
-// pieces of a row, and a lane ends up with eight neighbouring features of a row of Y: one 16-byte store.
-// picks word d of the operand of feature 2 w + odd
-template <typename Rows>
-__device__ __forceinline__ u32x4 operand_of(const Rows& x, int w, int odd) {
-  u32x4 b;
-#pragma unroll
-  for (int d = 0; d < 4; ++d)
-    b[d] = __builtin_amdgcn_perm(x[2 * d + 1][w], x[2 * d][w], odd ? 0x07060302 : 0x05040100);
-  return b;
-}
+// Lane (c, g) of a wavefront loads 8 features from each of 8 consecutive rows of X, 16 bytes a row, and makes eight MFMA
+// operands of them (lane_operand.h): the loads are whole 256- or 512-byte pieces of a row, and eight neighbouring features of a
+// row of Y are one 16-byte store.
+using stir::operand_of;
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// eight neighbouring features of a row of Y
+// Eight neighbouring features of a row of Y, by all four lanes of a quad, which have 32.
 template <bool BF16, int OUT>
 __device__ __forceinline__ void store_eight(void* __restrict__ Y, int64_t at, const float (&v)[8]) {
   if constexpr (OUT == 1) {
+    float d[2][4];  // floats 16 s + 4 (lane % 4) ... of the 32 that begin 8 (lane % 4) before `at`
+    stir::deal_out(v, d);
 #pragma unroll
-    for (int e = 0; e < 2; ++e)
-      __builtin_nontemporal_store(f32x4u{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]},
-                                  reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + at + 4 * e));
+    for (int s = 0; s < 2; ++s)
+      __builtin_nontemporal_store(f32x4u{d[s][0], d[s][1], d[s][2], d[s][3]},
+                                  reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + at + 16 * s - 4 * (threadIdx.x & 3)));
   } else {
     u32x4 w;
 #pragma unroll
@@ -1132,7 +1126,9 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // 1; 220 x 66, 5 steps, 288 features 6.9, 7.6; 396 x 27, 5 steps, 416 features 9.7, 10.5; but 166 x 95, 19 steps, 416 17.0, 16)
     if (blk == 32 && feat > kTileF && feat <= 4 * kTileF && steps <= 8 && x_tile_bytes(kWaveF) <= 2500000)
       return {BsrForm::kGroups, false, false, false, 1};
-    if (tiles * 4 <= 13 * cus && !few) return {BsrForm::kSplit, false, false, false, 2};
+    // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long: 11 x 119 blocks of 128, 92 steps,
+    // 2304 features 50, 57)
+    if (tiles * 4 <= 13 * cus && !few && (blk % 64 != 0 || steps < 48)) return {BsrForm::kSplit, false, false, false, 2};
   } else {
     // The split form wins as long as its workgroups are resident at once (two per CU with 32-row slices; four with 16-row
     // slices), and up to twice as many where block rows have enough steps to pay for the second turn.  Split against not, 256

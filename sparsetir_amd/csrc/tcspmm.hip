@@ -7,7 +7,7 @@
 // fp16 inputs, fp32 accumulation, fp16 or fp32 output.
 //
 // With a plan (stir_tc_plan: the long tiles listed once, longest first, in pieces) a product is one launch of
-// tcspmm_units_kernel.  Bound by the gather of rows of B where there are tiles enough, else by the chain id -> row of B
+// tcspmm_units_kernel, or of tcspmm_direct_kernel above 64 features.  Bound by the gather of rows of B where there are tiles enough, else by the chain id -> row of B
 // -> product of the longest unit.  Before, the tiles of up to 16 steps went as below and the pieces of the others in a
 // second launch, a workgroup of 16 wavefronts each.  Tiles of 16 rows, power-law rows of up to 500 to 17.5 k nonzeros,
 // uniform columns, us: 25.9 k rows, 626 k nonzeros, 32 features 22.4 -> 10.8; 167 k, 3.8 M, 32: 83 -> 66; 24 k, 244 k,
@@ -34,6 +34,7 @@
 
 #include "coherent.h"
 #include "common.h"
+#include "lane_operand.h"
 #include "../../include/sparsetir_amd.h"
 
 namespace {
@@ -43,6 +44,9 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// as stored at any element of C
+typedef uint32_t Half8 __attribute__((ext_vector_type(4), aligned(2)));
+typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kTileF = 128;
 constexpr int kGroup = 16;  // g
@@ -488,6 +492,47 @@ __device__ __forceinline__ void tc_store4(void* C, int64_t off, const float4& v,
   }
 }
 
+// What a workgroup does that has left a partial tile (of one feature tile) in memory.
+template <int T, int TF, int W, int OUT>
+__device__ __forceinline__ void tc_add_pieces(const TcPiece& pc, int64_t io, int f_tile, int f_tiles, int feat, void* C,
+                                              int aligned, float* scratch, uint32_t* arrived) {
+  // Every wavefront waits until its stores have arrived, then one thread counts the workgroup
+  // in: whoever counts last finds the partial tiles of all the others in memory.
+  __shared__ int last_of_tile;
+  const int tid = threadIdx.x, f0 = f_tile * TF;
+  const int64_t elems = (int64_t)T * feat;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    uint32_t* counter = arrived + (int64_t)pc.multi * f_tiles + f_tile;
+    const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = before + 1 == (uint32_t)pc.pieces;
+    if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    last_of_tile = last;
+  }
+  __syncthreads();
+  if (!last_of_tile) return;
+  // C[tile, f0 .. f0 + TF) = the partial tiles added in piece order, rounded once
+  float* first = scratch + (int64_t)pc.first_slot * elems;
+  for (int w = tid; w < T * (TF / 4); w += 64 * W) {
+    const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
+    if (fcol >= feat) continue;
+    const int64_t e = (int64_t)row * feat + fcol;
+    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int p0 = 0; p0 < pc.pieces; p0 += 8) {
+      float4 y[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        y[u] = stir::CoherentPiece(first + min(p0 + u, pc.pieces - 1) * elems, (uint32_t)(elems * 4)).load((uint32_t)e);
+      __builtin_amdgcn_sched_barrier(0);  // all eight, then the sums
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p0 + u < pc.pieces) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
+    }
+    tc_store4<OUT>(C, io * elems + e, sum, aligned);
+  }
+}
+
 template <int T, int NTL, int W, int OUT>
 __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t mb, int f_tiles, int64_t n_pieces,
                                                               const TcPiece* __restrict__ pieces,
@@ -505,7 +550,6 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
   constexpr int ATONCE = NTL * 8 / REGS ? NTL * 8 / REGS : 1;  // 32-feature tiles summed at a time: what fits
   constexpr int RB = ATONCE * REGS * 64 * 4;                   // bytes per wavefront of a sum
   __shared__ __attribute__((aligned(16))) char lds[W * (XB > RB ? XB : RB)];
-  __shared__ int last_of_tile;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int f_tile = (int)(blockIdx.x % f_tiles);
@@ -644,39 +688,181 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
       }
     }
   }
-  if (!part) return;
-  // Every wavefront waits until its stores have arrived, then one thread counts the workgroup
-  // in: whoever counts last finds the partial tiles of all the others in memory.
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t* counter = arrived + (int64_t)pc.multi * f_tiles + f_tile;
-    const uint32_t before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const bool last = before + 1 == (uint32_t)pc.pieces;
-    if (last) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-    last_of_tile = last;
+  if (part) tc_add_pieces<T, TF, W, OUT>(pc, io, f_tile, f_tiles, feat, C, aligned, scratch, arrived);
+}
+
+// A unit of 128 features with the operands made in registers (lane_operand.h): a lane loads 8 features of the eight gathered
+// rows 8 g ... 8 g + 7 of a step, and the row ids it needs for that; no LDS but for the sums over the W wavefronts at the
+// end.  Narrower units, whose rows of B are less than 256 bytes, stay with the kernel above: 8 or 4 bytes a lane fill an L1 at
+// 19 TB/s, 16 bytes at 33.  Through LDS / in registers, us: 169 k rows, 1.17 M nonzeros, 128 features, tiles of 16 rows 63.3 /
+// 57.9, of 32 72 / 65.4; 100 k, 1 M, 256 features, 16 rows 90.4 / 84.4; 150 k, 3 M, skewed columns, 128 86.8 / 81.0.  Bound by the rows of B
+// that miss an L2 (8.2 TB/s for rows out of 32 MB).
+template <int T, int W, int OUT>
+__global__ __launch_bounds__(64 * W, T == 32 ? 2 : T == 16 ? 3 : 4) void tcspmm_direct_kernel(
+    int feat, int64_t mb, int f_tiles, int64_t n_pieces, const TcPiece* __restrict__ pieces, const uint16_t* __restrict__ A,
+    const uint16_t* __restrict__ B, void* __restrict__ C, int aligned, float* scratch, uint32_t* arrived,
+    const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices) {
+  constexpr int TF = 128, RH = T == 32 ? 2 : 1;  // RH: operands of 16 rows
+  constexpr int D = T == 8 ? 1 : 2;              // steps on their way
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int f_tile = (int)(blockIdx.x % f_tiles);
+  const int64_t unit = blockIdx.x / f_tiles;
+  const int f0 = f_tile * TF;
+  TcPiece pc;
+  pc.slot = -1;
+  int64_t io = unit - n_pieces;
+  int s_begin = 0, s_end = 0;
+  if (unit < n_pieces) {
+    pc = pieces[unit];
+    io = pc.tile;
+    // a plan made from other contents of indptr: stay inside the tile as it is now
+    s_begin = pc.step_begin, s_end = min(pc.step_end, tile_steps(indptr, io));
+  } else {
+    if (io >= mb) return;
+    s_end = tile_steps(indptr, io);
+    if (s_end > kWholeSteps) return;  // in the list
   }
-  __syncthreads();
-  if (!last_of_tile) return;
-  // C[tile, f0 .. f0 + TF) = the partial tiles added in piece order, rounded once
-  float* first = scratch + (int64_t)pc.first_slot * elems;
-  for (int w = tid; w < T * (TF / 4); w += 64 * W) {
-    const int row = w / (TF / 4), fcol = f0 + (w % (TF / 4)) * 4;
-    if (fcol >= feat) continue;
-    const int64_t e = (int64_t)row * feat + fcol;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int p0 = 0; p0 < pc.pieces; p0 += 8) {
-      float4 y[8];
+  const int64_t g_begin = indptr[io];
+  const int groups = (int)(indptr[io + 1] - g_begin);
+  const int32_t* rowlist = indices + g_begin * kGroup;
+  const uint16_t* Bf = B + min(f0 + 8 * c, feat - 8);  // features beyond feat repeat the last ones: nobody stores them
+
+  f32x4 acc[RH][8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        y[u] = stir::CoherentPiece(first + min(p0 + u, pc.pieces - 1) * elems, (uint32_t)(elems * 4)).load((uint32_t)e);
-      __builtin_amdgcn_sched_barrier(0);  // all eight, then the sums
+  for (int r = 0; r < RH; ++r)
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (p0 + u < pc.pieces) sum.x += y[u].x, sum.y += y[u].y, sum.z += y[u].z, sum.w += y[u].w;
+    for (int t = 0; t < 8; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // Of a lane's group 2 step + g / 2; of one that is not there, what the group before it has: zeros are put in its place
+  // when the step is multiplied, and nothing is asked for that does not exist.
+  typedef int32_t Ids __attribute__((ext_vector_type(4), aligned(4)));
+  auto group_of = [&](int step) { return min(2 * step + (g >> 1), groups - 1); };
+  Ids ids[2];
+  u32x4 x[D][8], a[D][RH];
+  auto load_ids = [&](int step) {
+    const int32_t* p = rowlist + group_of(step) * kGroup + 8 * (g & 1);
+    ids[0] = *reinterpret_cast<const Ids*>(p), ids[1] = *reinterpret_cast<const Ids*>(p + 4);
+  };
+  auto fetch = [&](int s, int step) {  // whose ids are there
+#pragma unroll
+    for (int r = 0; r < RH; ++r) {
+      a[s][r] = u32x4{0, 0, 0, 0};  // rows T ... 15 of the operand
+      if (T >= 16 || c < T)
+        a[s][r] = *reinterpret_cast<const u32x4*>(A + ((g_begin + group_of(step)) * T + 16 * r + c) * kGroup + 8 * (g & 1));
     }
-    tc_store4<OUT>(C, io * elems + e, sum, aligned);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[s][q] = *reinterpret_cast<const u32x4*>(Bf + (int64_t)ids[q / 4][q % 4] * feat);
+  };
+  auto multiply = [&](int s, int step) {
+    if (2 * step + 1 >= groups) {
+      const uint32_t there = g < 2 ? ~0u : 0u;
+#pragma unroll
+      for (int r = 0; r < RH; ++r)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) a[s][r][d] &= there;
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) x[s][q][w] &= there;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const f16x8 b = __builtin_bit_cast(f16x8, stir::operand_of(x[s], t / 2, t % 2));
+#pragma unroll
+      for (int r = 0; r < RH; ++r)
+        acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a[s][r]), b, acc[r][t], 0, 0, 0);
+    }
+  };
+  // wavefront w takes the steps w, w + W, ...; the ids of a step are asked for a step (of its own) before its rows of B
+  int left = s_end - s_begin > wave ? (s_end - s_begin - wave + W - 1) / W : 0;
+  if (left > 0) {
+    int step = s_begin + wave;
+    const auto later = [&](int by) { return min(step + by * W, s_end - 1); };
+    load_ids(step);
+    if constexpr (D == 1) {
+#pragma unroll 1
+      for (; left > 0; --left, step += W) {
+        fetch(0, step);
+        load_ids(later(1));
+        multiply(0, step);
+      }
+    } else {
+      fetch(0, step);
+      load_ids(later(1));
+      if (left > 1) fetch(1, step + W);
+      load_ids(later(2));
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+      for (; left >= 4; left -= 2) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s, step += W) {
+          multiply(s, step);
+          __builtin_amdgcn_sched_barrier(0);
+          fetch(s, step + 2 * W);
+          load_ids(later(3));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      multiply(0, step);  // one to three are left
+      if (left > 2) fetch(0, step + 2 * W);
+      if (left > 1) multiply(1, step + W);
+      if (left > 2) multiply(0, step + 2 * W);
+    }
   }
+
+  // ---- the sums over the wavefronts: each adds 4 RH / W of the rows a lane has.  acc[r][t][v] is row 16 r + 4 g + v, feature
+  // 8 c + t.
+  __shared__ __attribute__((aligned(16))) f32x4 sums[W][4 * RH][2][64];
+  const int used = min(W, s_end - s_begin);
+  if (wave < used) {
+#pragma unroll
+    for (int at = 0; at < 4 * RH; ++at)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        sums[wave][at][e][lane] = f32x4{acc[at >> 2][4 * e][at & 3], acc[at >> 2][4 * e + 1][at & 3],
+                                        acc[at >> 2][4 * e + 2][at & 3], acc[at >> 2][4 * e + 3][at & 3]};
+  }
+  __syncthreads();
+  const int64_t elems = (int64_t)T * feat;
+  const bool part = pc.slot >= 0;
+  const stir::CoherentPiece partial(scratch + (part ? (int64_t)pc.slot * elems : 0), part ? (uint32_t)(elems * 4) : 0u);
+#pragma unroll
+  for (int q = 0; q < 4 * RH / W; ++q) {
+    const int at = wave * (4 * RH / W) + q, row = 16 * (at >> 2) + 4 * g + (at & 3);
+    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      if (w >= used) continue;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const f32x4 p = sums[w][at][e][lane];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
+      }
+    }
+    const bool there = f0 + 8 * c < feat && (T >= 16 || row < T);  // the same for the four lanes of a quad
+    if (OUT == 0 && !part) {
+      u32x4 w;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[2 * t]) |
+               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[2 * t + 1]) << 16;
+      if (there) *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
+      continue;
+    }
+    float d[2][4];
+    stir::deal_out(o, d);
+    if (!there) continue;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int fcol = f0 + 32 * (c >> 2) + 16 * s + 4 * (c & 3);
+      const float4 v = make_float4(d[s][0], d[s][1], d[s][2], d[s][3]);
+      if (part) partial.store((uint32_t)(row * feat + fcol), v);
+      else *reinterpret_cast<Float4*>(static_cast<float*>(C) + (io * T + row) * feat + fcol) = Float4{v.x, v.y, v.z, v.w};
+    }
+  }
+  if (part) tc_add_pieces<T, TF, W, OUT>(pc, io, f_tile, f_tiles, feat, C, aligned, scratch, arrived);
 }
 
 constexpr int kLongTF = 32 * kLongNT, kLongWaves = 32 / kLongNT;
@@ -726,16 +912,14 @@ template <int T>
 int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n_pieces, const TcPiece* d_pieces, float* d_scratch,
                    uint32_t* d_arrived, const uint16_t* A, const uint16_t* B, void* d_C, const int32_t* d_indptr,
                    const int32_t* d_indices, hipStream_t st) {
-  // Wide units (128 features) fetch A and the row ids once for all of them, narrow ones are more and finer: 128
-  // features of 8401 tiles of 16 rows 58.6 against 63.3 us, of 1250 tiles 16.9 against 14.3 us; 192 features, whose
-  // last wide unit is half empty, 56.4 against 45.6 us; 128 features of 21 k tiles of 8 rows, with little of A
-  // to fetch, 68.3 against 62.7 us, 256 of 12.5 k 86.2 against 91.4.
+  // Units of 128 features above 64 (tcspmm_direct_kernel), their last one however full; us with units of 64 features, by the
+  // kernel above, / of 128: 20 k rows, 300 k nonzeros, 128 features 16.2 / 14.4, 100 k, 500 k, 96 33.6 / 26.0, 120 k, 600 k, 160
+  // 61.2 / 53.7, 60 k, 900 k, 192 66.1 / 56.4 (skewed columns, 32 rows 54.3 / 55.7); and of 64 features alone 60 k, 900 k 25.7 /
+  // 29.5, 200 k, 4 M 66 / 80.
   // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
   // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
-  // 35.5 against 38.3 us; wide units, 5292 tiles of 7 steps 61.0 against 54.2, 3125 of 10 steps 50.7 against 53.0
-  // us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
-  const int past = feat % 128;
-  const bool wide = (T > 8 || feat >= 256) && feat > 64 && (past == 0 || past > 64) && mb * stir::ceil_div(feat, 128) >= 3000;
+  // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
+  const bool wide = feat > 64;
   const int ntl = feat <= 32 ? 1 : wide ? 4 : 2;
   const int f_tiles = (int)stir::ceil_div(feat, 32 * ntl);
   const int64_t blocks = (mb + n_pieces) * f_tiles;
@@ -746,13 +930,18 @@ int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n
   hipLaunchKernelGGL((tcspmm_units_kernel<T, NTL, W, OUT>), dim3((unsigned)blocks), dim3(64 * W), 0, st, feat,       \
                      (int64_t)mb, f_tiles, n_pieces, d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr,   \
                      d_indices)
+#define STIR_TC_D(W, OUT)                                                                                           \
+  hipLaunchKernelGGL((tcspmm_direct_kernel<T, W, OUT>), dim3((unsigned)blocks), dim3(64 * W), 0, st, feat,            \
+                     (int64_t)mb, f_tiles, n_pieces, d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr,   \
+                     d_indices)
 #define STIR_TC_W(NTL, W) if (out32) STIR_TC(NTL, W, 1); else STIR_TC(NTL, W, 0);
   if (pairs) {
-    if (ntl == 1) { STIR_TC_W(1, 2) } else if (ntl == 2) { STIR_TC_W(2, 2) } else { STIR_TC_W(4, 2) }
+    if (ntl == 1) { STIR_TC_W(1, 2) } else if (ntl == 2) { STIR_TC_W(2, 2) } else if (out32) { STIR_TC_D(2, 1); } else { STIR_TC_D(2, 0); }
   } else {
-    if (ntl == 1) { STIR_TC_W(1, 4) } else if (ntl == 2) { STIR_TC_W(2, 4) } else { STIR_TC_W(4, 4) }
+    if (ntl == 1) { STIR_TC_W(1, 4) } else if (ntl == 2) { STIR_TC_W(2, 4) } else if (out32) { STIR_TC_D(4, 1); } else { STIR_TC_D(4, 0); }
   }
 #undef STIR_TC_W
+#undef STIR_TC_D
 #undef STIR_TC
   STIR_LAUNCH_CHECK();
   return 0;

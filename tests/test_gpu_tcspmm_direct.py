@@ -1,0 +1,53 @@
+"""Condensed SpMM of more than 64 features with a plan: tiles of an odd number of groups, whose last step has one group only --
+an infinity among the rows of B that it gathers stays an infinity where every row of the tile has an entry, and reaches no
+other feature -- ragged feature tiles, and arrays that start at an odd element."""
+import numpy as np
+import pytest
+import torch
+
+import sparsetir_amd as st
+from sparsetir_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("t", [8, 16, 32])
+@pytest.mark.parametrize("feat", [96, 128, 224, 288])
+@pytest.mark.parametrize("out_dtype,start", [(torch.float16, 1), (torch.float32, 1), (torch.float32, 0)])
+def test_odd_groups(dev, t, feat, out_dtype, start):
+    rng = np.random.default_rng(feat + t)
+    n, counts = 900, [16, 48, 80, 32, 144, 0, 688]  # columns of a tile: 1, 3, 5, 2, 9, 0 and 43 groups
+    cols = [np.sort(rng.choice(np.arange(1, n), c, replace=False)) for c in counts]
+    rows = [c for c in cols for _ in range(t)]
+    indptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    gptr, tiles, mask = st.condense(indptr, np.concatenate(rows).astype(np.int32), t, 16)
+    mb = len(gptr) - 1
+    a = (mask * rng.uniform(0.1, 1.0, mask.shape)).astype(np.float16)
+    b = rng.standard_normal((n, feat)).astype(np.float16)
+    named = int(cols[1][-1])  # in the last group of the second tile
+    b[named, feat - 1] = np.inf
+
+    def place(v):
+        x = torch.empty(v.size + start, dtype=torch.float16, device=dev)[start:]
+        x.copy_(torch.from_numpy(v.reshape(-1)))
+        return x
+
+    td = lambda v: torch.from_numpy(np.ascontiguousarray(v)).to(dev)
+    c = torch.full((mb * t * feat + start,), float("nan"), dtype=out_dtype, device=dev)[start:]
+    f = ops.build_tcspmm(mb, tiles.shape[0], feat, t, 16, n, out_dtype)
+    f(place(a), place(b), c, td(gptr), td(tiles.ravel()))
+    got = c.float().cpu().numpy().reshape(mb, t, feat)
+    has = np.array([named in k for k in cols])
+    assert np.isposinf(got[has, :, feat - 1]).all()
+    b[named, feat - 1] = 0.0
+    got[has, :, feat - 1] = 0.0
+    for io in range(mb):
+        lo, hi = gptr[io], gptr[io + 1]
+        at = np.concatenate(list(a[lo:hi].astype(np.float64)), axis=1) if hi > lo else np.zeros((t, 0))
+        bt = b[tiles[lo:hi].reshape(-1)].astype(np.float64)
+        want, scale = at @ bt, np.abs(at) @ np.abs(bt)
+        if has[io]:
+            want[:, feat - 1], scale[:, feat - 1] = 0.0, 0.0
+        # fp32 sums of up to 688 exact products: 688 roundings of 2^-24 of the terms; one more of an fp16 result
+        bound = 688 * 2.0 ** -24 * scale + (2.0 ** -11 * np.abs(want) if out_dtype is torch.float16 else 0.0) + 1e-7
+        assert np.all(np.abs(got[io] - want) <= bound)

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -198,10 +199,12 @@ inline int long_row(int64_t m, int64_t nnz) {
 // 106 / 110 / 111).
 inline int long_piece(int64_t nnz) { return nnz < (1 << 18) ? 64 : nnz < (1 << 20) ? 128 : 256; }
 
-// Small products are one launch: rows above kBlockRow nonzeros are left until the workgroup has done
-// its other rows and takes them together, each wavefront a stretch of the row, the sums meeting in
-// LDS.  Left to one wavefront a row of 1024 nonzeros was 16 round trips to memory one after the other
-// and set the time of a 4096-row launch (70 k nonzeros, 32 features: 17 us, now 7 us).
+// Small products are one launch: rows above kBlockRow nonzeros are taken by all wavefronts of the
+// workgroup together, each a stretch of the row, the sums meeting in LDS.  Left to one wavefront a row
+// of 1024 nonzeros was 16 round trips to memory one after the other and set the time of a 4096-row
+// launch (70 k nonzeros, 32 features: 17 us, now 5.5 us).  us with 64 / 96 / 128 / 192 / 256 (csr_small_kernel):
+//   4096 rows, 65 k nonzeros, 32 features, rows of up to 1024 6.0 / 5.9 / 5.5 / 5.5 / 5.7, up to 128 5.3 / 4.9 / 4.0 / 4.3 /
+//   4.3; 3 k, 60 k, 48 6.9 / 7.2 / 7.3 / 7.5 / 8.8; 8 k, 170 k, 17 9.3 / 9.2 / 9.0 / 9.1 / 9.6.
 // The line lies at nnz * feat because what a compute unit can read sets how long a hub row takes it:
 // 80 k nonzeros with a row of 2000 cost the same either way at 64 features (13.3 us, split 13.9), at
 // 16 features 10.2 us (12.4), at 100 features 21.5 us (19.5).
@@ -256,58 +259,163 @@ __device__ __forceinline__ void block_rows(const BlockRow* list, int count, floa
   }
 }
 
-// One wavefront per row, WAVES rows per workgroup.  With WAVES = 4 the matrix is split: rows above
-// kLongRow are zero-filled here and added by csr_long_rows_kernel.
-template <int G, int REP, int WAVES, bool INDIRECT = false>
-__global__ __launch_bounds__(WAVES * kWave) void csr_spmm_kernel(int m, int feat, int long_row, const float* __restrict__ A,
+// One wavefront per row, four rows per workgroup: rows above long_row are zero-filled here and added by
+// csr_long_rows_kernel.
+template <int G, int REP, bool INDIRECT = false>
+__global__ __launch_bounds__(4 * kWave) void csr_spmm_kernel(int m, int feat, int long_row, const float* __restrict__ A,
                                                                  const float* __restrict__ B,
                                                                  float* __restrict__ C,
                                                                  const int32_t* __restrict__ indptr,
                                                                  const int32_t* __restrict__ indices) {
-  constexpr bool SPLIT = WAVES == 4;
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int row = blockIdx.x * WAVES + wave;
-  const int g = lane / G;
-  int start = 0, end = 0;
-  if (row < m) start = indptr[row], end = indptr[row + 1];
-  if constexpr (SPLIT) {
-    if (row >= m) return;
-  }
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= m) return;
+  const int start = indptr[row], end = indptr[row + 1];
   float4 acc[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const bool later = end - start > (SPLIT ? long_row : kBlockRow);
+  const bool later = end - start > long_row;
   if (!later) csr_accumulate<G, REP, INDIRECT>(acc, start, end, feat, A, B, indices, lane);
   reduce_groups<G, REP>(acc, kWave);
   if constexpr (INDIRECT) {
     // merged rows of a hyb plan: the operator adds to C, as its buckets do; this wavefront is the
     // row's only writer in this launch, long rows are left to csr_long_rows_kernel altogether
     if (later) return;
-    if (g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 2, nullptr);
-  } else if constexpr (SPLIT) {
-    if (g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 0, nullptr);
+    if (lane < G) write_row<G, REP>(C, row, feat, feat, lane, acc, 2, nullptr);
   } else {
-    __shared__ BlockRow list[WAVES];
-    __shared__ __attribute__((aligned(16))) float part[WAVES * 4 * G * REP];
-    if (row < m && !later && g == 0) write_row<G, REP>(C, row, feat, feat, lane, acc, 0, nullptr);
-    if (!__syncthreads_or(later)) return;
-    if (lane == 0) list[wave] = BlockRow{row, start, end};
-    __syncthreads();
-    for (int w = 0; w < WAVES; ++w)
-      if (list[w].end - list[w].start > kBlockRow)  // uniform
-        block_rows<G, REP, WAVES>(list + w, 1, part, feat, A, B, C, indices, lane, wave);
+    if (lane < G) write_row<G, REP>(C, row, feat, feat, lane, acc, 0, nullptr);
+  }
+}
+
+// Small products of few rows, one wavefront per row, kSmallWaves rows per workgroup.  Such a launch ends with the
+// workgroup that has a hub row, on a chain of round trips to memory: row pointers, columns and values, rows of B.
+// So that it has as few as possible,
+//   - every wavefront reads the row pointers of the whole workgroup and so knows its share of the long rows from the
+//     start, without an exchange;
+//   - its own row and its shares of the long ones are one sequence of up to 64 nonzeros at a time, the columns and
+//     values of the next 64 requested before the rows of B of these;
+//   - the shares' sums meet in LDS, as many rows at a time as 8 KB hold (wider ones: one).
+// 4096 rows, 65 k nonzeros, 32 features, rows of up to 1024: 5.5 us, of up to 128 4.0, all alike 3.2, an empty launch
+// 2.2.  With the long rows after the others, found by way of LDS and one load of columns before each set of rows of B:
+// 6.6, 5.1, 3.4.
+template <int G, int REP>
+__global__ __launch_bounds__(kSmallWaves * kWave) void csr_small_kernel(int m, int feat, const float* __restrict__ A,
+                                                                        const float* __restrict__ B,
+                                                                        float* __restrict__ C,
+                                                                        const int32_t* __restrict__ indptr,
+                                                                        const int32_t* __restrict__ indices) {
+  constexpr int NG = kWave / G;
+  constexpr int kWide = G == 4 ? 4 : 8 / REP;  // rows of B in flight per lane; NG * kWide divides 64
+  constexpr int kRound = G * REP >= 64 ? 1 : 64 / (G * REP) < kSmallWaves ? 64 / (G * REP) : kSmallWaves;
+  __shared__ float4 part[kRound * kSmallWaves * G * REP];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane / G, gl = lane % G;
+  const int64_t row0 = (int64_t)blockIdx.x * kSmallWaves;
+  const int ptr = indptr[min(row0 + min(lane, kSmallWaves), (int64_t)m)];
+  const int len = __shfl_down(ptr, 1, kWave) - ptr;
+  uint32_t shared = (uint32_t)__ballot(lane < kSmallWaves && len > kBlockRow);
+  // the nonzeros [s, e) that are being added up: the wavefront's own row, then its shares
+  int s = __builtin_amdgcn_readlane(ptr, wave), e = __builtin_amdgcn_readlane(ptr, wave + 1);
+  const bool left = shared >> wave & 1;
+  if (left) e = s;
+  bool own = true;
+  float4 acc[REP];
+#pragma unroll
+  for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+  int col = s + lane < e ? __builtin_nontemporal_load(indices + s + lane) : 0;
+  float val = s + lane < e ? __builtin_nontemporal_load(A + s + lane) : 0.f;
+  int held = 0;        // rows whose shares are in LDS,
+  uint32_t round = 0;  // and which rows of the workgroup these are
+  for (;;) {
+    // what comes next
+    const int cnt = min(kWave, e - s);
+    const bool done = s + kWave >= e;
+    const bool more = !done || shared;
+    int ns = s + kWave, ne = e;
+    uint32_t next_row = 0;
+    if (done && shared) {
+      const int nw = __builtin_ctz(shared);
+      next_row = 1u << nw;
+      const int rs = __builtin_amdgcn_readlane(ptr, nw), re = __builtin_amdgcn_readlane(ptr, nw + 1);
+      const int per = ((re - rs + kSmallWaves - 1) / kSmallWaves + 3) & ~3;
+      ns = min(re, rs + wave * per), ne = min(re, ns + per);
+      shared &= shared - 1;
+    }
+    int ncol = 0;
+    float nval = 0.f;
+    if (more && ns + lane < ne) {
+      ncol = __builtin_nontemporal_load(indices + ns + lane);
+      nval = __builtin_nontemporal_load(A + ns + lane);
+    }
+    const auto step = [&](int j0, auto in_flight) {
+      constexpr int U = decltype(in_flight)::value;
+      float4 x[U][REP];
+      float v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + u * NG + g;
+        const int c = __shfl(col, j, kWave);
+        v[u] = __shfl(val, j, kWave);
+        const float* bp = B + (int64_t)c * feat;
+#pragma unroll
+        for (int r = 0; r < REP; ++r) {
+          const int c0 = gl * 4 + r * G * 4;
+          x[u][r] = j < cnt && c0 < feat ? ld4(bp + chunk_offset(c0, feat)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int r = 0; r < REP; ++r) fma4(acc[r], v[u], x[u][r]);
+    };
+    int j0 = 0;
+    for (; j0 + NG * (kWide / 2) < cnt; j0 += NG * kWide) step(j0, std::integral_constant<int, kWide>());
+    if (j0 < cnt) step(j0, std::integral_constant<int, kWide / 2>());
+    if (done) {
+      reduce_groups<G, REP>(acc, kWave);
+      if (own) {
+        if (g == 0 && row0 + wave < m && !left) write_row<G, REP>(C, row0 + wave, feat, feat, lane, acc, 0, nullptr);
+        own = false;
+      } else {
+        if (g == 0)
+#pragma unroll
+          for (int r = 0; r < REP; ++r) part[((held * kSmallWaves + wave) * REP + r) * G + gl] = acc[r];
+        if (++held == kRound || !more) {
+          __syncthreads();
+          if (wave < held) {
+            for (int k = 0; k < wave; ++k) round &= round - 1;
+#pragma unroll
+            for (int r = 0; r < REP; ++r) {
+              acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+              for (int k = g; k < kSmallWaves; k += NG) {
+                const float4 o = part[((wave * kSmallWaves + k) * REP + r) * G + gl];
+                acc[r].x += o.x, acc[r].y += o.y, acc[r].z += o.z, acc[r].w += o.w;
+              }
+            }
+            reduce_groups<G, REP>(acc, kWave);
+            if (g == 0) write_row<G, REP>(C, row0 + __builtin_ctz(round), feat, feat, lane, acc, 0, nullptr);
+          }
+          if (more) __syncthreads();
+          held = 0, round = 0;
+        }
+      }
+      if (!more) break;
+#pragma unroll
+      for (int r = 0; r < REP; ++r) acc[r] = make_float4(0.f, 0.f, 0.f, 0.f);
+      round |= next_row;
+    }
+    s = ns, e = ne, col = ncol, val = nval;
   }
 }
 
 // Feature rows narrower than a wavefront (G < 64 lanes): a wavefront owns 64 / G consecutive rows
 // of the matrix, one per lane group.  A group walks its own row -- G nonzeros per index load, up
 // to eight gathers in flight per lane -- and stores it without any exchange between lanes; the
-// wavefront writes 64 / G consecutive rows of C.  With one wavefront per row (the kernel above) a
+// wavefront writes 64 / G consecutive rows of C.  With one wavefront per row (csr_spmm_kernel) a
 // row of seven nonzeros at 32 features keeps one lane group in eight busy for one step and still
 // pays the index round trip, the cross-lane sum and the store.  Rows of more than 2 * G nonzeros
 // would hold the other groups up: the wavefront takes those one by one afterwards, all groups
-// sharing the row as in the kernel above, up to the length that is left to csr_long_rows_kernel
+// sharing the row as in csr_spmm_kernel, up to the length that is left to csr_long_rows_kernel
 // (WAVES = 4, the matrix is split: zero-filled here) or to the workgroup.
 template <int G, int WAVES>
 __global__ __launch_bounds__(WAVES * kWave) void csr_spmm_rows_kernel(int m, int feat, int long_row,
@@ -967,7 +1075,7 @@ int launch_merged(const MergedRows& mr, int32_t m, int32_t n, int32_t feat, cons
   const float* vals = reinterpret_cast<const float*>(mr.vals);
 #define STIR_MERGED(G, REP)                                                                                   \
   {                                                                                                           \
-    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4, true>), grid, block, 0, st, m, feat, kLongRow, vals, d_B, d_C,       \
+    hipLaunchKernelGGL((csr_spmm_kernel<G, REP, true>), grid, block, 0, st, m, feat, kLongRow, vals, d_B, d_C,       \
                        mr.slot_ptr, mr.cols);                                                                 \
     hipLaunchKernelGGL((csr_long_rows_kernel<G, REP, true>), pieces, block, 0, st, m, feat, mr.slots, piece, kLongRow,   \
                        vals, d_B, d_C, mr.slot_ptr, mr.cols);                                                 \
@@ -1118,12 +1226,11 @@ int stir_csr_spmm_f32(int32_t m, int32_t n, int32_t feat, int64_t nnz, const flo
 #define STIR_CSR(G, REP)                                                                                   \
   {                                                                                                        \
     if (split) {                                                                                           \
-      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, 4>), grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, d_indptr, \
+      hipLaunchKernelGGL((csr_spmm_kernel<G, REP>), grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, d_indptr, \
                          d_indices);                                                                       \
       STIR_CSR_LONG(G, REP);                                                                               \
     } else {                                                                                               \
-      hipLaunchKernelGGL((csr_spmm_kernel<G, REP, kSmallWaves>), grid, block, 0, st, m, feat, longest, d_A, d_B, d_C, \
-                         d_indptr, d_indices);                                                             \
+      hipLaunchKernelGGL((csr_small_kernel<G, REP>), grid, block, 0, st, m, feat, d_A, d_B, d_C, d_indptr, d_indices); \
     }                                                                                                      \
   }
   // lane groups narrower than the wavefront: a lane group per row (csr_spmm_rows_kernel)

@@ -1,14 +1,13 @@
 // BSR SpMM on the gfx950 matrix cores: Y[i-th block row] = sum over stored blocks p of
 // A_p (blk x blk) * X[indices[p]-th block of rows], 16-bit inputs, fp32 accumulation.
 //
-// Slices of 32 rows: a wavefront owns 32 rows x 128 or 256 features, loads the rows of X into registers eight features to
+// Slices of 32 rows, 16 where the block is an odd multiple of that: a wavefront owns them x 128 or 256 features, loads the rows of X into registers eight features to
 // a lane and makes the MFMA B operand (8 consecutive k of one feature per lane) out of them with v_perm: no LDS and no
-// other wavefront is in the way (bsr_direct_kernel, bsr_wave_kernel).  In small launches the wavefronts of a workgroup
-// take the steps of one tile in turn.
+// other wavefront is in the way (bsr_direct_kernel, bsr_wave_kernel, bsr16_direct_kernel, bsr16_wave_kernel).  In small
+// launches the wavefronts of a workgroup take the steps of one tile in turn.
 // Slices of 64 rows (blocks that are a multiple of 64, where there are many): a workgroup of four wavefronts owns 64 rows
-// and a 128*NT-wide slice of the feature axis; both operands go through LDS (bsr_tile).  Odd multiples of 16 rows by
-// bsr16_wave_kernel, or by bsr16_spmm_kernel where those are few, or, as the smallest launches of long block rows
-// whatever the block, by bsr_split_kernel.
+// and a 128*NT-wide slice of the feature axis; both operands go through LDS (bsr_tile).  The smallest launches of
+// long block rows, whatever the block, by bsr_split_kernel.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -406,257 +405,6 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                   0, 0);
 }
 
-// A chunk of 16 columns: number `number` of a block row's chunks, columns 16 * col of block `block`
-struct Chunk {
-  int number, block, col;
-  __device__ __forceinline__ void advance(int by, int sub) {
-    number += by, col += by;
-    while (col >= sub) col -= sub, ++block;
-  }
-};
-
-// Few slices: a workgroup of four wavefronts owns (block row, 16-row slice, 128 * NT features), a wavefront 16 rows x
-// 32 * NT features.  Per step the 32 rows of X of two chunks go through LDS as in bsr_tile (two stages, one
-// barrier per step, the next step's loads in flight), the image's XOR extended by 2 * (k / 8 % 2): the two
-// blocks of 16 lanes that a transposing read serves together ask for the same units of k groups eight rows
-// apart here.  The A operand is one 16-byte load per lane from the block.
-// 60 x 200 blocks of 48, 10 %, 1024 features: 31 us.
-template <bool BF16, int OUT, int NT>
-__global__ __launch_bounds__(256) void bsr16_spmm_kernel(int blk, int feat, int64_t slices, int f_tiles,
-                                                         const uint16_t* __restrict__ A,
-                                                         const uint16_t* __restrict__ X, void* __restrict__ Y,
-                                                         const int32_t* __restrict__ indptr,
-                                                         const int32_t* __restrict__ indices,
-                                                         const int32_t* __restrict__ row_ids) {
-  constexpr int TF = kTileF * NT;
-  constexpr int FCN = TF / 8;          // 16-byte units per row of X
-  constexpr int XB = kTileK * TF * 2;  // bytes per stage
-  __shared__ __attribute__((aligned(16))) char xs[2 * XB];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int64_t slice;
-  int f_tile;
-  if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) return;
-  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
-  const int i = (int)(slice / sub), s = (int)(slice % sub);
-  const int i_out = row_ids ? row_ids[i] : i;
-  const int f0 = f_tile * TF;
-  // staging role: 2 * NT units of the wavefront's chunk (wavefronts 0, 1: the step's first; 2, 3: its second)
-  uint32_t xoff[2 * NT], xdst[2 * NT];
-#pragma unroll
-  for (int u = 0; u < 2 * NT; ++u) {
-    const int idx = 64 * (wave * 2 * NT + u) + lane, c = idx % FCN, k = idx / FCN;
-    xoff[u] = (uint32_t)((k & 15) * feat + 8 * c);
-    xdst[u] = (uint32_t)(((k >> 2) * 4 * FCN + (k & 3) * FCN + (c ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)))) * 16);
-  }
-  static_assert(64 % FCN == 0, "a lane's units share their feature column");
-  const bool xlive = f0 + 8 * (lane % FCN) < feat;
-  // operand role: row ii of the slice, k group q (8 of the step's 32 k)
-  const int ii = lane & 15, q = lane >> 4;
-  const uint32_t aoff = (uint32_t)((s * 16 + ii) * blk + 8 * (q & 1));
-  uint32_t bread[2 * NT];
-#pragma unroll
-  for (int t = 0; t < 2 * NT; ++t) {
-    const int kr = ii >> 2, c = wave * NT * 4 + 2 * t + ((ii & 3) >> 1);
-    bread[t] = (uint32_t)(((2 * q) * 4 * FCN + kr * FCN + (c ^ (4 * kr) ^ (2 * (q & 1)))) * 16 + (ii & 1) * 8);
-  }
-
-  const int p_begin = indptr[i];
-  const int chunks = (indptr[i + 1] - p_begin) * sub;
-  const int steps = (chunks + 1) / 2;
-
-  f32x4 acc[2 * NT];
-#pragma unroll
-  for (int t = 0; t < 2 * NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  // the chunks of the step to fetch next: of the wavefront's rows of X, and of the lane's piece of A; the block
-  // column is requested one step before the rows of X
-  Chunk mx{0, 0, 0}, ma{0, 0, 0};
-  mx.advance(wave >> 1, sub);
-  ma.advance(q >> 1, sub);
-  int j = mx.number < chunks ? indices[p_begin + mx.block] : 0;
-  u32x4 xr[2 * NT], a_next;
-  auto fetch = [&]() {
-    a_next = u32x4{0, 0, 0, 0};
-    if (ma.number < chunks)
-      a_next = *reinterpret_cast<const u32x4*>(A + (int64_t)(p_begin + ma.block) * blk * blk + aoff + 16 * ma.col);
-    const bool live = xlive && mx.number < chunks;
-    const uint16_t* xb = X + ((int64_t)j * blk + 16 * mx.col) * feat + f0;
-#pragma unroll
-    for (int u = 0; u < 2 * NT; ++u) {
-      xr[u] = u32x4{0, 0, 0, 0};
-      if (live) xr[u] = *reinterpret_cast<const u32x4*>(xb + xoff[u]);
-    }
-    ma.advance(2, sub);
-    mx.advance(2, sub);
-    if (mx.number < chunks) j = indices[p_begin + mx.block];
-  };
-
-  if (steps > 0) fetch();
-  for (int it = 0; it < steps; ++it) {
-    char* stage = xs + (it & 1) * XB;
-    const u32x4 a = a_next;
-#pragma unroll
-    for (int u = 0; u < 2 * NT; ++u) *reinterpret_cast<u32x4*>(stage + xdst[u]) = xr[u];
-    if (it + 1 < steps) fetch();
-    __syncthreads();
-#pragma unroll
-    for (int t = 0; t < 2 * NT; ++t) acc[t] = mfma16<BF16>(a, read_b(stage + bread[t], FCN * 64), acc[t]);
-  }
-#pragma unroll
-  for (int t = 0; t < 2 * NT; ++t) {
-    const int fcol = f0 + wave * 32 * NT + 16 * t;
-    if (fcol >= feat) continue;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int64_t off = ((int64_t)i_out * blk + s * 16 + 4 * q + v) * feat + fcol + ii;
-      if constexpr (OUT == 1)
-        static_cast<float*>(Y)[off] = acc[t][v];
-      else
-        static_cast<uint16_t*>(Y)[off] = to16<BF16>(acc[t][v]);
-    }
-  }
-}
-
-// A wavefront owns a 16-row slice and TF features (TF / 16 accumulators) and takes two chunks of 16 columns of the block
-// row per step: their 32 rows of X go through LDS of its own (image as in bsr_tile, the XOR extended by 2 * (k / 8 %
-// 2): the two blocks of 16 lanes that a transposing read serves together ask for the same units of k groups eight rows
-// apart here), the next step's loads in flight; no wavefront waits for another.  The A operand is one 16-byte load per
-// lane.  Bound by the rows of X that come out of L2: a slice uses each of them for 16 rows only.  Against four
-// wavefronts that shared 256 features and met at a barrier per step: 318 x 284 blocks of 16, 20 %, 3328 features 108
-// -> 95 us; 732 x 74, 14 %, 320 features 15.3 -> 10.6; 1024 x 1024, 10 %, 4096 features 1081 -> 614 with 256 features
-// in ranked order (722 with 128; 975 with 256 in plain order).
-template <bool BF16, int OUT, int TF, bool ONE>  // ONE: blk == 16, a chunk is a block
-__global__ __launch_bounds__(kWave, TF == 256 ? 2 : 4) void bsr16_wave_kernel(int blk, int feat, int64_t slices,
-                                                                              int f_tiles, int ranked,
-                                                                              const uint16_t* __restrict__ A,
-                                                                              const uint16_t* __restrict__ X,
-                                                                              void* __restrict__ Y,
-                                                                              const int32_t* __restrict__ indptr,
-                                                                              const int32_t* __restrict__ indices,
-                                                                              const int32_t* __restrict__ row_ids) {
-  constexpr int FT = TF / 16;   // accumulators
-  constexpr int FCN = TF / 8;   // 16-byte units per row of X
-  constexpr int KQ = 64 / FCN;  // rows of X per load
-  constexpr int XQ = 16 / KQ;   // loads per chunk
-  __shared__ __attribute__((aligned(16))) char stage[kTileK * TF * 2];
-  if (ONE) blk = 16;
-  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
-  int64_t slice;
-  int f_tile;
-  if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
-             : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
-    return;
-  const int lane = threadIdx.x, ii = lane & 15, g = lane >> 4;
-  // the same for all lanes, which the divisions hide from the compiler
-  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
-  int i = (int)slice / sub;
-  const int bi0 = (int)slice % sub * 16;
-  if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
-  const int i_out = row_ids ? row_ids[i] : i;
-  const int f0 = f_tile * TF;
-  // staging: unit c of the rows KQ * q + kq of a chunk.  Units beyond feat repeat the last one: features nobody stores.
-  const int c = lane % FCN, kq = lane / FCN;
-  const uint32_t xoff = (uint32_t)(kq * feat + min(8 * c, feat - f0 - 8)) * 2;
-  auto place = [&](int k) {
-    return (uint32_t)(((k >> 2) * 4 * FCN + (k & 3) * FCN + (c ^ (4 * (k & 3)) ^ (2 * ((k >> 3) & 1)))) * 16);
-  };
-  // operands: row ii of the slice, k group g (8 of the step's 32); tile t of X is where its bits 5 ... say
-  const uint32_t aoff = (uint32_t)((bi0 + ii) * blk + 8 * (g & 1)) * 2;
-  const int kr = ii >> 2;
-  const uint32_t bread = (uint32_t)(((2 * g) * 4 * FCN + kr * FCN + (((ii & 3) >> 1) ^ (4 * kr) ^ (2 * (g & 1)))) * 16 +
-                                    (ii & 1) * 8);
-
-  f32x4 acc[FT];
-#pragma unroll
-  for (int t = 0; t < FT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
-  const int chunks = nblk * sub;
-  // Block columns of the 64 blocks from `base` on and of the next 64.  Two chunks that are fetched together never lie on
-  // both sides: 64 blocks are an even number of chunks.
-  int base = 0;
-  int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
-  int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
-  int block = 0, col = 0;  // the next chunk to fetch
-  u32x4 xr[2][XQ], ar;
-  auto fetch = [&]() {
-    const int first = block;
-    uint32_t a_at[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const bool live = block < nblk;
-      const int of = block & (kWave - 1);
-      const int j = __builtin_amdgcn_readlane(j_lane, of);
-      const auto rx = window(X + ((int64_t)j * blk + 16 * col) * feat + f0, live ? 32u * feat : 0);
-#pragma unroll
-      for (int q = 0; q < XQ; ++q)
-        xr[b][q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff, q * KQ * 2 * feat, 0);
-      a_at[b] = live ? (uint32_t)((block - first) * blk * blk + 16 * col) * 2 + aoff : ~15u;
-      if (ONE || ++col == sub) col = 0, ++block;
-    }
-    const auto ra = window(A + (int64_t)(p_begin + first) * blk * blk, ONE ? 512u * max(min(nblk - first, 2), 0) : 4u * blk * blk);
-    ar = __builtin_amdgcn_raw_buffer_load_b128(ra, ONE ? aoff + 512 * (g >> 1) : g < 2 ? a_at[0] : a_at[1], 0, 0);
-    if (block >= base + kWave) {
-      base += kWave;
-      j_lane = j_more;
-      j_more = base + kWave + lane < nblk ? indices[p_begin + base + kWave + lane] : 0;
-    }
-  };
-  auto step = [&](bool more) {
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int q = 0; q < XQ; ++q) *reinterpret_cast<u32x4*>(stage + place(16 * b + KQ * q + kq)) = xr[b][q];
-    const u32x4 a = ar;
-    if (more) fetch();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int t = 0; t < FT; ++t) acc[t] = mfma16<BF16>(a, read_b(stage + (bread ^ (32 * t)), FCN * 64), acc[t]);
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();  // the next step's stores come after these reads
-  };
-  fetch();
-#pragma unroll 1
-  for (int it = 0; it < chunks / 2; ++it) step(true);
-  // The second chunk of an odd last step is multiplied by zeros of A and has to be zeros whatever X holds: said here, not
-  // left to an empty window whose loads carry a scalar offset.  (Lane offsets beyond any window cost 1 to 2 %, this
-  // nothing: 1024 x 1024 blocks of 16, 4096 features 607 -> 605 us.)
-  if (chunks & 1) {
-#pragma unroll
-    for (int q = 0; q < XQ; ++q) xr[1][q] = u32x4{0, 0, 0, 0};
-    step(false);
-  }
-  // acc[t][v] is row 4 g + v, column 16 t + ii; 16-bit results through LDS into 16-byte stores (see store_rows)
-  const int64_t row0 = (int64_t)i_out * blk + bi0;
-  if constexpr (OUT == 1) {
-#pragma unroll
-    for (int t = 0; t < FT; ++t) {
-      if (f0 + 16 * t >= feat) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        static_cast<float*>(Y)[(row0 + 4 * g + v) * feat + f0 + 16 * t + ii] = acc[t][v];
-    }
-  } else {
-#pragma unroll
-    for (int t = 0; t < FT; ++t)
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        *reinterpret_cast<uint16_t*>(stage + ((4 * g + v) * TF + 16 * t + ii) * 2) = to16<BF16>(acc[t][v]);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int q = 0; q < 16 * FCN / kWave; ++q) {
-      const int at = kWave * q + lane, row = at / FCN, u = at % FCN;
-      const u32x4 w = *reinterpret_cast<const u32x4*>(stage + at * 16);
-      if (f0 + 8 * u < feat)
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row0 + row) * feat + f0 +
-                                                                8 * u));
-    }
-  }
-}
-
 // ------------------------------------------------------------------ 32-row slices, X in registers
 // Lane (c, g) of a wavefront loads 8 features from each of 8 consecutive rows of X, 16 bytes a row, and makes eight MFMA
 // operands of them (lane_operand.h): the loads are whole 256- or 512-byte pieces of a row, and eight neighbouring features of a
@@ -822,6 +570,280 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void
   }
 }
 
+// ---- 16-row slices
+// A step is two chunks of 16 columns, and of the k slots 8 g ... of lane group g four are rows of the first and four of the
+// second, in A and X alike: so a load of X is of one chunk, whose place is the same for all lanes.  The groups have the rows 0, 8,
+// 4, 12 ... of a chunk: A comes 16 bytes a lane, columns 8 (g & 1) ... of chunk g / 2, and two swaps of half wavefronts put it
+// so.  Rows of X have their offsets in lanes' registers: what an empty window's loads with a scalar offset give is not zeros.
+__device__ __forceinline__ u32x4 two_chunks(u32x4 a) {
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    const u32x2 t = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane32_swap(a[w], a[w + 2], false, false));
+    a[w] = t[0], a[w + 2] = t[1];
+  }
+  return a;
+}
+__device__ __forceinline__ int first_row(int g) { return 8 * (g & 1) + 4 * (g >> 1); }
+
+// The sums of `used` of the W wavefronts at a tile, which have 4 / W (eight: the first four one) of a lane's four rows each; `at`
+// the place of the first.  part: those of this tile.
+template <bool BF16, int OUT, int W>
+__device__ __forceinline__ void add_up(const f32x4 (&acc)[8], f32x4 (&part)[W][8][kWave], int wave, int lane, int used,
+                                       void* __restrict__ Y, int64_t at, int feat, bool live) {
+  if (wave < used) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+        part[wave][2 * v + e][lane] = f32x4{acc[4 * e][v], acc[4 * e + 1][v], acc[4 * e + 2][v], acc[4 * e + 3][v]};
+  }
+  __syncthreads();
+  for (int v = wave; v < 4; v += W) {
+    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      if (w >= used) continue;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const f32x4 p = part[w][2 * v + e][lane];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
+      }
+    }
+    if (live) store_eight<BF16, OUT>(Y, at + (int64_t)v * feat, o);
+  }
+}
+
+// A tile of 16 rows x 128 features, eight accumulators of v_mfma_f32_16x16x32; W wavefronts take the steps in turn.  T such tiles
+// side by side to a workgroup, whose wavefronts find each other's A in L1.  Two steps of a wavefront are on their way.
+// Against X through LDS (wavefronts with 128 or 256 features, or four that met at a barrier per step), us: 398 x 310 blocks of
+// 16, 19 steps, 576 features 34 -> 20.5 (W = 4); 749 x 92, 8 steps, 160 features 15.4 -> 9.1 (T = 2); 342 x 83, 4 steps, 1728
+// features 18.5 -> 14.8 (W = 1); 154 tiles of 80 steps 16.8 -> 13.0 (W = 8).  LDS, which X passed twice, had been as busy as the
+// L1s.  Bound by the L1s and the trips to memory at small sizes, by X from beyond L2 at large ones.  A by two loads of 8 bytes a
+// lane, without the swaps: 3 % slower, blocks of 48 and 80 5 to 8 %.
+template <bool BF16, int OUT, int W, int T, bool ONE>
+__global__ __launch_bounds__(W * T * kWave, W == 1 ? 4 : 2) void bsr16_direct_kernel(
+    int blk, int feat, int64_t slices, int f_tiles, int ranked, const uint16_t* __restrict__ A,
+    const uint16_t* __restrict__ X, void* __restrict__ Y, const int32_t* __restrict__ indptr,
+    const int32_t* __restrict__ indices, const int32_t* __restrict__ row_ids) {
+  constexpr int D = 2;  // steps on their way
+  if (ONE) blk = 16;
+  const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) % W;
+  const int c = lane & 15, g = lane >> 4;
+  int64_t slice;
+  int f_tile;
+  if (W * T == 1 && ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
+                           : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
+    return;
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  int i = (int)slice / sub;
+  const int bi0 = (int)slice % sub * 16;
+  if (W * T == 1 && ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = (f_tile * T + __builtin_amdgcn_readfirstlane(tid >> 6) / W) * kTileF;  // feat and beyond: a tile without work
+  // features beyond feat repeat the last ones: nobody stores them
+  uint32_t xoff[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) xoff[q] = (uint32_t)((first_row(g) + q) * feat + min(8 * c, feat - f0 - 8)) * 2;
+  const uint32_t aoff = (uint32_t)((bi0 + c) * blk + 8 * (g & 1)) * 2;
+
+  f32x4 acc[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
+  const int chunks = nblk * sub, steps = T > 1 && f0 >= feat ? 0 : (chunks + 1) / 2, first = W == 1 ? 0 : wave;
+  if (first < steps) {
+    const int32_t* cols = indices + p_begin;
+    int left = (steps - first + W - 1) / W;
+    int block = 2 * first / sub, col = 2 * first % sub;  // of the step to fetch next
+    u32x4 x[D][8], a[D];
+    auto fetch = [&](int s) {
+      const auto ra = window(A + (int64_t)(p_begin + block) * blk * blk, (uint32_t)(min(nblk - block, 2) * blk * blk) * 2);
+      const int over = ONE || col + 1 == sub;  // the second chunk is the first of the next block
+      const int apart = over ? blk * blk - 16 * col : 16;
+      a[s] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + (16 * col + (g >> 1) * apart) * 2, 0, 0);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int at = block + (b && over), k0 = ONE || (b && over) ? 0 : 16 * (col + b);
+        const bool live = at < nblk;
+        const int j = cols[min(at, nblk - 1)];
+        const auto rx = window(X + ((int64_t)j * blk + k0) * feat + f0, live ? 32u * feat : 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[s][4 * b + q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[q], 0, 0);
+      }
+      block += 2 * W / sub, col += 2 * W % sub;
+      if (col >= sub) col -= sub, ++block;
+    };
+    auto multiply = [&](int s) {
+      const u32x4 rows = two_chunks(a[s]);
+#pragma unroll
+      for (int t = 0; t < 8; ++t) acc[t] = mfma16<BF16>(rows, operand_of(x[s], t / 2, t % 2), acc[t]);
+    };
+    fetch(0);
+    if (left > 1) fetch(1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (; left >= 2 * D; left -= D) {
+#pragma unroll
+      for (int s = 0; s < D; ++s) {
+        multiply(s);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(s);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    multiply(0);  // one to three are left
+    if (left > 2) fetch(0);
+    if (left > 1) multiply(1);
+    if (left > 2) multiply(0);
+  }
+
+  // acc[t][v] is row 4 g + v, feature 8 c + t
+  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
+  const bool live = f0 + 8 * c < feat;
+  if constexpr (W == 1) {
+    if (!live) return;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float o[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) o[t] = acc[t][v];
+      store_eight<BF16, OUT>(Y, (row0 + v) * feat + f0 + 8 * c, o);
+    }
+  } else {
+    __shared__ __attribute__((aligned(16))) f32x4 part[T][W][8][kWave];
+    add_up<BF16, OUT, W>(acc, part[(tid >> 6) / W], wave, lane, min(steps, W), Y, row0 * feat + f0 + 8 * c, feat, live);
+  }
+}
+
+// A tile of 16 rows x 256 features, sixteen accumulators, in two halves of 128 features: as soon as the last operand of a half is
+// made, the next step's half is asked for.  By a wavefront, or by four that take the steps in turn.  The columns come by scalar
+// loads, a step ahead: a vector load of them on a branch in the loop made every wait in it one for all loads (11 % slower).
+// 1024 x 300 blocks of 16, 12 steps, 1024 features 52 us with X through LDS, 43.7; 1024 x 1024, 51 steps 174 -> 161 ranked, where
+// X comes from beyond the L2s either way: 4096 features 656 -> 647.
+template <bool BF16, int OUT, int W, bool ONE>
+__global__ __launch_bounds__(W * kWave, 3) void bsr16_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
+                                                              const uint16_t* __restrict__ A,
+                                                              const uint16_t* __restrict__ X, void* __restrict__ Y,
+                                                              const int32_t* __restrict__ indptr,
+                                                              const int32_t* __restrict__ indices,
+                                                              const int32_t* __restrict__ row_ids) {
+  if (ONE) blk = 16;
+  const int sub = blk / 16;
+  int64_t slice;
+  int f_tile;
+  if (ranked ? !decode_ranked(blockIdx.x, slices, sub, f_tiles, slice, f_tile)
+             : !decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile))
+    return;
+  const int lane = threadIdx.x & 63, wave = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  // the same for all lanes, which the divisions hide from the compiler
+  slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
+  int i = (int)slice / sub;
+  const int bi0 = (int)slice % sub * 16;
+  if (ranked) i = __builtin_amdgcn_readfirstlane(row_of_rank(indptr, (int)(slices / sub), i));
+  const int i_out = row_ids ? row_ids[i] : i;
+  const int f0 = f_tile * kWaveF;
+  uint32_t xoff[2][4];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) xoff[m][q] = (uint32_t)((first_row(g) + q) * feat + min(128 * m + 8 * c, feat - f0 - 8)) * 2;
+  const uint32_t aoff = (uint32_t)((bi0 + c) * blk + 8 * (g & 1)) * 2;
+
+  f32x4 acc[2][8];
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int p_begin = indptr[i], nblk = indptr[i + 1] - p_begin;
+  const int steps = (nblk * sub + 1) / 2, mine = W == 1 ? steps : (steps - wave + W - 1) / W;
+  const int32_t* cols = indices + p_begin;
+  int block = 2 * wave / sub, col = 2 * wave % sub;  // of the step after the one that is being fetched
+  int at[2], j[2], k0[2], at_n[2], j_n[2], k0_n[2];  // the chunks of either
+  auto look = [&]() {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const bool over = ONE ? b != 0 : col + b == sub;
+      at_n[b] = block + over, k0_n[b] = ONE || over ? 0 : 16 * (col + b);
+      j_n[b] = cols[min(at_n[b], nblk - 1)];
+    }
+    block += 2 * W / sub, col += 2 * W % sub;
+    if (col >= sub) col -= sub, ++block;
+  };
+  auto next = [&]() {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) at[b] = at_n[b], j[b] = j_n[b], k0[b] = k0_n[b];
+    look();
+  };
+  u32x4 x[2][8];
+  u32x4 ar;
+  auto fetch_a = [&]() {
+    const uint32_t bytes = at[0] < nblk ? (at[0] + 1 < nblk ? 4 * blk * blk : 2 * blk * blk) : 0;
+    const auto ra = window(A + (int64_t)(p_begin + at[0]) * blk * blk, bytes);
+    ar = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + (g >> 1) * ((at[1] - at[0]) * blk * blk + k0[1] - k0[0]) * 2, k0[0] * 2, 0);
+  };
+  auto fetch_x = [&](int m) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const auto rx = window(X + ((int64_t)j[b] * blk + k0[b]) * feat + f0, at[b] < nblk ? 32u * feat : 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[m][4 * b + q] = __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[m][q], 0, 0);
+    }
+  };
+  if (mine > 0) {
+    look(), next(), fetch_a(), fetch_x(0), fetch_x(1);
+#pragma unroll 1
+    for (int it = 0; it < mine; ++it) {
+      const u32x4 a = two_chunks(ar);
+      next(), fetch_a();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        u32x4 b[2][2];
+        auto pick = [&](int w) { b[w % 2][0] = operand_of(x[m], w, 0), b[w % 2][1] = operand_of(x[m], w, 1); };
+        pick(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          if (w < 3) pick(w + 1); else fetch_x(m);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int e = 0; e < 2; ++e) acc[m][2 * w + e] = mfma16<BF16>(a, b[w % 2][e], acc[m][2 * w + e]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+  }
+  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
+  if constexpr (W == 1) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (f0 + 128 * m + 8 * c >= feat) return;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        float o[8];
+#pragma unroll
+        for (int t = 0; t < 8; ++t) o[t] = acc[m][t][v];
+        store_eight<BF16, OUT>(Y, (row0 + v) * feat + f0 + 128 * m + 8 * c, o);
+      }
+    }
+  } else {
+    __shared__ __attribute__((aligned(16))) f32x4 part[W][8][kWave];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (m) __syncthreads();
+      add_up<BF16, OUT, W>(acc[m], part, wave, lane, min(steps, W), Y, row0 * feat + f0 + 128 * m + 8 * c, feat,
+                           f0 + 128 * m + 8 * c < feat);
+    }
+  }
+}
+
+// ---- 32-row slices by a wavefront
 // A wavefront owns 32 rows x 256 features, eight accumulators of v_mfma_f32_32x32x16: a step of 32 k is two halves of eight
 // loads of X; as soon as the last operand of a half is made, the next step's half is asked for, so that 8 wavefronts per CU
 // have 128 KB on their way.  A comes in 16-byte pieces in memory order, a step ahead, and through 2 KB of LDS of the
@@ -937,7 +959,8 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
 // workgroup barrier in the loop: the LDS operations of one wavefront execute in order); the eight partial
 // results are added through LDS at the end.
 // The X tile is 32 rows of 8 units of 16 bytes; unit (k, c) sits at place c ^ 4 * (k / 2 % 2) of its row -- two
-// rows fill the 64 banks -- and, ROWS = 16, ^ 2 * (k / 8 % 2) (see bsr16_spmm_kernel).
+// rows fill the 64 banks -- and, ROWS = 16, ^ 2 * (k / 8 % 2): the two blocks of 16 lanes that
+// a transposing read serves together ask for the same units of k groups eight rows apart there.
 // Against four wavefronts that took the k halves of each step: 40 x 510 blocks of 32, 18 %, 288 features
 // 27.4 -> 15.9 us; 50 x 63 blocks of 128, 128 features 27.6 -> 17.2 us; 358 x 998 blocks of 16, 64 features
 // (which had no such form) 39 -> 11.8 us.
@@ -1092,7 +1115,8 @@ struct BsrForm {
   bool wide;     // tiles of 256 features, else of 128 (kSplit by bsr_split_kernel: of kSplitF)
   bool ranked;   // block rows in order of their length
   bool by_rows;  // block rows dealt to XCDs
-  int direct = 0;  // bsr_direct_kernel with so many wavefronts to a tile
+  int direct = 0;  // operands in registers, so many wavefronts to a tile (16-row slices: kWaves too may have several, and
+                   // kGroups with two of them has two tiles of 128 features to a workgroup)
 };
 
 inline int slice_rows(int blk, BsrForm::Kernel kernel) {  // blocks that are a multiple of 64 are no direct groups
@@ -1129,14 +1153,10 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long: 11 x 119 blocks of 128, 92 steps,
     // 2304 features 50, 57)
     if (tiles * 4 <= 13 * cus && !few && (blk % 64 != 0 || steps < 48)) return {BsrForm::kSplit, false, false, false, 2};
-  } else {
-    // The split form wins as long as its workgroups are resident at once (two per CU with 32-row slices; four with 16-row
-    // slices), and up to twice as many where block rows have enough steps to pay for the second turn.  Split against not, 256
-    // features: 16-row slices, 1000 workgroups of 4 steps 7.3 against 7.3 us, 2000 of 16 steps 16.9 against 16.2 us, of 24
-    // steps 20.2 against 21.3 us.
-    const int64_t at_once = (unit == 16 ? 4 : 2) * cus;
-    if (split <= at_once || (split <= 2 * at_once && steps >= (unit == 16 ? 24 : 32)))
-      return {BsrForm::kSplit, false, false, false};
+  } else if (unit == 32) {
+    // The split form wins as long as its workgroups are resident at once, two per CU, and up to twice as many where block rows
+    // have enough steps to pay for the second turn.
+    if (split <= 2 * cus || (split <= 4 * cus && steps >= 32)) return {BsrForm::kSplit, false, false, false};
   }
   constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kLastLevel = 256 << 20;
   const int64_t wide_tiles = stir::ceil_div(feat, kWaveF), waste = wide_tiles * kWaveF - feat;
@@ -1149,41 +1169,68 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
   //   columns, 16 steps 63 / 54;
   //   four wavefronts, blocks of 64: 1024 rows, 256 columns, 1024 features 12 steps 141 / 119, 24 208 / 209, 48 345 / 387;
   //   128 features a tile: 256 rows, 512 features 12 steps 24.5 / 22.3, 1024 rows, 24 steps 126 / 132, 48 224 / 246; lengths
-  //   that differ by a factor of ten, 500 rows, 152 columns, 512 features 33 steps 78 / 113;
-  //   16-row slices, 1025 columns (8.4 MB), 1024 features: 1024 rows 10 steps 56 / 56, 18 78 / 85, 40 138 / 156, 4096 rows 10
-  //   steps 197 / 227, 40 523 / 788.
+  //   that differ by a factor of ten, 500 rows, 152 columns, 512 features 33 steps 78 / 113.
   // Among those that come as they are, wavefronts of 128 features, whose X an L2 still holds, pass those of 256 then (10
-  // steps of the first and of the last 127 and 165 us).
+  // steps of the first 127 us).
   auto rank_pays = [&](int64_t x_bytes, int64_t tiles, int64_t count, int per_cu) {
     return x_tile_bytes(std::min(feat, kWaveF)) > kMuchX && count >= per_cu * cus &&
            (steps >= 28 || (steps >= 16 && tiles >= 2 && x_bytes > kBeyondL2));
   };
   if (unit == 16) {
-    // 256 features per wavefront with much X, unless the last tile would be mostly empty, wavefronts few (1024 x 1024
-    // blocks of 16, 1024 features 158 us, 171 with 128; 1006 x 599, 544 features 155, 140) or X as above.  Blocks of
-    // several slices, which read the same X, take 256 whatever X (1100 x 341 of 48, 10 steps, 1024 features 126 us, 136 with
-    // 128; 500 x 37 of 80, 20 steps, 1504 features 283, 334), but for short rows; and whatever the last tile if
-    // A, which every tile reads, is more than the last level holds (3000 x 68 of 80, 20 steps, 800 features 957, 1340).
+    // Offsets of a load in 32 bits: bsr16_direct_kernel and bsr16_wave_kernel allow for more than the others.
+    if (feat >= (1 << 27) || blk >= (1 << 15)) return {BsrForm::kSplit, false, false, false};
+    if (!wavefronts) return {BsrForm::kGroups, feat >= kWaveF, false, false, feat >= kWaveF ? 2 : 4};
+    // Below, "128" are tiles of 128 features by so many wavefronts, "two of 128" the two tiles of a workgroup by two wavefronts
+    // each, "256" tiles of 256 by one wavefront (or four); us.
     const bool several = blk > 16;
-    const int64_t waves = unit_slices * wide_tiles, narrow_tiles = stir::ceil_div(feat, kTileF);
-    const bool fits = waves >= 8 * cus &&
-                      (waste * 8 <= feat || (several && feat > kTileF && nnzb * blk * blk * 2 > kLastLevel));
-    const bool rank_wide = fits && rank_pays(x_tile_bytes(kWaveF), wide_tiles, waves, 8);
-    const bool wide = rank_wide || (fits && (several ? x_tile_bytes(kWaveF) > kMuchX || steps >= 16
-                                                     : x_tile_bytes(kWaveF) > kMuchX && x_tile_bytes(kWaveF) <= kBeyondL2));
-    const bool ranked =
-        rank_wide || (!fits && rank_pays(x_tile_bytes(kTileF), narrow_tiles, unit_slices * narrow_tiles, 10));
-    // A wavefront per slice once eight per CU have one: 60 x 200 blocks of 48, 1024 features (1440) 33.1 us against 31.0
-    // by the kernel below, 90 x 300 of 80, 512 features (1800) 48 against 44, 150 x 140 of 48 (3600) 39.3 against 43.4.
-    // Nor where blocks of several slices would take 128 features and either have less than a turn (600 x 650 of 48, 7 steps,
-    // 256 features, 3600 wavefronts 37, 28) or far more X than an L2 holds (1214 x 659 of 80, 10 steps, 416 features, 27 MB
-    // 178, 134; but 3693 x 559 of 48, 320 features, 13.7 MB 194, 238).
-    const bool narrow_loses =
-        several && !wide && !ranked && feat >= kWaveF && x_tile_bytes(kWaveF) > kMuchX &&
-        (unit_slices * narrow_tiles < 16 * cus || x_tile_bytes(kWaveF) > 5 * kBeyondL2);
-    if (unit_slices * narrow_tiles >= 8 * cus && !narrow_loses && wavefronts)
-      return {BsrForm::kWaves, wide, ranked, false};
-    return {BsrForm::kGroups, feat >= kWaveF, false, false};
+    const int64_t narrow_tiles = stir::ceil_div(feat, kTileF), waves = unit_slices * wide_tiles;
+    const int64_t x_bytes = x_tile_bytes(kWaveF), x_narrow = x_tile_bytes(kTileF);
+    const bool even = narrow_tiles % 2 == 0, fits = waves >= 8 * cus && waste * 8 <= feat;
+    // Long rows and hardly more tiles than CUs, eight wavefronts with 64 features through LDS / 128 by four / by eight: 29 x 148
+    // blocks of 80, 46 steps, 160 features 14.4 / 15.4 / 15.2, 100 x 592 of 16, 19 steps, 320 8.9 / 9.6 / -; and where 128 waste half
+    // of a load also up to eight of 64 to a CU: 64 features, 51 steps (402) 13.3 / 13.8 / 13.4, 192, 107 steps (1926) 58.8 / 65.0 / 62.9.
+    const bool half = feat % kTileF != 0 && feat % kTileF <= kSplitF;
+    if (tiles > cus && ((half && steps >= (feat <= kSplitF ? 32 : 64) && split <= 8 * cus) ||
+                        (steps >= 40 && split <= 2 * cus) || (steps >= 18 && tiles * 4 <= 5 * cus && split <= 2 * cus)))
+      return {BsrForm::kSplit, false, false, false};
+    // 128 by four / by eight: 80 steps, 96 features (154 tiles) 16.5 / 13.0, 33 steps (136) 8.5 / 7.6, 15 steps (220) 5.6 / 5.6; 60
+    // steps (399) 15.7 / 15.4, 22 steps (996) 14.8 / 16.0.
+    if (tiles <= cus && steps >= 20) return {BsrForm::kSplit, false, false, false, 8};
+    // Much X: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
+    // ranked / 256 ranked: blocks of 16, 1024 columns (8.4 MB), 51 steps, 1024 features 205 / 188 / 163, 24 steps 105 / 104 / 94,
+    // 4096 features 1204 / 780 / 650; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184; of 48, 65 steps,
+    // 3424 543 / 539 / 534.  Between 16 and 28 steps only with far more X than an L2 holds (575 columns, 16 steps, 2784 features
+    // 41 / 45 / 46) or with few tiles, where the order gives little: 490, 17 steps, 512 features 34 / 40 / 42; 330 of 48, 25 steps,
+    // 608 44 / 48 / 53.
+    const bool wide_ranked = fits && (even || waste * 16 <= feat);
+    if (x_bytes > kMuchX && feat > kTileF && steps >= 16) {
+      if (wide_ranked && (steps >= 28 || (wide_tiles >= 2 && x_bytes > kBeyondL2 && (wide_tiles <= 4 || x_bytes > 2 * kBeyondL2))))
+        return {BsrForm::kWaves, true, true, false, 1};
+      if (!wide_ranked && unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (steps >= 28 || x_narrow > kBeyondL2))
+        return {BsrForm::kWaves, false, true, false, 1};
+    }
+    // Blocks of several slices, which read the same X.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of 80, 10
+    // steps, 416 features 138 / 130, 600 x 650 of 48, 7 steps, 256 20.8 / 21.0.  Less of it, 256 by four / by one: 1100 x 341 of 48,
+    // 10 steps, 1024 features 147 / 169, 5 steps, 140 columns 26 / 22.  And A, which every tile reads, more than the last level
+    // holds, 128 by four / 256 by four / by one: 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.
+    if (several && feat >= kWaveF && x_bytes > 15000000) return {BsrForm::kGroups, true, false, false, 2};
+    if (several && feat > kTileF && ((fits && x_bytes > kMuchX) || nnzb * blk * blk * 2 > kLastLevel))
+      return {BsrForm::kWaves, true, false, false, steps >= 8 ? 4 : 1};
+    // X in an L2, 128 by one / by four / two of 128 / 256: 342 x 83 of 16, 4 steps, 1728 features 14.8 / 17.2 / 16.2 / 16.7; 420
+    // columns, 10 steps, 512 24.5 / 24.5 / - / 23.3; 300, 12 steps, 1024 47.8 / 47.2 / - / 43.7; 73, 8 steps, 3904 67 / 73 / 65 /
+    // 63; 65, 7 steps, 224 features (1254 tiles) 8.7 / 9.0 / 8.4 / 9.3; 92, 8 steps, 160 (1498) 11.1 / 11.5 / 9.1 / 9.9.
+    if (steps <= 4 && tiles >= 6 * cus && x_bytes <= 2500000) return {BsrForm::kWaves, false, false, false, 1};
+    if (fits && even && x_bytes <= 3500000) return {BsrForm::kWaves, true, false, false, 1};
+    if (feat > kTileF && x_bytes <= 2500000 && tiles * 4 >= (even ? 19 : 48) * cus && steps < 20)
+      return {BsrForm::kGroups, true, false, false, 2};
+    if (several && feat >= kWaveF && tiles < 16 * cus && x_bytes > kMuchX && steps < 12)
+      return {BsrForm::kGroups, true, false, false, 2};
+    // 128 by one / by four: 5 steps, 1696 features (1442 tiles) 9.4 / 9.8, 3 steps (1140) 9.1 / 7.6; 6 steps, 1024 columns (8000)
+    // 37.2 / 37.1; of 48, 11 steps, 320 features (33 k) 230 / 208, of 80, 8 steps, 800 (105 k) 468 / 473.
+    if ((steps <= 5 && tiles >= 5 * cus) || (steps <= 11 && tiles >= 40 * cus)) return {BsrForm::kWaves, false, false, false, 1};
+    // Many steps, by four / by eight: 202 columns of 80, 105 steps, 896 features (2135 tiles) 108.5 / 105.4, 68 steps, 96 features
+    // (842) 28.2 / 27.3; but 94 steps, 3776 (3450) 132 / 135.
+    return {tiles < 8 * cus ? BsrForm::kSplit : BsrForm::kWaves, false, false, false, steps >= 64 && tiles < 9 * cus ? 8 : 4};
   }
   const int rs = slice_rows(blk, BsrForm::kGroups) / 32;
   const int64_t slices = (int64_t)mb * (blk / (32 * rs));
@@ -1247,7 +1294,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   auto eights = [](int64_t n) { return 8 * stir::ceil_div(n, 8); };  // see decode_tile, decode_ranked
   const int64_t blocks = form.by_rows  ? eights(mb) * sub * f_tiles
                          : form.ranked ? eights((int64_t)mb * f_tiles) * sub
-                         : form.kernel == BsrForm::kGroups && form.direct ? eights(stir::ceil_div(slices * f_tiles, 4))
+                         : form.kernel == BsrForm::kGroups && form.direct == 1 ? eights(stir::ceil_div(slices * f_tiles, 4))
                                        : eights(slices * f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   const dim3 grid((unsigned)blocks);
@@ -1255,9 +1302,27 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
 #define STIR_BSR_GO(KERNEL, THREADS, ...)                                                                      \
   hipLaunchKernelGGL(KERNEL, grid, dim3(THREADS), 0, st, blk, feat, slices, f_tiles, ##__VA_ARGS__, A, X, d_Y, \
                      d_indptr, d_indices, d_row_ids)
+#define STIR_ARGS(...) __VA_ARGS__
+#define STIR_BSR_16(ARGS, WAVES)                                                                               \
+  do {                                                                                                         \
+    if (blk == 16) STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);          \
+    else STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, false>), (WAVES) * kWave, ranked);                   \
+  } while (0)
+#define STIR_BSR_16W(ARGS, WAVES)                                                                              \
+  do {                                                                                                         \
+    if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);            \
+    else STIR_BSR_GO((bsr16_wave_kernel<STIR_ARGS ARGS, false>), (WAVES) * kWave, ranked);                     \
+  } while (0)
 #define STIR_BSR(BF, OUT)                                                                                      \
   do {                                                                                                         \
-    if (form.direct) {                                                                                         \
+    if (form.direct && unit == 16) {                                                                           \
+      if (form.kernel == BsrForm::kGroups && form.direct == 2) STIR_BSR_16((BF, OUT, 2, 2), 4);                \
+      else if (form.wide && form.direct == 1) STIR_BSR_16W((BF, OUT, 1), 1);                                   \
+      else if (form.wide) STIR_BSR_16W((BF, OUT, 4), 4);                                                       \
+      else if (form.direct == 1) STIR_BSR_16((BF, OUT, 1, 1), 1);                                              \
+      else if (form.direct == 4) STIR_BSR_16((BF, OUT, 4, 1), 4);                                              \
+      else STIR_BSR_16((BF, OUT, 8, 1), 8);                                                                    \
+    } else if (form.direct) {                                                                                  \
       if (form.kernel == BsrForm::kGroups) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, true>), 4 * kWave);      \
       else if (form.direct == 1) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false>), kWave);                   \
       else if (form.direct == 8) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 8, false>), 8 * kWave);               \
@@ -1266,16 +1331,8 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     } else if (form.kernel == BsrForm::kSplit) {                                                               \
       if (unit == 16) STIR_BSR_GO((bsr_split_kernel<BF, OUT, 16>), kWave * kSplitWaves);                       \
       else STIR_BSR_GO((bsr_split_kernel<BF, OUT, 32>), kWave * kSplitWaves);                                  \
-    } else if (form.kernel == BsrForm::kWaves && unit == 16) {                                                 \
-      if (form.wide && blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kWaveF, true>), kWave, ranked);      \
-      else if (form.wide) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kWaveF, false>), kWave, ranked);             \
-      else if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, true>), kWave, ranked);              \
-      else STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, kTileF, false>), kWave, ranked);                            \
     } else if (form.kernel == BsrForm::kWaves) {                                                               \
       STIR_BSR_GO((bsr_wave_kernel<BF, OUT>), kWave, ranked);                                                  \
-    } else if (unit == 16) {                                                                                   \
-      if (form.wide) STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 2>), 256);                                        \
-      else STIR_BSR_GO((bsr16_spmm_kernel<BF, OUT, 1>), 256);                                                  \
     } else if (unit == 64) {                                                                                   \
       if (form.wide) STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 2, 2>), 256, by_rows, ranked);                      \
       else STIR_BSR_GO((bsr_spmm_kernel<BF, OUT, 1, 2>), 256, by_rows, ranked);                                \
@@ -1290,6 +1347,9 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     if (out_dtype == STIR_F32) STIR_BSR(false, 1); else STIR_BSR(false, 0);
   }
 #undef STIR_BSR
+#undef STIR_BSR_16W
+#undef STIR_BSR_16
+#undef STIR_ARGS
 #undef STIR_BSR_GO
   STIR_LAUNCH_CHECK();
   return 0;
@@ -1298,7 +1358,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
 extern "C" {
 
 // The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
-// in order of their length, 16 for block rows dealt to XCDs, 32 times the wavefronts that bsr_direct_kernel has at a tile;
+// in order of their length, 16 for block rows dealt to XCDs, 32 times the wavefronts at a tile of those that make their operands in registers (0: of bsr_wave_kernel, and of LDS forms);
 // -1 for what no product is.  For the tests, which say what they cover.
 int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
   if (cus <= 0 || mb <= 0 || nb < 0 || nnzb < 0 || blk <= 0 || blk % 16 != 0 || feat <= 0) return -1;

@@ -812,16 +812,17 @@ __global__ __launch_bounds__(64 * W, T == 32 ? 2 : T == 16 ? 3 : 4) void tcspmm_
   }
 
   // ---- the sums over the wavefronts: each adds 4 RH / W of the rows a lane has.  acc[r][t][v] is row 16 r + 4 g + v, feature
-  // 8 c + t.
-  __shared__ __attribute__((aligned(16))) f32x4 sums[W][4 * RH][2][64];
+  // 8 c + t.  Sixteen-bit results leave as they lie; floats are read four features to a lane in the order of the row, so that a
+  // store is of whole lines (halves of lines: 169 k rows, 8-row tiles, 128 features 68.5 us, now 66.5).
+  __shared__ __attribute__((aligned(16))) f32x4 sums[W][4 * RH][2][64];  // [e][lane ^ 8 e]: eight lanes in row order share no bank
   const int used = min(W, s_end - s_begin);
   if (wave < used) {
 #pragma unroll
     for (int at = 0; at < 4 * RH; ++at)
 #pragma unroll
       for (int e = 0; e < 2; ++e)
-        sums[wave][at][e][lane] = f32x4{acc[at >> 2][4 * e][at & 3], acc[at >> 2][4 * e + 1][at & 3],
-                                        acc[at >> 2][4 * e + 2][at & 3], acc[at >> 2][4 * e + 3][at & 3]};
+        sums[wave][at][e][lane ^ (8 * e)] = f32x4{acc[at >> 2][4 * e][at & 3], acc[at >> 2][4 * e + 1][at & 3],
+                                                  acc[at >> 2][4 * e + 2][at & 3], acc[at >> 2][4 * e + 3][at & 3]};
   }
   __syncthreads();
   const int64_t elems = (int64_t)T * feat;
@@ -829,35 +830,38 @@ __global__ __launch_bounds__(64 * W, T == 32 ? 2 : T == 16 ? 3 : 4) void tcspmm_
   const stir::CoherentPiece partial(scratch + (part ? (int64_t)pc.slot * elems : 0), part ? (uint32_t)(elems * 4) : 0u);
 #pragma unroll
   for (int q = 0; q < 4 * RH / W; ++q) {
-    const int at = wave * (4 * RH / W) + q, row = 16 * (at >> 2) + 4 * g + (at & 3);
-    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const int at = wave * (4 * RH / W) + q;
+    const bool floats = OUT == 1 || part;
+    f32x4 o[2];
+    int place[2];  // of o[i] in sums: lane ^ 8 e, with 64 e
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int piece = 64 * i + lane, e = floats ? piece & 1 : i;  // in row order: row piece / 32, features 4 (piece % 32) ...
+      place[i] = 64 * e + ((floats ? piece >> 1 : lane) ^ (8 * e));
+      o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
     for (int w = 0; w < W; ++w) {
       if (w >= used) continue;
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const f32x4 p = sums[w][at][e][lane];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
-      }
+      for (int i = 0; i < 2; ++i) o[i] += sums[w][at][0][place[i]];
     }
-    const bool there = f0 + 8 * c < feat && (T >= 16 || row < T);  // the same for the four lanes of a quad
-    if (OUT == 0 && !part) {
+    if (!floats) {
+      const int row = 16 * (at >> 2) + 4 * g + (at & 3);
       u32x4 w;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[2 * t]) |
-               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[2 * t + 1]) << 16;
-      if (there) *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
+        w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2)]) |
+               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2) + 1]) << 16;
+      if (f0 + 8 * c < feat && (T >= 16 || row < T))
+        *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
       continue;
     }
-    float d[2][4];
-    stir::deal_out(o, d);
-    if (!there) continue;
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int fcol = f0 + 32 * (c >> 2) + 16 * s + 4 * (c & 3);
-      const float4 v = make_float4(d[s][0], d[s][1], d[s][2], d[s][3]);
+    for (int i = 0; i < (T == 8 ? 1 : 2); ++i) {  // of 8 rows the other half is no rows
+      const int row = 16 * (at >> 2) + 8 * i + 4 * (lane >> 5) + (at & 3), fcol = f0 + 4 * (lane & 31);
+      if (fcol >= feat) continue;
+      const float4 v = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
       if (part) partial.store((uint32_t)(row * feat + fcol), v);
       else *reinterpret_cast<Float4*>(static_cast<float*>(C) + (io * T + row) * feat + fcol) = Float4{v.x, v.y, v.z, v.w};
     }
@@ -919,7 +923,9 @@ int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n
   // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
   // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
   // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
-  const bool wide = feat > 64;
+  // Not where 32 features would have a unit of 128 and B is small enough to come mostly out of the L2s: 160 features, 30 k rows
+  // (9.7 MB) 27.3 / 28.3, 18 k 16.2 / 17.1, 36 k (11.7 MB) 26.3 / 26.8; but 52 k 52.3 / 47.2, 60 k 59.6 / 52.3.
+  const bool wide = feat > 64 && (feat % 128 != 32 || (int64_t)mb * T * feat * 2 > 13000000);
   const int ntl = feat <= 32 ? 1 : wide ? 4 : 2;
   const int f_tiles = (int)stir::ceil_div(feat, 32 * ntl);
   const int64_t blocks = (mb + n_pieces) * f_tiles;

@@ -413,28 +413,80 @@ using stir::operand_of;
 
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// Eight neighbouring features of a row of Y, by all four lanes of a quad, which have 32.
-template <bool BF16, int OUT>
-__device__ __forceinline__ void store_eight(void* __restrict__ Y, int64_t at, const float (&v)[8]) {
+// Results of a wavefront whose lane (n, h), n of LANES, has eight neighbouring features, 8 n ..., of row 4 h of Y behind `row`: as
+// they are, 16 bytes a lane, if they have 16 bits.  Floats first go through 2 KB of LDS into row order, four features to a lane
+// and the rows one behind the other, so that a store is of whole lines: with halves of lines (an exchange within quads) 437 x 33
+// blocks of 32, 1 step, 2720 features took 48.7 us, now 33.4, 452 x 51, 3 steps, 3840 66.5, 49.6.
+// The place of piece e (features 4 e ...) of a lane is XORed by 8 e: eight lanes in row order share no bank.
+template <int LANES>
+__device__ __forceinline__ int piece_place(int h, int n, int e) { return (2 * h + e) * LANES + (n ^ (8 * e)); }
+
+template <bool BF16, int OUT, int LANES>
+__device__ __forceinline__ void store_rows8(void* __restrict__ Y, int64_t row, int feat, int f0, int lane, const float (&v)[8],
+                                            f32x4* stage) {
+  const int n = lane % LANES, h = lane / LANES;
   if constexpr (OUT == 1) {
-    float d[2][4];  // floats 16 s + 4 (lane % 4) ... of the 32 that begin 8 (lane % 4) before `at`
-    stir::deal_out(v, d);
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-      __builtin_nontemporal_store(f32x4u{d[s][0], d[s][1], d[s][2], d[s][3]},
-                                  reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + at + 16 * s - 4 * (threadIdx.x & 3)));
+    for (int e = 0; e < 2; ++e)
+      stage[piece_place<LANES>(h, n, e)] = f32x4{v[4 * e], v[4 * e + 1], v[4 * e + 2], v[4 * e + 3]};
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int at = kWave * i + lane, r = at / (2 * LANES), u = at % (2 * LANES);
+      const f32x4 d = stage[piece_place<LANES>(r, u >> 1, u & 1)];
+      if (f0 + 4 * u < feat)
+        __builtin_nontemporal_store(f32x4u{d[0], d[1], d[2], d[3]},
+                                    reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + (row + 4 * r) * feat + f0 + 4 * u));
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   } else {
     u32x4 w;
 #pragma unroll
     for (int t = 0; t < 4; ++t) w[t] = to16<BF16>(v[2 * t]) | (uint32_t)to16<BF16>(v[2 * t + 1]) << 16;
-    __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + at));
+    if (f0 + 8 * n < feat)
+      __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row + 4 * h) * feat + f0 + 8 * n));
+  }
+}
+
+// The same for what several wavefronts left in LDS, `used` of them: lane (c, g), c of 16, of wavefront w has its pieces e at
+// part[w * stride + 64 e + (lane ^ 8 e)].
+template <bool BF16, int OUT, int W>
+__device__ __forceinline__ void add_up8(const f32x4* part, int stride, int used, void* __restrict__ Y, int64_t row, int feat, int f0,
+                                        int lane) {
+  f32x4 o[2];
+  int place[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int at = kWave * i + lane, e = OUT == 1 ? at & 1 : i;
+    place[i] = 64 * e + ((OUT == 1 ? at >> 1 : lane) ^ (8 * e));
+    o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    if (w >= used) continue;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) o[i] += part[w * stride + place[i]];
+  }
+  if constexpr (OUT == 1) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = 2 * i + (lane >> 5), u = lane & 31;
+      if (f0 + 4 * u < feat)
+        __builtin_nontemporal_store(f32x4u{o[i][0], o[i][1], o[i][2], o[i][3]},
+                                    reinterpret_cast<f32x4u*>(static_cast<float*>(Y) + (row + 4 * r) * feat + f0 + 4 * u));
+    }
+  } else {
+    const float v[8] = {o[0][0], o[0][1], o[0][2], o[0][3], o[1][0], o[1][1], o[1][2], o[1][3]};
+    store_rows8<BF16, OUT, 16>(Y, row, feat, f0, lane, v, nullptr);
   }
 }
 
 // A tile of 32 rows x 128 features, 16 accumulators of v_mfma_f32_16x16x32, a step of 32 k in eight loads of X and two of A.
 // W wavefronts take the steps of a block row in turn and meet in LDS at the end (W = 1: none does).  GROUP: W = 1, and a
 // workgroup is four wavefronts with neighbouring tiles of one slice, which find each other's A in L1.
-// Two steps are on their way; nothing is asked for beyond the last one: a load outside its window costs as much as another
+// D steps are on their way; nothing is asked for beyond the last one: a load outside its window costs as much as another
 // (128 x 128 blocks of 32, 512 features, four wavefronts 9.8 -> 9.1 us).
 // Against four wavefronts that shared 128 features through LDS and met at a barrier per step, us as part of a graph:
 // 128 x 128 blocks of 32, 10 %, 512 features 11.1 -> 9.1 (W = 4); 256 x 256, 512 features 24.0 -> 20.1 (W = 1); 209 x 46, 2
@@ -442,13 +494,12 @@ __device__ __forceinline__ void store_eight(void* __restrict__ Y, int64_t at, co
 // features through LDS: 197 x 193, 37 steps, 224 features 23.0 -> 16.3 (W = 4), 131 x 322, 78 steps, 128 features 18.7 ->
 // 14.9 (W = 8).  Small launches are bound by the trips to memory one after the other -- indptr, block columns, rows of X,
 // 2.8 us with the launch -- and then by X and A coming through the L2s, which hold neither (config above: 22 MB, 2.7 us).
-template <bool BF16, int OUT, int W, bool GROUP>
-__global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void bsr_direct_kernel(
+template <bool BF16, int OUT, int W, bool GROUP, int D = 2>
+__global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, D == 1 ? 4 : W == 1 ? 3 : 2) void bsr_direct_kernel(
     int blk, int feat, int64_t slices, int f_tiles, const uint16_t* __restrict__ A, const uint16_t* __restrict__ X,
     void* __restrict__ Y, const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
     const int32_t* __restrict__ row_ids) {
   static_assert(!GROUP || W == 1, "a group's wavefronts have tiles of their own");
-  constexpr int D = 2;  // steps on their way
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   int64_t slice;
@@ -503,30 +554,42 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void
         for (int r = 0; r < 2; ++r) acc[r][t] = mfma16<BF16>(a[s][r], b, acc[r][t]);
       }
     };
-    fetch(0);
-    if (left > 1) fetch(1);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D == 1) {
+      fetch(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (; left >= 2 * D; left -= D) {
-#pragma unroll
-      for (int s = 0; s < D; ++s) {
-        multiply(s);
+      for (; left > 1; --left) {
+        multiply(0);
         __builtin_amdgcn_sched_barrier(0);
-        fetch(s);
+        fetch(0);
         __builtin_amdgcn_sched_barrier(0);
       }
+      multiply(0);
+    } else {
+      fetch(0);
+      if (left > 1) fetch(1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+      for (; left >= 2 * D; left -= D) {
+#pragma unroll
+        for (int s = 0; s < D; ++s) {
+          multiply(s);
+          __builtin_amdgcn_sched_barrier(0);
+          fetch(s);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      multiply(0);  // one to three are left
+      if (left > 2) fetch(0);
+      if (left > 1) multiply(1);
+      if (left > 2) multiply(0);
     }
-    multiply(0);  // one to three are left
-    if (left > 2) fetch(0);
-    if (left > 1) multiply(1);
-    if (left > 2) multiply(0);
   }
 
   // acc[r][t][v] is row 16 r + 4 g + v, feature 8 c + t
-  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
-  const bool live = f0 + 8 * c < feat;
+  const int64_t row0 = (int64_t)i_out * blk + bi0;
   if constexpr (W == 1) {
-    if (!live) return;
+    __shared__ f32x4 stage[GROUP ? 4 : 1][OUT == 1 ? 2 * kWave : 1];
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -534,11 +597,11 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void
         float o[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) o[t] = acc[r][t][v];
-        store_eight<BF16, OUT>(Y, (row0 + 16 * r + v) * feat + f0 + 8 * c, o);
+        store_rows8<BF16, OUT, 16>(Y, row0 + 16 * r + v, feat, f0, lane, o, stage[GROUP ? wave : 0]);
       }
   } else {
     // each wavefront adds 8 / W of the eight rows a lane has
-    __shared__ __attribute__((aligned(16))) f32x4 part[W][16][kWave];
+    __shared__ __attribute__((aligned(16))) f32x4 part[W][8][2][kWave];
     const int used = min(steps, W);
     if (wave < used) {
 #pragma unroll
@@ -547,25 +610,14 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, W == 1 ? 3 : 2) void
         for (int v = 0; v < 4; ++v)
 #pragma unroll
           for (int e = 0; e < 2; ++e)
-            part[wave][(4 * r + v) * 2 + e][lane] =
+            part[wave][4 * r + v][e][lane ^ (8 * e)] =
                 f32x4{acc[r][4 * e][v], acc[r][4 * e + 1][v], acc[r][4 * e + 2][v], acc[r][4 * e + 3][v]};
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < 8 / W; ++q) {
       const int at = wave * (8 / W) + q;
-      float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int w = 0; w < W; ++w) {
-        if (w >= used) continue;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const f32x4 p = part[w][at * 2 + e][lane];
-#pragma unroll
-          for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
-        }
-      }
-      if (live) store_eight<BF16, OUT>(Y, (row0 + 16 * (at >> 2) + (at & 3)) * feat + f0 + 8 * c, o);
+      add_up8<BF16, OUT, W>(part[0][at][0], 8 * 2 * kWave, used, Y, row0 + 16 * (at >> 2) + (at & 3), feat, f0, lane);
     }
   }
 }
@@ -585,33 +637,20 @@ __device__ __forceinline__ u32x4 two_chunks(u32x4 a) {
 }
 __device__ __forceinline__ int first_row(int g) { return 8 * (g & 1) + 4 * (g >> 1); }
 
-// The sums of `used` of the W wavefronts at a tile, which have 4 / W (eight: the first four one) of a lane's four rows each; `at`
-// the place of the first.  part: those of this tile.
+// The sums of `used` of the W wavefronts at a tile, which have 4 / W (eight: the first four one) of a lane's four rows each; part:
+// those of this tile.
 template <bool BF16, int OUT, int W>
-__device__ __forceinline__ void add_up(const f32x4 (&acc)[8], f32x4 (&part)[W][8][kWave], int wave, int lane, int used,
-                                       void* __restrict__ Y, int64_t at, int feat, bool live) {
+__device__ __forceinline__ void add_up(const f32x4 (&acc)[8], f32x4 (&part)[W][4][2][kWave], int wave, int lane, int used,
+                                       void* __restrict__ Y, int64_t row0, int feat, int f0) {
   if (wave < used) {
 #pragma unroll
     for (int v = 0; v < 4; ++v)
 #pragma unroll
       for (int e = 0; e < 2; ++e)
-        part[wave][2 * v + e][lane] = f32x4{acc[4 * e][v], acc[4 * e + 1][v], acc[4 * e + 2][v], acc[4 * e + 3][v]};
+        part[wave][v][e][lane ^ (8 * e)] = f32x4{acc[4 * e][v], acc[4 * e + 1][v], acc[4 * e + 2][v], acc[4 * e + 3][v]};
   }
   __syncthreads();
-  for (int v = wave; v < 4; v += W) {
-    float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      if (w >= used) continue;
-#pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const f32x4 p = part[w][2 * v + e][lane];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) o[4 * e + t] += p[t];
-      }
-    }
-    if (live) store_eight<BF16, OUT>(Y, at + (int64_t)v * feat, o);
-  }
+  for (int v = wave; v < 4; v += W) add_up8<BF16, OUT, W>(part[0][v][0], 4 * 2 * kWave, used, Y, row0 + v, feat, f0, lane);
 }
 
 // A tile of 16 rows x 128 features, eight accumulators of v_mfma_f32_16x16x32; W wavefronts take the steps in turn.  T such tiles
@@ -702,20 +741,20 @@ __global__ __launch_bounds__(W * T * kWave, W == 1 ? 4 : 2) void bsr16_direct_ke
   }
 
   // acc[t][v] is row 4 g + v, feature 8 c + t
-  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
-  const bool live = f0 + 8 * c < feat;
+  const int64_t row0 = (int64_t)i_out * blk + bi0;
   if constexpr (W == 1) {
-    if (!live) return;
+    static_assert(T == 1, "one wavefront to a workgroup");
+    __shared__ f32x4 stage[OUT == 1 ? 2 * kWave : 1];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       float o[8];
 #pragma unroll
       for (int t = 0; t < 8; ++t) o[t] = acc[t][v];
-      store_eight<BF16, OUT>(Y, (row0 + v) * feat + f0 + 8 * c, o);
+      store_rows8<BF16, OUT, 16>(Y, row0 + v, feat, f0, lane, o, stage);
     }
   } else {
-    __shared__ __attribute__((aligned(16))) f32x4 part[T][W][8][kWave];
-    add_up<BF16, OUT, W>(acc, part[(tid >> 6) / W], wave, lane, min(steps, W), Y, row0 * feat + f0 + 8 * c, feat, live);
+    __shared__ __attribute__((aligned(16))) f32x4 part[T][W][4][2][kWave];
+    add_up<BF16, OUT, W>(acc, part[(tid >> 6) / W], wave, lane, min(steps, W), Y, row0, feat, f0);
   }
 }
 
@@ -819,26 +858,24 @@ __global__ __launch_bounds__(W * kWave, 3) void bsr16_wave_kernel(int blk, int f
       }
     }
   }
-  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * g;
+  const int64_t row0 = (int64_t)i_out * blk + bi0;
   if constexpr (W == 1) {
+    __shared__ f32x4 stage[OUT == 1 ? 2 * kWave : 1];
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      if (f0 + 128 * m + 8 * c >= feat) return;
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         float o[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) o[t] = acc[m][t][v];
-        store_eight<BF16, OUT>(Y, (row0 + v) * feat + f0 + 128 * m + 8 * c, o);
+        store_rows8<BF16, OUT, 16>(Y, row0 + v, feat, f0 + 128 * m, lane, o, stage);
       }
-    }
   } else {
-    __shared__ __attribute__((aligned(16))) f32x4 part[W][8][kWave];
+    __shared__ __attribute__((aligned(16))) f32x4 part[W][4][2][kWave];
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       if (m) __syncthreads();
-      add_up<BF16, OUT, W>(acc[m], part, wave, lane, min(steps, W), Y, row0 * feat + f0 + 128 * m + 8 * c, feat,
-                           f0 + 128 * m + 8 * c < feat);
+      add_up<BF16, OUT, W>(acc[m], part, wave, lane, min(steps, W), Y, row0, feat, f0 + 128 * m);
     }
   }
 }
@@ -941,14 +978,13 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
     }
   }
   // acc[t][v] is row (v % 4) + 4 h + 8 (v / 4), feature 8 n + t
-  if (f0 + 8 * n >= feat) return;
-  const int64_t row0 = (int64_t)i_out * blk + bi0 + 4 * h;
+  const int64_t row0 = (int64_t)i_out * blk + bi0;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     float o[8];
 #pragma unroll
     for (int t = 0; t < FT; ++t) o[t] = acc[t][v];
-    store_eight<BF16, OUT>(Y, (row0 + (v & 3) + 8 * (v >> 2)) * feat + f0 + 8 * n, o);
+    store_rows8<BF16, OUT, 32>(Y, row0 + (v & 3) + 8 * (v >> 2), feat, f0, lane, o, reinterpret_cast<f32x4*>(piece));
   }
 }
 
@@ -1117,6 +1153,7 @@ struct BsrForm {
   bool by_rows;  // block rows dealt to XCDs
   int direct = 0;  // operands in registers, so many wavefronts to a tile (16-row slices: kWaves too may have several, and
                    // kGroups with two of them has two tiles of 128 features to a workgroup)
+  bool single = false;  // bsr_direct_kernel with one step of a wavefront on its way
 };
 
 inline int slice_rows(int blk, BsrForm::Kernel kernel) {  // blocks that are a multiple of 64 are no direct groups
@@ -1135,8 +1172,10 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // Tiles of 64 features, by eight wavefronts through LDS, where rows are long and tiles of 128 leave CUs without one or,
     // hardly more than the CUs, with twice as much as the next: 35 x 437 blocks, 97 steps, 96 features 14.6 us, 16.9 with 128;
     // 42 x 285, 70 steps, 64 10.6, 11.3; 93 x 431, 106 steps, 320 (279 tiles) 26.0, 29.6; but 136 x 333, 67 steps, 256 (272, and
-    // 544 of 64) 24.1, 20.8.
-    if (steps >= 40 && (split * 4 <= (feat % kSplitF ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus)))
+    // 544 of 64) 24.1, 20.8.  A little sooner where 128 waste half of a load: 8 x 35 of 128, 35 steps, 192 features 9.4, 10.1.
+    const bool half = feat % kTileF != 0 && feat % kTileF <= kSplitF;
+    if ((steps >= 40 && (split * 4 <= (feat % kSplitF ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus))) ||
+        (steps >= 32 && half && split <= cus))
       return {BsrForm::kSplit, false, false, false};
     // Steps in turn as long as that leaves a CU little more than two workgroups of four wavefronts, or four of two; us with W =
     // 1 / 2 / 4: 272 x 121 blocks, 25 steps, 224 features (544 tiles) 18.4 / 16.2 / 15.6, 292 x 182, 16 steps, 224 features
@@ -1150,9 +1189,11 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // 1; 220 x 66, 5 steps, 288 features 6.9, 7.6; 396 x 27, 5 steps, 416 features 9.7, 10.5; but 166 x 95, 19 steps, 416 17.0, 16)
     if (blk == 32 && feat > kTileF && feat <= 4 * kTileF && steps <= 8 && x_tile_bytes(kWaveF) <= 2500000)
       return {BsrForm::kGroups, false, false, false, 1};
-    // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long: 11 x 119 blocks of 128, 92 steps,
-    // 2304 features 50, 57)
-    if (tiles * 4 <= 13 * cus && !few && (blk % 64 != 0 || steps < 48)) return {BsrForm::kSplit, false, false, false, 2};
+    // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long and CUs have more than three
+    // tiles: blocks of 64, 672 features, 46 steps (804 tiles) 31 / 37, 928, 31 steps (817) 23 / 26, of 128, 2304, 92 steps (792) 50 /
+    // 57; but 1600, 69 steps (676) 43 / 38, of 64, 2240, 30 steps (755) 23.0 / 19.7)
+    const int quarters = blk % 64 != 0 || steps < 24 ? 13 : steps < 48 ? 12 : 11;
+    if (tiles * 4 <= quarters * cus && !few) return {BsrForm::kSplit, false, false, false, 2};
   } else if (unit == 32) {
     // The split form wins as long as its workgroups are resident at once, two per CU, and up to twice as many where block rows
     // have enough steps to pay for the second turn.
@@ -1199,14 +1240,16 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // Much X: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
     // ranked / 256 ranked: blocks of 16, 1024 columns (8.4 MB), 51 steps, 1024 features 205 / 188 / 163, 24 steps 105 / 104 / 94,
     // 4096 features 1204 / 780 / 650; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184; of 48, 65 steps,
-    // 3424 543 / 539 / 534.  Between 16 and 28 steps only with far more X than an L2 holds (575 columns, 16 steps, 2784 features
-    // 41 / 45 / 46) or with few tiles, where the order gives little: 490, 17 steps, 512 features 34 / 40 / 42; 330 of 48, 25 steps,
-    // 608 44 / 48 / 53.
+    // 3424 543 / 539 / 534.  Between 20 and 28 steps 128, with far more X than an L2 holds: 799 columns, 24 steps, 1632 features 167
+    // / 145 / 163, 993, 22 steps, 3744 108 / 101 / 115; less of it, 722 columns, 25 steps, 2752 174 / 176 / 173, 575, 16 steps, 2784
+    // 39 / 42 / 39.  From 16 steps on 256 with few tiles, where the order gives little: 1024 columns, 24 steps, 1024 features 100 / 99 /
+    // 90, but 490, 17 steps, 512 34 / 40 / 40.
     const bool wide_ranked = fits && (even || waste * 16 <= feat);
     if (x_bytes > kMuchX && feat > kTileF && steps >= 16) {
-      if (wide_ranked && (steps >= 28 || (wide_tiles >= 2 && x_bytes > kBeyondL2 && (wide_tiles <= 4 || x_bytes > 2 * kBeyondL2))))
+      if (wide_ranked && (steps >= 28 || (wide_tiles >= 2 && wide_tiles <= 4 && x_bytes > kBeyondL2)))
         return {BsrForm::kWaves, true, true, false, 1};
-      if (!wide_ranked && unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (steps >= 28 || x_narrow > kBeyondL2))
+      const bool long_enough = !wide_ranked && (steps >= 28 || x_narrow > kBeyondL2);
+      if (unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (long_enough || (steps >= 20 && x_bytes > 6200000)))
         return {BsrForm::kWaves, false, true, false, 1};
     }
     // Blocks of several slices, which read the same X.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of 80, 10
@@ -1248,11 +1291,20 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
   // steps, 2784 (957, 6.9 MB) 78 / 69.  Blocks of several slices, which read the same X, with much of it: 256 up to twice
   // what an L2 holds, or by workgroups: 400 x 170 of 96 (8.4 MB), 16 steps, 512 features 50 ranked, 60 with 256 as they come,
   // 65 with 128, 64 by workgroups; 1300 x 325 (16 MB), 8 steps, 1504 features 310, 352, 429, 280.
+  // Long rows, more X than an L2 holds and a turn of wavefronts: 128 with one step on their way each and four to a SIMD stay closer
+  // together in X; 128 / 128 with one step / 256 (6 to 8.2 MB of X in 256): 80 x 501, 61 steps, 2720 features (1760 wavefronts of 128)
+  // 88 / 74 / 87, 53 x 495, 45 steps, 3712 (1537) 52 / 50.5 / 59, 60 x 500, 101 steps, 2720 (1320) 96 / 86 / 88; but 40 x 500, 46
+  // steps, 3712 (1160) 41.6 / 43.2 / 47, and with many more 139 x 437, 24
+  // steps, 3040 (3336) 73 / 71 / 67.
+  // Up to four steps a row 128: the results are most of it, and leave sooner (381 x 87, 3 steps, 1536 features 15.2 / - / 15.7, fp32
+  // results 19.9 / - / 22.5).
   if (rs == 1 && wavefronts) {
     const bool one = blk == 32;
     const int64_t waves = slices * wide_tiles, x_bytes = x_tile_bytes(std::min(feat, kWaveF));
+    const bool crowd = one && steps >= 20 && x_bytes > kMuchX && tiles >= 5 * cus && tiles * 2 <= 17 * cus;
+    if (crowd) return {BsrForm::kWaves, false, false, false, 1, true};
     const bool ranked = waste * 3 <= feat && rank_pays(x_bytes, wide_tiles, waves, steps >= 64 && wide_tiles >= 4 ? 3 : 5);
-    const bool wide = ranked || (x_bytes <= kMuchX ? waste * 3 <= feat && waves * 10 >= 27 * cus
+    const bool wide = ranked || (x_bytes <= kMuchX ? waste * 3 <= feat && waves * 10 >= 27 * cus && steps > 4
                                  : !one            ? waste * 8 <= feat && x_bytes <= 2 * kBeyondL2 && waves >= 8 * cus
                                  : steps >= 24     ? waste * 4 <= feat && waves >= 3 * cus
                                                    : waste * 8 <= feat && x_bytes <= kBeyondL2 && waves >= 5 * cus);
@@ -1324,6 +1376,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       else STIR_BSR_16((BF, OUT, 8, 1), 8);                                                                    \
     } else if (form.direct) {                                                                                  \
       if (form.kernel == BsrForm::kGroups) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, true>), 4 * kWave);      \
+      else if (form.single) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false, 1>), kWave);                     \
       else if (form.direct == 1) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false>), kWave);                   \
       else if (form.direct == 8) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 8, false>), 8 * kWave);               \
       else if (form.direct == 4) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 4, false>), 4 * kWave);               \
@@ -1358,12 +1411,12 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
 extern "C" {
 
 // The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
-// in order of their length, 16 for block rows dealt to XCDs, 32 times the wavefronts at a tile of those that make their operands in registers (0: of bsr_wave_kernel, and of LDS forms);
-// -1 for what no product is.  For the tests, which say what they cover.
+// in order of their length, 16 for block rows dealt to XCDs, 32 times BsrForm::direct, 512 for BsrForm::single; -1 for what no
+// product is.  For the tests, which say what they cover.
 int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
   if (cus <= 0 || mb <= 0 || nb < 0 || nnzb < 0 || blk <= 0 || blk % 16 != 0 || feat <= 0) return -1;
   const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb);
-  return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows + 32 * f.direct;
+  return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows + 32 * f.direct + 512 * f.single;
 }
 
 int stir_bsr_spmm(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, int32_t blk, int32_t feat,

@@ -26,7 +26,7 @@ def _edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
     cfg["data"] = rng.standard_normal((nnzb, blk, blk)).astype(np.float32) * 0.1
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     code = _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb))
-    assert code // 32 == waves
+    assert code // 32 == waves  # 16 + 1: one wavefront with one step on its way
     out, start = (torch.float32, 1) if (mb & 1) == (dtype is torch.float16) else (dtype, 0)
 
     def place(values):
@@ -56,6 +56,7 @@ def _edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
     (331, 20, 32, 160, 5, 1),        # two tiles to a slice: two slices in a workgroup
     (300, 40, 32, 544, 7, 1),
     (160, 9, 96, 160, 3, 1),
+    (70, 240, 32, 2592, 60, 17),     # one step on its way; nothing to one step for some
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_direct_edges(dev, mb, nb, blk, feat, at_most, waves, dtype):

@@ -626,7 +626,7 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, D == 1 ? 4 : W == 1 
 // A step is two chunks of 16 columns, and of the k slots 8 g ... of lane group g four are rows of the first and four of the
 // second, in A and X alike: so a load of X is of one chunk, whose place is the same for all lanes.  The groups have the rows 0, 8,
 // 4, 12 ... of a chunk: A comes 16 bytes a lane, columns 8 (g & 1) ... of chunk g / 2, and two swaps of half wavefronts put it
-// so.  Rows of X have their offsets in lanes' registers: what an empty window's loads with a scalar offset give is not zeros.
+// so.  All offsets are in lanes' registers: an empty window's loads with scalar ones are not relied on to be zeros.
 __device__ __forceinline__ u32x4 two_chunks(u32x4 a) {
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
@@ -822,9 +822,9 @@ __global__ __launch_bounds__(W * kWave, 3) void bsr16_wave_kernel(int blk, int f
   u32x4 x[2][8];
   u32x4 ar;
   auto fetch_a = [&]() {
-    const uint32_t bytes = at[0] < nblk ? (at[0] + 1 < nblk ? 4 * blk * blk : 2 * blk * blk) : 0;
+    const uint32_t block_bytes = 2u * blk * blk, bytes = at[0] < nblk ? (at[0] + 1 < nblk ? 2 * block_bytes : block_bytes) : 0;
     const auto ra = window(A + (int64_t)(p_begin + at[0]) * blk * blk, bytes);
-    ar = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + (g >> 1) * ((at[1] - at[0]) * blk * blk + k0[1] - k0[0]) * 2, k0[0] * 2, 0);
+    ar = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + (k0[0] + (g >> 1) * ((at[1] - at[0]) * blk * blk + k0[1] - k0[0])) * 2, 0, 0);
   };
   auto fetch_x = [&](int m) {
 #pragma unroll
@@ -932,7 +932,9 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
     int block = 0, k0 = 0, j = cols[0], j_next = cols[min(1, nblk - 1)];
     u32x4 x[2][8], ar[2], a[2];
     auto fetch_a = [&]() {
-      const auto ra = window(A + (int64_t)(p_begin + block) * blk * blk + k0, block < nblk ? (uint32_t)(blk * blk - k0) * 2 : 0);
+      // the window begins inside A also when it is empty: nothing rests on what a scalar offset does to an empty one
+      const auto ra = window(A + (int64_t)(p_begin + min(block, nblk - 1)) * blk * blk + k0,
+                             block < nblk ? (uint32_t)(blk * blk - k0) * 2 : 0);
 #pragma unroll
       for (int m = 0; m < 2; ++m) ar[m] = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff, m * 32 * blk, 0);
     };

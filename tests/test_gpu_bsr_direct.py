@@ -56,7 +56,7 @@ def _edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
     (331, 20, 32, 160, 5, 1),        # two tiles to a slice: two slices in a workgroup
     (300, 40, 32, 544, 7, 1),
     (160, 9, 96, 160, 3, 1),
-    (70, 240, 32, 2592, 60, 17),     # one step on its way; nothing to one step for some
+    (70, 200, 32, 2336, 30, 17),     # one step on its way; nothing to one step for some
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_direct_edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
@@ -74,7 +74,7 @@ def test_direct_edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
     (160, 9, 112, 288, 3, 2),
     (420, 45, 16, 480, 7, 1),        # 128 features by one wavefront
     (1050, 20, 16, 480, 16, 1),      # 256
-    (110, 40, 80, 1024, 9, 1),
+    (205, 20, 80, 480, 4, 1),
     (230, 140, 48, 992, 12, 4),      # 256 by four
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -11,12 +11,9 @@ from sparsetir_amd import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("t", [8, 16, 32])
-@pytest.mark.parametrize("feat", [96, 128, 224, 288])
-@pytest.mark.parametrize("out_dtype,start", [(torch.float16, 1), (torch.float32, 1), (torch.float32, 0)])
-def test_odd_groups(dev, t, feat, out_dtype, start):
+def _odd_groups(dev, t, feat, out_dtype, start, empty=0):
     rng = np.random.default_rng(feat + t)
-    n, counts = 900, [16, 48, 80, 32, 144, 0, 688]  # columns of a tile: 1, 3, 5, 2, 9, 0 and 43 groups
+    n, counts = 900, [16, 48, 80, 32, 144, 0, 688] + [0] * empty  # columns of a tile: 1, 3, 5, 2, 9, 0 and 43 groups
     cols = [np.sort(rng.choice(np.arange(1, n), c, replace=False)) for c in counts]
     rows = [c for c in cols for _ in range(t)]
     indptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
@@ -51,3 +48,18 @@ def test_odd_groups(dev, t, feat, out_dtype, start):
         # fp32 sums of up to 688 exact products: 688 roundings of 2^-24 of the terms; one more of an fp16 result
         bound = 688 * 2.0 ** -24 * scale + (2.0 ** -11 * np.abs(want) if out_dtype is torch.float16 else 0.0) + 1e-7
         assert np.all(np.abs(got[io] - want) <= bound)
+
+
+@pytest.mark.parametrize("t", [8, 16, 32])
+@pytest.mark.parametrize("feat", [96, 128, 224, 288])
+@pytest.mark.parametrize("out_dtype,start", [(torch.float16, 1), (torch.float32, 1), (torch.float32, 0)])
+def test_odd_groups(dev, t, feat, out_dtype, start):
+    _odd_groups(dev, t, feat, out_dtype, start)
+
+
+@pytest.mark.parametrize("t", [8, 16, 32])
+@pytest.mark.parametrize("feat", [160, 288])
+@pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
+def test_a_unit_of_32_features(dev, t, feat, out_dtype):
+    """32 features have a unit of 128 to themselves only where B is taken to be large, as large as C: many rows, most of them empty."""
+    _odd_groups(dev, t, feat, out_dtype, 1, 13_000_000 // (2 * feat * t) + 1)

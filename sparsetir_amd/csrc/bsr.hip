@@ -654,18 +654,17 @@ __device__ __forceinline__ void add_up(const f32x4 (&acc)[8], f32x4 (&part)[W][4
 }
 
 // A tile of 16 rows x 128 features, eight accumulators of v_mfma_f32_16x16x32; W wavefronts take the steps in turn.  T such tiles
-// side by side to a workgroup, whose wavefronts find each other's A in L1.  Two steps of a wavefront are on their way.
+// side by side to a workgroup, whose wavefronts find each other's A in L1.  D steps of a wavefront are on their way.
 // Against X through LDS (wavefronts with 128 or 256 features, or four that met at a barrier per step), us: 398 x 310 blocks of
 // 16, 19 steps, 576 features 34 -> 20.5 (W = 4); 749 x 92, 8 steps, 160 features 15.4 -> 9.1 (T = 2); 342 x 83, 4 steps, 1728
 // features 18.5 -> 14.8 (W = 1); 154 tiles of 80 steps 16.8 -> 13.0 (W = 8).  LDS, which X passed twice, had been as busy as the
 // L1s.  Bound by the L1s and the trips to memory at small sizes, by X from beyond L2 at large ones.  A by two loads of 8 bytes a
 // lane, without the swaps: 3 % slower, blocks of 48 and 80 5 to 8 %.
-template <bool BF16, int OUT, int W, int T, bool ONE>
-__global__ __launch_bounds__(W * T * kWave, W == 1 ? 4 : 2) void bsr16_direct_kernel(
+template <bool BF16, int OUT, int W, int T, bool ONE, int D = 2>
+__global__ __launch_bounds__(W * T * kWave, D == 1 ? 5 : W == 1 ? 4 : 2) void bsr16_direct_kernel(
     int blk, int feat, int64_t slices, int f_tiles, int ranked, const uint16_t* __restrict__ A,
     const uint16_t* __restrict__ X, void* __restrict__ Y, const int32_t* __restrict__ indptr,
     const int32_t* __restrict__ indices, const int32_t* __restrict__ row_ids) {
-  constexpr int D = 2;  // steps on their way
   if (ONE) blk = 16;
   const int sub = blk / 16;  // 16-row slices per block row = 16-column chunks per block
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) % W;
@@ -721,23 +720,36 @@ __global__ __launch_bounds__(W * T * kWave, W == 1 ? 4 : 2) void bsr16_direct_ke
 #pragma unroll
       for (int t = 0; t < 8; ++t) acc[t] = mfma16<BF16>(rows, operand_of(x[s], t / 2, t % 2), acc[t]);
     };
-    fetch(0);
-    if (left > 1) fetch(1);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (D == 1) {
+      fetch(0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (; left >= 2 * D; left -= D) {
-#pragma unroll
-      for (int s = 0; s < D; ++s) {
-        multiply(s);
+      for (; left > 1; --left) {
+        multiply(0);
         __builtin_amdgcn_sched_barrier(0);
-        fetch(s);
+        fetch(0);
         __builtin_amdgcn_sched_barrier(0);
       }
+      multiply(0);
+    } else {
+      fetch(0);
+      if (left > 1) fetch(1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+      for (; left >= 2 * D; left -= D) {
+#pragma unroll
+        for (int s = 0; s < D; ++s) {
+          multiply(s);
+          __builtin_amdgcn_sched_barrier(0);
+          fetch(s);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      multiply(0);  // one to three are left
+      if (left > 2) fetch(0);
+      if (left > 1) multiply(1);
+      if (left > 2) multiply(0);
     }
-    multiply(0);  // one to three are left
-    if (left > 2) fetch(0);
-    if (left > 1) multiply(1);
-    if (left > 2) multiply(0);
   }
 
   // acc[t][v] is row 4 g + v, feature 8 c + t
@@ -1155,7 +1167,7 @@ struct BsrForm {
   bool by_rows;  // block rows dealt to XCDs
   int direct = 0;  // operands in registers, so many wavefronts to a tile (16-row slices: kWaves too may have several, and
                    // kGroups with two of them has two tiles of 128 features to a workgroup)
-  bool single = false;  // bsr_direct_kernel with one step of a wavefront on its way
+  bool single = false;  // the direct kernels with one step of a wavefront on its way
 };
 
 inline int slice_rows(int blk, BsrForm::Kernel kernel) {  // blocks that are a multiple of 64 are no direct groups
@@ -1254,6 +1266,12 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
       if (unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (long_enough || (steps >= 20 && x_bytes > 6200000)))
         return {BsrForm::kWaves, false, true, false, 1};
     }
+    // Long rows, far more X than an L2 holds and a turn of wavefronts: by one, which stay closer together in X, with one step on its
+    // way each where there are more of them; 128 by four / by one with two steps / with one: 95 x 793, 26 steps, 1856 features
+    // (1425 tiles) 24.8 / 22.1 / 23.7, 80 x 818, 23 steps, 2848 (1840) 34.5 / 30.9 / 28.6, 70 x 896, 40 steps, 2848 (1610) 48.4 / 40.6 /
+    // 37.8, 183 x 840, 64 steps, 1568 (2379) 84.5 / 83.5 / 80.6; but 4.35 tiles to a CU, 90 steps, 320 features 50.5 / 52.3 / 61.5.
+    if (!several && steps >= 20 && x_bytes > 6000000 && tiles * 10 >= 46 * cus && tiles < 10 * cus)
+      return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
     // Blocks of several slices, which read the same X.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of 80, 10
     // steps, 416 features 138 / 130, 600 x 650 of 48, 7 steps, 256 20.8 / 21.0.  Less of it, 256 by four / by one: 1100 x 341 of 48,
     // 10 steps, 1024 features 147 / 169, 5 steps, 140 columns 26 / 22.  And A, which every tile reads, more than the last level
@@ -1362,6 +1380,11 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     if (blk == 16) STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);          \
     else STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, false>), (WAVES) * kWave, ranked);                   \
   } while (0)
+#define STIR_BSR_16S(BF, OUT)                                                                                  \
+  do {                                                                                                         \
+    if (blk == 16) STIR_BSR_GO((bsr16_direct_kernel<BF, OUT, 1, 1, true, 1>), kWave, ranked);                  \
+    else STIR_BSR_GO((bsr16_direct_kernel<BF, OUT, 1, 1, false, 1>), kWave, ranked);                           \
+  } while (0)
 #define STIR_BSR_16W(ARGS, WAVES)                                                                              \
   do {                                                                                                         \
     if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);            \
@@ -1373,6 +1396,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       if (form.kernel == BsrForm::kGroups && form.direct == 2) STIR_BSR_16((BF, OUT, 2, 2), 4);                \
       else if (form.wide && form.direct == 1) STIR_BSR_16W((BF, OUT, 1), 1);                                   \
       else if (form.wide) STIR_BSR_16W((BF, OUT, 4), 4);                                                       \
+      else if (form.single) STIR_BSR_16S(BF, OUT);                                                             \
       else if (form.direct == 1) STIR_BSR_16((BF, OUT, 1, 1), 1);                                              \
       else if (form.direct == 4) STIR_BSR_16((BF, OUT, 4, 1), 4);                                              \
       else STIR_BSR_16((BF, OUT, 8, 1), 8);                                                                    \
@@ -1403,6 +1427,7 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   }
 #undef STIR_BSR
 #undef STIR_BSR_16W
+#undef STIR_BSR_16S
 #undef STIR_BSR_16
 #undef STIR_ARGS
 #undef STIR_BSR_GO

@@ -73,6 +73,7 @@ def test_direct_edges(dev, mb, nb, blk, feat, at_most, waves, dtype):
     (640, 25, 16, 608, 17, 2),       # ... of five
     (160, 9, 112, 288, 3, 2),
     (420, 45, 16, 480, 7, 1),        # 128 features by one wavefront
+    (96, 750, 16, 2176, 61, 17),     # one step on its way; nothing to one step for some
     (1050, 20, 16, 480, 16, 1),      # 256
     (205, 20, 80, 480, 4, 1),
     (230, 140, 48, 992, 12, 4),      # 256 by four

@@ -697,13 +697,16 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
 // 19 TB/s, 16 bytes at 33.  Through LDS / in registers, us: 169 k rows, 1.17 M nonzeros, 128 features, tiles of 16 rows 63.3 /
 // 57.9, of 32 72 / 65.4; 100 k, 1 M, 256 features, 16 rows 90.4 / 84.4; 150 k, 3 M, skewed columns, 128 86.8 / 81.0.  Bound by the rows of B
 // that miss an L2 (8.2 TB/s for rows out of 32 MB).
-template <int T, int W, int OUT>
-__global__ __launch_bounds__(64 * W, T == 32 ? 2 : T == 16 ? 3 : 4) void tcspmm_direct_kernel(
+// D steps of a wavefront are on their way.  With two, a SIMD has registers for 4 / 3 / 2 wavefronts (tiles of 8 / 16 / 32 rows) and
+// 32-row tiles leave 64 KB of sums for four wavefronts, 32 KB for two: few units at a time where tiles have a step or two for a
+// wavefront, which hide nothing in themselves.  With one it has 5 / 4 / 3, and 32-row tiles pass half of their sums at a time
+// through half of the LDS (tc_form says where which pays).
+template <int T, int W, int OUT, int D>
+__global__ __launch_bounds__(64 * W, T == 8 ? 4 : (T == 32 ? 2 : 3) + (D == 1)) void tcspmm_direct_kernel(
     int feat, int64_t mb, int f_tiles, int64_t n_pieces, const TcPiece* __restrict__ pieces, const uint16_t* __restrict__ A,
     const uint16_t* __restrict__ B, void* __restrict__ C, int aligned, float* scratch, uint32_t* arrived,
     const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices) {
   constexpr int TF = 128, RH = T == 32 ? 2 : 1;  // RH: operands of 16 rows
-  constexpr int D = T == 8 ? 1 : 2;              // steps on their way
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int f_tile = (int)(blockIdx.x % f_tiles);
@@ -811,59 +814,66 @@ __global__ __launch_bounds__(64 * W, T == 32 ? 2 : T == 16 ? 3 : 4) void tcspmm_
     }
   }
 
-  // ---- the sums over the wavefronts: each adds 4 RH / W of the rows a lane has.  acc[r][t][v] is row 16 r + 4 g + v, feature
-  // 8 c + t.  Sixteen-bit results leave as they lie; floats are read four features to a lane in the order of the row, so that a
-  // store is of whole lines (halves of lines: 169 k rows, 8-row tiles, 128 features 68.5 us, now 66.5).
-  __shared__ __attribute__((aligned(16))) f32x4 sums[W][4 * RH][2][64];  // [e][lane ^ 8 e]: eight lanes in row order share no bank
+  // ---- the sums over the wavefronts, `ROUND` operands of 16 rows at a time: each adds 4 ROUND / W of the rows a lane has.
+  // acc[r][t][v] is row 16 r + 4 g + v, feature 8 c + t.  Sixteen-bit results leave as they lie; floats are read four features to a
+  // lane in the order of the row, so that a store is of whole lines (halves of lines: 169 k rows, 8-row tiles, 128 features 68.5
+  // us, now 66.5).
+  constexpr int ROUND = D == 1 ? 1 : RH;
+  __shared__ __attribute__((aligned(16))) f32x4 sums[W][4 * ROUND][2][64];  // [e][lane ^ 8 e]: eight lanes in row order share no bank
   const int used = min(W, s_end - s_begin);
-  if (wave < used) {
-#pragma unroll
-    for (int at = 0; at < 4 * RH; ++at)
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-        sums[wave][at][e][lane ^ (8 * e)] = f32x4{acc[at >> 2][4 * e][at & 3], acc[at >> 2][4 * e + 1][at & 3],
-                                                  acc[at >> 2][4 * e + 2][at & 3], acc[at >> 2][4 * e + 3][at & 3]};
-  }
-  __syncthreads();
   const int64_t elems = (int64_t)T * feat;
   const bool part = pc.slot >= 0;
   const stir::CoherentPiece partial(scratch + (part ? (int64_t)pc.slot * elems : 0), part ? (uint32_t)(elems * 4) : 0u);
 #pragma unroll
-  for (int q = 0; q < 4 * RH / W; ++q) {
-    const int at = wave * (4 * RH / W) + q;
-    const bool floats = OUT == 1 || part;
-    f32x4 o[2];
-    int place[2];  // of o[i] in sums: lane ^ 8 e, with 64 e
+  for (int r0 = 0; r0 < RH; r0 += ROUND) {
+    if (r0) __syncthreads();  // the sums before have been read
+    if (wave < used) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int piece = 64 * i + lane, e = floats ? piece & 1 : i;  // in row order: row piece / 32, features 4 (piece % 32) ...
-      place[i] = 64 * e + ((floats ? piece >> 1 : lane) ^ (8 * e));
-      o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int at = 0; at < 4 * ROUND; ++at)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const auto& o = acc[r0 + (at >> 2)];
+          sums[wave][at][e][lane ^ (8 * e)] = f32x4{o[4 * e][at & 3], o[4 * e + 1][at & 3], o[4 * e + 2][at & 3], o[4 * e + 3][at & 3]};
+        }
     }
+    __syncthreads();
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      if (w >= used) continue;
+    for (int q = 0; q < 4 * ROUND / W; ++q) {
+      const int from = wave * (4 * ROUND / W) + q, at = 4 * r0 + from;
+      const bool floats = OUT == 1 || part;
+      f32x4 o[2];
+      int place[2];  // of o[i] in sums: lane ^ 8 e, with 64 e
 #pragma unroll
-      for (int i = 0; i < 2; ++i) o[i] += sums[w][at][0][place[i]];
-    }
-    if (!floats) {
-      const int row = 16 * (at >> 2) + 4 * g + (at & 3);
-      u32x4 w;
+      for (int i = 0; i < 2; ++i) {
+        const int piece = 64 * i + lane, e = floats ? piece & 1 : i;  // in row order: row piece / 32, features 4 (piece % 32) ...
+        place[i] = 64 * e + ((floats ? piece >> 1 : lane) ^ (8 * e));
+        o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2)]) |
-               (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2) + 1]) << 16;
-      if (f0 + 8 * c < feat && (T >= 16 || row < T))
-        *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
-      continue;
-    }
+      for (int w = 0; w < W; ++w) {
+        if (w >= used) continue;
 #pragma unroll
-    for (int i = 0; i < (T == 8 ? 1 : 2); ++i) {  // of 8 rows the other half is no rows
-      const int row = 16 * (at >> 2) + 8 * i + 4 * (lane >> 5) + (at & 3), fcol = f0 + 4 * (lane & 31);
-      if (fcol >= feat) continue;
-      const float4 v = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
-      if (part) partial.store((uint32_t)(row * feat + fcol), v);
-      else *reinterpret_cast<Float4*>(static_cast<float*>(C) + (io * T + row) * feat + fcol) = Float4{v.x, v.y, v.z, v.w};
+        for (int i = 0; i < 2; ++i) o[i] += sums[w][from][0][place[i]];
+      }
+      if (!floats) {
+        const int row = 16 * (at >> 2) + 4 * g + (at & 3);
+        u32x4 w;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2)]) |
+                 (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2) + 1]) << 16;
+        if (f0 + 8 * c < feat && (T >= 16 || row < T))
+          *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < (T == 8 ? 1 : 2); ++i) {  // of 8 rows the other half is no rows
+        const int row = 16 * (at >> 2) + 8 * i + 4 * (lane >> 5) + (at & 3), fcol = f0 + 4 * (lane & 31);
+        if (fcol >= feat) continue;
+        const float4 v = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+        if (part) partial.store((uint32_t)(row * feat + fcol), v);
+        else *reinterpret_cast<Float4*>(static_cast<float*>(C) + (io * T + row) * feat + fcol) = Float4{v.x, v.y, v.z, v.w};
+      }
     }
   }
   if (part) tc_add_pieces<T, TF, W, OUT>(pc, io, f_tile, f_tiles, feat, C, aligned, scratch, arrived);
@@ -912,48 +922,108 @@ int launch_unplanned(bool out32, int32_t mb, int32_t feat, const uint16_t* A, co
   return 0;
 }
 
+// How a product with a plan is launched.
+struct TcForm {
+  int tiles;      // of 32 features to a unit: 4 by tcspmm_direct_kernel, else by tcspmm_units_kernel
+  int waves;      // to a unit
+  bool one_step;  // tcspmm_direct_kernel with one step of a wavefront on its way
+};
+
+TcForm tc_form(int T, bool out32, int64_t mb, int feat, int64_t nnzb, int64_t n_pieces) {
+  // Units of 128 features above 64 (tcspmm_direct_kernel), their last one however full; us with units of 64 features, by the
+  // other kernel, / of 128: 20 k rows, 300 k nonzeros, 128 features 16.2 / 14.4, 100 k, 500 k, 96 33.6 / 26.0, 120 k, 600 k, 160
+  // 61.2 / 53.7, 60 k, 900 k, 192 66.1 / 56.4; 33 k, 160 features, 8-, 16-, 32-row tiles of 5 to 20 steps 0.82 to 0.98 of the time;
+  // and of 64 features alone 60 k, 900 k 25.7 / 29.5, 200 k, 4 M 66 / 80.  Two exceptions:
+  //   128 features, many 8-row tiles of several steps: there is little of A to fetch twice, and the two units of 64 of a tile are
+  //   neighbours, so that every other XCD has the same half of B in its L2: 50 k rows, 1.25 M nonzeros (6.5 steps) 42 / 47, 169 k,
+  //   4.2 M 154 / 165, skewed columns 123 / 135 (but of 50 k rows 40 / 35); 4 steps 116 / 110, 2.2 steps 29.9 / 30.1, 4125 tiles of
+  //   6.3 steps 26.4 / 25.2;
+  //   32 features in a unit of 128 of their own, 32-row tiles, of which hardly a turn is resident (64 KB of sums each): 12 k rows, 49
+  //   k nonzeros, 160 features 10.2 / 10.9; with units of 32 KB below that is no reason: 33 k, 165 k, 160 15.7 / 15.3.
+  const int64_t wide_units = (mb + n_pieces) * stir::ceil_div(feat, 128);
+  const bool halves = T == 8 && feat == 128 && mb >= 6000 && nnzb >= 9 * mb;
+  const bool lone = T == 32 && feat % 128 == 32 && wide_units < 1300;
+  const int tiles = feat <= 32 ? 1 : feat > 64 && !halves && !lone ? 4 : 2;
+  const int64_t units = (mb + n_pieces) * stir::ceil_div(feat, 32 * tiles);
+  // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
+  // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
+  // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
+  const int waves = units >= (tiles == 4 ? 5000 : 8000) && (tiles > 1 || nnzb < 4 * mb) ? 2 : 4;
+  // One step on its way (of two) where more units at a time count for more than the loads of a wavefront behind its products; us
+  // with one / two:
+  //   8-row tiles: four wavefronts 0.98 to 1.02, and many units of two: 169 k rows, 1.9 M nonzeros, 192 features (42 k units) 100.5 /
+  //   104.1, 850 k 72.5 / 75.5; but 33 k, 200 k, 192 (8250) 25.7 / 24.6, 20 k, 80 k, 224 (5000) 20.3 / 18.6;
+  //   32-row tiles, four wavefronts, from three turns of 64 KB on: 75 k rows, 375 k nonzeros, 192 features 33.4 / 40.1, 60 k, 300 k,
+  //   skewed columns 27.7 / 33.3; less of them 20 k, 80 k, 128 (625 units) 16.1 / 15.8;
+  //   two wavefronts, a last unit at most half full and a step or two for each: 169 k rows, 850 k nonzeros of skewed columns, 192
+  //   features, 32 rows 85 / 91.7, 16-bit results 69.4 / 76.3, 16 rows (2.7 steps) 80.3 / 83.3, 16-bit 57.7 / 63.1; but of uniform
+  //   columns 81.9 / 84.3 and 68.4 / 65.7, and with more steps 1.01 to 1.04 of the time.
+  const bool part_empty = feat % 128 != 0 && feat % 128 <= 64;
+  const bool one_step = T == 8    ? waves == 4 || units >= 20000
+                        : T == 16 ? waves == 2 && part_empty && nnzb < (out32 ? 6 : 5) * mb
+                        : waves == 4 ? units >= 1300
+                                     : part_empty && nnzb < 10 * mb;
+  return {tiles, waves, tiles == 4 && one_step};
+}
+
 template <int T>
 int launch_planned(bool out32, int32_t mb, int32_t feat, int64_t nnzb, int64_t n_pieces, const TcPiece* d_pieces, float* d_scratch,
                    uint32_t* d_arrived, const uint16_t* A, const uint16_t* B, void* d_C, const int32_t* d_indptr,
                    const int32_t* d_indices, hipStream_t st) {
-  // Units of 128 features above 64 (tcspmm_direct_kernel), their last one however full; us with units of 64 features, by the
-  // kernel above, / of 128: 20 k rows, 300 k nonzeros, 128 features 16.2 / 14.4, 100 k, 500 k, 96 33.6 / 26.0, 120 k, 600 k, 160
-  // 61.2 / 53.7, 60 k, 900 k, 192 66.1 / 56.4 (skewed columns, 32 rows 54.3 / 55.7); and of 64 features alone 60 k, 900 k 25.7 /
-  // 29.5, 200 k, 4 M 66 / 80.
-  // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2
-  // steps 49.3 against 36.5 and 71.7 against 57.5 us; 3025 tiles of 2.7 steps 12.5 against 13.7, 3125 of 14.7
-  // 35.5 against 38.3 us; 32 features, 12.5 k tiles of 2.7 steps 25.3 against 27.6, 25 k of 1.5 31.6 against 28.1.
-  // Not where 32 features would have a unit of 128 and B is small enough to come mostly out of the L2s: 160 features, 30 k rows
-  // (9.7 MB) 27.3 / 28.3, 18 k 16.2 / 17.1, 36 k (11.7 MB) 26.3 / 26.8; but 52 k 52.3 / 47.2, 60 k 59.6 / 52.3.
-  const bool wide = feat > 64 && (feat % 128 != 32 || (int64_t)mb * T * feat * 2 > 13000000);
-  const int ntl = feat <= 32 ? 1 : wide ? 4 : 2;
-  const int f_tiles = (int)stir::ceil_div(feat, 32 * ntl);
+  const TcForm form = tc_form(T, out32, mb, feat, nnzb, n_pieces);
+  const int f_tiles = (int)stir::ceil_div(feat, 32 * form.tiles);
   const int64_t blocks = (mb + n_pieces) * f_tiles;
-  const bool pairs = blocks >= (wide ? 5000 : 8000) && (ntl > 1 || nnzb < 4 * (int64_t)mb);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "tc_spmm: too many tiles for one launch");
   const int aligned = reinterpret_cast<uintptr_t>(d_C) % (out32 ? 16 : 8) == 0;
-#define STIR_TC(NTL, W, OUT)                                                                                        \
-  hipLaunchKernelGGL((tcspmm_units_kernel<T, NTL, W, OUT>), dim3((unsigned)blocks), dim3(64 * W), 0, st, feat,       \
-                     (int64_t)mb, f_tiles, n_pieces, d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr,   \
-                     d_indices)
-#define STIR_TC_D(W, OUT)                                                                                           \
-  hipLaunchKernelGGL((tcspmm_direct_kernel<T, W, OUT>), dim3((unsigned)blocks), dim3(64 * W), 0, st, feat,            \
-                     (int64_t)mb, f_tiles, n_pieces, d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr,   \
-                     d_indices)
-#define STIR_TC_W(NTL, W) if (out32) STIR_TC(NTL, W, 1); else STIR_TC(NTL, W, 0);
-  if (pairs) {
-    if (ntl == 1) { STIR_TC_W(1, 2) } else if (ntl == 2) { STIR_TC_W(2, 2) } else if (out32) { STIR_TC_D(2, 1); } else { STIR_TC_D(2, 0); }
+#define STIR_TC_GO(KERNEL, W)                                                                                        \
+  hipLaunchKernelGGL(KERNEL, dim3((unsigned)blocks), dim3(64 * W), 0, st, feat, (int64_t)mb, f_tiles, n_pieces,      \
+                     d_pieces, A, B, d_C, aligned, d_scratch, d_arrived, d_indptr, d_indices)
+#define STIR_TC(NTL, W)                                                                                              \
+  do {                                                                                                               \
+    if (out32) STIR_TC_GO((tcspmm_units_kernel<T, NTL, W, 1>), W);                                                   \
+    else STIR_TC_GO((tcspmm_units_kernel<T, NTL, W, 0>), W);                                                         \
+  } while (0)
+#define STIR_TC_D(W, D)                                                                                              \
+  do {                                                                                                               \
+    if (out32) STIR_TC_GO((tcspmm_direct_kernel<T, W, 1, D>), W);                                                    \
+    else STIR_TC_GO((tcspmm_direct_kernel<T, W, 0, D>), W);                                                          \
+  } while (0)
+  if (form.tiles == 1) {
+    if (form.waves == 2) STIR_TC(1, 2); else STIR_TC(1, 4);
+  } else if (form.tiles == 2) {
+    if (form.waves == 2) STIR_TC(2, 2); else STIR_TC(2, 4);
+  } else if constexpr (T == 8) {
+    if (form.waves == 4) STIR_TC_D(4, 1);
+    else if (form.one_step) STIR_TC_D(2, 1);
+    else STIR_TC_D(2, 2);
+  } else if constexpr (T == 16) {
+    if (form.waves == 4) STIR_TC_D(4, 2);
+    else if (form.one_step) STIR_TC_D(2, 1);
+    else STIR_TC_D(2, 2);
   } else {
-    if (ntl == 1) { STIR_TC_W(1, 4) } else if (ntl == 2) { STIR_TC_W(2, 4) } else if (out32) { STIR_TC_D(4, 1); } else { STIR_TC_D(4, 0); }
+    if (form.waves == 4 && form.one_step) STIR_TC_D(4, 1);
+    else if (form.waves == 4) STIR_TC_D(4, 2);
+    else if (form.one_step) STIR_TC_D(2, 1);
+    else STIR_TC_D(2, 2);
   }
-#undef STIR_TC_W
 #undef STIR_TC_D
 #undef STIR_TC
+#undef STIR_TC_GO
   STIR_LAUNCH_CHECK();
   return 0;
 }
 
 }  // namespace
+
+// The form of a product with a plan of so many pieces: tiles of 32 features to a unit, 8 times the wavefronts, 64 for one
+// step on its way; -1 for what no product is.  For the tests, which say what they cover.
+extern "C" int stir_tc_form(int32_t tile_size, int32_t out_dtype, int32_t mb, int32_t feat, int64_t nnzb, int64_t n_pieces) {
+  if ((tile_size != 8 && tile_size != 16 && tile_size != 32) || (out_dtype != STIR_F16 && out_dtype != STIR_F32) || mb <= 0 ||
+      feat <= 0 || nnzb < 0 || n_pieces < 0)
+    return -1;
+  const TcForm f = tc_form(tile_size, out_dtype == STIR_F32, mb, feat, nnzb, n_pieces);
+  return f.tiles + 8 * f.waves + 64 * f.one_step;
+}
 
 extern "C" int stir_tc_spmm_f16(int32_t out_dtype, int32_t mb, int32_t tile_size, int32_t group_size,
                                 int32_t feat, int64_t nnzb, const void* d_A, const void* d_B, void* d_C,

@@ -257,3 +257,15 @@ def bsr_form(mb, nb, blk, feat, nnzb, cus=256):
     if kernel == "split":
         return kernel
     return kernel + (" 256" if code & 4 else " 128") + (" ranked" if code & 8 else "") + (" by rows" if code & 16 else "")
+
+
+def tc_form(t, out_dtype, mb, feat, nnzb, pieces=0):
+    """How a condensed product with a plan is launched: features to a unit, wavefronts to a unit, and whether one step of a
+    wavefront is on its way (of two)."""
+    import ctypes
+
+    from sparsetir_amd import _lib
+
+    code = _lib.lib().stir_tc_form(t, 2 if "32" in str(out_dtype) else 0, mb, feat, ctypes.c_int64(nnzb), ctypes.c_int64(pieces))
+    assert code > 0
+    return f"{32 * (code % 8)} by {code // 8 % 8}" + (", one step" if code & 64 else "")

@@ -6,12 +6,14 @@ import pytest
 import torch
 
 import sparsetir_amd as st
+from helpers import tc_form
 from sparsetir_amd import ops
+from test_gpu_tcspmm import _run
 
 pytestmark = pytest.mark.gpu
 
 
-def _odd_groups(dev, t, feat, out_dtype, start, empty=0):
+def _odd_groups(dev, t, feat, out_dtype, start, empty=0, form=None):
     rng = np.random.default_rng(feat + t)
     n, counts = 900, [16, 48, 80, 32, 144, 0, 688] + [0] * empty  # columns of a tile: 1, 3, 5, 2, 9, 0 and 43 groups
     cols = [np.sort(rng.choice(np.arange(1, n), c, replace=False)) for c in counts]
@@ -19,6 +21,8 @@ def _odd_groups(dev, t, feat, out_dtype, start, empty=0):
     indptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
     gptr, tiles, mask = st.condense(indptr, np.concatenate(rows).astype(np.int32), t, 16)
     mb = len(gptr) - 1
+    # no tile is long: the longest has 43 groups, 22 steps
+    assert form is None or tc_form(t, out_dtype, mb, feat, tiles.shape[0]) == form
     a = (mask * rng.uniform(0.1, 1.0, mask.shape)).astype(np.float16)
     b = rng.standard_normal((n, feat)).astype(np.float16)
     named = int(cols[1][-1])  # in the last group of the second tile
@@ -61,5 +65,44 @@ def test_odd_groups(dev, t, feat, out_dtype, start):
 @pytest.mark.parametrize("feat", [160, 288])
 @pytest.mark.parametrize("out_dtype", [torch.float16, torch.float32])
 def test_a_unit_of_32_features(dev, t, feat, out_dtype):
-    """32 features have a unit of 128 to themselves only where B is taken to be large, as large as C: many rows, most of them empty."""
+    """32 features with a unit of 128 to themselves, in a launch of many units."""
     _odd_groups(dev, t, feat, out_dtype, 1, 13_000_000 // (2 * feat * t) + 1)
+
+
+# the forms of launches of many units, by empty tiles: two wavefronts to a unit, one step of a wavefront on its way
+@pytest.mark.parametrize("t,feat,out_dtype,empty,form", [
+    (8, 192, torch.float16, 2600, "128 by 2"),
+    (8, 192, torch.float32, 2600, "128 by 2"),
+    (8, 224, torch.float16, 10000, "128 by 2, one step"),
+    (8, 224, torch.float32, 10000, "128 by 2, one step"),
+    (16, 192, torch.float16, 2600, "128 by 2, one step"),
+    (16, 224, torch.float16, 2600, "128 by 2"),
+    (16, 192, torch.float32, 2600, "128 by 2, one step"),
+    (16, 256, torch.float32, 2600, "128 by 2"),
+    (32, 96, torch.float16, 1300, "128 by 4, one step"),
+    (32, 160, torch.float32, 650, "128 by 4, one step"),
+    (32, 160, torch.float32, 600, "64 by 4"),
+    (32, 192, torch.float16, 2600, "128 by 2, one step"),
+    (32, 192, torch.float32, 2600, "128 by 2, one step"),
+    (32, 256, torch.float16, 2600, "128 by 2"),
+])
+def test_forms(dev, t, feat, out_dtype, empty, form):
+    _odd_groups(dev, t, feat, out_dtype, 1, empty, form)
+
+
+@pytest.mark.parametrize("t,feat,tiles,deg,out_dtype,form", [
+    (8, 128, 6000, 18, torch.float16, "64 by 2"),             # two units of 64 to a tile of several steps
+    (32, 96, 1400, 1, torch.float32, "128 by 4, one step"),   # with tiles that are cut into pieces
+    (32, 192, 2600, 1, torch.float16, "128 by 2, one step"),
+])
+def test_forms_of_whole_graphs(dev, t, feat, tiles, deg, out_dtype, form):
+    rng = np.random.default_rng(tiles)
+    counts = np.full(tiles * t, deg)
+    if deg == 1:
+        counts[[t + 1, 5 * t]] = 1500
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    n = 12000
+    indices = ((np.arange(indptr[-1]) * 7 + rng.integers(0, 7, indptr[-1])) % n).astype(np.int32)  # distinct in a row
+    gptr = st.condense(indptr, indices, t, 16)[0]
+    assert tc_form(t, out_dtype, tiles, feat, int(gptr[-1])) == form
+    _run(dev, indptr, indices, n, feat, False, out_dtype, t=t)

@@ -8,35 +8,35 @@ from helpers import bsr_form
 
 @pytest.mark.parametrize("mb,nb,blk,steps,feat,form", [
     # 32-row slices: order of length by the steps, the X of a tile and how many wavefronts there are
-    (2048, 512, 32, 10, 1024, "waves 128"),
-    (2048, 512, 32, 16, 1024, "waves 256 ranked"),
-    (2048, 512, 32, 16, 256, "waves 128"),           # one feature tile
-    (2048, 512, 32, 32, 256, "waves 256 ranked"),
-    (2048, 207, 32, 16, 1024, "waves 256"),          # X in an L2
-    (2048, 207, 32, 32, 1024, "waves 256 ranked"),
-    (250, 512, 32, 16, 1024, "waves 128"),           # few
-    (2048, 512, 32, 16, 544, "waves 128"),           # a last tile mostly empty
-    (512, 512, 32, 51, 4096, "waves 256 ranked"),
-    (400, 170, 96, 6, 512, "groups 128"),
-    (400, 170, 96, 16, 512, "waves 256 ranked"),
-    (1300, 325, 96, 8, 1504, "groups 256"),
+    (2048, 512, 32, 10, 1024, "128 by 1"),
+    (2048, 512, 32, 16, 1024, "256 by 1 ranked"),
+    (2048, 512, 32, 16, 256, "128 by 1"),           # one feature tile
+    (2048, 512, 32, 32, 256, "256 by 1 ranked"),
+    (2048, 207, 32, 16, 1024, "256 by 1"),          # X in an L2
+    (2048, 207, 32, 32, 1024, "256 by 1 ranked"),
+    (250, 512, 32, 16, 1024, "128 by 1"),           # few
+    (2048, 512, 32, 16, 544, "128 by 1"),           # a last tile mostly empty
+    (512, 512, 32, 51, 4096, "256 by 1 ranked"),
+    (400, 170, 96, 6, 512, "LDS 32 x 128"),
+    (400, 170, 96, 16, 512, "256 by 1 ranked"),
+    (1300, 325, 96, 8, 1504, "LDS 32 x 256"),
     # 64 rows by four wavefronts
-    (1024, 256, 64, 12, 1024, "groups 256"),
-    (1024, 256, 64, 24, 1024, "groups 256 ranked"),
-    (256, 256, 64, 16, 256, "groups 128"),
-    (128, 128, 128, 51, 4096, "groups 256 ranked by rows"),
-    (12, 40, 128, 30, 3008, "groups 128"),
-    (45, 45, 128, 20, 1024, "groups 128 by rows"),
+    (1024, 256, 64, 12, 1024, "LDS 64 x 256"),
+    (1024, 256, 64, 24, 1024, "LDS 64 x 256 ranked"),
+    (256, 256, 64, 16, 256, "LDS 64 x 128"),
+    (128, 128, 128, 51, 4096, "LDS 64 x 256 ranked by rows"),
+    (12, 40, 128, 30, 3008, "LDS 64 x 128"),
+    (45, 45, 128, 20, 1024, "LDS 64 x 128 by rows"),
     # 16-row slices
-    (4096, 1025, 16, 10, 1024, "waves 128"),
-    (4096, 1025, 16, 18, 1024, "waves 256 ranked"),
-    (1024, 420, 16, 10, 512, "waves 256"),
-    (1100, 341, 48, 10, 1024, "waves 256"),
-    (600, 650, 48, 7, 256, "groups 256"),
-    (3693, 559, 48, 11, 320, "waves 128"),
-    (1214, 659, 80, 10, 416, "groups 256"),
-    (3000, 68, 80, 8, 800, "waves 128"),
-    (3000, 68, 80, 20, 800, "waves 256"),            # A beyond the last level
+    (4096, 1025, 16, 10, 1024, "128 by 1"),
+    (4096, 1025, 16, 18, 1024, "256 by 1 ranked"),
+    (1024, 420, 16, 10, 512, "256 by 1"),
+    (1100, 341, 48, 10, 1024, "256 by 4"),
+    (600, 650, 48, 7, 256, "128 by 2, two tiles"),
+    (3693, 559, 48, 11, 320, "128 by 1"),
+    (1214, 659, 80, 10, 416, "128 by 2, two tiles"),
+    (3000, 68, 80, 8, 800, "128 by 1"),
+    (3000, 68, 80, 20, 800, "256 by 4"),            # A beyond the last level
 ])
 def test_form(mb, nb, blk, steps, feat, form):
     nnzb = -(-steps * mb * 32 // blk)
@@ -44,10 +44,12 @@ def test_form(mb, nb, blk, steps, feat, form):
 
 
 def test_sizes_whose_offsets_do_not_fit():
-    """No wavefront form where a load's offset may not fit 32 bits."""
-    assert bsr_form(4, 4, 32, 1 << 25, 16).startswith("groups")
-    assert bsr_form(64, 4, 4096 + 32, 4096, 64).startswith("groups")
-    assert bsr_form(64, 4, 4096 + 16, 4096, 64).startswith("groups")
+    """Where a load's offset from the wavefront's first may not fit 32 bits: kernels that allow for more."""
+    assert bsr_form(4, 4, 32, 1 << 25, 16) == "LDS 32 x 256"
+    assert bsr_form(64, 4, 4096 + 32, 4096, 64) == "LDS 32 x 256"
+    assert bsr_form(64, 4, 4096 + 16, 4096, 64) == "128 by 2, two tiles"
+    assert bsr_form(64, 4, 32768 + 16, 4096, 64) == "LDS 64 by 8"
+    assert bsr_form(4, 4, 16, 1 << 27, 16) == "LDS 64 by 8"
 
 
 @pytest.mark.parametrize("mb,nb,blk,feat,nnzb,cus", [(0, 4, 32, 64, 0, 256), (4, 4, 24, 64, 4, 256), (4, 4, 32, 0, 4, 256),

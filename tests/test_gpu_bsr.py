@@ -75,8 +75,7 @@ def test_bsr_block64_and_empty_rows(dev):
     (256, 384, torch.bfloat16, True),    # four slices of 64 rows per block row, a partial last feature tile
 ])
 def test_bsr_tall_blocks(dev, blk, feat, dtype, out32):
-    """Blocks of 64 rows and more, few of them: 32-row slices by eight wavefronts each, or by four at 13 block rows and
-    1280 features."""
+    """Blocks of 64 rows and more, few of them: 32-row slices whose steps several wavefronts take in turn."""
     cfg = datasets.config4(seed=blk, mb=13 if blk >= 128 else 5, nb=6, blk=blk, density=0.35, feat=feat)
     got, a32, x32 = _run(dev, cfg, dtype, torch.float32 if out32 else None)
     _check(got, cfg, a32, x32, not out32, f"blk={blk} feat={feat} {dtype}")
@@ -90,8 +89,7 @@ def test_bsr_tall_blocks(dev, blk, feat, dtype, out32):
     (10, 4, 256, 1024, torch.bfloat16),   # 256-row blocks
 ])
 def test_bsr_many_workgroups(dev, mb, nb, blk, feat, dtype):
-    """More than two workgroups per CU: the kernel whose wavefronts split the feature axis (small
-    launches take the one whose wavefronts split the steps of a block row)."""
+    """More than 512 tiles of 32 x 128: two to a compute unit."""
     cfg = datasets.config4(seed=mb, mb=mb, nb=nb, blk=blk, density=0.3, feat=feat)
     assert mb * (blk // 32) * ((feat + 127) // 128) > 512
     got, a32, x32 = _run(dev, cfg, dtype)
@@ -99,10 +97,10 @@ def test_bsr_many_workgroups(dev, mb, nb, blk, feat, dtype):
 
 
 @pytest.mark.parametrize("dtype,out32,varied,mb,nb,form", [
-    (torch.float16, False, False, 1100, 208, "waves 256"),         # as they come
-    (torch.float16, False, False, 1100, 400, "waves 256 ranked"),
-    (torch.bfloat16, True, True, 1100, 1300, "waves 256 ranked"),
-    (torch.float16, True, True, 1000, 1300, "waves 256 ranked"),
+    (torch.float16, False, False, 1100, 208, "256 by 1"),         # as they come
+    (torch.float16, False, False, 1100, 400, "256 by 1 ranked"),
+    (torch.bfloat16, True, True, 1100, 1300, "256 by 1 ranked"),
+    (torch.float16, True, True, 1000, 1300, "256 by 1 ranked"),
 ])
 def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb, nb, form):
     """Large launches whose block rows are taken in order of their length, found by every wavefront on its own: 1000 rows

@@ -11,20 +11,21 @@ from sparsetir_amd import datasets, ops
 pytestmark = pytest.mark.gpu
 
 SHAPES = [
-    (1024, 60, 16, 0.1, 224, "waves 128"),     # 16-row slices by a wavefront each
-    (1024, 400, 16, 0.01, 512, "waves 256"),
-    (230, 50, 48, 0.05, 352, "waves 128"),     # three chunks a block
-    (230, 140, 48, 0.03, 1024, "waves 256"),
-    (150, 40, 16, 0.2, 1184, "groups 256"),    # by four wavefronts
-    (61, 23, 80, 0.3, 480, "groups 256"),
-    (3, 200, 16, 0.5, 64, "split"),            # by eight
-    (9, 90, 32, 0.6, 96, "split"),
-    (343, 200, 32, 0.01, 736, "waves 128"),    # 32-row slices by a wavefront each
-    (520, 200, 32, 0.01, 800, "waves 128"),
-    (650, 200, 32, 0.005, 512, "waves 256"),
-    (397, 30, 32, 0.2, 416, "groups 128"),     # by four
-    (147, 13, 64, 0.3, 2400, "groups 256"),
-    (14, 100, 128, 0.05, 160, "split"),
+    (1024, 60, 16, 0.1, 224, "128 by 1"),     # 16-row slices by a wavefront each
+    (1024, 400, 16, 0.01, 512, "256 by 1"),
+    (230, 50, 48, 0.05, 352, "128 by 1"),     # three chunks a block
+    (230, 140, 48, 0.03, 1024, "256 by 1"),
+    (150, 40, 16, 0.2, 1184, "128 by 2, two tiles"),
+    (61, 23, 80, 0.3, 480, "128 by 2, two tiles"),
+    (3, 200, 16, 0.5, 64, "128 by 8"),
+    (260, 60, 16, 0.75, 64, "LDS 64 by 8"),   # 64 features by eight, through LDS
+    (9, 90, 32, 0.6, 96, "LDS 64 by 8"),
+    (343, 200, 32, 0.01, 736, "128 by 1"),    # 32-row slices by a wavefront each
+    (520, 200, 32, 0.01, 800, "128 by 1"),
+    (650, 200, 32, 0.005, 512, "256 by 1"),
+    (397, 30, 32, 0.2, 416, "128 by 1, four tiles"),
+    (147, 13, 64, 0.3, 2400, "LDS 64 x 256"),  # 64 rows by four wavefronts
+    (14, 100, 128, 0.05, 160, "128 by 4"),
 ]
 
 

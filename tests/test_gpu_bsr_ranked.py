@@ -37,14 +37,14 @@ def _config(mb, nb, blk, density, feat, seed):
     (70, 70, 96, 0.04, 1440),      # three slices per block row, 5.6 feature tiles
     (257, 250, 32, 0.01, 832),
     (343, 200, 32, 0.01, 736),
-    (20, 200, 64, 0.03, 96),       # by eight wavefronts
+    (20, 200, 64, 0.03, 96),       # steps in turn by eight, four and two wavefronts
     (12, 100, 128, 0.05, 160),
     (14, 100, 128, 0.05, 160),
-    (60, 200, 64, 0.03, 416),      # four wavefronts per 64 rows
-    (33, 100, 128, 0.05, 544),     # too few block rows to deal them to XCDs
-    (36, 100, 128, 0.05, 544),     # block rows dealt to XCDs
-    (40, 20, 64, 0.1, 1056),       # few workgroups: 128 features each
-    (83, 20, 64, 0.1, 1056),       # as many as take 256 features each, the last with 32
+    (60, 200, 64, 0.03, 416),
+    (33, 100, 128, 0.05, 544),
+    (36, 100, 128, 0.05, 544),
+    (40, 20, 64, 0.1, 1056),
+    (83, 20, 64, 0.1, 1056),       # 64 rows by four wavefronts, 256 features each, the last with 32
     (1, 6200, 32, 0.001, 64),
     (1030, 90, 16, 0.02, 224),     # 16-row slices by a wavefront each: plain order
     (1024, 400, 16, 0.004, 512),   # 256 features
@@ -81,35 +81,35 @@ def _cus():
 
 
 @pytest.mark.parametrize("mb,nb,blk,density,feat,form", [
-    (430, 200, 32, 0.004, 288, "waves 128"),
-    (650, 200, 32, 0.005, 512, "waves 256"),
-    (83, 20, 64, 0.1, 1056, "groups 256"),
-    (1030, 90, 16, 0.02, 224, "waves 128"),
-    (1024, 400, 16, 0.004, 512, "waves 256"),
+    (430, 200, 32, 0.004, 288, "128 by 1"),
+    (650, 200, 32, 0.005, 512, "256 by 1"),
+    (83, 20, 64, 0.1, 1056, "LDS 64 x 256"),
+    (1030, 90, 16, 0.02, 224, "128 by 1"),
+    (1024, 400, 16, 0.004, 512, "256 by 1"),
     # 32-row slices by a wavefront each, in order of their length: the last of six feature tiles with 32
-    (257, 250, 32, 0.07, 1312, "waves 256 ranked"),
-    (1024, 250, 32, 0.07, 512, "waves 256 ranked"),    # as many block rows as a wavefront ranks
-    (1025, 250, 32, 0.07, 448, "waves 256 ranked"),    # two groups, of 513 and 512
-    (2051, 200, 32, 0.15, 256, "waves 256 ranked"),    # three, one feature tile for all XCDs, X in an L2 but long rows
-    (72, 90, 96, 0.07, 1440, "waves 256 ranked"),      # six tiles over eight XCDs: the slices of a block row on one of them
-    (40, 60, 160, 0.07, 1760, "waves 256 ranked"),
-    (220, 100, 96, 0.02, 1024, "waves 256"),
+    (257, 250, 32, 0.07, 1312, "256 by 1 ranked"),
+    (1024, 250, 32, 0.07, 512, "256 by 1 ranked"),    # as many block rows as a wavefront ranks
+    (1025, 250, 32, 0.07, 448, "256 by 1 ranked"),    # two groups, of 513 and 512
+    (2051, 200, 32, 0.15, 256, "256 by 1 ranked"),    # three, one feature tile for all XCDs, X in an L2 but long rows
+    (72, 90, 96, 0.07, 1440, "256 by 1 ranked"),      # six tiles over eight XCDs: the slices of a block row on one of them
+    (40, 60, 160, 0.07, 1760, "256 by 1 ranked"),
+    (220, 100, 96, 0.02, 1024, "256 by 1"),
     # 64 rows by four wavefronts
-    (200, 250, 64, 0.05, 416, "groups 128 ranked"),
-    (100, 130, 64, 0.08, 2048, "groups 256 ranked"),
-    (1030, 100, 64, 0.15, 256, "groups 128 ranked"),
-    (33, 100, 128, 0.06, 3072, "groups 256 ranked"),   # too few block rows to deal them to XCDs
-    (44, 100, 128, 0.06, 2304, "groups 256 ranked by rows"),
-    (16, 60, 128, 0.05, 2080, "groups 128 by rows"),
-    (16, 30, 192, 0.1, 1056, "groups 128 by rows"),
+    (200, 250, 64, 0.05, 416, "LDS 64 x 128 ranked"),
+    (100, 130, 64, 0.08, 2048, "LDS 64 x 256 ranked"),
+    (1030, 100, 64, 0.15, 256, "LDS 64 x 128 ranked"),
+    (33, 100, 128, 0.06, 3072, "LDS 64 x 256 ranked"),   # too few block rows to deal them to XCDs
+    (44, 100, 128, 0.06, 2304, "LDS 64 x 256 ranked by rows"),
+    (16, 60, 128, 0.05, 2080, "LDS 64 x 128 by rows"),
+    (16, 30, 192, 0.1, 1056, "LDS 64 x 128 by rows"),
     # 16-row slices
-    (1030, 490, 16, 0.07, 512, "waves 256 ranked"),
-    (430, 1000, 16, 0.04, 672, "waves 128 ranked"),
-    (171, 170, 48, 0.07, 1024, "waves 256 ranked"),
-    (200, 330, 48, 0.05, 608, "waves 128 ranked"),
-    (230, 140, 48, 0.03, 1024, "waves 256"),
-    (110, 40, 80, 0.2, 1024, "waves 256"),             # little X, long rows
-    (400, 140, 48, 0.03, 288, "groups 256"),           # wavefronts of 128 features would be few
+    (1030, 490, 16, 0.07, 512, "256 by 1 ranked"),
+    (430, 1000, 16, 0.04, 672, "128 by 1 ranked"),
+    (171, 170, 48, 0.07, 1024, "256 by 1 ranked"),
+    (200, 330, 48, 0.05, 608, "128 by 1 ranked"),
+    (230, 140, 48, 0.03, 1024, "256 by 1"),
+    (110, 40, 80, 0.2, 1024, "256 by 1"),             # little X, long rows
+    (400, 140, 48, 0.03, 288, "128 by 2, two tiles"),           # wavefronts of 128 features would be few
 ])
 def test_bsr_forms(dev, mb, nb, blk, density, feat, form):
     """Every form of a launch, with long and empty block rows and columns in any order, against the same sums in fp64 by

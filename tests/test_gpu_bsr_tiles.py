@@ -1,4 +1,4 @@
-"""BSR SpMM at the edges of its launch rules: few workgroups (block rows dealt to the wavefronts of a
+"""BSR SpMM at the edges of its launch rules: few workgroups (steps of a block row taken in turn by the wavefronts of a
 workgroup, more than 64 blocks in a row, rows with fewer steps than wavefronts and empty ones), blocks of an odd
 multiple of 16 with an odd number of column chunks, and feature-tile counts that are not multiples of the
 eight XCDs.  Checked against the fp64 oracle as in test_gpu_bsr.py."""

@@ -19,6 +19,7 @@
 
 namespace {
 
+using stir::Halves8;
 using stir::kWave;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -196,7 +197,7 @@ __device__ __forceinline__ void store_rows(char* __restrict__ own, const f32x16 
       const int at = kWave * q + lane, row = at / UN, u = at % UN;
       const u32x4 w = *reinterpret_cast<const u32x4*>(own + at * 16);
       if (f0 + 8 * u < feat)
-        __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row0 + row) * feat + f0 +
+        __builtin_nontemporal_store(Halves8(w), reinterpret_cast<Halves8*>(static_cast<uint16_t*>(Y) + (row0 + row) * feat + f0 +
                                                                 8 * u));
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -446,7 +447,7 @@ __device__ __forceinline__ void store_rows8(void* __restrict__ Y, int64_t row, i
 #pragma unroll
     for (int t = 0; t < 4; ++t) w[t] = to16<BF16>(v[2 * t]) | (uint32_t)to16<BF16>(v[2 * t + 1]) << 16;
     if (f0 + 8 * n < feat)
-      __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + (row + 4 * h) * feat + f0 + 8 * n));
+      __builtin_nontemporal_store(Halves8(w), reinterpret_cast<Halves8*>(static_cast<uint16_t*>(Y) + (row + 4 * h) * feat + f0 + 8 * n));
   }
 }
 
@@ -1077,13 +1078,13 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, in
     if constexpr (ROWS == 32) {
       const int b = it / ksteps, k0 = (it - b * ksteps) * kTileK;
       const uint16_t* ab = A + (int64_t)(p_begin + b) * blk * blk + (int64_t)(bi0 + n) * blk + k0 + 8 * h;
-      ar[0] = *reinterpret_cast<const u32x4*>(ab);
-      ar[1] = *reinterpret_cast<const u32x4*>(ab + 16);
+      ar[0] = *reinterpret_cast<const Halves8*>(ab);
+      ar[1] = *reinterpret_cast<const Halves8*>(ab + 16);
       const uint16_t* xb = X + (column(b) * blk + k0) * feat + f0 + xoff;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         xr[u] = u32x4{0, 0, 0, 0};
-        if (xlive) xr[u] = *reinterpret_cast<const u32x4*>(xb + (int64_t)(8 * u) * feat);
+        if (xlive) xr[u] = *reinterpret_cast<const Halves8*>(xb + (int64_t)(8 * u) * feat);
       }
     } else {
       const int c0 = 2 * it, b0 = c0 / sub, b1 = (c0 + 1) / sub;
@@ -1091,7 +1092,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, in
       const int ba = h >> 1 ? b1 : b0, ca = c0 + (h >> 1) - ba * sub;
       ar[0] = u32x4{0, 0, 0, 0};
       if (h < 2 || two)
-        ar[0] = *reinterpret_cast<const u32x4*>(A + (int64_t)(p_begin + ba) * blk * blk + (int64_t)(bi0 + n) * blk +
+        ar[0] = *reinterpret_cast<const Halves8*>(A + (int64_t)(p_begin + ba) * blk * blk + (int64_t)(bi0 + n) * blk +
                                                 16 * ca + 8 * (h & 1));
       const uint16_t* x0 = X + (column(b0) * blk + 16 * (c0 - b0 * sub)) * feat + f0 + xoff;
       const uint16_t* x1 = X + (column(two ? b1 : b0) * blk + 16 * (two ? c0 + 1 - b1 * sub : 0)) * feat + f0 + xoff;
@@ -1099,7 +1100,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void bsr_split_kernel(int blk, in
       for (int u = 0; u < 4; ++u) {
         xr[u] = u32x4{0, 0, 0, 0};
         if (xlive && (u < 2 || two))
-          xr[u] = *reinterpret_cast<const u32x4*>((u < 2 ? x0 : x1) + (int64_t)(8 * (u & 1)) * feat);
+          xr[u] = *reinterpret_cast<const Halves8*>((u < 2 ? x0 : x1) + (int64_t)(8 * (u & 1)) * feat);
       }
     }
   };

@@ -5,6 +5,9 @@
 namespace stir {
 
 typedef uint32_t Words4 __attribute__((ext_vector_type(4)));
+// Eight 16-bit values in a caller's array, which may start at any element of an allocation: loads and stores of 16 bytes take any
+// address, but nothing may be made of an alignment that is not there.
+typedef uint32_t Halves8 __attribute__((ext_vector_type(4), aligned(2)));
 
 // Lane (c, g) of a wavefront holds 8 features from each of 8 rows (k), 16 bytes a row in x[0 .. 7].  Word w of the rows 2 d and
 // 2 d + 1 holds the features 2 w and 2 w + 1 of both; one v_perm makes word d of the B operand of either, whose column is c.

@@ -44,8 +44,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+using stir::Halves8;
 // as stored at any element of C
-typedef uint32_t Half8 __attribute__((ext_vector_type(4), aligned(2)));
 typedef float Float4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kTileF = 128;
@@ -102,12 +102,12 @@ __device__ __forceinline__ void tc_load_a(u32x4 (&a)[2], const uint16_t* __restr
   a[0] = a[1] = u32x4{0, 0, 0, 0};
   if constexpr (T == 32) {
     const int n = lane & 31, h = lane >> 5;
-    a[0] = *reinterpret_cast<const u32x4*>(A + (jo * 32 + n) * kGroup + 8 * h);
-    if (jo + 1 < g_end) a[1] = *reinterpret_cast<const u32x4*>(A + ((jo + 1) * 32 + n) * kGroup + 8 * h);
+    a[0] = *reinterpret_cast<const Halves8*>(A + (jo * 32 + n) * kGroup + 8 * h);
+    if (jo + 1 < g_end) a[1] = *reinterpret_cast<const Halves8*>(A + ((jo + 1) * 32 + n) * kGroup + 8 * h);
   } else {
     const int i = lane & 15, q = lane >> 4;
     const int64_t grp = jo + (q >> 1);
-    if (i < T && grp < g_end) a[0] = *reinterpret_cast<const u32x4*>(A + (grp * T + i) * kGroup + 8 * (q & 1));
+    if (i < T && grp < g_end) a[0] = *reinterpret_cast<const Halves8*>(A + (grp * T + i) * kGroup + 8 * (q & 1));
   }
 }
 
@@ -223,8 +223,8 @@ __global__ __launch_bounds__(256) void tcspmm_kernel(int feat, int64_t mb, int f
     r0 = r1 = u32x4{0, 0, 0, 0};
     const int64_t k = (int64_t)it * 32 + 2 * kp;
     if (stage_live && k < rows_total) {
-      r0 = *reinterpret_cast<const u32x4*>(B + (int64_t)row_a * feat + f0 + fc * 8);
-      r1 = *reinterpret_cast<const u32x4*>(B + (int64_t)row_b * feat + f0 + fc * 8);
+      r0 = *reinterpret_cast<const Halves8*>(B + (int64_t)row_a * feat + f0 + fc * 8);
+      r1 = *reinterpret_cast<const Halves8*>(B + (int64_t)row_b * feat + f0 + fc * 8);
     }
     if (it + 1 < it_end) fetch_ids(it + 1);
   };
@@ -323,8 +323,8 @@ __device__ __forceinline__ void tcspmm_long_steps(uint32_t* __restrict__ lds, in
       r0[q] = r1[q] = u32x4{0, 0, 0, 0};
       const int64_t k = (int64_t)it * 32 + 2 * (kp + KP * q);
       if (stage_live && k < rows_total) {
-        r0[q] = *reinterpret_cast<const u32x4*>(B + (int64_t)row_a[q] * feat + f0 + fc * 8);
-        r1[q] = *reinterpret_cast<const u32x4*>(B + (int64_t)row_b[q] * feat + f0 + fc * 8);
+        r0[q] = *reinterpret_cast<const Halves8*>(B + (int64_t)row_a[q] * feat + f0 + fc * 8);
+        r1[q] = *reinterpret_cast<const Halves8*>(B + (int64_t)row_b[q] * feat + f0 + fc * 8);
       }
     }
     if (it + WAVES < s_end) fetch_ids(it + WAVES);
@@ -622,7 +622,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
     for (int u = 0; u < LOADS; ++u) {
       const int row = __shfl(id, k0 + u * (64 / FCN), 64);
       x[u] = u32x4{0, 0, 0, 0};
-      if (live && row >= 0) x[u] = *reinterpret_cast<const u32x4*>(B + (int64_t)row * feat + f0 + 8 * c);
+      if (live && row >= 0) x[u] = *reinterpret_cast<const Halves8*>(B + (int64_t)row * feat + f0 + 8 * c);
     }
     if (it + W < s_end) fetch_ids(it + W);
   };
@@ -752,10 +752,10 @@ __global__ __launch_bounds__(64 * W, T == 8 ? 4 : (T == 32 ? 2 : 3) + (D == 1)) 
     for (int r = 0; r < RH; ++r) {
       a[s][r] = u32x4{0, 0, 0, 0};  // rows T ... 15 of the operand
       if (T >= 16 || c < T)
-        a[s][r] = *reinterpret_cast<const u32x4*>(A + ((g_begin + group_of(step)) * T + 16 * r + c) * kGroup + 8 * (g & 1));
+        a[s][r] = *reinterpret_cast<const Halves8*>(A + ((g_begin + group_of(step)) * T + 16 * r + c) * kGroup + 8 * (g & 1));
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) x[s][q] = *reinterpret_cast<const u32x4*>(Bf + (int64_t)ids[q / 4][q % 4] * feat);
+    for (int q = 0; q < 8; ++q) x[s][q] = *reinterpret_cast<const Halves8*>(Bf + (int64_t)ids[q / 4][q % 4] * feat);
   };
   auto multiply = [&](int s, int step) {
     if (2 * step + 1 >= groups) {
@@ -863,7 +863,7 @@ __global__ __launch_bounds__(64 * W, T == 8 ? 4 : (T == 32 ? 2 : 3) + (D == 1)) 
           w[t] = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2)]) |
                  (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)o[t / 2][2 * (t % 2) + 1]) << 16;
         if (f0 + 8 * c < feat && (T >= 16 || row < T))
-          *reinterpret_cast<Half8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
+          *reinterpret_cast<Halves8*>(static_cast<uint16_t*>(C) + (io * T + row) * feat + f0 + 8 * c) = w;
         continue;
       }
 #pragma unroll

@@ -12,7 +12,7 @@ from test_gpu_bsr import _check
 pytestmark = pytest.mark.gpu
 
 
-def _edges(dev, mb, nb, blk, feat, at_most, form, dtype):
+def _edges(dev, mb, nb, blk, feat, at_most, form, dtype, out_start=None):
     rng = np.random.default_rng(mb + feat)
     cfg = datasets.config4(seed=mb, mb=mb, nb=nb, blk=blk, density=0.0, feat=feat)
     counts = rng.integers(at_most // 2, at_most + 1, mb)
@@ -25,7 +25,7 @@ def _edges(dev, mb, nb, blk, feat, at_most, form, dtype):
     cfg["data"] = rng.standard_normal((nnzb, blk, blk)).astype(np.float32) * 0.1
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert bsr_form(mb, nb, blk, feat, nnzb, cus) == form
-    out, start = (torch.float32, 1) if (mb & 1) == (dtype is torch.float16) else (dtype, 0)
+    out, start = out_start or ((torch.float32, 1) if (mb & 1) == (dtype is torch.float16) else (dtype, 0))
 
     def place(values):
         t = torch.empty(values.size + start, dtype=dtype, device=dev)[start:]
@@ -95,3 +95,20 @@ def test_direct16_edges(dev, mb, nb, blk, feat, at_most, form, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_lds_split_edges(dev, mb, nb, blk, feat, at_most, form, dtype):
     _edges(dev, mb, nb, blk, feat, at_most, form, dtype)
+
+
+# results of 16 bits leave 16 bytes at a time, wherever the array starts
+@pytest.mark.parametrize("mb,nb,blk,feat,at_most,form", [
+    (150, 25, 32, 352, 12, "128 by 4"),
+    (70, 200, 32, 2336, 30, "128 by 1, one step"),
+    (301, 17, 32, 608, 9, "256 by 1"),
+    (64, 30, 80, 160, 9, "128 by 4"),
+    (640, 25, 16, 608, 17, "128 by 2, two tiles"),
+    (1050, 20, 16, 480, 16, "256 by 1"),
+    (230, 140, 48, 992, 12, "256 by 4"),
+    (260, 90, 16, 64, 85, "LDS 64 by 8"),
+    (147, 13, 64, 2400, 8, "LDS 64 x 256"),
+])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_sixteen_bit_results_at_an_odd_element(dev, mb, nb, blk, feat, at_most, form, dtype):
+    _edges(dev, mb, nb, blk, feat, at_most, form, dtype, (dtype, 1))

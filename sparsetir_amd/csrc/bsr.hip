@@ -485,34 +485,25 @@ __device__ __forceinline__ void add_up8(const f32x4* part, int stride, int used,
 }
 
 // A tile of 32 rows x 128 features, 16 accumulators of v_mfma_f32_16x16x32, a step of 32 k in eight loads of X and two of A.
-// W wavefronts take the steps of a block row in turn and meet in LDS at the end (W = 1: none does).  GROUP: W = 1, and a
-// workgroup is four wavefronts with neighbouring tiles of one slice, which find each other's A in L1.
+// W wavefronts take the steps of a block row in turn and meet in LDS at the end (W = 1: none does).
 // D steps are on their way; nothing is asked for beyond the last one: a load outside its window costs as much as another
 // (128 x 128 blocks of 32, 512 features, four wavefronts 9.8 -> 9.1 us).
 // Against four wavefronts that shared 128 features through LDS and met at a barrier per step, us as part of a graph:
 // 128 x 128 blocks of 32, 10 %, 512 features 11.1 -> 9.1 (W = 4); 256 x 256, 512 features 24.0 -> 20.1 (W = 1); 209 x 46, 2
-// steps a row, 1216 features 9.3 -> 7.8 (W = 1); 451 x 87, 160 features 11.5 -> 9.4 (GROUP); against eight wavefronts with 64
+// steps a row, 1216 features 9.3 -> 7.8 (W = 1); against eight wavefronts with 64
 // features through LDS: 197 x 193, 37 steps, 224 features 23.0 -> 16.3 (W = 4), 131 x 322, 78 steps, 128 features 18.7 ->
 // 14.9 (W = 8).  Small launches are bound by the trips to memory one after the other -- indptr, block columns, rows of X,
 // 2.8 us with the launch -- and then by X and A coming through the L2s, which hold neither (config above: 22 MB, 2.7 us).
-template <bool BF16, int OUT, int W, bool GROUP, int D = 2>
-__global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, D == 1 ? 4 : W == 1 ? 3 : 2) void bsr_direct_kernel(
+template <bool BF16, int OUT, int W, int D = 2>
+__global__ __launch_bounds__(W * kWave, D == 1 ? 4 : W == 1 ? 3 : 2) void bsr_direct_kernel(
     int blk, int feat, int64_t slices, int f_tiles, const uint16_t* __restrict__ A, const uint16_t* __restrict__ X,
     void* __restrict__ Y, const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices,
     const int32_t* __restrict__ row_ids) {
-  static_assert(!GROUP || W == 1, "a group's wavefronts have tiles of their own");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   int64_t slice;
   int f_tile;
-  if constexpr (GROUP) {  // tiles slice by slice, an eighth of the workgroups to an XCD
-    const int64_t total = slices * f_tiles, per = (((total + 3) >> 2) + 7) >> 3;
-    const int64_t t = ((blockIdx.x & 7) * per + (blockIdx.x >> 3)) * 4 + wave;
-    if ((blockIdx.x >> 3) >= per || t >= total) return;
-    slice = t / f_tiles, f_tile = (int)(t % f_tiles);
-  } else if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) {
-    return;
-  }
+  if (!decode_tile(blockIdx.x, slices, f_tiles, slice, f_tile)) return;
   // the same for all lanes, which the divisions hide from the compiler
   slice = __builtin_amdgcn_readfirstlane((int)slice), f_tile = __builtin_amdgcn_readfirstlane(f_tile);
   const int sub = blk / 32;  // slices per block row = steps per block
@@ -590,7 +581,7 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, D == 1 ? 4 : W == 1 
   // acc[r][t][v] is row 16 r + 4 g + v, feature 8 c + t
   const int64_t row0 = (int64_t)i_out * blk + bi0;
   if constexpr (W == 1) {
-    __shared__ f32x4 stage[GROUP ? 4 : 1][OUT == 1 ? 2 * kWave : 1];
+    __shared__ f32x4 stage[OUT == 1 ? 2 * kWave : 1];
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -598,7 +589,7 @@ __global__ __launch_bounds__(GROUP ? 4 * kWave : W * kWave, D == 1 ? 4 : W == 1 
         float o[8];
 #pragma unroll
         for (int t = 0; t < 8; ++t) o[t] = acc[r][t][v];
-        store_rows8<BF16, OUT, 16>(Y, row0 + 16 * r + v, feat, f0, lane, o, stage[GROUP ? wave : 0]);
+        store_rows8<BF16, OUT, 16>(Y, row0 + 16 * r + v, feat, f0, lane, o, stage);
       }
   } else {
     // each wavefront adds 8 / W of the eight rows a lane has
@@ -1171,11 +1162,12 @@ struct BsrForm {
   bool single = false;  // the direct kernels with one step of a wavefront on its way
 };
 
-inline int slice_rows(int blk, BsrForm::Kernel kernel) {  // blocks that are a multiple of 64 are no direct groups
+inline int slice_rows(int blk, BsrForm::Kernel kernel) {
   return blk % 32 != 0 ? 16 : kernel == BsrForm::kGroups && blk % 64 == 0 ? 64 : 32;
 }
 
-BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
+// floats: fp32 results
+BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, bool floats) {
   const int unit = slice_rows(blk, BsrForm::kSplit);
   const int64_t unit_slices = (int64_t)mb * (blk / unit);
   const int64_t steps = nnzb * (blk / 16) / 2 / mb;  // of a slice, 32 columns each, on average
@@ -1188,27 +1180,29 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb) {
     // hardly more than the CUs, with twice as much as the next: 35 x 437 blocks, 97 steps, 96 features 14.6 us, 16.9 with 128;
     // 42 x 285, 70 steps, 64 10.6, 11.3; 93 x 431, 106 steps, 320 (279 tiles) 26.0, 29.6; but 136 x 333, 67 steps, 256 (272, and
     // 544 of 64) 24.1, 20.8.  A little sooner where 128 waste half of a load: 8 x 35 of 128, 35 steps, 192 features 9.4, 10.1.
+    // Of 64 features alone from 20 steps on: 77 x 115 of 128, 21 steps 13.3, 14.6, 24 x 99 of 64, 29 steps 8.6, 9.5.
     const bool half = feat % kTileF != 0 && feat % kTileF <= kSplitF;
     if ((steps >= 40 && (split * 4 <= (feat % kSplitF ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus))) ||
-        (steps >= 32 && half && split <= cus))
+        (steps >= 32 && half && split <= cus) || (steps >= 20 && feat <= kSplitF && split <= 2 * cus))
       return {BsrForm::kSplit, false, false, false};
-    // Steps in turn as long as that leaves a CU little more than two workgroups of four wavefronts, or four of two; us with W =
-    // 1 / 2 / 4: 272 x 121 blocks, 25 steps, 224 features (544 tiles) 18.4 / 16.2 / 15.6, 292 x 182, 16 steps, 224 features
-    // (584) 14.2 / 13.8 / 13.9, 57 x 128, 14 steps, 1536 (684) 12.7 / 12.3 / 13.4, 49 x 78, 17 steps, 1952 (784) 14.3 / 14.3 /
-    // 14.3, 77 x 65, 7 steps, 1312 (847) 10.1 / 10.6 / 11.2; sooner not where there are few steps (192 x 51, 2 steps, 160
-    // features 5.1 / 5.5 / 5.2).  Eight where a CU has one tile and many steps: 131 x 322, 78 steps, 128 features 14.9, four 16.2.
-    const bool few = steps < 4;
+    // Steps in turn as long as that leaves a CU little more than two workgroups of four wavefronts, or four of two.  Means over
+    // 5000 drawn shapes, four wavefronts to a tile / two: up to 1.5 tiles a CU 0.7 to 0.95, 1.5 to 2.25 0.92 to 1.0 (the latter for 4
+    // to 8 steps: 107 x 48 blocks, 544 features 8.3 / 7.3), 2.25 to 2.75 1.0 to 1.14; two / one: up to 3.25 0.6 to 0.97, 3.25 to 4
+    // 0.85 to 0.98, 4 to 5 0.91 to 1.17.  Several wavefronts store the results sooner, so two also where fp32 results are most of the
+    // work (up to 3 steps 0.96; 252 x 36, 3 steps, 320 features 7.4 / 8.9), but not for 16-bit ones (1.05; 62 x 35, 2 steps, 2048
+    // features 7.3 / 6.2).  With far more X than the L2s hold one passes two sooner, 37 x 441, 102 steps, 2848 features (3.3 tiles) 59
+    // / 69.  Eight where a CU has one tile and many steps: 131 x 322, 78 steps, 128 features 14.9, four 16.2.
+    const bool few = steps < 4, apart = blk % 64 != 0;  // apart: no workgroup of 64 rows
     if (tiles <= cus && steps >= 24) return {BsrForm::kSplit, false, false, false, 8};
-    if (tiles * 4 <= (few ? 6 : 9) * cus) return {BsrForm::kSplit, false, false, false, 4};
-    // Two to four tiles to a slice, few steps and X in an L2: neighbours share A (471 x 75, 7 steps, 160 features 8.2, 9.4 with W =
-    // 1; 220 x 66, 5 steps, 288 features 6.9, 7.6; 396 x 27, 5 steps, 416 features 9.7, 10.5; but 166 x 95, 19 steps, 416 17.0, 16)
-    if (blk == 32 && feat > kTileF && feat <= 4 * kTileF && steps <= 8 && x_tile_bytes(kWaveF) <= 2500000)
-      return {BsrForm::kGroups, false, false, false, 1};
+    const int four = apart ? (steps < 8 ? 8 : 9) : few ? 6 : 9;
+    if (tiles * 4 <= four * cus) return {BsrForm::kSplit, false, false, false, 4};
     // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long and CUs have more than three
     // tiles: blocks of 64, 672 features, 46 steps (804 tiles) 31 / 37, 928, 31 steps (817) 23 / 26, of 128, 2304, 92 steps (792) 50 /
-    // 57; but 1600, 69 steps (676) 43 / 38, of 64, 2240, 30 steps (755) 23.0 / 19.7)
-    const int quarters = blk % 64 != 0 || steps < 24 ? 13 : steps < 48 ? 12 : 11;
-    if (tiles * 4 <= quarters * cus && !few) return {BsrForm::kSplit, false, false, false, 2};
+    // 57; but 1600, 69 steps (676) 43 / 38, of 64, 2240, 30 steps (755) 23.0 / 19.7; and with few steps)
+    const int two = few && !(apart && floats)           ? 0
+                    : apart                             ? (x_tile_bytes(kWaveF) <= 6000000 ? 16 : 13)
+                    : steps < 24 ? 13 : steps < 48 ? 12 : 11;
+    if (tiles * 4 <= two * cus) return {BsrForm::kSplit, false, false, false, 2};
   } else if (unit == 32) {
     // The split form wins as long as its workgroups are resident at once, two per CU, and up to twice as many where block rows
     // have enough steps to pay for the second turn.
@@ -1360,14 +1354,13 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const uint16_t* A = static_cast<const uint16_t*>(d_A);
   const uint16_t* X = static_cast<const uint16_t*>(d_X);
-  const BsrForm form = bsr_form(stir::compute_units(), mb, nb, blk, feat, nnzb);
+  const BsrForm form = bsr_form(stir::compute_units(), mb, nb, blk, feat, nnzb, out_dtype == STIR_F32);
   const int unit = slice_rows(blk, form.kernel), sub = blk / unit;
   const int f_tiles = (int)stir::ceil_div(feat, form.kernel == BsrForm::kSplit && !form.direct ? kSplitF : form.wide ? kWaveF : kTileF);
   const int64_t slices = (int64_t)mb * sub;
   auto eights = [](int64_t n) { return 8 * stir::ceil_div(n, 8); };  // see decode_tile, decode_ranked
   const int64_t blocks = form.by_rows  ? eights(mb) * sub * f_tiles
                          : form.ranked ? eights((int64_t)mb * f_tiles) * sub
-                         : form.kernel == BsrForm::kGroups && form.direct == 1 ? eights(stir::ceil_div(slices * f_tiles, 4))
                                        : eights(slices * f_tiles);
   STIR_REQUIRE(blocks < (int64_t(1) << 31), "bsr_spmm: too many tiles for one launch");
   const dim3 grid((unsigned)blocks);
@@ -1402,12 +1395,11 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
       else if (form.direct == 4) STIR_BSR_16((BF, OUT, 4, 1), 4);                                              \
       else STIR_BSR_16((BF, OUT, 8, 1), 8);                                                                    \
     } else if (form.direct) {                                                                                  \
-      if (form.kernel == BsrForm::kGroups) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, true>), 4 * kWave);      \
-      else if (form.single) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false, 1>), kWave);                     \
-      else if (form.direct == 1) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, false>), kWave);                   \
-      else if (form.direct == 8) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 8, false>), 8 * kWave);               \
-      else if (form.direct == 4) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 4, false>), 4 * kWave);               \
-      else STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 2, false>), 2 * kWave);                                     \
+      if (form.single) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1, 1>), kWave);                                 \
+      else if (form.direct == 1) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 1>), kWave);                          \
+      else if (form.direct == 8) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 8>), 8 * kWave);                      \
+      else if (form.direct == 4) STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 4>), 4 * kWave);                      \
+      else STIR_BSR_GO((bsr_direct_kernel<BF, OUT, 2>), 2 * kWave);                                            \
     } else if (form.kernel == BsrForm::kSplit) {                                                               \
       if (unit == 16) STIR_BSR_GO((bsr_split_kernel<BF, OUT, 16>), kWave * kSplitWaves);                       \
       else STIR_BSR_GO((bsr_split_kernel<BF, OUT, 32>), kWave * kSplitWaves);                                  \
@@ -1441,9 +1433,9 @@ extern "C" {
 // The form of a product on a device of so many compute units: kernel, then 4 for 256 features a tile, 8 for block rows
 // in order of their length, 16 for block rows dealt to XCDs, 32 times BsrForm::direct, 512 for BsrForm::single; -1 for what no
 // product is.  For the tests, which say what they cover.
-int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb) {
+int stir_bsr_form(int32_t cus, int32_t mb, int32_t nb, int32_t blk, int32_t feat, int64_t nnzb, int32_t floats) {
   if (cus <= 0 || mb <= 0 || nb < 0 || nnzb < 0 || blk <= 0 || blk % 16 != 0 || feat <= 0) return -1;
-  const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb);
+  const BsrForm f = bsr_form(cus, mb, nb, blk, feat, nnzb, floats != 0);
   return f.kernel + 4 * f.wide + 8 * f.ranked + 16 * f.by_rows + 32 * f.direct + 512 * f.single;
 }
 

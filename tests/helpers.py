@@ -245,15 +245,15 @@ def assert_close(actual, desired, rtol, atol, what=""):
             f"worst at flat index {i}: got {actual.ravel()[i]!r}, want {desired.ravel()[i]!r}")
 
 
-def bsr_form(mb, nb, blk, feat, nnzb, cus=256):
-    """The kernel that a BSR product takes on a device of `cus` compute units.  "128 by 4": operands in registers, tiles of 128
+def bsr_form(mb, nb, blk, feat, nnzb, cus=256, floats=False):
+    """The kernel that a BSR product takes on a device of `cus` compute units (floats: with fp32 results).  "128 by 4": operands in registers, tiles of 128
     features by four wavefronts that take the steps in turn (one: none does); "LDS 64 by 8": bsr_split_kernel; "LDS 64 x 256":
     64 rows by a workgroup of bsr_spmm_kernel.  Then the order of the block rows and what else the kernel's instance is."""
     import ctypes
 
     from sparsetir_amd import _lib
 
-    code = _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb))
+    code = _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb), int(floats))
     assert code >= 0
     kernel, width, direct = ("split", "waves", "groups")[code % 4], 256 if code & 4 else 128, code // 32 % 16
     order = (" ranked" if code & 8 else "") + (" by rows" if code & 16 else "")
@@ -261,8 +261,6 @@ def bsr_form(mb, nb, blk, feat, nnzb, cus=256):
         return "LDS 64 by 8" + order
     if kernel == "groups" and not direct:
         return f"LDS {64 if blk % 64 == 0 else 32} x {width}" + order
-    if kernel == "groups" and blk % 32 == 0:
-        return f"{width} by {direct}, four tiles" + order
     if kernel == "groups" and direct == 2:  # the two tiles of 128 of a workgroup
         return f"128 by {direct}, two tiles" + order
     return f"{width} by {direct or 1}" + order + (", one step" if code & 512 else "")

@@ -20,6 +20,16 @@ from helpers import bsr_form
     (400, 170, 96, 6, 512, "LDS 32 x 128"),
     (400, 170, 96, 16, 512, "256 by 1 ranked"),
     (1300, 325, 96, 8, 1504, "LDS 32 x 256"),
+    # steps in turn, by the tiles a compute unit has
+    (291, 58, 32, 4, 160, "128 by 2"),
+    (107, 48, 32, 5, 544, "128 by 2"),
+    (107, 48, 32, 9, 544, "128 by 4"),
+    (256, 66, 32, 5, 512, "128 by 2"),
+    (258, 66, 32, 5, 512, "128 by 1"),
+    (37, 441, 32, 102, 2848, "128 by 1"),            # far more X than the L2s hold
+    (57, 18, 96, 8, 704, "128 by 1"),
+    (18, 12, 128, 3, 1344, "LDS 64 x 128"),          # few steps: 64 rows by a workgroup
+    (77, 115, 128, 21, 64, "LDS 64 by 8"),
     # 64 rows by four wavefronts
     (1024, 256, 64, 12, 1024, "LDS 64 x 256"),
     (1024, 256, 64, 24, 1024, "LDS 64 x 256 ranked"),
@@ -43,6 +53,17 @@ def test_form(mb, nb, blk, steps, feat, form):
     assert bsr_form(mb, nb, blk, feat, nnzb) == form
 
 
+@pytest.mark.parametrize("mb,nb,blk,steps,feat,form,floats", [
+    # several wavefronts to a tile store fp32 results sooner
+    (62, 35, 32, 2, 2048, "128 by 1", "128 by 2"),
+    (199, 36, 32, 2, 352, "128 by 1", "128 by 2"),
+    (38, 13, 96, 2, 608, "128 by 1", "128 by 2"),
+])
+def test_form_with_few_steps(mb, nb, blk, steps, feat, form, floats):
+    nnzb = -(-steps * mb * 32 // blk)
+    assert bsr_form(mb, nb, blk, feat, nnzb) == form and bsr_form(mb, nb, blk, feat, nnzb, floats=True) == floats
+
+
 def test_sizes_whose_offsets_do_not_fit():
     """Where a load's offset from the wavefront's first may not fit 32 bits: kernels that allow for more."""
     assert bsr_form(4, 4, 32, 1 << 25, 16) == "LDS 32 x 256"
@@ -57,4 +78,4 @@ def test_sizes_whose_offsets_do_not_fit():
 def test_what_no_product_is(mb, nb, blk, feat, nnzb, cus):
     from sparsetir_amd import _lib
 
-    assert _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb)) == -1
+    assert _lib.lib().stir_bsr_form(cus, mb, nb, blk, feat, ctypes.c_int64(nnzb), 0) == -1

@@ -122,7 +122,7 @@ def test_bsr_rows_in_order_of_length(dev, dtype, out32, varied, mb, nb, form):
     indices = np.nonzero(present)[1].astype(np.int32)
     nnzb = len(indices)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert bsr_form(mb, nb, blk, feat, nnzb, cus) == form
+    assert bsr_form(mb, nb, blk, feat, nnzb, cus, out32) == form
     gen = torch.Generator(device=dev).manual_seed(3)
     a = (torch.randn(nnzb * blk * blk, device=dev, generator=gen) * 0.02).to(dtype)
     x = torch.randn(nb * blk * feat, device=dev, generator=gen).to(dtype)

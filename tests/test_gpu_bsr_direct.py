@@ -24,8 +24,8 @@ def _edges(dev, mb, nb, blk, feat, at_most, form, dtype, out_start=None):
     nnzb = len(cfg["indices"])
     cfg["data"] = rng.standard_normal((nnzb, blk, blk)).astype(np.float32) * 0.1
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert bsr_form(mb, nb, blk, feat, nnzb, cus) == form
     out, start = out_start or ((torch.float32, 1) if (mb & 1) == (dtype is torch.float16) else (dtype, 0))
+    assert bsr_form(mb, nb, blk, feat, nnzb, cus, out is torch.float32) == form
 
     def place(values):
         t = torch.empty(values.size + start, dtype=dtype, device=dev)[start:]
@@ -50,10 +50,11 @@ def _edges(dev, mb, nb, blk, feat, at_most, form, dtype, out_start=None):
     (240, 40, 32, 288, 20, "128 by 2"),       # more steps than tiles side by side are good for
     (100, 40, 32, 800, 12, "128 by 2"),
     (40, 12, 64, 992, 6, "128 by 2"),
-    (230, 33, 32, 416, 6, "128 by 1, four tiles"),        # the last of 32 features
-    (331, 20, 32, 160, 5, "128 by 1, four tiles"),        # two tiles to a slice: two slices in a workgroup
+    (230, 33, 32, 416, 6, "128 by 2"),        # the last of 32 features
+    (331, 20, 32, 160, 7, "128 by 2"),        # two tiles to a slice
     (300, 40, 32, 544, 7, "128 by 1"),
-    (160, 9, 96, 160, 3, "128 by 1"),
+    (160, 9, 96, 160, 3, "128 by 2"),
+    (230, 9, 96, 160, 3, "128 by 1"),
     (70, 200, 32, 2336, 30, "128 by 1, one step"),     # nothing to one step for some
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])

@@ -23,7 +23,7 @@ SHAPES = [
     (343, 200, 32, 0.01, 736, "128 by 1"),    # 32-row slices by a wavefront each
     (520, 200, 32, 0.01, 800, "128 by 1"),
     (650, 200, 32, 0.005, 512, "256 by 1"),
-    (397, 30, 32, 0.2, 416, "128 by 1, four tiles"),
+    (397, 30, 32, 0.2, 416, "128 by 1"),
     (147, 13, 64, 0.3, 2400, "LDS 64 x 256"),  # 64 rows by four wavefronts
     (14, 100, 128, 0.05, 160, "128 by 4"),
 ]
@@ -47,7 +47,7 @@ def test_non_finite_x(dev, mb, nb, blk, density, feat, form, dtype):
     unnamed = np.array([0, 1, nb - 1])
     cfg = _without(datasets.config4(seed=mb + feat, mb=mb, nb=nb, blk=blk, density=density, feat=feat), unnamed)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    assert bsr_form(mb, nb, blk, feat, len(cfg["indices"]), cus) == form
+    assert bsr_form(mb, nb, blk, feat, len(cfg["indices"]), cus, floats=True) == form
     x = cfg["x"].reshape(nb, blk, feat)
     x[unnamed[0]], x[unnamed[1]], x[unnamed[2]] = np.inf, np.nan, -np.inf
     named = int(cfg["indices"][len(cfg["indices"]) // 2])

@@ -116,8 +116,8 @@ def test_bsr_forms(dev, mb, nb, blk, density, feat, form):
     torch, block by block."""
     cfg = _config(mb, nb, blk, density, feat, seed=mb + feat)
     nnzb = len(cfg["indices"])
-    assert bsr_form(mb, nb, blk, feat, nnzb, _cus()) == form
     dtype, out = ((torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16))[mb & 1]
+    assert bsr_form(mb, nb, blk, feat, nnzb, _cus(), out is torch.float32) == form
     a, x = (torch.from_numpy(cfg[k]).to(dev).to(dtype) for k in ("data", "x"))
     y = torch.full((mb * blk * feat,), float("nan"), dtype=out, device=dev)
     d_ptr, d_idx = torch.from_numpy(cfg["indptr"]).to(dev), torch.from_numpy(cfg["indices"]).to(dev)

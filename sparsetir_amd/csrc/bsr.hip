@@ -1246,15 +1246,22 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // 128 by four / by eight: 80 steps, 96 features (154 tiles) 16.5 / 13.0, 33 steps (136) 8.5 / 7.6, 15 steps (220) 5.6 / 5.6; 60
     // steps (399) 15.7 / 15.4, 22 steps (996) 14.8 / 16.0.
     if (tiles <= cus && steps >= 20) return {BsrForm::kSplit, false, false, false, 8};
-    // Much X: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
+    // Much X and long rows, blocks of several slices, which read the same X: 256 by four in order of length.  Of the time by one
+    // wavefront (ranked), blocks of 80 and 112, 28 to 44 steps 0.88 to 0.97, more 0.9, as they come 0.9 to 0.97; of 48, 28 to 34 steps
+    // 1.0, 0.98 as they come (328 x 190, 29 steps, 1376 features 169, 157 by one) but 1.2 where X is far more than an L2 holds (224 x
+    // 336, 35 steps, 2208 features 260, 216 by one), more 0.96, 1.0 to 1.02.
+    if (several && x_bytes > kMuchX && feat > kTileF && steps >= (blk > 48 || x_bytes > 6200000 ? 28 : 36) &&
+        waste * 8 <= feat && waves >= 6 * cus)
+      return {BsrForm::kWaves, true, true, false, 4};
+    // Much X else: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
     // ranked / 256 ranked: blocks of 16, 1024 columns (8.4 MB), 51 steps, 1024 features 205 / 188 / 163, 24 steps 105 / 104 / 94,
-    // 4096 features 1204 / 780 / 650; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184; of 48, 65 steps,
-    // 3424 543 / 539 / 534.  Between 20 and 28 steps 128, with far more X than an L2 holds: 799 columns, 24 steps, 1632 features 167
+    // 4096 features 1204 / 736 / 618; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184.
+    // Between 20 and 28 steps 128, with far more X than an L2 holds: 799 columns, 24 steps, 1632 features 167
     // / 145 / 163, 993, 22 steps, 3744 108 / 101 / 115; less of it, 722 columns, 25 steps, 2752 174 / 176 / 173, 575, 16 steps, 2784
     // 39 / 42 / 39.  From 16 steps on 256 with few tiles, where the order gives little: 1024 columns, 24 steps, 1024 features 100 / 99 /
     // 90, but 490, 17 steps, 512 34 / 40 / 40.
     const bool wide_ranked = fits && (even || waste * 16 <= feat);
-    if (x_bytes > kMuchX && feat > kTileF && steps >= 16) {
+    if (x_bytes > kMuchX && feat > kTileF && steps >= 16 && !(several && fits)) {
       if (wide_ranked && (steps >= 28 || (wide_tiles >= 2 && wide_tiles <= 4 && x_bytes > kBeyondL2)))
         return {BsrForm::kWaves, true, true, false, 1};
       const bool long_enough = !wide_ranked && (steps >= 28 || x_narrow > kBeyondL2);
@@ -1267,21 +1274,21 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // 37.8, 183 x 840, 64 steps, 1568 (2379) 84.5 / 83.5 / 80.6; but 4.35 tiles to a CU, 90 steps, 320 features 50.5 / 52.3 / 61.5.
     if (!several && steps >= 20 && x_bytes > 6000000 && tiles * 10 >= 46 * cus && tiles < 10 * cus)
       return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
-    // Blocks of several slices, which read the same X.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of 80, 10
-    // steps, 416 features 138 / 130, 600 x 650 of 48, 7 steps, 256 20.8 / 21.0.  Less of it, 256 by four / by one: 1100 x 341 of 48,
-    // 10 steps, 1024 features 147 / 169, 5 steps, 140 columns 26 / 22.  And A, which every tile reads, more than the last level
-    // holds, 128 by four / 256 by four / by one: 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.
-    if (several && feat >= kWaveF && x_bytes > 15000000) return {BsrForm::kGroups, true, false, false, 2};
-    if (several && feat > kTileF && ((fits && x_bytes > kMuchX) || nnzb * blk * blk * 2 > kLastLevel))
-      return {BsrForm::kWaves, true, false, false, steps >= 8 ? 4 : 1};
+    // Blocks of several slices else.  A, which every tile reads, more than the last level holds, 128 by four / 256 by four / by one:
+    // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of
+    // 80, 10 steps, 416 features 138 / 130.  Wide tiles and enough of them: from 16 steps on 256 by four, 0.92 to 1.0 of the time by one;
+    // with 5 to 15 steps two of 128, 0.91 to 0.97 of the time of 256 by one whatever X (1100 x
+    // 341 of 48, 10 steps, 1024 features 256 by one / by four / two of 128 142 / 135 / 118); with fewer 128 by one (below), 0.92.
+    if (several && feat > kTileF && (nnzb * blk * blk * 2 > kLastLevel || (fits && steps >= 16 && (even || x_bytes > kMuchX))))
+      return {BsrForm::kWaves, true, false, false, 4};
+    if (several && feat >= kWaveF && (x_bytes > 15000000 || (fits && steps >= 5 && steps < 16)))
+      return {BsrForm::kGroups, true, false, false, 2};
     // X in an L2, 128 by one / by four / two of 128 / 256: 342 x 83 of 16, 4 steps, 1728 features 14.8 / 17.2 / 16.2 / 16.7; 420
     // columns, 10 steps, 512 24.5 / 24.5 / - / 23.3; 300, 12 steps, 1024 47.8 / 47.2 / - / 43.7; 73, 8 steps, 3904 67 / 73 / 65 /
     // 63; 65, 7 steps, 224 features (1254 tiles) 8.7 / 9.0 / 8.4 / 9.3; 92, 8 steps, 160 (1498) 11.1 / 11.5 / 9.1 / 9.9.
     if (steps <= 4 && tiles >= 6 * cus && x_bytes <= 2500000) return {BsrForm::kWaves, false, false, false, 1};
-    if (fits && even && x_bytes <= 3500000) return {BsrForm::kWaves, true, false, false, 1};
+    if (!several && fits && even && x_bytes <= 3500000) return {BsrForm::kWaves, true, false, false, 1};
     if (feat > kTileF && x_bytes <= 2500000 && tiles * 4 >= (even ? 19 : 48) * cus && steps < 20)
-      return {BsrForm::kGroups, true, false, false, 2};
-    if (several && feat >= kWaveF && tiles < 16 * cus && x_bytes > kMuchX && steps < 12)
       return {BsrForm::kGroups, true, false, false, 2};
     // 128 by one / by four: 5 steps, 1696 features (1442 tiles) 9.4 / 9.8, 3 steps (1140) 9.1 / 7.6; 6 steps, 1024 columns (8000)
     // 37.2 / 37.1; of 48, 11 steps, 320 features (33 k) 230 / 208, of 80, 8 steps, 800 (105 k) 468 / 473.

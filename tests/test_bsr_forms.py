@@ -41,7 +41,19 @@ from helpers import bsr_form
     (4096, 1025, 16, 10, 1024, "128 by 1"),
     (4096, 1025, 16, 18, 1024, "256 by 1 ranked"),
     (1024, 420, 16, 10, 512, "256 by 1"),
-    (1100, 341, 48, 10, 1024, "256 by 4"),
+    (1100, 341, 48, 10, 1024, "128 by 2, two tiles"),
+    (137, 84, 80, 27, 1824, "256 by 4"),
+    (137, 84, 80, 29, 1824, "256 by 4 ranked"),
+    (330, 320, 48, 39, 1280, "256 by 4 ranked"),
+    (137, 84, 80, 29, 1312, "128 by 1 ranked"),       # a last tile of 256 mostly empty
+    (30, 84, 80, 29, 1824, "128 by 4"),               # few
+    (97, 38, 112, 27, 2720, "256 by 4"),              # X in an L2
+    (97, 38, 112, 15, 2720, "128 by 2, two tiles"),
+    (97, 38, 112, 4, 2720, "128 by 1"),
+    (328, 190, 48, 29, 1376, "256 by 4"),
+    (224, 336, 48, 29, 2208, "256 by 4 ranked"),
+    (97, 38, 112, 19, 2400, "128 by 2, two tiles"),   # an odd number of tiles of 128
+    (22, 174, 48, 11, 320, "128 by 4"),
     (600, 650, 48, 7, 256, "128 by 2, two tiles"),
     (3693, 559, 48, 11, 320, "128 by 1"),
     (1214, 659, 80, 10, 416, "128 by 2, two tiles"),

@@ -74,8 +74,9 @@ def test_direct_edges(dev, mb, nb, blk, feat, at_most, form, dtype):
     (420, 45, 16, 480, 7, "128 by 1"),
     (96, 750, 16, 2176, 61, "128 by 1, one step"),     # nothing to one step for some
     (1050, 20, 16, 480, 16, "256 by 1"),
-    (205, 20, 80, 480, 4, "256 by 1"),
-    (230, 140, 48, 992, 12, "256 by 4"),
+    (205, 20, 80, 480, 4, "128 by 2, two tiles"),
+    (180, 60, 48, 992, 24, "256 by 4"),
+    (180, 140, 48, 992, 40, "256 by 4 ranked"),
 ])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_direct16_edges(dev, mb, nb, blk, feat, at_most, form, dtype):
@@ -106,7 +107,7 @@ def test_lds_split_edges(dev, mb, nb, blk, feat, at_most, form, dtype):
     (64, 30, 80, 160, 9, "128 by 4"),
     (640, 25, 16, 608, 17, "128 by 2, two tiles"),
     (1050, 20, 16, 480, 16, "256 by 1"),
-    (230, 140, 48, 992, 12, "256 by 4"),
+    (180, 60, 48, 992, 24, "256 by 4"),
     (260, 90, 16, 64, 85, "LDS 64 by 8"),
     (147, 13, 64, 2400, 8, "LDS 64 x 256"),
 ])

@@ -14,7 +14,8 @@ SHAPES = [
     (1024, 60, 16, 0.1, 224, "128 by 1"),     # 16-row slices by a wavefront each
     (1024, 400, 16, 0.01, 512, "256 by 1"),
     (230, 50, 48, 0.05, 352, "128 by 1"),     # three chunks a block
-    (230, 140, 48, 0.03, 1024, "256 by 1"),
+    (230, 140, 48, 0.03, 1024, "128 by 2, two tiles"),
+    (180, 50, 48, 0.35, 1024, "256 by 4"),
     (150, 40, 16, 0.2, 1184, "128 by 2, two tiles"),
     (61, 23, 80, 0.3, 480, "128 by 2, two tiles"),
     (3, 200, 16, 0.5, 64, "128 by 8"),

@@ -105,11 +105,12 @@ def _cus():
     # 16-row slices
     (1030, 490, 16, 0.07, 512, "256 by 1 ranked"),
     (430, 1000, 16, 0.04, 672, "128 by 1 ranked"),
-    (171, 170, 48, 0.07, 1024, "256 by 1 ranked"),
+    (171, 170, 48, 0.07, 1024, "256 by 4"),
+    (171, 170, 48, 0.16, 1024, "256 by 4 ranked"),     # the slices of a block row on one XCD
     (200, 330, 48, 0.05, 608, "128 by 1 ranked"),
-    (230, 140, 48, 0.03, 1024, "256 by 1"),
-    (110, 40, 80, 0.2, 1024, "256 by 1"),             # little X, long rows
-    (400, 140, 48, 0.03, 288, "128 by 2, two tiles"),           # wavefronts of 128 features would be few
+    (230, 140, 48, 0.03, 1024, "128 by 2, two tiles"),
+    (110, 40, 80, 0.2, 1024, "256 by 4"),             # little X, long rows
+    (400, 140, 48, 0.03, 288, "128 by 4"),
 ])
 def test_bsr_forms(dev, mb, nb, blk, density, feat, form):
     """Every form of a launch, with long and empty block rows and columns in any order, against the same sums in fp64 by

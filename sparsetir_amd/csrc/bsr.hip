@@ -1175,6 +1175,8 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
   const int64_t split = 8 * stir::ceil_div(unit_slices * stir::ceil_div(feat, kSplitF), 8);
   const int64_t tiles = unit_slices * stir::ceil_div(feat, kTileF);
   auto x_tile_bytes = [&](int width) { return (int64_t)nb * blk * 2 * width; };
+  // Of the rows of X that a tile of 256 features reads: what an L2 holds beside A, an L2, far more; of A: the last level.
+  constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kFarX = 6000000, kLastLevel = 256 << 20;
   if (unit == 32 && wavefronts) {
     // Tiles of 64 features, by eight wavefronts through LDS, where rows are long and tiles of 128 leave CUs without one or,
     // hardly more than the CUs, with twice as much as the next: 35 x 437 blocks, 97 steps, 96 features 14.6 us, 16.9 with 128;
@@ -1200,7 +1202,7 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // tiles: blocks of 64, 672 features, 46 steps (804 tiles) 31 / 37, 928, 31 steps (817) 23 / 26, of 128, 2304, 92 steps (792) 50 /
     // 57; but 1600, 69 steps (676) 43 / 38, of 64, 2240, 30 steps (755) 23.0 / 19.7; and with few steps)
     const int two = few && !(apart && floats)           ? 0
-                    : apart                             ? (x_tile_bytes(kWaveF) <= 6000000 ? 16 : 13)
+                    : apart                             ? (x_tile_bytes(kWaveF) <= kFarX ? 16 : 13)
                     : steps < 24 ? 13 : steps < 48 ? 12 : 11;
     if (tiles * 4 <= two * cus) return {BsrForm::kSplit, false, false, false, 2};
   } else if (unit == 32) {
@@ -1208,7 +1210,6 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // have enough steps to pay for the second turn.
     if (split <= 2 * cus || (split <= 4 * cus && steps >= 32)) return {BsrForm::kSplit, false, false, false};
   }
-  constexpr int64_t kMuchX = 3 << 20, kBeyondL2 = 4000000, kLastLevel = 256 << 20;
   const int64_t wide_tiles = stir::ceil_div(feat, kWaveF), waste = wide_tiles * kWaveF - feat;
   // Slices in order of their length (row_of_rank) where that makes up for finding the row, which costs as much as 2 or 3
   // steps: with the rows of X of a feature tile (x_bytes) more than an XCD's L2 holds beside A, since what runs side by
@@ -1250,29 +1251,31 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // wavefront (ranked), blocks of 80 and 112, 28 to 44 steps 0.88 to 0.97, more 0.9, as they come 0.9 to 0.97; of 48, 28 to 34 steps
     // 1.0, 0.98 as they come (328 x 190, 29 steps, 1376 features 169, 157 by one) but 1.2 where X is far more than an L2 holds (224 x
     // 336, 35 steps, 2208 features 260, 216 by one), more 0.96, 1.0 to 1.02.
-    if (several && x_bytes > kMuchX && feat > kTileF && steps >= (blk > 48 || x_bytes > 6200000 ? 28 : 36) &&
+    if (several && x_bytes > kMuchX && feat > kTileF && steps >= (blk > 48 || x_bytes > kFarX ? 28 : 36) &&
         waste * 8 <= feat && waves >= 6 * cus)
       return {BsrForm::kWaves, true, true, false, 4};
     // Much X else: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
     // ranked / 256 ranked: blocks of 16, 1024 columns (8.4 MB), 51 steps, 1024 features 205 / 188 / 163, 24 steps 105 / 104 / 94,
     // 4096 features 1204 / 736 / 618; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184.
-    // Between 20 and 28 steps 128, with far more X than an L2 holds: 799 columns, 24 steps, 1632 features 167
-    // / 145 / 163, 993, 22 steps, 3744 108 / 101 / 115; less of it, 722 columns, 25 steps, 2752 174 / 176 / 173, 575, 16 steps, 2784
+    // With far more X than an L2 holds and many tiles 128 from 20 steps on and 256 only from 44: 799 columns, 24 steps, 1632 features 167
+    // / 145 / 163, 993, 22 steps, 3744 108 / 101 / 115, 872, 32 steps, 3168 231 / 206 / 234, 905, 32 steps, 3680, fp32 results 256 / 223 /
+    // 250, 31 drawn shapes of 28 to 44 steps 0.96 of the time of 256; less of it, 722 columns, 25 steps, 2752 174 / 176 / 173, 575, 16 steps, 2784
     // 39 / 42 / 39.  From 16 steps on 256 with few tiles, where the order gives little: 1024 columns, 24 steps, 1024 features 100 / 99 /
     // 90, but 490, 17 steps, 512 34 / 40 / 40.
     const bool wide_ranked = fits && (even || waste * 16 <= feat);
     if (x_bytes > kMuchX && feat > kTileF && steps >= 16 && !(several && fits)) {
-      if (wide_ranked && (steps >= 28 || (wide_tiles >= 2 && wide_tiles <= 4 && x_bytes > kBeyondL2)))
+      const int wide_from = x_bytes > kFarX && wide_tiles > 4 ? 44 : 28;
+      if (wide_ranked && (steps >= wide_from || (wide_tiles >= 2 && wide_tiles <= 4 && x_bytes > kBeyondL2)))
         return {BsrForm::kWaves, true, true, false, 1};
       const bool long_enough = !wide_ranked && (steps >= 28 || x_narrow > kBeyondL2);
-      if (unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (long_enough || (steps >= 20 && x_bytes > 6200000)))
+      if (unit_slices * narrow_tiles >= (fits ? 8 : 10) * cus && (long_enough || (steps >= 20 && x_bytes > kFarX)))
         return {BsrForm::kWaves, false, true, false, 1};
     }
     // Long rows, far more X than an L2 holds and a turn of wavefronts: by one, which stay closer together in X, with one step on its
     // way each where there are more of them; 128 by four / by one with two steps / with one: 95 x 793, 26 steps, 1856 features
     // (1425 tiles) 24.8 / 22.1 / 23.7, 80 x 818, 23 steps, 2848 (1840) 34.5 / 30.9 / 28.6, 70 x 896, 40 steps, 2848 (1610) 48.4 / 40.6 /
     // 37.8, 183 x 840, 64 steps, 1568 (2379) 84.5 / 83.5 / 80.6; but 4.35 tiles to a CU, 90 steps, 320 features 50.5 / 52.3 / 61.5.
-    if (!several && steps >= 20 && x_bytes > 6000000 && tiles * 10 >= 46 * cus && tiles < 10 * cus)
+    if (!several && steps >= 20 && x_bytes > kFarX && tiles * 10 >= 46 * cus && tiles < 10 * cus)
       return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
     // Blocks of several slices else.  A, which every tile reads, more than the last level holds, 128 by four / 256 by four / by one:
     // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of

@@ -41,6 +41,10 @@ from helpers import bsr_form
     (4096, 1025, 16, 10, 1024, "128 by 1"),
     (4096, 1025, 16, 18, 1024, "256 by 1 ranked"),
     (1024, 420, 16, 10, 512, "256 by 1"),
+    (521, 872, 16, 32, 3168, "128 by 1 ranked"),      # far more X than an L2 holds, many tiles
+    (521, 872, 16, 44, 3168, "256 by 1 ranked"),
+    (521, 700, 16, 32, 3168, "256 by 1 ranked"),
+    (1024, 872, 16, 32, 1024, "256 by 1 ranked"),     # few
     (1100, 341, 48, 10, 1024, "128 by 2, two tiles"),
     (137, 84, 80, 27, 1824, "256 by 4"),
     (137, 84, 80, 29, 1824, "256 by 4 ranked"),

@@ -763,17 +763,16 @@ __global__ __launch_bounds__(W * T * kWave, D == 1 ? 5 : W == 1 ? 4 : 2) void bs
 }
 
 // A tile of 16 rows x 256 features, sixteen accumulators, in two halves of 128 features: as soon as the last operand of a half is
-// made, the next step's half is asked for.  By a wavefront, or by four that take the steps in turn.  The columns come by scalar
+// made, the next step's half is asked for.  By a wavefront (blocks of 16), or by four that take the steps in turn.  The columns come by scalar
 // loads, a step ahead: a vector load of them on a branch in the loop made every wait in it one for all loads (11 % slower).
 // 1024 x 300 blocks of 16, 12 steps, 1024 features 52 us with X through LDS, 43.7; 1024 x 1024, 51 steps 174 -> 161 ranked, where
 // X comes from beyond the L2s either way: 4096 features 656 -> 647.
-template <bool BF16, int OUT, int W, bool ONE>
-__global__ __launch_bounds__(W * kWave, 3) void bsr16_wave_kernel(int blk, int feat, int64_t slices, int f_tiles, int ranked,
-                                                              const uint16_t* __restrict__ A,
-                                                              const uint16_t* __restrict__ X, void* __restrict__ Y,
-                                                              const int32_t* __restrict__ indptr,
-                                                              const int32_t* __restrict__ indices,
-                                                              const int32_t* __restrict__ row_ids) {
+template <bool BF16, int OUT, bool ONE>
+__global__ __launch_bounds__((ONE ? 1 : 4) * kWave, 3) void bsr16_wave_kernel(
+    int blk, int feat, int64_t slices, int f_tiles, int ranked, const uint16_t* __restrict__ A,
+    const uint16_t* __restrict__ X, void* __restrict__ Y, const int32_t* __restrict__ indptr,
+    const int32_t* __restrict__ indices, const int32_t* __restrict__ row_ids) {
+  constexpr int W = ONE ? 1 : 4;
   if (ONE) blk = 16;
   const int sub = blk / 16;
   int64_t slice;
@@ -1384,23 +1383,14 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     if (blk == 16) STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);          \
     else STIR_BSR_GO((bsr16_direct_kernel<STIR_ARGS ARGS, false>), (WAVES) * kWave, ranked);                   \
   } while (0)
-#define STIR_BSR_16S(BF, OUT)                                                                                  \
-  do {                                                                                                         \
-    if (blk == 16) STIR_BSR_GO((bsr16_direct_kernel<BF, OUT, 1, 1, true, 1>), kWave, ranked);                  \
-    else STIR_BSR_GO((bsr16_direct_kernel<BF, OUT, 1, 1, false, 1>), kWave, ranked);                           \
-  } while (0)
-#define STIR_BSR_16W(ARGS, WAVES)                                                                              \
-  do {                                                                                                         \
-    if (blk == 16) STIR_BSR_GO((bsr16_wave_kernel<STIR_ARGS ARGS, true>), (WAVES) * kWave, ranked);            \
-    else STIR_BSR_GO((bsr16_wave_kernel<STIR_ARGS ARGS, false>), (WAVES) * kWave, ranked);                     \
-  } while (0)
 #define STIR_BSR(BF, OUT)                                                                                      \
   do {                                                                                                         \
     if (form.direct && unit == 16) {                                                                           \
       if (form.kernel == BsrForm::kGroups && form.direct == 2) STIR_BSR_16((BF, OUT, 2, 2), 4);                \
-      else if (form.wide && form.direct == 1) STIR_BSR_16W((BF, OUT, 1), 1);                                   \
-      else if (form.wide) STIR_BSR_16W((BF, OUT, 4), 4);                                                       \
-      else if (form.single) STIR_BSR_16S(BF, OUT);                                                             \
+      else if (form.wide && blk == 16) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, true>), kWave, ranked);         \
+      else if (form.wide) STIR_BSR_GO((bsr16_wave_kernel<BF, OUT, false>), 4 * kWave, ranked);                 \
+      else if (form.single && blk == 16)                                                                       \
+        STIR_BSR_GO((bsr16_direct_kernel<BF, OUT, 1, 1, true, 1>), kWave, ranked);                             \
       else if (form.direct == 1) STIR_BSR_16((BF, OUT, 1, 1), 1);                                              \
       else if (form.direct == 4) STIR_BSR_16((BF, OUT, 4, 1), 4);                                              \
       else STIR_BSR_16((BF, OUT, 8, 1), 8);                                                                    \
@@ -1429,8 +1419,6 @@ static int bsr_launch(int32_t dtype, int32_t out_dtype, int32_t mb, int32_t nb, 
     if (out_dtype == STIR_F32) STIR_BSR(false, 1); else STIR_BSR(false, 0);
   }
 #undef STIR_BSR
-#undef STIR_BSR_16W
-#undef STIR_BSR_16S
 #undef STIR_BSR_16
 #undef STIR_ARGS
 #undef STIR_BSR_GO

@@ -542,6 +542,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
                                                               const int32_t* __restrict__ indptr,
                                                               const int32_t* __restrict__ indices) {
   using Acc = TcAcc<T == 32>;
+  static_assert(NTL == 1 || NTL == 2, "wider units: tcspmm_direct_kernel");
   constexpr int TF = 32 * NTL;
   constexpr int FCN = TF / 8;             // 16-byte units of a staged row
   constexpr int LOADS = FCN / 2;          // ... of a step's 32 rows per lane
@@ -575,7 +576,7 @@ __global__ __launch_bounds__(64 * W) void tcspmm_units_kernel(int feat, int64_t 
   char* image = lds + wave * XB;
 
   auto swizzle = [](int k) {
-    return (FCN == 4 ? 0 : FCN == 8 ? 4 * ((k >> 1) & 1) : 4 * (k & 3)) ^ (T == 32 ? 0 : 2 * ((k >> 3) & 1));
+    return (FCN == 4 ? 0 : 4 * ((k >> 1) & 1)) ^ (T == 32 ? 0 : 2 * ((k >> 3) & 1));
   };
   // staging role: unit c of the rows k0 + u * (64 / FCN)
   const int c = lane % FCN, k0 = lane / FCN;

@@ -1,5 +1,6 @@
 """How BSR products are launched, on either side of each line that was measured (256 compute units; no GPU needed)."""
 import ctypes
+import random
 
 import pytest
 
@@ -78,6 +79,18 @@ def test_form(mb, nb, blk, steps, feat, form):
 def test_form_with_few_steps(mb, nb, blk, steps, feat, form, floats):
     nnzb = -(-steps * mb * 32 // blk)
     assert bsr_form(mb, nb, blk, feat, nnzb) == form and bsr_form(mb, nb, blk, feat, nnzb, floats=True) == floats
+
+
+def test_16_row_slices_name_instances_that_exist():
+    """Tiles of 256 features are by one wavefront in blocks of 16 and by four in others; one step on its way in blocks of 16 only."""
+    rng = random.Random(3)
+    for _ in range(20000):
+        blk = rng.choice([16, 48, 80, 112, 144])
+        mb, nb, feat = (int(2 ** rng.uniform(0, top)) for top in (12, 11, 7))
+        form = bsr_form(mb, nb, blk, 32 * feat, int(mb * nb * 2 ** rng.uniform(-8, 0)), floats=rng.random() < 0.5)
+        if form.startswith("256"):
+            assert form.startswith("256 by 1" if blk == 16 else "256 by 4")
+        assert blk == 16 or "one step" not in form
 
 
 def test_sizes_whose_offsets_do_not_fit():

@@ -298,6 +298,10 @@ __global__ __launch_bounds__(4 * kWave) void csr_spmm_kernel(int m, int feat, in
 // 4096 rows, 65 k nonzeros, 32 features, rows of up to 1024: 5.5 us, of up to 128 4.0, all alike 3.2, an empty launch
 // 2.2.  With the long rows after the others, found by way of LDS and one load of columns before each set of rows of B:
 // 6.6, 5.1, 3.4.
+// Above 256 features (REP = 2) a lane holds two chunks of each row and still eight rows, 105 registers: a row of 107
+// nonzeros is a chain of that many / 8 steps, at 288 features 13.9 us, with four rows a step 15.3 (one of 212 in eight
+// shares, 416 features: 7.1 and 7.6).  The last one or two rows are a step of their own, rows of up to four
+// nonzeros being 3 % slower with four loads for them.
 template <int G, int REP>
 __global__ __launch_bounds__(kSmallWaves * kWave) void csr_small_kernel(int m, int feat, const float* __restrict__ A,
                                                                         const float* __restrict__ B,
@@ -305,7 +309,7 @@ __global__ __launch_bounds__(kSmallWaves * kWave) void csr_small_kernel(int m, i
                                                                         const int32_t* __restrict__ indptr,
                                                                         const int32_t* __restrict__ indices) {
   constexpr int NG = kWave / G;
-  constexpr int kWide = G == 4 ? 4 : 8 / REP;  // rows of B in flight per lane; NG * kWide divides 64
+  constexpr int kWide = G == 4 ? 4 : 8;  // rows of B in flight per lane group; NG * kWide divides 64
   constexpr int kRound = G * REP >= 64 ? 1 : 64 / (G * REP) < kSmallWaves ? 64 / (G * REP) : kSmallWaves;
   __shared__ float4 part[kRound * kSmallWaves * G * REP];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -370,7 +374,10 @@ __global__ __launch_bounds__(kSmallWaves * kWave) void csr_small_kernel(int m, i
     };
     int j0 = 0;
     for (; j0 + NG * (kWide / 2) < cnt; j0 += NG * kWide) step(j0, std::integral_constant<int, kWide>());
-    if (j0 < cnt) step(j0, std::integral_constant<int, kWide / 2>());
+    if (REP > 1 && j0 < cnt && j0 + NG * 2 >= cnt)
+      step(j0, std::integral_constant<int, 2>());
+    else if (j0 < cnt)
+      step(j0, std::integral_constant<int, kWide / 2>());
     if (done) {
       reduce_groups<G, REP>(acc, kWave);
       if (own) {

@@ -28,3 +28,21 @@ def test_own_and_shared_rows(dev, feat, groups):
     assert np.all(got[np.asarray(deg) == 0] == 0.0)
     _check(got, indptr, indices, vals, x, f"feat={feat}")
     assert np.array_equal(got, _run_csr(dev, indptr, indices, vals, x, feat))  # no atomics: the same bits
+
+
+@pytest.mark.parametrize("feat", [257, 260, 384, 509, 512])
+def test_wide_rows_end_in_two_four_or_eight(dev, feat):
+    """Above 256 features the rows of B are in flight eight at a time, and the last ones of up to 64 nonzeros in steps of
+    four or two: own rows and shares of long ones that end in each."""
+    deg = list(range(0, 19)) + [61, 62, 63, 64, 65, 66, 68, 71, 128, 129, 136, 137, 160, 200, 250, 264]
+    n = 700
+    rng = np.random.default_rng(feat)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    assert indptr[-1] * feat < 3_000_000
+    indices = np.concatenate([np.sort(rng.choice(n, d, replace=False)) for d in deg]).astype(np.int32)
+    vals = rng.random(len(indices), dtype=np.float32) - 0.4
+    x = rng.standard_normal((n, feat), dtype=np.float32)
+    got = _run_csr(dev, indptr, indices, vals, x, feat)
+    assert got[0].max() == 0.0 == got[0].min()
+    _check(got, indptr, indices, vals, x, f"feat={feat}")
+    assert np.array_equal(got, _run_csr(dev, indptr, indices, vals, x, feat))

@@ -1,13 +1,14 @@
 // BSR SpMM on the gfx950 matrix cores: Y[i-th block row] = sum over stored blocks p of
 // A_p (blk x blk) * X[indices[p]-th block of rows], 16-bit inputs, fp32 accumulation.
 //
-// Slices of 32 rows, 16 where the block is an odd multiple of that: a wavefront owns them x 128 or 256 features, loads the rows of X into registers eight features to
-// a lane and makes the MFMA B operand (8 consecutive k of one feature per lane) out of them with v_perm: no LDS and no
-// other wavefront is in the way (bsr_direct_kernel, bsr_wave_kernel, bsr16_direct_kernel, bsr16_wave_kernel).  In small
-// launches the wavefronts of a workgroup take the steps of one tile in turn.
+// Slices of 32 rows, 16 where the block is an odd multiple of that: a wavefront owns them x 128 or 256 features, loads the
+// rows of X into registers eight features to a lane and makes the MFMA B operand (8 consecutive k of one feature per lane)
+// out of them with v_perm: no LDS and no other wavefront is in the way (bsr_direct_kernel, bsr_wave_kernel,
+// bsr16_direct_kernel, bsr16_wave_kernel).  In small launches, and in larger ones of 16-row slices, the wavefronts of a
+// workgroup take the steps of one tile in turn.
 // Slices of 64 rows (blocks that are a multiple of 64, where there are many): a workgroup of four wavefronts owns 64 rows
-// and a 128*NT-wide slice of the feature axis; both operands go through LDS (bsr_tile).  The smallest launches of
-// long block rows, whatever the block, by bsr_split_kernel.
+// and a 128*NT-wide slice of the feature axis; both operands go through LDS (bsr_tile).  Small launches of long block rows
+// whose tiles of 128 features leave CUs idle, whatever the block, by bsr_split_kernel.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>
@@ -281,9 +282,9 @@ __device__ __forceinline__ void bsr_tile(char* __restrict__ lds, int blk, int fe
 
   // The step to fetch next: block pb of the row, k offset k0; nothing beyond the last, so that no load depends on a
   // branch.  The block columns of the 64 blocks in hand and of the next 64 are in registers, one per lane: asked for
-  // one by one, each block waited for a scalar load (128 x 128 blocks of 32, 512 features 11.7 -> 11.3 us; 60 x 60 of
-  // 64, 512 features 13.0 -> 11.9; 430 x 120 of 32, 1120 features 62.5 -> 59.3).  Two to four steps in registers at a
-  // time gain on the first two (11.0 and 10.7 with four) and lose 3 to 15 % on larger ones.
+  // one by one, each block waited for a scalar load (430 x 120 blocks of 32, 1120 features, by this kernel 62.5 -> 59.3 us).
+  // Two to four steps in registers at a time gain 3 to 10 % with two workgroups to a CU, sizes that other forms take, and
+  // lose 3 to 15 % on larger ones.
   int pb = 0, k0 = 0;
   int j_lane = lane < nblk ? indices[p_begin + lane] : 0;
   int j_more = kWave + lane < nblk ? indices[p_begin + kWave + lane] : 0;
@@ -489,7 +490,7 @@ __device__ __forceinline__ void add_up8(const f32x4* part, int stride, int used,
 // D steps are on their way; nothing is asked for beyond the last one: a load outside its window costs as much as another
 // (128 x 128 blocks of 32, 512 features, four wavefronts 9.8 -> 9.1 us).
 // Against four wavefronts that shared 128 features through LDS and met at a barrier per step, us as part of a graph:
-// 128 x 128 blocks of 32, 10 %, 512 features 11.1 -> 9.1 (W = 4); 256 x 256, 512 features 24.0 -> 20.1 (W = 1); 209 x 46, 2
+// 128 x 128 blocks of 32, 10 %, 512 features 11.1 -> 9.1 (W = 4); 256 x 256, 512 features 24.0 -> 20.1 (W = 1; 2 now); 209 x 46, 2
 // steps a row, 1216 features 9.3 -> 7.8 (W = 1); against eight wavefronts with 64
 // features through LDS: 197 x 193, 37 steps, 224 features 23.0 -> 16.3 (W = 4), 131 x 322, 78 steps, 128 features 18.7 ->
 // 14.9 (W = 8).  Small launches are bound by the trips to memory one after the other -- indptr, block columns, rows of X,
@@ -763,10 +764,11 @@ __global__ __launch_bounds__(W * T * kWave, D == 1 ? 5 : W == 1 ? 4 : 2) void bs
 }
 
 // A tile of 16 rows x 256 features, sixteen accumulators, in two halves of 128 features: as soon as the last operand of a half is
-// made, the next step's half is asked for.  By a wavefront (blocks of 16), or by four that take the steps in turn.  The columns come by scalar
-// loads, a step ahead: a vector load of them on a branch in the loop made every wait in it one for all loads (11 % slower).
+// made, the next step's half is asked for.  By a wavefront (blocks of 16), or by four that take the steps in turn (the others).
+// The columns come by scalar loads, a step ahead: a vector load of them on a branch in the loop made every wait in it one for
+// all loads (11 % slower).
 // 1024 x 300 blocks of 16, 12 steps, 1024 features 52 us with X through LDS, 43.7; 1024 x 1024, 51 steps 174 -> 161 ranked, where
-// X comes from beyond the L2s either way: 4096 features 656 -> 647.
+// X comes from beyond the L2s either way 16384 x 16384, 10 %, 4096 features 611 to 632 -> 606 to 619, 30 % more of it missing L2.
 template <bool BF16, int OUT, bool ONE>
 __global__ __launch_bounds__((ONE ? 1 : 4) * kWave, 3) void bsr16_wave_kernel(
     int blk, int feat, int64_t slices, int f_tiles, int ranked, const uint16_t* __restrict__ A,
@@ -1003,8 +1005,7 @@ __global__ __launch_bounds__(kWave, 2) void bsr_wave_kernel(int blk, int feat, i
 // rows fill the 64 banks -- and, ROWS = 16, ^ 2 * (k / 8 % 2): the two blocks of 16 lanes that
 // a transposing read serves together ask for the same units of k groups eight rows apart there.
 // Against four wavefronts that took the k halves of each step: 40 x 510 blocks of 32, 18 %, 288 features
-// 27.4 -> 15.9 us; 50 x 63 blocks of 128, 128 features 27.6 -> 17.2 us; 358 x 998 blocks of 16, 64 features
-// (which had no such form) 39 -> 11.8 us.
+// 27.4 -> 15.9 us; 358 x 998 blocks of 16, 64 features (which had no such form) 39 -> 11.8 us.
 constexpr int kSplitWaves = 8;
 constexpr int kSplitF = 64;
 

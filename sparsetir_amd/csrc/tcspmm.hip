@@ -7,8 +7,8 @@
 // fp16 inputs, fp32 accumulation, fp16 or fp32 output.
 //
 // With a plan (stir_tc_plan: the long tiles listed once, longest first, in pieces) a product is one launch of
-// tcspmm_units_kernel, or of tcspmm_direct_kernel above 64 features.  Bound by the gather of rows of B where there are tiles enough, else by the chain id -> row of B
-// -> product of the longest unit.  Before, the tiles of up to 16 steps went as below and the pieces of the others in a
+// tcspmm_units_kernel, or of tcspmm_direct_kernel above 64 features (tc_form).  Bound by the gather of rows of B where there
+// are tiles enough, else by the chain id -> row of B -> product of the longest unit.  Before, the tiles of up to 16 steps went as below and the pieces of the others in a
 // second launch, a workgroup of 16 wavefronts each.  Tiles of 16 rows, power-law rows of up to 500 to 17.5 k nonzeros,
 // uniform columns, us: 25.9 k rows, 626 k nonzeros, 32 features 22.4 -> 10.8; 167 k, 3.8 M, 32: 83 -> 66; 24 k, 244 k,
 // 64: 22.2 -> 10.8; 200 k, 4 M, 64: 101 -> 90; 33 k, 648 k, 224: 61 -> 48; 169 k, 1.17 M, 128: 62.1 -> 62.7 over the

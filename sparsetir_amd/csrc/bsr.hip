@@ -1262,8 +1262,11 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // 250, 31 drawn shapes of 28 to 44 steps 0.96 of the time of 256; less of it, 722 columns, 25 steps, 2752 174 / 176 / 173, 575, 16 steps, 2784
     // 39 / 42 / 39.  From 16 steps on 256 with few tiles, where the order gives little: 1024 columns, 24 steps, 1024 features 100 / 99 /
     // 90, but 490, 17 steps, 512 34 / 40 / 40.
+    // Blocks of several slices, with what such tiles of 256 would waste or too few of them, from 36 steps on; 128 by four as they come
+    // are 0.89 to 0.95 of the time below (600 drawn shapes, 4 to 40 MB of X; none above 1.11), 0.92 to 1.02 above: 78 x 108 of 112, 26
+    // steps, 832 features 83 ranked, 72.
     const bool wide_ranked = fits && (even || waste * 16 <= feat);
-    if (x_bytes > kMuchX && feat > kTileF && steps >= 16 && !(several && fits)) {
+    if (x_bytes > kMuchX && feat > kTileF && steps >= (several ? 36 : 16) && !(several && fits)) {
       const int wide_from = x_bytes > kFarX && wide_tiles > 4 ? 44 : 28;
       if (wide_ranked && (steps >= wide_from || (wide_tiles >= 2 && wide_tiles <= 4 && x_bytes > kBeyondL2)))
         return {BsrForm::kWaves, true, true, false, 1};
@@ -1278,13 +1281,14 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     if (!several && steps >= 20 && x_bytes > kFarX && tiles * 10 >= 46 * cus && tiles < 10 * cus)
       return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
     // Blocks of several slices else.  A, which every tile reads, more than the last level holds, 128 by four / 256 by four / by one:
-    // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Far more X than an L2 holds, 128 by four / two of 128: 1214 x 659 of
-    // 80, 10 steps, 416 features 138 / 130.  Wide tiles and enough of them: from 16 steps on 256 by four, 0.92 to 1.0 of the time by one;
-    // with 5 to 15 steps two of 128, 0.91 to 0.97 of the time of 256 by one whatever X (1100 x
-    // 341 of 48, 10 steps, 1024 features 256 by one / by four / two of 128 142 / 135 / 118); with fewer 128 by one (below), 0.92.
+    // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Wide tiles and enough of them: from 16 steps on 256 by four, 0.92
+    // to 1.0 of the time by one; with 5 to 15 steps two of 128, 0.91 to 0.97 of the time of 256 by one whatever X (1100 x 341 of 48, 10
+    // steps, 1024 features 256 by one / by four / two of 128 142 / 135 / 118); with fewer 128 by one (below), 0.92.  Far more X than
+    // an L2 holds and less than 16 steps, 128 by four / two of 128: 1214 x 659 of 80, 10 steps, 416 features 138 / 130, with more steps
+    // 0.84 / 1.
     if (several && feat > kTileF && (nnzb * blk * blk * 2 > kLastLevel || (fits && steps >= 16 && (even || x_bytes > kMuchX))))
       return {BsrForm::kWaves, true, false, false, 4};
-    if (several && feat >= kWaveF && (x_bytes > 15000000 || (fits && steps >= 5 && steps < 16)))
+    if (several && feat >= kWaveF && steps < 16 && (x_bytes > 15000000 || (fits && steps >= 5)))
       return {BsrForm::kGroups, true, false, false, 2};
     // X in an L2, 128 by one / by four / two of 128 / 256: 342 x 83 of 16, 4 steps, 1728 features 14.8 / 17.2 / 16.2 / 16.7; 420
     // columns, 10 steps, 512 24.5 / 24.5 / - / 23.3; 300, 12 steps, 1024 47.8 / 47.2 / - / 43.7; 73, 8 steps, 3904 67 / 73 / 65 /

@@ -50,7 +50,12 @@ from helpers import bsr_form
     (137, 84, 80, 27, 1824, "256 by 4"),
     (137, 84, 80, 29, 1824, "256 by 4 ranked"),
     (330, 320, 48, 39, 1280, "256 by 4 ranked"),
-    (137, 84, 80, 29, 1312, "128 by 1 ranked"),       # a last tile of 256 mostly empty
+    (137, 84, 80, 29, 1312, "128 by 4"),              # a last tile of 256 mostly empty
+    (137, 84, 80, 35, 1312, "128 by 4"),
+    (137, 84, 80, 36, 1312, "128 by 1 ranked"),
+    (78, 108, 112, 26, 832, "128 by 4"),
+    (430, 650, 48, 15, 608, "128 by 2, two tiles"),   # far more X than an L2 holds
+    (430, 650, 48, 17, 608, "128 by 4"),
     (30, 84, 80, 29, 1824, "128 by 4"),               # few
     (97, 38, 112, 27, 2720, "256 by 4"),              # X in an L2
     (97, 38, 112, 15, 2720, "128 by 2, two tiles"),

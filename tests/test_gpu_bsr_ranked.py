@@ -107,7 +107,8 @@ def _cus():
     (430, 1000, 16, 0.04, 672, "128 by 1 ranked"),
     (171, 170, 48, 0.07, 1024, "256 by 4"),
     (171, 170, 48, 0.16, 1024, "256 by 4 ranked"),     # the slices of a block row on one XCD
-    (200, 330, 48, 0.05, 608, "128 by 1 ranked"),
+    (200, 330, 48, 0.05, 608, "128 by 4"),
+    (200, 330, 48, 0.08, 608, "128 by 1 ranked"),
     (230, 140, 48, 0.03, 1024, "128 by 2, two tiles"),
     (110, 40, 80, 0.2, 1024, "256 by 4"),             # little X, long rows
     (400, 140, 48, 0.03, 288, "128 by 4"),

@@ -1248,12 +1248,14 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // steps (399) 15.7 / 15.4, 22 steps (996) 14.8 / 16.0.
     if (tiles <= cus && steps >= 20) return {BsrForm::kSplit, false, false, false, 8};
     // Much X and long rows, blocks of several slices, which read the same X: 256 by four in order of length.  Of the time by one
-    // wavefront (ranked), blocks of 80 and 112, 28 to 44 steps 0.88 to 0.97, more 0.9, as they come 0.9 to 0.97; of 48, 28 to 34 steps
-    // 1.0, 0.98 as they come (328 x 190, 29 steps, 1376 features 169, 157 by one) but 1.2 where X is far more than an L2 holds (224 x
-    // 336, 35 steps, 2208 features 260, 216 by one), more 0.96, 1.0 to 1.02.
-    if (several && x_bytes > kMuchX && feat > kTileF && steps >= (blk > 48 || x_bytes > kFarX ? 28 : 36) &&
-        waste * 8 <= feat && waves >= 6 * cus)
-      return {BsrForm::kWaves, true, true, false, 4};
+    // wavefront (ranked), 28 steps and more, blocks of 80 and up 0.89 to 0.95, as they come 0.93 to 0.97, 128 by four 0.96 to 1.0; of
+    // 48, 0.90 with more than 9 MB of X, 0.98 from 36 steps on.  With less of both 1.02, as they come 1.01, 128 by four 0.97 (388 x
+    // 309, 28 steps, 1408 features 176 / 164 / 148).  And one feature tile gives the order nothing to share: 128 by four 0.81 to 0.95
+    // of the time in order with 28 to 35 steps, 0.89 to 1.02 with more (763 x 273 of 48, 30 steps 79 / 62).
+    if (several && x_bytes > kMuchX && feat > kTileF && steps >= 28 && waste * 8 <= feat && waves >= 6 * cus) {
+      const bool order = wide_tiles > 1 && (blk > 48 || steps >= 36 || x_bytes > 9000000);
+      return {BsrForm::kWaves, order, order, false, 4};
+    }
     // Much X else: in order of length, by one wavefront, 128 or 256 by what the last tile of 256 wastes.  128 by four as they come / 128
     // ranked / 256 ranked: blocks of 16, 1024 columns (8.4 MB), 51 steps, 1024 features 205 / 188 / 163, 24 steps 105 / 104 / 94,
     // 4096 features 1204 / 736 / 618; 829 columns, 49 steps, 1632 features (12.75 tiles of 128) 200 / 170 / 184.

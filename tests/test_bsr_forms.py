@@ -50,6 +50,10 @@ from helpers import bsr_form
     (137, 84, 80, 27, 1824, "256 by 4"),
     (137, 84, 80, 29, 1824, "256 by 4 ranked"),
     (330, 320, 48, 39, 1280, "256 by 4 ranked"),
+    (763, 273, 48, 30, 256, "128 by 4"),              # one feature tile
+    (763, 273, 48, 36, 480, "256 by 4 ranked"),
+    (763, 371, 48, 30, 480, "256 by 4 ranked"),       # far more X than an L2 holds
+    (137, 84, 80, 29, 256, "128 by 4"),
     (137, 84, 80, 29, 1312, "128 by 4"),              # a last tile of 256 mostly empty
     (137, 84, 80, 35, 1312, "128 by 4"),
     (137, 84, 80, 36, 1312, "128 by 1 ranked"),
@@ -60,8 +64,8 @@ from helpers import bsr_form
     (97, 38, 112, 27, 2720, "256 by 4"),              # X in an L2
     (97, 38, 112, 15, 2720, "128 by 2, two tiles"),
     (97, 38, 112, 4, 2720, "128 by 1"),
-    (328, 190, 48, 29, 1376, "256 by 4"),
-    (224, 336, 48, 29, 2208, "256 by 4 ranked"),
+    (328, 190, 48, 29, 1376, "128 by 4"),
+    (224, 336, 48, 29, 2208, "128 by 4"),
     (97, 38, 112, 19, 2400, "128 by 2, two tiles"),   # an odd number of tiles of 128
     (22, 174, 48, 11, 320, "128 by 4"),
     (600, 650, 48, 7, 256, "128 by 2, two tiles"),

@@ -1196,14 +1196,18 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // / 69.  Eight where a CU has one tile and many steps: 131 x 322, 78 steps, 128 features 14.9, four 16.2.
     const bool few = steps < 4, apart = blk % 64 != 0;  // apart: no workgroup of 64 rows
     if (tiles <= cus && steps >= 24) return {BsrForm::kSplit, false, false, false, 8};
-    const int four = apart ? (steps < 8 ? 8 : 9) : few ? 6 : 9;
+    const int four = apart ? (steps < 8 ? 8 : 9) : few ? 6 : steps < 48 ? 9 : 11;
     if (tiles * 4 <= four * cus) return {BsrForm::kSplit, false, false, false, 4};
     // (64 rows that share X, by a workgroup below, pass two wavefronts in turn where rows are long and CUs have more than three
     // tiles: blocks of 64, 672 features, 46 steps (804 tiles) 31 / 37, 928, 31 steps (817) 23 / 26, of 128, 2304, 92 steps (792) 50 /
-    // 57; but 1600, 69 steps (676) 43 / 38, of 64, 2240, 30 steps (755) 23.0 / 19.7; and with few steps)
+    // 57; but of 64, 2240, 30 steps (755) 23.0 / 19.7; and with few steps.  Four pass two from 48 steps on up to 2.75 tiles, 0.93 of
+    // the time over 3200 drawn shapes: 22 x 126 of 128, 136 steps, 864 features, fp32 results 66 / 74.  Up to 24 steps two keep 3 to
+    // 3.25 tiles of blocks of 64 where there is X enough, 0.99; over little of it the workgroups take 0.95, and of 128 dealt to XCDs
+    // 0.97: 51 x 7 of 128, 21 steps, 416 features, fp32 results 13.2 / 17.1)
     const int two = few && !(apart && floats)           ? 0
                     : apart                             ? (x_tile_bytes(kWaveF) <= kFarX ? 16 : 13)
-                    : steps < 24 ? 13 : steps < 48 ? 12 : 11;
+                    : steps >= 48   ? 0
+                                    : (blk < 128 && steps < 24 && x_tile_bytes(kWaveF) > 1000000 ? 13 : 12);
     if (tiles * 4 <= two * cus) return {BsrForm::kSplit, false, false, false, 2};
   } else if (unit == 32) {
     // The split form wins as long as its workgroups are resident at once, two per CU, and up to twice as many where block rows

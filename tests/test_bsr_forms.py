@@ -31,6 +31,12 @@ from helpers import bsr_form
     (57, 18, 96, 8, 704, "128 by 1"),
     (18, 12, 128, 3, 1344, "LDS 64 x 128"),          # few steps: 64 rows by a workgroup
     (77, 115, 128, 21, 64, "LDS 64 by 8"),
+    (22, 126, 128, 136, 864, "128 by 4"),            # 2.4 tiles a compute unit
+    (22, 126, 128, 47, 864, "128 by 2"),
+    (26, 126, 128, 136, 864, "LDS 64 x 128"),        # 2.8
+    (102, 140, 64, 21, 416, "128 by 2"),             # 3.2
+    (102, 14, 64, 21, 416, "LDS 64 x 128"),          # little X
+    (51, 7, 128, 21, 416, "LDS 64 x 128 by rows"),
     # 64 rows by four wavefronts
     (1024, 256, 64, 12, 1024, "LDS 64 x 256"),
     (1024, 256, 64, 24, 1024, "LDS 64 x 256 ranked"),

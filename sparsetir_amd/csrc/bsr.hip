@@ -1182,10 +1182,14 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // hardly more than the CUs, with twice as much as the next: 35 x 437 blocks, 97 steps, 96 features 14.6 us, 16.9 with 128;
     // 42 x 285, 70 steps, 64 10.6, 11.3; 93 x 431, 106 steps, 320 (279 tiles) 26.0, 29.6; but 136 x 333, 67 steps, 256 (272, and
     // 544 of 64) 24.1, 20.8.  A little sooner where 128 waste half of a load: 8 x 35 of 128, 35 steps, 192 features 9.4, 10.1.
-    // Of 64 features alone from 20 steps on: 77 x 115 of 128, 21 steps 13.3, 14.6, 24 x 99 of 64, 29 steps 8.6, 9.5.
+    // Of 64 features alone from 20 steps on: 77 x 115 of 128, 21 steps 13.3, 14.6, 24 x 99 of 64, 29 steps 8.6, 9.5; and from 32
+    // steps on in two turns: 189 x 56 of 128, 154 steps (756) 58.5, 76.4 (260 drawn shapes 0.87 of the time, none above 1.04).
+    // Three quarters of a turn where the last 64 are half empty, 62 x 196 of 32, 66 steps, 224 features (248) 12.1, 11.6; all of it from
+    // 100 steps on: 17 x 150 of 96, 275 steps, 224 features 35.5, 42.8 (1000 drawn shapes 0.91, none above 1.03).
     const bool half = feat % kTileF != 0 && feat % kTileF <= kSplitF;
-    if ((steps >= 40 && (split * 4 <= (feat % kSplitF ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus))) ||
-        (steps >= 32 && half && split <= cus) || (steps >= 20 && feat <= kSplitF && split <= 2 * cus))
+    const bool ragged = feat % kSplitF != 0 && (steps < 100 || feat <= kTileF);
+    if ((steps >= 40 && (split * 4 <= (ragged ? 3 : 4) * cus || (tiles > cus && split <= 2 * cus))) ||
+        (steps >= 32 && half && split <= cus) || (steps >= 20 && feat <= kSplitF && split <= (steps < 32 ? 2 : 4) * cus))
       return {BsrForm::kSplit, false, false, false};
     // Steps in turn as long as that leaves a CU little more than two workgroups of four wavefronts, or four of two.  Means over
     // 5000 drawn shapes, four wavefronts to a tile / two: up to 1.5 tiles a CU 0.7 to 0.95, 1.5 to 2.25 0.92 to 1.0 (the latter for 4
@@ -1250,6 +1254,9 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
       return {BsrForm::kSplit, false, false, false};
     // 128 by four / by eight: 80 steps, 96 features (154 tiles) 16.5 / 13.0, 33 steps (136) 8.5 / 7.6, 15 steps (220) 5.6 / 5.6; 60
     // steps (399) 15.7 / 15.4, 22 steps (996) 14.8 / 16.0.
+    // Of blocks of several slices with much X, 64 by eight through LDS also where 128 have no more than a turn, from 100 steps on: 3 x
+    // 68 of 144, 196 steps, 416 features 24.3, 28.5 (1300 drawn shapes of 80 and more 0.91 of the time).
+    if (blk >= 80 && feat > kTileF && steps >= 100 && x_bytes > kBeyondL2 && split <= cus) return {BsrForm::kSplit, false, false, false};
     if (tiles <= cus && steps >= 20) return {BsrForm::kSplit, false, false, false, 8};
     // Much X and long rows, blocks of several slices, which read the same X: 256 by four in order of length.  Of the time by one
     // wavefront (ranked), 28 steps and more, blocks of 80 and up 0.89 to 0.95, as they come 0.93 to 0.97, 128 by four 0.96 to 1.0; of

@@ -37,6 +37,12 @@ from helpers import bsr_form
     (102, 140, 64, 21, 416, "128 by 2"),             # 3.2
     (102, 14, 64, 21, 416, "LDS 64 x 128"),          # little X
     (51, 7, 128, 21, 416, "LDS 64 x 128 by rows"),
+    (17, 150, 96, 275, 224, "LDS 64 by 8"),          # 64 features by eight: a turn of them
+    (17, 150, 96, 99, 224, "128 by 8"),              # ... of which the last are half empty
+    (30, 150, 96, 275, 96, "LDS 64 by 8"),
+    (40, 150, 96, 275, 96, "128 by 8"),              # ... of one tile of 128
+    (360, 190, 64, 234, 64, "LDS 64 by 8"),          # two turns of 64 features alone
+    (360, 190, 64, 31, 64, "128 by 2"),
     # 64 rows by four wavefronts
     (1024, 256, 64, 12, 1024, "LDS 64 x 256"),
     (1024, 256, 64, 24, 1024, "LDS 64 x 256 ranked"),
@@ -77,6 +83,9 @@ from helpers import bsr_form
     (600, 650, 48, 7, 256, "128 by 2, two tiles"),
     (3693, 559, 48, 11, 320, "128 by 1"),
     (1214, 659, 80, 10, 416, "128 by 2, two tiles"),
+    (3, 68, 144, 196, 416, "LDS 64 by 8"),            # long rows, much X, a turn of 64 features by eight
+    (3, 68, 144, 99, 416, "128 by 8"),
+    (3, 50, 144, 196, 416, "128 by 8"),
     (3000, 68, 80, 8, 800, "128 by 1"),
     (3000, 68, 80, 20, 800, "256 by 4"),            # A beyond the last level
 ])

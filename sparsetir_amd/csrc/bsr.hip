@@ -1291,7 +1291,10 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
     // way each where there are more of them; 128 by four / by one with two steps / with one: 95 x 793, 26 steps, 1856 features
     // (1425 tiles) 24.8 / 22.1 / 23.7, 80 x 818, 23 steps, 2848 (1840) 34.5 / 30.9 / 28.6, 70 x 896, 40 steps, 2848 (1610) 48.4 / 40.6 /
     // 37.8, 183 x 840, 64 steps, 1568 (2379) 84.5 / 83.5 / 80.6; but 4.35 tiles to a CU, 90 steps, 320 features 50.5 / 52.3 / 61.5.
-    if (!several && steps >= 20 && x_bytes > kFarX && tiles * 10 >= 46 * cus && tiles < 10 * cus)
+    // With many feature tiles from 15 steps and 5 MB on, 0.93 of the time of 128 by four over 2300 drawn shapes: 100 x 902, 18 steps,
+    // 2912 features (2300) 29.7 / 36.6, 79 x 657, 20 steps, 3616 (2291) 29.9 / 36.6, 44 x 626, 26 steps, 4064 (1408) 24.8 / 30.7.
+    const bool far = (steps >= 20 && x_bytes > kFarX) || (steps >= 15 && x_bytes > 5000000 && wide_tiles > 4);
+    if (!several && far && tiles * 10 >= 46 * cus && tiles < 10 * cus)
       return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
     // Blocks of several slices else.  A, which every tile reads, more than the last level holds, 128 by four / 256 by four / by one:
     // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Wide tiles and enough of them: from 16 steps on 256 by four, 0.92

@@ -58,6 +58,12 @@ from helpers import bsr_form
     (521, 872, 16, 44, 3168, "256 by 1 ranked"),
     (521, 700, 16, 32, 3168, "256 by 1 ranked"),
     (1024, 872, 16, 32, 1024, "256 by 1 ranked"),     # few
+    (100, 902, 16, 18, 2912, "128 by 1, one step"),   # a turn of wavefronts over far more X than the L2s hold
+    (79, 657, 16, 20, 3616, "128 by 1, one step"),
+    (44, 626, 16, 26, 4064, "128 by 1"),
+    (44, 626, 16, 14, 4064, "128 by 4"),
+    (79, 600, 16, 20, 3616, "128 by 4"),
+    (250, 657, 16, 20, 992, "128 by 4"),              # few feature tiles
     (1100, 341, 48, 10, 1024, "128 by 2, two tiles"),
     (137, 84, 80, 27, 1824, "256 by 4"),
     (137, 84, 80, 29, 1824, "256 by 4 ranked"),

@@ -1298,11 +1298,12 @@ BsrForm bsr_form(int64_t cus, int mb, int nb, int blk, int feat, int64_t nnzb, b
       return {BsrForm::kWaves, false, false, false, 1, tiles >= 6 * cus};
     // Blocks of several slices else.  A, which every tile reads, more than the last level holds, 128 by four / 256 by four / by one:
     // 3000 x 68 of 80, 20 steps, 800 features 1317 / 1009 / 1067.  Wide tiles and enough of them: from 16 steps on 256 by four, 0.92
-    // to 1.0 of the time by one; with 5 to 15 steps two of 128, 0.91 to 0.97 of the time of 256 by one whatever X (1100 x 341 of 48, 10
+    // to 1.0 of the time by one (blocks of 48 with much X 128 by four, 0.965 of that: 269 x 331, 25 steps, 1248 features, fp32 results
+    // 109 / 118); with 5 to 15 steps two of 128, 0.91 to 0.97 of the time of 256 by one whatever X (1100 x 341 of 48, 10
     // steps, 1024 features 256 by one / by four / two of 128 142 / 135 / 118); with fewer 128 by one (below), 0.92.  Far more X than
     // an L2 holds and less than 16 steps, 128 by four / two of 128: 1214 x 659 of 80, 10 steps, 416 features 138 / 130, with more steps
     // 0.84 / 1.
-    if (several && feat > kTileF && (nnzb * blk * blk * 2 > kLastLevel || (fits && steps >= 16 && (even || x_bytes > kMuchX))))
+    if (several && feat > kTileF && (nnzb * blk * blk * 2 > kLastLevel || (fits && steps >= 16 && (x_bytes > kMuchX ? blk > 48 : even))))
       return {BsrForm::kWaves, true, false, false, 4};
     if (several && feat >= kWaveF && steps < 16 && (x_bytes > 15000000 || (fits && steps >= 5)))
       return {BsrForm::kGroups, true, false, false, 2};

@@ -78,6 +78,8 @@ from helpers import bsr_form
     (78, 108, 112, 26, 832, "128 by 4"),
     (430, 650, 48, 15, 608, "128 by 2, two tiles"),   # far more X than an L2 holds
     (430, 650, 48, 17, 608, "128 by 4"),
+    (269, 331, 48, 25, 1248, "128 by 4"),             # blocks of 48 with much X
+    (269, 120, 48, 25, 1248, "256 by 4"),
     (30, 84, 80, 29, 1824, "128 by 4"),               # few
     (97, 38, 112, 27, 2720, "256 by 4"),              # X in an L2
     (97, 38, 112, 15, 2720, "128 by 2, two tiles"),

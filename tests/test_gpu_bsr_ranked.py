@@ -105,7 +105,7 @@ def _cus():
     # 16-row slices
     (1030, 490, 16, 0.07, 512, "256 by 1 ranked"),
     (430, 1000, 16, 0.04, 672, "128 by 1 ranked"),
-    (171, 170, 48, 0.07, 1024, "256 by 4"),
+    (171, 120, 48, 0.1, 1024, "256 by 4"),
     (171, 170, 48, 0.16, 1024, "256 by 4 ranked"),     # the slices of a block row on one XCD
     (200, 330, 48, 0.05, 608, "128 by 4"),
     (200, 330, 48, 0.08, 608, "128 by 1 ranked"),

@@ -940,10 +940,12 @@ TcForm tc_form(int T, bool out32, int64_t mb, int feat, int64_t nnzb, int64_t n_
   //   4.2 M 154 / 165, skewed columns 123 / 135 (but of 50 k rows 40 / 35); 4 steps 116 / 110, 2.2 steps 29.9 / 30.1, 4125 tiles of
   //   6.3 steps 26.4 / 25.2;
   //   32 features in a unit of 128 of their own, 32-row tiles, of which hardly a turn is resident (64 KB of sums each): 12 k rows, 49
-  //   k nonzeros, 160 features 10.2 / 10.9; with units of 32 KB below that is no reason: 33 k, 165 k, 160 15.7 / 15.3.
+  //   k nonzeros, 160 features 10.2 / 10.9; with units of 32 KB below that is no reason: 33 k, 165 k, 160 15.7 / 15.3.  Of 8-row tiles
+  //   where the empty part is about what another turn is of: 14 k, 370 k, 160 20.7 / 22.1 (1300 to 2000 tiles 0.95 to 0.97 of the
+  //   time, 2.4 to 13 steps; fewer 1.02, more 0.99 to 1.4).
   const int64_t wide_units = (mb + n_pieces) * stir::ceil_div(feat, 128);
   const bool halves = T == 8 && feat == 128 && mb >= 6000 && nnzb >= 9 * mb;
-  const bool lone = T == 32 && feat % 128 == 32 && wide_units < 1300;
+  const bool lone = feat % 128 == 32 && (T == 32 ? wide_units < 1300 : T == 8 && wide_units >= 2600 && wide_units < 4000);
   const int tiles = feat <= 32 ? 1 : feat > 64 && !halves && !lone ? 4 : 2;
   const int64_t units = (mb + n_pieces) * stir::ceil_div(feat, 32 * tiles);
   // Four wavefronts shorten a unit, two leave fewer of them without a step: 64 features, 25 k tiles of 1.5 and of 5.2

@@ -82,6 +82,7 @@ def test_a_unit_of_32_features(dev, t, feat, out_dtype):
     (32, 96, torch.float16, 1300, "128 by 4, one step"),
     (32, 160, torch.float32, 650, "128 by 4, one step"),
     (32, 160, torch.float32, 600, "64 by 4"),
+    (8, 160, torch.float16, 1500, "64 by 4"),
     (32, 192, torch.float16, 2600, "128 by 2, one step"),
     (32, 192, torch.float32, 2600, "128 by 2, one step"),
     (32, 256, torch.float16, 2600, "128 by 2"),

@@ -32,7 +32,10 @@ from helpers import tc_form
     (8, 21168, 256, 13, "f16", "128 by 2, one step"),
     (8, 2500, 224, 3, "f32", "128 by 2"),
     (8, 4125, 192, 4, "f16", "128 by 2"),
-    # 32 features in a unit of their own, whatever the rows of B; not in a small launch of 32-row tiles
+    # 32 features in a unit of their own; not in a small launch of 32-row tiles or a turn of 8-row ones
+    (8, 1793, 160, 13, "f16", "64 by 4"),
+    (8, 1250, 160, 13, "f16", "128 by 4, one step"),
+    (8, 2050, 160, 3, "f16", "128 by 4, one step"),
     (16, 1250, 160, 5, "f16", "128 by 4"),
     (8, 2500, 160, 3, "f32", "128 by 2"),
     (32, 375, 160, 8, "f32", "64 by 4"),
